@@ -277,6 +277,47 @@ int hiprwkv_rwkv7_vmix(hiprwkv_stream stream, int io_dtype, int64_t rows, int64_
 int hiprwkv_rwkv7_vmix_bwd(hiprwkv_stream stream, int io_dtype, int64_t rows, int64_t C, const void* v, const void* v_first,
                            const void* x, const void* v0, const void* g, void* dv, void* dv_first, void* dx, float* dv0);
 
+/* ---- RWKV-7 sub-block head: residual addition, LayerNorm, token shift, interpolation --------------------
+ * rwkv7.py:8-12 and :226-235 / :192-195 in one pass:
+ *     xs = x + dx ,  xn = layer_norm(xs; ln_w, ln_b, eps) ,  sx_t = (new_starts[t] ? 0 : xn_{t-1}) - xn_t ,
+ *     out_i = xn + sx . mix_i ,  i < n_out  (6, 1; 0: out_0 = xn)
+ * Every tensor io_dtype; xs and xn are rounded to it.  dx may be NULL (xs is then x and is not written).  `prev` as in
+ * hiprwkv_rwkv7_shiftmix (unused for n_out = 0).  shift (may be NULL): row b, `shift_batch_stride` elements after row
+ * b - 1, receives xn of token (length[b] - 1) mod T; length (B,) int32 or NULL (= T).  stats (may be NULL): (B*T, 2) fp32
+ * mean and 1/std of xs for the backward pass.  C a multiple of 8, at most 4096. */
+int hiprwkv_rwkv7_ln_shiftmix(hiprwkv_stream stream, int io_dtype, int64_t B, int64_t T, int64_t C, int n_out,
+                              const void* x, const void* dx, const void* ln_w, const void* ln_b, float eps,
+                              const void* prev, int64_t prev_batch_stride, const uint8_t* new_starts,
+                              const int32_t* length, const void* const* mix, void* const* out, void* xs, void* shift,
+                              int64_t shift_batch_stride, float* stats);
+size_t hiprwkv_rwkv7_ln_shiftmix_bwd_workspace_bytes(int64_t B, int64_t T, int64_t C, int n_out);
+/* Cotangents for g[i] (B,T,C) of the outputs, gx (B,T,C, may be NULL) of xs and gshift (B,C, may be NULL) of the shift rows:
+ * dxs (B,T,C), the cotangent of x and of dx; dprev (B,C, may be NULL); dparam: n_out + 2 arrays (C,) io_dtype, the mix
+ * vectors' then ln_w's and ln_b's.  xs and stats are the forward's. */
+int hiprwkv_rwkv7_ln_shiftmix_bwd(hiprwkv_stream stream, int io_dtype, int64_t B, int64_t T, int64_t C, int n_out,
+                                  const void* xs, const float* stats, const void* ln_w, const void* ln_b,
+                                  const void* prev, int64_t prev_batch_stride, const uint8_t* new_starts,
+                                  const int32_t* length, const void* const* mix, const void* const* g, const void* gx,
+                                  const void* gshift, void* dxs, void* dprev, void* const* dparam, void* workspace,
+                                  size_t workspace_bytes);
+
+/* ---- RWKV-7: everything element-wise between the projections and the WKV op ----------------------------
+ * hiprwkv_rwkv7_decay, _vmix, _agate and _premix in one pass, with their results: token tensors (rows, H, 64),
+ * parameters (H, 64), all io_dtype.  v_first NULL: no value residual (v, xv, v0, v_out unused). */
+int hiprwkv_rwkv7_pre(hiprwkv_stream stream, int io_dtype, int64_t rows, int64_t H, int64_t N, const void* xw,
+                      const void* k, const void* xa, const void* v, const void* v_first, const void* xv, const void* w0,
+                      const void* a0, const void* v0, const void* k_k, const void* k_a, void* w, void* k_out,
+                      void* v_out, void* a_out, void* b_out);
+size_t hiprwkv_rwkv7_pre_bwd_workspace_bytes(int64_t rows, int64_t H, int64_t N);
+/* From the cotangents of w, k_out, v_out, a_out, b_out to those of the inputs; dparam: (H, 64) io_dtype arrays of w0, a0,
+ * k_k, k_a and, with v_first, v0. */
+int hiprwkv_rwkv7_pre_bwd(hiprwkv_stream stream, int io_dtype, int64_t rows, int64_t H, int64_t N, const void* xw,
+                          const void* k, const void* xa, const void* v, const void* v_first, const void* xv,
+                          const void* w0, const void* a0, const void* v0, const void* k_k, const void* k_a,
+                          const void* gw, const void* gk_out, const void* gv_out, const void* ga_out,
+                          const void* gb_out, void* dxw, void* dk, void* dv, void* dv_first, void* dxv, void* dxa,
+                          void* const* dparam, void* workspace, size_t workspace_bytes);
+
 /* ---- RWKV-7 time-mixing stages around the op ------------------------------------------
  * The element-wise work the reference does in jnp on either side of inner_loop (rwkv7.py:248-252, 257 and :263-265),
  * fused into one pass each; it has no counterpart among the reference's ffi targets.  `rows` = number of tokens

@@ -55,6 +55,13 @@ SIGNATURES = {
     "hiprwkv_rwkv7_relusq_bwd": (_int, [_vp, _int, _i64, _vp, _vp, _vp]),
     "hiprwkv_rwkv7_vmix": (_int, [_vp, _int, _i64, _i64, _vp, _vp, _vp, _vp, _vp]),
     "hiprwkv_rwkv7_vmix_bwd": (_int, [_vp, _int, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "hiprwkv_rwkv7_ln_shiftmix": (_int, [_vp, _int, _i64, _i64, _i64, _int] + [_vp] * 4 + [ctypes.c_float, _vp, _i64]
+                                  + [_vp] * 6 + [_i64, _vp]),
+    "hiprwkv_rwkv7_ln_shiftmix_bwd_workspace_bytes": (_sz, [_i64] * 3 + [_int]),
+    "hiprwkv_rwkv7_ln_shiftmix_bwd": (_int, [_vp, _int, _i64, _i64, _i64, _int] + [_vp] * 5 + [_i64] + [_vp] * 10 + [_sz]),
+    "hiprwkv_rwkv7_pre": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 16),
+    "hiprwkv_rwkv7_pre_bwd_workspace_bytes": (_sz, [_i64] * 3),
+    "hiprwkv_rwkv7_pre_bwd": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 24 + [_sz]),
     "hiprwkv_rwkv7_premix": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 7),
     "hiprwkv_rwkv7_postmix": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 8 + [ctypes.c_float, _vp]),
     "hiprwkv_rwkv7_premix_bwd": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 11),

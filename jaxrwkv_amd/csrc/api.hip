@@ -672,4 +672,143 @@ int hiprwkv_rwkv7_postmix_bwd(hiprwkv_stream stream, int io_dtype, int64_t rows,
   return HIPRWKV_OK;
 }
 
+namespace {
+int check_ln_mix(const char* op, int io_dtype, const LnMixArgs& A, int n_out, const void* const* per_out,
+                 std::initializer_list<const void*> req, std::initializer_list<const void*> opt) {
+  if (!dtype_ok(io_dtype)) return fail(HIPRWKV_EINVAL, "%s: dtype must be HIPRWKV_F32 or HIPRWKV_BF16", op);
+  if (A.B <= 0 || A.T <= 0 || A.C <= 0 || A.C % 8 != 0 || A.C > 4096)
+    return fail(HIPRWKV_EINVAL, "%s: B, T must be positive and C a positive multiple of 8 of at most 4096", op);
+  if (A.B * A.T > 0x7fffffffLL) return fail(HIPRWKV_EINVAL, "%s: too many tokens for one launch", op);
+  if (n_out != 0 && n_out != 1 && n_out != 6) return fail(HIPRWKV_EINVAL, "%s: n_out must be 0, 1 or 6", op);
+  for (const void* p : req)
+    if (p == nullptr || !aligned16(p)) return fail(HIPRWKV_EINVAL, "%s: null or misaligned tensor pointer (16 bytes)", op);
+  for (const void* p : opt)
+    if (p != nullptr && !aligned16(p)) return fail(HIPRWKV_EINVAL, "%s: tensor pointers must be 16-byte aligned", op);
+  const int64_t elem = io_dtype == HIPRWKV_F32 ? 4 : 2;
+  if (n_out != 0) {
+    if (A.prev == nullptr || !aligned16(A.prev)) return fail(HIPRWKV_EINVAL, "%s: null or misaligned shift row", op);
+    if (A.prev_bstride < A.C || (A.prev_bstride * elem) % 16 != 0)
+      return fail(HIPRWKV_EINVAL, "%s: the batch stride of the shift row must be at least C and a multiple of 16 bytes", op);
+  }
+  if (A.shift != nullptr && (A.shift_bstride < A.C || (A.shift_bstride * elem) % 16 != 0))
+    return fail(HIPRWKV_EINVAL, "%s: the batch stride of the new shift row must be at least C and a multiple of 16 bytes", op);
+  for (int i = 0; i < n_out; ++i)
+    if (A.mix[i] == nullptr || !aligned16(A.mix[i])) return fail(HIPRWKV_EINVAL, "%s: null or misaligned mix vector", op);
+  for (int i = 0; i < (n_out ? n_out : 1); ++i)
+    if (per_out[i] == nullptr || !aligned16(per_out[i])) return fail(HIPRWKV_EINVAL, "%s: null or misaligned tensor pointer", op);
+  return HIPRWKV_OK;
+}
+}  // namespace
+
+int hiprwkv_rwkv7_ln_shiftmix(hiprwkv_stream stream, int io_dtype, int64_t B, int64_t T, int64_t C, int n_out,
+                              const void* x, const void* dx, const void* ln_w, const void* ln_b, float eps,
+                              const void* prev, int64_t prev_batch_stride, const uint8_t* new_starts,
+                              const int32_t* length, const void* const* mix, void* const* out, void* xs, void* shift,
+                              int64_t shift_batch_stride, float* stats) {
+  LnMixArgs A;
+  memset(&A, 0, sizeof(A));
+  A.B = B; A.T = T; A.C = C;
+  A.x = x; A.dx = dx; A.ln_w = ln_w; A.ln_b = ln_b; A.eps = eps;
+  A.prev = prev; A.prev_bstride = prev_batch_stride; A.ns = new_starts; A.length = length;
+  A.xs = xs; A.shift = shift; A.shift_bstride = shift_batch_stride; A.stats = stats;
+  if ((n_out != 0 && mix == nullptr) || out == nullptr) return fail(HIPRWKV_EINVAL, "rwkv7_ln_shiftmix: null pointer array");
+  if (dx != nullptr && xs == nullptr) return fail(HIPRWKV_EINVAL, "rwkv7_ln_shiftmix: dx needs xs");
+  for (int i = 0; i < n_out && i < 6; ++i) A.mix[i] = mix[i];
+  for (int i = 0; i < (n_out ? n_out : 1) && i < 6; ++i) A.out[i] = out[i];
+  if (int rc = check_ln_mix("rwkv7_ln_shiftmix", io_dtype, A, n_out, A.out, {x, ln_w, ln_b}, {dx, xs, shift, stats})) return rc;
+  return gate_done("rwkv7_ln_shiftmix", launch_ln_shiftmix(io_dtype == HIPRWKV_F32, n_out, A, static_cast<hipStream_t>(stream)));
+}
+
+size_t hiprwkv_rwkv7_ln_shiftmix_bwd_workspace_bytes(int64_t B, int64_t T, int64_t C, int n_out) {
+  const int64_t run = ln_shiftmix_bwd_run(B * T);
+  return (size_t)((B * T + run - 1) / run) * (n_out + 2) * C * sizeof(float);
+}
+
+int hiprwkv_rwkv7_ln_shiftmix_bwd(hiprwkv_stream stream, int io_dtype, int64_t B, int64_t T, int64_t C, int n_out,
+                                  const void* xs, const float* stats, const void* ln_w, const void* ln_b,
+                                  const void* prev, int64_t prev_batch_stride, const uint8_t* new_starts,
+                                  const int32_t* length, const void* const* mix, const void* const* g, const void* gx,
+                                  const void* gshift, void* dxs, void* dprev, void* const* dparam, void* workspace,
+                                  size_t workspace_bytes) {
+  LnMixArgs A;
+  memset(&A, 0, sizeof(A));
+  A.B = B; A.T = T; A.C = C;
+  A.xs = const_cast<void*>(xs); A.stats = const_cast<float*>(stats); A.ln_w = ln_w; A.ln_b = ln_b;
+  A.prev = prev; A.prev_bstride = prev_batch_stride; A.ns = new_starts; A.length = length;
+  A.gx = gx; A.gshift = gshift; A.dxs = dxs; A.dprev = dprev; A.part = static_cast<float*>(workspace);
+  if ((n_out != 0 && mix == nullptr) || g == nullptr || dparam == nullptr)
+    return fail(HIPRWKV_EINVAL, "rwkv7_ln_shiftmix_bwd: null pointer array");
+  for (int i = 0; i < n_out && i < 6; ++i) A.mix[i] = mix[i];
+  for (int i = 0; i < (n_out ? n_out : 1) && i < 6; ++i) A.g[i] = g[i];
+  if (int rc = check_ln_mix("rwkv7_ln_shiftmix_bwd", io_dtype, A, n_out, A.g, {xs, stats, ln_w, ln_b, dxs, workspace}, {gx, gshift, dprev}))
+    return rc;
+  for (int i = 0; i < n_out + 2; ++i)
+    if (dparam[i] == nullptr) return fail(HIPRWKV_EINVAL, "rwkv7_ln_shiftmix_bwd: null tensor pointer");
+  const size_t need = hiprwkv_rwkv7_ln_shiftmix_bwd_workspace_bytes(B, T, C, n_out);
+  if (workspace_bytes < need)
+    return fail(HIPRWKV_ENOSPACE, "rwkv7_ln_shiftmix_bwd: workspace has %zu bytes, %zu needed", workspace_bytes, need);
+  return gate_done("rwkv7_ln_shiftmix_bwd", launch_ln_shiftmix_bwd(io_dtype == HIPRWKV_F32, n_out, A, dparam, static_cast<hipStream_t>(stream)));
+}
+
+namespace {
+int check_pre(const char* op, int io_dtype, int64_t N, const PreArgs& A, std::initializer_list<const void*> req,
+              std::initializer_list<const void*> with_vf) {
+  if (!dtype_ok(io_dtype)) return fail(HIPRWKV_EINVAL, "%s: dtype must be HIPRWKV_F32 or HIPRWKV_BF16", op);
+  if (N != 64) return fail(HIPRWKV_EINVAL, "%s: head size N=%lld not supported (64 only)", op, (long long)N);
+  if (A.rows <= 0 || A.H <= 0 || A.H > 65536 || (A.rows * A.H + 3) / 4 > 0x7fffffffLL) return fail(HIPRWKV_EINVAL, "%s: bad rows/H", op);
+  for (const void* p : req)
+    if (p == nullptr || !aligned16(p)) return fail(HIPRWKV_EINVAL, "%s: null or misaligned tensor pointer (16 bytes)", op);
+  if (A.vf != nullptr)
+    for (const void* p : with_vf)
+      if (p == nullptr || !aligned16(p)) return fail(HIPRWKV_EINVAL, "%s: null or misaligned tensor pointer (16 bytes)", op);
+  return HIPRWKV_OK;
+}
+}  // namespace
+
+int hiprwkv_rwkv7_pre(hiprwkv_stream stream, int io_dtype, int64_t rows, int64_t H, int64_t N, const void* xw,
+                      const void* k, const void* xa, const void* v, const void* v_first, const void* xv, const void* w0,
+                      const void* a0, const void* v0, const void* k_k, const void* k_a, void* w, void* k_out,
+                      void* v_out, void* a_out, void* b_out) {
+  PreArgs A;
+  memset(&A, 0, sizeof(A));
+  A.rows = rows; A.H = H;
+  A.xw = xw; A.k = k; A.xa = xa; A.v = v; A.vf = v_first; A.xv = xv;
+  A.w0 = w0; A.a0 = a0; A.v0 = v0; A.k_k = k_k; A.k_a = k_a;
+  A.w = w; A.k_out = k_out; A.v_out = v_out; A.a_out = a_out; A.b_out = b_out;
+  if (int rc = check_pre("rwkv7_pre", io_dtype, N, A, {xw, k, xa, w0, a0, k_k, k_a, w, k_out, a_out, b_out}, {v, v_first, xv, v0, v_out}))
+    return rc;
+  return gate_done("rwkv7_pre", launch_rwkv7_pre(io_dtype == HIPRWKV_F32, A, static_cast<hipStream_t>(stream)));
+}
+
+size_t hiprwkv_rwkv7_pre_bwd_workspace_bytes(int64_t rows, int64_t H, int64_t N) {
+  return (size_t)rwkv7_pre_bwd_rows(rows, H) * 5 * H * N * sizeof(float);
+}
+
+int hiprwkv_rwkv7_pre_bwd(hiprwkv_stream stream, int io_dtype, int64_t rows, int64_t H, int64_t N, const void* xw,
+                          const void* k, const void* xa, const void* v, const void* v_first, const void* xv,
+                          const void* w0, const void* a0, const void* v0, const void* k_k, const void* k_a,
+                          const void* gw, const void* gk_out, const void* gv_out, const void* ga_out,
+                          const void* gb_out, void* dxw, void* dk, void* dv, void* dv_first, void* dxv, void* dxa,
+                          void* const* dparam, void* workspace, size_t workspace_bytes) {
+  PreArgs A;
+  memset(&A, 0, sizeof(A));
+  A.rows = rows; A.H = H;
+  A.xw = xw; A.k = k; A.xa = xa; A.v = v; A.vf = v_first; A.xv = xv;
+  A.w0 = w0; A.a0 = a0; A.v0 = v0; A.k_k = k_k; A.k_a = k_a;
+  A.gw = gw; A.gk = gk_out; A.gv = gv_out; A.ga = ga_out; A.gb = gb_out;
+  A.dxw = dxw; A.dk = dk; A.dv = dv; A.dvf = dv_first; A.dxv = dxv; A.dxa = dxa;
+  A.part = static_cast<float*>(workspace);
+  if (int rc = check_pre("rwkv7_pre_bwd", io_dtype, N, A,
+                         {xw, k, xa, w0, a0, k_k, k_a, gw, gk_out, ga_out, gb_out, dxw, dk, dxa, workspace},
+                         {v, v_first, xv, v0, gv_out, dv, dv_first, dxv}))
+    return rc;
+  if (dparam == nullptr) return fail(HIPRWKV_EINVAL, "rwkv7_pre_bwd: null pointer array");
+  for (int i = 0; i < (v_first != nullptr ? 5 : 4); ++i)
+    if (dparam[i] == nullptr) return fail(HIPRWKV_EINVAL, "rwkv7_pre_bwd: null tensor pointer");
+  const size_t need = hiprwkv_rwkv7_pre_bwd_workspace_bytes(rows, H, N);
+  if (workspace_bytes < need)
+    return fail(HIPRWKV_ENOSPACE, "rwkv7_pre_bwd: workspace has %zu bytes, %zu needed", workspace_bytes, need);
+  return gate_done("rwkv7_pre_bwd", launch_rwkv7_pre_bwd(io_dtype == HIPRWKV_F32, A, dparam, static_cast<hipStream_t>(stream)));
+}
+
 }  // extern "C"

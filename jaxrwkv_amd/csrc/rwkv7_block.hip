@@ -1,0 +1,422 @@
+// The head of an RWKV-7 sub-block in one pass: residual addition, LayerNorm, token shift and interpolation
+// (reference: /root/reference/src/jaxrwkv/rwkv7.py:8-12, :226-235 / :192-195 and :269-291):
+//     xs  = x (+ dx)                                   the residual stream, rounded to the I/O dtype as stored
+//     xn  = (xs - mean) rstd ln_w + ln_b               rounded to the I/O dtype, as the reference's layer_norm returns it
+//     out_i = xn + (xn_prev - xn) mix_i                xn_prev: the token before, the state row at t = 0, 0 at new_starts
+// NOUT = 6 (time mixing), 1 (channel mixing) or 0 (the norm alone: out_0 = xn).  The xn of token (length - 1) mod T of
+// every sequence goes to the shift row of the new model state.
+//
+// Memory bound.  As separate operations (addition, cast to fp32, norm, cast back, gather of the state row, shift and
+// interpolation) the six-output head of a layer moved 21 token tensors in bf16 units, this moves 9.  Measured in bf16 at
+// B=4 T=1021 C=2048: 37 us (4.1 TB/s) and 24 us with one output, against 72 and 55 us for the separate kernels; backward
+// with six cotangents at B=4 T=512 C=768: 27 + 9 us with its reduction, against 66 us for the shift kernel alone.
+// A workgroup spans all channels (eight per thread, one 16-byte access in bf16) and walks a run of consecutive tokens,
+// FWD_GROUP at a time so that the loads of a group are in flight together and a pair of barriers serves all of them; the
+// xn of the token before stays in registers.  The first token of a run needs the xn of the one before it, which is
+// computed again: with runs of 8 tokens an eighth of the reads of x, which come from L2.
+//
+// Backward, for cotangents g_i of the outputs, gx of xs and gshift of the shift row:
+//     dxn_t = sum_i g_i,t (1 - mix_i) + (t+1 < T and not new_starts[t+1]) sum_i g_i,t+1 mix_i (+ gshift_t)
+//     dxs   = rstd (dxn w - mean(dxn w) - xhat mean(dxn w xhat)) + gx         (the cotangent of x and of dx)
+//     dmix_i = sum g_i (xn_prev - xn), dln_w = sum dxn xhat, dln_b = sum dxn,  dprev = not new_starts[0] ? sum_i g_i,0 mix_i : 0
+// The runs are walked downwards, sums over tokens stay in registers and every workgroup writes them once to a workspace;
+// a second small kernel adds the workgroups' rows and rounds to the parameters' type.  (One fp32 atomic per channel and
+// workgroup instead, with the zero fills and casts around it, is what the separate shift kernel does: its time is set by
+// the atomics from 512 workgroups on.)
+#include "common.h"
+#include "wkv_args.h"
+
+namespace hiprwkv {
+
+namespace {
+
+constexpr int MAX_WAVES = 8;           // 512 threads: C <= 4096, and 256 registers per thread (with 16 waves the kernels spill)
+constexpr int FWD_GROUP = 4;           // tokens whose loads are in flight together, forward
+// The same, backward: with six cotangents one token is eight 16-byte loads per thread, and two spill.
+template <int NOUT>
+constexpr int BWD_GROUP_OF = NOUT == 6 ? 1 : 2;
+
+// sum over the 16 lanes of a DPP row, delivered to all of them
+__device__ __forceinline__ float row_sum(float x) {
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x128, 0xf, 0xf, false));   // row_ror:8
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x124, 0xf, 0xf, false));   // row_ror:4
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x122, 0xf, 0xf, false));   // row_ror:2
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x121, 0xf, 0xf, false));   // row_ror:1
+  return x;
+}
+
+// G sums over the workgroup at once.  `buf` is not read by anyone when a thread gets here (callers alternate two).
+template <int G>
+__device__ __forceinline__ void block_sum(float (&x)[G], float* buf) {
+  const int row = threadIdx.x >> 4, nrow = blockDim.x >> 4;
+#pragma unroll
+  for (int j = 0; j < G; ++j) x[j] = row_sum(x[j]);
+  if ((threadIdx.x & 15) == 0) {
+#pragma unroll
+    for (int j = 0; j < G; ++j) buf[row * G + j] = x[j];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < G; ++j) x[j] = 0.f;
+  for (int r = 0; r < nrow; r += 4)            // blockDim.x is a multiple of 64
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int j = 0; j < G; ++j) x[j] += buf[(r + q) * G + j];
+}
+
+template <typename T>
+__device__ __forceinline__ float round_io(float x);
+template <>
+__device__ __forceinline__ float round_io<float>(float x) { return x; }
+template <>
+__device__ __forceinline__ float round_io<bf16_t>(float x) { return bf16_to_f32(f32_to_bf16(x)); }
+
+template <typename T>
+__device__ __forceinline__ void zero_or_ld8(const T* p, bool take, float (&o)[8]) {
+  if (take) {
+    ld8(p, o);
+  } else {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) o[c] = 0.f;
+  }
+}
+
+// Eight values kept as they lie in memory: in bf16 half the registers of eight floats
+template <typename T>
+struct Held;
+template <>
+struct Held<float> {
+  float v[8];
+  __device__ __forceinline__ void load(const float* p) { ld8(p, v); }
+  __device__ __forceinline__ void pin() {}
+  __device__ __forceinline__ float operator[](int c) const { return v[c]; }
+};
+template <>
+struct Held<bf16_t> {
+  uint32_t v[4];
+  __device__ __forceinline__ void load(const bf16_t* p) {
+    const uint4 a = *reinterpret_cast<const uint4*>(p);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+  }
+  // in a loop: keeps the compiler from unpacking once in front of it
+  __device__ __forceinline__ void pin() { asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3])); }
+  __device__ __forceinline__ float operator[](int c) const {
+    return __uint_as_float((c & 1) ? (v[c >> 1] & 0xffff0000u) : (v[c >> 1] << 16));
+  }
+};
+
+// in-sequence index of the token whose xn the state keeps: x[length - 1] with the wrap-around of negative indices
+__device__ __forceinline__ int64_t last_token(const int32_t* length, int64_t b, int64_t T) {
+  if (length == nullptr) return T - 1;
+  int64_t L = length[b];
+  L = (L < 0 ? 0 : L) - 1;
+  return L < 0 ? T - 1 : L % T;
+}
+
+template <typename T, int NOUT>
+__global__ __launch_bounds__(64 * MAX_WAVES) void ln_shiftmix_kernel(LnMixArgs A) {
+  __shared__ float buf[2][FWD_GROUP * MAX_WAVES * 4];
+  const int64_t C = A.C, Tn = A.T, total = A.B * A.T;
+  const int c8 = threadIdx.x * 8;
+  const bool on = c8 < C;
+  const int cc = on ? c8 : 0;
+  const float invC = 1.f / (float)C;
+  Held<T> w, bias, m[NOUT ? NOUT : 1];
+  w.load(reinterpret_cast<const T*>(A.ln_w) + cc);
+  bias.load(reinterpret_cast<const T*>(A.ln_b) + cc);
+#pragma unroll
+  for (int i = 0; i < NOUT; ++i) m[i].load(reinterpret_cast<const T*>(A.mix[i]) + cc);
+  const int64_t n0 = (int64_t)blockIdx.x * A.run;
+  const int64_t n1 = n0 + A.run < total ? n0 + A.run : total;
+  // the token before the run, unless the run starts a sequence
+  const int64_t first = (NOUT != 0 && n0 % Tn != 0) ? n0 - 1 : n0;
+  float before[8];                             // xn of the last token handled
+#pragma unroll
+  for (int c = 0; c < 8; ++c) before[c] = 0.f;
+  for (int64_t g0 = first; g0 < n1; g0 += FWD_GROUP) {
+    w.pin(); bias.pin();
+#pragma unroll
+    for (int i = 0; i < NOUT; ++i) m[i].pin();
+    float x[FWD_GROUP][8], s[FWD_GROUP];
+#pragma unroll
+    for (int j = 0; j < FWD_GROUP; ++j) {
+      const int64_t n = g0 + j < n1 ? g0 + j : n1 - 1;
+      zero_or_ld8(reinterpret_cast<const T*>(A.x) + n * C + cc, on, x[j]);
+    }
+    if (A.dx != nullptr) {
+#pragma unroll
+      for (int j = 0; j < FWD_GROUP; ++j) {
+        const int64_t n = g0 + j < n1 ? g0 + j : n1 - 1;
+        float d[8];
+        zero_or_ld8(reinterpret_cast<const T*>(A.dx) + n * C + cc, on, d);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) x[j][c] = round_io<T>(x[j][c] + d[c]);
+        if (on && g0 + j >= n0 && g0 + j < n1) st8(reinterpret_cast<T*>(A.xs) + n * C + cc, x[j]);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < FWD_GROUP; ++j) {
+      s[j] = 0.f;
+#pragma unroll
+      for (int c = 0; c < 8; ++c) s[j] += x[j][c];
+    }
+    block_sum(s, buf[0]);
+    float q[FWD_GROUP];
+#pragma unroll
+    for (int j = 0; j < FWD_GROUP; ++j) {
+      s[j] *= invC;
+      q[j] = 0.f;
+#pragma unroll
+      for (int c = 0; c < 8; ++c) { const float d = x[j][c] - s[j]; q[j] = fmaf(d, d, q[j]); }
+      if (!on) q[j] = 0.f;
+    }
+    block_sum(q, buf[1]);
+#pragma unroll
+    for (int j = 0; j < FWD_GROUP; ++j) {
+      const int64_t n = g0 + j;
+      if (n >= n1) break;
+      const float rstd = rsqrtf(q[j] * invC + A.eps);
+      float xn[8];
+#pragma unroll
+      for (int c = 0; c < 8; ++c) xn[c] = round_io<T>(fmaf((x[j][c] - s[j]) * rstd, w[c], bias[c]));
+      if (n >= n0) {
+        if (A.stats != nullptr && threadIdx.x == 0) *reinterpret_cast<float2*>(A.stats + 2 * n) = make_float2(s[j], rstd);
+        if (on) {
+          if (NOUT == 0) {
+            st8(reinterpret_cast<T*>(A.out[0]) + n * C + c8, xn);
+          } else {
+            const int64_t b = n / Tn, t = n - b * Tn;
+            if (A.shift != nullptr && t == last_token(A.length, b, Tn)) st8(reinterpret_cast<T*>(A.shift) + b * A.shift_bstride + c8, xn);
+            const bool reset = A.ns != nullptr && A.ns[n] != 0;
+            float pv[8];
+            if (t == 0) ld8(reinterpret_cast<const T*>(A.prev) + b * A.prev_bstride + c8, pv);
+#pragma unroll
+            for (int c = 0; c < 8; ++c) pv[c] = reset ? 0.f : (t == 0 ? pv[c] : before[c]);
+#pragma unroll
+            for (int i = 0; i < NOUT; ++i) {
+              float o[8];
+#pragma unroll
+              for (int c = 0; c < 8; ++c) o[c] = fmaf(pv[c] - xn[c], m[i][c], xn[c]);
+              st8(reinterpret_cast<T*>(A.out[i]) + n * C + c8, o);
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < 8; ++c) before[c] = xn[c];
+    }
+  }
+}
+
+template <typename T, int NOUT>
+__global__ __launch_bounds__(64 * MAX_WAVES) void ln_shiftmix_bwd_kernel(LnMixArgs A) {
+  constexpr int NG = NOUT ? NOUT : 1;          // cotangent tensors
+  constexpr int BWD_GROUP = BWD_GROUP_OF<NOUT>;
+  constexpr int NP = NOUT + 2;                 // parameter cotangents: mix_0.., ln_w, ln_b
+  __shared__ float buf[2][2 * BWD_GROUP * MAX_WAVES * 4];
+  const int64_t C = A.C, Tn = A.T, total = A.B * A.T;
+  const int c8 = threadIdx.x * 8;
+  const bool on = c8 < C;
+  const int cc = on ? c8 : 0;
+  const float invC = 1.f / (float)C;
+  float acc[NP][8];
+  Held<T> w, bias, m[NG];
+  w.load(reinterpret_cast<const T*>(A.ln_w) + cc);
+  bias.load(reinterpret_cast<const T*>(A.ln_b) + cc);
+#pragma unroll
+  for (int i = 0; i < NOUT; ++i) m[i].load(reinterpret_cast<const T*>(A.mix[i]) + cc);
+#pragma unroll
+  for (int i = 0; i < NP; ++i)
+#pragma unroll
+    for (int c = 0; c < 8; ++c) acc[i][c] = 0.f;
+  const int64_t n0 = (int64_t)blockIdx.x * A.run;
+  const int64_t n1 = (n0 + A.run < total ? n0 + A.run : total) - 1;      // last token of the run
+  // sum_i g_i mix_i of the token after, if that token takes its shifted value from the one before it
+  float gm_next[8];
+#pragma unroll
+  for (int c = 0; c < 8; ++c) gm_next[c] = 0.f;
+  if (NOUT != 0 && n1 + 1 < total && (n1 + 1) % Tn != 0 && !(A.ns != nullptr && A.ns[n1 + 1] != 0)) {
+#pragma unroll
+    for (int i = 0; i < NOUT; ++i) {
+      float g[8];
+      zero_or_ld8(reinterpret_cast<const T*>(A.g[i]) + (n1 + 1) * C + cc, on, g);
+#pragma unroll
+      for (int c = 0; c < 8; ++c) gm_next[c] = fmaf(g[c], m[i][c], gm_next[c]);
+    }
+  }
+  int ph = 0;
+  for (int64_t top = n1; top >= n0; top -= BWD_GROUP, ph ^= 1) {
+    w.pin(); bias.pin();
+#pragma unroll
+    for (int i = 0; i < NOUT; ++i) m[i].pin();
+    float gx[BWD_GROUP][8], xh[BWD_GROUP][8], rstd[BWD_GROUP], red[2 * BWD_GROUP];
+    // xs of the group's tokens and of the one before the group
+    float xs[BWD_GROUP + 1][8];
+    float2 st[BWD_GROUP + 1];
+#pragma unroll
+    for (int j = 0; j <= BWD_GROUP; ++j) {
+      int64_t n = top - j;
+      n = n < 0 ? 0 : n;
+      if (NOUT != 0 || j < BWD_GROUP) {
+        zero_or_ld8(reinterpret_cast<const T*>(A.xs) + n * C + cc, on, xs[j]);
+        st[j] = *reinterpret_cast<const float2*>(A.stats + 2 * n);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < BWD_GROUP; ++j) {
+      const int64_t n = top - j;
+      const bool live = n >= n0;
+      const int64_t nn = live ? n : n0;
+      const int64_t b = nn / Tn, t = nn - b * Tn;
+      rstd[j] = st[j].y;
+      float dxn[8];
+#pragma unroll
+      for (int c = 0; c < 8; ++c) xh[j][c] = (xs[j][c] - st[j].x) * st[j].y;
+      if (NOUT == 0) {
+        zero_or_ld8(reinterpret_cast<const T*>(A.g[0]) + nn * C + cc, on && live, dxn);
+      } else {
+        const bool reset = A.ns != nullptr && A.ns[nn] != 0;
+        float pv[8], d[8];
+        if (t == 0) ld8(reinterpret_cast<const T*>(A.prev) + b * A.prev_bstride + cc, pv);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+          const float xn = round_io<T>(fmaf(xh[j][c], w[c], bias[c]));
+          const float xb = round_io<T>(fmaf((xs[j + 1][c] - st[j + 1].x) * st[j + 1].y, w[c], bias[c]));
+          d[c] = (reset ? 0.f : (t == 0 ? pv[c] : xb)) - xn;
+        }
+        float gm[8];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) { gm[c] = 0.f; dxn[c] = 0.f; }
+#pragma unroll
+        for (int i = 0; i < NOUT; ++i) {
+          float g[8];
+          zero_or_ld8(reinterpret_cast<const T*>(A.g[i]) + nn * C + cc, on && live, g);
+#pragma unroll
+          for (int c = 0; c < 8; ++c) {
+            dxn[c] += g[c];
+            gm[c] = fmaf(g[c], m[i][c], gm[c]);
+            acc[i][c] = fmaf(g[c], d[c], acc[i][c]);
+          }
+        }
+        if (live) {
+          const bool last_of_seq = t == Tn - 1;
+#pragma unroll
+          for (int c = 0; c < 8; ++c) dxn[c] += (last_of_seq ? 0.f : gm_next[c]) - gm[c];
+          if (A.gshift != nullptr && t == last_token(A.length, b, Tn)) {
+            float gs[8];
+            zero_or_ld8(reinterpret_cast<const T*>(A.gshift) + b * C + cc, on, gs);
+#pragma unroll
+            for (int c = 0; c < 8; ++c) dxn[c] += gs[c];
+          }
+#pragma unroll
+          for (int c = 0; c < 8; ++c) gm_next[c] = reset ? 0.f : gm[c];
+          if (t == 0 && on && A.dprev != nullptr) st8(reinterpret_cast<T*>(A.dprev) + b * C + c8, gm_next);
+        }
+      }
+      red[2 * j] = red[2 * j + 1] = 0.f;
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        acc[NOUT][c] = fmaf(dxn[c], xh[j][c], acc[NOUT][c]);
+        acc[NOUT + 1][c] += dxn[c];
+        gx[j][c] = dxn[c] * w[c];
+        red[2 * j] += gx[j][c];
+        red[2 * j + 1] = fmaf(gx[j][c], xh[j][c], red[2 * j + 1]);
+      }
+    }
+    block_sum(red, buf[ph]);
+#pragma unroll
+    for (int j = 0; j < BWD_GROUP; ++j) {
+      const int64_t n = top - j;
+      if (n < n0 || !on) break;
+      const float s1 = red[2 * j] * invC, s2 = red[2 * j + 1] * invC;
+      float o[8];
+      zero_or_ld8(reinterpret_cast<const T*>(A.gx) + n * C + c8, A.gx != nullptr, o);
+#pragma unroll
+      for (int c = 0; c < 8; ++c) o[c] += rstd[j] * (gx[j][c] - s1 - xh[j][c] * s2);
+      st8(reinterpret_cast<T*>(A.dxs) + n * C + c8, o);
+    }
+  }
+  if (on) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) st8(A.part + ((size_t)blockIdx.x * NP + i) * C + c8, acc[i]);
+  }
+}
+
+// out_k[c] = sum over p of part[p][k][c]; a workgroup owns 64 consecutive of the nk*C columns, its four waves a quarter
+// of the rows each
+template <typename T>
+__global__ __launch_bounds__(256) void reduce_parts_kernel(ReduceArgs A) {
+  __shared__ float red[4][64];
+  const int64_t cols = (int64_t)A.nk * A.C;
+  const int64_t col = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
+  const int wv = threadIdx.x >> 6;
+  float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
+  if (col < cols) {
+    const float* p = A.part + col;
+    int64_t r = wv;
+    for (; r + 12 < A.rows; r += 16) {
+      s0 += p[r * cols]; s1 += p[(r + 4) * cols]; s2 += p[(r + 8) * cols]; s3 += p[(r + 12) * cols];
+    }
+    for (; r < A.rows; r += 4) s0 += p[r * cols];
+  }
+  red[wv][threadIdx.x & 63] = (s0 + s1) + (s2 + s3);
+  __syncthreads();
+  if (wv == 0 && col < cols) {
+    const float s = (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
+    st_f(reinterpret_cast<T*>(A.out[col / A.C]) + col % A.C, s);
+  }
+}
+
+}  // namespace
+
+hipError_t launch_reduce_parts(int io_f32, const ReduceArgs& A, hipStream_t stream) {
+  const dim3 grid((unsigned)(((int64_t)A.nk * A.C + 63) / 64)), block(256);
+  if (io_f32) hipLaunchKernelGGL(reduce_parts_kernel<float>, grid, block, 0, stream, A);
+  else hipLaunchKernelGGL(reduce_parts_kernel<bf16_t>, grid, block, 0, stream, A);
+  return hipGetLastError();
+}
+
+// Tokens per workgroup.  Forward: 8 keep the re-reading of the token before a run at an eighth; shorter runs while that
+// leaves fewer than 1024 workgroups.
+int64_t ln_shiftmix_run(int64_t rows) {
+  const int64_t run = rows / 1024;
+  return run < 1 ? 1 : run > 8 ? 8 : run;
+}
+// Backward: a workgroup writes NP rows of C sums, so runs grow with the token count (at most about 1024 workgroups).
+int64_t ln_shiftmix_bwd_run(int64_t rows) {
+  const int64_t run = (rows + 1023) / 1024;
+  return run < 4 ? 4 : (run + 1) / 2 * 2;
+}
+
+#define HIPRWKV_BLOCK_DISPATCH(KERNEL)                                                                       \
+  if (io_f32) {                                                                                              \
+    if (n_out == 6) hipLaunchKernelGGL((KERNEL<float, 6>), grid, block, 0, stream, A);                       \
+    else if (n_out == 1) hipLaunchKernelGGL((KERNEL<float, 1>), grid, block, 0, stream, A);                  \
+    else hipLaunchKernelGGL((KERNEL<float, 0>), grid, block, 0, stream, A);                                  \
+  } else {                                                                                                   \
+    if (n_out == 6) hipLaunchKernelGGL((KERNEL<bf16_t, 6>), grid, block, 0, stream, A);                      \
+    else if (n_out == 1) hipLaunchKernelGGL((KERNEL<bf16_t, 1>), grid, block, 0, stream, A);                 \
+    else hipLaunchKernelGGL((KERNEL<bf16_t, 0>), grid, block, 0, stream, A);                                 \
+  }
+
+hipError_t launch_ln_shiftmix(int io_f32, int n_out, LnMixArgs A, hipStream_t stream) {
+  A.run = ln_shiftmix_run(A.B * A.T);
+  const dim3 grid((unsigned)((A.B * A.T + A.run - 1) / A.run)), block((unsigned)((A.C / 8 + 63) / 64 * 64));
+  HIPRWKV_BLOCK_DISPATCH(ln_shiftmix_kernel)
+  return hipGetLastError();
+}
+
+hipError_t launch_ln_shiftmix_bwd(int io_f32, int n_out, LnMixArgs A, void* const* dparam, hipStream_t stream) {
+  A.run = ln_shiftmix_bwd_run(A.B * A.T);
+  const dim3 grid((unsigned)((A.B * A.T + A.run - 1) / A.run)), block((unsigned)((A.C / 8 + 63) / 64 * 64));
+  HIPRWKV_BLOCK_DISPATCH(ln_shiftmix_bwd_kernel)
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  ReduceArgs R;
+  R.part = A.part; R.rows = grid.x; R.nk = n_out + 2; R.C = A.C;
+  for (int i = 0; i < n_out + 2; ++i) R.out[i] = dparam[i];
+  return launch_reduce_parts(io_f32, R, stream);
+}
+
+}  // namespace hiprwkv

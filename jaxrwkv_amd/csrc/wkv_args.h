@@ -78,6 +78,54 @@ struct Wkv4Args {
   float* ckpt;      // workspace: (B, ceil(T/16), 3, C) states entering every 16th step (forward: optional output)
 };
 
+// Residual addition + LayerNorm + token shift and interpolation (rwkv7_block.hip); tensors in the I/O dtype
+struct LnMixArgs {
+  int64_t B, T, C, run;
+  const void *x, *dx;            // (B,T,C); dx may be null (then xs is x itself and is not written)
+  const void *ln_w, *ln_b;       // (C,)
+  float eps;
+  const void* prev;              // (B,C) rows, prev_bstride elements apart: the token before t = 0
+  int64_t prev_bstride;
+  const uint8_t* ns;
+  const int32_t* length;         // (B,) or null: which token's norm goes to `shift`
+  const void* mix[6];            // (C,) each
+  void* out[6];
+  void* xs;                      // forward: x + dx out; backward: the same array in
+  void* shift;                   // (B,C) rows, shift_bstride elements apart; may be null
+  int64_t shift_bstride;
+  float* stats;                  // (B*T, 2) mean and 1/std; forward: may be null
+  // backward
+  const void* g[6];
+  const void *gx, *gshift;       // cotangents of xs and of the shift row (B,C), each may be null
+  void *dxs, *dprev;             // dprev (B,C) may be null
+  float* part;                   // workspace (workgroups, n_out + 2, C)
+};
+struct ReduceArgs {
+  const float* part;             // (rows, nk, C)
+  int64_t rows, C;
+  int nk;
+  void* out[8];                  // nk arrays (C,)
+};
+hipError_t launch_reduce_parts(int io_f32, const ReduceArgs& A, hipStream_t stream);
+int64_t ln_shiftmix_bwd_run(int64_t rows);
+hipError_t launch_ln_shiftmix(int io_f32, int n_out, LnMixArgs A, hipStream_t stream);
+hipError_t launch_ln_shiftmix_bwd(int io_f32, int n_out, LnMixArgs A, void* const* dparam, hipStream_t stream);
+
+// Element-wise work between the projections and the WKV op (rwkv7_pre.hip); token tensors (rows, H, 64), parameters (H, 64)
+struct PreArgs {
+  int64_t rows, H;
+  const void *xw, *k, *xa, *v, *vf, *xv;       // vf null: no value residual (v, vf, xv, v0, v_out and dv, dvf, dxv unused)
+  const void *w0, *a0, *v0, *k_k, *k_a;
+  void *w, *k_out, *v_out, *a_out, *b_out;
+  // backward
+  const void *gw, *gk, *gv, *ga, *gb;          // cotangents of w, k_out, v_out, a_out, b_out
+  void *dxw, *dk, *dv, *dvf, *dxv, *dxa;
+  float* part;                                 // workspace (rwkv7_pre_bwd_rows, 4 or 5, H*64)
+};
+int64_t rwkv7_pre_bwd_rows(int64_t rows, int64_t H);
+hipError_t launch_rwkv7_pre(int io_f32, const PreArgs& A, hipStream_t stream);
+hipError_t launch_rwkv7_pre_bwd(int io_f32, const PreArgs& A, void* const* dparam, hipStream_t stream);
+
 // Raises a kernel's dynamic-LDS limit once per kernel and device instead of at every enqueue (the attribute call
 // goes to the driver; hipGetDevice does not).
 struct LdsAttrOnce {

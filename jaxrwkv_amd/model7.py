@@ -2,9 +2,9 @@
 
 It mirrors the reference's ``RWKV.forward(params, tokens, state, length=, new_starts=)`` and ``default_state``
 (/root/reference/src/jaxrwkv/llm.py:71-84, rwkv7.py:176-198, 223-291) with an explicit leading batch axis (the
-reference batches with ``jax.vmap``).  Everything except the recurrence is plain torch (projections, LayerNorm,
-token shift, LoRA gates, group norm, channel mix): plumbing that stays in the host framework; the recurrence goes
-through ``HipRWKV.inner_loop``.  The parameter tree has the reference's names and stacked-per-layer shapes
+reference batches with ``jax.vmap``).  Projections are torch's; the element-wise work between them (residual addition and
+LayerNorm, token shift, gates, group norm) runs on fused kernels of this library, and the recurrence goes through
+``HipRWKV.inner_loop``.  The parameter tree has the reference's names and stacked-per-layer shapes
 (rwkv7.py:81-173) so that a converted checkpoint would drop in; ``randomize_weights`` follows the same schedules and
 distributions with torch's generator (the reference's threefry streams cannot be reproduced without jax).
 
@@ -120,8 +120,8 @@ class RWKV7:
     """``forward`` / ``default_state`` with the reference's argument names; batched over the leading axis."""
 
     inner = HipRWKV
-    #: use the fused kernels beside the recurrence (ops.rwkv7_shiftmix, rwkv7_decay, rwkv7_vmix, rwkv7_agate,
-    #: rwkv7_premix, rwkv7_postmix), with or without autograd
+    #: use the fused kernels beside the recurrence (ops.rwkv7_ln_shiftmix, rwkv7_pre, rwkv7_postmix, rwkv7_relusq), with or
+    #: without autograd; models wider than ops.LN_SHIFTMIX_MAX_C channels run the separate steps
     fuse_mix = True
 
     @classmethod
@@ -132,82 +132,80 @@ class RWKV7:
         return torch.zeros((batch, L, 2 + N, emb.shape[1]), dtype=emb.dtype, device=emb.device)
 
     @classmethod
-    def _shift(cls, x, prev, new_starts):
-        """Token shift of rwkv7.py:227-229 / 192-194: previous token (state row for t = 0), zero at new_starts."""
-        sx = torch.cat([prev[:, None], x[:, :-1]], dim=1)
-        sx = torch.where(new_starts[:, :, None], torch.zeros_like(sx), sx)
-        return sx - x
+    def _mix_head(cls, x, dx, ln, prev, new_starts, length, mix, fused, shift_out=None):
+        """Residual addition, LayerNorm, token shift of rwkv7.py:227-229 / 192-194 (previous token, the state row for
+        t = 0, zero at new_starts) and interpolation; returns (x + dx, new shift row, interpolations)."""
+        if fused:
+            return ops.rwkv7_ln_shiftmix(x, dx, ln, prev, new_starts, length, mix, shift_out=shift_out)
+        B, T, C = x.shape
+        if dx is not None:
+            x = x + dx
+        xn = layer_norm(x, ln)
+        sx = torch.cat([prev[:, None], xn[:, :-1]], dim=1)
+        if new_starts is not None:
+            sx = torch.where(new_starts[:, :, None], torch.zeros_like(sx), sx)
+        sx = sx - xn
+        # xn[length - 1] with the wrap-around of negative indices
+        last = (length.long() - 1) % T if length is not None else torch.full((B,), T - 1, device=x.device)
+        return x, xn[torch.arange(B, device=x.device), last], [xn + sx * m for m in mix]
 
     @classmethod
-    def channel_mixing_seq(cls, x, state_row, ffn, last_idx, new_starts):
-        """rwkv7.py:190-198"""
-        if cls.fuse_mix:
-            xk, = ops.rwkv7_shiftmix(x, state_row, new_starts, [ffn["x_k"]])
-        else:
-            xk = x + cls._shift(x, state_row, new_starts) * ffn["x_k"]
+    def channel_mixing_seq(cls, x, dx, ln, state_row, ffn, length, new_starts, fused, shift_out=None):
+        """rwkv7.py:190-198 with the residual addition and the norm in front; returns (x + dx, output, new shift row)."""
+        x, shift, (xk,) = cls._mix_head(x, dx, ln, state_row, new_starts, length, [ffn["x_k"]], fused, shift_out)
         k = xk @ ffn["key"]["weight"].T
-        k = ops.rwkv7_relusq(k) if cls.fuse_mix else torch.square(torch.relu(k))
-        return k @ ffn["value"]["weight"].T, x[torch.arange(x.shape[0], device=x.device), last_idx]
+        k = ops.rwkv7_relusq(k) if fused else torch.square(torch.relu(k))
+        return x, k @ ffn["value"]["weight"].T, shift
 
     @classmethod
-    def time_mixing_seq(cls, x, shift_row, wkv_state, v_first, att, length, last_idx, new_starts, layer_id,
-                        wkv_out=None):
-        """rwkv7.py:223-267.  wkv_state (B, N, C) is the layer's rows 2.. of the model state.  With ``wkv_out`` (the
-        same rows of the new model state; decode steps without autograd) the recurrence reads and writes the two views
-        in place and the third result is None."""
+    def time_mixing_seq(cls, x, dx, ln, shift_row, wkv_state, v_first, att, length, new_starts, layer_id, fused,
+                        shift_out=None, wkv_out=None):
+        """rwkv7.py:223-267 with the residual addition and the norm in front.  wkv_state (B, N, C) is the layer's rows 2..
+        of the model state.  With ``wkv_out`` (the same rows of the new model state; decode steps without autograd) the
+        recurrence reads and writes the two views in place and the new state is returned as None.
+        Returns (x + dx, output, new shift row, new wkv state, v_first)."""
         B, T, C = x.shape
         H, N = att["r_k"].shape
-        mix_names = ("x_r", "x_w", "x_k", "x_v", "x_a", "x_g")
-        if cls.fuse_mix:
-            xr, xw, xk, xv, xa, xg = ops.rwkv7_shiftmix(x, shift_row, new_starts, [att[n] for n in mix_names])
-        else:
-            sx = cls._shift(x, shift_row, new_starts)
-            xr, xw, xk, xv, xa, xg = (x + sx * att[n] for n in mix_names)
-        r = xr @ att["receptance"]["weight"].T
-        w_lora = torch.tanh(xw @ att["w1"]) @ att["w2"]
-        if cls.fuse_mix:
-            w = ops.rwkv7_decay(w_lora, att["w0"])
-        else:
-            w = -F.softplus(-(att["w0"] + w_lora).float()).to(x.dtype) - 0.5
-        k = xk @ att["key"]["weight"].T
-        v = xv @ att["value"]["weight"].T
+        mix = [att[n] for n in ("x_r", "x_w", "x_k", "x_v", "x_a", "x_g")]
+        x, shift, (xr, xw, xk, xv, xa, xg) = cls._mix_head(x, dx, ln, shift_row, new_starts, length, mix, fused, shift_out)
+        heads = lambda t: t.reshape(B, T, H, N)
+        r = heads(xr @ att["receptance"]["weight"].T)
+        k = heads(xk @ att["key"]["weight"].T)
+        v = heads(xv @ att["value"]["weight"].T)
+        w_lora = heads(torch.tanh(xw @ att["w1"]) @ att["w2"])
+        a_lora = heads((xa @ att["a1"]) @ att["a2"])
+        v_lora = heads((xv @ att["v1"]) @ att["v2"]) if layer_id != 0 else None
+        g = heads(torch.sigmoid(xg @ att["g1"]) @ att["g2"])
         if layer_id == 0:
             v_first = v
-        else:
-            v_lora = (xv @ att["v1"]) @ att["v2"]
-            if cls.fuse_mix:
-                v = ops.rwkv7_vmix(v, v_first, v_lora, att["v0"])
-            else:
-                v = v + (v_first - v) * torch.sigmoid(att["v0"] + v_lora)
-        a_lora = (xa @ att["a1"]) @ att["a2"]
-        a = ops.rwkv7_agate(a_lora, att["a0"]) if cls.fuse_mix else torch.sigmoid(att["a0"] + a_lora)
-        g = torch.sigmoid(xg @ att["g1"]) @ att["g2"]
-        new_shift = x[torch.arange(B, device=x.device), last_idx]
-        fused = cls.fuse_mix
-        rh, wh, vh = (t.reshape(B, T, H, N) for t in (r, w, v))
         if fused:
-            kh, ah, bh = ops.rwkv7_premix(k.reshape(B, T, H, N), a.reshape(B, T, H, N), att["k_k"], att["k_a"])
+            w, k, v, a, b = ops.rwkv7_pre(w_lora, k, a_lora, v, None if layer_id == 0 else v_first, v_lora, att["w0"],
+                                          att["a0"], att["v0"], att["k_k"], att["k_a"])
         else:
-            kk = (k * att["k_k"]).reshape(B, T, H, N)
-            kk = (kk / torch.clamp(torch.linalg.vector_norm(kk.float(), dim=-1, keepdim=True), min=1e-12).to(kk.dtype))
-            kk = kk.reshape(B, T, C)
-            k = k * (1 + (a - 1) * att["k_a"])
-            kh, ah, bh = (t.reshape(B, T, H, N) for t in (k, -kk, kk * a))
+            par = lambda n: att[n].reshape(H, N)
+            w = -F.softplus(-(par("w0") + w_lora).float()).to(x.dtype) - 0.5
+            if layer_id != 0:
+                v = v + (v_first - v) * torch.sigmoid(par("v0") + v_lora)
+            a = torch.sigmoid(par("a0") + a_lora)
+            kk = k * par("k_k")
+            kk = kk / torch.clamp(torch.linalg.vector_norm(kk.float(), dim=-1, keepdim=True), min=1e-12).to(kk.dtype)
+            k = k * (1 + (a - 1) * par("k_a"))
+            a, b = -kk, kk * a
         if wkv_out is not None:
-            s_new, out = None, cls.inner.step_packed(rh, wh, kh, vh, ah, bh, wkv_state, wkv_out, length, new_starts)
+            s_new, out = None, cls.inner.step_packed(r, w, k, v, a, b, wkv_state, wkv_out, length, new_starts)
         else:
-            s_new, out = cls.inner.inner_loop(rh, wh, kh, vh, ah, bh, wkv_state.reshape(B, H, N, N), length, new_starts)
+            s_new, out = cls.inner.inner_loop(r, w, k, v, a, b, wkv_state.reshape(B, H, N, N), length, new_starts)
             s_new = s_new.reshape(B, N, C)
         if fused:
-            y = ops.rwkv7_postmix(out, rh, kh, vh, g.reshape(B, T, H, N), att["ln_x"]["weight"], att["ln_x"]["bias"],
-                                  att["r_k"], 64e-5).reshape(B, T, C)
+            y = ops.rwkv7_postmix(out, r, k, v, g, att["ln_x"]["weight"], att["ln_x"]["bias"], att["r_k"], 64e-5)
+            y = y.reshape(B, T, C)
         else:
-            y = out.reshape(B * T, H, N).float()
-            y = F.group_norm(y.reshape(B * T, C), H, att["ln_x"]["weight"].float(), att["ln_x"]["bias"].float(), 64e-5)
+            y = out.reshape(B * T, C).float()
+            y = F.group_norm(y, H, att["ln_x"]["weight"].float(), att["ln_x"]["bias"].float(), 64e-5)
             y = y.to(x.dtype).reshape(B, T, C)
-            bonus = ((rh * kh * att["r_k"]).sum(-1, keepdim=True) * vh).reshape(B, T, C)
-            y = (y + bonus) * g
-        return y @ att["output"]["weight"].T, new_shift, s_new, v_first
+            bonus = ((r * k * att["r_k"]).sum(-1, keepdim=True) * v).reshape(B, T, C)
+            y = (y + bonus) * g.reshape(B, T, C)
+        return x, y @ att["output"]["weight"].T, shift, s_new, v_first
 
     @classmethod
     def forward(cls, params, tokens, state, length=None, new_starts=None):
@@ -215,36 +213,39 @@ class RWKV7:
         Returns (logits (B,T,vocab), new state).  llm.py:71-84 + rwkv7.py:269-291."""
         B, T = tokens.shape
         dev = tokens.device
-        if length is None:
-            length = torch.full((B,), T, dtype=torch.int32, device=dev)
-        length = torch.as_tensor(length, device=dev).to(torch.int32).reshape(-1).expand(B)
-        if new_starts is None:
-            new_starts = torch.zeros((B, T), dtype=torch.bool, device=dev)
-        last_idx = (length.long() - 1) % T          # x[length - 1] with the wrap-around of negative indices
-        x = params["emb"]["weight"][tokens]
-        x = layer_norm(x, params["ln0"])
-        L = params["blocks"]["att"]["r_k"].shape[0]
+        if length is not None:
+            length = torch.as_tensor(length, device=dev).to(torch.int32).reshape(-1).expand(B).contiguous()
+        if new_starts is not None:
+            new_starts = torch.as_tensor(new_starts, device=dev).to(torch.bool).expand(B, T).contiguous()
+        L, H, N = params["blocks"]["att"]["r_k"].shape
+        C = H * N
+        fused = cls.fuse_mix and C <= ops.LN_SHIFTMIX_MAX_C
+        norm = (lambda x, dx, ln: ops.rwkv7_ln_shiftmix(x, dx, ln, None, None, None, [])[2][0]) if fused else \
+               (lambda x, dx, ln: layer_norm(x if dx is None else x + dx, ln))
+        x = norm(params["emb"]["weight"][tokens], None, params["ln0"])
         blocks = unstack(params["blocks"], L)
-        # decode steps: the recurrence works on the layers' rows of the two model states directly (no copies of them)
-        packed = (T <= 8 and hasattr(cls.inner, "step_packed")
-                  and not (torch.is_grad_enabled() and (x.requires_grad or state.requires_grad)))
-        new_state = torch.empty_like(state) if packed else None
-        rows = []                                   # the new state's parts in memory order, joined once at the end
-        v_first = x
+        grad = torch.is_grad_enabled() and (x.requires_grad or state.requires_grad)
+        # without autograd the layers write their rows of the new state where they belong; decode steps read and write the
+        # recurrence's rows in place as well
+        in_place = fused and not grad and state.dtype == x.dtype and (C * x.element_size()) % 16 == 0
+        packed = T <= 8 and hasattr(cls.inner, "step_packed") and not grad
+        new_state = torch.empty_like(state) if (in_place or packed) else None
+        rows = []                                   # otherwise: the new state's parts in memory order, joined at the end
+        v_first, dx = None, None
         for i, blk in enumerate(blocks):
-            st = state[:, i]
-            dx, shift1, wkv, v_first = cls.time_mixing_seq(layer_norm(x, blk["ln1"]), st[:, 1], st[:, 2:], v_first,
-                                                           blk["att"], length, last_idx, new_starts, i,
-                                                           new_state[:, i, 2:] if packed else None)
-            x = x + dx
-            dx, shift0 = cls.channel_mixing_seq(layer_norm(x, blk["ln2"]), st[:, 0], blk["ffn"], last_idx, new_starts)
-            x = x + dx
-            if packed:
-                new_state[:, i, 0] = shift0
-                new_state[:, i, 1] = shift1
-            else:
+            st, nst = state[:, i], (None if new_state is None else new_state[:, i])
+            x, dx, shift1, wkv, v_first = cls.time_mixing_seq(
+                x, dx, blk["ln1"], st[:, 1], st[:, 2:], v_first, blk["att"], length, new_starts, i, fused,
+                nst[:, 1] if in_place else None, nst[:, 2:] if packed else None)
+            x, dx, shift0 = cls.channel_mixing_seq(x, dx, blk["ln2"], st[:, 0], blk["ffn"], length, new_starts, fused,
+                                                   nst[:, 0] if in_place else None)
+            if new_state is None:
                 rows += [shift0[:, None], shift1[:, None], wkv]
-        if not packed:
+                continue
+            if not in_place:
+                nst[:, 0], nst[:, 1] = shift0, shift1
+            if not packed:
+                nst[:, 2:] = wkv
+        if new_state is None:
             new_state = torch.cat([r.to(state.dtype) for r in rows], dim=1).reshape(state.shape)
-        logits = layer_norm(x, params["ln_out"]) @ params["head"]["weight"].T
-        return logits, new_state
+        return norm(x, dx, params["ln_out"]) @ params["head"]["weight"].T, new_state

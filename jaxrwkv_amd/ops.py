@@ -688,3 +688,139 @@ def rwkv7_postmix(y, r, k, v, g, ln_w, ln_b, r_k, eps=64e-5):
     if torch.is_grad_enabled() and any(t.requires_grad for t in (y, r, k, v, g, ln_w, ln_b, r_k)):
         return _Postmix.apply(y, r, k, v, g, ln_w2, ln_b2, r_k2, eps)
     return _postmix_fwd(y, r, k, v, g, ln_w2, ln_b2, r_k2, eps)
+
+
+# ----------------------------------------------------------------------------- RWKV-7 sub-block head and op inputs
+LN_SHIFTMIX_MAX_C = 4096      # channels that one workgroup of the fused kernels spans
+
+
+def _ln_shiftmix_fwd(x, dx, ln_w, ln_b, eps, prev, prev_stride, ns, length, mix, shift_out, stats):
+    """``shift_out``: a (B,C) view with contiguous rows that receives the new shift row, or None."""
+    lib = _lib.load()
+    B, T, C = x.shape
+    n_out = len(mix)
+    outs = [torch.empty_like(x) for _ in range(max(n_out, 1))]
+    xs = x if dx is None else torch.empty_like(x)
+    rc = lib.hiprwkv_rwkv7_ln_shiftmix(_stream(), _DT[x.dtype], B, T, C, n_out, _p(x), _p(dx), _p(ln_w), _p(ln_b), eps,
+                                       _p(prev), prev_stride, _p(ns), _p(length), _ptr_array(mix), _ptr_array(outs),
+                                       _p(xs), _p(shift_out), C if shift_out is None else shift_out.stride(0), _p(stats))
+    _lib.check(rc, "hiprwkv_rwkv7_ln_shiftmix")
+    return xs, outs
+
+
+class _LnShiftMix(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, dx, ln_w, ln_b, prev, ns, length, eps, *mix):
+        B, T, C = x.shape
+        prev_t, stride = (None, C) if prev is None else _shift_row(prev, B, C, x.dtype)
+        stats = torch.empty((B * T, 2), dtype=torch.float32, device=x.device)
+        shift = None if prev is None else torch.empty((B, C), dtype=x.dtype, device=x.device)
+        xs, outs = _ln_shiftmix_fwd(x, dx, ln_w, ln_b, eps, prev_t, stride, ns, length, mix, shift, stats)
+        ctx.save_for_backward(xs, stats, ln_w, ln_b, prev_t, ns, length, *mix)
+        ctx.stride, ctx.has_dx, ctx.need_prev = stride, dx is not None, prev is not None and ctx.needs_input_grad[4]
+        ctx.set_materialize_grads(False)
+        return (xs.view_as(xs) if dx is None else xs, shift) + tuple(outs)
+
+    @staticmethod
+    def backward(ctx, gx, gshift, *gs):
+        xs, stats, ln_w, ln_b, prev, ns, length, *mix = ctx.saved_tensors
+        lib = _lib.load()
+        io = xs.dtype
+        B, T, C = xs.shape
+        n_out = len(mix)
+        gs = [torch.zeros_like(xs) if g is None else _dev(g, io) for g in gs]
+        gx, gshift = (None if g is None else _dev(g, io) for g in (gx, gshift))
+        dxs = torch.empty_like(xs)
+        dprev = torch.empty((B, C), dtype=io, device=xs.device) if ctx.need_prev else None
+        dparam = torch.empty((n_out + 2, C), dtype=io, device=xs.device).unbind(0)
+        nbytes = lib.hiprwkv_rwkv7_ln_shiftmix_bwd_workspace_bytes(B, T, C, n_out)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=xs.device)
+        rc = lib.hiprwkv_rwkv7_ln_shiftmix_bwd(_stream(), _DT[io], B, T, C, n_out, _p(xs), _p(stats), _p(ln_w), _p(ln_b),
+                                               _p(prev), ctx.stride, _p(ns), _p(length), _ptr_array(mix), _ptr_array(gs),
+                                               _p(gx), _p(gshift), _p(dxs), _p(dprev), _ptr_array(dparam), _p(ws), nbytes)
+        _lib.check(rc, "hiprwkv_rwkv7_ln_shiftmix_bwd")
+        return (dxs, dxs if ctx.has_dx else None, dparam[-2], dparam[-1], dprev, None, None, None) + tuple(dparam[:-2])
+
+
+def rwkv7_ln_shiftmix(x, dx, ln, prev, new_starts, length, mix, eps=1e-5, shift_out=None):
+    """The head of a sub-block in one pass: ``xs = x + dx`` (``dx`` may be None), ``xn = layer_norm(xs)`` with
+    ``ln = {"weight", "bias"}``, then token shift and interpolation of ``xn`` as in ``rwkv7_shiftmix``.  Returns
+    (xs, new shift row (B,C), the tuple of interpolations); the new shift row is ``xn`` of token ``(length - 1) mod T``.
+    With an empty ``mix`` (``prev`` None) the one output is ``xn`` itself and there is no shift row.  ``shift_out``: write
+    the shift row there (a (B,C) view with contiguous rows, no autograd).  ``length`` (B,) int32 or None; C at most
+    ``LN_SHIFTMIX_MAX_C``.  Differentiable in x, dx, prev, the norm's and the mix parameters."""
+    io = x.dtype
+    B, T, C = x.shape
+    assert len(mix) in (0, 1, 6) and C % 8 == 0 and C <= LN_SHIFTMIX_MAX_C, (len(mix), C)
+    x = _dev(x, io)
+    dx = None if dx is None else _dev(dx, io)
+    ln_w, ln_b = _dev(ln["weight"], io), _dev(ln["bias"], io)
+    mix2 = [_dev(m.reshape(C), io) for m in mix]
+    if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, dx, ln_w, ln_b, prev, *mix2)):
+        xs, shift, *outs = _LnShiftMix.apply(x, dx, ln_w, ln_b, prev, new_starts, length, eps, *mix2)
+        return xs, shift, outs
+    prev_t, stride = (None, C) if prev is None else _shift_row(prev, B, C, io)
+    if shift_out is None and prev is not None:
+        shift_out = torch.empty((B, C), dtype=io, device=x.device)
+    xs, outs = _ln_shiftmix_fwd(x, dx, ln_w, ln_b, eps, prev_t, stride, new_starts, length, mix2, shift_out, None)
+    return xs, shift_out, outs
+
+
+def _pre_fwd(xw, k, xa, v, vf, xv, w0, a0, v0, k_k, k_a):
+    lib = _lib.load()
+    H, N = k.shape[-2:]
+    w, k_out, a_out, b_out = (torch.empty_like(k) for _ in range(4))
+    v_out = None if vf is None else torch.empty_like(k)
+    rc = lib.hiprwkv_rwkv7_pre(_stream(), _DT[k.dtype], k.numel() // (H * N), H, N, _p(xw), _p(k), _p(xa), _p(v), _p(vf),
+                               _p(xv), _p(w0), _p(a0), _p(v0), _p(k_k), _p(k_a), _p(w), _p(k_out), _p(v_out), _p(a_out),
+                               _p(b_out))
+    _lib.check(rc, "hiprwkv_rwkv7_pre")
+    return w, k_out, v_out, a_out, b_out
+
+
+class _Pre(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, xw, k, xa, v, vf, xv, w0, a0, v0, k_k, k_a):
+        ctx.save_for_backward(xw, k, xa, v, vf, xv, w0, a0, v0, k_k, k_a)
+        return _pre_fwd(xw, k, xa, v, vf, xv, w0, a0, v0, k_k, k_a)
+
+    @staticmethod
+    def backward(ctx, gw, gk, gv, ga, gb):
+        xw, k, xa, v, vf, xv, w0, a0, v0, k_k, k_a = ctx.saved_tensors
+        lib = _lib.load()
+        io = k.dtype
+        H, N = k.shape[-2:]
+        rows = k.numel() // (H * N)
+        gw, gk, ga, gb = (_dev(g, io) for g in (gw, gk, ga, gb))
+        dxw, dk, dxa = (torch.empty_like(k) for _ in range(3))
+        dv = dvf = dxv = None
+        if vf is not None:
+            gv = _dev(gv, io)
+            dv, dvf, dxv = (torch.empty_like(k) for _ in range(3))
+        dparam = torch.empty((5, H * N), dtype=io, device=k.device).unbind(0)
+        nbytes = lib.hiprwkv_rwkv7_pre_bwd_workspace_bytes(rows, H, N)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=k.device)
+        rc = lib.hiprwkv_rwkv7_pre_bwd(_stream(), _DT[io], rows, H, N, _p(xw), _p(k), _p(xa), _p(v), _p(vf), _p(xv), _p(w0),
+                                       _p(a0), _p(v0), _p(k_k), _p(k_a), _p(gw), _p(gk), None if vf is None else _p(gv),
+                                       _p(ga), _p(gb), _p(dxw), _p(dk), _p(dv), _p(dvf), _p(dxv), _p(dxa),
+                                       _ptr_array(dparam), _p(ws), nbytes)
+        _lib.check(rc, "hiprwkv_rwkv7_pre_bwd")
+        dw0, da0, dk_k, dk_a, dv0 = dparam
+        return dxw, dk, dxa, dv, dvf, dxv, dw0, da0, (None if vf is None else dv0), dk_k, dk_a
+
+
+def rwkv7_pre(xw, k, xa, v, v_first, xv, w0, a0, v0, k_k, k_a):
+    """``rwkv7_decay``, ``rwkv7_vmix``, ``rwkv7_agate`` and ``rwkv7_premix`` in one pass: xw, xa, xv the low-rank terms of
+    decay, gate and value residual, k and v the projections, all (..., H, N); parameters (C,).  Returns (w, k', v', a_i,
+    b_i), the WKV op's inputs.  The first layer has no value residual: ``v_first``, ``xv``, ``v0`` None, and v' is ``v``."""
+    io = k.dtype
+    C = k.shape[-2] * k.shape[-1]
+    xw, k, xa, v = (_dev(t, io) for t in (xw, k, xa, v))
+    w0, a0, k_k, k_a = (_dev(t.reshape(C), io) for t in (w0, a0, k_k, k_a))
+    if v_first is None:
+        args = (xw, k, xa, None, None, None, w0, a0, None, k_k, k_a)
+    else:
+        args = (xw, k, xa, v, _dev(v_first, io), _dev(xv, io), w0, a0, _dev(v0.reshape(C), io), k_k, k_a)
+    grad = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in args)
+    w, k_out, v_out, a_out, b_out = _Pre.apply(*args) if grad else _pre_fwd(*args)
+    return w, k_out, (v if v_first is None else v_out), a_out, b_out
