@@ -318,6 +318,32 @@ int hiprwkv_rwkv7_pre_bwd(hiprwkv_stream stream, int io_dtype, int64_t rows, int
                           const void* gb_out, void* dxw, void* dk, void* dv, void* dv_first, void* dxv, void* dxa,
                           void* const* dparam, void* workspace, size_t workspace_bytes);
 
+/* ---- RWKV-7: a decode step of the whole model ---------------------------------------------------------
+ * rwkv7.py:190-198, :223-291 for at most HIPRWKV_SMALL_T tokens per sequence and HIPRWKV_DECODE_MAX_ROWS tokens in all, bf16
+ * throughout, from the embedded tokens to the last norm (and, where `logits` is given, through the head).  Parameters are
+ * the reference's arrays stacked over the L layers, contiguous: vectors (L, C), r_k (L, H, 64), receptance / key / value /
+ * output (L, C, C) and ffn_key (L, F, C), ffn_value (L, C, F) used as x W^T, the low-rank factors (L, C, d) and (L, d, C)
+ * used as x W; head (vocab, C).  state and new_state are (B, L, 2 + 64, C) and different arrays; length (B,) int32 or
+ * NULL (= T), new_starts (B, T) or NULL.  C = 64 H at most 4096; d_* and F multiples of 32; vocab a multiple of 16.
+ * x (B*T, C) in, xn (B*T, C) out, logits (B*T, vocab) out or NULL.  flags: HIPRWKV_COMPAT_ASSOC. */
+#define HIPRWKV_DECODE_MAX_ROWS 256
+typedef struct hiprwkv_rwkv7_decode_args {
+  int64_t B, T, L, C, H, F, vocab, d_decay, d_aaa, d_mv, d_gate;
+  const void *x, *state;
+  void *new_state;
+  const int32_t* length;
+  const uint8_t* new_starts;
+  const void *ln0_w, *ln0_b, *ln_out_w, *ln_out_b, *head, *ln1_w, *ln1_b, *ln2_w, *ln2_b;
+  const void *x_r, *x_w, *x_k, *x_v, *x_a, *x_g;
+  const void *w0, *w1, *w2, *a0, *a1, *a2, *v0, *v1, *v2, *g1, *g2, *k_k, *k_a, *r_k;
+  const void *receptance, *key, *value, *output, *lnx_w, *lnx_b, *ffn_x_k, *ffn_key, *ffn_value;
+  void *xn, *logits, *workspace;
+  uint64_t workspace_bytes;
+  uint64_t flags;
+} hiprwkv_rwkv7_decode_args;
+size_t hiprwkv_rwkv7_decode_workspace_bytes(const hiprwkv_rwkv7_decode_args* args);
+int hiprwkv_rwkv7_decode(hiprwkv_stream stream, const hiprwkv_rwkv7_decode_args* args);
+
 /* ---- RWKV-7 time-mixing stages around the op ------------------------------------------
  * The element-wise work the reference does in jnp on either side of inner_loop (rwkv7.py:248-252, 257 and :263-265),
  * fused into one pass each; it has no counterpart among the reference's ffi targets.  `rows` = number of tokens

@@ -19,6 +19,18 @@ PUBLIC_FLAGS = COMPAT_ASSOC | FORCE_SEQ | NO_SMALL_T | W_PER_HEAD | CKPT_READY
 
 _vp, _i64, _int, _u32, _sz = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_uint, ctypes.c_size_t
 
+
+
+class Rwkv7DecodeArgs(ctypes.Structure):
+    """``hiprwkv_rwkv7_decode_args``"""
+    _fields_ = ([(n, _i64) for n in "B T L C H F vocab d_decay d_aaa d_mv d_gate".split()]
+                + [(n, _vp) for n in ("x state new_state length new_starts ln0_w ln0_b ln_out_w ln_out_b head ln1_w ln1_b "
+                                      "ln2_w ln2_b x_r x_w x_k x_v x_a x_g w0 w1 w2 a0 a1 a2 v0 v1 v2 g1 g2 k_k k_a r_k "
+                                      "receptance key value output lnx_w lnx_b ffn_x_k ffn_key ffn_value xn logits "
+                                      "workspace").split()]
+                + [("workspace_bytes", ctypes.c_uint64), ("flags", ctypes.c_uint64)])
+
+
 # name -> (restype, argtypes); mirrors include/hiprwkv.h declaration by declaration
 SIGNATURES = {
     "hiprwkv_last_error": (ctypes.c_char_p, []),
@@ -62,6 +74,8 @@ SIGNATURES = {
     "hiprwkv_rwkv7_pre": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 16),
     "hiprwkv_rwkv7_pre_bwd_workspace_bytes": (_sz, [_i64] * 3),
     "hiprwkv_rwkv7_pre_bwd": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 24 + [_sz]),
+    "hiprwkv_rwkv7_decode_workspace_bytes": (_sz, [ctypes.POINTER(Rwkv7DecodeArgs)]),
+    "hiprwkv_rwkv7_decode": (_int, [_vp, ctypes.POINTER(Rwkv7DecodeArgs)]),
     "hiprwkv_rwkv7_premix": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 7),
     "hiprwkv_rwkv7_postmix": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 8 + [ctypes.c_float, _vp]),
     "hiprwkv_rwkv7_premix_bwd": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 11),

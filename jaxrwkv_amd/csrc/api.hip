@@ -811,4 +811,31 @@ int hiprwkv_rwkv7_pre_bwd(hiprwkv_stream stream, int io_dtype, int64_t rows, int
   return gate_done("rwkv7_pre_bwd", launch_rwkv7_pre_bwd(io_dtype == HIPRWKV_F32, A, dparam, static_cast<hipStream_t>(stream)));
 }
 
+size_t hiprwkv_rwkv7_decode_workspace_bytes(const hiprwkv_rwkv7_decode_args* args) { return rwkv7_decode_workspace(*args); }
+
+int hiprwkv_rwkv7_decode(hiprwkv_stream stream, const hiprwkv_rwkv7_decode_args* args) {
+  if (args == nullptr) return fail(HIPRWKV_EINVAL, "rwkv7_decode: null arguments");
+  const hiprwkv_rwkv7_decode_args& D = *args;
+  if (D.B <= 0 || D.T <= 0 || D.L <= 0 || D.T > HIPRWKV_SMALL_T || D.B * D.T > HIPRWKV_DECODE_MAX_ROWS)
+    return fail(HIPRWKV_EINVAL, "rwkv7_decode: B, T, L must be positive, T at most %d and B*T at most %d", HIPRWKV_SMALL_T, HIPRWKV_DECODE_MAX_ROWS);
+  if (D.C != D.H * 64 || D.C > 4096) return fail(HIPRWKV_EINVAL, "rwkv7_decode: C must be 64 H and at most 4096");
+  for (int64_t d : {D.F, D.d_decay, D.d_aaa, D.d_mv, D.d_gate})
+    if (d <= 0 || d % 32 != 0) return fail(HIPRWKV_EINVAL, "rwkv7_decode: inner sizes must be positive multiples of 32");
+  if (D.logits != nullptr && (D.vocab <= 0 || D.vocab % 16 != 0)) return fail(HIPRWKV_EINVAL, "rwkv7_decode: vocab must be a positive multiple of 16");
+  if (D.flags & ~(uint64_t)HIPRWKV_COMPAT_ASSOC) return fail(HIPRWKV_EINVAL, "rwkv7_decode: unknown flag bits");
+  const void* req[] = {D.x, D.state, D.new_state, D.ln0_w, D.ln0_b, D.ln_out_w, D.ln_out_b, D.ln1_w, D.ln1_b, D.ln2_w,
+                       D.ln2_b, D.x_r, D.x_w, D.x_k, D.x_v, D.x_a, D.x_g, D.w0, D.w1, D.w2, D.a0, D.a1, D.a2, D.v0, D.v1,
+                       D.v2, D.g1, D.g2, D.k_k, D.k_a, D.r_k, D.receptance, D.key, D.value, D.output, D.lnx_w, D.lnx_b,
+                       D.ffn_x_k, D.ffn_key, D.ffn_value, D.xn, D.workspace};
+  for (const void* p : req)
+    if (p == nullptr || !aligned16(p)) return fail(HIPRWKV_EINVAL, "rwkv7_decode: null or misaligned tensor pointer (16 bytes)");
+  if (D.logits != nullptr && (D.head == nullptr || !aligned16(D.head) || !aligned16(D.logits)))
+    return fail(HIPRWKV_EINVAL, "rwkv7_decode: null or misaligned head or logits");
+  if (D.state == D.new_state) return fail(HIPRWKV_EINVAL, "rwkv7_decode: state and new_state must be different arrays");
+  const size_t need = rwkv7_decode_workspace(D);
+  if (D.workspace_bytes < need)
+    return fail(HIPRWKV_ENOSPACE, "rwkv7_decode: workspace has %llu bytes, %zu needed", (unsigned long long)D.workspace_bytes, need);
+  return gate_done("rwkv7_decode", launch_rwkv7_decode(D, static_cast<hipStream_t>(stream)));
+}
+
 }  // extern "C"

@@ -2,8 +2,11 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <string.h>
 
 #include <atomic>
+
+#include "../../include/hiprwkv.h"
 
 namespace hiprwkv {
 
@@ -125,6 +128,10 @@ struct PreArgs {
 int64_t rwkv7_pre_bwd_rows(int64_t rows, int64_t H);
 hipError_t launch_rwkv7_pre(int io_f32, const PreArgs& A, hipStream_t stream);
 hipError_t launch_rwkv7_pre_bwd(int io_f32, const PreArgs& A, void* const* dparam, hipStream_t stream);
+
+using Rwkv7Decode = ::hiprwkv_rwkv7_decode_args;
+size_t rwkv7_decode_workspace(const Rwkv7Decode& D);
+hipError_t launch_rwkv7_decode(const Rwkv7Decode& D, hipStream_t stream);
 
 // Raises a kernel's dynamic-LDS limit once per kernel and device instead of at every enqueue (the attribute call
 // goes to the driver; hipGetDevice does not).

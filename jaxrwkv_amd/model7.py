@@ -220,11 +220,17 @@ class RWKV7:
         L, H, N = params["blocks"]["att"]["r_k"].shape
         C = H * N
         fused = cls.fuse_mix and C <= ops.LN_SHIFTMIX_MAX_C
+        x = params["emb"]["weight"][tokens]
+        grad = torch.is_grad_enabled() and (x.requires_grad or state.requires_grad)
+        # decode steps whose recurrence is this package's: the whole step from native code
+        if fused and not grad and T <= 8 and cls.inner.inner_loop == HipRWKV.inner_loop and not HipRWKV.force_seq:
+            step = ops.rwkv7_decode(params, x, state, length, new_starts, HipRWKV.assoc_compat)
+            if step is not None:
+                return step
         norm = (lambda x, dx, ln: ops.rwkv7_ln_shiftmix(x, dx, ln, None, None, None, [])[2][0]) if fused else \
                (lambda x, dx, ln: layer_norm(x if dx is None else x + dx, ln))
-        x = norm(params["emb"]["weight"][tokens], None, params["ln0"])
+        x = norm(x, None, params["ln0"])
         blocks = unstack(params["blocks"], L)
-        grad = torch.is_grad_enabled() and (x.requires_grad or state.requires_grad)
         # without autograd the layers write their rows of the new state where they belong; decode steps read and write the
         # recurrence's rows in place as well
         in_place = fused and not grad and state.dtype == x.dtype and (C * x.element_size()) % 16 == 0

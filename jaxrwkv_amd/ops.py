@@ -824,3 +824,63 @@ def rwkv7_pre(xw, k, xa, v, v_first, xv, w0, a0, v0, k_k, k_a):
     grad = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in args)
     w, k_out, v_out, a_out, b_out = _Pre.apply(*args) if grad else _pre_fwd(*args)
     return w, k_out, (v if v_first is None else v_out), a_out, b_out
+
+
+# ----------------------------------------------------------------------------- RWKV-7 decode step
+DECODE_MAX_ROWS = 256         # HIPRWKV_DECODE_MAX_ROWS
+DECODE_HEAD_ROWS = 64         # up to here the head's product is a stream of its weights; beyond, the library's is faster
+
+
+def _decode_tensors(params, C, F, vocab):
+    """(argument name, tensor, shape after the layer axis) of every parameter of a decode step."""
+    att, ffn = params["blocks"]["att"], params["blocks"]["ffn"]
+    ln1, ln2 = params["blocks"]["ln1"], params["blocks"]["ln2"]
+    vec = [(n, att[n]) for n in ("x_r", "x_w", "x_k", "x_v", "x_a", "x_g", "w0", "a0", "v0", "k_k", "k_a")]
+    vec += [("ln1_w", ln1["weight"]), ("ln1_b", ln1["bias"]), ("ln2_w", ln2["weight"]), ("ln2_b", ln2["bias"]),
+            ("lnx_w", att["ln_x"]["weight"]), ("lnx_b", att["ln_x"]["bias"]), ("ffn_x_k", ffn["x_k"])]
+    out = [(n, t, (C,)) for n, t in vec]
+    out += [(n, att[n]["weight"], (C, C)) for n in ("receptance", "key", "value", "output")]
+    for n, d in (("w", "d_decay"), ("a", "d_aaa"), ("v", "d_mv"), ("g", "d_gate")):
+        t1, t2 = att[n + "1"], att[n + "2"]
+        out += [(n + "1", t1, (C, t1.shape[-1])), (n + "2", t2, (t1.shape[-1], C))]
+    out += [("r_k", att["r_k"], (C // 64, 64)), ("ffn_key", ffn["key"]["weight"], (F, C)),
+            ("ffn_value", ffn["value"]["weight"], (C, F))]
+    return out
+
+
+def rwkv7_decode(params, x, state, length, new_starts, compat=True):
+    """A decode step of the whole RWKV-7 model from native code: x (B,T,C) the embedded tokens, state (B,L,2+64,C), length
+    (B,) int32 or None, new_starts (B,T) bool or None.  Returns (logits, new state), or None where the step's kernels do
+    not cover the call: they take bf16, contiguous stacked parameters, at most ``DECODE_MAX_ROWS`` tokens of which at most
+    8 per sequence, and inner sizes that are multiples of 32.  No autograd."""
+    B, T, C = x.shape
+    bf = torch.bfloat16
+    L, H, N = params["blocks"]["att"]["r_k"].shape
+    head = params["head"]["weight"]
+    F, vocab = params["blocks"]["ffn"]["key"]["weight"].shape[-2], head.shape[0]
+    att = params["blocks"]["att"]
+    dims = [att[n].shape[-1] for n in ("w1", "a1", "v1", "g1")]
+    if (T > 8 or B * T > DECODE_MAX_ROWS or N != 64 or C != H * N or C > LN_SHIFTMIX_MAX_C or vocab % 16
+            or any(d % 32 for d in (F, *dims)) or not x.is_cuda or x.dtype != bf
+            or state.shape != (B, L, 2 + N, C) or state.dtype != bf or not state.is_contiguous() or state.data_ptr() % 16):
+        return None
+    A = _lib.Rwkv7DecodeArgs(B=B, T=T, L=L, C=C, H=H, F=F, vocab=vocab, d_decay=dims[0], d_aaa=dims[1], d_mv=dims[2],
+                             d_gate=dims[3])
+    tensors = [(n, t, (L,) + s) for n, t, s in _decode_tensors(params, C, F, vocab)]
+    tensors += [(n + k, params[n]["weight" if k == "_w" else "bias"], (C,)) for n in ("ln0", "ln_out") for k in ("_w", "_b")]
+    for name, t, shape in tensors + [("head", head, (vocab, C))]:
+        ptr = t.data_ptr()
+        if t.dtype != bf or t.shape != shape or not t.is_contiguous() or ptr % 16 or t.device != x.device:
+            return None
+        setattr(A, name, ptr)
+    lib = _lib.load()
+    x = x.contiguous()
+    new_state, xn = torch.empty_like(state), torch.empty_like(x)
+    logits = torch.empty((B, T, vocab), dtype=bf, device=x.device) if B * T <= DECODE_HEAD_ROWS else None
+    nbytes = lib.hiprwkv_rwkv7_decode_workspace_bytes(ctypes.byref(A))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    A.x, A.state, A.new_state, A.length, A.new_starts = _p(x), _p(state), _p(new_state), _p(length), _p(new_starts)
+    A.xn, A.logits, A.workspace, A.workspace_bytes = _p(xn), _p(logits), _p(ws), nbytes
+    A.flags = _lib.COMPAT_ASSOC if compat else 0
+    _lib.check(lib.hiprwkv_rwkv7_decode(_stream(), ctypes.byref(A)), "hiprwkv_rwkv7_decode")
+    return (xn @ head.T if logits is None else logits), new_state
