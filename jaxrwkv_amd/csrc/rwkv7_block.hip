@@ -144,12 +144,24 @@ __global__ __launch_bounds__(64 * MAX_WAVES) void ln_shiftmix_kernel(LnMixArgs A
       const int64_t n = g0 + j < n1 ? g0 + j : n1 - 1;
       zero_or_ld8(reinterpret_cast<const T*>(A.x) + n * C + cc, on, x[j]);
     }
-    if (A.dx != nullptr) {
+    if (A.dx != nullptr || A.n_part > 1) {
 #pragma unroll
       for (int j = 0; j < FWD_GROUP; ++j) {
         const int64_t n = g0 + j < n1 ? g0 + j : n1 - 1;
         float d[8];
-        zero_or_ld8(reinterpret_cast<const T*>(A.dx) + n * C + cc, on, d);
+        if (A.n_part > 1) {                    // a product's partial sums: dx is their sum, rounded as the product's result
+          zero_or_ld8(A.part + n * C + cc, on, d);
+          for (int p = 1; p < A.n_part; ++p) {
+            float e[8];
+            zero_or_ld8(A.part + (p * total + n) * C + cc, on, e);
+#pragma unroll
+            for (int c = 0; c < 8; ++c) d[c] += e[c];
+          }
+#pragma unroll
+          for (int c = 0; c < 8; ++c) d[c] = round_io<T>(d[c]);
+        } else {
+          zero_or_ld8(reinterpret_cast<const T*>(A.dx) + n * C + cc, on, d);
+        }
 #pragma unroll
         for (int c = 0; c < 8; ++c) x[j][c] = round_io<T>(x[j][c] + d[c]);
         if (on && g0 + j >= n0 && g0 + j < n1) st8(reinterpret_cast<T*>(A.xs) + n * C + cc, x[j]);

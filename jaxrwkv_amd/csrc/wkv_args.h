@@ -101,7 +101,9 @@ struct LnMixArgs {
   const void* g[6];
   const void *gx, *gshift;       // cotangents of xs and of the shift row (B,C), each may be null
   void *dxs, *dprev;             // dprev (B,C) may be null
-  float* part;                   // workspace (workgroups, n_out + 2, C)
+  // backward: workspace (workgroups, n_out + 2, C).  Forward: dx as n_part > 1 partial sums (n_part, B*T, C) in place of `dx`
+  float* part;
+  int n_part;
 };
 struct ReduceArgs {
   const float* part;             // (rows, nk, C)
