@@ -66,13 +66,16 @@ extern "C" {
 /* hiprwkv_wkv4_bwd: the workspace already holds the checkpoints that hiprwkv_wkv4_fwd_ckpt wrote for the same
  * inputs; the backward then skips its own first pass over k and v. */
 #define HIPRWKV_CKPT_READY 0x20u
+/* hiprwkv_wkv4_*: `w` is the parameter time_decay itself; the op's decay is -exp(w), rounded to io_dtype
+ * (rwkv4.py:312), and the cotangent returned is the one of w. */
+#define HIPRWKV_W_RAW 0x80u
 /* Test hook for the chunked kernels' bounded hand-shake: the producer wave of the last chunk does not publish it, the
  * consumer waves' wait runs out (a few milliseconds), every wave still ends normally, the outputs of every
  * (sequence, head) are NaN and hiprwkv_handshake_failures() has advanced by B*H per kernel. */
 #define HIPRWKV_DEBUG_DROP_PUBLISH 0x100u
 /* Every flag a production caller may pass.  Entry points refuse other bits, and refuse HIPRWKV_DEBUG_DROP_PUBLISH
  * unless the process runs with HIPRWKV_ENABLE_DEBUG_FLAGS=1 in its environment. */
-#define HIPRWKV_PUBLIC_FLAGS (HIPRWKV_COMPAT_ASSOC | HIPRWKV_FORCE_SEQ | HIPRWKV_NO_SMALL_T | HIPRWKV_W_PER_HEAD | HIPRWKV_CKPT_READY)
+#define HIPRWKV_PUBLIC_FLAGS (HIPRWKV_COMPAT_ASSOC | HIPRWKV_FORCE_SEQ | HIPRWKV_NO_SMALL_T | HIPRWKV_W_PER_HEAD | HIPRWKV_CKPT_READY | HIPRWKV_W_RAW)
 
 typedef void* hiprwkv_stream; /* a hipStream_t */
 
@@ -237,6 +240,24 @@ int hiprwkv_wkv4_bwd_noalloc(hiprwkv_stream stream, int io_dtype,
                              const void* w, const void* u, const void* k, const void* v, const void* gy, const void* s,
                              const uint32_t* length, const uint8_t* new_starts, const void* gs_new,
                              float* gw, float* gu, void* gk, void* gv, void* gs, unsigned flags);
+
+/* inner_loop of RWKV-4 around the op (rwkv4.py:402-406): out = r . wkv, wkv rounded to io_dtype first; r NULL: the op alone.
+ * Where B and C leave most of the GPU idle the sequences are cut into parts whose summaries are made first, in
+ * `workspace` (hiprwkv_wkv4_mix_workspace_bytes, may be 0).  ckpt as in hiprwkv_wkv4_fwd_ckpt, or NULL. */
+size_t hiprwkv_wkv4_mix_workspace_bytes(int64_t B, int64_t T, int64_t C);
+int hiprwkv_wkv4_mix(hiprwkv_stream stream, int io_dtype, int64_t B, int64_t T, int64_t C,
+                     const void* w, const void* u, const void* k, const void* v, const void* r, const void* s,
+                     const uint32_t* length, const uint8_t* new_starts, void* new_s, void* out,
+                     void* ckpt, size_t ckpt_bytes, void* workspace, size_t workspace_bytes, unsigned flags);
+/* Its cotangents for gout, the one of out: gw and gu (C,) io_dtype summed over the sequences, gk, gv, gr (B,T,C), gs.  ckpt:
+ * hiprwkv_wkv4_bwd_workspace_bytes, filled by hiprwkv_wkv4_mix when HIPRWKV_CKPT_READY is set.  r and gr both NULL: the op
+ * alone. */
+size_t hiprwkv_wkv4_mix_bwd_workspace_bytes(int64_t B, int64_t T, int64_t C);
+int hiprwkv_wkv4_mix_bwd(hiprwkv_stream stream, int io_dtype, int64_t B, int64_t T, int64_t C,
+                         const void* w, const void* u, const void* k, const void* v, const void* r, const void* gout,
+                         const void* s, const uint32_t* length, const uint8_t* new_starts, const void* gs_new,
+                         void* ckpt, size_t ckpt_bytes, void* gw, void* gu, void* gk, void* gv, void* gr, void* gs,
+                         void* workspace, size_t workspace_bytes, unsigned flags);
 
 /* ---- RWKV-7 token shift and interpolation ---------------------------------------------------
  * The head of time_mixing_seq and channel_mixing_seq (rwkv7.py:226-235 and :192-195), which the reference computes in

@@ -14,8 +14,9 @@ FORCE_SEQ = 2
 NO_SMALL_T = 4
 W_PER_HEAD = 0x10
 CKPT_READY = 0x20
+W_RAW = 0x80
 DEBUG_DROP_PUBLISH = 0x100      # refused unless the process runs with HIPRWKV_ENABLE_DEBUG_FLAGS=1
-PUBLIC_FLAGS = COMPAT_ASSOC | FORCE_SEQ | NO_SMALL_T | W_PER_HEAD | CKPT_READY
+PUBLIC_FLAGS = COMPAT_ASSOC | FORCE_SEQ | NO_SMALL_T | W_PER_HEAD | CKPT_READY | W_RAW
 
 _vp, _i64, _int, _u32, _sz = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_uint, ctypes.c_size_t
 
@@ -57,6 +58,10 @@ SIGNATURES = {
                          + [_vp, _sz, _u32]),
     "hiprwkv_wkv4_bwd_noalloc_max_bytes": (_sz, []),
     "hiprwkv_wkv4_bwd_noalloc": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 6 + [_vp, _vp] + [_vp] + [_vp] * 5 + [_u32]),
+    "hiprwkv_wkv4_mix_workspace_bytes": (_sz, [_i64] * 3),
+    "hiprwkv_wkv4_mix": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 10 + [_vp, _sz, _vp, _sz, _u32]),
+    "hiprwkv_wkv4_mix_bwd_workspace_bytes": (_sz, [_i64] * 3),
+    "hiprwkv_wkv4_mix_bwd": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 10 + [_vp, _sz] + [_vp] * 6 + [_vp, _sz, _u32]),
     "hiprwkv_rwkv7_shiftmix": (_int, [_vp, _int, _i64, _i64, _i64, _int, _vp, _vp, _i64, _vp, _vp, _vp]),
     "hiprwkv_rwkv7_shiftmix_bwd": (_int, [_vp, _int, _i64, _i64, _i64, _int, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _vp]),
     "hiprwkv_rwkv7_decay": (_int, [_vp, _int, _i64, _i64, _vp, _vp, _vp]),

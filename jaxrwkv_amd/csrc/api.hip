@@ -427,6 +427,7 @@ static int wkv4_fwd_impl(hiprwkv_stream stream, int io_dtype, int64_t B, int64_t
   A.length = length; A.ns = new_starts;
   A.new_s = new_s; A.out = out;
   A.ckpt = ckpt;
+  A.nz = 1; A.part = (T + 15) / 16 * 16;
   A.io_f32 = io_dtype == HIPRWKV_F32;
   A.flags = flags;
   hipError_t e = launch_wkv4_fwd(A, static_cast<hipStream_t>(stream));
@@ -464,7 +465,8 @@ int hiprwkv_wkv4_bwd(hiprwkv_stream stream, int io_dtype, int64_t B, int64_t T, 
   A.io_f32 = io_dtype == HIPRWKV_F32;
   A.flags = flags;
   A.gy = gy; A.gs_new = gs_new;
-  A.gk = gk; A.gv = gv; A.gs = gs; A.gw = gw; A.gu = gu;
+  A.gk = gk; A.gv = gv; A.gs = gs; A.gw = gw; A.gu = gu; A.gw_stride = C;
+  A.nz = 1; A.part = (T + 15) / 16 * 16;
   A.ckpt = static_cast<float*>(workspace);
   hipError_t e = launch_wkv4_bwd(A, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail(HIPRWKV_ELAUNCH, "wkv4_bwd: %s", hipGetErrorString(e));
@@ -836,6 +838,100 @@ int hiprwkv_rwkv7_decode(hiprwkv_stream stream, const hiprwkv_rwkv7_decode_args*
   if (D.workspace_bytes < need)
     return fail(HIPRWKV_ENOSPACE, "rwkv7_decode: workspace has %llu bytes, %zu needed", (unsigned long long)D.workspace_bytes, need);
   return gate_done("rwkv7_decode", launch_rwkv7_decode(D, static_cast<hipStream_t>(stream)));
+}
+
+// ---- WKV4 with the receptance applied, sequences cut into parts where the batch leaves the GPU idle
+namespace {
+size_t wkv4_part_bytes(int64_t B, int64_t T, int64_t C, int floats) {
+  int64_t part;
+  const int64_t nz = wkv4_parts(B, T, C, &part);
+  return align256((size_t)B * (nz - 1) * C * floats * sizeof(float));
+}
+int check_wkv4(const char* op, int io_dtype, int64_t B, int64_t T, int64_t C, unsigned flags, std::initializer_list<const void*> req,
+               std::initializer_list<const void*> opt) {
+  if (int rc = check_flags(op, flags)) return rc;
+  if (!dtype_ok(io_dtype)) return fail(HIPRWKV_EINVAL, "%s: dtype must be HIPRWKV_F32 or HIPRWKV_BF16", op);
+  if (B <= 0 || T <= 0 || C <= 0) return fail(HIPRWKV_EINVAL, "%s: B,T,C must be positive", op);
+  if (B * ((C + 63) / 64) > 0x7fffffffLL) return fail(HIPRWKV_EINVAL, "%s: B*C exceeds the grid limit", op);
+  if (C > (1LL << 23)) return fail(HIPRWKV_EINVAL, "%s: C exceeds 2^23 channels", op);
+  for (const void* p : req)
+    if (p == nullptr || !aligned16(p)) return fail(HIPRWKV_EINVAL, "%s: null or misaligned tensor pointer (16 bytes)", op);
+  for (const void* p : opt)
+    if (p != nullptr && !aligned16(p)) return fail(HIPRWKV_EINVAL, "%s: tensor pointers must be 16-byte aligned", op);
+  return HIPRWKV_OK;
+}
+}  // namespace
+
+size_t hiprwkv_wkv4_mix_workspace_bytes(int64_t B, int64_t T, int64_t C) { return wkv4_part_bytes(B, T, C, 4); }
+
+int hiprwkv_wkv4_mix(hiprwkv_stream stream, int io_dtype, int64_t B, int64_t T, int64_t C, const void* w, const void* u,
+                     const void* k, const void* v, const void* r, const void* s, const uint32_t* length,
+                     const uint8_t* new_starts, void* new_s, void* out, void* ckpt, size_t ckpt_bytes, void* workspace,
+                     size_t workspace_bytes, unsigned flags) {
+  if (int rc = check_wkv4("wkv4_mix", io_dtype, B, T, C, flags, {w, u, k, v, s, new_s, out}, {r, ckpt, workspace})) return rc;
+  const size_t need = hiprwkv_wkv4_mix_workspace_bytes(B, T, C);
+  if (workspace_bytes < need || (need != 0 && workspace == nullptr))
+    return fail(HIPRWKV_ENOSPACE, "wkv4_mix: workspace has %zu bytes, %zu needed", workspace_bytes, need);
+  if (ckpt != nullptr && ckpt_bytes < hiprwkv_wkv4_bwd_workspace_bytes(B, T, C))
+    return fail(HIPRWKV_ENOSPACE, "wkv4_mix: checkpoint array has %zu bytes, %zu needed", ckpt_bytes, hiprwkv_wkv4_bwd_workspace_bytes(B, T, C));
+  Wkv4Args A;
+  memset(&A, 0, sizeof(A));
+  A.B = B; A.T = T; A.C = C;
+  A.w = w; A.u = u; A.k = k; A.v = v; A.r = r; A.s = s;
+  A.length = length; A.ns = new_starts;
+  A.new_s = new_s; A.out = out;
+  A.ckpt = static_cast<float*>(ckpt);
+  A.io_f32 = io_dtype == HIPRWKV_F32;
+  A.flags = flags;
+  A.nz = wkv4_parts(B, T, C, &A.part);
+  A.sums = static_cast<float*>(workspace);
+  return gate_done("wkv4_mix", launch_wkv4_fwd(A, static_cast<hipStream_t>(stream)));
+}
+
+size_t hiprwkv_wkv4_mix_bwd_workspace_bytes(int64_t B, int64_t T, int64_t C) {
+  int64_t part;
+  const int64_t nz = wkv4_parts(B, T, C, &part);
+  return wkv4_part_bytes(B, T, C, 8) + align256((size_t)B * nz * 2 * C * sizeof(float));
+}
+
+int hiprwkv_wkv4_mix_bwd(hiprwkv_stream stream, int io_dtype, int64_t B, int64_t T, int64_t C, const void* w,
+                         const void* u, const void* k, const void* v, const void* r, const void* gout, const void* s,
+                         const uint32_t* length, const uint8_t* new_starts, const void* gs_new, void* ckpt,
+                         size_t ckpt_bytes, void* gw, void* gu, void* gk, void* gv, void* gr, void* gs, void* workspace,
+                         size_t workspace_bytes, unsigned flags) {
+  if (int rc = check_wkv4("wkv4_mix_bwd", io_dtype, B, T, C, flags, {w, u, k, v, gout, s, ckpt, gk, gv, gs, workspace}, {r, gr, gs_new}))
+    return rc;
+  if (gw == nullptr || gu == nullptr || ((r == nullptr) != (gr == nullptr)))
+    return fail(HIPRWKV_EINVAL, "wkv4_mix_bwd: null tensor pointer");
+  if (ckpt_bytes < hiprwkv_wkv4_bwd_workspace_bytes(B, T, C))
+    return fail(HIPRWKV_ENOSPACE, "wkv4_mix_bwd: checkpoint array has %zu bytes, %zu needed", ckpt_bytes, hiprwkv_wkv4_bwd_workspace_bytes(B, T, C));
+  const size_t need = hiprwkv_wkv4_mix_bwd_workspace_bytes(B, T, C);
+  if (workspace_bytes < need)
+    return fail(HIPRWKV_ENOSPACE, "wkv4_mix_bwd: workspace has %zu bytes, %zu needed", workspace_bytes, need);
+  Wkv4Args A;
+  memset(&A, 0, sizeof(A));
+  A.B = B; A.T = T; A.C = C;
+  A.w = w; A.u = u; A.k = k; A.v = v; A.r = r; A.s = s;
+  A.length = length; A.ns = new_starts;
+  A.io_f32 = io_dtype == HIPRWKV_F32;
+  A.flags = flags;
+  A.gy = gout; A.gs_new = gs_new;
+  A.gk = gk; A.gv = gv; A.gr = gr; A.gs = gs;
+  A.ckpt = static_cast<float*>(ckpt);
+  A.nz = wkv4_parts(B, T, C, &A.part);
+  A.maps = static_cast<float*>(workspace);
+  A.gw = reinterpret_cast<float*>(static_cast<char*>(workspace) + wkv4_part_bytes(B, T, C, 8));
+  A.gu = A.gw + C;
+  A.gw_stride = 2 * C;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  hipError_t e = launch_wkv4_bwd(A, st);
+  if (e == hipSuccess) {
+    ReduceArgs R;
+    R.part = A.gw; R.rows = B * A.nz; R.nk = 2; R.C = C;
+    R.out[0] = gw; R.out[1] = gu;
+    e = launch_reduce_parts(A.io_f32, R, st);
+  }
+  return gate_done("wkv4_mix_bwd", e);
 }
 
 }  // extern "C"

@@ -63,6 +63,8 @@ struct Wkv6Args {
 
 // Wkv4Args::flags bit: the workspace already holds the checkpoints (HIPRWKV_CKPT_READY)
 constexpr unsigned FLAG_CKPT_READY = 0x20u;
+// Wkv4Args::flags bit: w is the raw time_decay, the decay is -exp(w) (HIPRWKV_W_RAW)
+constexpr unsigned FLAG_W_RAW = 0x80u;
 
 struct Wkv4Args {
   int64_t B, T, C;
@@ -77,9 +79,18 @@ struct Wkv4Args {
   const void* gy;
   const void* gs_new;
   void *gk, *gv, *gs;
-  float *gw, *gu;   // (B,C) each
+  float *gw, *gu;   // rows of C, gw_stride floats apart: one per sequence and part
+  int64_t gw_stride;
   float* ckpt;      // workspace: (B, ceil(T/16), 3, C) states entering every 16th step (forward: optional output)
+  // receptance (may be null): out = r wkv, and the backward returns gr
+  const void* r;
+  void* gr;
+  // the sequence in parts of `part` tokens (wkv4_parts); nz = 1: whole, no workspace
+  int64_t nz, part;
+  float* sums;      // workspace (B, nz-1, C, 4): the parts' summaries
+  float* maps;      // workspace (B, nz-1, 2, C, 4): the parts' cotangent maps
 };
+int64_t wkv4_parts(int64_t B, int64_t T, int64_t C, int64_t* part);
 
 // Residual addition + LayerNorm + token shift and interpolation (rwkv7_block.hip); tensors in the I/O dtype
 struct LnMixArgs {

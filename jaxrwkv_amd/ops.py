@@ -369,30 +369,81 @@ def wkv4_bwd(w_neg, u, k, v, s, length, new_starts, gy, gs_new=None, compat=True
     return gw.sum(0).to(io), gu.sum(0).to(io), gk, gv, gs
 
 
+def _workspace(nbytes, device):
+    return torch.empty(nbytes, dtype=torch.uint8, device=device)
+
+
+def _wkv4_mix_fwd(w, u, k, v, r, s, length, new_starts, flags, want_ckpt):
+    lib = _lib.load()
+    io = k.dtype
+    B, T, C = k.shape
+    assert s.shape == (B, 3, C) and w.shape == (C,) and u.shape == (C,)
+    y, new_s = torch.empty_like(k), torch.empty_like(s)
+    ckpt = _workspace(lib.hiprwkv_wkv4_bwd_workspace_bytes(B, T, C), k.device) if want_ckpt else None
+    nbytes = lib.hiprwkv_wkv4_mix_workspace_bytes(B, T, C)
+    ws = _workspace(nbytes, k.device) if nbytes else None
+    rc = lib.hiprwkv_wkv4_mix(_stream(), _DT[io], B, T, C, _p(w), _p(u), _p(k), _p(v), _p(r), _p(s), _p(length),
+                              _p(new_starts), _p(new_s), _p(y), _p(ckpt), ckpt.numel() if want_ckpt else 0, _p(ws), nbytes,
+                              flags)
+    _lib.check(rc, "hiprwkv_wkv4_mix")
+    return new_s, y, ckpt
+
+
 class _Wkv4(torch.autograd.Function):
-    """custom VJP, the counterpart of ``wkv4_cuda`` (rwkv4.py:379-383)."""
+    """custom VJP, the counterpart of ``wkv4_cuda`` (rwkv4.py:379-383), with the receptance where ``r`` is given."""
 
     @staticmethod
-    def forward(ctx, w_neg, u, k, v, s, length, new_starts, compat):
-        new_s, y, ckpt = wkv4_fwd(w_neg, u, k, v, s, length, new_starts, compat, want_ckpt=True)
-        ctx.compat = compat
-        ctx.save_for_backward(w_neg, u, k, v, s, length, new_starts, ckpt)
+    def forward(ctx, w, u, k, v, r, s, length, new_starts, flags):
+        io = k.dtype
+        k, v, s, w, u = (_dev(x, io) for x in (k, v, s, w, u))
+        r = None if r is None else _dev(r, io)
+        new_s, y, ckpt = _wkv4_mix_fwd(w, u, k, v, r, s, length, new_starts, flags, True)
+        ctx.flags = flags
+        ctx.save_for_backward(w, u, k, v, r, s, length, new_starts, ckpt)
+        ctx.set_materialize_grads(False)
         return new_s, y
 
     @staticmethod
     def backward(ctx, gs_new, gy):
-        w_neg, u, k, v, s, length, new_starts, ckpt = ctx.saved_tensors
-        if gy is None:
-            gy = torch.zeros_like(k)
-        gw, gu, gk, gv, gs = wkv4_bwd(w_neg, u, k, v, s, length, new_starts, gy, gs_new, ctx.compat, ckpt=ckpt)
-        return gw, gu, gk, gv, gs, None, None, None
+        w, u, k, v, r, s, length, new_starts, ckpt = ctx.saved_tensors
+        lib = _lib.load()
+        io = k.dtype
+        B, T, C = k.shape
+        gy = torch.zeros_like(k) if gy is None else _dev(gy, io)
+        gs_new = None if gs_new is None else _dev(gs_new, io)
+        gk, gv, gs = torch.empty_like(k), torch.empty_like(v), torch.empty_like(s)
+        gr = None if r is None else torch.empty_like(r)
+        gw, gu = torch.empty_like(w), torch.empty_like(u)
+        nbytes = lib.hiprwkv_wkv4_mix_bwd_workspace_bytes(B, T, C)
+        ws = _workspace(nbytes, k.device)
+        rc = lib.hiprwkv_wkv4_mix_bwd(_stream(), _DT[io], B, T, C, _p(w), _p(u), _p(k), _p(v), _p(r), _p(gy), _p(s),
+                                      _p(length), _p(new_starts), _p(gs_new), _p(ckpt), ckpt.numel(), _p(gw), _p(gu), _p(gk),
+                                      _p(gv), _p(gr), _p(gs), _p(ws), nbytes, ctx.flags | _lib.CKPT_READY)
+        _lib.check(rc, "hiprwkv_wkv4_mix_bwd")
+        return gw, gu, gk, gv, gr, gs, None, None, None
 
 
 def wkv4(w_neg, u, k, v, s, length=None, new_starts=None, compat=True):
     """Differentiable WKV4 in the op's convention (w_neg = -exp(time_decay), no receptance): returns (new_s, wkv)."""
     B, T = k.shape[:2]
     length, new_starts = _length_ns(length, new_starts, B, T, k.device)
-    return _Wkv4.apply(w_neg, u, k, v, s, length, new_starts, compat)
+    return _wkv4_apply(w_neg, u, k, v, None, s, length, new_starts, _flags(compat))
+
+
+def _wkv4_apply(w, u, k, v, r, s, length, new_starts, flags):
+    if torch.is_grad_enabled() and any(x is not None and x.requires_grad for x in (w, u, k, v, r, s)):
+        return _Wkv4.apply(w, u, k, v, r, s, length, new_starts, flags)
+    w, u, k, v, s = (_dev(x, k.dtype) for x in (w, u, k, v, s))
+    r = None if r is None else _dev(r, k.dtype)
+    return _wkv4_mix_fwd(w, u, k, v, r, s, length, new_starts, flags, False)[:2]
+
+
+def wkv4_mix(r, k, v, w, u, s, length=None, new_starts=None, compat=True):
+    """RWKV-4's ``inner_loop`` with a batch axis: the op with decay ``-exp(w)`` and its output times the receptance ``r``,
+    all tensors in one dtype.  Returns (new_s, r wkv); differentiable in r, k, v, w, u and s."""
+    B, T = k.shape[:2]
+    length, new_starts = _length_ns(length, new_starts, B, T, k.device)
+    return _wkv4_apply(w, u, k, v, r, s, length, new_starts, _flags(compat) | _lib.W_RAW)
 
 
 # ----------------------------------------------------------------------------- RWKV-7 time-mixing stages
