@@ -66,6 +66,8 @@ extern "C" {
 /* hiprwkv_wkv4_bwd: the workspace already holds the checkpoints that hiprwkv_wkv4_fwd_ckpt wrote for the same
  * inputs; the backward then skips its own first pass over k and v. */
 #define HIPRWKV_CKPT_READY 0x20u
+/* `length` holds int32 values, and a negative one counts as 0 (without the flag: uint32). */
+#define HIPRWKV_LENGTH_I32 0x40u
 /* hiprwkv_wkv4_*: `w` is the parameter time_decay itself; the op's decay is -exp(w), rounded to io_dtype
  * (rwkv4.py:312), and the cotangent returned is the one of w. */
 #define HIPRWKV_W_RAW 0x80u
@@ -75,7 +77,7 @@ extern "C" {
 #define HIPRWKV_DEBUG_DROP_PUBLISH 0x100u
 /* Every flag a production caller may pass.  Entry points refuse other bits, and refuse HIPRWKV_DEBUG_DROP_PUBLISH
  * unless the process runs with HIPRWKV_ENABLE_DEBUG_FLAGS=1 in its environment. */
-#define HIPRWKV_PUBLIC_FLAGS (HIPRWKV_COMPAT_ASSOC | HIPRWKV_FORCE_SEQ | HIPRWKV_NO_SMALL_T | HIPRWKV_W_PER_HEAD | HIPRWKV_CKPT_READY | HIPRWKV_W_RAW)
+#define HIPRWKV_PUBLIC_FLAGS (HIPRWKV_COMPAT_ASSOC | HIPRWKV_FORCE_SEQ | HIPRWKV_NO_SMALL_T | HIPRWKV_W_PER_HEAD | HIPRWKV_CKPT_READY | HIPRWKV_LENGTH_I32 | HIPRWKV_W_RAW)
 
 typedef void* hiprwkv_stream; /* a hipStream_t */
 

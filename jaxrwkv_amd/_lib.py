@@ -14,9 +14,10 @@ FORCE_SEQ = 2
 NO_SMALL_T = 4
 W_PER_HEAD = 0x10
 CKPT_READY = 0x20
+LENGTH_I32 = 0x40
 W_RAW = 0x80
 DEBUG_DROP_PUBLISH = 0x100      # refused unless the process runs with HIPRWKV_ENABLE_DEBUG_FLAGS=1
-PUBLIC_FLAGS = COMPAT_ASSOC | FORCE_SEQ | NO_SMALL_T | W_PER_HEAD | CKPT_READY | W_RAW
+PUBLIC_FLAGS = COMPAT_ASSOC | FORCE_SEQ | NO_SMALL_T | W_PER_HEAD | CKPT_READY | LENGTH_I32 | W_RAW
 
 _vp, _i64, _int, _u32, _sz = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_uint, ctypes.c_size_t
 

@@ -17,6 +17,14 @@ __device__ __forceinline__ float ld_f(const bf16_t* p) { return bf16_to_f32(p->b
 __device__ __forceinline__ void st_f(float* p, float x) { *p = x; }
 __device__ __forceinline__ void st_f(bf16_t* p, float x) { p->bits = f32_to_bf16(x); }
 
+// Tokens of sequence b that count: at most T.  FLAG_LENGTH_I32 (HIPRWKV_LENGTH_I32): the array is int32, negative = 0.
+constexpr unsigned FLAG_LENGTH_I32 = 0x40u;
+__device__ __forceinline__ int64_t seq_length(const uint32_t* length, int64_t b, int64_t T, unsigned flags) {
+  if (length == nullptr) return T;
+  const uint32_t L = length[b];
+  return (flags & FLAG_LENGTH_I32) && (int32_t)L < 0 ? 0 : (int64_t)L;
+}
+
 // 8 consecutive elements <-> 8 floats (pointer must be 16-byte aligned for bf16, 32 for fp32)
 __device__ __forceinline__ void ld8(const float* p, float (&o)[8]) {
   float4 a = *reinterpret_cast<const float4*>(p);

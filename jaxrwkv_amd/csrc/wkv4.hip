@@ -158,7 +158,7 @@ __global__ __launch_bounds__(W4_THREADS) void wkv4_fwd_kernel(Wkv4Args A) {
   const float u = ld_f(reinterpret_cast<const IO*>(A.u) + cc);
   float aa, bb, pp;
   entering_state<IO>(A, P, w, aa, bb, pp);
-  int64_t L = A.length ? (int64_t)A.length[b] : A.T;
+  int64_t L = seq_length(A.length, b, A.T, A.flags);
   L = L < A.T ? L : A.T;
   const bool q2drop = (A.flags & 1u) && L < A.T && A.ns != nullptr && A.ns[(size_t)b * A.T + L] != 0;
   auto snapshot = [&]() {
@@ -411,7 +411,7 @@ __global__ __launch_bounds__(W4_THREADS) void wkv4_bwd_kernel(Wkv4Args A) {
   const float u = ld_f(reinterpret_cast<const IO*>(A.u) + c);
   const int voff = (int)(c * sizeof(IO));
   const int stride = (int)(A.C * sizeof(IO));
-  int64_t L = A.length ? (int64_t)A.length[b] : A.T;
+  int64_t L = seq_length(A.length, b, A.T, A.flags);
   L = L < A.T ? L : A.T;
   const bool q2drop = (A.flags & 1u) && L < A.T && ns != nullptr && ns[L] != 0;
   float inj_a = 0.f, inj_b = 0.f, inj_p = 0.f;   // cotangent of the returned state

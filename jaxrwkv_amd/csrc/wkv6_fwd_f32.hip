@@ -403,7 +403,7 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv6_fwd_f32_kernel(Wkv6
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int64_t b = blockIdx.x / A.H, h = blockIdx.x % A.H;
-  int64_t L = A.length ? (int64_t)A.length[b] : A.T;
+  int64_t L = seq_length(A.length, b, A.T, A.flags);
   L = L < A.T ? L : A.T;
   const int nch = (int)((A.T + CK - 1) / CK);
   if (threadIdx.x < sizeof(Sync) / sizeof(int)) reinterpret_cast<int*>(sy)[threadIdx.x] = 0;

@@ -42,7 +42,7 @@ __device__ __forceinline__ Ids6 ids6(const Wkv6Args& A) {
   id.h = blockIdx.x % A.H;
   id.line = threadIdx.x >> 2;
   id.q = threadIdx.x & 3;
-  int64_t L = A.length ? (int64_t)A.length[id.b] : A.T;
+  int64_t L = seq_length(A.length, id.b, A.T, A.flags);
   id.L = L < A.T ? L : A.T;
   id.q2drop = (A.flags & 1u) && id.L < A.T && A.ns != nullptr && A.ns[id.b * A.T + id.L] != 0;
   return id;

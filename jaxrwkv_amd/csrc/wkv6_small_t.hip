@@ -29,7 +29,7 @@ template <typename IO, typename ST>
 __global__ __launch_bounds__(256) void wkv6_small_t_kernel(Wkv6Args A) {
   const int64_t b = blockIdx.x / A.H, h = blockIdx.x % A.H;
   const int j = threadIdx.x >> 2, q = threadIdx.x & 3, c0 = 16 * q;
-  int64_t L = A.length ? (int64_t)A.length[b] : A.T;
+  int64_t L = seq_length(A.length, b, A.T, A.flags);
   L = L < A.T ? L : A.T;
   const uint8_t* ns = A.ns ? A.ns + b * A.T : nullptr;
   // the returned state is the reset state there (associative-scan rule)

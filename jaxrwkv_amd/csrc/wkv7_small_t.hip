@@ -30,7 +30,7 @@ template <typename IO, typename ST>
 __global__ __launch_bounds__(256) void wkv7_small_t_kernel(Wkv7Args A) {
   const int64_t b = blockIdx.x / A.H, h = blockIdx.x % A.H;
   const int i = threadIdx.x >> 2, q = threadIdx.x & 3, c0 = 16 * q;
-  int64_t L = A.length ? (int64_t)A.length[b] : A.T;
+  int64_t L = seq_length(A.length, b, A.T, A.flags);
   L = L < A.T ? L : A.T;
   const bool compat = (A.flags & 1u) != 0;
   const uint8_t* ns = A.ns ? A.ns + b * A.T : nullptr;

@@ -17,7 +17,7 @@ _SA_DT = {torch.float32: torch.float32, torch.bfloat16: torch.float16}   # type 
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _p(t):
@@ -49,9 +49,9 @@ def _phase(t):
 def _empty_phased(shape, dtype, device, phase):
     """An uninitialised contiguous tensor whose address is ``phase`` 128-byte steps past a 1 KiB boundary (a view
     into a buffer 1 KiB larger); small tensors are allocated plainly."""
-    n = torch.empty((), dtype=dtype).element_size()
+    n = dtype.itemsize
     for d in shape:
-        n *= int(d)
+        n *= d
     if n < _PHASED_MIN_BYTES:
         return torch.empty(shape, dtype=dtype, device=device)
     buf = torch.empty(n + _PHASE_BYTES * _PHASES, dtype=torch.uint8, device=device)
@@ -64,15 +64,25 @@ def _empty_like_phased(ref, steps):
     return _empty_phased(tuple(ref.shape), ref.dtype, ref.device, _phase(ref) + steps)
 
 
-def _length_ns(length, new_starts, B, T, device):
+def _length_ns(length, new_starts, B, T, device, keep=False):
+    """``length`` as a contiguous (B,) int32 tensor (the kernels count a negative length as 0) and ``new_starts`` as a
+    contiguous (B,T) bool one.  ``keep``: for a backward pass to come, so that ``length`` is never the caller's own memory."""
     if length is not None:
-        length = torch.as_tensor(length, device=device).to(torch.int32).reshape(-1)
+        if not torch.is_tensor(length) or length.device != device:
+            length = torch.as_tensor(length, device=device)
+        given = length
+        if length.dtype != torch.int32:
+            length = length.to(torch.int32)
+        length = length.reshape(-1)
         if length.numel() == 1 and B > 1:
             length = length.expand(B)
-        length = length.clamp(min=0).contiguous()
+        length = length.contiguous()
         assert length.numel() == B
+        if keep and length.data_ptr() == given.data_ptr():
+            length = length.clone()
     if new_starts is not None:
-        new_starts = torch.as_tensor(new_starts, device=device).to(torch.bool)
+        if not torch.is_tensor(new_starts) or new_starts.device != device or new_starts.dtype != torch.bool:
+            new_starts = torch.as_tensor(new_starts, device=device).to(torch.bool)
         if new_starts.dim() == 1:
             new_starts = new_starts[None].expand(B, T)
         new_starts = new_starts.contiguous()
@@ -80,8 +90,12 @@ def _length_ns(length, new_starts, B, T, device):
     return length, new_starts
 
 
+def _needs_grad(*tensors):
+    return torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
+
+
 def _flags(compat, force_seq=False, small_t=True, debug=0):
-    return ((_lib.COMPAT_ASSOC if compat else 0) | (_lib.FORCE_SEQ if force_seq else 0)
+    return (_lib.LENGTH_I32 | (_lib.COMPAT_ASSOC if compat else 0) | (_lib.FORCE_SEQ if force_seq else 0)
             | (0 if small_t else _lib.NO_SMALL_T) | int(debug))
 
 
@@ -208,7 +222,9 @@ class _Wkv7(torch.autograd.Function):
 def wkv7(r, w, k, v, a, b, s, length=None, new_starts=None, compat=True, force_seq=False):
     """Differentiable WKV7: returns (new_s, y).  ``force_seq`` runs the sequential fp32 kernels whatever the dtype."""
     B, T = r.shape[:2]
-    length, new_starts = _length_ns(length, new_starts, B, T, r.device)
+    if not _needs_grad(r, w, k, v, a, b, s):
+        return wkv7_fwd(r, w, k, v, a, b, s, length, new_starts, compat, force_seq=force_seq)[:2]
+    length, new_starts = _length_ns(length, new_starts, B, T, r.device, keep=True)
     return _Wkv7.apply(r, w, k, v, a, b, s, length, new_starts, compat, force_seq)
 
 
@@ -313,7 +329,9 @@ class _Wkv6(torch.autograd.Function):
 def wkv6(r, k, v, w, u, s, length=None, new_starts=None, compat=True, force_seq=False):
     """Differentiable WKV6: returns (new_s, y).  ``force_seq`` runs the sequential fp32 kernels whatever the dtype."""
     B, T = r.shape[:2]
-    length, new_starts = _length_ns(length, new_starts, B, T, r.device)
+    if not _needs_grad(r, k, v, w, u, s):
+        return wkv6_fwd(r, k, v, w, u, s, length, new_starts, compat, force_seq=force_seq)
+    length, new_starts = _length_ns(length, new_starts, B, T, r.device, keep=True)
     return _Wkv6.apply(r, k, v, w, u, s, length, new_starts, compat, force_seq)
 
 
@@ -425,13 +443,14 @@ class _Wkv4(torch.autograd.Function):
 
 def wkv4(w_neg, u, k, v, s, length=None, new_starts=None, compat=True):
     """Differentiable WKV4 in the op's convention (w_neg = -exp(time_decay), no receptance): returns (new_s, wkv)."""
-    B, T = k.shape[:2]
-    length, new_starts = _length_ns(length, new_starts, B, T, k.device)
     return _wkv4_apply(w_neg, u, k, v, None, s, length, new_starts, _flags(compat))
 
 
 def _wkv4_apply(w, u, k, v, r, s, length, new_starts, flags):
-    if torch.is_grad_enabled() and any(x is not None and x.requires_grad for x in (w, u, k, v, r, s)):
+    B, T = k.shape[:2]
+    grad = _needs_grad(w, u, k, v, s) or (r is not None and _needs_grad(r))
+    length, new_starts = _length_ns(length, new_starts, B, T, k.device, keep=grad)
+    if grad:
         return _Wkv4.apply(w, u, k, v, r, s, length, new_starts, flags)
     w, u, k, v, s = (_dev(x, k.dtype) for x in (w, u, k, v, s))
     r = None if r is None else _dev(r, k.dtype)
@@ -441,8 +460,6 @@ def _wkv4_apply(w, u, k, v, r, s, length, new_starts, flags):
 def wkv4_mix(r, k, v, w, u, s, length=None, new_starts=None, compat=True):
     """RWKV-4's ``inner_loop`` with a batch axis: the op with decay ``-exp(w)`` and its output times the receptance ``r``,
     all tensors in one dtype.  Returns (new_s, r wkv); differentiable in r, k, v, w, u and s."""
-    B, T = k.shape[:2]
-    length, new_starts = _length_ns(length, new_starts, B, T, k.device)
     return _wkv4_apply(w, u, k, v, r, s, length, new_starts, _flags(compat) | _lib.W_RAW)
 
 
