@@ -333,13 +333,30 @@ int hiprwkv_rwkv7_pre(hiprwkv_stream stream, int io_dtype, int64_t rows, int64_t
                       void* v_out, void* a_out, void* b_out);
 size_t hiprwkv_rwkv7_pre_bwd_workspace_bytes(int64_t rows, int64_t H, int64_t N);
 /* From the cotangents of w, k_out, v_out, a_out, b_out to those of the inputs; dparam: (H, 64) io_dtype arrays of w0, a0,
- * k_k, k_a and, with v_first, v0. */
+ * k_k, k_a and, with v_first, v0.  gk_out2, gv_out2 (may be NULL) are added to gk_out and gv_out; dr (may be NULL) = gr + gr2:
+ * r, k_out and v_out have a second use after the op. */
 int hiprwkv_rwkv7_pre_bwd(hiprwkv_stream stream, int io_dtype, int64_t rows, int64_t H, int64_t N, const void* xw,
                           const void* k, const void* xa, const void* v, const void* v_first, const void* xv,
                           const void* w0, const void* a0, const void* v0, const void* k_k, const void* k_a,
                           const void* gw, const void* gk_out, const void* gv_out, const void* ga_out,
-                          const void* gb_out, void* dxw, void* dk, void* dv, void* dv_first, void* dxv, void* dxa,
+                          const void* gb_out, const void* gk_out2, const void* gv_out2, const void* gr, const void* gr2,
+                          void* dr, void* dxw, void* dk, void* dv, void* dv_first, void* dxv, void* dxa,
                           void* const* dparam, void* workspace, size_t workspace_bytes);
+
+/* ---- Several narrow products in one launch -------------------------------------------------------------
+ * bf16, fp32 accumulation: out[m][n] = f(sum_k x(m, k) w(n, k)), out (M, N) row-major.  x is (M, K) row-major, with km its
+ * transpose (K, M); w is (N, K), with kn (K, N).  For the low-rank factors of RWKV-7's decay, gates and value residual
+ * (rwkv7.py:237-245) and their cotangents.  f: without aux 0 none, 1 tanh, 2 sigmoid, 3 relu(.)^2; with aux, an (M, N) array:
+ * 0 + aux, 1 times 1 - aux^2, 2 times aux (1 - aux) (the derivatives in terms of the activations' values).  Sizes that are
+ * contiguous in memory must be multiples of 8. */
+#define HIPRWKV_GEMM_MAX_JOBS 8
+typedef struct hiprwkv_gemm_job {
+  const void *x, *w, *aux;
+  void* out;
+  int32_t M, N, K, km, kn, act;
+  int32_t tile0, pad;      /* used by the library */
+} hiprwkv_gemm_job;
+int hiprwkv_gemm(hiprwkv_stream stream, int n_jobs, const hiprwkv_gemm_job* jobs);
 
 /* ---- RWKV-7: a decode step of the whole model ---------------------------------------------------------
  * rwkv7.py:190-198, :223-291 for at most HIPRWKV_SMALL_T tokens per sequence and HIPRWKV_DECODE_MAX_ROWS tokens in all, bf16
@@ -394,6 +411,15 @@ int hiprwkv_rwkv7_postmix_bwd(hiprwkv_stream stream, int io_dtype, int64_t rows,
                               const void* ln_w, const void* ln_b, const void* r_k, float eps, const void* gout,
                               void* gy, void* gr, void* gk, void* gv, void* gg,
                               float* gln_w, float* gln_b, float* gr_k);
+
+/* hiprwkv_rwkv7_postmix_bwd with the parameter cotangents as three (H, 64) io_dtype arrays, dparam = ln_w, ln_b, r_k, summed
+ * through `workspace` instead of atomics. */
+size_t hiprwkv_rwkv7_postmix_bwd2_workspace_bytes(int64_t rows, int64_t H, int64_t N);
+int hiprwkv_rwkv7_postmix_bwd2(hiprwkv_stream stream, int io_dtype, int64_t rows, int64_t H, int64_t N,
+                               const void* y, const void* r, const void* k, const void* v, const void* g,
+                               const void* ln_w, const void* ln_b, const void* r_k, float eps, const void* gout,
+                               void* gy, void* gr, void* gk, void* gv, void* gg, void* const* dparam, void* workspace,
+                               size_t workspace_bytes);
 
 #ifdef __cplusplus
 }

@@ -33,6 +33,12 @@ class Rwkv7DecodeArgs(ctypes.Structure):
                 + [("workspace_bytes", ctypes.c_uint64), ("flags", ctypes.c_uint64)])
 
 
+class GemmJob(ctypes.Structure):
+    """``hiprwkv_gemm_job``"""
+    _fields_ = ([(n, _vp) for n in ("x", "w", "aux", "out")]
+                + [(n, ctypes.c_int32) for n in ("M", "N", "K", "km", "kn", "act", "tile0", "pad")])
+
+
 # name -> (restype, argtypes); mirrors include/hiprwkv.h declaration by declaration
 SIGNATURES = {
     "hiprwkv_last_error": (ctypes.c_char_p, []),
@@ -79,7 +85,10 @@ SIGNATURES = {
     "hiprwkv_rwkv7_ln_shiftmix_bwd": (_int, [_vp, _int, _i64, _i64, _i64, _int] + [_vp] * 5 + [_i64] + [_vp] * 10 + [_sz]),
     "hiprwkv_rwkv7_pre": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 16),
     "hiprwkv_rwkv7_pre_bwd_workspace_bytes": (_sz, [_i64] * 3),
-    "hiprwkv_rwkv7_pre_bwd": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 24 + [_sz]),
+    "hiprwkv_rwkv7_pre_bwd": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 29 + [_sz]),
+    "hiprwkv_rwkv7_postmix_bwd2_workspace_bytes": (_sz, [_i64] * 3),
+    "hiprwkv_rwkv7_postmix_bwd2": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 8 + [ctypes.c_float] + [_vp] * 8 + [_sz]),
+    "hiprwkv_gemm": (_int, [_vp, _int, ctypes.POINTER(GemmJob)]),
     "hiprwkv_rwkv7_decode_workspace_bytes": (_sz, [ctypes.POINTER(Rwkv7DecodeArgs)]),
     "hiprwkv_rwkv7_decode": (_int, [_vp, ctypes.POINTER(Rwkv7DecodeArgs)]),
     "hiprwkv_rwkv7_premix": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 7),

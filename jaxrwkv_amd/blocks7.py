@@ -1,0 +1,333 @@
+"""The stack of RWKV-7 blocks as one operator over whole sequences, with and without autograd (rwkv7.py:190-198, 223-291).
+
+Autograd over the single steps spends longer on the host than the GPU needs for a training step of a small model (0.1B shape,
+B=4 T=512: about 1000 launches, 23 ms against 13 ms of GPU time).  Here the whole stack is one node: the backward is
+written out over the library's kernels and ``torch.mm``, writes every layer's parameter cotangents into their place in the
+stacked arrays, and adds up nothing that a kernel can add on its way (the second cotangents of r, k and v, the value
+residual's).  The low-rank factors of decay, gates and value residual run several to a launch (``hiprwkv_gemm``) in bf16.
+"""
+import torch
+
+from . import _lib, ops
+from .rwkv7 import HipRWKV
+
+#: parameter name -> path inside params["blocks"]; the order of the operator's arguments
+PATHS = {n: ("att", n) for n in ("x_r", "x_w", "x_k", "x_v", "x_a", "x_g", "w0", "w1", "w2", "a0", "a1", "a2", "v0", "v1", "v2",
+                                 "g1", "g2", "k_k", "k_a", "r_k")}
+PATHS.update({n: ("att", n, "weight") for n in ("receptance", "key", "value", "output")})
+PATHS.update(lnx_w=("att", "ln_x", "weight"), lnx_b=("att", "ln_x", "bias"), ffn_x_k=("ffn", "x_k"),
+             ffn_key=("ffn", "key", "weight"), ffn_value=("ffn", "value", "weight"), ln1_w=("ln1", "weight"),
+             ln1_b=("ln1", "bias"), ln2_w=("ln2", "weight"), ln2_b=("ln2", "bias"))
+NAMES = tuple(PATHS)
+MIX = ("x_r", "x_w", "x_k", "x_v", "x_a", "x_g")
+EPS_X = 64e-5
+_NONE, _TANH, _SIGMOID = 0, 1, 2             # hiprwkv_gemm_job.act without aux; with aux: add, tanh', sigmoid'
+_LORA = (("w", _TANH), ("a", _NONE), ("g", _SIGMOID), ("v", _NONE))
+
+
+def gather(blocks):
+    out = []
+    for path in PATHS.values():
+        t = blocks
+        for p in path:
+            t = t[p]
+        out.append(t)
+    return out
+
+
+def _gemm(jobs):
+    """Several products in one launch: (out, x, w, km, kn, act, aux) with out (M, N), x (M, K) or, km, (K, M), w (N, K) or,
+    kn, (K, N)."""
+    arr = (_lib.GemmJob * len(jobs))()
+    for j, (out, x, w, km, kn, act, aux) in zip(arr, jobs):
+        j.out, j.x, j.w, j.aux = out.data_ptr(), x.data_ptr(), w.data_ptr(), None if aux is None else aux.data_ptr()
+        j.M, j.N = out.shape
+        j.K = x.shape[0] if km else x.shape[1]
+        j.km, j.kn, j.act = km, kn, act
+    _lib.check(_lib.load().hiprwkv_gemm(ops._stream(), len(jobs), arr), "hiprwkv_gemm")
+
+
+def _grouped(p):
+    """Whether the grouped products take the low-rank factors: bf16, inner sizes multiples of 8."""
+    return p["w1"].dtype == torch.bfloat16 and all(p[n].shape[-1] % 8 == 0 for n in ("w1", "a1", "v1", "g1"))
+
+
+def _lora_fwd(p, mix, names, like):
+    """Hidden values (activation applied) and results of the low-rank terms ``names``; mix: name -> (M, C) input."""
+    hid, out = {}, {}
+    if _grouped(p):
+        M, C = like.shape
+        for n, _ in names:
+            hid[n] = torch.empty((M, p[n + "1"].shape[-1]), dtype=like.dtype, device=like.device)
+            out[n] = torch.empty_like(like)
+        _gemm([(hid[n], mix[n], p[n + "1"], 0, 1, act, None) for n, act in names])
+        _gemm([(out[n], hid[n], p[n + "2"], 0, 1, _NONE, None) for n, _ in names])
+        return hid, out
+    for n, act in names:
+        h = mix[n] @ p[n + "1"]
+        hid[n] = torch.tanh_(h) if act == _TANH else torch.sigmoid_(h) if act == _SIGMOID else h
+        out[n] = hid[n] @ p[n + "2"]
+    return hid, out
+
+
+def _lora_bwd(p, grad, mix, hid, gout, dmix, names):
+    """From the cotangents ``gout`` of the low-rank terms: the parameters' cotangents into ``grad`` and the inputs' into
+    ``dmix`` (the value residual's is added to what is there)."""
+    if _grouped(p):
+        dh = {n: torch.empty_like(hid[n]) for n, _ in names}
+        _gemm([(dh[n], gout[n], p[n + "2"], 0, 0, act, hid[n] if act else None) for n, act in names])
+        _gemm([(dmix[n], dh[n], p[n + "1"], 0, 0, 0, dmix[n] if n == "v" else None) for n, _ in names])
+        _gemm([(grad[n + "1"], mix[n], dh[n], 1, 1, _NONE, None) for n, _ in names]
+              + [(grad[n + "2"], hid[n], gout[n], 1, 1, _NONE, None) for n, _ in names])
+        return
+    for n, act in names:
+        torch.mm(hid[n].T, gout[n], out=grad[n + "2"])
+        dh = gout[n] @ p[n + "2"].T
+        if act == _TANH:
+            dh = torch.ops.aten.tanh_backward(dh, hid[n])
+        elif act == _SIGMOID:
+            dh = torch.ops.aten.sigmoid_backward(dh, hid[n])
+        torch.mm(mix[n].T, dh, out=grad[n + "1"])
+        if n == "v":
+            dmix[n].addmm_(dh, p[n + "1"].T)
+        else:
+            torch.mm(dh, p[n + "1"].T, out=dmix[n])
+
+
+def _ln_mix(p, x, dx, ln, state_row, ns, length, mix, shift_out, keep):
+    """``rwkv7_ln_shiftmix`` on (B,T,C) without autograd; ``keep``: also the statistics for the backward."""
+    B, T, C = x.shape
+    stats = torch.empty((B * T, 2), dtype=torch.float32, device=x.device) if keep else None
+    prev, stride = ops._shift_row(state_row, B, C, x.dtype)
+    xs, outs = ops._ln_shiftmix_fwd(x, dx, p[ln + "_w"], p[ln + "_b"], 1e-5, prev, stride, ns, length,
+                                    [p[n] for n in mix], shift_out, stats)
+    return xs, outs, (stats, prev, stride)
+
+
+def _layer_fwd(i, p, x, dx, st, nst, v_first, ns, length, keep):
+    """One block on x (B,T,C) (+ dx): returns (x, dx, v_first, saved tensors).  st, nst: the layer's rows of the model
+    states."""
+    B, T, C = x.shape
+    H, N = p["r_k"].shape
+    M = B * T
+    flat = lambda t: t.view(M, -1)
+    heads = lambda t: t.view(B, T, H, N)
+    x, outs, head1 = _ln_mix(p, x, dx, "ln1", st[:, 1], ns, length, MIX, nst[:, 1], keep)
+    xr, xw, xk, xv, xa, xg = map(flat, outs)
+    r, k, v = (torch.mm(a, p[n].T) for a, n in ((xr, "receptance"), (xk, "key"), (xv, "value")))
+    mix = {"w": xw, "a": xa, "g": xg, "v": xv}
+    hid, lora = _lora_fwd(p, mix, _LORA if i else _LORA[:3], r)
+    if i == 0:
+        v_first = v
+    par = lambda n: p[n].reshape(C)
+    pre = ops._pre_fwd(heads(lora["w"]), heads(k), heads(lora["a"]), heads(v), heads(v_first) if i else None,
+                       heads(lora["v"]) if i else None, par("w0"), par("a0"), par("v0") if i else None, par("k_k"), par("k_a"))
+    w, k2, v2, a, b = pre
+    if i == 0:
+        v2 = heads(v)
+    s = st[:, 2:].reshape(B, H, N, N)
+    new_s, yw, sa = ops.wkv7_fwd(heads(r), w, k2, v2, a, b, s, length, ns, HipRWKV.assoc_compat, want_sa=keep)
+    nst[:, 2:] = new_s.view(B, N, C)
+    y = flat(ops._postmix_fwd(yw, heads(r), k2, v2, heads(lora["g"]), par("lnx_w"), par("lnx_b"), par("r_k"), EPS_X))
+    dx1 = torch.mm(y, p["output"].T).view(B, T, C)
+    x2, (xk2,), head2 = _ln_mix(p, x, dx1, "ln2", st[:, 0], ns, length, ("ffn_x_k",), nst[:, 0], keep)
+    ff = torch.mm(flat(xk2), p["ffn_key"].T)
+    fr = ops._relusq_fwd(ff)
+    dx2 = torch.mm(fr, p["ffn_value"].T).view(B, T, C)
+    saved = None
+    if keep:
+        saved = dict(x=x, head1=head1, xr=xr, xk=xk, mix=mix, r=r, k=k, v=v, hid=hid, lora=lora, w=w, k2=k2, v2=v2, a=a, b=b,
+                     s=s, sa=sa, yw=yw, y=y, x2=x2, head2=head2, xk2=xk2, ff=ff, fr=fr)
+    return x2, dx2, v_first, saved
+
+
+def _ln_mix_bwd(p, grad, xs, head, ln, ns, length, mix, gs, gx, gshift, need_prev):
+    lib = _lib.load()
+    stats, prev, stride = head
+    io = xs.dtype
+    B, T, C = xs.shape
+    dxs = torch.empty_like(xs)
+    dprev = torch.empty((B, C), dtype=io, device=xs.device) if need_prev else None
+    params = [p[n] for n in mix]
+    nbytes = lib.hiprwkv_rwkv7_ln_shiftmix_bwd_workspace_bytes(B, T, C, len(mix))
+    ws = ops._workspace(nbytes, xs.device)
+    rc = lib.hiprwkv_rwkv7_ln_shiftmix_bwd(
+        ops._stream(), ops._DT[io], B, T, C, len(mix), ops._p(xs), ops._p(stats), ops._p(p[ln + "_w"]), ops._p(p[ln + "_b"]),
+        ops._p(prev), stride, ops._p(ns), ops._p(length), ops._ptr_array(params), ops._ptr_array(gs), ops._p(gx), ops._p(gshift),
+        ops._p(dxs), ops._p(dprev), ops._ptr_array([grad[n] for n in mix] + [grad[ln + "_w"], grad[ln + "_b"]]), ops._p(ws), nbytes)
+    _lib.check(rc, "hiprwkv_rwkv7_ln_shiftmix_bwd")
+    return dxs, dprev
+
+
+def _layer_bwd(i, p, grad, S, ns, length, g_x, g_dx, g_state, g_in, g_vfirst, v_first):
+    """The cotangents of one block: g_x, g_dx of what it returns, g_state (or None) of its rows of the new model state (B,66,C).
+    Fills ``grad`` (the layer's slices of the stacked cotangents) and ``g_in`` (or None), the cotangent of its rows of the input
+    state; accumulates ``g_vfirst``.  Returns the cotangent of its input x (and of the dx added to it) and g_vfirst."""
+    lib = _lib.load()
+    x, x2 = S["x"], S["x2"]
+    B, T, C = x.shape
+    H, N = p["r_k"].shape
+    M = B * T
+    io = x.dtype
+    flat = lambda t: t.view(M, -1)
+    heads = lambda t: t.view(B, T, H, N)
+    row = lambda j: None if g_state is None else g_state[:, j].contiguous()
+    # channel mixing
+    g2 = flat(g_dx)
+    torch.mm(g2.T, S["fr"], out=grad["ffn_value"])
+    gf = torch.mm(g2, p["ffn_value"])
+    gff = torch.empty_like(gf)
+    _lib.check(lib.hiprwkv_rwkv7_relusq_bwd(ops._stream(), ops._DT[io], gf.numel(), ops._p(S["ff"]), ops._p(gf), ops._p(gff)),
+               "hiprwkv_rwkv7_relusq_bwd")
+    torch.mm(gff.T, flat(S["xk2"]), out=grad["ffn_key"])
+    gxk2 = torch.mm(gff, p["ffn_key"]).view(B, T, C)
+    dx2, dprev = _ln_mix_bwd(p, grad, x2, S["head2"], "ln2", ns, length, ("ffn_x_k",), [gxk2], g_x, row(0), g_in is not None)
+    if g_in is not None:
+        g_in[:, 0] = dprev
+    # time mixing: output projection, group norm and gate
+    g1 = flat(dx2)
+    torch.mm(g1.T, S["y"], out=grad["output"])
+    gy = torch.mm(g1, p["output"])
+    e = lambda: torch.empty((B, T, H, N), dtype=io, device=x.device)
+    gyw, gr1, gk1, gv1, gg = (e() for _ in range(5))
+    nbytes = lib.hiprwkv_rwkv7_postmix_bwd2_workspace_bytes(M, H, N)
+    ws = ops._workspace(nbytes, x.device)
+    rc = lib.hiprwkv_rwkv7_postmix_bwd2(
+        ops._stream(), ops._DT[io], M, H, N, ops._p(S["yw"]), ops._p(S["r"]), ops._p(S["k2"]), ops._p(S["v2"]),
+        ops._p(S["lora"]["g"]), ops._p(p["lnx_w"]), ops._p(p["lnx_b"]), ops._p(p["r_k"]), EPS_X, ops._p(gy), ops._p(gyw),
+        ops._p(gr1), ops._p(gk1), ops._p(gv1), ops._p(gg),
+        ops._ptr_array([grad["lnx_w"], grad["lnx_b"], grad["r_k"]]), ops._p(ws), nbytes)
+    _lib.check(rc, "hiprwkv_rwkv7_postmix_bwd2")
+    # the recurrence
+    gs_out = None if g_state is None else g_state[:, 2:].reshape(B, H, N, N)
+    gr2, gw, gk2, gv2, ga, gb, gs = ops.wkv7_bwd(heads(S["r"]), S["w"], S["k2"], S["v2"], S["a"], S["b"], S["s"], length, ns,
+                                                 gyw, S["sa"], gs_out, HipRWKV.assoc_compat)
+    if g_in is not None:
+        g_in[:, 2:] = gs.reshape(B, N, C)
+    # gates
+    par = lambda n: p[n].reshape(C)
+    lora, dxw, dk, dxa, gr = S["lora"], e(), e(), e(), e()
+    names = _LORA if i else _LORA[:3]
+    if i:
+        dv, dvf, dxv = e(), e(), e()
+    else:
+        dv, dvf, dxv = gv1.add_(gv2), None, None
+        if g_vfirst is not None:
+            dv.add_(g_vfirst)
+    nbytes = lib.hiprwkv_rwkv7_pre_bwd_workspace_bytes(M, H, N)
+    ws = ops._workspace(nbytes, x.device)
+    P = ops._p
+    rc = lib.hiprwkv_rwkv7_pre_bwd(
+        ops._stream(), ops._DT[io], M, H, N, P(lora["w"]), P(S["k"]), P(lora["a"]), P(S["v"]), P(v_first) if i else None,
+        P(lora["v"]) if i else None, P(par("w0")), P(par("a0")), P(par("v0")) if i else None, P(par("k_k")), P(par("k_a")),
+        P(gw), P(gk1), P(gv1) if i else None, P(ga), P(gb), P(gk2), P(gv2) if i else None, P(gr1), P(gr2), P(gr),
+        P(dxw), P(dk), P(dv) if i else None, P(dvf), P(dxv), P(dxa),
+        ops._ptr_array([grad[n] for n in ("w0", "a0", "k_k", "k_a", "v0")]), P(ws), nbytes)
+    _lib.check(rc, "hiprwkv_rwkv7_pre_bwd")
+    if i:
+        g_vfirst = dvf if g_vfirst is None else g_vfirst.add_(dvf)
+    # projections
+    gr, dk, dv = flat(gr), flat(dk), flat(dv)
+    mix = S["mix"]
+    for g, a, n in ((gr, S["xr"], "receptance"), (dk, S["xk"], "key"), (dv, mix["v"], "value")):
+        torch.mm(g.T, a, out=grad[n])
+    dxr, dxk, dxv_ = torch.mm(gr, p["receptance"]), torch.mm(dk, p["key"]), torch.mm(dv, p["value"])
+    dmix = {n: torch.empty_like(dxr) for n in ("w", "a", "g")}
+    dmix["v"] = dxv_
+    gout = {"w": flat(dxw), "a": flat(dxa), "g": flat(gg)}
+    if i:
+        gout["v"] = flat(dxv)
+    _lora_bwd(p, grad, mix, S["hid"], gout, dmix, names)
+    gmix = [t.view(B, T, C) for t in (dxr, dmix["w"], dxk, dxv_, dmix["a"], dmix["g"])]
+    dx, dprev = _ln_mix_bwd(p, grad, x, S["head1"], "ln1", ns, length, MIX, gmix, dx2, row(1), g_in is not None)
+    if g_in is not None:
+        g_in[:, 1] = dprev
+    return dx, g_vfirst
+
+
+def _pack(tree, tensors):
+    """``tree`` with its tensors moved to the list ``tensors`` and their places left in it."""
+    if torch.is_tensor(tree):
+        tensors.append(tree)
+        return len(tensors) - 1, None
+    if isinstance(tree, dict):
+        return {k: _pack(v, tensors) for k, v in tree.items()}
+    if isinstance(tree, (list, tuple)):
+        return [_pack(v, tensors) for v in tree]
+    return None, tree
+
+
+def _unpack(tree, tensors):
+    if isinstance(tree, dict):
+        return {k: _unpack(v, tensors) for k, v in tree.items()}
+    if isinstance(tree, list):
+        return [_unpack(v, tensors) for v in tree]
+    return tree[1] if tree[0] is None else tensors[tree[0]]
+
+
+class _Blocks(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, state, ns, length, *params):
+        ctx.set_materialize_grads(False)
+        x, dx, new_state, saved, v_first = _run(x, state, ns, length, params, True)
+        tensors = []
+        ctx.places = _pack([saved, v_first, ns, length], tensors)
+        ctx.n = len(tensors)
+        ctx.save_for_backward(*tensors, state, *params)
+        return x, dx, new_state
+
+    @staticmethod
+    def backward(ctx, g_x, g_dx, g_state):
+        tensors = ctx.saved_tensors
+        saved, v_first, ns, length = _unpack(ctx.places, tensors)
+        state, *params = tensors[ctx.n:]
+        L = params[0].shape[0]
+        like = saved[-1]["x2"]
+        io = like.dtype
+        g_x = torch.zeros_like(like) if g_x is None else ops._dev(g_x, io)
+        g_dx = torch.zeros_like(like) if g_dx is None else ops._dev(g_dx, io)
+        g_state = None if g_state is None else g_state.to(io)
+        grads = [torch.empty_like(t) for t in params]
+        for t, n in zip(grads, NAMES):
+            if n in ("v0", "v1", "v2"):
+                t[0].zero_()                    # the first layer has no value residual
+        g_in = torch.empty_like(state) if ctx.needs_input_grad[1] else None
+        g_vfirst = None
+        layers = list(zip(*(t.unbind(0) for t in params)))
+        glayers = list(zip(*(t.unbind(0) for t in grads)))
+        for i in reversed(range(L)):
+            dx, g_vfirst = _layer_bwd(i, dict(zip(NAMES, layers[i])), dict(zip(NAMES, glayers[i])), saved[i], ns,
+                                      length, g_x, g_dx, None if g_state is None else g_state[:, i],
+                                      None if g_in is None else g_in[:, i], g_vfirst, v_first)
+            g_x = g_dx = dx
+        need = ctx.needs_input_grad[4:]
+        return (g_x, g_in, None, None) + tuple(g if n else None for g, n in zip(grads, need))
+
+
+def _run(x, state, ns, length, params, keep):
+    L = params[0].shape[0]
+    layers = list(zip(*(t.unbind(0) for t in params)))
+    new_state = torch.empty_like(state)
+    dx = v_first = None
+    saved = [] if keep else None
+    for i in range(L):
+        x, dx, v_first, S = _layer_fwd(i, dict(zip(NAMES, layers[i])), x, dx, state[:, i], new_state[:, i], v_first, ns,
+                                       length, keep)
+        if keep:
+            saved.append(S)
+    return x, dx, new_state, saved, v_first
+
+
+def covers(params, x, state):
+    """Whether the operator takes the call: one dtype throughout and contiguous stacked parameters."""
+    io = x.dtype
+    return (io in ops._DT and state.dtype == io and x.shape[-1] <= ops.LN_SHIFTMIX_MAX_C
+            and all(t.dtype == io and t.is_contiguous() and t.is_cuda for t in params))
+
+
+def run(params, x, state, ns, length, grad):
+    """The stack on x (B,T,C) and state (B,L,2+N,C): returns (x, dx, new_state) whose sum x + dx is the residual stream."""
+    if grad:
+        length = None if length is None else length.clone()          # the caller may change its own before the backward
+        return _Blocks.apply(x, state, ns, length, *params)
+    return _run(x, state, ns, length, params, False)[:3]

@@ -669,7 +669,7 @@ int hiprwkv_rwkv7_postmix_bwd(hiprwkv_stream stream, int io_dtype, int64_t rows,
     if (!aligned16(p)) return fail(HIPRWKV_EINVAL, "rwkv7_postmix_bwd: tensor pointers must be 16-byte aligned");
   }
   hipError_t e = launch_rwkv7_postmix_bwd(io_dtype == HIPRWKV_F32, rows, H, y, r, k, v, g, ln_w, ln_b, r_k, eps, gout,
-                                          gy, gr, gk, gv, gg, gln_w, gln_b, gr_k, static_cast<hipStream_t>(stream));
+                                          gy, gr, gk, gv, gg, gln_w, gln_b, gr_k, nullptr, nullptr, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail(HIPRWKV_ELAUNCH, "rwkv7_postmix_bwd: %s", hipGetErrorString(e));
   return HIPRWKV_OK;
 }
@@ -790,7 +790,8 @@ int hiprwkv_rwkv7_pre_bwd(hiprwkv_stream stream, int io_dtype, int64_t rows, int
                           const void* k, const void* xa, const void* v, const void* v_first, const void* xv,
                           const void* w0, const void* a0, const void* v0, const void* k_k, const void* k_a,
                           const void* gw, const void* gk_out, const void* gv_out, const void* ga_out,
-                          const void* gb_out, void* dxw, void* dk, void* dv, void* dv_first, void* dxv, void* dxa,
+                          const void* gb_out, const void* gk_out2, const void* gv_out2, const void* gr, const void* gr2,
+                          void* dr, void* dxw, void* dk, void* dv, void* dv_first, void* dxv, void* dxa,
                           void* const* dparam, void* workspace, size_t workspace_bytes) {
   PreArgs A;
   memset(&A, 0, sizeof(A));
@@ -798,6 +799,10 @@ int hiprwkv_rwkv7_pre_bwd(hiprwkv_stream stream, int io_dtype, int64_t rows, int
   A.xw = xw; A.k = k; A.xa = xa; A.v = v; A.vf = v_first; A.xv = xv;
   A.w0 = w0; A.a0 = a0; A.v0 = v0; A.k_k = k_k; A.k_a = k_a;
   A.gw = gw; A.gk = gk_out; A.gv = gv_out; A.ga = ga_out; A.gb = gb_out;
+  A.gk2 = gk_out2; A.gv2 = gv_out2; A.gr = gr; A.gr2 = gr2; A.dr = dr;
+  for (const void* p : {gk_out2, gv_out2, gr, gr2, static_cast<const void*>(dr)})
+    if (p != nullptr && !aligned16(p)) return fail(HIPRWKV_EINVAL, "rwkv7_pre_bwd: tensor pointers must be 16-byte aligned");
+  if (dr != nullptr && (gr == nullptr || gr2 == nullptr)) return fail(HIPRWKV_EINVAL, "rwkv7_pre_bwd: dr needs gr and gr2");
   A.dxw = dxw; A.dk = dk; A.dv = dv; A.dvf = dv_first; A.dxv = dxv; A.dxa = dxa;
   A.part = static_cast<float*>(workspace);
   if (int rc = check_pre("rwkv7_pre_bwd", io_dtype, N, A,
@@ -932,6 +937,50 @@ int hiprwkv_wkv4_mix_bwd(hiprwkv_stream stream, int io_dtype, int64_t B, int64_t
     e = launch_reduce_parts(A.io_f32, R, st);
   }
   return gate_done("wkv4_mix_bwd", e);
+}
+
+int hiprwkv_gemm(hiprwkv_stream stream, int n_jobs, const hiprwkv_gemm_job* jobs) {
+  if (n_jobs <= 0 || n_jobs > GEMM_MAX_JOBS || jobs == nullptr)
+    return fail(HIPRWKV_EINVAL, "gemm: 1 to %d jobs", GEMM_MAX_JOBS);
+  GemmArgs A;
+  memset(&A, 0, sizeof(A));
+  A.n_jobs = n_jobs;
+  int64_t tiles = 0;
+  for (int i = 0; i < n_jobs; ++i) {
+    const hiprwkv_gemm_job& J = jobs[i];
+    if (J.M <= 0 || J.N <= 0 || J.K <= 0 || J.N % 8 || (!J.kn && J.K % 8) || (J.km ? J.M % 8 : J.K % 8))
+      return fail(HIPRWKV_EINVAL, "gemm: job %d: sizes must be positive, those contiguous in memory multiples of 8", i);
+    if (J.act < 0 || J.act > (J.aux ? 2 : 3)) return fail(HIPRWKV_EINVAL, "gemm: job %d: unknown function", i);
+    for (const void* p : {J.x, J.w, static_cast<const void*>(J.out)})
+      if (p == nullptr || !aligned16(p)) return fail(HIPRWKV_EINVAL, "gemm: job %d: null or misaligned tensor pointer (16 bytes)", i);
+    if (J.aux != nullptr && !aligned16(J.aux)) return fail(HIPRWKV_EINVAL, "gemm: job %d: misaligned tensor pointer (16 bytes)", i);
+    tiles += (int64_t)((J.N + 511) / 512 * 8) * ((J.M + 63) / 64);
+    A.job[i] = J;
+  }
+  if (tiles > 0x7fffffffLL) return fail(HIPRWKV_EINVAL, "gemm: too many tiles for one launch");
+  return gate_done("gemm", launch_gemm(A, 1, static_cast<hipStream_t>(stream)));
+}
+
+size_t hiprwkv_rwkv7_postmix_bwd2_workspace_bytes(int64_t rows, int64_t H, int64_t N) {
+  return (size_t)rwkv7_postmix_bwd_rows(rows, H) * 3 * H * N * sizeof(float);
+}
+
+int hiprwkv_rwkv7_postmix_bwd2(hiprwkv_stream stream, int io_dtype, int64_t rows, int64_t H, int64_t N, const void* y,
+                               const void* r, const void* k, const void* v, const void* g, const void* ln_w,
+                               const void* ln_b, const void* r_k, float eps, const void* gout, void* gy, void* gr,
+                               void* gk, void* gv, void* gg, void* const* dparam, void* workspace, size_t workspace_bytes) {
+  PreArgs A;      // shape checks as for rwkv7_pre
+  memset(&A, 0, sizeof(A));
+  A.rows = rows; A.H = H;
+  if (int rc = check_pre("rwkv7_postmix_bwd2", io_dtype, N, A, {y, r, k, v, g, ln_w, ln_b, r_k, gout, gy, gr, gk, gv, gg, workspace}, {})) return rc;
+  if (dparam == nullptr || dparam[0] == nullptr || dparam[1] == nullptr || dparam[2] == nullptr)
+    return fail(HIPRWKV_EINVAL, "rwkv7_postmix_bwd2: null tensor pointer");
+  const size_t need = hiprwkv_rwkv7_postmix_bwd2_workspace_bytes(rows, H, N);
+  if (workspace_bytes < need)
+    return fail(HIPRWKV_ENOSPACE, "rwkv7_postmix_bwd2: workspace has %zu bytes, %zu needed", workspace_bytes, need);
+  return gate_done("rwkv7_postmix_bwd2", launch_rwkv7_postmix_bwd(io_dtype == HIPRWKV_F32, rows, H, y, r, k, v, g, ln_w, ln_b, r_k, eps,
+                                                                   gout, gy, gr, gk, gv, gg, nullptr, nullptr, nullptr,
+                                                                   static_cast<float*>(workspace), dparam, static_cast<hipStream_t>(stream)));
 }
 
 }  // extern "C"

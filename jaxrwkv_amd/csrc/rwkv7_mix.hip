@@ -118,7 +118,8 @@ __global__ void zero_f32_kernel(float* p, int n) {
 
 // adds NP per-lane partial sums (four channels each) over the workgroup's lane rows and into out[p][h][64]
 template <int NP>
-__device__ __forceinline__ void reduce_params(const float (&part)[NP][4], float* const (&out)[NP], int64_t h) {
+__device__ __forceinline__ void reduce_params(const float (&part)[NP][4], float* const (&out)[NP], int64_t h,
+                                              float* rows = nullptr, int64_t row = 0, int64_t C = 0) {
   __shared__ float red[NP][BWD_ROWS][64];
   const int grp = threadIdx.x >> 4, c4 = 4 * (threadIdx.x & 15);
 #pragma unroll
@@ -130,7 +131,8 @@ __device__ __forceinline__ void reduce_params(const float (&part)[NP][4], float*
     float sum = 0.f;
 #pragma unroll
     for (int g = 0; g < BWD_ROWS; ++g) sum += red[p][g][c];
-    atomicAdd(out[p] + h * 64 + c, sum);
+    if (rows != nullptr) rows[(row * NP + p) * C + h * 64 + c] = sum;       // launch_reduce_parts adds the rows
+    else atomicAdd(out[p] + h * 64 + c, sum);
   }
 }
 
@@ -188,7 +190,7 @@ __global__ __launch_bounds__(MIX_THREADS) void rwkv7_postmix_bwd_kernel(
     const T* __restrict__ v, const T* __restrict__ g, const T* __restrict__ ln_w, const T* __restrict__ ln_b,
     const T* __restrict__ r_k, float eps, const T* __restrict__ go, T* __restrict__ gy, T* __restrict__ gr,
     T* __restrict__ gk, T* __restrict__ gv, T* __restrict__ gg, float* __restrict__ gln_w, float* __restrict__ gln_b,
-    float* __restrict__ gr_k) {
+    float* __restrict__ gr_k, float* __restrict__ prows) {
   const int64_t h = blockIdx.x % H, rb = blockIdx.x / H, nrb = gridDim.x / H;
   const int grp = threadIdx.x >> 4, c4 = 4 * (threadIdx.x & 15);
   float lw[4], lb[4], rk[4];
@@ -240,7 +242,7 @@ __global__ __launch_bounds__(MIX_THREADS) void rwkv7_postmix_bwd_kernel(
     if (active) { st4(gy + el, oy); st4(gr + el, orr); st4(gk + el, okk); st4(gv + el, ov); st4(gg + el, og); }
   }
   float* const outs[3] = {gln_w, gln_b, gr_k};
-  reduce_params<3>(part, outs, h);
+  reduce_params<3>(part, outs, h, prows, rb, H * 64);
 }
 
 // workgroups per head: enough to fill the GPU, never more than there are 16-token groups
@@ -297,26 +299,43 @@ hipError_t launch_rwkv7_premix_bwd(int io_f32, int64_t rows, int64_t H, const vo
   return hipGetLastError();
 }
 
+// workgroups per head when their parameter sums leave as rows of a workspace: about four per CU in all
+int64_t rwkv7_postmix_bwd_rows(int64_t rows, int64_t H) {
+  const int64_t want = (1024 + H - 1) / H, have = (rows + BWD_ROWS - 1) / BWD_ROWS;
+  return want < have ? want : have;
+}
+
+// part: null, or a workspace (rwkv7_postmix_bwd_rows, 3, H*64); then the parameter cotangents go to dparam (ln_w, ln_b, r_k) in
+// the I/O dtype and the fp32 arrays are not used
 hipError_t launch_rwkv7_postmix_bwd(int io_f32, int64_t rows, int64_t H, const void* y, const void* r, const void* k,
                                     const void* v, const void* g, const void* ln_w, const void* ln_b, const void* r_k,
                                     float eps, const void* go, void* gy, void* gr, void* gk, void* gv, void* gg,
-                                    float* gln_w, float* gln_b, float* gr_k, hipStream_t stream) {
+                                    float* gln_w, float* gln_b, float* gr_k, float* part, void* const* dparam,
+                                    hipStream_t stream) {
   const int np = (int)(H * 64);
-  hipLaunchKernelGGL(zero_f32_kernel, dim3((np + 255) / 256), dim3(256), 0, stream, gln_w, np);
-  hipLaunchKernelGGL(zero_f32_kernel, dim3((np + 255) / 256), dim3(256), 0, stream, gln_b, np);
-  hipLaunchKernelGGL(zero_f32_kernel, dim3((np + 255) / 256), dim3(256), 0, stream, gr_k, np);
-  const dim3 grid((unsigned)H * bwd_row_blocks(rows, H)), block(MIX_THREADS);
+  if (part == nullptr) {
+    hipLaunchKernelGGL(zero_f32_kernel, dim3((np + 255) / 256), dim3(256), 0, stream, gln_w, np);
+    hipLaunchKernelGGL(zero_f32_kernel, dim3((np + 255) / 256), dim3(256), 0, stream, gln_b, np);
+    hipLaunchKernelGGL(zero_f32_kernel, dim3((np + 255) / 256), dim3(256), 0, stream, gr_k, np);
+  }
+  const int64_t row_blocks = part != nullptr ? rwkv7_postmix_bwd_rows(rows, H) : (int64_t)bwd_row_blocks(rows, H);
+  const dim3 grid((unsigned)(H * row_blocks)), block(MIX_THREADS);
   if (io_f32)
     hipLaunchKernelGGL(rwkv7_postmix_bwd_kernel<float>, grid, block, 0, stream, rows, H, (const float*)y,
                        (const float*)r, (const float*)k, (const float*)v, (const float*)g, (const float*)ln_w,
                        (const float*)ln_b, (const float*)r_k, eps, (const float*)go, (float*)gy, (float*)gr,
-                       (float*)gk, (float*)gv, (float*)gg, gln_w, gln_b, gr_k);
+                       (float*)gk, (float*)gv, (float*)gg, gln_w, gln_b, gr_k, part);
   else
     hipLaunchKernelGGL(rwkv7_postmix_bwd_kernel<bf16_t>, grid, block, 0, stream, rows, H, (const bf16_t*)y,
                        (const bf16_t*)r, (const bf16_t*)k, (const bf16_t*)v, (const bf16_t*)g, (const bf16_t*)ln_w,
                        (const bf16_t*)ln_b, (const bf16_t*)r_k, eps, (const bf16_t*)go, (bf16_t*)gy, (bf16_t*)gr,
-                       (bf16_t*)gk, (bf16_t*)gv, (bf16_t*)gg, gln_w, gln_b, gr_k);
-  return hipGetLastError();
+                       (bf16_t*)gk, (bf16_t*)gv, (bf16_t*)gg, gln_w, gln_b, gr_k, part);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || part == nullptr) return e;
+  ReduceArgs R;
+  R.part = part; R.rows = row_blocks; R.nk = 3; R.C = np;
+  for (int i = 0; i < 3; ++i) R.out[i] = dparam[i];
+  return launch_reduce_parts(io_f32, R, stream);
 }
 
 }  // namespace hiprwkv

@@ -104,9 +104,22 @@ __global__ __launch_bounds__(PRE_THREADS) void rwkv7_pre_bwd_kernel(PreArgs A) {
     float xw[8], k[8], xa[8], gw[8], gk[8], gai[8], gbi[8], o[8];
     in(A.xw, el, xw); in(A.k, el, k); in(A.xa, el, xa);
     in(A.gw, el, gw); in(A.gk, el, gk); in(A.ga, el, gai); in(A.gb, el, gbi);
+    auto add = [&](const void* p, float (&x)[8]) {
+      float y[8];
+      in(p, el, y);
+#pragma unroll
+      for (int c = 0; c < 8; ++c) x[c] += y[c];
+    };
+    if (A.gk2 != nullptr) add(A.gk2, gk);
+    if (A.dr != nullptr) {
+      in(A.gr, el, o);
+      add(A.gr2, o);
+      put(A.dr, o);
+    }
     if (VMIX) {
       float v[8], vf[8], xv[8], gv[8], o1[8], o2[8];
       in(A.v, el, v); in(A.vf, el, vf); in(A.xv, el, xv); in(A.gv, el, gv);
+      if (A.gv2 != nullptr) add(A.gv2, gv);
 #pragma unroll
       for (int c = 0; c < 8; ++c) {
         const float s = sigmoidf(v0[c] + xv[c]);

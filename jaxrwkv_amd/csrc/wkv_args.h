@@ -135,12 +135,31 @@ struct PreArgs {
   void *w, *k_out, *v_out, *a_out, *b_out;
   // backward
   const void *gw, *gk, *gv, *ga, *gb;          // cotangents of w, k_out, v_out, a_out, b_out
+  const void *gk2, *gv2;                       // second cotangents of k_out and v_out, added to the first; may be null
+  const void *gr, *gr2;                        // two cotangents of r to be added up in dr; may be null
+  void* dr;
   void *dxw, *dk, *dv, *dvf, *dxv, *dxa;
   float* part;                                 // workspace (rwkv7_pre_bwd_rows, 4 or 5, H*64)
 };
 int64_t rwkv7_pre_bwd_rows(int64_t rows, int64_t H);
 hipError_t launch_rwkv7_pre(int io_f32, const PreArgs& A, hipStream_t stream);
 hipError_t launch_rwkv7_pre_bwd(int io_f32, const PreArgs& A, void* const* dparam, hipStream_t stream);
+
+// Several products per launch (rwkv7_gemm.hip), bf16: out[m][n] = f(sum_k x(m, k) w(n, k)).  The job is the C ABI's
+// (hiprwkv_gemm_job); tile0 is the launcher's.
+using GemmJob = ::hiprwkv_gemm_job;
+constexpr int GEMM_ACT_NONE = 0, GEMM_ACT_TANH = 1, GEMM_ACT_SIGMOID = 2, GEMM_ACT_RELUSQ = 3;      // f without aux
+constexpr int GEMM_ADD = 0, GEMM_DTANH = 1, GEMM_DSIGMOID = 2;                                      // f with aux
+constexpr int GEMM_MAX_JOBS = HIPRWKV_GEMM_MAX_JOBS;
+constexpr int GEMM_TILE_ROWS = 65;     // rows from which the LDS-tiled kernel takes over
+constexpr int GEMM_MAX_SPLIT = 4;
+struct GemmArgs {
+  GemmJob job[GEMM_MAX_JOBS];
+  int n_jobs;
+  float* part;         // not null: (split, M, N) fp32 partial sums instead of out; one job, no f
+};
+int gemm_split(int M, int64_t K, int64_t N);
+hipError_t launch_gemm(GemmArgs A, int split, hipStream_t stream);
 
 using Rwkv7Decode = ::hiprwkv_rwkv7_decode_args;
 size_t rwkv7_decode_workspace(const Rwkv7Decode& D);
@@ -214,6 +233,8 @@ hipError_t launch_rwkv7_premix_bwd(int io_f32, int64_t rows, int64_t H, const vo
 hipError_t launch_rwkv7_postmix_bwd(int io_f32, int64_t rows, int64_t H, const void* y, const void* r, const void* k,
                                     const void* v, const void* g, const void* ln_w, const void* ln_b, const void* r_k,
                                     float eps, const void* go, void* gy, void* gr, void* gk, void* gv, void* gg,
-                                    float* gln_w, float* gln_b, float* gr_k, hipStream_t stream);
+                                    float* gln_w, float* gln_b, float* gr_k, float* part, void* const* dparam,
+                                    hipStream_t stream);
+int64_t rwkv7_postmix_bwd_rows(int64_t rows, int64_t H);
 
 }  // namespace hiprwkv

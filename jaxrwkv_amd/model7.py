@@ -17,7 +17,7 @@ import math
 import torch
 import torch.nn.functional as F
 
-from . import ops
+from . import blocks7, ops
 from .rwkv7 import HipRWKV
 
 HEAD_SIZE = 64
@@ -114,6 +114,10 @@ def unstack(tree, n_layer):
     training step: 860 launches and 5 ms of the GPU's time)."""
     split = tree_map(lambda t: t.unbind(0), tree)
     return [tree_map(lambda ts: ts[i], split) for i in range(n_layer)]
+
+
+def _needs_grad(tensors):
+    return torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
 
 
 class RWKV7:
@@ -222,14 +226,20 @@ class RWKV7:
         fused = cls.fuse_mix and C <= ops.LN_SHIFTMIX_MAX_C
         x = params["emb"]["weight"][tokens]
         grad = torch.is_grad_enabled() and (x.requires_grad or state.requires_grad)
-        # decode steps whose recurrence is this package's: the whole step from native code
-        if fused and not grad and T <= 8 and cls.inner.inner_loop == HipRWKV.inner_loop and not HipRWKV.force_seq:
+        # where the recurrence is this package's: decode steps from native code, whole sequences as one operator
+        own = fused and cls.inner.inner_loop == HipRWKV.inner_loop and not HipRWKV.force_seq
+        if own and not grad and T <= 8:
             step = ops.rwkv7_decode(params, x, state, length, new_starts, HipRWKV.assoc_compat)
             if step is not None:
                 return step
         norm = (lambda x, dx, ln: ops.rwkv7_ln_shiftmix(x, dx, ln, None, None, None, [])[2][0]) if fused else \
                (lambda x, dx, ln: layer_norm(x if dx is None else x + dx, ln))
         x = norm(x, None, params["ln0"])
+        stacked = blocks7.gather(params["blocks"]) if own and T > 8 else ()
+        if stacked and blocks7.covers(stacked, x, state):
+            grad = grad or _needs_grad(stacked)
+            x, dx, new_state = blocks7.run(stacked, x, state, new_starts, length, grad)
+            return norm(x, dx, params["ln_out"]) @ params["head"]["weight"].T, new_state
         blocks = unstack(params["blocks"], L)
         # without autograd the layers write their rows of the new state where they belong; decode steps read and write the
         # recurrence's rows in place as well

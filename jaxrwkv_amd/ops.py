@@ -870,7 +870,7 @@ class _Pre(torch.autograd.Function):
         ws = torch.empty(nbytes, dtype=torch.uint8, device=k.device)
         rc = lib.hiprwkv_rwkv7_pre_bwd(_stream(), _DT[io], rows, H, N, _p(xw), _p(k), _p(xa), _p(v), _p(vf), _p(xv), _p(w0),
                                        _p(a0), _p(v0), _p(k_k), _p(k_a), _p(gw), _p(gk), None if vf is None else _p(gv),
-                                       _p(ga), _p(gb), _p(dxw), _p(dk), _p(dv), _p(dvf), _p(dxv), _p(dxa),
+                                       _p(ga), _p(gb), None, None, None, None, None, _p(dxw), _p(dk), _p(dv), _p(dvf), _p(dxv), _p(dxa),
                                        _ptr_array(dparam), _p(ws), nbytes)
         _lib.check(rc, "hiprwkv_rwkv7_pre_bwd")
         dw0, da0, dk_k, dk_a, dv0 = dparam
