@@ -344,7 +344,7 @@ int hiprwkv_rwkv7_pre_bwd(hiprwkv_stream stream, int io_dtype, int64_t rows, int
                           void* const* dparam, void* workspace, size_t workspace_bytes);
 
 /* ---- Several narrow products in one launch -------------------------------------------------------------
- * bf16, fp32 accumulation: out[m][n] = f(sum_k x(m, k) w(n, k)), out (M, N) row-major.  x is (M, K) row-major, with km its
+ * bf16, fp32 accumulation, the sum rounded to bf16 before f: out[m][n] = f(sum_k x(m, k) w(n, k)), out (M, N) row-major.  x is (M, K) row-major, with km its
  * transpose (K, M); w is (N, K), with kn (K, N).  For the low-rank factors of RWKV-7's decay, gates and value residual
  * (rwkv7.py:237-245) and their cotangents.  f: without aux 0 none, 1 tanh, 2 sigmoid, 3 relu(.)^2; with aux, an (M, N) array:
  * 0 + aux, 1 times 1 - aux^2, 2 times aux (1 - aux) (the derivatives in terms of the activations' values).  Sizes that are

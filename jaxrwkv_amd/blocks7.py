@@ -47,15 +47,17 @@ def _gemm(jobs):
     _lib.check(_lib.load().hiprwkv_gemm(ops._stream(), len(jobs), arr), "hiprwkv_gemm")
 
 
-def _grouped(p):
-    """Whether the grouped products take the low-rank factors: bf16, inner sizes multiples of 8."""
-    return p["w1"].dtype == torch.bfloat16 and all(p[n].shape[-1] % 8 == 0 for n in ("w1", "a1", "v1", "g1"))
+def _grouped(p, like):
+    """Whether the grouped products take the low-rank factors beside a (M, C) array: bf16, inner sizes multiples of 8, no
+    operand of 2 GiB."""
+    return (like.dtype == torch.bfloat16 and like.numel() < 2 ** 30
+            and all(p[n].shape[-1] % 8 == 0 for n in ("w1", "a1", "v1", "g1")))
 
 
 def _lora_fwd(p, mix, names, like):
     """Hidden values (activation applied) and results of the low-rank terms ``names``; mix: name -> (M, C) input."""
     hid, out = {}, {}
-    if _grouped(p):
+    if _grouped(p, like):
         M, C = like.shape
         for n, _ in names:
             hid[n] = torch.empty((M, p[n + "1"].shape[-1]), dtype=like.dtype, device=like.device)
@@ -73,7 +75,7 @@ def _lora_fwd(p, mix, names, like):
 def _lora_bwd(p, grad, mix, hid, gout, dmix, names):
     """From the cotangents ``gout`` of the low-rank terms: the parameters' cotangents into ``grad`` and the inputs' into
     ``dmix`` (the value residual's is added to what is there)."""
-    if _grouped(p):
+    if _grouped(p, gout["w"]):
         dh = {n: torch.empty_like(hid[n]) for n, _ in names}
         _gemm([(dh[n], gout[n], p[n + "2"], 0, 0, act, hid[n] if act else None) for n, act in names])
         _gemm([(dmix[n], dh[n], p[n + "1"], 0, 0, 0, dmix[n] if n == "v" else None) for n, _ in names])

@@ -6,6 +6,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <initializer_list>
 #include <mutex>
 
@@ -950,11 +951,13 @@ int hiprwkv_gemm(hiprwkv_stream stream, int n_jobs, const hiprwkv_gemm_job* jobs
     const hiprwkv_gemm_job& J = jobs[i];
     if (J.M <= 0 || J.N <= 0 || J.K <= 0 || J.N % 8 || (!J.kn && J.K % 8) || (J.km ? J.M % 8 : J.K % 8))
       return fail(HIPRWKV_EINVAL, "gemm: job %d: sizes must be positive, those contiguous in memory multiples of 8", i);
+    if (std::max((int64_t)(J.km ? J.M : 0), (int64_t)(J.kn ? J.N : 0)) * J.K * 2 >= 0x7fffffffLL || (int64_t)J.K * 256 >= 0x7fffffffLL)
+      return fail(HIPRWKV_EINVAL, "gemm: job %d: an operand of 2 GiB or more", i);
     if (J.act < 0 || J.act > (J.aux ? 2 : 3)) return fail(HIPRWKV_EINVAL, "gemm: job %d: unknown function", i);
     for (const void* p : {J.x, J.w, static_cast<const void*>(J.out)})
       if (p == nullptr || !aligned16(p)) return fail(HIPRWKV_EINVAL, "gemm: job %d: null or misaligned tensor pointer (16 bytes)", i);
     if (J.aux != nullptr && !aligned16(J.aux)) return fail(HIPRWKV_EINVAL, "gemm: job %d: misaligned tensor pointer (16 bytes)", i);
-    tiles += (int64_t)((J.N + 511) / 512 * 8) * ((J.M + 63) / 64);
+    tiles += (int64_t)((J.N + 511) / 512 * 8) * ((J.M + 511) / 512 * 8);
     A.job[i] = J;
   }
   if (tiles > 0x7fffffffLL) return fail(HIPRWKV_EINVAL, "gemm: too many tiles for one launch");

@@ -16,7 +16,11 @@ using chunk::mfma;
 
 constexpr int GEMM_WAVES = 8;
 
+// f of a product, which is rounded to bf16 first, where the separate product would be stored
+__device__ __forceinline__ float rnd(float x) { return bf16_to_f32(f32_to_bf16(x)); }
 __device__ __forceinline__ float activate(float x, int act) {
+  if (act == GEMM_ACT_NONE) return x;
+  x = rnd(x);
   switch (act) {
     case GEMM_ACT_TANH: return 1.f - 2.f / (1.f + __expf(2.f * x));
     case GEMM_ACT_SIGMOID: return 1.f / (1.f + __expf(-x));
@@ -103,12 +107,16 @@ __global__ __launch_bounds__(64 * GEMM_WAVES) void skinny_gemm_kernel(GemmArgs A
 
 // 64 x 64 tiles, 64 of k per step through two LDS buffers: a thread carries two 16-byte pieces of either operand, requested two
 // steps ahead, and four workgroups share a CU, so loads, LDS writes and matrix instructions of different workgroups
-// overlap.  An operand that lies k-major (km, kn) goes to LDS as it lies and is read with the transposing load.  The row tiles
-// of one column tile run on one XCD (workgroups go to the eight XCDs round-robin), whose L2 then reads the weights once.
-// At 256 rows against 6656 columns of 2048 (a decode step of 256 users) the weights' stream needs 5.3 us and the operand reads
-// from LDS 6 us; measured 25.  Where one product leaves CUs idle (the output and value projections there: 128 tiles) K is
-// split over gridDim.y and the parts are added by the norm that reads the result.
+// overlap.  An operand that lies k-major (km, kn) goes to LDS as it lies and is read with the transposing load.  Workgroups go
+// to the eight XCDs round-robin; the tiles that share a piece of the longer operand run on one XCD, whose L2 reads it once.
+// Bound by the CU's paths to the cache and to LDS (16 KiB in, 16 KiB to LDS and 32 KiB from it per step: 790 cycles with two
+// workgroups on a CU, 1000 with one).  Weights straight from memory into the matrix operands instead were slower (a
+// cache line per lane: 2200 cycles for 128 x 64 x 128), and so were four steps in flight.  Where one product leaves CUs idle
+// (a decode step's output and value projections: 128 tiles) K is split over gridDim.y and the parts are added by the norm
+// that reads the result.  Low-rank products at 4084 tokens of 2048 channels: 35 us for the four into the inner sizes (74 with
+// the row tiles of a narrow product on one XCD), 48 us out of them (67 MB written).
 constexpr int TG = 64, TG_RS = TG + 8;         // tile edge; LDS row stride: 16-byte rows 144 bytes apart
+constexpr int AHEAD = 2;                       // steps whose operands are in flight (four: 212 registers, 1.6 times slower for short K)
 typedef uint16_t TileLds[2][2][TG][TG_RS];     // [buffer][x | w]
 
 __device__ __forceinline__ uint2 lds_tr4(const uint16_t* p) {      // see wkv7_fwd.hip
@@ -117,37 +125,48 @@ __device__ __forceinline__ uint2 lds_tr4(const uint16_t* p) {      // see wkv7_f
   return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p)));
 }
 
-// One operand of a tile: R rows (of m or n) by K of k, row-major R x K, or with TR its transpose.
-template <bool TR>
+using chunk::rsrc_t;
+using chunk::make_rsrc;
+__device__ __forceinline__ u32x4_t buf_ld16(rsrc_t r, int voff, int soff) {
+  return __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+}
+
+// One operand of a tile: R rows (of m or n) by K of k, row-major R x K, or with TR its transpose.  Addressed through a buffer
+// descriptor: a lane's offset is computed once and a step's is a scalar, so that a request costs one instruction.  Rows
+// beyond the edge re-read the last one (what they give is not stored).  EXACT: K is a multiple of the step; otherwise k beyond K
+// re-reads the last piece and is zeroed on its way to LDS.  Requests beyond the last step re-read it.
+template <bool TR, bool EXACT>
 struct TileOperand {
-  const uint4* p[2];
-  int row, col, R, K, r0;
-  __device__ __forceinline__ TileOperand(const void* base, int R_, int K_, int r0_) : R(R_), K(K_), r0(r0_) {
-    row = threadIdx.x >> 3;
-    col = (threadIdx.x & 7) * 8;
+  rsrc_t rs;
+  int voff[2], row, col, R, K, last;
+  __device__ __forceinline__ TileOperand(const void* base, int R_, int K_, int r0, int tid) : R(R_), K(K_) {
+    row = tid >> 3;
+    col = (tid & 7) * 8;
+    last = (K - 1) / TG;
+    // the descriptor starts at the tile, so that offsets stay small whatever the operand's size
+    const int64_t first = TR ? (int64_t)(r0 < R ? r0 : R - 8) : (int64_t)(r0 < R ? r0 : R - 1) * K;
+    rs = make_rsrc(static_cast<const bf16_t*>(base) + first);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      const int rr = r0 + row + 32 * i < R ? r0 + row + 32 * i : R - 1, cc = r0 + col < R ? r0 + col : R - 8;
-      p[i] = reinterpret_cast<const uint4*>(static_cast<const bf16_t*>(base) + (TR ? (size_t)cc : (size_t)rr * K));
+      const int rr = r0 + row + 32 * i < R ? row + 32 * i : R - 1 - r0, cc = r0 + col < R ? col : R - 8 - r0;
+      voff[i] = TR ? ((row + 32 * i) * R + cc) * 2 : (rr * K + col) * 2;
     }
   }
-  // Addresses stay inside the operand: rows and k beyond an edge re-read its last piece.
   __device__ __forceinline__ void load(u32x4_t (&v)[2], int s) const {
+    s = s < last ? s : last;
+    const int soff = TR ? s * TG * R * 2 : s * TG * 2;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      if (TR) {
-        const int kk = s * TG + row + 32 * i < K ? s * TG + row + 32 * i : K - 1;
-        v[i] = *reinterpret_cast<const u32x4_t*>(p[i] + (size_t)kk * (R / 8));
-      } else {
-        const int k = s * TG + col < K ? s * TG + col : K - 8;
-        v[i] = *reinterpret_cast<const u32x4_t*>(p[i] + k / 8);
+      int o = voff[i];
+      if (!EXACT) {
+        if (TR) o -= s * TG + row + 32 * i < K ? 0 : (s * TG + row + 32 * i - (K - 1)) * R * 2;
+        else o -= s * TG + col < K ? 0 : (s * TG + col - (K - 8)) * 2;
       }
+      v[i] = buf_ld16(rs, o, soff);
     }
   }
-  // What lies beyond K is zeroed on its way to LDS (in the last step only); what lies beyond R reaches results that are not
-  // stored.
   __device__ __forceinline__ void store(u32x4_t (&v)[2], int s, uint16_t (&lds)[TG][TG_RS]) const {
-    if ((s + 1) * TG > K) {
+    if (!EXACT && (s + 1) * TG > K) {
       chunk::rare_path();
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
@@ -170,13 +189,37 @@ struct TileOperand {
   }
 };
 
-template <bool KM, bool KN>
+// f and the store of one lane's four consecutive columns
+__device__ __forceinline__ void finish(const GemmArgs& A, const GemmJob& J, int n, int m, f32x4_t v) {
+  if (n >= J.N || m >= J.M) return;
+  if (A.part != nullptr) {
+    *reinterpret_cast<f32x4_t*>(A.part + ((size_t)blockIdx.y * J.M + m) * J.N + n) = v;
+    return;
+  }
+  const size_t el = (size_t)m * J.N + n;
+  if (J.aux != nullptr) {
+    const uint2 q = *reinterpret_cast<const uint2*>(static_cast<const bf16_t*>(J.aux) + el);
+    const float h[4] = {__uint_as_float(q.x << 16), __uint_as_float(q.x & 0xffff0000u), __uint_as_float(q.y << 16),
+                        __uint_as_float(q.y & 0xffff0000u)};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = rnd(v[i]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      v[i] = J.act == GEMM_ADD ? v[i] + h[i] : J.act == GEMM_DTANH ? v[i] * (1.f - h[i] * h[i]) : v[i] * (h[i] * (1.f - h[i]));
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = activate(v[i], J.act);
+  }
+  *reinterpret_cast<uint2*>(static_cast<bf16_t*>(J.out) + el) = make_uint2(chunk::pack_rn(v[0], v[1]), chunk::pack_rn(v[2], v[3]));
+}
+
+template <bool KM, bool KN, bool EXACT>
 __device__ __forceinline__ void tile_gemm_body(const GemmArgs& A, const GemmJob& J, int n0, int m0, TileLds& lds) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
   const int all = (J.K + TG - 1) / TG;
   const int s0 = all * (int)blockIdx.y / (int)gridDim.y, s1 = all * ((int)blockIdx.y + 1) / (int)gridDim.y;
-  const TileOperand<KM> X(J.x, J.M, J.K, m0);
-  const TileOperand<KN> W(J.w, J.N, J.K, n0);
+  const TileOperand<KM, EXACT> X(J.x, J.M, J.K, m0, threadIdx.x);
+  const TileOperand<KN, EXACT> W(J.w, J.N, J.K, n0, threadIdx.x);
   f32x4_t acc[2][2];
 #pragma unroll
   for (int i = 0; i < 4; ++i) acc[i >> 1][i & 1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -187,8 +230,8 @@ __device__ __forceinline__ void tile_gemm_body(const GemmArgs& A, const GemmJob&
       u32x4_t wf[2], xf[2];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        xf[t] = TileOperand<KM>::frag(lds[buf][0], wm + 16 * t, kh, r, g);
-        wf[t] = TileOperand<KN>::frag(lds[buf][1], wn + 16 * t, kh, r, g);
+        xf[t] = TileOperand<KM, EXACT>::frag(lds[buf][0], wm + 16 * t, kh, r, g);
+        wf[t] = TileOperand<KN, EXACT>::frag(lds[buf][1], wn + 16 * t, kh, r, g);
       }
 #pragma unroll
       for (int t = 0; t < 2; ++t)
@@ -196,85 +239,84 @@ __device__ __forceinline__ void tile_gemm_body(const GemmArgs& A, const GemmJob&
         for (int u = 0; u < 2; ++u) acc[t][u] = mfma(wf[t], xf[u], acc[t][u]);
     }
   };
-  u32x4_t x0[2], w0[2], x1[2], w1[2];
-  X.load(x0, s0); W.load(w0, s0);
-  X.load(x1, s0 + 1); W.load(w1, s0 + 1);
+  u32x4_t x[AHEAD][2], w[AHEAD][2];
+#pragma unroll
+  for (int j = 0; j < AHEAD; ++j) { X.load(x[j], s0 + j); W.load(w[j], s0 + j); }
   int s = s0;
-  for (; s + 1 < s1; s += 2) {
-    // a buffer is written after the barrier that follows its last readers' step
-    X.store(x0, s, lds[0][0]); W.store(w0, s, lds[0][1]);
-    X.load(x0, s + 2); W.load(w0, s + 2);
-    __syncthreads();
-    compute(0);
-    X.store(x1, s + 1, lds[1][0]); W.store(w1, s + 1, lds[1][1]);
-    X.load(x1, s + 3); W.load(w1, s + 3);
-    __syncthreads();
-    compute(1);
+  // no branches in the loop: the waits for memory then name exactly the loads that a step needs
+  for (; s + AHEAD <= s1; s += AHEAD) {
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) {
+      // a buffer is written after the barrier that follows its last readers' step
+      X.store(x[j], s + j, lds[j & 1][0]); W.store(w[j], s + j, lds[j & 1][1]);
+      X.load(x[j], s + j + AHEAD); W.load(w[j], s + j + AHEAD);
+      __syncthreads();
+      compute(j & 1);
+    }
   }
-  if (s < s1) {
-    X.store(x0, s, lds[0][0]); W.store(w0, s, lds[0][1]);
-    __syncthreads();
-    compute(0);
+#pragma unroll
+  for (int j = 0; j < AHEAD - 1; ++j) {
+    if (s + j < s1) {
+      X.store(x[j], s + j, lds[j & 1][0]); W.store(w[j], s + j, lds[j & 1][1]);
+      __syncthreads();
+      compute(j & 1);
+    }
   }
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int n = n0 + wn + 16 * t + 4 * g, m = m0 + wm + 16 * u + r;
-      if (n >= J.N || m >= J.M) continue;
-      f32x4_t v = acc[t][u];
-      if (A.part != nullptr) {
-        *reinterpret_cast<f32x4_t*>(A.part + ((size_t)blockIdx.y * J.M + m) * J.N + n) = v;
-        continue;
-      }
-      const size_t el = (size_t)m * J.N + n;
-      if (J.aux != nullptr) {
-        const uint2 q = *reinterpret_cast<const uint2*>(static_cast<const bf16_t*>(J.aux) + el);
-        const float h[4] = {__uint_as_float(q.x << 16), __uint_as_float(q.x & 0xffff0000u), __uint_as_float(q.y << 16),
-                            __uint_as_float(q.y & 0xffff0000u)};
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          v[i] = J.act == GEMM_ADD ? v[i] + h[i] : J.act == GEMM_DTANH ? v[i] * (1.f - h[i] * h[i]) : v[i] * (h[i] * (1.f - h[i]));
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = activate(v[i], J.act);
-      }
-      *reinterpret_cast<uint2*>(static_cast<bf16_t*>(J.out) + el) = make_uint2(chunk::pack_rn(v[0], v[1]), chunk::pack_rn(v[2], v[3]));
-    }
+    for (int u = 0; u < 2; ++u) finish(A, J, n0 + wn + 16 * t + 4 * g, m0 + wm + 16 * u + r, acc[t][u]);
+}
+
+// job and tile of a workgroup: along the longer side of the tile grid eight tiles at a time, one per XCD; all tiles across from
+// each on the same XCD
+__device__ __forceinline__ bool tile_of(const GemmArgs& A, int& ji, int& n0, int& m0) {
+  ji = 0;
+  for (int i = 1; i < A.n_jobs; ++i) ji = (int)blockIdx.x >= A.job[i].tile0 ? i : ji;
+  const int M = A.job[ji].M, N = A.job[ji].N;
+  const int mt = (M + TG - 1) / TG, nt = (N + TG - 1) / TG, local = (int)blockIdx.x - A.job[ji].tile0;
+  const int across = mt < nt ? mt : nt;
+  const int p = local / (8 * across) * 8 + local % 8, q = local % (8 * across) / 8;
+  n0 = (mt < nt ? p : q) * TG;
+  m0 = (mt < nt ? q : p) * TG;
+  return n0 < N && m0 < M;
+}
+int tiles_of(const GemmJob& J) {
+  const int mt = (J.M + TG - 1) / TG, nt = (J.N + TG - 1) / TG;
+  return ((mt < nt ? nt : mt) + 7) / 8 * 8 * (mt < nt ? mt : nt);
 }
 
 __global__ __launch_bounds__(256) void tile_gemm_kernel(GemmArgs A) {
   __shared__ __align__(16) TileLds lds;
-  int ji = 0;
-  for (int i = 1; i < A.n_jobs; ++i) ji = (int)blockIdx.x >= A.job[i].tile0 ? i : ji;
+  int ji, n0, m0;
+  if (!tile_of(A, ji, n0, m0)) return;
   const GemmJob J = A.job[ji];
-  // eight column tiles at a time, all row tiles of each on one XCD
-  const int mt = (J.M + TG - 1) / TG, local = (int)blockIdx.x - J.tile0;
-  const int grp = local / (8 * mt), in = local % (8 * mt);
-  const int n0 = (grp * 8 + in % 8) * TG, m0 = in / 8 * TG;
-  if (n0 >= J.N) return;
-  if (J.km) {
-    if (J.kn) tile_gemm_body<true, true>(A, J, n0, m0, lds);
-    else tile_gemm_body<true, false>(A, J, n0, m0, lds);
-  } else {
-    if (J.kn) tile_gemm_body<false, true>(A, J, n0, m0, lds);
-    else tile_gemm_body<false, false>(A, J, n0, m0, lds);
+  switch ((J.km ? 4 : 0) + (J.kn ? 2 : 0) + (J.K % TG == 0 ? 1 : 0)) {
+    case 0: tile_gemm_body<false, false, false>(A, J, n0, m0, lds); break;
+    case 1: tile_gemm_body<false, false, true>(A, J, n0, m0, lds); break;
+    case 2: tile_gemm_body<false, true, false>(A, J, n0, m0, lds); break;
+    case 3: tile_gemm_body<false, true, true>(A, J, n0, m0, lds); break;
+    case 4: tile_gemm_body<true, false, false>(A, J, n0, m0, lds); break;
+    case 5: tile_gemm_body<true, false, true>(A, J, n0, m0, lds); break;
+    case 6: tile_gemm_body<true, true, false>(A, J, n0, m0, lds); break;
+    default: tile_gemm_body<true, true, true>(A, J, n0, m0, lds); break;
   }
 }
 
 }  // namespace
 
-// Parts that a product's K is split into: enough tiles for about two workgroups per CU
+// Parts that a product's K is split into: enough tiles for about two workgroups per CU, at least 256 of k each
 int gemm_split(int M, int64_t K, int64_t N) {
   if (M < GEMM_TILE_ROWS) return 1;
   const int64_t tiles = (M + TG - 1) / TG * ((N + TG - 1) / TG);
-  const int64_t want = 512 / tiles, most = K / (8 * TG);
+  const int64_t want = 512 / tiles, most = K / 256;
   const int64_t n = want < most ? want : most;
   return (int)(n < 1 ? 1 : n > GEMM_MAX_SPLIT ? GEMM_MAX_SPLIT : n);
 }
 
-// Up to 64 rows one row tile of the streaming kernel reads the weights once; K is then a multiple of 32, N of 16.  Beyond,
-// every further row tile would stream them again (256 rows, 2048 channels: 51 us a launch on average against 18 us tiled).
+// Up to 32 rows the streaming kernel (K a multiple of 32, N of 16, no aux): its operand loads touch a cache line per lane,
+// 64 cycles a KiB, which a stream of weights can afford but repeated reads of x cannot (8192 columns of 2048: 14 us at 32
+// rows, 16 at 33, 21 at 64; tiled 15 us up to 128 rows, 22 at 256).
 hipError_t launch_gemm(GemmArgs A, int split, hipStream_t stream) {
   bool skinny = A.part == nullptr;
   int M = 0, tiles = 0;
@@ -286,13 +328,12 @@ hipError_t launch_gemm(GemmArgs A, int split, hipStream_t stream) {
   for (int i = 0; i < A.n_jobs; ++i) {
     GemmJob& J = A.job[i];
     J.tile0 = tiles;
-    tiles += skinny ? J.N / 16 : (J.N + 8 * TG - 1) / (8 * TG) * 8 * ((J.M + TG - 1) / TG);
+    tiles += skinny ? J.N / 16 : tiles_of(J);
   }
   const dim3 block(64 * GEMM_WAVES);
   if (!skinny) hipLaunchKernelGGL(tile_gemm_kernel, dim3(tiles, split), dim3(256), 0, stream, A);
   else if (M <= 16) hipLaunchKernelGGL(skinny_gemm_kernel<1>, dim3(tiles), block, 0, stream, A);
-  else if (M <= 32) hipLaunchKernelGGL(skinny_gemm_kernel<2>, dim3(tiles), block, 0, stream, A);
-  else hipLaunchKernelGGL(skinny_gemm_kernel<4>, dim3(tiles), block, 0, stream, A);
+  else hipLaunchKernelGGL(skinny_gemm_kernel<2>, dim3(tiles), block, 0, stream, A);
   return hipGetLastError();
 }
 

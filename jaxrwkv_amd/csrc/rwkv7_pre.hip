@@ -108,7 +108,7 @@ __global__ __launch_bounds__(PRE_THREADS) void rwkv7_pre_bwd_kernel(PreArgs A) {
       float y[8];
       in(p, el, y);
 #pragma unroll
-      for (int c = 0; c < 8; ++c) x[c] += y[c];
+      for (int c = 0; c < 8; ++c) x[c] = round_io<T>(x[c] + y[c]);      // as their separate sum would be
     };
     if (A.gk2 != nullptr) add(A.gk2, gk);
     if (A.dr != nullptr) {

@@ -151,8 +151,8 @@ using GemmJob = ::hiprwkv_gemm_job;
 constexpr int GEMM_ACT_NONE = 0, GEMM_ACT_TANH = 1, GEMM_ACT_SIGMOID = 2, GEMM_ACT_RELUSQ = 3;      // f without aux
 constexpr int GEMM_ADD = 0, GEMM_DTANH = 1, GEMM_DSIGMOID = 2;                                      // f with aux
 constexpr int GEMM_MAX_JOBS = HIPRWKV_GEMM_MAX_JOBS;
-constexpr int GEMM_TILE_ROWS = 65;     // rows from which the LDS-tiled kernel takes over
-constexpr int GEMM_MAX_SPLIT = 4;
+constexpr int GEMM_TILE_ROWS = 33;     // rows from which the kernel with LDS tiles takes over
+constexpr int GEMM_MAX_SPLIT = 8;
 struct GemmArgs {
   GemmJob job[GEMM_MAX_JOBS];
   int n_jobs;

@@ -68,8 +68,9 @@ def test_blocks_equal_the_steps(L, B, T, C, dtype, monkeypatch):
 @pytest.mark.parametrize("M,N,K", [(8, 8, 8), (64, 64, 64), (72, 200, 40), (333, 64, 96), (1000, 136, 2048)])
 @pytest.mark.parametrize("km,kn", [(0, 0), (0, 1), (1, 0), (1, 1)])
 def test_grouped_products(M, N, K, km, kn):
-    """One rounding of the result (2^-8) plus fp32 sums of products of bf16 values, and 2e-3 of the rms for the hardware
-    exponential behind tanh and sigmoid."""
+    """The sum is rounded to bf16 before f and the result after it, each by at most 2^-8 of its size.  relu(x)^2 doubles the
+    first: 3 * 2^-8 relative; where aux is added the first is relative to the product (below 5 here) and not to the sum: 5 * 2^-8,
+    2e-2 of the rms of about 1."""
     from jaxrwkv_amd import blocks7
     if km:
         M = (M + 7) // 8 * 8
@@ -84,5 +85,5 @@ def test_grouped_products(M, N, K, km, kn):
     outs = [torch.full((M, N), 7.0, device="cuda", dtype=torch.bfloat16) for _ in want]
     blocks7._gemm([(o, x, w, km, kn, i if i < 4 else i - 4, None if i < 4 else aux) for i, o in enumerate(outs)])
     for i, (o, ref) in enumerate(zip(outs, want)):
-        bound = 2.0 ** -8 * ref.abs() + 2e-3 * ref.pow(2).mean().sqrt()
+        bound = 3 * 2.0 ** -8 * ref.abs() + 2e-2 * ref.pow(2).mean().sqrt()
         assert ((o.float() - ref).abs() <= bound).all(), (i, ((o.float() - ref).abs() / bound).max().item())
