@@ -7,6 +7,7 @@ stacked arrays, and adds up nothing that a kernel can add on its way (the second
 residual's).  The low-rank factors of decay, gates and value residual run several to a launch (``hiprwkv_gemm``) in bf16.
 """
 import torch
+from torch.autograd.function import once_differentiable
 
 from . import _lib, ops
 from .rwkv7 import HipRWKV
@@ -279,6 +280,7 @@ class _Blocks(torch.autograd.Function):
         return x, dx, new_state
 
     @staticmethod
+    @once_differentiable              # create_graph=True: first cotangents as ever, an error for those of the cotangents
     def backward(ctx, g_x, g_dx, g_state):
         tensors = ctx.saved_tensors
         saved, v_first, ns, length = _unpack(ctx.places, tensors)

@@ -87,3 +87,18 @@ def test_grouped_products(M, N, K, km, kn):
     for i, (o, ref) in enumerate(zip(outs, want)):
         bound = 3 * 2.0 ** -8 * ref.abs() + 2e-2 * ref.pow(2).mean().sqrt()
         assert ((o.float() - ref).abs() <= bound).all(), (i, ((o.float() - ref).abs() / bound).max().item())
+
+
+def test_create_graph_keeps_the_first_cotangents():
+    """A caller that asks for a graph of the cotangents gets the cotangents as without; only differentiating those again is an
+    error."""
+    from jaxrwkv_amd.model7 import RWKV7, randomize_weights
+    params = randomize_weights(3, 2, 128, 96, dtype=torch.bfloat16, device="cuda", zero_init=False)
+    w = params["blocks"]["ffn"]["key"]["weight"].requires_grad_()
+    tok = torch.randint(0, 96, (2, 20), device="cuda", generator=torch.Generator("cuda").manual_seed(1))
+    logits, _ = RWKV7.forward(params, tok, RWKV7.default_state(params, 2))
+    plain, = torch.autograd.grad(logits.float().square().mean(), w, retain_graph=True)
+    graph, = torch.autograd.grad(logits.float().square().mean(), w, create_graph=True)
+    assert torch.equal(plain, graph)
+    with pytest.raises(RuntimeError):
+        torch.autograd.grad(graph.float().sum(), w)
