@@ -122,6 +122,17 @@ int hiprwkv_wkv7_fwd(hiprwkv_stream stream, int io_dtype, int state_dtype,
                      const uint32_t* length, const uint8_t* new_starts,
                      void* out, void* sa, void* new_s, unsigned flags);
 
+/* The same with `workspace` (hiprwkv_wkv7_fwd_workspace_bytes, 0 where it is of no use; NULL: as hiprwkv_wkv7_fwd).  Where
+ * B*H leaves most of the GPU idle, bf16 sequences are cut into parts whose summaries (state maps) are made first.  A
+ * part whose hand-shake fails counts as one of its own in hiprwkv_handshake_failures and makes its own rows NaN. */
+size_t hiprwkv_wkv7_fwd_workspace_bytes(int io_dtype, int64_t B, int64_t T, int64_t H, int64_t N);
+int hiprwkv_wkv7_fwd_parts(hiprwkv_stream stream, int io_dtype, int state_dtype,
+                           int64_t B, int64_t T, int64_t H, int64_t N,
+                           const void* w, const void* r, const void* k, const void* v,
+                           const void* a, const void* b, const void* s,
+                           const uint32_t* length, const uint8_t* new_starts,
+                           void* out, void* sa, void* new_s, void* workspace, size_t workspace_bytes, unsigned flags);
+
 /* A decode step (T <= HIPRWKV_SMALL_T tokens per sequence) on a state that lives inside the packed model state of the
  * reference: there a sequence's state is (L, 2+N, C) and layer l's rows 2.. are the (H,N,N) WKV state, flat
  * (rwkv7.py:176-180 default_state, :254-260 the slice and reshape around inner_loop), so with a batch axis in front

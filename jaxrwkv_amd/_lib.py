@@ -46,6 +46,8 @@ SIGNATURES = {
     "hiprwkv_handshake_failures": (_int, [_vp, ctypes.POINTER(ctypes.c_uint)]),
     "hiprwkv_numeric_events": (_int, [_vp, ctypes.POINTER(ctypes.c_uint)]),
     "hiprwkv_wkv7_fwd": (_int, [_vp, _int, _int, _i64, _i64, _i64, _i64] + [_vp] * 7 + [_vp, _vp] + [_vp, _vp, _vp, _u32]),
+    "hiprwkv_wkv7_fwd_workspace_bytes": (_sz, [_int] + [_i64] * 4),
+    "hiprwkv_wkv7_fwd_parts": (_int, [_vp, _int, _int, _i64, _i64, _i64, _i64] + [_vp] * 7 + [_vp, _vp] + [_vp] * 4 + [_sz, _u32]),
     "hiprwkv_wkv7_step": (_int, [_vp, _int, _int, _i64, _i64, _i64, _i64] + [_vp] * 6 + [_vp, _i64] + [_vp, _vp]
                           + [_vp, _vp, _i64, _u32]),
     "hiprwkv_wkv7_bwd_workspace_bytes": (_sz, [_i64] * 4),

@@ -153,6 +153,19 @@ int hiprwkv_wkv7_fwd(hiprwkv_stream stream, int io_dtype, int state_dtype, int64
                      const void* w, const void* r, const void* k, const void* v, const void* a, const void* b,
                      const void* s, const uint32_t* length, const uint8_t* new_starts, void* out, void* sa,
                      void* new_s, unsigned flags) {
+  return hiprwkv_wkv7_fwd_parts(stream, io_dtype, state_dtype, B, T, H, N, w, r, k, v, a, b, s, length, new_starts, out, sa, new_s,
+                                nullptr, 0, flags);
+}
+
+size_t hiprwkv_wkv7_fwd_workspace_bytes(int io_dtype, int64_t B, int64_t T, int64_t H, int64_t N) {
+  if (io_dtype != HIPRWKV_BF16 || N != 64 || B <= 0 || T <= HIPRWKV_SMALL_T || H <= 0 || B * H > 0x7fffffffLL) return 0;
+  return wkv7_fwd_parts_bytes(B * H, T);
+}
+
+int hiprwkv_wkv7_fwd_parts(hiprwkv_stream stream, int io_dtype, int state_dtype, int64_t B, int64_t T, int64_t H, int64_t N,
+                           const void* w, const void* r, const void* k, const void* v, const void* a, const void* b,
+                           const void* s, const uint32_t* length, const uint8_t* new_starts, void* out, void* sa,
+                           void* new_s, void* workspace, size_t workspace_bytes, unsigned flags) {
   int rc = check_matrix_shape("wkv7_fwd", io_dtype, state_dtype, B, T, H, N);
   if (rc) return rc;
   if ((rc = check_flags("wkv7_fwd", flags)) != HIPRWKV_OK) return rc;
@@ -162,6 +175,10 @@ int hiprwkv_wkv7_fwd(hiprwkv_stream stream, int io_dtype, int state_dtype, int64
     if (!aligned16(p)) return fail(HIPRWKV_EINVAL, "wkv7_fwd: tensor pointers must be 16-byte aligned");
   }
   if (sa && !aligned16(sa)) return fail(HIPRWKV_EINVAL, "wkv7_fwd: sa must be 16-byte aligned");
+  if (workspace && !aligned16(workspace)) return fail(HIPRWKV_EINVAL, "wkv7_fwd: workspace must be 16-byte aligned");
+  const size_t need = workspace != nullptr ? hiprwkv_wkv7_fwd_workspace_bytes(io_dtype, B, T, H, N) : 0;
+  if (workspace_bytes < need)
+    return fail(HIPRWKV_ENOSPACE, "wkv7_fwd: workspace has %zu bytes, %zu needed", workspace_bytes, need);
   Wkv7Args A;
   memset(&A, 0, sizeof(A));
   A.B = B; A.T = T; A.H = H;
@@ -171,6 +188,7 @@ int hiprwkv_wkv7_fwd(hiprwkv_stream stream, int io_dtype, int state_dtype, int64
   A.io_f32 = io_dtype == HIPRWKV_F32; A.st_f32 = state_dtype == HIPRWKV_F32;
   A.flags = flags;
   A.status = status_word();
+  A.parts = need != 0 ? workspace : nullptr;
   // T <= 8 (decode) runs on the small-T kernel; otherwise the chunked matrix-core kernels (fp16 operands for bf16
   // I/O, fp32 operands for fp32 I/O); HIPRWKV_FORCE_SEQ selects the sequential kernel
   const bool small_t = T <= HIPRWKV_SMALL_T && !(flags & HIPRWKV_NO_SMALL_T);

@@ -99,13 +99,15 @@ __device__ __forceinline__ rsrc_t make_rsrc(const void* base) {
 // bounded wait runs out while every wave still ends normally.
 constexpr unsigned FLAG_DROP_PUBLISH = 0x100u;
 
-// NaN into this head's rows of a (B,T,H,64) tensor; elem = bytes per element (2: bf16, 4: fp32)
-__device__ __forceinline__ void poison_token_rows(void* base, int elem, int64_t b, int64_t h, int64_t T, int64_t H) {
+// NaN into this head's rows (t0 .. t0 + rows - 1, all T by default) of a (B,T,H,64) tensor; elem = bytes per element (2: bf16, 4: fp32)
+__device__ __forceinline__ void poison_token_rows(void* base, int elem, int64_t b, int64_t h, int64_t T, int64_t H,
+                                                  int64_t t0 = 0, int64_t rows = -1) {
   if (base == nullptr) return;
+  if (rows < 0) rows = T;
   const int pieces = 64 * elem / 16;
   const uint32_t nan = elem == 2 ? 0x7fc07fc0u : 0x7fc00000u;
-  for (int64_t i = threadIdx.x; i < T * pieces; i += blockDim.x) {
-    const int64_t t = i / pieces;
+  for (int64_t i = threadIdx.x; i < rows * pieces; i += blockDim.x) {
+    const int64_t t = t0 + i / pieces;
     const int pc = (int)(i % pieces);
     char* p = static_cast<char*>(base) + ((((size_t)b * T + t) * H + h) * 64) * elem + 16 * pc;
     *reinterpret_cast<uint4*>(p) = make_uint4(nan, nan, nan, nan);

@@ -41,6 +41,9 @@ using namespace chunk;
 constexpr int NPROD = 8;          // producer waves; producer p owns chunks p, p + NPROD, ...
 constexpr int RING = 10;          // slots in flight
 
+// What a workgroup does with its sequence (see wkv7_fwd_kernel): all of it, a part's summary, or a part.
+enum { WHOLE = 0, SUMMARY = 1, PART = 2 };
+
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
@@ -111,6 +114,7 @@ struct Raw {
 };
 
 // Loads always touch a valid token (the last one of the sequence for lanes beyond it); mask_raw zeroes those lanes.
+template <int MODE>
 __device__ __forceinline__ void load_raw(Raw& x, const Wkv7Args& A, int64_t b, int64_t h, int64_t c0, int lane) {
   const int t = lane & 15, g = lane >> 4;
   const int64_t tok = (c0 + t < A.T) ? c0 + t : A.T - 1;
@@ -119,7 +123,8 @@ __device__ __forceinline__ void load_raw(Raw& x, const Wkv7Args& A, int64_t b, i
     o[0] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(p) + off);
     o[1] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(p) + off + 64);
   };
-  ld(A.r, x.r); ld(A.w, x.w); ld(A.k, x.k); ld(A.v, x.v); ld(A.a, x.a); ld(A.b, x.b);
+  if (MODE != SUMMARY) ld(A.r, x.r);
+  ld(A.w, x.w); ld(A.k, x.k); ld(A.v, x.v); ld(A.a, x.a); ld(A.b, x.b);
 }
 __device__ __forceinline__ void mask_raw(Raw& x, int nvalid, int lane) {
   if (nvalid != CK) {
@@ -144,6 +149,8 @@ __device__ __forceinline__ uint4 pack_h8(const float (&f)[8]) {
 // priority as it advances through its chunk evens that out and makes an isolated launch 4 % faster, but launches
 // issued back to back (the GPU at its power limit) 2.8 % slower, so this kernel's producers stay at the default
 // priority; the WKV6 forward, where the same steps gain 3.5 % back to back, has them.
+// SUMMARY: without what only y needs (r and its products).
+template <int MODE>
 __device__ __forceinline__ void produce(int lane, const Raw& x, const ChunkFlags& F, Slot* __restrict__ slot,
                                         SnapSlot* __restrict__ snap, unsigned* events) {
   const int t = lane & 15, g = lane >> 4;
@@ -216,7 +223,8 @@ __device__ __forceinline__ void produce(int lane, const Raw& x, const ChunkFlags
     float fat[8], fqt[8], fkh[8], fbh[8], fke[8], fbe[8];
     {
       float fr[8], fk[8], fb[8];
-      unpack8(x.r[hf], fr); unpack8(x.k[hf], fk); unpack8(x.b[hf], fb);
+      if (MODE != SUMMARY) unpack8(x.r[hf], fr);
+      unpack8(x.k[hf], fk); unpack8(x.b[hf], fb);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         // cap_chunk_decay keeps the running sums at or above MIN_CUM_L2: exp2(-l2) is finite
@@ -228,7 +236,7 @@ __device__ __forceinline__ void produce(int lane, const Raw& x, const ChunkFlags
         // multiplies a zero.
         const float fa0 = (t == 0) ? fa[e] : 0.f;
         fat[e] = fmaf(fa[e], row_prev0(E[e]), fa0);
-        fqt[e] = fr[e] * E[e];
+        fqt[e] = MODE == SUMMARY ? 0.f : fr[e] * E[e];
         fkh[e] = fk[e] * einv;
         fbh[e] = fb[e] * einv;
         // times the decay from the (last) segment start to the chunk end
@@ -287,7 +295,7 @@ __device__ __forceinline__ void produce(int lane, const Raw& x, const ChunkFlags
         *reinterpret_cast<uint2*>(row + e0 + 8) = make_uint2(v.z, v.w);
       };
       put(slot->AQ[0][t], ah);
-      put(slot->AQ[1][t], qh);
+      if (MODE != SUMMARY) put(slot->AQ[1][t], qh);
     }
     // ---- bf16 hi/lo pairs of the Gram operands and the partial Gram sums over this half's keys
     u32x4_t at_h, at_l, qt_h, qt_l, kh_h, kh_l, bh_h, bh_l;
@@ -309,6 +317,7 @@ __device__ __forceinline__ void produce(int lane, const Raw& x, const ChunkFlags
       Gab = mfma(bA, aB, Gab);      // [m][n] = bh_m . at_n
       GabT = mfma(aA, bB, GabT);    // [m][n] = at_m . bh_n
       G1 = mfma(kA, aB, G1);        // Mka[m][n] = kh_m . at_n
+      if (MODE == SUMMARY) continue;
       G2 = mfma(bA, qB, G2);        // Mbr[m][n] = bh_m . qt_n
       G3 = mfma(kA, qB, G3);        // Mkr[m][n] = kh_m . qt_n
     }
@@ -354,7 +363,7 @@ __device__ __forceinline__ void produce(int lane, const Raw& x, const ChunkFlags
   }
   slot->P[lane] = pack_h4(Pm);
   slot->Ka[lane] = pack_h4(G1);
-  {
+  if (MODE != SUMMARY) {
     const u32x2_t br = pack_h4(G2), kr = pack_h4(G3);
     slot->BrKr[lane] = u32x4_t{br[0], br[1], kr[0], kr[1]};
     const f16x4_t krh = __builtin_bit_cast(f16x4_t, kr);
@@ -407,17 +416,20 @@ struct Ops {
   int keep_end;
 };
 
+template <int MODE>
 __device__ __forceinline__ void load_ops(Ops& o, const Slot* __restrict__ slot, const LaneOffs& f) {
   const char* const sb = reinterpret_cast<const char*>(slot);
 #pragma unroll
-  for (int ar = 0; ar < 2; ++ar)
+  for (int ar = 0; ar < (MODE == SUMMARY ? 1 : 2); ++ar)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
       o.aq[ar][j] = *reinterpret_cast<const u32x4_t*>(sb + f.aq + ar * (CK * RS * 2) + j * 64);
   o.P = *reinterpret_cast<const u32x2_t*>(sb + f.l8);
   o.Ka = *reinterpret_cast<const u32x2_t*>(sb + f.l8 + (offsetof(Slot, Ka) - offsetof(Slot, P)));
-  o.BrKr = *reinterpret_cast<const u32x4_t*>(sb + f.l16);
-  o.KrLo = *reinterpret_cast<const u32x2_t*>(sb + f.l8 + (offsetof(Slot, KrLo) - offsetof(Slot, P)));
+  if (MODE != SUMMARY) {
+    o.BrKr = *reinterpret_cast<const u32x4_t*>(sb + f.l16);
+    o.KrLo = *reinterpret_cast<const u32x2_t*>(sb + f.l8 + (offsetof(Slot, KrLo) - offsetof(Slot, P)));
+  }
   o.vv = lds_tr4(reinterpret_cast<const uint16_t*>(sb + f.vv));
   o.keep_end = slot->keep_end;
 }
@@ -461,11 +473,12 @@ __device__ __forceinline__ void store_state_tile(void* p, int f32, size_t off, c
 
 // The state-dependent part of one chunk.  `next` is the slot of the chunk handled after this one (null after the
 // last one); `next_ready` waits until its producer has published it.  Returns false when that wait ran out.
-template <bool PARK, class PeekNext, class WaitNext>
+// `emit` (PART only): whether the chunk's outputs are this workgroup's to write.
+template <bool PARK, int MODE, class PeekNext, class WaitNext>
 __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restrict__ slot,
                                         const Slot* __restrict__ next, const SnapSlot* __restrict__ snapslot,
                                         const Wkv7Args& A, int64_t b, int64_t h, int nvalid, bool is_snap, bool q2drop,
-                                        OutCursor& oc, PeekNext&& peek_next, WaitNext&& next_ready) {
+                                        bool emit, OutCursor& oc, PeekNext&& peek_next, WaitNext&& next_ready) {
   const int lane = C.lane, g = lane >> 4;
   const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
   // the next chunk's sequence number, requested now and looked at after the W / SA / Y chain
@@ -489,24 +502,27 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
     Sh[j] = u32x4_t{pack_h(C.S[2 * j][0], C.S[2 * j][1]), pack_h(C.S[2 * j][2], C.S[2 * j][3]),
                     pack_h(C.S[2 * j + 1][0], C.S[2 * j + 1][1]), pack_h(C.S[2 * j + 1][2], C.S[2 * j + 1][3])};
   f32x4_t W = zero4;              // [token 4g+i][value n], two interleaved accumulation chains
-  f32x4_t Y = mfma_h16(o.KrLo, o.vv, zero4);    // the low part of Mkr^T V^T: no state in it, off the critical path
-  mfma_shape_fence(Y);                          // a K = 16 result enters a K = 32 chain
+  f32x4_t Y = zero4;
+  if (MODE != SUMMARY) {
+    Y = mfma_h16(o.KrLo, o.vv, zero4);          // the low part of Mkr^T V^T: no state in it, off the critical path
+    mfma_shape_fence(Y);                        // a K = 16 result enters a K = 32 chain
+  }
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     W = mfma_h(o.aq[0][j], Sh[j], W);
-    Y = mfma_h(o.aq[1][j], Sh[j], Y);
+    if (MODE != SUMMARY) Y = mfma_h(o.aq[1][j], Sh[j], Y);
   }
   mfma_shape_fence(W);                          // a K = 32 result enters a K = 16 instruction: the pairing that fails
   W = mfma_h16(o.Ka, o.vv, W);                  // W += Mka^T V^T
   const f32x4_t SA = mfma_h16(o.P, pack_h4(W), zero4);
   const u32x2_t sp = pack_h4(SA);
   const u32x4_t sv = {sp[0], sp[1], o.vv[0], o.vv[1]};   // SA^T (tokens 4g..4g+3) then v^T: B operand of Y and the update
-  Y = mfma_h(o.BrKr, sv, Y);                    // Y += Mbr^T SA^T + Mkr^T V^T
+  if (MODE != SUMMARY) Y = mfma_h(o.BrKr, sv, Y);   // Y += Mbr^T SA^T + Mkr^T V^T
   // everything fetched a chunk ahead is dead now: fetch the next chunk's into the same registers
   bool ok = true;
   if (next != nullptr) {
     ok = next_ready(peeked);
-    load_ops(o, next, C.off);
+    load_ops<MODE>(o, next, C.off);
   }
   // state snapshot for `length` (one chunk per sequence)
   if (is_snap) {
@@ -539,6 +555,7 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
 #pragma unroll
     for (int tile = 0; tile < 4; ++tile) C.S[tile] = mfma_h(up[tile], sv, zero4);
   }
+  if (MODE == SUMMARY) return ok;
   // outputs: register i is token 4g+i, lanes n = 16 consecutive values
   const uint32_t y01 = pack_rn(Y[0], Y[1]), y23 = pack_rn(Y[2], Y[3]);
   if (PARK) {
@@ -553,7 +570,9 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
     *reinterpret_cast<uint16_t*>(yp + 3 * RS * 2) = (uint16_t)(y23 >> 16);
   }
   char* const yl = oc.y + (size_t)oc.voff * 2;
-  if (nvalid == CK) {
+  if (MODE == PART && !emit) {
+    rare_path();
+  } else if (nvalid == CK) {
     if (!PARK) {
       *reinterpret_cast<uint16_t*>(yl) = (uint16_t)(y01 & 0xffffu);
       *reinterpret_cast<uint16_t*>(yl + oc.tok_bytes) = (uint16_t)(y01 >> 16);
@@ -600,14 +619,95 @@ __device__ __forceinline__ void flush_y(const Slot* __restrict__ slot, const Wkv
   if (r + 8 < nvalid) *reinterpret_cast<uint4*>(y0 + (size_t)8 * A.H * 128) = hi;
 }
 
+// A part's summary: S_end = S_start M + B for the state entering and leaving it, one record per (sequence, head, part) in fp32,
+// laid out as the operands that the fold takes (rows of 256 bytes instead: 64 cycles a KiB, 2.3 us a predecessor), and eight
+// words (one per consumer wave of the two workgroups that make it) that are not zero where the summary must not be used.
+struct PartSum {
+  f32x4_t M[4][4][64];     // [tile][jt], lane (x, g): M[key 16 tile + 4g + i][key 16 jt + x]
+  f32x4_t B[4][4][64];     // [q][tile]: consumer q's state tiles
+};
+constexpr float PART_MAX_GAIN = 4.f;
+__device__ __forceinline__ PartSum* part_sum(const Wkv7Args& A, int64_t head, int part) {
+  return reinterpret_cast<PartSum*>(A.parts) + head * (A.n_part - 1) + part;
+}
+__device__ __forceinline__ int* part_flags(const Wkv7Args& A, int64_t head, int part) {
+  return reinterpret_cast<int*>(reinterpret_cast<PartSum*>(A.parts) + A.B * A.H * (A.n_part - 1)) +
+         (head * (A.n_part - 1) + part) * 8;
+}
+
+// The state entering part `part` > 0, S <- S M + B over the summaries before it, in fp32.  The state tiles are the B operand
+// of the products M^T S^T as they are (k-slot g of step i of a tile is key 16 tile + 4g + i); a predecessor costs a consumer 64
+// instructions of 32 cycles and 20 KiB from the cache.
+__device__ __forceinline__ void fold_parts(Consumer& C, const Wkv7Args& A, int64_t head, int part) {
+#pragma unroll
+  for (int tile = 0; tile < 4; ++tile) C.S[tile] = part_sum(A, head, 0)->B[C.q][tile][C.lane];
+  if (part < 2) return;
+  // a predecessor's 20 KiB are requested while the one before it is multiplied
+  f32x4_t acc[4], m[4][4];
+  auto load_m = [&](int p, int tile) {
+#pragma unroll
+    for (int jt = 0; jt < 4; ++jt)
+      m[tile][jt] = part_sum(A, head, p)->M[tile][jt][C.lane];
+  };
+#pragma unroll
+  for (int jt = 0; jt < 4; ++jt) acc[jt] = part_sum(A, head, 1)->B[C.q][jt][C.lane];
+#pragma unroll
+  for (int tile = 0; tile < 4; ++tile) load_m(1, tile);
+  for (int p = 1; p < part; ++p) {
+    const int next = p + 1 < part ? p + 1 : p;
+    f32x4_t b[4];
+#pragma unroll
+    for (int jt = 0; jt < 4; ++jt) b[jt] = part_sum(A, head, next)->B[C.q][jt][C.lane];
+#pragma unroll
+    for (int tile = 0; tile < 4; ++tile) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int jt = 0; jt < 4; ++jt) acc[jt] = __builtin_amdgcn_mfma_f32_16x16x4f32(m[tile][jt][i], C.S[tile][i], acc[jt], 0, 0, 0);
+      load_m(next, tile);
+    }
+#pragma unroll
+    for (int jt = 0; jt < 4; ++jt) {
+      C.S[jt] = acc[jt];
+      acc[jt] = b[jt];
+    }
+  }
+}
+// writes a consumer's rows of one half of a summary; not zero if it must not be used
+__device__ __forceinline__ int store_summary(const Consumer& C, PartSum& ps, bool map) {
+  const int x = C.lane & 15, g = C.lane >> 4;
+  const float limit = map ? PART_MAX_GAIN : 3.0e38f;
+  bool bad = false;
+#pragma unroll
+  for (int tile = 0; tile < 4; ++tile) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      bad |= !(fabsf(C.S[tile][i]) <= limit);
+      if (map) reinterpret_cast<float*>(&ps.M[C.q][tile][16 * (x >> 2) + 4 * g + i])[x & 3] = C.S[tile][i];
+    }
+    if (!map) ps.B[C.q][tile][C.lane] = C.S[tile];
+  }
+  return __ballot(bad) != 0 ? 1 : 0;
+}
+
 }  // namespace
 
 // Step j handles chunk j in slot j % RING.  Producer p fills the slot once every consumer has released step j - RING,
 // then publishes ready = j + 1; consumers take the steps in order.  Every wait is for a strictly earlier step, so
 // the hand-shake cannot cycle.
-// PARK: the consumers leave y in the slot and the producers write it out (see `consume`); steps nch .. nch + RING - 1
+// PARK: the consumers leave y in the slot and the producers write it out (see `consume`); steps n .. n + RING - 1
 // of the producers then produce nothing and only write out the y of the last RING chunks.
-template <bool PARK>
+//
+// MODE.  A workgroup per (sequence, head) leaves most of the GPU idle where there are few of them, and the chunks of one form a
+// serial chain (0.7 us each).  The sequence is then cut into n_part parts (wkv7_fwd_parts), in two launches:
+// SUMMARY  one workgroup runs a part from a zero state (part 0: from the given one), which leaves B; another from the
+//          identity with v = 0, which leaves M.  No y.
+// PART     a workgroup per part folds the summaries before it into its entering state (fp32 matrix instructions) and runs.
+// Where a summary is not usable (M amplifies by more than PART_MAX_GAIN, which a decayed state with removal along a unit vector
+// does not, or something in it is not finite), the workgroups after it run its chunks themselves, without output.
+// Measured per call (whole -> parts): B=1 T=2047, H=32 89.6 -> 57.1 us (5 parts), H=12 89.4 -> 47.6 (10); T=4096 H=12 169 -> 63; with
+// sa 193 -> 64.  Of the 57: 24 the summaries, 33 the parts (about 4 us each to start, 0.66 us a chunk, 1.2 us a predecessor).
+template <bool PARK, int MODE>
 __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_kernel(Wkv7Args A) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Slot* slots = reinterpret_cast<Slot*>(smem_raw);
@@ -615,10 +715,31 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_kernel(Wkv7Args
   Sync* sy = reinterpret_cast<Sync*>(smem_raw + RING * sizeof(Slot) + sizeof(SnapSlot));
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int64_t b = blockIdx.x / A.H, h = blockIdx.x % A.H;
+  // head, part and (SUMMARY) which half of the summary
+  const int per_head = MODE == SUMMARY ? 2 * A.n_part - 3 : MODE == PART ? A.n_part : 1;
+  const int64_t head = MODE == WHOLE ? (int64_t)blockIdx.x : (int64_t)(blockIdx.x / per_head);
+  const int unit = MODE == WHOLE ? 0 : (int)(blockIdx.x % per_head);
+  const bool map = MODE == SUMMARY && unit >= A.n_part - 1;           // this workgroup makes M
+  const int part = MODE == SUMMARY && map ? unit - (A.n_part - 2) : unit;
+  const int64_t b = head / A.H, h = head % A.H;
   int64_t L = seq_length(A.length, b, A.T, A.flags);
   L = L < A.T ? L : A.T;
   const int nch = (int)((A.T + CK - 1) / CK);
+  // chunks j0 .. j0 + n - 1; output from chunk j_out on
+  int j0 = 0, n = nch, j_out = 0, part0 = 0;
+  if (MODE != WHOLE) {
+    j_out = part * A.part_chunks;
+    const int end = j_out + A.part_chunks < nch ? j_out + A.part_chunks : nch;
+    part0 = part;
+    if (MODE == PART && part > 0) {
+      // the first part before this one whose summary is not usable; a lane looks at four of its eight words
+      const int4 f = lane < 2 * part ? *reinterpret_cast<const int4*>(part_flags(A, head, 0) + 4 * lane) : make_int4(0, 0, 0, 0);
+      const uint64_t bad = __ballot((f.x | f.y | f.z | f.w) != 0);
+      if (bad != 0) part0 = __builtin_ctzll(bad) >> 1;
+    }
+    j0 = part0 * A.part_chunks;
+    n = end - j0;
+  }
   // the returned state is the reset state there (associative-scan rule), a constant
   const bool q2drop = (A.flags & 1u) && L < A.T && A.ns != nullptr && A.ns[b * A.T + L] != 0;
   if (threadIdx.x < sizeof(Sync) / sizeof(int)) reinterpret_cast<int*>(sy)[threadIdx.x] = 0;
@@ -629,9 +750,12 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_kernel(Wkv7Args
   // faster than one consumer and two producers on every SIMD: a producer's vector instructions delay the consumer
   // that shares its SIMD, and this way each consumer has one such neighbour instead of two.
   static_assert(NPROD == 8, "the wave-to-role map below is written for 4 consumers and 8 producers");
-  const bool is_cons = (wave & 2) == 0 && wave < 8;
-  const int cq = (wave & 1) | ((wave >> 1) & 2);                                 // waves 0,1,4,5 -> 0..3
-  const int pp = wave >= 8 ? wave - 4 : ((wave & 1) | ((wave >> 1) & 2));        // waves 2,3,6,7 -> 0..3, 8..11 -> 4..7
+  // A part with a long fold in front (64 instructions of 32 cycles per consumer and predecessor) has one consumer per SIMD.
+  const bool spread = MODE == PART && part0 > 4;
+  const bool is_cons = spread ? wave < NCONS : (wave & 2) == 0 && wave < 8;
+  const int cq = spread ? wave : (wave & 1) | ((wave >> 1) & 2);                 // waves 0,1,4,5 -> 0..3
+  const int pp = spread || wave >= 8 ? wave - NCONS : ((wave & 1) | ((wave >> 1) & 2));         // 2,3,6,7 -> 0..3, 8..11 -> 4..7
+  int unusable = 0;                                                              // SUMMARY: this wave's word
   if (is_cons) {
     // the chunk-to-chunk dependency runs through the consumers: let them issue ahead of the producers
     __builtin_amdgcn_s_setprio(3);
@@ -640,33 +764,44 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_kernel(Wkv7Args
     C.lane = lane;
     C.off = lane_offs(cq, lane);
     const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
+    if (MODE == WHOLE || (part0 == 0 && !map)) {
 #pragma unroll
-    for (int tile = 0; tile < 4; ++tile) C.S[tile] = load_state_tile(A.s, A.st_f32, state_off(A, b, h, cq, lane, tile));
+      for (int tile = 0; tile < 4; ++tile) C.S[tile] = load_state_tile(A.s, A.st_f32, state_off(A, b, h, cq, lane, tile));
+    } else if (MODE == SUMMARY) {
+#pragma unroll
+      for (int tile = 0; tile < 4; ++tile)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          C.S[tile][i] = map && 16 * cq + (lane & 15) == 16 * tile + 4 * (lane >> 4) + i ? 1.f : 0.f;
+    } else {
+      fold_parts(C, A, head, part0);
+    }
     // length == 0: the returned state is the input state (rwkv7.py:203), or the reset state under the associative rule
-    if (L == 0) {
+    if (L == 0 && (MODE == WHOLE || (MODE == PART && part == 0))) {
 #pragma unroll
       for (int tile = 0; tile < 4; ++tile)
         store_state_tile(A.new_s, A.st_f32, state_off(A, b, h, cq, lane, tile), q2drop ? zero4 : C.S[tile]);
     }
     OutCursor oc;
     oc.tok_bytes = (size_t)A.H * 64 * 2;
-    const size_t el0 = (((size_t)b * A.T) * A.H + h) * 64;
+    const size_t el0 = (((size_t)b * A.T + (size_t)j0 * CK) * A.H + h) * 64;
     oc.y = reinterpret_cast<char*>(A.out) + el0 * 2;
     oc.sa = A.sa ? reinterpret_cast<char*>(A.sa) + el0 * 2 : nullptr;
     oc.voff = (uint32_t)((4 * (lane >> 4)) * (int)A.H * 64 + 16 * cq + (lane & 15));
-    const int csnap = L >= 1 ? (int)((L - 1) / CK) : -1;
+    // the chunk of token length-1, if this workgroup writes the returned state
+    const int csnap = MODE != SUMMARY && L >= 1 && (int)((L - 1) / CK) >= j_out ? (int)((L - 1) / CK) - j0 : -1;
     Ops ops;
     bool ok = true;
-    if (nch > 0) {
+    if (n > 0) {
       ok = wait_ready(sy, 0, 1);
-      load_ops(ops, &slots[0], C.off);
+      load_ops<MODE>(ops, &slots[0], C.off);
     }
     int si = 0;                       // j % RING, kept by counting
-    for (int j = 0; j < nch && ok; ++j) {
-      const int nvalid = (j + 1 < nch || A.T % CK == 0) ? CK : (int)(A.T % CK);
+    for (int j = 0; j < n && ok; ++j) {
+      const int nvalid = (j0 + j + 1 < nch || A.T % CK == 0) ? CK : (int)(A.T % CK);
       const int sn = (si + 1 == RING) ? 0 : si + 1;
-      const Slot* next = (j + 1 < nch) ? &slots[sn] : nullptr;
-      ok = consume<PARK>(C, ops, &slots[si], next, snapslot, A, b, h, nvalid, j == csnap, q2drop, oc,
+      const Slot* next = (j + 1 < n) ? &slots[sn] : nullptr;
+      ok = consume<PARK, MODE>(C, ops, &slots[si], next, snapslot, A, b, h, nvalid, j == csnap, q2drop, j0 + j >= j_out, oc,
                    [&]() { return peek_ready(sy, sn); },
                    [&](int peeked) {
                      return wait_ready_peeked(sy, sn, j + 2, peeked);
@@ -675,20 +810,25 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_kernel(Wkv7Args
       if (lane == 0) __hip_atomic_store(&sy->consumed[cq][si], j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
       si = sn;
     }
-    // an operand beyond the fp16 range leaves inf or NaN in the carried state (until a reset discards it): count it
-    count_nonfinite(C.S, lane, events_word(A.status));
+    if (MODE == SUMMARY) {
+      unusable = store_summary(C, *part_sum(A, head, part), map);
+    } else {
+      // an operand beyond the fp16 range leaves inf or NaN in the carried state (until a reset discards it): count it
+      count_nonfinite(C.S, lane, events_word(A.status));
+    }
   } else {
     const int p = pp;
     Raw raw;
+    unsigned* const events = MODE == SUMMARY ? nullptr : events_word(A.status);     // the launch after it counts
     // this lane's new_starts byte of the chunk loaded next: fetched a step ahead, behind the operands (measured: 1.6 %
     // faster here than in front of them, where the other sweeps have it)
     uint32_t ns_mine = 0u;
-    if (p < nch) {
-      load_raw(raw, A, b, h, (int64_t)p * CK, lane);
-      ns_mine = chunk_flag_prefetch(A.ns, A.T, b, (int64_t)p * CK, lane);
+    if (p < n) {
+      load_raw<MODE>(raw, A, b, h, (int64_t)(j0 + p) * CK, lane);
+      ns_mine = chunk_flag_prefetch(A.ns, A.T, b, (int64_t)(j0 + p) * CK, lane);
     }
-    for (int j = p; j < nch + (PARK ? RING : 0); j += NPROD) {
-      const int64_t c0 = (int64_t)j * CK;
+    for (int j = p; j < n + (PARK ? RING : 0); j += NPROD) {
+      const int64_t c0 = (int64_t)(j0 + j) * CK;
       const int si = j % RING;
       Slot* slot = &slots[si];
       if (PARK) {
@@ -698,46 +838,82 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_kernel(Wkv7Args
       }
       if (j >= RING) {
         if (!wait_consumed_lazy(sy, si, j - RING + 1, lane)) break;
-        if (PARK) flush_y(slot, A, b, h, j - RING, nch, lane);
+        if (PARK && (MODE != PART || j0 + j - RING >= j_out)) flush_y(slot, A, b, h, j0 + j - RING, nch, lane);
       }
-      if (PARK && j >= nch) continue;
-      const ChunkFlags F = chunk_flags_of(A.ns, ns_mine, A.flags, A.T, c0, L);
+      if (PARK && j >= n) continue;
+      const ChunkFlags F = chunk_flags_of(A.ns, ns_mine, A.flags, A.T, c0, MODE == SUMMARY ? 0 : L);
       mask_raw(raw, F.nvalid, lane);
-      produce(lane, raw, F, slot, snapslot, events_word(A.status));
-      if (j + NPROD < nch) {
-        load_raw(raw, A, b, h, c0 + (int64_t)NPROD * CK, lane);
+      if (MODE == SUMMARY && map) raw.v[0] = raw.v[1] = make_uint4(0, 0, 0, 0);
+      produce<MODE>(lane, raw, F, slot, snapslot, events);
+      if (j + NPROD < n) {
+        load_raw<MODE>(raw, A, b, h, c0 + (int64_t)NPROD * CK, lane);
         ns_mine = chunk_flag_prefetch(A.ns, A.T, b, c0 + (int64_t)NPROD * CK, lane);
       }
-      if ((A.flags & FLAG_DROP_PUBLISH) && j + 1 == nch) break;
+      if ((A.flags & FLAG_DROP_PUBLISH) && j + 1 == n) break;
       // the release orders this wave's LDS writes before the sequence number
       if (lane == 0) __hip_atomic_store(&sy->ready[si], j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
+    if (MODE == SUMMARY) raw.r[0] = raw.r[1] = make_uint4(0, 0, 0, 0);
     retire_loads(raw, ns_mine);
   }
   __syncthreads();
-  if (head_broken(sy, A.status)) {
-    poison_token_rows(A.out, 2, b, h, A.T, A.H);
-    poison_token_rows(A.sa, 2, b, h, A.T, A.H);
-    poison_state(A.new_s, A.st_f32, b, h, A.H);
+  const bool broken = head_broken(sy, A.status);
+  if (MODE == SUMMARY) {
+    if (is_cons && lane == 0) part_flags(A, head, part)[(map ? 4 : 0) + cq] = unusable | (broken ? 1 : 0);
+    if (is_cons && lane == 0 && !map && part == 0) part_flags(A, head, 0)[4 + cq] = 0;     // part 0 has no M
+  } else if (broken) {
+    const int64_t t0 = (int64_t)j_out * CK, rows = MODE == WHOLE || (int64_t)(j0 + n) * CK > A.T ? A.T - t0 : (int64_t)(j0 + n) * CK - t0;
+    poison_token_rows(A.out, 2, b, h, A.T, A.H, t0, rows);
+    poison_token_rows(A.sa, 2, b, h, A.T, A.H, t0, rows);
+    if (MODE == WHOLE || (L == 0 ? part == 0 : L - 1 >= t0 && L - 1 < t0 + rows)) poison_state(A.new_s, A.st_f32, b, h, A.H);
   }
 }
 
-hipError_t launch_wkv7_chunk_fwd(const Wkv7Args& A, hipStream_t stream) {
+// Parts a sequence is cut into, and the chunks of a part.  In units of a chunk's time: a launch costs its workgroups' rounds over
+// 256 CUs times the chunks of a part, the second launch and the fold cost PART_COST + 2 per part (8 us + 1.3 us).  No shape on
+// which it decides for parts was slower with them (B=5 T=1021 H=16: 49.9 -> 48.4 us, T=777 H=1 38.9 -> 30.7); below
+// about 600 tokens and above 85 heads the whole sequence is faster.
+constexpr int CUS = 256, MAX_PARTS = 32, PART_COST = 12;
+int wkv7_fwd_parts(int64_t heads, int64_t T, int* chunks) {
+  const int64_t nch = (T + CK - 1) / CK;
+  auto rounds = [&](int64_t groups) { return (groups + CUS - 1) / CUS; };
+  int64_t best = nch * rounds(heads), best_chunks = nch;
+  for (int64_t p = 2; p <= MAX_PARTS && p <= nch; ++p) {
+    const int64_t c = (nch + p - 1) / p, np = (nch + c - 1) / c;
+    if (np < 2) continue;
+    const int64_t cost = c * (rounds(heads * (2 * np - 3)) + rounds(heads * np)) + PART_COST + 2 * np;
+    if (cost < best) { best = cost; best_chunks = c; }
+  }
+  *chunks = (int)best_chunks;
+  return (int)((nch + best_chunks - 1) / best_chunks);
+}
+size_t wkv7_fwd_parts_bytes(int64_t heads, int64_t T) {
+  int c;
+  const int np = wkv7_fwd_parts(heads, T, &c);
+  return np < 2 ? 0 : (size_t)heads * (np - 1) * (sizeof(PartSum) + 8 * sizeof(int));
+}
+
+namespace {
+template <bool PARK, int MODE>
+hipError_t launch_mode(const Wkv7Args& A, int64_t groups, hipStream_t stream) {
   static_assert(RING <= MAX_RING, "the hand-shake words cover MAX_RING slots");
   const size_t smem = RING * sizeof(Slot) + sizeof(SnapSlot) + sizeof(Sync);
-  const dim3 grid((unsigned)(A.B * A.H)), block(64 * (NCONS + NPROD));
-  if (A.sa != nullptr) {
-    static LdsAttrOnce once;
-    const hipError_t attr = allow_dynamic_lds(once, reinterpret_cast<const void*>(wkv7_fwd_kernel<true>), smem);
-    if (attr != hipSuccess) return attr;
-    hipLaunchKernelGGL(wkv7_fwd_kernel<true>, grid, block, smem, stream, A);
-  } else {
-    static LdsAttrOnce once;
-    const hipError_t attr = allow_dynamic_lds(once, reinterpret_cast<const void*>(wkv7_fwd_kernel<false>), smem);
-    if (attr != hipSuccess) return attr;
-    hipLaunchKernelGGL(wkv7_fwd_kernel<false>, grid, block, smem, stream, A);
-  }
+  static LdsAttrOnce once;
+  const hipError_t attr = allow_dynamic_lds(once, reinterpret_cast<const void*>(wkv7_fwd_kernel<PARK, MODE>), smem);
+  if (attr != hipSuccess) return attr;
+  hipLaunchKernelGGL((wkv7_fwd_kernel<PARK, MODE>), dim3((unsigned)groups), dim3(64 * (NCONS + NPROD)), smem, stream, A);
   return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_wkv7_chunk_fwd(const Wkv7Args& A0, hipStream_t stream) {
+  Wkv7Args A = A0;
+  const int64_t heads = A.B * A.H;
+  A.n_part = A.parts != nullptr ? wkv7_fwd_parts(heads, A.T, &A.part_chunks) : 1;
+  if (A.n_part < 2) return A.sa != nullptr ? launch_mode<true, WHOLE>(A, heads, stream) : launch_mode<false, WHOLE>(A, heads, stream);
+  const hipError_t e = launch_mode<false, SUMMARY>(A, heads * (2 * A.n_part - 3), stream);
+  if (e != hipSuccess) return e;
+  return A.sa != nullptr ? launch_mode<true, PART>(A, heads * A.n_part, stream) : launch_mode<false, PART>(A, heads * A.n_part, stream);
 }
 
 }  // namespace hiprwkv

@@ -34,7 +34,12 @@ struct Wkv7Args {
   // Elements between the states of consecutive sequences in `s` / `new_s`; 0 = dense (H*64*64).  Honoured by the
   // small-T kernel only (states read and written inside a packed model state).
   int64_t s_bstride, new_s_bstride;
+  // forward, bf16 I/O: workspace for a sequence in parts (wkv7_fwd_parts), null: whole; the launcher sets the other two
+  void* parts;
+  int n_part, part_chunks;
 };
+int wkv7_fwd_parts(int64_t heads, int64_t T, int* chunks);
+size_t wkv7_fwd_parts_bytes(int64_t heads, int64_t T);
 
 // Wkv6Args::flags bit: w is (H,64), shared by every token and sequence (HIPRWKV_W_PER_HEAD)
 constexpr unsigned FLAG_W_PER_HEAD = 0x10u;

@@ -138,9 +138,11 @@ def wkv7_fwd(r, w, k, v, a, b, s, length=None, new_starts=None, compat=True, wan
     new_s = torch.empty_like(s)
     # the residual for the backward pass: fp32 beside fp32 I/O, fp16 beside bf16 I/O
     sa = _empty_phased((B, T, H, N), _SA_DT[io], r.device, _phase(r) + 2) if want_sa else None
-    rc = lib.hiprwkv_wkv7_fwd(_stream(), _DT[io], _DT[s.dtype], B, T, H, N, _p(w), _p(r), _p(k), _p(v), _p(a), _p(b),
-                              _p(s), _p(length), _p(new_starts), _p(y), _p(sa), _p(new_s),
-                              _flags(compat, force_seq, small_t, debug_flags))
+    nbytes = 0 if force_seq else lib.hiprwkv_wkv7_fwd_workspace_bytes(_DT[io], B, T, H, N)
+    ws = _workspace(nbytes, r.device) if nbytes else None
+    rc = lib.hiprwkv_wkv7_fwd_parts(_stream(), _DT[io], _DT[s.dtype], B, T, H, N, _p(w), _p(r), _p(k), _p(v), _p(a), _p(b),
+                                    _p(s), _p(length), _p(new_starts), _p(y), _p(sa), _p(new_s), _p(ws), nbytes,
+                                    _flags(compat, force_seq, small_t, debug_flags))
     _lib.check(rc, "hiprwkv_wkv7_fwd")
     return new_s, y, sa
 

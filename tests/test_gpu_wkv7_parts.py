@@ -1,0 +1,99 @@
+"""The WKV7 bf16 forward with its sequences cut into parts (few sequences and heads) against the oracle and against the same
+kernel over the whole sequence, to which it falls back without a workspace.
+
+The parts add one product per part in fp32 to the whole sequence's arithmetic; the operand rounding (fp16, 2^-11) is the same and
+sets the error of both.  The bounds against the oracle are those of the whole sequence (test_gpu_wkv7_chunked); where the
+state is carried over many parts (slow decay) the rms errors of the two are compared: rounding errors of the same size in another
+order, so a quarter more is allowed."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import wkv7 as o7
+from tests.inputs import bf16_round, wkv7_inputs
+from tests.test_gpu_wkv7_chunked import check, run
+
+pytestmark = pytest.mark.gpu
+
+
+def lib():
+    from jaxrwkv_amd import _lib
+    return _lib.load()
+
+
+def split(B, T, H):
+    return lib().hiprwkv_wkv7_fwd_workspace_bytes(1, B, T, H, 64) // (32768 + 32) // (B * H) + 1
+
+
+def whole(monkeypatch, *a, **k):
+    with monkeypatch.context() as m:
+        m.setattr(lib(), "hiprwkv_wkv7_fwd_workspace_bytes", lambda *_: 0)
+        return run(*a, **k)
+
+
+@pytest.mark.parametrize("B,T,H,seed,p", [(1, 1000, 1, 0, 0.0), (1, 1009, 2, 1, 0.01), (2, 1025, 3, 2, 0.002), (3, 2047, 12, 3, 0.001)])
+@pytest.mark.parametrize("compat", [True, False])
+def test_against_the_oracle(B, T, H, seed, p, compat):
+    P = split(B, T, H)
+    assert P >= 2
+    x = wkv7_inputs(B, T, H, 64, seed=seed, bf16=True, p_reset=p, min_len_frac=0.0)
+    chunks = -(-(-(-T // 16)) // P)
+    x["length"][0] = 16 * chunks                       # the last token of the first part
+    x["new_starts"][-1, 16 * chunks] = True            # a reset at the first token of the second
+    for want_sa in (False, True):
+        check(x, compat, *run(x, compat, want_sa=want_sa))
+
+
+@pytest.mark.parametrize("L", [0, 1, 15, 500, 1017])
+def test_lengths(L):
+    x = wkv7_inputs(1, 1017, 2, 64, seed=L, bf16=True, p_reset=0.003)
+    x["length"][:] = L
+    for compat in (True, False):
+        check(x, compat, *run(x, compat))
+
+
+def rms(a):
+    return float(np.sqrt(np.mean(np.square(a))))
+
+
+@pytest.mark.parametrize("decay", [-2.5, -5.0, -8.0])
+@pytest.mark.parametrize("B,T,H", [(1, 2048, 2), (2, 1777, 12)])
+def test_state_carried_over_the_parts(B, T, H, decay, monkeypatch):
+    x = wkv7_inputs(B, T, H, 64, seed=5, bf16=True, resets=False)
+    x["w"] = bf16_round(x["w"] + 0.5 + decay).astype(np.float64)
+    ref = o7.wkv7_base(x["r"], x["w"], x["k"], x["v"], x["a"], x["b"], x["s"], x["length"], x["new_starts"], compat=True, return_sa=True)
+    assert split(B, T, H) >= 2
+    got, base = run(x, True), whole(monkeypatch, x, True)
+    for g, w, e in zip(got, base, ref):
+        assert rms(g - e) <= 1.25 * rms(w - e) + 1e-6 * rms(e)
+
+
+def test_summaries_that_amplify_are_not_used(monkeypatch):
+    """b = +0.02 |a|^2-direction for the first 300 tokens, no decay to speak of: the state map grows by e^6 along one vector.  The
+    parts after it run the chunks before them themselves and give the whole sequence's bits from there on."""
+    x = wkv7_inputs(1, 1200, 2, 64, seed=6, bf16=True, resets=False, lengths=False)
+    x["w"][:] = -9.0
+    x["a"][:, :300] = x["a"][:, :1]
+    x["b"][:, :300] = bf16_round(0.02 * x["a"][:, :300])
+    assert split(1, 1200, 2) >= 4
+    got, base = run(x, True), whole(monkeypatch, x, True)
+    ref = o7.wkv7_base(x["r"], x["w"], x["k"], x["v"], x["a"], x["b"], x["s"], x["length"], x["new_starts"], compat=True, return_sa=True)
+    for g, w, e in zip(got, base, ref):
+        assert np.isfinite(g).all()
+        assert rms(g - e) <= 1.25 * rms(w - e) + 1e-6 * rms(e)
+    big = wkv7_inputs(1, 1200, 1, 64, seed=7, bf16=True, resets=False, lengths=False)
+    big["v"][:, 5] = 3e38                               # beyond the fp16 operands: the whole sequence turns non-finite, and so do the parts
+    assert np.isnan(run(big, True)[0]).any() and np.isnan(whole(monkeypatch, big, True)[0]).any()
+
+
+def test_a_broken_handshake_poisons_every_part(monkeypatch):
+    from jaxrwkv_amd import _lib, ops
+    monkeypatch.setenv("HIPRWKV_ENABLE_DEBUG_FLAGS", "1")
+    x = wkv7_inputs(1, 1000, 1, 64, seed=8, bf16=True)
+    from tests.gpu_util import dev
+    t = [dev(x[n], torch.bfloat16) for n in ("r", "w", "k", "v", "a", "b")]
+    try:
+        new_s, y, sa = ops.wkv7_fwd(*t, dev(x["s"]), want_sa=True, debug_flags=0x100)
+    except _lib.HipRwkvError:
+        pytest.skip("the debug flag is read once per process and another test came first without it")
+    assert torch.isnan(new_s).all() and torch.isnan(y).all() and torch.isnan(sa).all()
