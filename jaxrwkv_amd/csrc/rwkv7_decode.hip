@@ -1,13 +1,13 @@
 // An RWKV-7 decode step (at most 8 tokens per sequence, at most 256 tokens in all, bf16) layer by layer from native code:
 // eight launches per layer instead of the ~30 operations of the general path, whose host side alone takes 5 ms for 12 layers.
 //     1  residual addition, norm, shift and six interpolations               (rwkv7_block.hip)
-//     2  r, k, v and the first low-rank factors, tanh / sigmoid applied       skinny_gemm, seven products in one grid
-//     3  the second low-rank factors                                          skinny_gemm, four products
+//     2  r, k, v and the first low-rank factors, tanh / sigmoid applied       rwkv7_gemm.hip, seven products in one grid
+//     3  the second low-rank factors                                          rwkv7_gemm.hip, four products
 //     4  gates, WKV step on the packed state, group norm, bonus, gate         decode_core_kernel
-//     5  output projection                                                    skinny_gemm
+//     5  output projection                                                    rwkv7_gemm.hip
 //     6  residual addition, norm, shift and interpolation                     (rwkv7_block.hip)
-//     7  key projection with relu(.)^2                                        skinny_gemm
-//     8  value projection                                                     skinny_gemm
+//     7  key projection with relu(.)^2                                        rwkv7_gemm.hip
+//     8  value projection                                                     rwkv7_gemm.hip
 // Measured (eager, host included): 12 layers of 768 channels, one user 5.4 ms -> 0.56 ms a step; 24 layers of 2048 channels,
 // 256 users 10.9 -> 3.6 ms (7.5 with the weight-streaming product alone: 51 us a launch at 256 rows, 18 tiled).
 // References: /root/reference/src/jaxrwkv/rwkv7.py:190-198, :223-267, :269-291.  Products accumulate in fp32 and are rounded

@@ -105,7 +105,7 @@ __global__ __launch_bounds__(64 * GEMM_WAVES) void skinny_gemm_kernel(GemmArgs A
   }
 }
 
-// 64 x 64 tiles, 64 of k per step through two LDS buffers: a thread carries two 16-byte pieces of either operand, requested two
+// 64 x 64 tiles through registers, any K, 64 of it per step through two LDS buffers: a thread carries two 16-byte pieces of either operand, requested two
 // steps ahead, and four workgroups share a CU, so loads, LDS writes and matrix instructions of different workgroups
 // overlap.  An operand that lies k-major (km, kn) goes to LDS as it lies and is read with the transposing load.  Workgroups go
 // to the eight XCDs round-robin; the tiles that share a piece of the longer operand run on one XCD, whose L2 reads it once.
@@ -270,26 +270,162 @@ __device__ __forceinline__ void tile_gemm_body(const GemmArgs& A, const GemmJob&
 
 // job and tile of a workgroup: along the longer side of the tile grid eight tiles at a time, one per XCD; all tiles across from
 // each on the same XCD
-__device__ __forceinline__ bool tile_of(const GemmArgs& A, int& ji, int& n0, int& m0) {
+__device__ __forceinline__ bool tile_of(const GemmArgs& A, int tm, int& ji, int& n0, int& m0) {
   ji = 0;
   for (int i = 1; i < A.n_jobs; ++i) ji = (int)blockIdx.x >= A.job[i].tile0 ? i : ji;
   const int M = A.job[ji].M, N = A.job[ji].N;
-  const int mt = (M + TG - 1) / TG, nt = (N + TG - 1) / TG, local = (int)blockIdx.x - A.job[ji].tile0;
+  const int mt = (M + tm - 1) / tm, nt = (N + TG - 1) / TG, local = (int)blockIdx.x - A.job[ji].tile0;
   const int across = mt < nt ? mt : nt;
   const int p = local / (8 * across) * 8 + local % 8, q = local % (8 * across) / 8;
   n0 = (mt < nt ? p : q) * TG;
-  m0 = (mt < nt ? q : p) * TG;
+  m0 = (mt < nt ? q : p) * tm;
   return n0 < N && m0 < M;
 }
-int tiles_of(const GemmJob& J) {
-  const int mt = (J.M + TG - 1) / TG, nt = (J.N + TG - 1) / TG;
+int tiles_of(const GemmJob& J, int tm) {
+  const int mt = (J.M + tm - 1) / tm, nt = (J.N + TG - 1) / TG;
   return ((mt < nt ? nt : mt) + 7) / 8 * 8 * (mt < nt ? mt : nt);
+}
+
+// The same tiles with the operands requested straight into LDS, BUFS - 1 steps ahead: no registers are held by what is in
+// flight.  K is a multiple of the step.  A wave's request fills eight rows of 128 bytes as they lie, so rows cannot be padded:
+// 16-byte piece p of row q lies at p ^ swizzle(q) instead (no bank conflicts counted).  Weights that no cache holds, against the
+// tiles through registers: 64 rows of 2048 channels into 8192 columns 19.0 -> 15.3 us, K = 8192 into 2048 unsplit 57.9 -> 37.8;
+// 128 rows 19.3 -> 15.4; r, k, v and the low-rank inputs at 128 rows 20.5 -> 16.6; 256 rows into 8192 columns 23.5 -> 22.8 with
+// 64-row tiles, 19.9 with 128.  Bound by the wait for the weights (56 % of the waves' time); five and seven steps in flight took as
+// long, and so did a first step that differs from tile to tile.
+constexpr int stream_step(int tm) { return (tm + TG) * TG; }       // bf16 values of a step in LDS: TM rows of x, TG of w
+typedef __attribute__((address_space(3))) uint16_t* lds_u16_ptr;
+
+// 16 bytes per lane to 1 KiB of LDS at `lds` (a wave-uniform address).  In assembly because the compiler waits for every request
+// under way before any LDS read; it has no result registers, the waits are the reader's.
+__device__ __forceinline__ void request_lds(u32x4_t rs, int voff, int soff, uint32_t lds) {
+  asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(rs), "s"(soff), "{m0}"(lds) : "memory");
+}
+
+// ROWS (64 or 128) rows of m or n by 64 of k; with TR the operand lies k-major and so does its piece of LDS
+template <bool TR, int ROWS>
+struct StreamOperand {
+  static constexpr int PIECES = ROWS / 32;                           // requests of a wave per step
+  static constexpr int PER_ROW = TR ? ROWS / 8 : TG / 8;             // 16-byte pieces of an LDS row
+  static constexpr int LINES = 64 / PER_ROW;                         // LDS rows that a request fills
+  u32x4_t rs;
+  int voff[PIECES], stride, last, at;
+  static __device__ __forceinline__ int swizzle(int q) {
+    return TR ? 2 * ((q ^ (q >> 3)) & 3) : (q & 3) | ((q >> 1) & 4);
+  }
+  __device__ __forceinline__ StreamOperand(const void* base, int R, int K, int r0, int wave, int lane) {
+    last = K / TG - 1;
+    stride = TR ? TG * R * 2 : TG * 2;
+    const uint64_t first = reinterpret_cast<uint64_t>(static_cast<const bf16_t*>(base) + (TR ? (int64_t)r0 : (int64_t)r0 * K));
+    rs = u32x4_t{(uint32_t)first, (uint32_t)(first >> 32) & 0xffffu, 0x7fffffffu, 0x00020000u};      // as make_rsrc
+    at = wave * PIECES * 1024;
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+      const int q = LINES * (PIECES * wave + i) + lane / PER_ROW, c = 8 * ((lane % PER_ROW) ^ swizzle(q));
+      voff[i] = TR ? (q * R + (r0 + c < R ? c : R - 8 - r0)) * 2 : ((r0 + q < R ? q : R - 1 - r0) * K + c) * 2;
+    }
+  }
+  __device__ __forceinline__ void request(int s, uint16_t* lds) const {
+    const int soff = (s < last ? s : last) * stride;
+    const uint32_t to = (uint32_t)(uintptr_t)(lds_u16_ptr)(lds) + at;
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) request_lds(rs, voff[i], soff, to + 1024 * i);
+  }
+  // eight of k (32 kh + 8g ..) of row n; with TR the lane's own row comes out of the transposing read, n is that of its request
+  static __device__ __forceinline__ u32x4_t frag(const uint16_t* lds, int n, int kh, int r, int g) {
+    if (TR) {
+      const int k = 32 * kh + 8 * g + (r >> 2);
+      const uint2 lo = lds_tr4(lds + k * ROWS + 8 * ((n >> 3) ^ swizzle(k)) + (n & 7));
+      const uint2 hi = lds_tr4(lds + (k + 4) * ROWS + 8 * ((n >> 3) ^ swizzle(k + 4)) + (n & 7));
+      return u32x4_t{lo.x, lo.y, hi.x, hi.y};
+    }
+    return *reinterpret_cast<const u32x4_t*>(lds + n * TG + 8 * ((4 * kh + g) ^ swizzle(n)));
+  }
+};
+
+// TM x 64 tiles, four waves of TM/2 x 32
+template <int TM, int BUFS, bool KM, bool KN>
+__device__ __forceinline__ void stream_gemm_body(const GemmArgs& A, const GemmJob& J, int n0, int m0, uint16_t* lds) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  constexpr int MT = TM / 32, STEP = stream_step(TM), IN_STEP = TM / 32 + TG / 32;
+  const int all = J.K / TG;
+  const int s0 = all * (int)blockIdx.y / (int)gridDim.y, s1 = all * ((int)blockIdx.y + 1) / (int)gridDim.y;
+  typedef StreamOperand<KM, TM> OpX;
+  typedef StreamOperand<KN, TG> OpW;
+  const OpX X(J.x, J.M, J.K, m0, wave, lane);
+  const OpW W(J.w, J.N, J.K, n0, wave, lane);
+  f32x4_t acc[2][MT];
+#pragma unroll
+  for (int i = 0; i < 2 * MT; ++i) acc[i / MT][i % MT] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int wn = 32 * (wave & 1), wm = TM / 2 * (wave >> 1);
+  auto request = [&](int s, int buf) {
+    X.request(s, lds + buf * STEP);
+    W.request(s, lds + buf * STEP + TM * TG);
+  };
+#pragma unroll
+  for (int j = 0; j < BUFS - 1; ++j) request(s0 + j, j);
+  auto step = [&](int s, int buf) {
+    // this wave's part of step s has arrived; after the barrier all parts, and nobody reads the buffer of step s - 1 any more
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(IN_STEP * (BUFS - 2)) : "memory");
+    request(s + BUFS - 1, (buf + BUFS - 1) % BUFS);
+    const uint16_t* const xs = lds + buf * STEP;
+    const uint16_t* const ws = xs + TM * TG;
+#pragma unroll
+    for (int kh = 0; kh < 2; ++kh) {
+      u32x4_t wf[2], xf[MT];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) wf[t] = OpW::frag(ws, wn + 16 * t + (KN ? 4 * (r & 3) : r), kh, r, g);
+#pragma unroll
+      for (int u = 0; u < MT; ++u) xf[u] = OpX::frag(xs, wm + 16 * u + (KM ? 4 * (r & 3) : r), kh, r, g);
+#pragma unroll
+      for (int u = 0; u < MT; ++u)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) acc[t][u] = mfma(wf[t], xf[u], acc[t][u]);
+    }
+  };
+  int s = s0;
+  for (; s + BUFS <= s1; s += BUFS)
+#pragma unroll
+    for (int j = 0; j < BUFS; ++j) step(s + j, j);
+#pragma unroll
+  for (int j = 0; j < BUFS - 1; ++j)
+    if (s + j < s1) step(s + j, j);
+  // the requests beyond the last step write to LDS as well: none may be under way when the workgroup gives its LDS back
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int u = 0; u < MT; ++u) finish(A, J, n0 + wn + 16 * t + 4 * g, m0 + wm + 16 * u + r, acc[t][u]);
+}
+
+template <int TM, int BUFS>
+__global__ __launch_bounds__(256) void stream_gemm_kernel(GemmArgs A) {
+  extern __shared__ __align__(1024) uint16_t stream_lds[];
+  int ji, n0, m0;
+  if (!tile_of(A, TM, ji, n0, m0)) return;
+  const GemmJob J = A.job[ji];
+  switch ((J.km ? 2 : 0) + (J.kn ? 1 : 0)) {
+    case 0: stream_gemm_body<TM, BUFS, false, false>(A, J, n0, m0, stream_lds); break;
+    case 1: stream_gemm_body<TM, BUFS, false, true>(A, J, n0, m0, stream_lds); break;
+    case 2: stream_gemm_body<TM, BUFS, true, false>(A, J, n0, m0, stream_lds); break;
+    default: stream_gemm_body<TM, BUFS, true, true>(A, J, n0, m0, stream_lds); break;
+  }
+}
+template <int TM, int BUFS>
+hipError_t launch_stream(const GemmArgs& A, int tiles, int split, hipStream_t stream) {
+  static LdsAttrOnce attr;
+  constexpr size_t bytes = (size_t)BUFS * stream_step(TM) * 2;
+  const auto kernel = stream_gemm_kernel<TM, BUFS>;
+  hipError_t e = allow_dynamic_lds(attr, reinterpret_cast<const void*>(kernel), bytes);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kernel, dim3(tiles, split), dim3(256), bytes, stream, A);
+  return hipGetLastError();
 }
 
 __global__ __launch_bounds__(256) void tile_gemm_kernel(GemmArgs A) {
   __shared__ __align__(16) TileLds lds;
   int ji, n0, m0;
-  if (!tile_of(A, ji, n0, m0)) return;
+  if (!tile_of(A, TG, ji, n0, m0)) return;
   const GemmJob J = A.job[ji];
   switch ((J.km ? 4 : 0) + (J.kn ? 2 : 0) + (J.K % TG == 0 ? 1 : 0)) {
     case 0: tile_gemm_body<false, false, false>(A, J, n0, m0, lds); break;
@@ -317,20 +453,36 @@ int gemm_split(int M, int64_t K, int64_t N) {
 // Up to 32 rows the streaming kernel (K a multiple of 32, N of 16, no aux): its operand loads touch a cache line per lane,
 // 64 cycles a KiB, which a stream of weights can afford but repeated reads of x cannot (8192 columns of 2048: 14 us at 32
 // rows, 16 at 33, 21 at 64; tiled 15 us up to 128 rows, 22 at 256).
+// From 33 rows the tiles: through registers only where some K of the launch is no multiple of a step (the second low-rank factors),
+// else straight to LDS, which was never slower (48 to 4084 rows, 768 to 2048 channels).  128-row tiles, which read the weights
+// half as often, where they are one round that fills the GPU: below that 64-row tiles use more CUs (256 rows of 1024 channels), above
+// it the last round is nearly empty (4084 rows into the low-rank sizes: 288 tiles 37 us, 576 small ones 34, through registers 36).
+constexpr int CUS = 256, WIDE_TILES = 192;
 hipError_t launch_gemm(GemmArgs A, int split, hipStream_t stream) {
-  bool skinny = A.part == nullptr;
+  bool skinny = A.part == nullptr, stream_k = true;
   int M = 0, tiles = 0;
   for (int i = 0; i < A.n_jobs; ++i) {
     const GemmJob& J = A.job[i];
     M = J.M > M ? J.M : M;
+    stream_k = stream_k && J.K % TG == 0;
     skinny = skinny && J.M < GEMM_TILE_ROWS && !J.km && J.aux == nullptr && J.K % 32 == 0 && J.N % 16 == 0;
   }
-  for (int i = 0; i < A.n_jobs; ++i) {
-    GemmJob& J = A.job[i];
-    J.tile0 = tiles;
-    tiles += skinny ? J.N / 16 : tiles_of(J);
-  }
+  auto place = [&](int tm) {
+    tiles = 0;
+    for (int i = 0; i < A.n_jobs; ++i) {
+      GemmJob& J = A.job[i];
+      J.tile0 = tiles;
+      tiles += skinny ? J.N / 16 : tiles_of(J, tm);
+    }
+  };
   const dim3 block(64 * GEMM_WAVES);
+  if (!skinny && stream_k) {
+    place(2 * TG);
+    if (M > TG && tiles * split >= WIDE_TILES && tiles * split <= CUS) return launch_stream<2 * TG, 4>(A, tiles, split, stream);
+    place(TG);
+    return launch_stream<TG, 4>(A, tiles, split, stream);
+  }
+  place(TG);
   if (!skinny) hipLaunchKernelGGL(tile_gemm_kernel, dim3(tiles, split), dim3(256), 0, stream, A);
   else if (M <= 16) hipLaunchKernelGGL(skinny_gemm_kernel<1>, dim3(tiles), block, 0, stream, A);
   else hipLaunchKernelGGL(skinny_gemm_kernel<2>, dim3(tiles), block, 0, stream, A);

@@ -1,0 +1,37 @@
+"""Products whose operands are requested straight into LDS (K a multiple of 64) against the product in fp64.
+
+bf16 inputs, fp32 sums: a sum of K products is off by at most a few 2^-24 of sum |x w| and is rounded once to bf16 (2^-9 of the
+value), hence |d| <= 2^-8 |value| + 2^-18 sqrt(K) for inputs of size one."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# K from one step to more than two turns of the buffers, M and N around the tile's edge and at one row past it
+@pytest.mark.parametrize("km,kn", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(40, 8, 64), (64, 64, 128), (72, 72, 192), (256, 200, 256), (136, 64, 320), (64, 1032, 576), (520, 136, 2048), (136, 6144, 320),
+                                   (264, 8200, 192)])
+def test_product(M, N, K, km, kn):
+    from jaxrwkv_amd import blocks7
+    g = torch.Generator("cuda").manual_seed(M + N + K)
+    x = torch.randn((K, M) if km else (M, K), device="cuda", generator=g).bfloat16()
+    w = torch.randn((K, N) if kn else (N, K), device="cuda", generator=g).bfloat16()
+    guard = torch.full((M + 2, N), 7.0, device="cuda", dtype=torch.bfloat16)
+    blocks7._gemm([(guard[1:-1], x, w, km, kn, 0, None)])
+    want = (x.double().T if km else x.double()) @ (w.double() if kn else w.double().T)
+    d = (guard[1:-1].double() - want).abs()
+    assert (d <= want.abs() * 2.0 ** -8 + 2.0 ** -18 * K ** 0.5).all()
+    assert (guard[0] == 7).all() and (guard[-1] == 7).all()
+
+
+def test_several_products_in_one_launch():
+    from jaxrwkv_amd import blocks7
+    g = torch.Generator("cuda").manual_seed(5)
+    x = torch.randn((300, 256), device="cuda", generator=g).bfloat16()
+    ws = [torch.randn((n, 256), device="cuda", generator=g).bfloat16() for n in (8, 256, 96)]
+    outs = [torch.empty((300, w.shape[0]), device="cuda", dtype=torch.bfloat16) for w in ws]
+    blocks7._gemm([(o, x, w, 0, 0, 0, None) for o, w in zip(outs, ws)])
+    for o, w in zip(outs, ws):
+        want = x.double() @ w.double().T
+        assert ((o.double() - want).abs() <= want.abs() * 2.0 ** -8 + 2.0 ** -14).all()
