@@ -178,6 +178,14 @@ int hiprwkv_wkv6_fwd(hiprwkv_stream stream, int io_dtype, int state_dtype,
                      const void* u, const void* s,
                      const uint32_t* length, const uint8_t* new_starts,
                      void* out, void* new_s, unsigned flags);
+/* The same with `workspace`, as hiprwkv_wkv7_fwd_parts. */
+size_t hiprwkv_wkv6_fwd_workspace_bytes(int io_dtype, int64_t B, int64_t T, int64_t H, int64_t N);
+int hiprwkv_wkv6_fwd_parts(hiprwkv_stream stream, int io_dtype, int state_dtype,
+                     int64_t B, int64_t T, int64_t H, int64_t N,
+                     const void* r, const void* k, const void* v, const void* w,
+                     const void* u, const void* s,
+                     const uint32_t* length, const uint8_t* new_starts,
+                     void* out, void* new_s, void* workspace, size_t workspace_bytes, unsigned flags);
 
 /* hiprwkv_wkv6_fwd for a decode step (T <= HIPRWKV_SMALL_T) on a state inside the reference's packed model state
  * (rwkv6.py:148-153 default_state: (L, 2+N, C) per sequence; :221-224 the slice state[1:] of the time-mixing part,

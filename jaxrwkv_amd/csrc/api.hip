@@ -290,6 +290,19 @@ int hiprwkv_wkv7_bwd(hiprwkv_stream stream, int io_dtype, int state_dtype, int64
 int hiprwkv_wkv6_fwd(hiprwkv_stream stream, int io_dtype, int state_dtype, int64_t B, int64_t T, int64_t H, int64_t N,
                      const void* r, const void* k, const void* v, const void* w, const void* u, const void* s,
                      const uint32_t* length, const uint8_t* new_starts, void* out, void* new_s, unsigned flags) {
+  return hiprwkv_wkv6_fwd_parts(stream, io_dtype, state_dtype, B, T, H, N, r, k, v, w, u, s, length, new_starts, out, new_s, nullptr, 0,
+                                flags);
+}
+
+size_t hiprwkv_wkv6_fwd_workspace_bytes(int io_dtype, int64_t B, int64_t T, int64_t H, int64_t N) {
+  if (io_dtype != HIPRWKV_BF16 || N != 64 || B <= 0 || T <= HIPRWKV_SMALL_T || H <= 0 || B * H > 0x7fffffffLL) return 0;
+  return wkv6_fwd_parts_bytes(B * H, T);
+}
+
+int hiprwkv_wkv6_fwd_parts(hiprwkv_stream stream, int io_dtype, int state_dtype, int64_t B, int64_t T, int64_t H, int64_t N,
+                           const void* r, const void* k, const void* v, const void* w, const void* u, const void* s,
+                           const uint32_t* length, const uint8_t* new_starts, void* out, void* new_s, void* workspace,
+                           size_t workspace_bytes, unsigned flags) {
   int rc = check_matrix_shape("wkv6_fwd", io_dtype, state_dtype, B, T, H, N);
   if (rc) return rc;
   if ((rc = check_flags("wkv6_fwd", flags)) != HIPRWKV_OK) return rc;
@@ -298,6 +311,10 @@ int hiprwkv_wkv6_fwd(hiprwkv_stream stream, int io_dtype, int state_dtype, int64
     if (p == nullptr) return fail(HIPRWKV_EINVAL, "wkv6_fwd: null tensor pointer");
     if (!aligned16(p)) return fail(HIPRWKV_EINVAL, "wkv6_fwd: tensor pointers must be 16-byte aligned");
   }
+  if (workspace && !aligned16(workspace)) return fail(HIPRWKV_EINVAL, "wkv6_fwd: workspace must be 16-byte aligned");
+  const size_t need = workspace != nullptr ? hiprwkv_wkv6_fwd_workspace_bytes(io_dtype, B, T, H, N) : 0;
+  if (workspace_bytes < need)
+    return fail(HIPRWKV_ENOSPACE, "wkv6_fwd: workspace has %zu bytes, %zu needed", workspace_bytes, need);
   Wkv6Args A;
   memset(&A, 0, sizeof(A));
   A.B = B; A.T = T; A.H = H;
@@ -306,6 +323,7 @@ int hiprwkv_wkv6_fwd(hiprwkv_stream stream, int io_dtype, int state_dtype, int64
   A.out = out; A.new_s = new_s;
   A.io_f32 = io_dtype == HIPRWKV_F32; A.st_f32 = state_dtype == HIPRWKV_F32;
   A.flags = flags;
+  A.parts = need != 0 ? workspace : nullptr;
   A.status = status_word();
   // chunked matrix-core kernels (fp16 operands for bf16 I/O, fp32 operands for fp32 I/O) unless HIPRWKV_FORCE_SEQ
   const bool chunked = !(flags & HIPRWKV_FORCE_SEQ);

@@ -64,7 +64,12 @@ struct Wkv6Args {
   // Elements between the states of consecutive sequences in `s` / `new_s`; 0 = dense (H*64*64).  Honoured by the
   // small-T kernel only (states read and written inside a packed model state).
   int64_t s_bstride, new_s_bstride;
+  // forward, bf16 I/O: workspace for a sequence in parts (wkv6_fwd_parts), null: whole; the launcher sets the other two
+  void* parts;
+  int n_part, part_chunks;
 };
+int wkv6_fwd_parts(int64_t heads, int64_t T, int* chunks);
+size_t wkv6_fwd_parts_bytes(int64_t heads, int64_t T);
 
 // Wkv4Args::flags bit: the workspace already holds the checkpoints (HIPRWKV_CKPT_READY)
 constexpr unsigned FLAG_CKPT_READY = 0x20u;

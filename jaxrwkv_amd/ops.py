@@ -249,9 +249,11 @@ def wkv6_fwd(r, k, v, w, u, s, length=None, new_starts=None, compat=True, force_
     length, new_starts = _length_ns(length, new_starts, B, T, r.device)
     y = _empty_like_phased(r, 1)
     new_s = torch.empty_like(s)
-    rc = lib.hiprwkv_wkv6_fwd(_stream(), _DT[io], _DT[s.dtype], B, T, H, N, _p(r), _p(k), _p(v), _p(w), _p(u), _p(s),
-                              _p(length), _p(new_starts), _p(y), _p(new_s),
-                              _flags(compat, force_seq, small_t, debug_flags) | (_lib.W_PER_HEAD if per_head else 0))
+    nbytes = 0 if force_seq else lib.hiprwkv_wkv6_fwd_workspace_bytes(_DT[io], B, T, H, N)
+    ws = _workspace(nbytes, r.device) if nbytes else None
+    rc = lib.hiprwkv_wkv6_fwd_parts(_stream(), _DT[io], _DT[s.dtype], B, T, H, N, _p(r), _p(k), _p(v), _p(w), _p(u), _p(s),
+                                    _p(length), _p(new_starts), _p(y), _p(new_s), _p(ws), nbytes,
+                                    _flags(compat, force_seq, small_t, debug_flags) | (_lib.W_PER_HEAD if per_head else 0))
     _lib.check(rc, "hiprwkv_wkv6_fwd")
     return new_s, y
 
