@@ -41,6 +41,7 @@ def _gemm(jobs):
     kn, (K, N)."""
     arr = (_lib.GemmJob * len(jobs))()
     for j, (out, x, w, km, kn, act, aux) in zip(arr, jobs):
+        ops._one_dtype(torch.bfloat16, out, x, w, aux)
         j.out, j.x, j.w, j.aux = out.data_ptr(), x.data_ptr(), w.data_ptr(), None if aux is None else aux.data_ptr()
         j.M, j.N = out.shape
         j.K = x.shape[0] if km else x.shape[1]
@@ -299,11 +300,13 @@ class _Blocks(torch.autograd.Function):
         g_vfirst = None
         layers = list(zip(*(t.unbind(0) for t in params)))
         glayers = list(zip(*(t.unbind(0) for t in grads)))
-        for i in reversed(range(L)):
-            dx, g_vfirst = _layer_bwd(i, dict(zip(NAMES, layers[i])), dict(zip(NAMES, glayers[i])), saved[i], ns,
-                                      length, g_x, g_dx, None if g_state is None else g_state[:, i],
-                                      None if g_in is None else g_in[:, i], g_vfirst, v_first)
-            g_x = g_dx = dx
+        # products in the operands' own dtype even where the caller's backward runs under autocast
+        with torch.autocast(like.device.type, enabled=False):
+            for i in reversed(range(L)):
+                dx, g_vfirst = _layer_bwd(i, dict(zip(NAMES, layers[i])), dict(zip(NAMES, glayers[i])), saved[i], ns,
+                                          length, g_x, g_dx, None if g_state is None else g_state[:, i],
+                                          None if g_in is None else g_in[:, i], g_vfirst, v_first)
+                g_x = g_dx = dx
         need = ctx.needs_input_grad[4:]
         return (g_x, g_in, None, None) + tuple(g if n else None for g, n in zip(grads, need))
 

@@ -227,7 +227,8 @@ class RWKV7:
         x = params["emb"]["weight"][tokens]
         grad = torch.is_grad_enabled() and (x.requires_grad or state.requires_grad)
         # where the recurrence is this package's: decode steps from native code, whole sequences as one operator
-        own = fused and cls.inner.inner_loop == HipRWKV.inner_loop and not HipRWKV.force_seq
+        own = (fused and cls.inner.inner_loop == HipRWKV.inner_loop and not HipRWKV.force_seq
+               and not ops.autocast_elsewhere(x))
         if own and not grad and T <= 8:
             step = ops.rwkv7_decode(params, x, state, length, new_starts, HipRWKV.assoc_compat)
             if step is not None:

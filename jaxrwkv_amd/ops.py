@@ -94,6 +94,19 @@ def _needs_grad(*tensors):
     return torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
 
 
+def autocast_elsewhere(x):
+    """Whether ``torch.autocast`` makes products of x's dtype come out in another one."""
+    dev = x.device.type
+    return torch.is_autocast_enabled(dev) and torch.get_autocast_dtype(dev) != x.dtype
+
+
+def _one_dtype(io, *tensors):
+    """Kernels take one I/O dtype for all their operands: an operand of another would be read past its end."""
+    for t in tensors:
+        if t is not None and t.dtype != io:
+            raise _lib.HipRwkvError(f"operand of {t.dtype} beside {io}")
+
+
 def _flags(compat, force_seq=False, small_t=True, debug=0):
     return (_lib.LENGTH_I32 | (_lib.COMPAT_ASSOC if compat else 0) | (_lib.FORCE_SEQ if force_seq else 0)
             | (0 if small_t else _lib.NO_SMALL_T) | int(debug))
@@ -485,6 +498,7 @@ def _postmix_fwd(y, r, k, v, g, ln_w, ln_b, r_k, eps):
     io = y.dtype
     H, N = y.shape[-2:]
     rows = y.numel() // (H * N)
+    _one_dtype(io, r, k, v, g, ln_w, ln_b, r_k)
     out = torch.empty_like(y)
     rc = lib.hiprwkv_rwkv7_postmix(_stream(), _DT[io], rows, H, N, _p(y), _p(r), _p(k), _p(v), _p(g), _p(ln_w), _p(ln_b),
                                    _p(r_k), float(eps), _p(out))
@@ -771,6 +785,7 @@ def _ln_shiftmix_fwd(x, dx, ln_w, ln_b, eps, prev, prev_stride, ns, length, mix,
     lib = _lib.load()
     B, T, C = x.shape
     n_out = len(mix)
+    _one_dtype(x.dtype, dx, ln_w, ln_b, prev, shift_out, *mix)
     outs = [torch.empty_like(x) for _ in range(max(n_out, 1))]
     xs = x if dx is None else torch.empty_like(x)
     rc = lib.hiprwkv_rwkv7_ln_shiftmix(_stream(), _DT[x.dtype], B, T, C, n_out, _p(x), _p(dx), _p(ln_w), _p(ln_b), eps,
@@ -841,6 +856,7 @@ def rwkv7_ln_shiftmix(x, dx, ln, prev, new_starts, length, mix, eps=1e-5, shift_
 def _pre_fwd(xw, k, xa, v, vf, xv, w0, a0, v0, k_k, k_a):
     lib = _lib.load()
     H, N = k.shape[-2:]
+    _one_dtype(k.dtype, xw, xa, v, vf, xv, w0, a0, v0, k_k, k_a)
     w, k_out, a_out, b_out = (torch.empty_like(k) for _ in range(4))
     v_out = None if vf is None else torch.empty_like(k)
     rc = lib.hiprwkv_rwkv7_pre(_stream(), _DT[k.dtype], k.numel() // (H * N), H, N, _p(xw), _p(k), _p(xa), _p(v), _p(vf),
