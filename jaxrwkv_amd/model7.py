@@ -116,8 +116,17 @@ def unstack(tree, n_layer):
     return [tree_map(lambda ts: ts[i], split) for i in range(n_layer)]
 
 
-def _needs_grad(tensors):
-    return torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
+def _leaves(tree):
+    for v in tree.values():
+        if isinstance(v, dict):
+            yield from _leaves(v)
+        else:
+            yield v
+
+
+def _needs_grad(x, state, tree):
+    """Whether a derivative is asked for with respect to anything that what follows depends on."""
+    return torch.is_grad_enabled() and any(t.requires_grad for t in (x, state, *_leaves(tree)))
 
 
 class RWKV7:
@@ -225,20 +234,20 @@ class RWKV7:
         C = H * N
         fused = cls.fuse_mix and C <= ops.LN_SHIFTMIX_MAX_C
         x = params["emb"]["weight"][tokens]
-        grad = torch.is_grad_enabled() and (x.requires_grad or state.requires_grad)
         # where the recurrence is this package's: decode steps from native code, whole sequences as one operator
         own = (fused and cls.inner.inner_loop == HipRWKV.inner_loop and not HipRWKV.force_seq
                and not ops.autocast_elsewhere(x))
-        if own and not grad and T <= 8:
+        if own and T <= 8 and not _needs_grad(x, state, params):
             step = ops.rwkv7_decode(params, x, state, length, new_starts, HipRWKV.assoc_compat)
             if step is not None:
                 return step
         norm = (lambda x, dx, ln: ops.rwkv7_ln_shiftmix(x, dx, ln, None, None, None, [])[2][0]) if fused else \
                (lambda x, dx, ln: layer_norm(x if dx is None else x + dx, ln))
         x = norm(x, None, params["ln0"])
+        # x is ln0's result here: a trainable norm counts as well as a trainable embedding.  What trains after the blocks does not.
+        grad = _needs_grad(x, state, params["blocks"])
         stacked = blocks7.gather(params["blocks"]) if own and T > 8 else ()
         if stacked and blocks7.covers(stacked, x, state):
-            grad = grad or _needs_grad(stacked)
             x, dx, new_state = blocks7.run(stacked, x, state, new_starts, length, grad)
             return norm(x, dx, params["ln_out"]) @ params["head"]["weight"].T, new_state
         blocks = unstack(params["blocks"], L)

@@ -47,3 +47,74 @@ def test_backward_inside_autocast(monkeypatch):
     with torch.autocast("cpu", torch.bfloat16):
         (logits.float().sum() + new_state.float().sum()).backward()
     assert all(p.grad.dtype == torch.float32 for _, p in leaves(params))
+
+
+def frozen(params, keep):
+    """Only the parameters that ``keep`` names get a gradient; returns them."""
+    out = {}
+    for name, p in leaves(params):
+        p.requires_grad_(bool(keep(name)))
+        if keep(name):
+            out[name] = p
+    return out
+
+
+KEEP = {"all but the embedding": lambda n: not n.startswith("emb"), "blocks": lambda n: n.startswith("blocks"),
+        "one vector": lambda n: n == "blocks.att.w0", "ln0": lambda n: n.startswith("ln0"),
+        "after the blocks": lambda n: n.split(".")[0] in ("ln_out", "head")}
+
+
+@pytest.mark.parametrize("keep", list(KEEP))
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,B", [(1, 2), (3, 2), (8, 9), (20, 2)])
+def test_every_trainable_parameter_gets_its_gradient(monkeypatch, T, B, dtype, keep):
+    """Whatever is frozen: the derivative is asked for by any tensor that the results depend on, not by the embedding alone.  The
+    new state is written whole on every route."""
+    stub_library.install(monkeypatch)
+    params = model(dtype)
+    trainable = frozen(params, KEEP[keep])
+    logits, new_state = call(params, T, B)
+    assert not new_state.isnan().any() and not logits.isnan().any()
+    assert logits.requires_grad
+    if keep in ("all but the embedding", "blocks", "ln0"):
+        assert new_state.requires_grad
+    (logits.float().sum() + new_state.float().sum()).backward()
+    # a first layer has no value residual, but later ones share the stacked parameter
+    assert [n for n, p in trainable.items() if p.grad is None] == []
+
+
+@pytest.mark.parametrize("T", [3, 20])
+def test_frozen_embedding_with_another_recurrence(monkeypatch, T):
+    from jaxrwkv_amd.model7 import RWKV7
+    from jaxrwkv_amd.rwkv7 import HipRWKV
+    stub_library.install(monkeypatch)
+
+    class Own(HipRWKV):
+        pass
+
+    monkeypatch.setattr(RWKV7, "inner", Own)
+    params = model(torch.bfloat16)
+    trainable = frozen(params, KEEP["blocks"])
+    logits, new_state = call(params, T)
+    assert not new_state.isnan().any()
+    (logits.float().sum() + new_state.float().sum()).backward()
+    assert [n for n, p in trainable.items() if p.grad is None] == []
+
+
+def test_no_derivative_no_graph(monkeypatch):
+    """Training the head alone leaves the blocks on the inference route; without autograd decode steps are native."""
+    from jaxrwkv_amd import blocks7, ops
+    stub_library.install(monkeypatch)
+    params = model(torch.bfloat16)
+    frozen(params, KEEP["after the blocks"])
+    kept = []
+    run = blocks7._run
+    monkeypatch.setattr(blocks7, "_run", lambda *a: kept.append(a[-1]) or run(*a))
+    call(params, 20)
+    assert kept == [False]
+    native = []
+    monkeypatch.setattr(ops, "rwkv7_decode", lambda *a: native.append(1) or ("logits", "state"))
+    call(params, 1)
+    assert not native
+    with torch.no_grad():
+        assert call(params, 1) == ("logits", "state")
