@@ -844,6 +844,8 @@ def rwkv7_ln_shiftmix(x, dx, ln, prev, new_starts, length, mix, eps=1e-5, shift_
     ln_w, ln_b = _dev(ln["weight"], io), _dev(ln["bias"], io)
     mix2 = [_dev(m.reshape(C), io) for m in mix]
     if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, dx, ln_w, ln_b, prev, *mix2)):
+        if shift_out is not None:
+            raise ValueError("rwkv7_ln_shiftmix: shift_out is for calls without autograd")
         xs, shift, *outs = _LnShiftMix.apply(x, dx, ln_w, ln_b, prev, new_starts, length, eps, *mix2)
         return xs, shift, outs
     prev_t, stride = (None, C) if prev is None else _shift_row(prev, B, C, io)

@@ -118,3 +118,13 @@ def test_no_derivative_no_graph(monkeypatch):
     assert not native
     with torch.no_grad():
         assert call(params, 1) == ("logits", "state")
+
+
+def test_a_shift_row_is_not_dropped_under_autograd(monkeypatch):
+    from jaxrwkv_amd import ops
+    stub_library.install(monkeypatch)
+    p = model(torch.float32)["blocks"]
+    ln = {k: v[0].requires_grad_() for k, v in p["ln1"].items()}
+    out = torch.zeros((2, C))
+    with pytest.raises(ValueError):
+        ops.rwkv7_ln_shiftmix(torch.randn(2, 3, C), None, ln, torch.zeros(2, C), None, None, [p["ffn"]["x_k"][0]], shift_out=out)
