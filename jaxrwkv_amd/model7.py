@@ -12,6 +12,7 @@ Model state per sequence, as in the reference (rwkv7.py:176-180, 254-260, 283-28
 parameter dtype; row 0 = channel-mix token-shift state, row 1 = time-mix token-shift state, rows 2.. = the WKV state
 of the layer, a flat reinterpretation of ``(H, N, N)`` [value row, key column].
 """
+import itertools
 import math
 
 import torch
@@ -126,7 +127,8 @@ def _leaves(tree):
 
 def _needs_grad(x, state, tree):
     """Whether a derivative is asked for with respect to anything that what follows depends on."""
-    return torch.is_grad_enabled() and any(t.requires_grad for t in (x, state, *_leaves(tree)))
+    tensors = lambda: itertools.chain((x, state), _leaves(tree))
+    return (torch.is_grad_enabled() and any(t.requires_grad for t in tensors())) or ops.has_tangent(tensors())
 
 
 class RWKV7:
@@ -232,8 +234,10 @@ class RWKV7:
             new_starts = torch.as_tensor(new_starts, device=dev).to(torch.bool).expand(B, T).contiguous()
         L, H, N = params["blocks"]["att"]["r_k"].shape
         C = H * N
-        fused = cls.fuse_mix and C <= ops.LN_SHIFTMIX_MAX_C
         x = params["emb"]["weight"][tokens]
+        # the separate steps carry forward-mode tangents where torch does; the recurrence refuses those that reach it
+        fused = (cls.fuse_mix and C <= ops.LN_SHIFTMIX_MAX_C
+                 and not ops.has_tangent(itertools.chain((x, state), _leaves(params))))
         # where the recurrence is this package's: decode steps from native code, whole sequences as one operator
         own = (fused and cls.inner.inner_loop == HipRWKV.inner_loop and not HipRWKV.force_seq
                and not ops.autocast_elsewhere(x))

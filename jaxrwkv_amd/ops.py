@@ -9,6 +9,7 @@ when new_starts[length]).
 import ctypes
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 
@@ -90,8 +91,15 @@ def _length_ns(length, new_starts, B, T, device, keep=False):
     return length, new_starts
 
 
+def has_tangent(tensors):
+    """Whether one of the tensors carries a forward-mode tangent (with or without autograd enabled)."""
+    return forward_ad._current_level >= 0 and any(forward_ad.unpack_dual(t).tangent is not None for t in tensors)
+
+
 def _needs_grad(*tensors):
-    return torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
+    """Whether the call goes through its autograd function, which also is what refuses forward mode."""
+    tensors = [t for t in tensors if t is not None]
+    return (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)) or has_tangent(tensors)
 
 
 def autocast_elsewhere(x):
@@ -465,7 +473,7 @@ def wkv4(w_neg, u, k, v, s, length=None, new_starts=None, compat=True):
 
 def _wkv4_apply(w, u, k, v, r, s, length, new_starts, flags):
     B, T = k.shape[:2]
-    grad = _needs_grad(w, u, k, v, s) or (r is not None and _needs_grad(r))
+    grad = _needs_grad(w, u, k, v, r, s)
     length, new_starts = _length_ns(length, new_starts, B, T, k.device, keep=grad)
     if grad:
         return _Wkv4.apply(w, u, k, v, r, s, length, new_starts, flags)
@@ -843,7 +851,7 @@ def rwkv7_ln_shiftmix(x, dx, ln, prev, new_starts, length, mix, eps=1e-5, shift_
     dx = None if dx is None else _dev(dx, io)
     ln_w, ln_b = _dev(ln["weight"], io), _dev(ln["bias"], io)
     mix2 = [_dev(m.reshape(C), io) for m in mix]
-    if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, dx, ln_w, ln_b, prev, *mix2)):
+    if _needs_grad(x, dx, ln_w, ln_b, prev, *mix2):
         if shift_out is not None:
             raise ValueError("rwkv7_ln_shiftmix: shift_out is for calls without autograd")
         xs, shift, *outs = _LnShiftMix.apply(x, dx, ln_w, ln_b, prev, new_starts, length, eps, *mix2)
@@ -911,8 +919,7 @@ def rwkv7_pre(xw, k, xa, v, v_first, xv, w0, a0, v0, k_k, k_a):
         args = (xw, k, xa, None, None, None, w0, a0, None, k_k, k_a)
     else:
         args = (xw, k, xa, v, _dev(v_first, io), _dev(xv, io), w0, a0, _dev(v0.reshape(C), io), k_k, k_a)
-    grad = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in args)
-    w, k_out, v_out, a_out, b_out = _Pre.apply(*args) if grad else _pre_fwd(*args)
+    w, k_out, v_out, a_out, b_out = _Pre.apply(*args) if _needs_grad(*args) else _pre_fwd(*args)
     return w, k_out, (v if v_first is None else v_out), a_out, b_out
 
 

@@ -128,3 +128,58 @@ def test_a_shift_row_is_not_dropped_under_autograd(monkeypatch):
     out = torch.zeros((2, C))
     with pytest.raises(ValueError):
         ops.rwkv7_ln_shiftmix(torch.randn(2, 3, C), None, ln, torch.zeros(2, C), None, None, [p["ffn"]["x_k"][0]], shift_out=out)
+
+
+TANGENT = {"state": "state", "embedding": "emb.weight", "block": "blocks.att.x_r"}
+
+
+@pytest.mark.parametrize("where", list(TANGENT))
+@pytest.mark.parametrize("T", [1, 20])
+@pytest.mark.parametrize("grad", [False, True])
+def test_forward_mode_is_refused_and_not_dropped(monkeypatch, where, T, grad):
+    """The recurrence has no forward-mode derivative: a tangent that reaches it is an error."""
+    from torch.autograd import forward_ad
+    stub_library.install(monkeypatch)
+    params = model(torch.bfloat16)
+    state = torch.zeros((2, L, 66, C), dtype=torch.bfloat16)
+    with forward_ad.dual_level(), torch.set_grad_enabled(grad):
+        dual = lambda t: forward_ad.make_dual(t, torch.ones_like(t))
+        if where == "state":
+            state = dual(state)
+        elif where == "embedding":
+            params["emb"]["weight"] = dual(params["emb"]["weight"])
+        else:
+            params["blocks"]["att"]["x_r"] = dual(params["blocks"]["att"]["x_r"])
+        with pytest.raises(RuntimeError, match="jvp"):
+            call(params, T, state=state)
+
+
+@pytest.mark.parametrize("T", [1, 20])
+def test_forward_mode_after_the_blocks(monkeypatch, T):
+    """What follows the recurrence is torch's: its tangents are right."""
+    from torch.autograd import forward_ad
+    stub_library.install(monkeypatch)
+    params = model(torch.float32)
+    with forward_ad.dual_level():
+        for name in ("ln_out", "head"):
+            w = params[name]["weight"]
+            params[name]["weight"] = forward_ad.make_dual(w, w)
+        logits, _ = call(params, T)
+        value, tangent = forward_ad.unpack_dual(logits)
+    # logits are linear in head and in ln_out's weight (its bias is zero): each tangent is the value itself
+    torch.testing.assert_close(tangent, 2 * value, rtol=1e-4, atol=1e-6)
+
+
+@pytest.mark.parametrize("op", ["wkv4", "wkv6", "wkv7"])
+def test_operators_refuse_tangents(monkeypatch, op):
+    from torch.autograd import forward_ad
+    from jaxrwkv_amd import ops
+    stub_library.install(monkeypatch)
+    tok = lambda: torch.randn(2, 20, 1, 64)
+    args = {"wkv4": [torch.randn(64), torch.randn(64), torch.randn(2, 20, 64), torch.randn(2, 20, 64), torch.zeros(2, 3, 64)],
+            "wkv6": [tok(), tok(), tok(), tok(), torch.randn(1, 64), torch.zeros(2, 1, 64, 64)],
+            "wkv7": [tok() for _ in range(6)] + [torch.zeros(2, 1, 64, 64)]}[op]
+    for i in range(len(args)):
+        with forward_ad.dual_level():
+            with pytest.raises(RuntimeError, match="jvp"):
+                getattr(ops, op)(*args[:i], forward_ad.make_dual(args[i], torch.ones_like(args[i])), *args[i + 1:])
