@@ -314,7 +314,7 @@ class _Blocks(torch.autograd.Function):
 def _run(x, state, ns, length, params, keep):
     L = params[0].shape[0]
     layers = list(zip(*(t.unbind(0) for t in params)))
-    new_state = torch.empty_like(state)
+    new_state = torch.empty_like(state, memory_format=torch.contiguous_format)      # the kernels write rows of neighbours
     dx = v_first = None
     saved = [] if keep else None
     for i in range(L):
@@ -322,6 +322,8 @@ def _run(x, state, ns, length, params, keep):
                                        length, keep)
         if keep:
             saved.append(S)
+    if not state.is_contiguous():
+        new_state = torch.empty_like(state).copy_(new_state)                          # in the order of the caller's
     return x, dx, new_state, saved, v_first
 
 

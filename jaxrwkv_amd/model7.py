@@ -260,6 +260,7 @@ class RWKV7:
         in_place = fused and not grad and state.dtype == x.dtype and (C * x.element_size()) % 16 == 0
         packed = T <= 8 and hasattr(cls.inner, "step_packed") and not grad
         new_state = torch.empty_like(state) if (in_place or packed) else None
+        in_place = in_place and new_state.is_contiguous()
         rows = []                                   # otherwise: the new state's parts in memory order, joined at the end
         v_first, dx = None, None
         for i, blk in enumerate(blocks):

@@ -89,3 +89,15 @@ def test_frozen_embedding(T, dtype):
         assert g is not None, n
         if full[2][n].abs().max() > 0:
             assert rel(g, full[2][n]) < (1e-5 if dtype == torch.float32 else 2e-3), (n, rel(g, full[2][n]))
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_state_in_another_memory_order(grad):
+    from jaxrwkv_amd.model7 import RWKV7
+    tok, state = inputs(3, 20, torch.bfloat16)
+    params = model(torch.bfloat16)
+    for _, p in leaves(params):
+        p.requires_grad_(grad)
+    other = state.transpose(2, 3).contiguous().transpose(2, 3)
+    a, b = RWKV7.forward(params, tok, state), RWKV7.forward(params, tok, other)
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1]) and b[1].stride() == other.stride()

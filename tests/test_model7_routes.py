@@ -183,3 +183,25 @@ def test_operators_refuse_tangents(monkeypatch, op):
         with forward_ad.dual_level():
             with pytest.raises(RuntimeError, match="jvp"):
                 getattr(ops, op)(*args[:i], forward_ad.make_dual(args[i], torch.ones_like(args[i])), *args[i + 1:])
+
+
+@pytest.mark.parametrize("T,grad", [(3, True), (20, False), (20, True)])
+def test_state_in_another_memory_order(monkeypatch, T, grad):
+    """A model state whose channels do not lie next to each other: every row of the new state is written, and nothing beside it.  The
+    stub fills what a kernel is told to: C elements from the pointer on."""
+    stub = stub_library.install(monkeypatch)
+    params = model(torch.float32)
+    state = torch.randn(2, L, C, 66).transpose(2, 3)
+    if grad:
+        frozen(params, KEEP["blocks"])
+    seen = []
+    call_ = stub_library.fill
+
+    def fill(tensors):
+        seen.extend(t for t in tensors if t.shape == (2, C))
+        call_(tensors)
+
+    monkeypatch.setattr(stub_library, "fill", fill)
+    _, new_state = call(params, T, state=state)
+    assert not new_state.isnan().any()
+    assert seen and all(t.stride(1) == 1 for t in seen)          # shift rows: what the kernels take is a row of neighbours
