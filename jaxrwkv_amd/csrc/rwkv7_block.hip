@@ -109,9 +109,8 @@ struct Held<bf16_t> {
 // in-sequence index of the token whose xn the state keeps: x[length - 1] with the wrap-around of negative indices
 __device__ __forceinline__ int64_t last_token(const int32_t* length, int64_t b, int64_t T) {
   if (length == nullptr) return T - 1;
-  int64_t L = length[b];
-  L = (L < 0 ? 0 : L) - 1;
-  return L < 0 ? T - 1 : L % T;
+  const int64_t t = ((int64_t)length[b] - 1) % T;
+  return t < 0 ? t + T : t;
 }
 
 template <typename T, int NOUT>

@@ -101,3 +101,20 @@ def test_state_in_another_memory_order(grad):
     other = state.transpose(2, 3).contiguous().transpose(2, 3)
     a, b = RWKV7.forward(params, tok, state), RWKV7.forward(params, tok, other)
     assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1]) and b[1].stride() == other.stride()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T", [5, 20])
+def test_lengths_outside_the_sequence(T, dtype, monkeypatch):
+    """The shift row is that of token (length - 1) mod T whatever the length; the recurrence counts a negative one as none."""
+    from jaxrwkv_amd.model7 import RWKV7
+    length = torch.tensor([-1, -2 * T - 2, 0, 1, T, T + 3, -(2 ** 31)], device="cuda", dtype=torch.int32)
+    tok, state = inputs(len(length), T, dtype)
+    params = model(dtype)
+    with torch.no_grad():
+        got = RWKV7.forward(params, tok, state, length)
+        monkeypatch.setattr(RWKV7, "fuse_mix", False)
+        want = RWKV7.forward(params, tok, state, length)
+    for i in range(len(length)):
+        for rows in (slice(0, 1), slice(1, 2), slice(2, 66)):           # a wrong token's row would be about 1 away
+            assert rel(got[1][i, :, rows], want[1][i, :, rows]) < (1e-4 if dtype == torch.float32 else 3e-2), (i, rows)
