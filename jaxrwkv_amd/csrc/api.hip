@@ -759,6 +759,7 @@ int hiprwkv_rwkv7_ln_shiftmix(hiprwkv_stream stream, int io_dtype, int64_t B, in
 }
 
 size_t hiprwkv_rwkv7_ln_shiftmix_bwd_workspace_bytes(int64_t B, int64_t T, int64_t C, int n_out) {
+  if (B <= 0 || T <= 0 || C <= 0 || n_out < 0) return 0;
   const int64_t run = ln_shiftmix_bwd_run(B * T);
   return (size_t)((B * T + run - 1) / run) * (n_out + 2) * C * sizeof(float);
 }
@@ -820,7 +821,7 @@ int hiprwkv_rwkv7_pre(hiprwkv_stream stream, int io_dtype, int64_t rows, int64_t
 }
 
 size_t hiprwkv_rwkv7_pre_bwd_workspace_bytes(int64_t rows, int64_t H, int64_t N) {
-  return (size_t)rwkv7_pre_bwd_rows(rows, H) * 5 * H * N * sizeof(float);
+  return rows <= 0 || H <= 0 || N <= 0 ? 0 : (size_t)rwkv7_pre_bwd_rows(rows, H) * 5 * H * N * sizeof(float);
 }
 
 int hiprwkv_rwkv7_pre_bwd(hiprwkv_stream stream, int io_dtype, int64_t rows, int64_t H, int64_t N, const void* xw,
@@ -855,7 +856,9 @@ int hiprwkv_rwkv7_pre_bwd(hiprwkv_stream stream, int io_dtype, int64_t rows, int
   return gate_done("rwkv7_pre_bwd", launch_rwkv7_pre_bwd(io_dtype == HIPRWKV_F32, A, dparam, static_cast<hipStream_t>(stream)));
 }
 
-size_t hiprwkv_rwkv7_decode_workspace_bytes(const hiprwkv_rwkv7_decode_args* args) { return rwkv7_decode_workspace(*args); }
+size_t hiprwkv_rwkv7_decode_workspace_bytes(const hiprwkv_rwkv7_decode_args* args) {
+  return args == nullptr || args->B <= 0 || args->T <= 0 ? 0 : rwkv7_decode_workspace(*args);
+}
 
 int hiprwkv_rwkv7_decode(hiprwkv_stream stream, const hiprwkv_rwkv7_decode_args* args) {
   if (args == nullptr) return fail(HIPRWKV_EINVAL, "rwkv7_decode: null arguments");
@@ -904,7 +907,9 @@ int check_wkv4(const char* op, int io_dtype, int64_t B, int64_t T, int64_t C, un
 }
 }  // namespace
 
-size_t hiprwkv_wkv4_mix_workspace_bytes(int64_t B, int64_t T, int64_t C) { return wkv4_part_bytes(B, T, C, 4); }
+size_t hiprwkv_wkv4_mix_workspace_bytes(int64_t B, int64_t T, int64_t C) {
+  return B <= 0 || T <= 0 || C <= 0 ? 0 : wkv4_part_bytes(B, T, C, 4);
+}
 
 int hiprwkv_wkv4_mix(hiprwkv_stream stream, int io_dtype, int64_t B, int64_t T, int64_t C, const void* w, const void* u,
                      const void* k, const void* v, const void* r, const void* s, const uint32_t* length,
@@ -931,6 +936,7 @@ int hiprwkv_wkv4_mix(hiprwkv_stream stream, int io_dtype, int64_t B, int64_t T, 
 }
 
 size_t hiprwkv_wkv4_mix_bwd_workspace_bytes(int64_t B, int64_t T, int64_t C) {
+  if (B <= 0 || T <= 0 || C <= 0) return 0;
   int64_t part;
   const int64_t nz = wkv4_parts(B, T, C, &part);
   return wkv4_part_bytes(B, T, C, 8) + align256((size_t)B * nz * 2 * C * sizeof(float));
@@ -1001,7 +1007,7 @@ int hiprwkv_gemm(hiprwkv_stream stream, int n_jobs, const hiprwkv_gemm_job* jobs
 }
 
 size_t hiprwkv_rwkv7_postmix_bwd2_workspace_bytes(int64_t rows, int64_t H, int64_t N) {
-  return (size_t)rwkv7_postmix_bwd_rows(rows, H) * 3 * H * N * sizeof(float);
+  return rows <= 0 || H <= 0 || N <= 0 ? 0 : (size_t)rwkv7_postmix_bwd_rows(rows, H) * 3 * H * N * sizeof(float);
 }
 
 int hiprwkv_rwkv7_postmix_bwd2(hiprwkv_stream stream, int io_dtype, int64_t rows, int64_t H, int64_t N, const void* y,

@@ -223,3 +223,21 @@ def test_phased_allocation_gives_the_asked_address_phase():
     assert small.shape == (4, 1, 8, 64) and small._base is None
     f16 = ops._empty_phased((2, 512, 8, 64), torch.float16, "cpu", 5)
     assert ops._phase(f16) == 5 and f16.dtype == torch.float16
+
+
+def test_workspace_sizes_of_empty_calls():
+    """A size is asked for before the call that refuses empty arguments: it is zero, not a division by one of them."""
+    from jaxrwkv_amd import _lib
+    lib = _lib.load()
+    for B, T, C in ((0, 8, 64), (2, 0, 64), (2, 8, 0), (-1, 8, 64), (2, -8, 64), (2, 8, -64)):
+        assert lib.hiprwkv_wkv4_mix_workspace_bytes(B, T, C) == 0
+        assert lib.hiprwkv_wkv4_mix_bwd_workspace_bytes(B, T, C) == 0
+        assert lib.hiprwkv_rwkv7_ln_shiftmix_bwd_workspace_bytes(B, T, C, 6) == 0
+    for rows, H in ((0, 2), (5, 0), (-5, 2), (5, -2)):
+        assert lib.hiprwkv_rwkv7_pre_bwd_workspace_bytes(rows, H, 64) == 0
+        assert lib.hiprwkv_rwkv7_postmix_bwd2_workspace_bytes(rows, H, 64) == 0
+    for dtype, B, T, H in ((1, 0, 999, 2), (1, 2, 0, 2), (1, 2, 999, 0), (1, -2, 999, 2)):
+        assert lib.hiprwkv_wkv7_fwd_workspace_bytes(dtype, B, T, H, 64) == 0
+        assert lib.hiprwkv_wkv6_fwd_workspace_bytes(dtype, B, T, H, 64) == 0
+    assert lib.hiprwkv_rwkv7_decode_workspace_bytes(None) == 0
+    assert lib.hiprwkv_rwkv7_decode_workspace_bytes(ctypes.byref(_lib.Rwkv7DecodeArgs())) == 0
