@@ -109,6 +109,10 @@ def tree_map(fn, tree):
     return {k: tree_map(fn, v) if isinstance(v, dict) else fn(v) for k, v in tree.items()}
 
 
+def layer_of(tree, i):
+    return tree_map(lambda t: t[i], tree)
+
+
 def unstack(tree, n_layer):
     """The per-layer trees of a tree of stacked parameters.  One ``unbind`` per parameter: its backward is one ``stack``,
     where a slice per layer would add a zero-filled copy of the whole stack per layer and parameter (0.1B shape, one
@@ -135,8 +139,8 @@ class RWKV7:
     """``forward`` / ``default_state`` with the reference's argument names; batched over the leading axis."""
 
     inner = HipRWKV
-    #: use the fused kernels beside the recurrence (ops.rwkv7_ln_shiftmix, rwkv7_pre, rwkv7_postmix, rwkv7_relusq), with or
-    #: without autograd; models wider than ops.LN_SHIFTMIX_MAX_C channels run the separate steps
+    #: use the fused kernels beside the recurrence, with or without autograd: ops.rwkv7_ln_shiftmix (up to
+    #: ops.LN_SHIFTMIX_MAX_C channels; wider models: torch's norm and ops.rwkv7_shiftmix), rwkv7_pre, rwkv7_postmix, rwkv7_relusq
     fuse_mix = True
 
     @classmethod
@@ -147,42 +151,49 @@ class RWKV7:
         return torch.zeros((batch, L, 2 + N, emb.shape[1]), dtype=emb.dtype, device=emb.device)
 
     @classmethod
-    def _mix_head(cls, x, dx, ln, prev, new_starts, length, mix, fused, shift_out=None):
-        """Residual addition, LayerNorm, token shift of rwkv7.py:227-229 / 192-194 (previous token, the state row for
-        t = 0, zero at new_starts) and interpolation; returns (x + dx, new shift row, interpolations)."""
-        if fused:
-            return ops.rwkv7_ln_shiftmix(x, dx, ln, prev, new_starts, length, mix, shift_out=shift_out)
-        B, T, C = x.shape
-        if dx is not None:
-            x = x + dx
-        xn = layer_norm(x, ln)
-        sx = torch.cat([prev[:, None], xn[:, :-1]], dim=1)
+    def _shift(cls, x, prev, new_starts):
+        """Token shift of rwkv7.py:227-229 / 192-194: previous token (state row for t = 0), zero at new_starts."""
+        sx = torch.cat([prev[:, None], x[:, :-1]], dim=1)
         if new_starts is not None:
             sx = torch.where(new_starts[:, :, None], torch.zeros_like(sx), sx)
-        sx = sx - xn
-        # xn[length - 1] with the wrap-around of negative indices
-        last = (length.long() - 1) % T if length is not None else torch.full((B,), T - 1, device=x.device)
-        return x, xn[torch.arange(B, device=x.device), last], [xn + sx * m for m in mix]
+        return sx - x
 
     @classmethod
-    def channel_mixing_seq(cls, x, dx, ln, state_row, ffn, length, new_starts, fused, shift_out=None):
-        """rwkv7.py:190-198 with the residual addition and the norm in front; returns (x + dx, output, new shift row)."""
-        x, shift, (xk,) = cls._mix_head(x, dx, ln, state_row, new_starts, length, [ffn["x_k"]], fused, shift_out)
+    def _interpolate(cls, x, prev, new_starts, mix):
+        if cls.fuse_mix and not ops.has_tangent((x, prev, *mix)):
+            return ops.rwkv7_shiftmix(x, prev, new_starts, mix)
+        sx = cls._shift(x, prev, new_starts)
+        return [x + sx * m for m in mix]
+
+    @classmethod
+    def _channel_mix(cls, xk, ffn):
         k = xk @ ffn["key"]["weight"].T
-        k = ops.rwkv7_relusq(k) if fused else torch.square(torch.relu(k))
-        return x, k @ ffn["value"]["weight"].T, shift
+        k = ops.rwkv7_relusq(k) if cls.fuse_mix and not ops.has_tangent((k,)) else torch.square(torch.relu(k))
+        return k @ ffn["value"]["weight"].T
 
     @classmethod
-    def time_mixing_seq(cls, x, dx, ln, shift_row, wkv_state, v_first, att, length, new_starts, layer_id, fused,
-                        shift_out=None, wkv_out=None):
-        """rwkv7.py:223-267 with the residual addition and the norm in front.  wkv_state (B, N, C) is the layer's rows 2..
-        of the model state.  With ``wkv_out`` (the same rows of the new model state; decode steps without autograd) the
-        recurrence reads and writes the two views in place and the new state is returned as None.
-        Returns (x + dx, output, new shift row, new wkv state, v_first)."""
-        B, T, C = x.shape
+    def channel_mixing_seq(cls, x, state_row, ffn, last_idx, new_starts):
+        """rwkv7.py:190-198; x is the norm's result.  Returns (output, new shift row)."""
+        xk, = cls._interpolate(x, state_row, new_starts, [ffn["x_k"]])
+        return cls._channel_mix(xk, ffn), x[torch.arange(x.shape[0], device=x.device), last_idx]
+
+    @classmethod
+    def time_mixing_seq(cls, x, shift_row, wkv_state, v_first, att, length, last_idx, new_starts, layer_id,
+                        wkv_out=None):
+        """rwkv7.py:223-267; x is the norm's result, wkv_state (B, N, C) the layer's rows 2.. of the model state.  With
+        ``wkv_out`` (the same rows of the new model state; decode steps without autograd) the recurrence reads and writes the
+        two views in place and the third result is None.  Returns (output, new shift row, new wkv state, v_first)."""
+        mixed = cls._interpolate(x, shift_row, new_starts, [att[n] for n in blocks7.MIX])
+        y, s_new, v_first = cls._time_mix(mixed, wkv_state, v_first, att, length, new_starts, layer_id, wkv_out)
+        return y, x[torch.arange(x.shape[0], device=x.device), last_idx], s_new, v_first
+
+    @classmethod
+    def _time_mix(cls, mixed, wkv_state, v_first, att, length, new_starts, layer_id, wkv_out):
+        """``time_mixing_seq`` from the six interpolations on."""
+        xr, xw, xk, xv, xa, xg = mixed
+        B, T, C = xr.shape
         H, N = att["r_k"].shape
-        mix = [att[n] for n in ("x_r", "x_w", "x_k", "x_v", "x_a", "x_g")]
-        x, shift, (xr, xw, xk, xv, xa, xg) = cls._mix_head(x, dx, ln, shift_row, new_starts, length, mix, fused, shift_out)
+        fused = cls.fuse_mix and not ops.has_tangent(itertools.chain(mixed, (wkv_state, v_first), _leaves(att)))
         heads = lambda t: t.reshape(B, T, H, N)
         r = heads(xr @ att["receptance"]["weight"].T)
         k = heads(xk @ att["key"]["weight"].T)
@@ -192,15 +203,15 @@ class RWKV7:
         v_lora = heads((xv @ att["v1"]) @ att["v2"]) if layer_id != 0 else None
         g = heads(torch.sigmoid(xg @ att["g1"]) @ att["g2"])
         if layer_id == 0:
-            v_first = v
+            v_first = v.reshape(B, T, C)
         if fused:
-            w, k, v, a, b = ops.rwkv7_pre(w_lora, k, a_lora, v, None if layer_id == 0 else v_first, v_lora, att["w0"],
+            w, k, v, a, b = ops.rwkv7_pre(w_lora, k, a_lora, v, None if layer_id == 0 else heads(v_first), v_lora, att["w0"],
                                           att["a0"], att["v0"], att["k_k"], att["k_a"])
         else:
             par = lambda n: att[n].reshape(H, N)
-            w = -F.softplus(-(par("w0") + w_lora).float()).to(x.dtype) - 0.5
+            w = -F.softplus(-(par("w0") + w_lora).float()).to(xr.dtype) - 0.5
             if layer_id != 0:
-                v = v + (v_first - v) * torch.sigmoid(par("v0") + v_lora)
+                v = v + (heads(v_first) - v) * torch.sigmoid(par("v0") + v_lora)
             a = torch.sigmoid(par("a0") + a_lora)
             kk = k * par("k_k")
             kk = kk / torch.clamp(torch.linalg.vector_norm(kk.float(), dim=-1, keepdim=True), min=1e-12).to(kk.dtype)
@@ -217,10 +228,10 @@ class RWKV7:
         else:
             y = out.reshape(B * T, C).float()
             y = F.group_norm(y, H, att["ln_x"]["weight"].float(), att["ln_x"]["bias"].float(), 64e-5)
-            y = y.to(x.dtype).reshape(B, T, C)
+            y = y.to(xr.dtype).reshape(B, T, C)
             bonus = ((r * k * att["r_k"]).sum(-1, keepdim=True) * v).reshape(B, T, C)
             y = (y + bonus) * g.reshape(B, T, C)
-        return x, y @ att["output"]["weight"].T, shift, s_new, v_first
+        return y @ att["output"]["weight"].T, s_new, v_first
 
     @classmethod
     def forward(cls, params, tokens, state, length=None, new_starts=None):
@@ -238,8 +249,10 @@ class RWKV7:
         # the separate steps carry forward-mode tangents where torch does; the recurrence refuses those that reach it
         fused = (cls.fuse_mix and C <= ops.LN_SHIFTMIX_MAX_C
                  and not ops.has_tangent(itertools.chain((x, state), _leaves(params))))
-        # where the recurrence is this package's: decode steps from native code, whole sequences as one operator
-        own = (fused and cls.inner.inner_loop == HipRWKV.inner_loop and not HipRWKV.force_seq
+        # a subclass's own mixing methods get what they always got: the norm's result, and every argument as a tensor
+        steps = any(getattr(cls, n).__func__ is not getattr(RWKV7, n).__func__ for n in ("time_mixing_seq", "channel_mixing_seq"))
+        # where everything is this package's: decode steps from native code, whole sequences as one operator
+        own = (fused and not steps and cls.inner.inner_loop == HipRWKV.inner_loop and not HipRWKV.force_seq
                and not ops.autocast_elsewhere(x))
         if own and T <= 8 and not _needs_grad(x, state, params):
             step = ops.rwkv7_decode(params, x, state, length, new_starts, HipRWKV.assoc_compat)
@@ -255,21 +268,36 @@ class RWKV7:
             x, dx, new_state = blocks7.run(stacked, x, state, new_starts, length, grad)
             return norm(x, dx, params["ln_out"]) @ params["head"]["weight"].T, new_state
         blocks = unstack(params["blocks"], L)
+        head = fused and not steps
+        if steps:
+            length = torch.full((B,), T, dtype=torch.int32, device=dev) if length is None else length
+            new_starts = torch.zeros((B, T), dtype=torch.bool, device=dev) if new_starts is None else new_starts
+        if not head:                                # xn[length - 1] with the wrap-around of negative indices
+            last = torch.full((B,), T - 1, device=dev) if length is None else (length.long() - 1) % T
         # without autograd the layers write their rows of the new state where they belong; decode steps read and write the
         # recurrence's rows in place as well
-        in_place = fused and not grad and state.dtype == x.dtype and (C * x.element_size()) % 16 == 0
+        in_place = head and not grad and state.dtype == x.dtype and (C * x.element_size()) % 16 == 0
         packed = T <= 8 and hasattr(cls.inner, "step_packed") and not grad
         new_state = torch.empty_like(state) if (in_place or packed) else None
         in_place = in_place and new_state.is_contiguous()
         rows = []                                   # otherwise: the new state's parts in memory order, joined at the end
-        v_first, dx = None, None
+        v_first, dx = x, None
         for i, blk in enumerate(blocks):
             st, nst = state[:, i], (None if new_state is None else new_state[:, i])
-            x, dx, shift1, wkv, v_first = cls.time_mixing_seq(
-                x, dx, blk["ln1"], st[:, 1], st[:, 2:], v_first, blk["att"], length, new_starts, i, fused,
-                nst[:, 1] if in_place else None, nst[:, 2:] if packed else None)
-            x, dx, shift0 = cls.channel_mixing_seq(x, dx, blk["ln2"], st[:, 0], blk["ffn"], length, new_starts, fused,
-                                                   nst[:, 0] if in_place else None)
+            att, ffn, wkv_out = blk["att"], blk["ffn"], (nst[:, 2:] if packed else None)
+            if head:
+                x, shift1, mixed = ops.rwkv7_ln_shiftmix(x, dx, blk["ln1"], st[:, 1], new_starts, length,
+                                                         [att[n] for n in blocks7.MIX], shift_out=nst[:, 1] if in_place else None)
+                dx, wkv, v_first = cls._time_mix(mixed, st[:, 2:], v_first, att, length, new_starts, i, wkv_out)
+                x, shift0, (xk,) = ops.rwkv7_ln_shiftmix(x, dx, blk["ln2"], st[:, 0], new_starts, length, [ffn["x_k"]],
+                                                         shift_out=nst[:, 0] if in_place else None)
+                dx = cls._channel_mix(xk, ffn)
+            else:
+                x = x if dx is None else x + dx
+                dx, shift1, wkv, v_first = cls.time_mixing_seq(layer_norm(x, blk["ln1"]), st[:, 1], st[:, 2:], v_first, att, length,
+                                                               last, new_starts, i, wkv_out)
+                x = x + dx
+                dx, shift0 = cls.channel_mixing_seq(layer_norm(x, blk["ln2"]), st[:, 0], ffn, last, new_starts)
             if new_state is None:
                 rows += [shift0[:, None], shift1[:, None], wkv]
                 continue

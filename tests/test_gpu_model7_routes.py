@@ -118,3 +118,25 @@ def test_lengths_outside_the_sequence(T, dtype, monkeypatch):
     for i in range(len(length)):
         for rows in (slice(0, 1), slice(1, 2), slice(2, 66)):           # a wrong token's row would be about 1 away
             assert rel(got[1][i, :, rows], want[1][i, :, rows]) < (1e-4 if dtype == torch.float32 else 3e-2), (i, rows)
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("T", [3, 20])
+def test_wide_models(T, grad, monkeypatch):
+    """The route of models too wide for the fused head against the other one: sums of the norm in another order (fp32)."""
+    from jaxrwkv_amd import ops
+    from jaxrwkv_amd.model7 import RWKV7
+    tok, state = inputs(3, T, torch.float32)
+    ns = torch.rand((3, T), device="cuda", generator=torch.Generator("cuda").manual_seed(3)) < 0.1
+    length = torch.tensor([1, T, 0], device="cuda", dtype=torch.int32)
+
+    def run():
+        params = model(torch.float32)
+        ps = [p.requires_grad_(grad) for _, p in leaves(params)]
+        outs = RWKV7.forward(params, tok, state, length, ns)
+        return list(outs) + (list(torch.autograd.grad(outs, ps, [torch.ones_like(o) for o in outs])) if grad else [])
+
+    want = run()
+    monkeypatch.setattr(ops, "LN_SHIFTMIX_MAX_C", 64)
+    for i, (a, b) in enumerate(zip(run(), want)):
+        assert rel(a, b) < 2e-4, (i, tuple(a.shape), rel(a, b))

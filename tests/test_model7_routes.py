@@ -205,3 +205,55 @@ def test_state_in_another_memory_order(monkeypatch, T, grad):
     _, new_state = call(params, T, state=state)
     assert not new_state.isnan().any()
     assert seen and all(t.stride(1) == 1 for t in seen)          # shift rows: what the kernels take is a row of neighbours
+
+
+@pytest.mark.parametrize("T", [3, 20])
+def test_wide_models_keep_the_fused_steps(monkeypatch, T):
+    """Channels that one workgroup of the fused head cannot span: norm and residual are torch's, everything else stays fused."""
+    from jaxrwkv_amd import ops
+    stub = stub_library.install(monkeypatch)
+    monkeypatch.setattr(ops, "LN_SHIFTMIX_MAX_C", C - 8)
+    with torch.no_grad():
+        _, new_state = call(model(torch.bfloat16), T)
+    assert not new_state.isnan().any()
+    assert "hiprwkv_rwkv7_ln_shiftmix" not in stub.calls and "hiprwkv_gemm" not in stub.calls
+    for name, n in (("shiftmix", 2 * L), ("pre", L), ("postmix", L), ("relusq", L)):
+        assert stub.calls.count("hiprwkv_rwkv7_" + name) == n, name
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("T", [1, 3, 20])
+def test_a_subclass_with_mixing_methods_of_its_own(monkeypatch, T, grad):
+    """They are called for every layer, with the norm's result and tensors for length and new_starts."""
+    from jaxrwkv_amd.model7 import RWKV7
+    stub_library.install(monkeypatch)
+    seen = []
+
+    class Model(RWKV7):
+        @classmethod
+        def time_mixing_seq(cls, x, shift_row, wkv_state, v_first, att, length, last_idx, new_starts, layer_id, wkv_out=None):
+            assert v_first.shape == x.shape == (2, T, C) and length.shape == (2,) and new_starts.shape == (2, T)
+            seen.append(("time", layer_id))
+            out, *rest = super().time_mixing_seq(x, shift_row, wkv_state, v_first, att, length, last_idx, new_starts, layer_id, wkv_out)
+            return (0 * out, *rest)
+
+        @classmethod
+        def channel_mixing_seq(cls, x, state_row, ffn, last_idx, new_starts):
+            assert last_idx.tolist() == [T - 1] * 2
+            seen.append(("channel", state_row.shape))
+            return torch.ones_like(x), x[:, -1]
+
+    params = model(torch.bfloat16)
+    frozen(params, KEEP["all but the embedding"] if grad else (lambda n: False))
+    tok = torch.arange(2 * T).reshape(2, T) % V
+    logits, new_state = Model.forward(params, tok, RWKV7.default_state(params, 2))
+    assert seen == [x for i in range(L) for x in (("time", i), ("channel", (2, C)))]
+    assert not new_state.isnan().any() and logits.shape == (2, T, V)
+
+
+def test_layer_of():
+    from jaxrwkv_amd.model7 import layer_of, unstack
+    params = model(torch.float32)["blocks"]
+    for i, tree in enumerate(unstack(params, L)):
+        for (n, a), (m, b) in zip(leaves(layer_of(params, i)), leaves(tree)):
+            assert n == m and torch.equal(a, b)
