@@ -258,8 +258,10 @@ class RWKV7:
             step = ops.rwkv7_decode(params, x, state, length, new_starts, HipRWKV.assoc_compat)
             if step is not None:
                 return step
-        norm = (lambda x, dx, ln: ops.rwkv7_ln_shiftmix(x, dx, ln, None, None, None, [])[2][0]) if fused else \
-               (lambda x, dx, ln: layer_norm(x if dx is None else x + dx, ln))
+        # the fused norm takes one dtype: a norm held in another (fp32 beside bf16) is not rounded to it
+        fits = lambda *lns: fused and all(t.dtype == x.dtype for ln in lns for t in ln.values())
+        norm = lambda x, dx, ln: (ops.rwkv7_ln_shiftmix(x, dx, ln, None, None, None, [])[2][0] if fits(ln) else
+                                  layer_norm(x if dx is None else x + dx, ln))
         x = norm(x, None, params["ln0"])
         # x is ln0's result here: a trainable norm counts as well as a trainable embedding.  What trains after the blocks does not.
         grad = _needs_grad(x, state, params["blocks"])
@@ -268,7 +270,7 @@ class RWKV7:
             x, dx, new_state = blocks7.run(stacked, x, state, new_starts, length, grad)
             return norm(x, dx, params["ln_out"]) @ params["head"]["weight"].T, new_state
         blocks = unstack(params["blocks"], L)
-        head = fused and not steps
+        head = not steps and fits(params["blocks"]["ln1"], params["blocks"]["ln2"])
         if steps:
             length = torch.full((B,), T, dtype=torch.int32, device=dev) if length is None else length
             new_starts = torch.zeros((B, T), dtype=torch.bool, device=dev) if new_starts is None else new_starts

@@ -257,3 +257,22 @@ def test_layer_of():
     for i, tree in enumerate(unstack(params, L)):
         for (n, a), (m, b) in zip(leaves(layer_of(params, i)), leaves(tree)):
             assert n == m and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("T", [3, 20])
+def test_norms_held_in_fp32_stay_so(monkeypatch, T):
+    """fp32 norms in a bf16 model: the fused head takes one type, and rounding the parameter to it would lose what the model has."""
+    stub = stub_library.install(monkeypatch)
+    params = model(torch.bfloat16)
+    for ln in (params["ln0"], params["ln_out"], params["blocks"]["ln1"], params["blocks"]["ln2"]):
+        for k in ln:
+            ln[k] = ln[k].float()
+    with torch.no_grad():
+        call(params, T)
+    assert "hiprwkv_rwkv7_ln_shiftmix" not in stub.calls and "hiprwkv_rwkv7_shiftmix" in stub.calls
+    stub.calls.clear()
+    params["ln_out"]["weight"] = params["ln_out"]["weight"].bfloat16()
+    params["blocks"]["ln2"] = {k: v.bfloat16() for k, v in params["blocks"]["ln2"].items()}
+    with torch.no_grad():
+        call(params, T)                              # one norm's bias or one norm alone
+    assert "hiprwkv_rwkv7_ln_shiftmix" not in stub.calls
