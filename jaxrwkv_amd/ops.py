@@ -33,6 +33,11 @@ def _dev(x, dtype=None):
     return x.contiguous()
 
 
+def _aligned(x):
+    """x, or a copy of it where it does not lie on a 16-byte boundary (a slice of a flat array of parameters)."""
+    return x if x.data_ptr() % 16 == 0 else x.clone()
+
+
 # Placement of the (B,T,H,N) arrays one call touches.  Rows of different arrays at the same (token, head) are accessed
 # together; when the arrays' base addresses are congruent modulo 1 KiB (any two large allocations of a caching
 # allocator are: they start on 2 MiB boundaries) those rows compete for the same part of the memory system, and the
@@ -849,7 +854,7 @@ def rwkv7_ln_shiftmix(x, dx, ln, prev, new_starts, length, mix, eps=1e-5, shift_
     assert len(mix) in (0, 1, 6) and C % 8 == 0 and C <= LN_SHIFTMIX_MAX_C, (len(mix), C)
     x = _dev(x, io)
     dx = None if dx is None else _dev(dx, io)
-    ln_w, ln_b = _dev(ln["weight"], io), _dev(ln["bias"], io)
+    ln_w, ln_b = (_aligned(_dev(ln[n].reshape(C), io)) for n in ("weight", "bias"))
     mix2 = [_dev(m.reshape(C), io) for m in mix]
     if _needs_grad(x, dx, ln_w, ln_b, prev, *mix2):
         if shift_out is not None:

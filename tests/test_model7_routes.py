@@ -276,3 +276,23 @@ def test_norms_held_in_fp32_stay_so(monkeypatch, T):
     with torch.no_grad():
         call(params, T)                              # one norm's bias or one norm alone
     assert "hiprwkv_rwkv7_ln_shiftmix" not in stub.calls
+
+
+@pytest.mark.parametrize("T", [3, 20])
+@pytest.mark.parametrize("name", ["ln0", "ln1"])
+def test_norms_anywhere_in_memory(monkeypatch, T, name):
+    """A norm's parameter that does not lie on a 16-byte boundary (a slice of one flat array) is copied for the kernels."""
+    from jaxrwkv_amd import blocks7
+    stub_library.install(monkeypatch)
+    monkeypatch.setattr(blocks7, "covers", lambda *a: False)
+    params = model(torch.float32)
+    tree = params if name == "ln0" else params["blocks"]
+    w = tree[name]["weight"]
+    tree[name]["weight"] = torch.cat([torch.zeros(1), w.flatten()])[1:].view(w.shape)
+    from jaxrwkv_amd import ops
+    seen = []
+    fwd = ops._ln_shiftmix_fwd
+    monkeypatch.setattr(ops, "_ln_shiftmix_fwd", lambda *a: seen.append(a[2].data_ptr() % 16 + a[3].data_ptr() % 16) or fwd(*a))
+    with torch.no_grad():
+        call(params, T)
+    assert seen and not any(seen)
