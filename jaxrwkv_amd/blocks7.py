@@ -327,11 +327,25 @@ def _run(x, state, ns, length, params, keep):
     return x, dx, new_state, saved, v_first
 
 
+_FACTORS = ("w1", "w2", "a1", "a2", "v1", "v2", "g1", "g2")
+_PRODUCTS = ("receptance", "key", "value", "output", "ffn_key", "ffn_value")       # torch looks at these itself
+
+
 def covers(params, x, state):
-    """Whether the operator takes the call: one dtype throughout and contiguous stacked parameters."""
-    io = x.dtype
-    return (io in ops._DT and state.dtype == io and x.shape[-1] <= ops.LN_SHIFTMIX_MAX_C
-            and all(t.dtype == io and t.is_contiguous() and t.is_cuda for t in params))
+    """Whether the operator takes the call: one dtype and device throughout, stacked parameters of the sizes that the kernels
+    read, contiguous and on 16-byte boundaries."""
+    io, dev, C = x.dtype, x.device, x.shape[-1]
+    n = params[0].shape[0] * C
+    if not (io in ops._DT and x.is_cuda and state.dtype == io and state.device == dev and C <= ops.LN_SHIFTMIX_MAX_C):
+        return False
+    for name, t in zip(NAMES, params):
+        if t.dtype != io or t.device != dev or not t.is_contiguous() or t.data_ptr() % 16:
+            return False
+        if name not in _PRODUCTS and name not in _FACTORS and t.numel() != n:
+            return False
+    p = dict(zip(NAMES, params))
+    return all(p[f + "1"].shape[-2] == C and p[f + "2"].shape[-2:] == (p[f + "1"].shape[-1], C)
+               and p[f + "1"].numel() == p[f + "2"].numel() == n * p[f + "1"].shape[-1] for f in "wavg")
 
 
 def run(params, x, state, ns, length, grad):

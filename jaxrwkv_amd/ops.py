@@ -852,6 +852,8 @@ def rwkv7_ln_shiftmix(x, dx, ln, prev, new_starts, length, mix, eps=1e-5, shift_
     io = x.dtype
     B, T, C = x.shape
     assert len(mix) in (0, 1, 6) and C % 8 == 0 and C <= LN_SHIFTMIX_MAX_C, (len(mix), C)
+    assert dx is None or dx.shape == x.shape, (dx.shape, x.shape)
+    length, new_starts = _length_ns(length, new_starts, B, T, x.device)
     x = _dev(x, io)
     dx = None if dx is None else _dev(dx, io)
     ln_w, ln_b = (_aligned(_dev(ln[n].reshape(C), io)) for n in ("weight", "bias"))
@@ -918,6 +920,7 @@ def rwkv7_pre(xw, k, xa, v, v_first, xv, w0, a0, v0, k_k, k_a):
     b_i), the WKV op's inputs.  The first layer has no value residual: ``v_first``, ``xv``, ``v0`` None, and v' is ``v``."""
     io = k.dtype
     C = k.shape[-2] * k.shape[-1]
+    assert all(t is None or t.shape == k.shape for t in (xw, xa, v, v_first, xv)), [t if t is None else t.shape for t in (xw, k, xa, v, v_first, xv)]
     xw, k, xa, v = (_dev(t, io) for t in (xw, k, xa, v))
     w0, a0, k_k, k_a = (_dev(t.reshape(C), io) for t in (w0, a0, k_k, k_a))
     if v_first is None:

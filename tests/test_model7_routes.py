@@ -296,3 +296,46 @@ def test_norms_anywhere_in_memory(monkeypatch, T, name):
     with torch.no_grad():
         call(params, T)
     assert seen and not any(seen)
+
+
+def _flat(w):
+    return torch.cat([torch.zeros(1, dtype=w.dtype), w.flatten()])[1:].view(w.shape)
+
+
+BAD = {"a vector of another size": ("x_k", lambda w: w[:, :32].contiguous()), "a factor of another size": ("w1", lambda w: w[:, :32].contiguous()),
+       "a second factor of another size": ("g2", lambda w: w[:, :, :32].contiguous()),
+       "one layer less": ("a0", lambda w: w[:1].contiguous()), "off a 16-byte boundary": ("v1", _flat),
+       "on another device": ("k_a", lambda w: w.to("meta"))}
+
+
+@pytest.mark.parametrize("bad", list(BAD))
+def test_the_stack_operator_takes_what_its_kernels_can_read(monkeypatch, bad):
+    from jaxrwkv_amd import blocks7
+    stub_library.install(monkeypatch)
+    params = model(torch.bfloat16)
+    x, state = torch.zeros((2, 20, C), dtype=torch.bfloat16), torch.zeros((2, L, 66, C), dtype=torch.bfloat16)
+    assert blocks7.covers(blocks7.gather(params["blocks"]), x, state)
+    name, change = BAD[bad]
+    params["blocks"]["att"][name] = change(params["blocks"]["att"][name])
+    assert not blocks7.covers(blocks7.gather(params["blocks"]), x, state)
+    if bad == "off a 16-byte boundary":                         # torch's products take it
+        with torch.no_grad():
+            assert not call(params, 20)[1].isnan().any()
+
+
+def test_fused_steps_look_at_their_operands(monkeypatch):
+    from jaxrwkv_amd import ops
+    stub_library.install(monkeypatch)
+    n = lambda *s: torch.zeros(s)
+    ln = {"weight": n(C), "bias": n(C)}
+    head = lambda dx=n(2, 20, C), ns=None, length=None: ops.rwkv7_ln_shiftmix(n(2, 20, C), dx, ln, n(2, C), ns, length, [n(C)])
+    head(ns=torch.zeros(20, dtype=torch.bool), length=3)        # broadcast over the batch as in the other operators
+    for kw in (dict(dx=n(2, 19, C)), dict(ns=torch.zeros((2, 19), dtype=torch.bool)), dict(length=torch.ones(3))):
+        with pytest.raises(AssertionError):
+            head(**kw)
+    tok, par = (n(2, 20, 1, 64) for _ in range(6)), [n(64) for _ in range(5)]
+    tok = list(tok)
+    ops.rwkv7_pre(*tok, *par)
+    for i in range(6):
+        with pytest.raises(AssertionError):
+            ops.rwkv7_pre(*tok[:i], n(2, 19, 1, 64), *tok[i + 1:], *par)
