@@ -853,12 +853,13 @@ def rwkv7_ln_shiftmix(x, dx, ln, prev, new_starts, length, mix, eps=1e-5, shift_
     B, T, C = x.shape
     assert len(mix) in (0, 1, 6) and C % 8 == 0 and C <= LN_SHIFTMIX_MAX_C, (len(mix), C)
     assert dx is None or dx.shape == x.shape, (dx.shape, x.shape)
-    length, new_starts = _length_ns(length, new_starts, B, T, x.device)
     x = _dev(x, io)
     dx = None if dx is None else _dev(dx, io)
     ln_w, ln_b = (_aligned(_dev(ln[n].reshape(C), io)) for n in ("weight", "bias"))
     mix2 = [_dev(m.reshape(C), io) for m in mix]
-    if _needs_grad(x, dx, ln_w, ln_b, prev, *mix2):
+    grad = _needs_grad(x, dx, ln_w, ln_b, prev, *mix2)
+    length, new_starts = _length_ns(length, new_starts, B, T, x.device, keep=grad)
+    if grad:
         if shift_out is not None:
             raise ValueError("rwkv7_ln_shiftmix: shift_out is for calls without autograd")
         xs, shift, *outs = _LnShiftMix.apply(x, dx, ln_w, ln_b, prev, new_starts, length, eps, *mix2)

@@ -339,3 +339,14 @@ def test_fused_steps_look_at_their_operands(monkeypatch):
     for i in range(6):
         with pytest.raises(AssertionError):
             ops.rwkv7_pre(*tok[:i], n(2, 19, 1, 64), *tok[i + 1:], *par)
+
+
+@pytest.mark.parametrize("T", [3, 20])
+def test_the_caller_may_reuse_length_before_the_backward(monkeypatch, T):
+    stub_library.install(monkeypatch)
+    params = model(torch.float32)
+    frozen(params, KEEP["blocks"])
+    length = torch.tensor([1, 2], dtype=torch.int32)
+    logits, new_state = call(params, T, length=length)
+    length.fill_(0)
+    (logits.sum() + new_state.sum()).backward()
