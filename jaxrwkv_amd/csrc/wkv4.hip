@@ -383,7 +383,8 @@ struct Seg4 {
 
 // The chain back through the tokens is affine in the cotangent (g_aa, g_bb, g_pp) of the state after a part: with the
 // states known, aa' = alpha g_aa + o1, bb' = alpha g_bb + o2, pp' = q1 g_aa + q2 g_bb + q3 g_pp + o3.  SUMMARY runs a part (all
-// but the first) from a zero cotangent, keeps those seven numbers (two float4 per channel and part) and stores nothing else;
+// but the first) from a zero cotangent, keeps those seven numbers and whether a reset cuts the chain (two float4 per channel and
+// part) and stores nothing else;
 // the full run then starts every part from the cotangent that the later parts' maps give.
 template <typename IO, bool GATED, bool SUMMARY>
 __global__ __launch_bounds__(W4_THREADS) void wkv4_bwd_kernel(Wkv4Args A) {
@@ -420,15 +421,16 @@ __global__ __launch_bounds__(W4_THREADS) void wkv4_bwd_kernel(Wkv4Args A) {
     inj_a = ld_f(gp); inj_b = ld_f(gp + A.C); inj_p = ld_f(gp + 2 * A.C);
   }
   float g_aa = 0.f, g_bb = 0.f, g_pp = 0.f, gw = 0.f, gu = 0.f;
-  float alpha = 1.f, q1 = 0.f, q2 = 0.f, q3 = 1.f;
+  float alpha = 1.f, q1 = 0.f, q2 = 0.f, q3 = 1.f, cut = 0.f;
   float4* const maps = reinterpret_cast<float4*>(A.maps) + (size_t)b * (A.nz - 1) * 2 * A.C + c;
   if (!SUMMARY) {
 #pragma unroll 4
     for (int64_t z = A.nz - 1; z > P.z; --z) {
       const float4 m = maps[(2 * (z - 1)) * A.C], o = maps[(2 * (z - 1) + 1) * A.C];
-      g_pp = fmaf(m.y, g_aa, fmaf(m.z, g_bb, fmaf(m.w, g_pp, o.z)));
-      g_aa = fmaf(m.x, g_aa, o.x);
-      g_bb = fmaf(m.x, g_bb, o.y);
+      const bool past = o.w != 0.f;        // a reset in the part: nothing from behind it, were it inf or NaN
+      g_pp = past ? o.z : fmaf(m.y, g_aa, fmaf(m.z, g_bb, fmaf(m.w, g_pp, o.z)));
+      g_aa = past ? o.x : fmaf(m.x, g_aa, o.x);
+      g_bb = past ? o.y : fmaf(m.x, g_bb, o.y);
     }
   }
 
@@ -522,7 +524,7 @@ __global__ __launch_bounds__(W4_THREADS) void wkv4_bwd_kernel(Wkv4Args A) {
           if (GATED) buf_st(grseq, go * rounded<IO>(An * rB), rgr, voff, soff);
         }
         const bool reset = (rmask >> x) & 1u;
-        if (SUMMARY && reset) alpha = q1 = q2 = q3 = 0.f;
+        if (SUMMARY && reset) { alpha = q1 = q2 = q3 = 0.f; cut = 1.f; }
         g_aa = reset ? 0.f : n_aa;
         g_bb = reset ? 0.f : n_bb;
         g_pp = reset ? 0.f : n_pp;
@@ -558,7 +560,7 @@ __global__ __launch_bounds__(W4_THREADS) void wkv4_bwd_kernel(Wkv4Args A) {
   }
   if (SUMMARY) {
     maps[(2 * (P.z - 1)) * A.C] = make_float4(alpha, q1, q2, q3);
-    maps[(2 * (P.z - 1) + 1) * A.C] = make_float4(g_aa, g_bb, g_pp, 0.f);
+    maps[(2 * (P.z - 1) + 1) * A.C] = make_float4(g_aa, g_bb, g_pp, cut);
     return;
   }
   const size_t row = (size_t)b * A.nz + P.z;

@@ -55,3 +55,26 @@ def test_inner_loop(B, T, C, p_reset, compat, dtype, monkeypatch):
     close("state", new_s[fine], ref_s[fine], *tol)
     for name, a, b in zip(("r", "k", "v", "w", "u", "s"), grads, want):
         close("g" + name, a, b, *((1e-4, 2e-5) if f32 else tol))
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_a_reset_keeps_a_cotangent_that_is_not_finite_behind_it(bad):
+    """Tokens before a reset do not depend on what comes after it, whatever its cotangent (one sequence of 64 channels: in parts
+    of 16 tokens): bit for bit the cotangents that a finite one gives."""
+    from jaxrwkv_amd.rwkv4 import HipRWKV
+    g = torch.Generator("cuda").manual_seed(4)
+    B, T, C, t0 = 1, 1000, 64, 605
+    n = lambda *s: torch.randn(s, device="cuda", generator=g)
+    s = torch.stack([n(B, C), n(B, C).abs() + 0.5, n(B, C)], 1)
+    args = [t.requires_grad_() for t in (n(B, T, C).sigmoid(), n(B, T, C), n(B, T, C), n(C), 0.5 * n(C), s)]
+    ns = torch.zeros((B, T), dtype=torch.bool, device="cuda")
+    ns[:, t0] = True
+    go = n(B, T, C)
+    _, out = HipRWKV.inner_loop(*args, None, ns)
+    want = torch.autograd.grad(out, args, go, retain_graph=True)
+    go[:, 900] = bad
+    got = torch.autograd.grad(out, args, go)
+    for i in (0, 1, 2):
+        assert torch.equal(got[i][:, :t0], want[i][:, :t0]) and torch.isfinite(got[i][:, :t0]).all()
+    assert torch.equal(got[5], want[5])
+    assert not torch.isfinite(got[2][:, t0:]).all()
