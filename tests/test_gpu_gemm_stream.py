@@ -35,3 +35,22 @@ def test_several_products_in_one_launch():
     for o, w in zip(outs, ws):
         want = x.double() @ w.double().T
         assert ((o.double() - want).abs() <= want.abs() * 2.0 ** -8 + 2.0 ** -14).all()
+
+
+@pytest.mark.parametrize("M,K", [(8, 64), (40, 64), (40, 72)])
+def test_tanh_of_small_values(M, K):
+    """The first low-rank factor of the decay starts at zero, so its hidden values start small: tanh keeps their relative precision.
+    x is one times a power of two in one place, so the sum is exact in bf16, and the result is tanh rounded once: 2^-8 of it.
+    The three shapes are the three kernels."""
+    from jaxrwkv_amd import blocks7
+    N = 64
+    g = torch.Generator("cuda").manual_seed(K)
+    x = torch.zeros((M, K), device="cuda")
+    x[:, 3] = 2.0 ** -torch.arange(M, device="cuda").float()
+    w = torch.zeros((K, N), device="cuda")
+    w[3] = torch.rand(N, device="cuda", generator=g) + 0.5
+    x, w = x.bfloat16(), w.bfloat16()
+    out = torch.empty((M, N), device="cuda", dtype=torch.bfloat16)
+    blocks7._gemm([(out, x, w, 0, 1, 1, None)])
+    want = torch.tanh((x.double() @ w.double()).bfloat16().double())
+    assert ((out.double() - want).abs() <= 2.0 ** -8 * want.abs()).all()
