@@ -443,8 +443,8 @@ class _Wkv4(torch.autograd.Function):
     @staticmethod
     def forward(ctx, w, u, k, v, r, s, length, new_starts, flags):
         io = k.dtype
-        k, v, s, w, u = (_dev(x, io) for x in (k, v, s, w, u))
-        r = None if r is None else _dev(r, io)
+        k, v, s, u = (_dev(x, io) for x in (k, v, s, u))
+        w, r = _aligned(_dev(w, io)), (None if r is None else _aligned(_dev(r, io)))
         new_s, y, ckpt = _wkv4_mix_fwd(w, u, k, v, r, s, length, new_starts, flags, True)
         ctx.flags = flags
         ctx.save_for_backward(w, u, k, v, r, s, length, new_starts, ckpt)
@@ -482,8 +482,8 @@ def _wkv4_apply(w, u, k, v, r, s, length, new_starts, flags):
     length, new_starts = _length_ns(length, new_starts, B, T, k.device, keep=grad)
     if grad:
         return _Wkv4.apply(w, u, k, v, r, s, length, new_starts, flags)
-    w, u, k, v, s = (_dev(x, k.dtype) for x in (w, u, k, v, s))
-    r = None if r is None else _dev(r, k.dtype)
+    u, k, v, s = (_dev(x, k.dtype) for x in (u, k, v, s))
+    w, r = _aligned(_dev(w, k.dtype)), (None if r is None else _aligned(_dev(r, k.dtype)))
     return _wkv4_mix_fwd(w, u, k, v, r, s, length, new_starts, flags, False)[:2]
 
 

@@ -1,5 +1,5 @@
 """The Python side of the operators on CPU tensors: the library's entry points are replaced by a stub that looks at every tensor
-handed to it (its type against the I/O type named in the call) and fills what the call would write.
+handed to it (its type against the I/O type named in the call, its alignment) and fills what the call would write.
 
 New memory is NaN until a stub fills it, so that a result nobody wrote shows.  The values mean nothing; what is checked are the
 routes, the operands' types and the graph."""
@@ -37,6 +37,7 @@ class Library:
             self.calls.append(name)
             fill([t for _, t in _tensors(args)])
             for i, t in _tensors(args):
+                assert t.data_ptr() % 16 == 0 or not t.is_floating_point(), (name, i + 2)
                 if t.is_floating_point() and i + 2 not in OTHER.get(name, ()):
                     assert t.dtype == IO[io], (name, i + 2, t.dtype, IO[io])
             return 0

@@ -1,0 +1,28 @@
+"""What the operators hand to the library, on the CPU with the library stubbed out."""
+import pytest
+import torch
+
+from tests import stub_library
+
+
+def off(t):
+    """The same values one element past a 16-byte boundary."""
+    return torch.cat([torch.zeros(1, dtype=t.dtype), t.flatten()])[1:].view(t.shape)
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_wkv4_receptance_and_decay_anywhere_in_memory(monkeypatch, dtype, grad):
+    from jaxrwkv_amd.rwkv4 import HipRWKV
+    stub_library.install(monkeypatch)
+    B, T, C = 2, 5, 64
+    n = lambda *s: torch.randn(s).to(dtype)
+    r, w = off(n(B, T, C)), off(n(C))
+    if grad:
+        w.requires_grad_()
+    assert r.data_ptr() % 16 and w.data_ptr() % 16
+    new_s, out = HipRWKV.inner_loop(r, n(B, T, C), n(B, T, C), w, n(C), n(B, 3, C), None, None)
+    assert not out.isnan().any()
+    if grad:
+        out.float().sum().backward()
+        assert w.grad is not None
