@@ -291,7 +291,7 @@ class _Blocks(torch.autograd.Function):
         io = like.dtype
         g_x = torch.zeros_like(like) if g_x is None else ops._dev(g_x, io)
         g_dx = torch.zeros_like(like) if g_dx is None else ops._dev(g_dx, io)
-        g_state = None if g_state is None else g_state.to(io)
+        g_state = None if g_state is None else ops._aligned(g_state.to(io))
         grads = [torch.empty_like(t) for t in params]
         for t, n in zip(grads, NAMES):
             if n in ("v0", "v1", "v2"):

@@ -210,7 +210,7 @@ def wkv7_bwd(r, w, k, v, a, b, s, length, new_starts, gy, sa, gs_out=None, compa
     r, w, k, v, a, b, gy = (_dev(x, io) for x in (r, w, k, v, a, b, gy))
     s = _dev(s)
     sa = _dev(sa, _SA_DT[io])
-    gs_out = None if gs_out is None else _dev(gs_out, s.dtype)
+    gs_out = None if gs_out is None else _aligned(_dev(gs_out, s.dtype))
     B, T, H, N = r.shape
     length, new_starts = _length_ns(length, new_starts, B, T, r.device)
     gw, gr, gk, gv, ga, gb = (_empty_like_phased(r, i) for i in range(1, 7))
@@ -457,7 +457,7 @@ class _Wkv4(torch.autograd.Function):
         lib = _lib.load()
         io = k.dtype
         B, T, C = k.shape
-        gy = torch.zeros_like(k) if gy is None else _dev(gy, io)
+        gy = torch.zeros_like(k) if gy is None else _aligned(_dev(gy, io))
         gs_new = None if gs_new is None else _dev(gs_new, io)
         gk, gv, gs = torch.empty_like(k), torch.empty_like(v), torch.empty_like(s)
         gr = None if r is None else torch.empty_like(r)
@@ -828,8 +828,8 @@ class _LnShiftMix(torch.autograd.Function):
         io = xs.dtype
         B, T, C = xs.shape
         n_out = len(mix)
-        gs = [torch.zeros_like(xs) if g is None else _dev(g, io) for g in gs]
-        gx, gshift = (None if g is None else _dev(g, io) for g in (gx, gshift))
+        gs = [torch.zeros_like(xs) if g is None else _aligned(_dev(g, io)) for g in gs]
+        gx, gshift = (None if g is None else _aligned(_dev(g, io)) for g in (gx, gshift))
         dxs = torch.empty_like(xs)
         dprev = torch.empty((B, C), dtype=io, device=xs.device) if ctx.need_prev else None
         dparam = torch.empty((n_out + 2, C), dtype=io, device=xs.device).unbind(0)

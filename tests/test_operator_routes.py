@@ -26,3 +26,23 @@ def test_wkv4_receptance_and_decay_anywhere_in_memory(monkeypatch, dtype, grad):
     if grad:
         out.float().sum().backward()
         assert w.grad is not None
+
+
+def test_wkv4_cotangent_anywhere_in_memory(monkeypatch):
+    """The output's cotangent is the caller's own: with the receptance inside the op no product of torch's comes before it."""
+    from jaxrwkv_amd.rwkv4 import HipRWKV
+    stub_library.install(monkeypatch)
+    n = lambda *s: torch.randn(s)
+    w = n(64).requires_grad_()
+    _, out = HipRWKV.inner_loop(n(2, 5, 64), n(2, 5, 64), n(2, 5, 64), w, n(64), n(2, 3, 64), None, None)
+    torch.autograd.grad(out, w, off(n(2, 5, 64)))
+
+
+@pytest.mark.parametrize("T", [3, 20])
+def test_model_state_cotangent_anywhere_in_memory(monkeypatch, T):
+    from tests.test_model7_routes import L, C, call, leaves, model
+    stub_library.install(monkeypatch)
+    params = model(torch.float32)
+    ps = [p.requires_grad_() for _, p in leaves(params["blocks"])]
+    _, new_state = call(params, T, B=1)
+    torch.autograd.grad(new_state, ps, off(torch.randn(1, L, 66, C)), allow_unused=True)
