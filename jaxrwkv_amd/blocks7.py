@@ -74,24 +74,31 @@ def _lora_fwd(p, mix, names, like):
     return hid, out
 
 
+def _weight_grad(grad, name, a, b):
+    if name in grad:
+        torch.mm(a.T, b, out=grad[name])
+
+
 def _lora_bwd(p, grad, mix, hid, gout, dmix, names):
-    """From the cotangents ``gout`` of the low-rank terms: the parameters' cotangents into ``grad`` and the inputs' into
-    ``dmix`` (the value residual's is added to what is there)."""
+    """From the cotangents ``gout`` of the low-rank terms: the parameters' cotangents into ``grad`` (those it has) and the
+    inputs' into ``dmix`` (the value residual's is added to what is there)."""
     if _grouped(p, gout["w"]):
-        dh = {n: torch.empty_like(hid[n]) for n, _ in names}
+        dh = {n: gout[n].new_empty((gout[n].shape[0], p[n + "1"].shape[-1])) for n, _ in names}
         _gemm([(dh[n], gout[n], p[n + "2"], 0, 0, act, hid[n] if act else None) for n, act in names])
         _gemm([(dmix[n], dh[n], p[n + "1"], 0, 0, 0, dmix[n] if n == "v" else None) for n, _ in names])
-        _gemm([(grad[n + "1"], mix[n], dh[n], 1, 1, _NONE, None) for n, _ in names]
-              + [(grad[n + "2"], hid[n], gout[n], 1, 1, _NONE, None) for n, _ in names])
+        jobs = ([(grad[n + "1"], mix[n], dh[n], 1, 1, _NONE, None) for n, _ in names if n + "1" in grad]
+                + [(grad[n + "2"], hid[n], gout[n], 1, 1, _NONE, None) for n, _ in names if n + "2" in grad])
+        if jobs:
+            _gemm(jobs)
         return
     for n, act in names:
-        torch.mm(hid[n].T, gout[n], out=grad[n + "2"])
+        _weight_grad(grad, n + "2", hid[n], gout[n])
         dh = gout[n] @ p[n + "2"].T
         if act == _TANH:
             dh = torch.ops.aten.tanh_backward(dh, hid[n])
         elif act == _SIGMOID:
             dh = torch.ops.aten.sigmoid_backward(dh, hid[n])
-        torch.mm(mix[n].T, dh, out=grad[n + "1"])
+        _weight_grad(grad, n + "1", mix[n], dh)
         if n == "v":
             dmix[n].addmm_(dh, p[n + "1"].T)
         else:
@@ -108,9 +115,10 @@ def _ln_mix(p, x, dx, ln, state_row, ns, length, mix, shift_out, keep):
     return xs, outs, (stats, prev, stride)
 
 
-def _layer_fwd(i, p, x, dx, st, nst, v_first, ns, length, keep):
+def _layer_fwd(i, p, x, dx, st, nst, v_first, ns, length, need):
     """One block on x (B,T,C) (+ dx): returns (x, dx, v_first, saved tensors).  st, nst: the layer's rows of the model
-    states."""
+    states.  need: None without a backward to come, else the names of the parameters whose cotangents it will make."""
+    keep = need is not None
     B, T, C = x.shape
     H, N = p["r_k"].shape
     M = B * T
@@ -140,12 +148,22 @@ def _layer_fwd(i, p, x, dx, st, nst, v_first, ns, length, keep):
     dx2 = torch.mm(fr, p["ffn_value"].T).view(B, T, C)
     saved = None
     if keep:
-        saved = dict(x=x, head1=head1, xr=xr, xk=xk, mix=mix, r=r, k=k, v=v, hid=hid, lora=lora, w=w, k2=k2, v2=v2, a=a, b=b,
-                     s=s, sa=sa, yw=yw, y=y, x2=x2, head2=head2, xk2=xk2, ff=ff, fr=fr)
+        # an operand of a weight's cotangent alone is kept for that weight only
+        only = lambda t, *names: t if need.intersection(names) else None
+        saved = dict(x=x, head1=head1, xr=only(xr, "receptance"), xk=only(xk, "key"),
+                     mix={n: only(t, n + "1", *(("value",) if n == "v" else ())) for n, t in mix.items()},
+                     r=r, k=k, v=v, hid={n: hid[n] if act else only(hid[n], n + "2") for n, act in _LORA if n in hid}, lora=lora,
+                     w=w, k2=k2, v2=v2, a=a, b=b, s=s, sa=sa, yw=yw, y=only(y, "output"), x2=x2, head2=head2,
+                     xk2=only(flat(xk2), "ffn_key"), ff=ff, fr=only(fr, "ffn_value"))
     return x2, dx2, v_first, saved
 
 
-def _ln_mix_bwd(p, grad, xs, head, ln, ns, length, mix, gs, gx, gshift, need_prev):
+def _vectors(grad, names, scratch):
+    """The places for the cotangents of parameters that a kernel makes together: ``scratch`` for those nobody asked for."""
+    return ops._ptr_array([grad.get(n, scratch) for n in names])
+
+
+def _ln_mix_bwd(p, grad, scratch, xs, head, ln, ns, length, mix, gs, gx, gshift, need_prev):
     lib = _lib.load()
     stats, prev, stride = head
     io = xs.dtype
@@ -158,14 +176,14 @@ def _ln_mix_bwd(p, grad, xs, head, ln, ns, length, mix, gs, gx, gshift, need_pre
     rc = lib.hiprwkv_rwkv7_ln_shiftmix_bwd(
         ops._stream(), ops._DT[io], B, T, C, len(mix), ops._p(xs), ops._p(stats), ops._p(p[ln + "_w"]), ops._p(p[ln + "_b"]),
         ops._p(prev), stride, ops._p(ns), ops._p(length), ops._ptr_array(params), ops._ptr_array(gs), ops._p(gx), ops._p(gshift),
-        ops._p(dxs), ops._p(dprev), ops._ptr_array([grad[n] for n in mix] + [grad[ln + "_w"], grad[ln + "_b"]]), ops._p(ws), nbytes)
+        ops._p(dxs), ops._p(dprev), _vectors(grad, (*mix, ln + "_w", ln + "_b"), scratch), ops._p(ws), nbytes)
     _lib.check(rc, "hiprwkv_rwkv7_ln_shiftmix_bwd")
     return dxs, dprev
 
 
-def _layer_bwd(i, p, grad, S, ns, length, g_x, g_dx, g_state, g_in, g_vfirst, v_first):
+def _layer_bwd(i, p, grad, scratch, S, ns, length, g_x, g_dx, g_state, g_in, g_vfirst, v_first):
     """The cotangents of one block: g_x, g_dx of what it returns, g_state (or None) of its rows of the new model state (B,66,C).
-    Fills ``grad`` (the layer's slices of the stacked cotangents) and ``g_in`` (or None), the cotangent of its rows of the input
+    Fills ``grad`` (the layer's slices of the stacked cotangents, of those asked for; scratch: C elements) and ``g_in`` (or None), the cotangent of its rows of the input
     state; accumulates ``g_vfirst``.  Returns the cotangent of its input x (and of the dx added to it) and g_vfirst."""
     lib = _lib.load()
     x, x2 = S["x"], S["x2"]
@@ -178,19 +196,19 @@ def _layer_bwd(i, p, grad, S, ns, length, g_x, g_dx, g_state, g_in, g_vfirst, v_
     row = lambda j: None if g_state is None else g_state[:, j].contiguous()
     # channel mixing
     g2 = flat(g_dx)
-    torch.mm(g2.T, S["fr"], out=grad["ffn_value"])
+    _weight_grad(grad, "ffn_value", g2, S["fr"])
     gf = torch.mm(g2, p["ffn_value"])
     gff = torch.empty_like(gf)
     _lib.check(lib.hiprwkv_rwkv7_relusq_bwd(ops._stream(), ops._DT[io], gf.numel(), ops._p(S["ff"]), ops._p(gf), ops._p(gff)),
                "hiprwkv_rwkv7_relusq_bwd")
-    torch.mm(gff.T, flat(S["xk2"]), out=grad["ffn_key"])
+    _weight_grad(grad, "ffn_key", gff, S["xk2"])
     gxk2 = torch.mm(gff, p["ffn_key"]).view(B, T, C)
-    dx2, dprev = _ln_mix_bwd(p, grad, x2, S["head2"], "ln2", ns, length, ("ffn_x_k",), [gxk2], g_x, row(0), g_in is not None)
+    dx2, dprev = _ln_mix_bwd(p, grad, scratch, x2, S["head2"], "ln2", ns, length, ("ffn_x_k",), [gxk2], g_x, row(0), g_in is not None)
     if g_in is not None:
         g_in[:, 0] = dprev
     # time mixing: output projection, group norm and gate
     g1 = flat(dx2)
-    torch.mm(g1.T, S["y"], out=grad["output"])
+    _weight_grad(grad, "output", g1, S["y"])
     gy = torch.mm(g1, p["output"])
     e = lambda: torch.empty((B, T, H, N), dtype=io, device=x.device)
     gyw, gr1, gk1, gv1, gg = (e() for _ in range(5))
@@ -200,7 +218,7 @@ def _layer_bwd(i, p, grad, S, ns, length, g_x, g_dx, g_state, g_in, g_vfirst, v_
         ops._stream(), ops._DT[io], M, H, N, ops._p(S["yw"]), ops._p(S["r"]), ops._p(S["k2"]), ops._p(S["v2"]),
         ops._p(S["lora"]["g"]), ops._p(p["lnx_w"]), ops._p(p["lnx_b"]), ops._p(p["r_k"]), EPS_X, ops._p(gy), ops._p(gyw),
         ops._p(gr1), ops._p(gk1), ops._p(gv1), ops._p(gg),
-        ops._ptr_array([grad["lnx_w"], grad["lnx_b"], grad["r_k"]]), ops._p(ws), nbytes)
+        _vectors(grad, ("lnx_w", "lnx_b", "r_k"), scratch), ops._p(ws), nbytes)
     _lib.check(rc, "hiprwkv_rwkv7_postmix_bwd2")
     # the recurrence
     gs_out = None if g_state is None else g_state[:, 2:].reshape(B, H, N, N)
@@ -226,7 +244,7 @@ def _layer_bwd(i, p, grad, S, ns, length, g_x, g_dx, g_state, g_in, g_vfirst, v_
         P(lora["v"]) if i else None, P(par("w0")), P(par("a0")), P(par("v0")) if i else None, P(par("k_k")), P(par("k_a")),
         P(gw), P(gk1), P(gv1) if i else None, P(ga), P(gb), P(gk2), P(gv2) if i else None, P(gr1), P(gr2), P(gr),
         P(dxw), P(dk), P(dv) if i else None, P(dvf), P(dxv), P(dxa),
-        ops._ptr_array([grad[n] for n in ("w0", "a0", "k_k", "k_a", "v0")]), P(ws), nbytes)
+        _vectors(grad, ("w0", "a0", "k_k", "k_a", "v0"), scratch), P(ws), nbytes)
     _lib.check(rc, "hiprwkv_rwkv7_pre_bwd")
     if i:
         g_vfirst = dvf if g_vfirst is None else g_vfirst.add_(dvf)
@@ -234,7 +252,7 @@ def _layer_bwd(i, p, grad, S, ns, length, g_x, g_dx, g_state, g_in, g_vfirst, v_
     gr, dk, dv = flat(gr), flat(dk), flat(dv)
     mix = S["mix"]
     for g, a, n in ((gr, S["xr"], "receptance"), (dk, S["xk"], "key"), (dv, mix["v"], "value")):
-        torch.mm(g.T, a, out=grad[n])
+        _weight_grad(grad, n, g, a)
     dxr, dxk, dxv_ = torch.mm(gr, p["receptance"]), torch.mm(dk, p["key"]), torch.mm(dv, p["value"])
     dmix = {n: torch.empty_like(dxr) for n in ("w", "a", "g")}
     dmix["v"] = dxv_
@@ -243,7 +261,7 @@ def _layer_bwd(i, p, grad, S, ns, length, g_x, g_dx, g_state, g_in, g_vfirst, v_
         gout["v"] = flat(dxv)
     _lora_bwd(p, grad, mix, S["hid"], gout, dmix, names)
     gmix = [t.view(B, T, C) for t in (dxr, dmix["w"], dxk, dxv_, dmix["a"], dmix["g"])]
-    dx, dprev = _ln_mix_bwd(p, grad, x, S["head1"], "ln1", ns, length, MIX, gmix, dx2, row(1), g_in is not None)
+    dx, dprev = _ln_mix_bwd(p, grad, scratch, x, S["head1"], "ln1", ns, length, MIX, gmix, dx2, row(1), g_in is not None)
     if g_in is not None:
         g_in[:, 1] = dprev
     return dx, g_vfirst
@@ -273,7 +291,8 @@ class _Blocks(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, state, ns, length, *params):
         ctx.set_materialize_grads(False)
-        x, dx, new_state, saved, v_first = _run(x, state, ns, length, params, True)
+        need = {n for n, asked in zip(NAMES, ctx.needs_input_grad[4:]) if asked}
+        x, dx, new_state, saved, v_first = _run(x, state, ns, length, params, need)
         tensors = []
         ctx.places = _pack([saved, v_first, ns, length], tensors)
         ctx.n = len(tensors)
@@ -292,36 +311,34 @@ class _Blocks(torch.autograd.Function):
         g_x = torch.zeros_like(like) if g_x is None else ops._dev(g_x, io)
         g_dx = torch.zeros_like(like) if g_dx is None else ops._dev(g_dx, io)
         g_state = None if g_state is None else ops._aligned(g_state.to(io))
-        grads = [torch.empty_like(t) for t in params]
-        for t, n in zip(grads, NAMES):
-            if n in ("v0", "v1", "v2"):
-                t[0].zero_()                    # the first layer has no value residual
+        grads = {n: torch.empty_like(t) for n, t, asked in zip(NAMES, params, ctx.needs_input_grad[4:]) if asked}
+        for n in ("v0", "v1", "v2"):
+            if n in grads:
+                grads[n][0].zero_()             # the first layer has no value residual
+        scratch = torch.empty(like.shape[-1], dtype=io, device=like.device)
         g_in = torch.empty_like(state) if ctx.needs_input_grad[1] else None
         g_vfirst = None
         layers = list(zip(*(t.unbind(0) for t in params)))
-        glayers = list(zip(*(t.unbind(0) for t in grads)))
         # products in the operands' own dtype even where the caller's backward runs under autocast
         with torch.autocast(like.device.type, enabled=False):
             for i in reversed(range(L)):
-                dx, g_vfirst = _layer_bwd(i, dict(zip(NAMES, layers[i])), dict(zip(NAMES, glayers[i])), saved[i], ns,
-                                          length, g_x, g_dx, None if g_state is None else g_state[:, i],
+                dx, g_vfirst = _layer_bwd(i, dict(zip(NAMES, layers[i])), {n: t[i] for n, t in grads.items()}, scratch, saved[i],
+                                          ns, length, g_x, g_dx, None if g_state is None else g_state[:, i],
                                           None if g_in is None else g_in[:, i], g_vfirst, v_first)
                 g_x = g_dx = dx
-        need = ctx.needs_input_grad[4:]
-        return (g_x, g_in, None, None) + tuple(g if n else None for g, n in zip(grads, need))
+        return (g_x, g_in, None, None) + tuple(grads.get(n) for n in NAMES)
 
 
-def _run(x, state, ns, length, params, keep):
+def _run(x, state, ns, length, params, need):
     L = params[0].shape[0]
     layers = list(zip(*(t.unbind(0) for t in params)))
     new_state = torch.empty_like(state, memory_format=torch.contiguous_format)      # the kernels write rows of neighbours
     dx = v_first = None
-    saved = [] if keep else None
+    saved = []
     for i in range(L):
         x, dx, v_first, S = _layer_fwd(i, dict(zip(NAMES, layers[i])), x, dx, state[:, i], new_state[:, i], v_first, ns,
-                                       length, keep)
-        if keep:
-            saved.append(S)
+                                       length, need)
+        saved.append(S)
     if not state.is_contiguous():
         new_state = torch.empty_like(state).copy_(new_state)                          # in the order of the caller's
     return x, dx, new_state, saved, v_first
@@ -353,4 +370,4 @@ def run(params, x, state, ns, length, grad):
     if grad:
         length = None if length is None else length.clone()          # the caller may change its own before the backward
         return _Blocks.apply(x, state, ns, length, *params)
-    return _run(x, state, ns, length, params, False)[:3]
+    return _run(x, state, ns, length, params, None)[:3]

@@ -70,6 +70,8 @@ def install(monkeypatch):
 
     monkeypatch.setattr(torch, "empty", lambda *a, **k: nan(empty(*a, **k)))
     monkeypatch.setattr(torch, "empty_like", lambda *a, **k: nan(empty_like(*a, **k)))
+    new_empty = torch.Tensor.new_empty
+    monkeypatch.setattr(torch.Tensor, "new_empty", lambda *a, **k: nan(new_empty(*a, **k)))
     monkeypatch.setattr(torch.Tensor, "is_cuda", property(lambda t: True))
     monkeypatch.setattr(_lib, "load", lambda: stub)
     monkeypatch.setattr(ops, "_stream", lambda: 0)

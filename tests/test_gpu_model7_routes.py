@@ -140,3 +140,26 @@ def test_wide_models(T, grad, monkeypatch):
     monkeypatch.setattr(ops, "LN_SHIFTMIX_MAX_C", 64)
     for i, (a, b) in enumerate(zip(run(), want)):
         assert rel(a, b) < 2e-4, (i, tuple(a.shape), rel(a, b))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("keep", [(), ("att.x_a", "att.v0"), ("ffn.key.weight",), ("att.w1", "att.g2", "att.ln_x.bias", "ln1.weight")])
+def test_frozen_parameters_of_the_stack(keep, dtype):
+    """Whatever of the blocks is frozen, the other cotangents and the state's are those of a full training step, bit for bit."""
+    from jaxrwkv_amd.model7 import RWKV7
+    tok, state = inputs(3, 45, dtype)
+    g = torch.Generator("cuda").manual_seed(2)
+    cot = [torch.randn(s, device="cuda", generator=g).to(dtype) for s in ((3, 45, V), state.shape)]
+
+    def run(trains):
+        params = model(dtype)
+        ps = {n: p.requires_grad_() for n, p in leaves(params) if trains(n)}
+        st = state.clone().requires_grad_()
+        outs = RWKV7.forward(params, tok, st)
+        return dict(zip(["state", *ps], torch.autograd.grad(outs, [st, *ps.values()], cot)))
+
+    full = run(lambda n: True)
+    part = run(lambda n: n.removeprefix("blocks.") in keep)
+    assert len(part) == 1 + len(keep)
+    for n, t in part.items():
+        assert torch.equal(t, full[n]), n

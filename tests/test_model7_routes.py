@@ -111,7 +111,7 @@ def test_no_derivative_no_graph(monkeypatch):
     run = blocks7._run
     monkeypatch.setattr(blocks7, "_run", lambda *a: kept.append(a[-1]) or run(*a))
     call(params, 20)
-    assert kept == [False]
+    assert kept == [None]
     native = []
     monkeypatch.setattr(ops, "rwkv7_decode", lambda *a: native.append(1) or ("logits", "state"))
     call(params, 1)
@@ -350,3 +350,42 @@ def test_the_caller_may_reuse_length_before_the_backward(monkeypatch, T):
     logits, new_state = call(params, T, length=length)
     length.fill_(0)
     (logits.sum() + new_state.sum()).backward()
+
+
+def _count_mm(monkeypatch):
+    from jaxrwkv_amd import blocks7
+    count, mm, gemm = [], torch.mm, blocks7._gemm
+    monkeypatch.setattr(torch, "mm", lambda *a, **k: count.append(1) or mm(*a, **k))
+    monkeypatch.setattr(blocks7, "_gemm", lambda jobs: count.extend(jobs) or gemm(jobs))
+    return count
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_nothing_is_made_for_frozen_parameters(monkeypatch, dtype):
+    """Products, cotangent arrays and saved activations follow what is trainable: the state alone, one vector, one matrix, all."""
+    stub_library.install(monkeypatch)
+    cost = {}
+    subsets = {"state": lambda n: False, "vector": lambda n: n == "blocks.att.x_a", "matrix": lambda n: n == "blocks.ffn.key.weight",
+               "all": lambda n: n.startswith("blocks")}
+    for what, keep in subsets.items():
+        with monkeypatch.context() as m:
+            params = model(dtype)
+            state = torch.zeros((2, L, 66, C), dtype=dtype).requires_grad_(what == "state")
+            trainable = frozen(params, keep)
+            saved = []
+            with torch.autograd.graph.saved_tensors_hooks(lambda t: saved.append(t.numel()) or t, lambda t: t):
+                logits, new_state = call(params, 20, state=state)
+            made, like = [], torch.empty_like
+            products = _count_mm(m)
+            m.setattr(torch, "empty_like", lambda t, **k: made.append(tuple(t.shape)) or like(t, **k))
+            ins = list(trainable.values()) or [state]
+            grads = torch.autograd.grad((logits, new_state), ins, (torch.ones_like(logits), torch.ones_like(new_state)))
+            assert not any(g.isnan().any() for g in grads)
+            stacked = {tuple(p.shape) for _, p in leaves(params["blocks"])}
+            cost[what] = (len(products), sum(saved), sum(s in stacked and len(s) == 3 for s in made))
+    lora = 4 * L - 1 if dtype == torch.bfloat16 else 0             # the low-rank products are torch's own in fp32 (@, not counted)
+    weights = 6 * L + 2 * lora
+    assert cost["state"][0] == cost["vector"][0] == cost["all"][0] - weights - (2 * (4 * L - 1) if dtype == torch.float32 else 0)
+    assert cost["matrix"][0] == cost["state"][0] + L
+    assert cost["state"][1] < cost["all"][1] and cost["matrix"][1] < cost["all"][1]
+    assert cost["state"][2] == cost["vector"][2] == 0 and cost["matrix"][2] <= 1
