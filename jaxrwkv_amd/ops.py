@@ -968,7 +968,8 @@ def rwkv7_decode(params, x, state, length, new_starts, compat=True):
     dims = [att[n].shape[-1] for n in ("w1", "a1", "v1", "g1")]
     if (T > 8 or B * T > DECODE_MAX_ROWS or N != 64 or C != H * N or C > LN_SHIFTMIX_MAX_C or vocab % 16
             or any(d % 32 for d in (F, *dims)) or not x.is_cuda or x.dtype != bf
-            or state.shape != (B, L, 2 + N, C) or state.dtype != bf or not state.is_contiguous() or state.data_ptr() % 16):
+            or state.shape != (B, L, 2 + N, C) or state.dtype != bf or state.device != x.device or not state.is_contiguous()
+            or state.data_ptr() % 16):
         return None
     A = _lib.Rwkv7DecodeArgs(B=B, T=T, L=L, C=C, H=H, F=F, vocab=vocab, d_decay=dims[0], d_aaa=dims[1], d_mv=dims[2],
                              d_gate=dims[3])

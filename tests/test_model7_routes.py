@@ -389,3 +389,16 @@ def test_nothing_is_made_for_frozen_parameters(monkeypatch, dtype):
     assert cost["matrix"][0] == cost["state"][0] + L
     assert cost["state"][1] < cost["all"][1] and cost["matrix"][1] < cost["all"][1]
     assert cost["state"][2] == cost["vector"][2] == 0 and cost["matrix"][2] <= 1
+
+
+def test_native_step_leaves_a_state_elsewhere_alone(monkeypatch):
+    """The native step takes the state by its pointer; a state on another device goes to the separate steps, which refuse it."""
+    from jaxrwkv_amd import ops
+    from jaxrwkv_amd.model7 import RWKV7
+    stub_library.install(monkeypatch)
+    params = model(torch.bfloat16)
+    x, state = torch.zeros(2, 1, C, dtype=torch.bfloat16), RWKV7.default_state(params, 2)
+    monkeypatch.setattr(ops, "_p", lambda t: None if t is None else t.data_ptr())
+    monkeypatch.setattr(ops.ctypes, "byref", lambda a: torch.zeros(1, dtype=torch.bfloat16))
+    assert ops.rwkv7_decode(params, x, state, None, None) is not None
+    assert ops.rwkv7_decode(params, x, state.to("meta"), None, None) is None
