@@ -238,14 +238,14 @@ class RWKV7:
         """tokens (B,T) int; state (B,L,2+N,C); length (B,) or None (= T); new_starts (B,T) bool or None.
         Returns (logits (B,T,vocab), new state).  llm.py:71-84 + rwkv7.py:269-291."""
         B, T = tokens.shape
-        dev = tokens.device
+        L, H, N = params["blocks"]["att"]["r_k"].shape
+        C = H * N
+        x = params["emb"]["weight"][tokens]
+        dev = x.device                              # the tokens themselves may lie in host memory
         if length is not None:
             length = torch.as_tensor(length, device=dev).to(torch.int32).reshape(-1).expand(B).contiguous()
         if new_starts is not None:
             new_starts = torch.as_tensor(new_starts, device=dev).to(torch.bool).expand(B, T).contiguous()
-        L, H, N = params["blocks"]["att"]["r_k"].shape
-        C = H * N
-        x = params["emb"]["weight"][tokens]
         # the separate steps carry forward-mode tangents where torch does; the recurrence refuses those that reach it
         fused = (cls.fuse_mix and C <= ops.LN_SHIFTMIX_MAX_C
                  and not ops.has_tangent(itertools.chain((x, state), _leaves(params))))

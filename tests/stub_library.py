@@ -47,7 +47,7 @@ class Library:
 def fill(tensors):
     with torch.no_grad():
         for t in tensors:
-            if t.is_floating_point() and t.isnan().any():
+            if t.is_floating_point() and not t.is_meta and t.isnan().any():
                 t.data.masked_fill_(t.isnan(), 0.01)
 
 

@@ -402,3 +402,21 @@ def test_native_step_leaves_a_state_elsewhere_alone(monkeypatch):
     monkeypatch.setattr(ops.ctypes, "byref", lambda a: torch.zeros(1, dtype=torch.bfloat16))
     assert ops.rwkv7_decode(params, x, state, None, None) is not None
     assert ops.rwkv7_decode(params, x, state.to("meta"), None, None) is None
+
+
+@pytest.mark.parametrize("T", [3, 20])
+def test_tokens_in_host_memory(monkeypatch, T):
+    """Tokens may index the embedding from the host; ``length`` and ``new_starts`` go to the kernels' device all the same."""
+    from jaxrwkv_amd import blocks7, ops
+    from jaxrwkv_amd.model7 import tree_map
+    stub_library.install(monkeypatch)
+    got = []
+
+    def route(*args):
+        got.append([a.device.type for a in args if torch.is_tensor(a)])
+        return (torch.zeros((2, T, C), dtype=torch.bfloat16, device="meta"),) * 3
+    monkeypatch.setattr(ops, "autocast_elsewhere", lambda x: False)          # knows no such device
+    monkeypatch.setattr(blocks7, "run", route)
+    monkeypatch.setattr(ops, "rwkv7_decode", route)
+    call(tree_map(lambda t: t.to("meta"), model(torch.bfloat16)), T, length=torch.tensor([2, 3]), new_starts=torch.zeros((2, T), dtype=torch.bool))
+    assert got == [["meta"] * 4]
