@@ -112,7 +112,7 @@ def _ln_mix(p, x, dx, ln, state_row, ns, length, mix, shift_out, keep):
     prev, stride = ops._shift_row(state_row, B, C, x.dtype)
     xs, outs = ops._ln_shiftmix_fwd(x, dx, p[ln + "_w"], p[ln + "_b"], 1e-5, prev, stride, ns, length,
                                     [p[n] for n in mix], shift_out, stats)
-    return xs, outs, (stats, prev, stride)
+    return xs, outs, (stats, prev)
 
 
 def _layer_fwd(i, p, x, dx, st, nst, v_first, ns, length, need):
@@ -165,9 +165,10 @@ def _vectors(grad, names, scratch):
 
 def _ln_mix_bwd(p, grad, scratch, xs, head, ln, ns, length, mix, gs, gx, gshift, need_prev):
     lib = _lib.load()
-    stats, prev, stride = head
+    stats, prev = head
     io = xs.dtype
     B, T, C = xs.shape
+    prev, stride = ops._shift_row(prev, B, C, io)             # a saved-tensor hook may have moved it
     dxs = torch.empty_like(xs)
     dprev = torch.empty((B, C), dtype=io, device=xs.device) if need_prev else None
     params = [p[n] for n in mix]

@@ -599,7 +599,7 @@ class _ShiftMix(torch.autograd.Function):
     def forward(ctx, x, prev, ns, *mix):
         prev_t, stride = _shift_row(prev, x.shape[0], x.shape[2], x.dtype)
         ctx.save_for_backward(x, prev_t, *mix)
-        ctx.ns, ctx.stride = ns, stride
+        ctx.ns = ns
         return _shiftmix_fwd(x, prev_t, stride, ns, mix)
 
     @staticmethod
@@ -608,11 +608,12 @@ class _ShiftMix(torch.autograd.Function):
         lib = _lib.load()
         io = x.dtype
         B, T, C = x.shape
+        prev, stride = _shift_row(prev, B, C, io)         # a saved-tensor hook may have moved it
         gs = [_dev(g, io) for g in gs]
         dx = torch.empty_like(x)
         dprev = torch.empty((B, C), dtype=io, device=x.device)
         dmix = torch.empty((len(mix), C), dtype=torch.float32, device=x.device)
-        rc = lib.hiprwkv_rwkv7_shiftmix_bwd(_stream(), _DT[io], B, T, C, len(mix), _p(x), _p(prev), ctx.stride,
+        rc = lib.hiprwkv_rwkv7_shiftmix_bwd(_stream(), _DT[io], B, T, C, len(mix), _p(x), _p(prev), stride,
                                             _p(ctx.ns), _ptr_array(mix), _ptr_array(gs), _p(dx), _p(dprev), C, _p(dmix))
         _lib.check(rc, "hiprwkv_rwkv7_shiftmix_bwd")
         return (dx, dprev, None) + tuple(dmix[i].to(io) for i in range(len(mix)))
@@ -817,7 +818,7 @@ class _LnShiftMix(torch.autograd.Function):
         shift = None if prev is None else torch.empty((B, C), dtype=x.dtype, device=x.device)
         xs, outs = _ln_shiftmix_fwd(x, dx, ln_w, ln_b, eps, prev_t, stride, ns, length, mix, shift, stats)
         ctx.save_for_backward(xs, stats, ln_w, ln_b, prev_t, ns, length, *mix)
-        ctx.stride, ctx.has_dx, ctx.need_prev = stride, dx is not None, prev is not None and ctx.needs_input_grad[4]
+        ctx.has_dx, ctx.need_prev = dx is not None, prev is not None and ctx.needs_input_grad[4]
         ctx.set_materialize_grads(False)
         return (xs.view_as(xs) if dx is None else xs, shift) + tuple(outs)
 
@@ -828,6 +829,7 @@ class _LnShiftMix(torch.autograd.Function):
         io = xs.dtype
         B, T, C = xs.shape
         n_out = len(mix)
+        prev, stride = (None, C) if prev is None else _shift_row(prev, B, C, io)      # a saved-tensor hook may have moved it
         gs = [torch.zeros_like(xs) if g is None else _aligned(_dev(g, io)) for g in gs]
         gx, gshift = (None if g is None else _aligned(_dev(g, io)) for g in (gx, gshift))
         dxs = torch.empty_like(xs)
@@ -836,7 +838,7 @@ class _LnShiftMix(torch.autograd.Function):
         nbytes = lib.hiprwkv_rwkv7_ln_shiftmix_bwd_workspace_bytes(B, T, C, n_out)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=xs.device)
         rc = lib.hiprwkv_rwkv7_ln_shiftmix_bwd(_stream(), _DT[io], B, T, C, n_out, _p(xs), _p(stats), _p(ln_w), _p(ln_b),
-                                               _p(prev), ctx.stride, _p(ns), _p(length), _ptr_array(mix), _ptr_array(gs),
+                                               _p(prev), stride, _p(ns), _p(length), _ptr_array(mix), _ptr_array(gs),
                                                _p(gx), _p(gshift), _p(dxs), _p(dprev), _ptr_array(dparam), _p(ws), nbytes)
         _lib.check(rc, "hiprwkv_rwkv7_ln_shiftmix_bwd")
         return (dxs, dxs if ctx.has_dx else None, dparam[-2], dparam[-1], dprev, None, None, None) + tuple(dparam[:-2])

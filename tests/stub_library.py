@@ -14,6 +14,10 @@ OTHER = {
     "hiprwkv_rwkv7_shiftmix_bwd": {15},
 }
 
+#: position of the shift row, whose batch stride follows it
+SHIFT_ROW = {"hiprwkv_rwkv7_ln_shiftmix": 11, "hiprwkv_rwkv7_ln_shiftmix_bwd": 10, "hiprwkv_rwkv7_shiftmix": 7,
+             "hiprwkv_rwkv7_shiftmix_bwd": 7}
+
 
 def _tensors(args):
     for i, a in enumerate(args):
@@ -36,6 +40,9 @@ class Library:
         def call(stream, io, *args):
             self.calls.append(name)
             fill([t for _, t in _tensors(args)])
+            if name in SHIFT_ROW:
+                row, stride = args[SHIFT_ROW[name] - 2:][:2]
+                assert row is None or len(row) == 1 or row.stride(0) == stride, (name, row.stride(), stride)
             for i, t in _tensors(args):
                 assert t.data_ptr() % 16 == 0 or not t.is_floating_point(), (name, i + 2)
                 if t.is_floating_point() and i + 2 not in OTHER.get(name, ()):

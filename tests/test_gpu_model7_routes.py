@@ -163,3 +163,22 @@ def test_frozen_parameters_of_the_stack(keep, dtype):
     assert len(part) == 1 + len(keep)
     for n, t in part.items():
         assert torch.equal(t, full[n]), n
+
+
+def test_saved_tensors_kept_in_host_memory():
+    """Saved tensors that come back as dense copies give the same bits."""
+    from jaxrwkv_amd.model7 import RWKV7
+    tok, state = inputs(3, 45, torch.bfloat16)
+    params = model(torch.bfloat16)
+    ps = [p.requires_grad_() for _, p in leaves(params)]
+
+    def run():
+        outs = RWKV7.forward(params, tok, state)
+        return outs, (outs[0].float().square().sum() + outs[1].float().square().sum())
+
+    _, loss = run()
+    want = torch.autograd.grad(loss, ps)
+    with torch.autograd.graph.save_on_cpu():
+        _, loss = run()
+    for a, b in zip(torch.autograd.grad(loss, ps), want):
+        assert torch.equal(a, b)

@@ -420,3 +420,17 @@ def test_tokens_in_host_memory(monkeypatch, T):
     monkeypatch.setattr(ops, "rwkv7_decode", route)
     call(tree_map(lambda t: t.to("meta"), model(torch.bfloat16)), T, length=torch.tensor([2, 3]), new_starts=torch.zeros((2, T), dtype=torch.bool))
     assert got == [["meta"] * 4]
+
+
+@pytest.mark.parametrize("C", [64, 4160])
+@pytest.mark.parametrize("T", [3, 20])
+def test_saved_tensors_may_come_back_in_another_memory_order(monkeypatch, T, C):
+    """A saved-tensor hook gives the values back, not the strides: those of a state's row are not kept from the forward."""
+    from jaxrwkv_amd.model7 import RWKV7, randomize_weights
+    stub_library.install(monkeypatch)
+    params = randomize_weights(1, 1, C, V, dtype=torch.float32, device="cpu", zero_init=False)
+    for _, p in leaves(params):
+        p.requires_grad_()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.detach().clone(memory_format=torch.contiguous_format), lambda t: t):
+        logits, new_state = call(params, T)
+    (logits.sum() + new_state.sum()).backward()
