@@ -86,6 +86,24 @@ def test_summaries_that_amplify_are_not_used(monkeypatch):
     assert np.isnan(run(big, True)[0]).any() and np.isnan(whole(monkeypatch, big, True)[0]).any()
 
 
+def test_numeric_events_are_those_of_the_whole_sequence(monkeypatch):
+    """Every chunk and every carried state counts once, also where parts run the chunks before them again."""
+    from jaxrwkv_amd import ops
+
+    def events(x, f):
+        before = ops.numeric_events()
+        f(x, True)
+        return ops.numeric_events() - before
+
+    x = wkv7_inputs(1, 1200, 1, 64, seed=7, bf16=True, resets=False, lengths=False)
+    x["w"][:, 700:716] = 3.0                            # e^-20 a token: a capped chunk
+    capped = events(x, lambda *a: whole(monkeypatch, *a))
+    assert split(1, 1200, 1) >= 4 and capped > 0 and events(x, run) == capped
+    x["v"][:, 5] = 3e38                                 # no summary is usable, and the state turns non-finite
+    both = events(x, lambda *a: whole(monkeypatch, *a))
+    assert both > capped and events(x, run) == both
+
+
 def test_a_broken_handshake_poisons_every_part(monkeypatch):
     from jaxrwkv_amd import _lib, ops
     monkeypatch.setenv("HIPRWKV_ENABLE_DEBUG_FLAGS", "1")
