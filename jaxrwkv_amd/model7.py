@@ -226,9 +226,9 @@ class RWKV7:
             y = ops.rwkv7_postmix(out, r, k, v, g, att["ln_x"]["weight"], att["ln_x"]["bias"], att["r_k"], 64e-5)
             y = y.reshape(B, T, C)
         else:
-            y = out.reshape(B * T, C).float()
-            y = F.group_norm(y, H, att["ln_x"]["weight"].float(), att["ln_x"]["bias"].float(), 64e-5)
-            y = y.to(xr.dtype).reshape(B, T, C)
+            # not F.group_norm: in torch 2.10 for ROCm its weight's and bias's cotangents are wrong beyond some 100 rows
+            y = F.layer_norm(out.reshape(B, T, H, N).float(), (N,), eps=64e-5).reshape(B, T, C)
+            y = (y * att["ln_x"]["weight"].float() + att["ln_x"]["bias"].float()).to(xr.dtype)
             bonus = ((r * k * att["r_k"]).sum(-1, keepdim=True) * v).reshape(B, T, C)
             y = (y + bonus) * g.reshape(B, T, C)
         return y @ att["output"]["weight"].T, s_new, v_first
