@@ -865,7 +865,7 @@ int hiprwkv_rwkv7_decode(hiprwkv_stream stream, const hiprwkv_rwkv7_decode_args*
   const hiprwkv_rwkv7_decode_args& D = *args;
   if (D.B <= 0 || D.T <= 0 || D.L <= 0 || D.T > HIPRWKV_SMALL_T || D.B * D.T > HIPRWKV_DECODE_MAX_ROWS)
     return fail(HIPRWKV_EINVAL, "rwkv7_decode: B, T, L must be positive, T at most %d and B*T at most %d", HIPRWKV_SMALL_T, HIPRWKV_DECODE_MAX_ROWS);
-  if (D.C != D.H * 64 || D.C > 4096) return fail(HIPRWKV_EINVAL, "rwkv7_decode: C must be 64 H and at most 4096");
+  if (D.H <= 0 || D.H > 64 || D.C != D.H * 64) return fail(HIPRWKV_EINVAL, "rwkv7_decode: C must be 64 H, positive and at most 4096");
   for (int64_t d : {D.F, D.d_decay, D.d_aaa, D.d_mv, D.d_gate})
     if (d <= 0 || d % 32 != 0) return fail(HIPRWKV_EINVAL, "rwkv7_decode: inner sizes must be positive multiples of 32");
   if (D.logits != nullptr && (D.vocab <= 0 || D.vocab % 16 != 0)) return fail(HIPRWKV_EINVAL, "rwkv7_decode: vocab must be a positive multiple of 16");

@@ -241,3 +241,15 @@ def test_workspace_sizes_of_empty_calls():
         assert lib.hiprwkv_wkv6_fwd_workspace_bytes(dtype, B, T, H, 64) == 0
     assert lib.hiprwkv_rwkv7_decode_workspace_bytes(None) == 0
     assert lib.hiprwkv_rwkv7_decode_workspace_bytes(ctypes.byref(_lib.Rwkv7DecodeArgs())) == 0
+
+
+def test_decode_step_of_no_channels_is_refused():
+    """Not a division by the tiles of an empty product."""
+    from jaxrwkv_amd import _lib
+    lib = _lib.load()
+    for H in (0, -1, 65):
+        args = _lib.Rwkv7DecodeArgs(**{n: 0x10000 for n, t in _lib.Rwkv7DecodeArgs._fields_ if t is ctypes.c_void_p})
+        args.B, args.T, args.L, args.H, args.C, args.F = 64, 1, 1, H, 64 * H, 64
+        args.d_decay = args.d_aaa = args.d_mv = args.d_gate = 32
+        args.vocab, args.new_state, args.workspace_bytes = 64, 0x20000, 1 << 40
+        assert lib.hiprwkv_rwkv7_decode(None, ctypes.byref(args)) == -1 and b"64 H" in lib.hiprwkv_last_error()
