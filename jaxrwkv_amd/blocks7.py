@@ -357,7 +357,7 @@ def covers(params, x, state):
     if not (io in ops._DT and x.is_cuda and state.dtype == io and state.device == dev and C <= ops.LN_SHIFTMIX_MAX_C):
         return False
     for name, t in zip(NAMES, params):
-        if t.dtype != io or t.device != dev or not t.is_contiguous() or t.data_ptr() % 16:
+        if t.dtype != io or t.device != dev or len(t) != len(params[0]) or not t.is_contiguous() or t.data_ptr() % 16:
             return False
         if name not in _PRODUCTS and name not in _FACTORS and t.numel() != n:
             return False

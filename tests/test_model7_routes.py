@@ -305,7 +305,7 @@ def _flat(w):
 BAD = {"a vector of another size": ("x_k", lambda w: w[:, :32].contiguous()), "a factor of another size": ("w1", lambda w: w[:, :32].contiguous()),
        "a second factor of another size": ("g2", lambda w: w[:, :, :32].contiguous()),
        "one layer less": ("a0", lambda w: w[:1].contiguous()), "off a 16-byte boundary": ("v1", _flat),
-       "on another device": ("k_a", lambda w: w.to("meta"))}
+       "a vector of another shape": ("x_v", lambda w: w.reshape(2 * L, -1)), "on another device": ("k_a", lambda w: w.to("meta"))}
 
 
 @pytest.mark.parametrize("bad", list(BAD))
@@ -318,6 +318,9 @@ def test_the_stack_operator_takes_what_its_kernels_can_read(monkeypatch, bad):
     name, change = BAD[bad]
     params["blocks"]["att"][name] = change(params["blocks"]["att"][name])
     assert not blocks7.covers(blocks7.gather(params["blocks"]), x, state)
+    if bad == "a vector of another shape":                      # torch refuses it
+        with pytest.raises(RuntimeError):
+            call(params, 20)
     if bad == "off a 16-byte boundary":                         # torch's products take it
         with torch.no_grad():
             assert not call(params, 20)[1].isnan().any()
