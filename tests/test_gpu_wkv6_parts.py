@@ -3,7 +3,9 @@ kernel over the whole sequence, to which it falls back without a workspace.
 
 The chunks and their operands are the whole sequence's; a part adds one fp32 multiply-add per state element.  The bounds against
 the oracle are those of the whole sequence (test_gpu_wkv6_chunked); the rms errors of the two are compared as well: the same
-fp16 roundings of a state that differs by a few 2^-24, hence a tenth more."""
+fp16 roundings of a state that differs by a few 2^-24.  Measured against 64 bits over three shapes and log decays of 1, 2^-6, 2^-10 and 0
+times the usual: state 0.9e-4 / 2.0e-4 / 2.0e-4 / 2e-7 relative to the result, y 1.66e-3 to 1.70e-3, in parts the same to three digits (without
+decay 0.5 to 0.7 times the state's).  A twentieth more is allowed."""
 import numpy as np
 import pytest
 import torch
@@ -71,7 +73,7 @@ def test_state_carried_over_the_parts(B, T, H, decay, monkeypatch):
     assert split(B, T, H) >= 2
     got, base = run(x, True), whole(monkeypatch, x, True)
     for g, w, e in zip(got, base, ref):
-        assert rms(g - e) <= 1.1 * rms(w - e) + 1e-6 * rms(e)
+        assert rms(g - e) <= 1.05 * rms(w - e) + 1e-6 * rms(e)
 
 
 def test_one_decay_for_all_tokens(monkeypatch):

@@ -3,8 +3,9 @@ kernel over the whole sequence, to which it falls back without a workspace.
 
 The parts add one product per part in fp32 to the whole sequence's arithmetic; the operand rounding (fp16, 2^-11) is the same and
 sets the error of both.  The bounds against the oracle are those of the whole sequence (test_gpu_wkv7_chunked); where the
-state is carried over many parts (slow decay) the rms errors of the two are compared: rounding errors of the same size in another
-order, so a quarter more is allowed."""
+state is carried over many parts (slow decay) the rms errors of the two are compared.  Measured against 64 bits at log decays of
+-0.5, -2.5, -5 and -8 over five shapes of 700 to 4096 tokens, relative to the result: state 1.2e-4 / 2.1e-4 / 2.9e-4 / 3.7e-4 whole, in
+parts 0.991 to 1.004 times that; y 1.66e-3 to 1.72e-3, the same to three digits.  A twentieth more is allowed."""
 import numpy as np
 import pytest
 import torch
@@ -65,22 +66,28 @@ def test_state_carried_over_the_parts(B, T, H, decay, monkeypatch):
     assert split(B, T, H) >= 2
     got, base = run(x, True), whole(monkeypatch, x, True)
     for g, w, e in zip(got, base, ref):
-        assert rms(g - e) <= 1.25 * rms(w - e) + 1e-6 * rms(e)
+        assert rms(g - e) <= 1.05 * rms(w - e) + 1e-6 * rms(e)
 
 
 def test_summaries_that_amplify_are_not_used(monkeypatch):
-    """b = +0.02 |a|^2-direction for the first 300 tokens, no decay to speak of: the state map grows by e^6 along one vector.  The
-    parts after it run the chunks before them themselves and give the whole sequence's bits from there on."""
+    """b = +0.03 a with a along one key for the second part's tokens, no decay to speak of: its state map grows by 1.03^160 = 100
+    along that key.  The state entering that part is the first part's own, so the parts after it, which run its chunks again
+    themselves, give the whole sequence's bits; with a summary that is used (the same without growth) the state's differ."""
     x = wkv7_inputs(1, 1200, 2, 64, seed=6, bf16=True, resets=False, lengths=False)
+    P = split(1, 1200, 2)
+    n = 16 * -(-75 // P)                                # tokens of a part
+    assert P >= 4 and n >= 128
     x["w"][:] = -9.0
-    x["a"][:, :300] = x["a"][:, :1]
-    x["b"][:, :300] = bf16_round(0.02 * x["a"][:, :300])
-    assert split(1, 1200, 2) >= 4
-    got, base = run(x, True), whole(monkeypatch, x, True)
-    ref = o7.wkv7_base(x["r"], x["w"], x["k"], x["v"], x["a"], x["b"], x["s"], x["length"], x["new_starts"], compat=True, return_sa=True)
-    for g, w, e in zip(got, base, ref):
-        assert np.isfinite(g).all()
-        assert rms(g - e) <= 1.25 * rms(w - e) + 1e-6 * rms(e)
+    for gain in (0.03, -0.03):
+        x["a"][:, n:2 * n] = 0.0
+        x["a"][:, n:2 * n, :, 5] = 1.0
+        x["b"][:, n:2 * n] = bf16_round(gain * x["a"][:, n:2 * n])
+        got, base = run(x, True), whole(monkeypatch, x, True)
+        ref = o7.wkv7_base(x["r"], x["w"], x["k"], x["v"], x["a"], x["b"], x["s"], x["length"], x["new_starts"], compat=True, return_sa=True)
+        assert np.array_equal(got[0], base[0]) == (gain > 0)
+        for g, w, e in zip(got, base, ref):
+            assert np.isfinite(g).all()
+            assert np.array_equal(g, w) if gain > 0 else rms(g - e) <= 1.05 * rms(w - e) + 1e-6 * rms(e)
     big = wkv7_inputs(1, 1200, 1, 64, seed=7, bf16=True, resets=False, lengths=False)
     big["v"][:, 5] = 3e38                               # beyond the fp16 operands: the whole sequence turns non-finite, and so do the parts
     assert np.isnan(run(big, True)[0]).any() and np.isnan(whole(monkeypatch, big, True)[0]).any()
