@@ -18,15 +18,17 @@ constexpr int GEMM_WAVES = 8;
 
 // f of a product, which is rounded to bf16 first, where the separate product would be stored
 __device__ __forceinline__ float rnd(float x) { return bf16_to_f32(f32_to_bf16(x)); }
+// tanh is 1 - 2 / (1 + e^2x) where that keeps its value to 1e-6 (its error is 1e-7 of one whatever x is) and the series below (the
+// next term is 62/2835 x^8).  This code is inlined at every store of every kernel here and its length costs all of them, so tanh
+// and sigmoid share the quotient.
 __device__ __forceinline__ float activate(float x, int act) {
   if (act == GEMM_ACT_NONE) return x;
   x = rnd(x);
-  switch (act) {
-    case GEMM_ACT_TANH: return tanhf(x);       // 1 - 2 / (1 + e^2x) has an error of 1e-7 of one, whatever x is
-    case GEMM_ACT_SIGMOID: return 1.f / (1.f + __expf(-x));
-    case GEMM_ACT_RELUSQ: { const float r = fmaxf(x, 0.f); return r * r; }
-    default: return x;
-  }
+  if (act == GEMM_ACT_RELUSQ) { const float r = fmaxf(x, 0.f); return r * r; }
+  const bool th = act == GEMM_ACT_TANH;
+  const float q = 1.f / (1.f + __expf(th ? 2.f * x : -x)), s = x * x;
+  const float series = x * fmaf(s, fmaf(s, fmaf(s, -17.f / 315.f, 2.f / 15.f), -1.f / 3.f), 1.f);
+  return !th ? q : fabsf(x) < 0.25f ? series : 1.f - 2.f * q;
 }
 
 // Weight-streaming product for few rows: bound by reading w once.  A workgroup owns 16 columns of one product and 16 MT
