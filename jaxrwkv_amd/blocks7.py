@@ -41,7 +41,6 @@ def _gemm(jobs):
     kn, (K, N)."""
     arr = (_lib.GemmJob * len(jobs))()
     for j, (out, x, w, km, kn, act, aux) in zip(arr, jobs):
-        ops._one_dtype(torch.bfloat16, out, x, w, aux)
         j.out, j.x, j.w, j.aux = out.data_ptr(), x.data_ptr(), w.data_ptr(), None if aux is None else aux.data_ptr()
         j.M, j.N = out.shape
         j.K = x.shape[0] if km else x.shape[1]
@@ -83,7 +82,7 @@ def _lora_bwd(p, grad, mix, hid, gout, dmix, names):
     """From the cotangents ``gout`` of the low-rank terms: the parameters' cotangents into ``grad`` (those it has) and the
     inputs' into ``dmix`` (the value residual's is added to what is there)."""
     if _grouped(p, gout["w"]):
-        dh = {n: gout[n].new_empty((gout[n].shape[0], p[n + "1"].shape[-1])) for n, _ in names}
+        dh = {n: gout[n].new_empty((len(gout[n]), p[n + "1"].shape[-1])) if hid[n] is None else torch.empty_like(hid[n]) for n, _ in names}
         _gemm([(dh[n], gout[n], p[n + "2"], 0, 0, act, hid[n] if act else None) for n, act in names])
         _gemm([(dmix[n], dh[n], p[n + "1"], 0, 0, 0, dmix[n] if n == "v" else None) for n, _ in names])
         jobs = ([(grad[n + "1"], mix[n], dh[n], 1, 1, _NONE, None) for n, _ in names if n + "1" in grad]
@@ -112,7 +111,7 @@ def _ln_mix(p, x, dx, ln, state_row, ns, length, mix, shift_out, keep):
     prev, stride = ops._shift_row(state_row, B, C, x.dtype)
     xs, outs = ops._ln_shiftmix_fwd(x, dx, p[ln + "_w"], p[ln + "_b"], 1e-5, prev, stride, ns, length,
                                     [p[n] for n in mix], shift_out, stats)
-    return xs, outs, (stats, prev)
+    return xs, outs, (stats, prev, stride)
 
 
 def _layer_fwd(i, p, x, dx, st, nst, v_first, ns, length, need):
@@ -127,6 +126,8 @@ def _layer_fwd(i, p, x, dx, st, nst, v_first, ns, length, need):
     x, outs, head1 = _ln_mix(p, x, dx, "ln1", st[:, 1], ns, length, MIX, nst[:, 1], keep)
     xr, xw, xk, xv, xa, xg = map(flat, outs)
     r, k, v = (torch.mm(a, p[n].T) for a, n in ((xr, "receptance"), (xk, "key"), (xv, "value")))
+    # `covers` has seen the call's own tensors; under an autocast that the caller overlooked products come out in another type
+    ops._one_dtype(x.dtype, r)
     mix = {"w": xw, "a": xa, "g": xg, "v": xv}
     hid, lora = _lora_fwd(p, mix, _LORA if i else _LORA[:3], r)
     if i == 0:
@@ -149,7 +150,7 @@ def _layer_fwd(i, p, x, dx, st, nst, v_first, ns, length, need):
     saved = None
     if keep:
         # an operand of a weight's cotangent alone is kept for that weight only
-        only = lambda t, *names: t if need.intersection(names) else None
+        only = (lambda t, *names: t) if len(need) == len(NAMES) else (lambda t, *names: t if need.intersection(names) else None)
         saved = dict(x=x, head1=head1, xr=only(xr, "receptance"), xk=only(xk, "key"),
                      mix={n: only(t, n + "1", *(("value",) if n == "v" else ())) for n, t in mix.items()},
                      r=r, k=k, v=v, hid={n: hid[n] if act else only(hid[n], n + "2") for n, act in _LORA if n in hid}, lora=lora,
@@ -165,10 +166,11 @@ def _vectors(grad, names, scratch):
 
 def _ln_mix_bwd(p, grad, scratch, xs, head, ln, ns, length, mix, gs, gx, gshift, need_prev):
     lib = _lib.load()
-    stats, prev = head
+    stats, prev, stride = head
     io = xs.dtype
     B, T, C = xs.shape
-    prev, stride = ops._shift_row(prev, B, C, io)             # a saved-tensor hook may have moved it
+    if prev.stride(1) != 1 or (B > 1 and prev.stride(0) != stride):
+        prev, stride = ops._shift_row(prev, B, C, io)         # a saved-tensor hook has moved it
     dxs = torch.empty_like(xs)
     dprev = torch.empty((B, C), dtype=io, device=xs.device) if need_prev else None
     params = [p[n] for n in mix]
@@ -320,10 +322,11 @@ class _Blocks(torch.autograd.Function):
         g_in = torch.empty_like(state) if ctx.needs_input_grad[1] else None
         g_vfirst = None
         layers = list(zip(*(t.unbind(0) for t in params)))
+        glayers = list(zip(*(t.unbind(0) for t in grads.values()))) or [()] * L
         # products in the operands' own dtype even where the caller's backward runs under autocast
         with torch.autocast(like.device.type, enabled=False):
             for i in reversed(range(L)):
-                dx, g_vfirst = _layer_bwd(i, dict(zip(NAMES, layers[i])), {n: t[i] for n, t in grads.items()}, scratch, saved[i],
+                dx, g_vfirst = _layer_bwd(i, dict(zip(NAMES, layers[i])), dict(zip(grads, glayers[i])), scratch, saved[i],
                                           ns, length, g_x, g_dx, None if g_state is None else g_state[:, i],
                                           None if g_in is None else g_in[:, i], g_vfirst, v_first)
                 g_x = g_dx = dx
@@ -353,11 +356,12 @@ def covers(params, x, state):
     """Whether the operator takes the call: one dtype and device throughout, stacked parameters of the sizes that the kernels
     read, contiguous and on 16-byte boundaries."""
     io, dev, C = x.dtype, x.device, x.shape[-1]
-    n = params[0].shape[0] * C
+    L = params[0].shape[0]
+    n = L * C
     if not (io in ops._DT and x.is_cuda and state.dtype == io and state.device == dev and C <= ops.LN_SHIFTMIX_MAX_C):
         return False
     for name, t in zip(NAMES, params):
-        if t.dtype != io or t.device != dev or len(t) != len(params[0]) or not t.is_contiguous() or t.data_ptr() % 16:
+        if t.dtype != io or t.device != dev or t.shape[0] != L or not t.is_contiguous() or t.data_ptr() % 16:
             return False
         if name not in _PRODUCTS and name not in _FACTORS and t.numel() != n:
             return False

@@ -511,7 +511,6 @@ def _postmix_fwd(y, r, k, v, g, ln_w, ln_b, r_k, eps):
     io = y.dtype
     H, N = y.shape[-2:]
     rows = y.numel() // (H * N)
-    _one_dtype(io, r, k, v, g, ln_w, ln_b, r_k)
     out = torch.empty_like(y)
     rc = lib.hiprwkv_rwkv7_postmix(_stream(), _DT[io], rows, H, N, _p(y), _p(r), _p(k), _p(v), _p(g), _p(ln_w), _p(ln_b),
                                    _p(r_k), float(eps), _p(out))
@@ -799,7 +798,6 @@ def _ln_shiftmix_fwd(x, dx, ln_w, ln_b, eps, prev, prev_stride, ns, length, mix,
     lib = _lib.load()
     B, T, C = x.shape
     n_out = len(mix)
-    _one_dtype(x.dtype, dx, ln_w, ln_b, prev, shift_out, *mix)
     outs = [torch.empty_like(x) for _ in range(max(n_out, 1))]
     xs = x if dx is None else torch.empty_like(x)
     rc = lib.hiprwkv_rwkv7_ln_shiftmix(_stream(), _DT[x.dtype], B, T, C, n_out, _p(x), _p(dx), _p(ln_w), _p(ln_b), eps,
@@ -866,6 +864,7 @@ def rwkv7_ln_shiftmix(x, dx, ln, prev, new_starts, length, mix, eps=1e-5, shift_
             raise ValueError("rwkv7_ln_shiftmix: shift_out is for calls without autograd")
         xs, shift, *outs = _LnShiftMix.apply(x, dx, ln_w, ln_b, prev, new_starts, length, eps, *mix2)
         return xs, shift, outs
+    _one_dtype(io, shift_out)
     prev_t, stride = (None, C) if prev is None else _shift_row(prev, B, C, io)
     if shift_out is None and prev is not None:
         shift_out = torch.empty((B, C), dtype=io, device=x.device)
@@ -876,7 +875,6 @@ def rwkv7_ln_shiftmix(x, dx, ln, prev, new_starts, length, mix, eps=1e-5, shift_
 def _pre_fwd(xw, k, xa, v, vf, xv, w0, a0, v0, k_k, k_a):
     lib = _lib.load()
     H, N = k.shape[-2:]
-    _one_dtype(k.dtype, xw, xa, v, vf, xv, w0, a0, v0, k_k, k_a)
     w, k_out, a_out, b_out = (torch.empty_like(k) for _ in range(4))
     v_out = None if vf is None else torch.empty_like(k)
     rc = lib.hiprwkv_rwkv7_pre(_stream(), _DT[k.dtype], k.numel() // (H * N), H, N, _p(xw), _p(k), _p(xa), _p(v), _p(vf),
