@@ -29,9 +29,9 @@ B, T, H, N = 8, 4096, 32, 64
 # figures in profiles/), each with the sha1 prefix of the kernel source it was measured on: when the source has
 # changed since, `roofline.traffic` is null instead of a stale figure.
 MEASURED_TRAFFIC = {
-    "wkv7_fwd": (948.7e6, "wkv7_fwd.hip", "51a3d3ca403c", "profiles/wkv7_fwd_B8_T4096_H32_bf16.md"),
-    "wkv4_fwd": (4028.7e6, "wkv4.hip", "d83a0992a92e", "profiles/wkv4_fwd_B32_T4096_C2560_f32.md"),
-    "wkv6_fwd": (688.4e6, "wkv6_fwd.hip", "e577f9812ac6", "profiles/wkv6_fwd_bwd_B16_T2048_H32_bf16.md"),
+    "wkv7_fwd": (948.7e6, "wkv7_fwd.hip", "24d8d052dad9", "profiles/wkv7_fwd_B8_T4096_H32_bf16.md"),
+    "wkv4_fwd": (4028.7e6, "wkv4.hip", "224549c5651e", "profiles/wkv4_fwd_B32_T4096_C2560_f32.md"),
+    "wkv6_fwd": (688.4e6, "wkv6_fwd.hip", "ffdebea1aab9", "profiles/wkv6_fwd_bwd_B16_T2048_H32_bf16.md"),
 }
 
 
@@ -48,7 +48,7 @@ def measured_traffic(name):
 
 
 def make_inputs(torch, seed=0):
-    """Config-2 inputs, generated on the host with a fixed stream and uploaded once."""
+    """The headline inputs, generated on the host with a fixed stream and uploaded once."""
     g = np.random.default_rng(seed)
     shp = (B, T, H, N)
     f = lambda x: torch.from_numpy(np.ascontiguousarray(x, dtype=np.float32)).cuda()
@@ -250,7 +250,7 @@ def bench_wkv7(torch, ops, args):
     fwd_bytes = 7 * tokens * H * N * 2 + 2 * B * H * N * N * 4 + B * T + B * 4
     out = base_record("WKV7 fwd tokens/s (B8 T4096 H32 N64 bf16)", tokens / (ms_step * 1e-3), ms_step, args, "bf16",
                       "isolated WKV7 op, B=8 T=4096 H=32 N=64, bf16 r/w/k/v/a/b/y, fp32 state, "
-                      "new_starts~Bernoulli(1/1024), length~U{T/2..T} (BASELINE configs[1])",
+                      "new_starts~Bernoulli(1/1024), length~U{T/2..T}",
                       {"kernel": "sequential fp32 VALU" if args.seq else "chunked MFMA (fp16 operands, bf16 pairs in the Gram tiles, fp32 state)"})
     out["roofline"] = roofline(fwd_bytes, kern_ms, None if args.seq else measured_traffic("wkv7_fwd"))
     if not args.no_bwd:
@@ -386,8 +386,7 @@ def bench_wkv6(torch, ops, args):
     ms_step = 1e3 * wall / args.steps
     fwd_bytes = 5 * tokens * H * N * 2 + 2 * b6 * H * N * N * 4 + b6 * t6
     out = base_record("WKV6 fwd tokens/s (B16 T2048 H32 N64 bf16)", tokens / (ms_step * 1e-3), ms_step, args, "bf16",
-                      "isolated WKV6 op, B=16 T=2048 H=32 N=64 bf16, zero state, new_starts~Bernoulli(1/512) "
-                      "(BASELINE configs[2])",
+                      "isolated WKV6 op, B=16 T=2048 H=32 N=64 bf16, zero state, new_starts~Bernoulli(1/512)",
                       {"kernel": "chunked MFMA; forward on fp16 operands (bf16 pairs in the Gram tile), backward sweeps on "
                                  "bf16 hi+lo pairs; fp32 state and accumulation"})
     out["roofline"] = roofline(fwd_bytes, kern_ms, measured_traffic("wkv6_fwd"))
@@ -441,8 +440,8 @@ def bench_wkv4(torch, ops, args):
     ms_step = 1e3 * wall / args.steps
     fwd_bytes = 3 * tokens * c4 * 4 + 2 * b4 * 3 * c4 * 4
     out = base_record("WKV4 fwd tokens/s (B32 T4096 C2560 fp32)", tokens / (ms_step * 1e-3), ms_step, args, "f32",
-                      "isolated WKV4 op, B=32 T=4096 C=2560 fp32, state (0,0,-1e38), length~U{1024..4096} "
-                      "(BASELINE configs[3])", {"kernel": "one thread per (sequence, channel)"})
+                      "isolated WKV4 op, B=32 T=4096 C=2560 fp32, state (0,0,-1e38), length~U{1024..4096}",
+                      {"kernel": "one thread per (sequence, channel)"})
     out["roofline"] = roofline(fwd_bytes, kern_ms, measured_traffic("wkv4_fwd"))
     if not args.no_bwd:
         gy = f(g.standard_normal((b4, t4, c4), dtype=np.float32))
@@ -468,7 +467,7 @@ def bench_wkv4(torch, ops, args):
 
 
 def bench_model7(torch, ops, args):
-    """BASELINE configs[4]: RWKV-7 1.5B-shaped random-init model through the torch harness with HipRWKV.inner_loop:
+    """RWKV-7 1.5B-shaped random-init model through the torch harness with HipRWKV.inner_loop:
     prefill B=16 T=4096 (new_starts ~ Bernoulli(1/2048)) and decode B=256 single-token steps from a carried state."""
     from jaxrwkv_amd.model7 import RWKV7, randomize_weights
     L, C, vocab = 24, 2048, 65536
@@ -530,7 +529,7 @@ def bench_model7(torch, ops, args):
         graph_ok = f"capture failed: {type(exc).__name__}: {exc}"[:200]
     out = base_record("RWKV7 1.5B-shaped prefill tokens/s (B16 T4096 bf16, HipRWKV)", bp * tp / (ms_p * 1e-3), ms_p,
                       args, "bf16", "full model L=24 C=2048 H=32 N=64 vocab=65536, bf16 random-init weights, torch "
-                      "harness + HipRWKV.inner_loop; prefill B=16 T=4096 new_starts~Bernoulli(1/2048) (BASELINE configs[4])")
+                      "harness + HipRWKV.inner_loop; prefill B=16 T=4096 new_starts~Bernoulli(1/2048)")
     out["steps"], out["warmup"] = steps, 1
     out["prefill"] = {"ms_per_step": ms_p, "wkv_ms_all_layers": L * op_ms, "wkv_fraction": L * op_ms / ms_p}
     out["decode"] = {"tokens_per_s": bd / (ms_d * 1e-3), "ms_per_step": ms_d, "batch": bd,

@@ -1,6 +1,6 @@
 // Products beside the RWKV-7 recurrence that a library call serves badly, several of them per launch, bf16 in and out, fp32
 // accumulation:
-//   * a decode step's projections (few rows: a stream of the weights), skinny_gemm_kernel and, from 65 rows on, tile_gemm_kernel;
+//   * a decode step's projections (few rows: a stream of the weights), skinny_gemm_kernel and, from 33 rows on, tiles;
 //   * the low-rank factors of decay, gate, value residual and output gate in whole-sequence passes, forward and backward
 //     (rwkv7.py:237-245): narrow on one side, so that a library call of 10-18 us each is mostly launch and latency.
 #include "chunk_common.h"
@@ -111,12 +111,12 @@ __global__ __launch_bounds__(64 * GEMM_WAVES) void skinny_gemm_kernel(GemmArgs A
 // steps ahead, and four workgroups share a CU, so loads, LDS writes and matrix instructions of different workgroups
 // overlap.  An operand that lies k-major (km, kn) goes to LDS as it lies and is read with the transposing load.  Workgroups go
 // to the eight XCDs round-robin; the tiles that share a piece of the longer operand run on one XCD, whose L2 reads it once.
-// Bound by the CU's paths to the cache and to LDS (16 KiB in, 16 KiB to LDS and 32 KiB from it per step: 790 cycles with two
-// workgroups on a CU, 1000 with one).  Weights straight from memory into the matrix operands instead were slower (a
-// cache line per lane: 2200 cycles for 128 x 64 x 128), and so were four steps in flight.  Where one product leaves CUs idle
+// Its waves wait half of their time at 4084 rows and three quarters in a decode step (profiles/rwkv7_model_bf16.md): a step moves
+// 16 KiB in, 16 KiB to LDS and 32 KiB from it for 32 matrix instructions.  Weights straight from memory into the matrix operands
+// were slower (a cache line per lane), and so were four steps in flight.  Where one product leaves CUs idle
 // (a decode step's output and value projections: 128 tiles) K is split over gridDim.y and the parts are added by the norm
-// that reads the result.  Low-rank products at 4084 tokens of 2048 channels: 35 us for the four into the inner sizes (74 with
-// the row tiles of a narrow product on one XCD), 48 us out of them (67 MB written).
+// that reads the result.  Low-rank products at 4084 tokens of 2048 channels, through registers: 36 us for the four into the inner
+// sizes (74 with the row tiles of a narrow product on one XCD), 47 us out of them (67 MB written).
 constexpr int TG = 64, TG_RS = TG + 8;         // tile edge; LDS row stride: 16-byte rows 144 bytes apart
 constexpr int AHEAD = 2;                       // steps whose operands are in flight (four: 212 registers, 1.6 times slower for short K)
 typedef uint16_t TileLds[2][2][TG][TG_RS];     // [buffer][x | w]
@@ -293,8 +293,9 @@ int tiles_of(const GemmJob& J, int tm) {
 // 16-byte piece p of row q lies at p ^ swizzle(q) instead (no bank conflicts counted).  Weights that no cache holds, against the
 // tiles through registers: 64 rows of 2048 channels into 8192 columns 19.0 -> 15.3 us, K = 8192 into 2048 unsplit 57.9 -> 37.8;
 // 128 rows 19.3 -> 15.4; r, k, v and the low-rank inputs at 128 rows 20.5 -> 16.6; 256 rows into 8192 columns 23.5 -> 22.8 with
-// 64-row tiles, 19.9 with 128.  Bound by the wait for the weights (56 % of the waves' time); five and seven steps in flight took as
-// long, and so did a first step that differs from tile to tile.
+// 64-row tiles, 19.9 with 128.  Bound by the wait for the weights (47 to 55 % of the waves' time in a step of 256 users,
+// profiles/rwkv7_model_bf16.md); five and seven steps in flight took as long, and so did a first step that differs from tile to
+// tile.
 constexpr int stream_step(int tm) { return (tm + TG) * TG; }       // bf16 values of a step in LDS: TM rows of x, TG of w
 typedef __attribute__((address_space(3))) uint16_t* lds_u16_ptr;
 

@@ -161,7 +161,7 @@ def test_wkv4_split_call_equals_single_call_at_the_benchmark_shape():
 
 
 def test_wkv7_prefill_shape_of_the_1p5b_config():
-    """BASELINE configs[4], prefill: the op at B=16, T=4096, H=32, bf16, new_starts ~ Bernoulli(1/2048).  Chunked
+    """The model's prefill: the op at B=16, T=4096, H=32, bf16, new_starts ~ Bernoulli(1/2048).  Chunked
     against sequential kernel, and a split call with the carried state against the single call."""
     from jaxrwkv_amd import ops
     x = wkv7_full(B=16, seed=5, p_reset=1.0 / 2048)
@@ -189,7 +189,7 @@ def test_wkv7_prefill_shape_of_the_1p5b_config():
 
 @pytest.mark.parametrize("st", [torch.float32, torch.bfloat16])
 def test_wkv7_decode_shape_of_the_1p5b_config(st):
-    """BASELINE configs[4], decode: one token for B=256 sequences x 32 heads from a carried state, against the float64
+    """The model's decode step: one token for B=256 sequences x 32 heads from a carried state, against the float64
     oracle (bf16 inputs; fp32 state to the fp32 bar, bf16 state and y within one bf16 ulp)."""
     import numpy as np
     from jaxrwkv_amd import ops

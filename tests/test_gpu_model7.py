@@ -65,7 +65,7 @@ def test_small_bf16_model():
 
 
 def test_rwkv7_0p1b_shape_fp32():
-    """L=12, C=768, H=12, head size 64, vocab 65536, fp32, B=1, T=512, default zero state."""
+    """The 0.1B shape: L=12, C=768, H=12, head size 64, vocab 65536, fp32, B=1, T=512, default zero state."""
     lg, st, rlg, rst = run_case(L=12, C=768, vocab=65536, B=1, T=512, dtype=torch.float32, seed=7, p_reset=0.0)
     assert rel_rms(lg, rlg) < 1e-3, rel_rms(lg, rlg)
     assert rel_rms(st, rst) < 1e-3, rel_rms(st, rst)
@@ -413,7 +413,7 @@ def test_bf16_logits_tvd_of_the_chunked_kernels_is_below_1e_3():
 
 
 def test_rwkv7_1p5b_shape_bf16_few_tokens():
-    """BASELINE configs[4] shape (L=24, C=2048, H=32; vocabulary cut to 4096), bf16, B=2, T=48 with resets and short
+    """The 1.5B shape (L=24, C=2048, H=32; vocabulary cut to 4096), bf16, B=2, T=48 with resets and short
     lengths: logits against the float64 full-model oracle on the same bf16 weights (tolerances of the small bf16
     model: every activation of the harness is rounded to bf16), and the kernel-only logits TVD below 1e-3."""
     lg, st, rlg, rst = run_case(L=24, C=2048, vocab=4096, B=2, T=48, dtype=torch.bfloat16, seed=23, p_reset=0.03)
@@ -425,7 +425,7 @@ def test_rwkv7_1p5b_shape_bf16_few_tokens():
 
 
 def test_rwkv7_1p5b_at_the_real_sizes_prefill_and_decode():
-    """BASELINE configs[4] at its real sizes (L=24, C=2048, H=32, N=64, vocab 65536, bf16): prefill B=16 T=4096 with
+    """The 1.5B shape at its real sizes (L=24, C=2048, H=32, N=64, vocab 65536, bf16): prefill B=16 T=4096 with
     new_starts ~ Bernoulli(1/2048) gives finite logits, and the state of a call split at token 2048 with the carried
     state agrees with the single call's (the recurrence is bit-identical at a chunk-aligned split; torch's projections
     may pick other GEMM kernels for the other row count, hence a tolerance of the bf16 model tests' size); decode B=256,
