@@ -449,6 +449,8 @@ class _Wkv4(torch.autograd.Function):
         ctx.flags = flags
         ctx.save_for_backward(w, u, k, v, r, s, length, new_starts, ckpt)
         ctx.set_materialize_grads(False)
+        if not any(ctx.needs_input_grad[i] for i in (0, 1, 2, 3, 5)):
+            ctx.mark_non_differentiable(new_s)            # the state does not depend on the receptance
         return new_s, y
 
     @staticmethod
@@ -457,7 +459,8 @@ class _Wkv4(torch.autograd.Function):
         lib = _lib.load()
         io = k.dtype
         B, T, C = k.shape
-        gy = torch.zeros_like(k) if gy is None else _aligned(_dev(gy, io))
+        given = gy is not None
+        gy = _aligned(_dev(gy, io)) if given else torch.zeros_like(k)
         gs_new = None if gs_new is None else _dev(gs_new, io)
         gk, gv, gs = torch.empty_like(k), torch.empty_like(v), torch.empty_like(s)
         gr = None if r is None else torch.empty_like(r)
@@ -468,7 +471,7 @@ class _Wkv4(torch.autograd.Function):
                                       _p(length), _p(new_starts), _p(gs_new), _p(ckpt), ckpt.numel(), _p(gw), _p(gu), _p(gk),
                                       _p(gv), _p(gr), _p(gs), _p(ws), nbytes, ctx.flags | _lib.CKPT_READY)
         _lib.check(rc, "hiprwkv_wkv4_mix_bwd")
-        return gw, gu, gk, gv, gr, gs, None, None, None
+        return gw, gu, gk, gv, (gr if given else None), gs, None, None, None
 
 
 def wkv4(w_neg, u, k, v, s, length=None, new_starts=None, compat=True):

@@ -46,3 +46,17 @@ def test_model_state_cotangent_anywhere_in_memory(monkeypatch, T):
     ps = [p.requires_grad_() for _, p in leaves(params["blocks"])]
     _, new_state = call(params, T, B=1)
     torch.autograd.grad(new_state, ps, off(torch.randn(1, L, 66, C)), allow_unused=True)
+
+
+def test_wkv4_state_and_receptance_are_apart(monkeypatch):
+    """The new state has no derivative in the receptance: no graph, and no cotangent of zeros for it."""
+    from jaxrwkv_amd.rwkv4 import HipRWKV
+    stub_library.install(monkeypatch)
+    n = lambda *s: torch.randn(s)
+    r, k = n(2, 5, 64).requires_grad_(), n(2, 5, 64)
+    new_s, out = HipRWKV.inner_loop(r, k, n(2, 5, 64), n(64), n(64), n(2, 3, 64), None, None)
+    assert not new_s.requires_grad and torch.autograd.grad(out.sum(), r)[0] is not None
+    k.requires_grad_()
+    new_s, out = HipRWKV.inner_loop(r, k, n(2, 5, 64), n(64), n(64), n(2, 3, 64), None, None)
+    gr, gk = torch.autograd.grad(new_s.sum(), (r, k), allow_unused=True)
+    assert gr is None and gk is not None
