@@ -314,10 +314,12 @@ class _Blocks(torch.autograd.Function):
         g_x = torch.zeros_like(like) if g_x is None else ops._dev(g_x, io)
         g_dx = torch.zeros_like(like) if g_dx is None else ops._dev(g_dx, io)
         g_state = None if g_state is None else ops._aligned(g_state.to(io))
-        grads = {n: torch.empty_like(t) for n, t, asked in zip(NAMES, params, ctx.needs_input_grad[4:]) if asked}
-        for n in ("v0", "v1", "v2"):
+        residual = ("v0", "v1", "v2")           # the first layer has no value residual
+        grads = {n: torch.empty_like(t) for n, t, asked in zip(NAMES, params, ctx.needs_input_grad[4:])
+                 if asked and (L > 1 or n not in residual)}
+        for n in residual:
             if n in grads:
-                grads[n][0].zero_()             # the first layer has no value residual
+                grads[n][0].zero_()
         scratch = torch.empty(like.shape[-1], dtype=io, device=like.device)
         g_in = torch.empty_like(state) if ctx.needs_input_grad[1] else None
         g_vfirst = None

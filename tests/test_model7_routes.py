@@ -437,3 +437,14 @@ def test_saved_tensors_may_come_back_in_another_memory_order(monkeypatch, T, C):
     with torch.autograd.graph.saved_tensors_hooks(lambda t: t.detach().clone(memory_format=torch.contiguous_format), lambda t: t):
         logits, new_state = call(params, T)
     (logits.sum() + new_state.sum()).backward()
+
+
+@pytest.mark.parametrize("T", [3, 20])
+def test_one_layer_has_no_value_residual(monkeypatch, T):
+    from jaxrwkv_amd.model7 import randomize_weights
+    stub_library.install(monkeypatch)
+    params = randomize_weights(1, 1, C, V, dtype=torch.bfloat16, device="cpu", zero_init=False)
+    ps = {n: p.requires_grad_() for n, p in leaves(params)}
+    logits, new_state = call(params, T)
+    grads = torch.autograd.grad(logits.float().sum() + new_state.float().sum(), ps.values(), allow_unused=True)
+    assert [n for n, g in zip(ps, grads) if g is None] == ["blocks.att.v0", "blocks.att.v1", "blocks.att.v2"]
