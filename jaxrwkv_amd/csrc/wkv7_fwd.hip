@@ -821,7 +821,7 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_kernel(Wkv7Args
     const int p = pp;
     Raw raw;
     // every chunk counts once: in the launch after the summaries, where its output is written
-    unsigned* const events = MODE == SUMMARY ? nullptr : events_word(A.status);
+    unsigned* events = MODE == SUMMARY || (MODE == PART && part0 != part) ? nullptr : events_word(A.status);
     // this lane's new_starts byte of the chunk loaded next: fetched a step ahead, behind the operands (measured: 1.6 %
     // faster here than in front of them, where the other sweeps have it)
     uint32_t ns_mine = 0u;
@@ -846,7 +846,8 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_kernel(Wkv7Args
       const ChunkFlags F = chunk_flags_of(A.ns, ns_mine, A.flags, A.T, c0, MODE == SUMMARY ? 0 : L);
       mask_raw(raw, F.nvalid, lane);
       if (MODE == SUMMARY && map) raw.v[0] = raw.v[1] = make_uint4(0, 0, 0, 0);
-      produce<MODE>(lane, raw, F, slot, snapslot, MODE == PART && j0 + j < j_out ? nullptr : events);
+      if (MODE == PART && part0 != part && j0 + j >= j_out) events = events_word(A.status);
+      produce<MODE>(lane, raw, F, slot, snapslot, events);
       if (j + NPROD < n) {
         load_raw<MODE>(raw, A, b, h, c0 + (int64_t)NPROD * CK, lane);
         ns_mine = chunk_flag_prefetch(A.ns, A.T, b, c0 + (int64_t)NPROD * CK, lane);
