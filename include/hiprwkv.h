@@ -133,6 +133,17 @@ int hiprwkv_wkv7_fwd_parts(hiprwkv_stream stream, int io_dtype, int state_dtype,
                            const uint32_t* length, const uint8_t* new_starts,
                            void* out, void* sa, void* new_s, void* workspace, size_t workspace_bytes, unsigned flags);
 
+/* The same for a call with a backward to come: `ends` (hiprwkv_wkv7_ends_bytes, 0 where it is of no use, 16-byte aligned; NULL: none
+ * wanted; not with HIPRWKV_FORCE_SEQ) receives the states at which hiprwkv_wkv7_bwd_ends, given the same array, cuts the
+ * sequence into parts that run at the same time. */
+size_t hiprwkv_wkv7_ends_bytes(int io_dtype, int64_t B, int64_t T, int64_t H, int64_t N);
+int hiprwkv_wkv7_fwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype,
+                          int64_t B, int64_t T, int64_t H, int64_t N,
+                          const void* w, const void* r, const void* k, const void* v,
+                          const void* a, const void* b, const void* s,
+                          const uint32_t* length, const uint8_t* new_starts,
+                          void* out, void* sa, void* new_s, void* ends, void* workspace, size_t workspace_bytes, unsigned flags);
+
 /* A decode step (T <= HIPRWKV_SMALL_T tokens per sequence) on a state that lives inside the packed model state of the
  * reference: there a sequence's state is (L, 2+N, C) and layer l's rows 2.. are the (H,N,N) WKV state, flat
  * (rwkv7.py:176-180 default_state, :254-260 the slice and reshape around inner_loop), so with a batch axis in front
@@ -167,6 +178,18 @@ int hiprwkv_wkv7_bwd(hiprwkv_stream stream, int io_dtype, int state_dtype,
                      const void* gy, const void* sa, const void* gs_out,
                      void* gw, void* gr, void* gk, void* gv, void* ga, void* gb, void* gs,
                      void* workspace, size_t workspace_bytes, unsigned flags);
+
+/* The same with the `ends` of hiprwkv_wkv7_fwd_ends (NULL: as hiprwkv_wkv7_bwd) and a workspace of
+ * hiprwkv_wkv7_bwd_ends_workspace_bytes: few sequences and heads run in parts. */
+size_t hiprwkv_wkv7_bwd_ends_workspace_bytes(int io_dtype, int64_t B, int64_t T, int64_t H, int64_t N);
+int hiprwkv_wkv7_bwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype,
+                          int64_t B, int64_t T, int64_t H, int64_t N,
+                          const void* w, const void* r, const void* k, const void* v,
+                          const void* a, const void* b, const void* s,
+                          const uint32_t* length, const uint8_t* new_starts,
+                          const void* gy, const void* sa, const void* gs_out, const void* ends,
+                          void* gw, void* gr, void* gk, void* gv, void* ga, void* gb, void* gs,
+                          void* workspace, size_t workspace_bytes, unsigned flags);
 
 /* ---- WKV6 ------------------------------------------------------------------
  * The reference has no native WKV6 op (README.md:93-99); the operand order follows

@@ -48,11 +48,16 @@ SIGNATURES = {
     "hiprwkv_wkv7_fwd": (_int, [_vp, _int, _int, _i64, _i64, _i64, _i64] + [_vp] * 7 + [_vp, _vp] + [_vp, _vp, _vp, _u32]),
     "hiprwkv_wkv7_fwd_workspace_bytes": (_sz, [_int] + [_i64] * 4),
     "hiprwkv_wkv7_fwd_parts": (_int, [_vp, _int, _int, _i64, _i64, _i64, _i64] + [_vp] * 7 + [_vp, _vp] + [_vp] * 4 + [_sz, _u32]),
+    "hiprwkv_wkv7_ends_bytes": (_sz, [_int] + [_i64] * 4),
+    "hiprwkv_wkv7_fwd_ends": (_int, [_vp, _int, _int, _i64, _i64, _i64, _i64] + [_vp] * 7 + [_vp, _vp] + [_vp] * 5 + [_sz, _u32]),
     "hiprwkv_wkv7_step": (_int, [_vp, _int, _int, _i64, _i64, _i64, _i64] + [_vp] * 6 + [_vp, _i64] + [_vp, _vp]
                           + [_vp, _vp, _i64, _u32]),
     "hiprwkv_wkv7_bwd_workspace_bytes": (_sz, [_i64] * 4),
     "hiprwkv_wkv7_bwd": (_int, [_vp, _int, _int, _i64, _i64, _i64, _i64] + [_vp] * 7 + [_vp, _vp] + [_vp] * 3
                          + [_vp] * 7 + [_vp, _sz, _u32]),
+    "hiprwkv_wkv7_bwd_ends_workspace_bytes": (_sz, [_int] + [_i64] * 4),
+    "hiprwkv_wkv7_bwd_ends": (_int, [_vp, _int, _int, _i64, _i64, _i64, _i64] + [_vp] * 7 + [_vp, _vp] + [_vp] * 4
+                              + [_vp] * 7 + [_vp, _sz, _u32]),
     "hiprwkv_wkv6_fwd": (_int, [_vp, _int, _int, _i64, _i64, _i64, _i64] + [_vp] * 6 + [_vp, _vp] + [_vp, _vp, _u32]),
     "hiprwkv_wkv6_fwd_workspace_bytes": (_sz, [_int] + [_i64] * 4),
     "hiprwkv_wkv6_fwd_parts": (_int, [_vp, _int, _int, _i64, _i64, _i64, _i64] + [_vp] * 6 + [_vp, _vp] + [_vp] * 3 + [_sz, _u32]),

@@ -139,7 +139,7 @@ def _layer_fwd(i, p, x, dx, st, nst, v_first, ns, length, need):
     if i == 0:
         v2 = heads(v)
     s = st[:, 2:].reshape(B, H, N, N)
-    new_s, yw, sa = ops.wkv7_fwd(heads(r), w, k2, v2, a, b, s, length, ns, HipRWKV.assoc_compat, want_sa=keep)
+    new_s, yw, sa, ends = ops._wkv7_fwd(heads(r), w, k2, v2, a, b, s, length, ns, HipRWKV.assoc_compat, want_sa=keep, want_ends=keep)
     nst[:, 2:] = new_s.view(B, N, C)
     y = flat(ops._postmix_fwd(yw, heads(r), k2, v2, heads(lora["g"]), par("lnx_w"), par("lnx_b"), par("r_k"), EPS_X))
     dx1 = torch.mm(y, p["output"].T).view(B, T, C)
@@ -154,7 +154,7 @@ def _layer_fwd(i, p, x, dx, st, nst, v_first, ns, length, need):
         saved = dict(x=x, head1=head1, xr=only(xr, "receptance"), xk=only(xk, "key"),
                      mix={n: only(t, n + "1", *(("value",) if n == "v" else ())) for n, t in mix.items()},
                      r=r, k=k, v=v, hid={n: hid[n] if act else only(hid[n], n + "2") for n, act in _LORA if n in hid}, lora=lora,
-                     w=w, k2=k2, v2=v2, a=a, b=b, s=s, sa=sa, yw=yw, y=only(y, "output"), x2=x2, head2=head2,
+                     w=w, k2=k2, v2=v2, a=a, b=b, s=s, sa=sa, ends=ends, yw=yw, y=only(y, "output"), x2=x2, head2=head2,
                      xk2=only(flat(xk2), "ffn_key"), ff=ff, fr=only(fr, "ffn_value"))
     return x2, dx2, v_first, saved
 
@@ -226,7 +226,7 @@ def _layer_bwd(i, p, grad, scratch, S, ns, length, g_x, g_dx, g_state, g_in, g_v
     # the recurrence
     gs_out = None if g_state is None else g_state[:, 2:].reshape(B, H, N, N)
     gr2, gw, gk2, gv2, ga, gb, gs = ops.wkv7_bwd(heads(S["r"]), S["w"], S["k2"], S["v2"], S["a"], S["b"], S["s"], length, ns,
-                                                 gyw, S["sa"], gs_out, HipRWKV.assoc_compat)
+                                                 gyw, S["sa"], gs_out, HipRWKV.assoc_compat, ends=S["ends"])
     if g_in is not None:
         g_in[:, 2:] = gs.reshape(B, N, C)
     # gates

@@ -166,6 +166,19 @@ int hiprwkv_wkv7_fwd_parts(hiprwkv_stream stream, int io_dtype, int state_dtype,
                            const void* w, const void* r, const void* k, const void* v, const void* a, const void* b,
                            const void* s, const uint32_t* length, const uint8_t* new_starts, void* out, void* sa,
                            void* new_s, void* workspace, size_t workspace_bytes, unsigned flags) {
+  return hiprwkv_wkv7_fwd_ends(stream, io_dtype, state_dtype, B, T, H, N, w, r, k, v, a, b, s, length, new_starts, out, sa, new_s,
+                               nullptr, workspace, workspace_bytes, flags);
+}
+
+size_t hiprwkv_wkv7_ends_bytes(int io_dtype, int64_t B, int64_t T, int64_t H, int64_t N) {
+  if (io_dtype != HIPRWKV_BF16 || N != 64 || B <= 0 || T <= HIPRWKV_SMALL_T || H <= 0 || B * H > 0x7fffffffLL) return 0;
+  return (size_t)(B * H) * (wkv7_bwd_parts(B * H, T).n_end - 1) * 4096 * sizeof(float);
+}
+
+int hiprwkv_wkv7_fwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype, int64_t B, int64_t T, int64_t H, int64_t N,
+                          const void* w, const void* r, const void* k, const void* v, const void* a, const void* b,
+                          const void* s, const uint32_t* length, const uint8_t* new_starts, void* out, void* sa,
+                          void* new_s, void* ends, void* workspace, size_t workspace_bytes, unsigned flags) {
   int rc = check_matrix_shape("wkv7_fwd", io_dtype, state_dtype, B, T, H, N);
   if (rc) return rc;
   if ((rc = check_flags("wkv7_fwd", flags)) != HIPRWKV_OK) return rc;
@@ -175,6 +188,8 @@ int hiprwkv_wkv7_fwd_parts(hiprwkv_stream stream, int io_dtype, int state_dtype,
     if (!aligned16(p)) return fail(HIPRWKV_EINVAL, "wkv7_fwd: tensor pointers must be 16-byte aligned");
   }
   if (sa && !aligned16(sa)) return fail(HIPRWKV_EINVAL, "wkv7_fwd: sa must be 16-byte aligned");
+  if (ends && (!aligned16(ends) || !sa || (flags & HIPRWKV_FORCE_SEQ)))
+    return fail(HIPRWKV_EINVAL, "wkv7_fwd: ends must be 16-byte aligned and goes with sa, without HIPRWKV_FORCE_SEQ");
   if (workspace && !aligned16(workspace)) return fail(HIPRWKV_EINVAL, "wkv7_fwd: workspace must be 16-byte aligned");
   const size_t need = workspace != nullptr ? hiprwkv_wkv7_fwd_workspace_bytes(io_dtype, B, T, H, N) : 0;
   if (workspace_bytes < need)
@@ -189,6 +204,10 @@ int hiprwkv_wkv7_fwd_parts(hiprwkv_stream stream, int io_dtype, int state_dtype,
   A.flags = flags;
   A.status = status_word();
   A.parts = need != 0 ? workspace : nullptr;
+  if (ends != nullptr && hiprwkv_wkv7_ends_bytes(io_dtype, B, T, H, N) != 0) {
+    const Wkv7BwdSplit S = wkv7_bwd_parts(B * H, T);
+    A.ends = static_cast<float*>(ends); A.n_end = S.n_end; A.end_chunks = S.end_chunks;
+  }
   // T <= 8 (decode) runs on the small-T kernel; otherwise the chunked matrix-core kernels (fp16 operands for bf16
   // I/O, fp32 operands for fp32 I/O); HIPRWKV_FORCE_SEQ selects the sequential kernel
   const bool small_t = T <= HIPRWKV_SMALL_T && !(flags & HIPRWKV_NO_SMALL_T);
@@ -245,6 +264,20 @@ int hiprwkv_wkv7_bwd(hiprwkv_stream stream, int io_dtype, int state_dtype, int64
                      const void* s, const uint32_t* length, const uint8_t* new_starts, const void* gy, const void* sa,
                      const void* gs_out, void* gw, void* gr, void* gk, void* gv, void* ga, void* gb, void* gs,
                      void* workspace, size_t workspace_bytes, unsigned flags) {
+  return hiprwkv_wkv7_bwd_ends(stream, io_dtype, state_dtype, B, T, H, N, w, r, k, v, a, b, s, length, new_starts, gy, sa, gs_out,
+                               nullptr, gw, gr, gk, gv, ga, gb, gs, workspace, workspace_bytes, flags);
+}
+
+size_t hiprwkv_wkv7_bwd_ends_workspace_bytes(int io_dtype, int64_t B, int64_t T, int64_t H, int64_t N) {
+  const size_t base = hiprwkv_wkv7_bwd_workspace_bytes(B, T, H, N), ends = hiprwkv_wkv7_ends_bytes(io_dtype, B, T, H, N);
+  return ends == 0 ? base : base + 16 + ends + wkv7_bwd_sums_bytes(B * H, wkv7_bwd_parts(B * H, T));
+}
+
+int hiprwkv_wkv7_bwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype, int64_t B, int64_t T, int64_t H, int64_t N,
+                          const void* w, const void* r, const void* k, const void* v, const void* a, const void* b,
+                          const void* s, const uint32_t* length, const uint8_t* new_starts, const void* gy, const void* sa,
+                          const void* gs_out, const void* ends, void* gw, void* gr, void* gk, void* gv, void* ga, void* gb,
+                          void* gs, void* workspace, size_t workspace_bytes, unsigned flags) {
   int rc = check_matrix_shape("wkv7_bwd", io_dtype, state_dtype, B, T, H, N);
   if (rc) return rc;
   if ((rc = check_flags("wkv7_bwd", flags)) != HIPRWKV_OK) return rc;
@@ -253,7 +286,10 @@ int hiprwkv_wkv7_bwd(hiprwkv_stream stream, int io_dtype, int state_dtype, int64
     if (p == nullptr) return fail(HIPRWKV_EINVAL, "wkv7_bwd: null tensor pointer");
     if (!aligned16(p)) return fail(HIPRWKV_EINVAL, "wkv7_bwd: tensor pointers must be 16-byte aligned");
   }
-  const size_t need = hiprwkv_wkv7_bwd_workspace_bytes(B, T, H, N);
+  if (ends && (!aligned16(ends) || (flags & HIPRWKV_FORCE_SEQ)))
+    return fail(HIPRWKV_EINVAL, "wkv7_bwd: ends must be 16-byte aligned and does not go with HIPRWKV_FORCE_SEQ");
+  const size_t base = hiprwkv_wkv7_bwd_workspace_bytes(B, T, H, N);
+  const size_t need = ends != nullptr ? hiprwkv_wkv7_bwd_ends_workspace_bytes(io_dtype, B, T, H, N) : base;
   if (workspace_bytes < need)
     return fail(HIPRWKV_ENOSPACE, "wkv7_bwd: workspace has %zu bytes, %zu needed", workspace_bytes, need);
   Wkv7Args A;
@@ -266,8 +302,17 @@ int hiprwkv_wkv7_bwd(hiprwkv_stream stream, int io_dtype, int state_dtype, int64
   A.status = status_word();
   A.gy = gy; A.sa_in = sa; A.gs_out = gs_out;
   A.gw = gw; A.gr = gr; A.gk = gk; A.gv = gv; A.ga = ga; A.gb = gb; A.gs = gs;
-  const size_t one = need / 3 - PHASE_SPAN;
+  const size_t one = base / 3 - PHASE_SPAN;
   char* ws = static_cast<char*>(workspace);
+  A.n_end = 1; A.end_chunks = (int)((T + 15) / 16);
+  if (const size_t bytes = ends != nullptr ? hiprwkv_wkv7_ends_bytes(io_dtype, B, T, H, N) : 0) {
+    const Wkv7BwdSplit S = wkv7_bwd_parts(B * H, T);
+    A.n_end = S.n_end; A.end_chunks = S.end_chunks;
+    A.ends = const_cast<float*>(static_cast<const float*>(ends));
+    char* const more = ws + (base + 15) / 16 * 16;
+    A.gends = reinterpret_cast<float*>(more);
+    if (S.a_parts) { A.parts = more + bytes; A.n_part = S.n_end; A.part_chunks = S.end_chunks; }
+  }
   A.dsa = reinterpret_cast<float*>(at_phase(ws, r, 3));
   A.e2 = reinterpret_cast<float*>(at_phase(reinterpret_cast<char*>(A.dsa) + one, r, 5));
   A.e3 = reinterpret_cast<float*>(at_phase(reinterpret_cast<char*>(A.e2) + one, r, 7));

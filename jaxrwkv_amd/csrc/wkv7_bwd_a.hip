@@ -35,6 +35,7 @@
 // to a total of -80, so that 1/E_s stays finite in fp32 (cap_chunk_decay), as in the forward kernel.
 #include "chunk_common.h"
 #include "wkv_args.h"
+#include "wkv7_parts.h"
 
 namespace hiprwkv {
 
@@ -83,6 +84,7 @@ struct Raw {
 };
 
 // Loads always touch a valid token (the last one of the sequence for lanes beyond it); mask_raw zeroes those lanes.
+template <int MODE>
 __device__ __forceinline__ void load_raw(Raw& x, const Wkv7Args& A, int64_t b, int64_t h, int64_t c0, int lane) {
   const int t = lane & 15, g = lane >> 4;
   const int64_t tok = (c0 + t < A.T) ? c0 + t : A.T - 1;
@@ -91,7 +93,8 @@ __device__ __forceinline__ void load_raw(Raw& x, const Wkv7Args& A, int64_t b, i
     o[0] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(p) + off);
     o[1] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(p) + off + 64);
   };
-  ld(A.r, x.r); ld(A.w, x.w); ld(A.k, x.k); ld(A.gy, x.v); ld(A.a, x.a); ld(A.b, x.b);
+  if (MODE != SUMMARY) ld(A.k, x.k);
+  ld(A.r, x.r); ld(A.w, x.w); ld(A.gy, x.v); ld(A.a, x.a); ld(A.b, x.b);
 }
 __device__ __forceinline__ void mask_raw(Raw& x, int nvalid, int lane) {
   if (nvalid != CK) {
@@ -111,7 +114,8 @@ struct Producer {
 
 // Everything of one chunk that does not depend on the carried state.  The two 32-key halves go through the
 // same pipeline one after the other (scan, scaling, hi/lo split, LDS parking, transposes, partial Gram sums),
-// which keeps the live register set small.
+// which keeps the live register set small.  SUMMARY: without what only gv needs (k and its products).
+template <int MODE>
 __device__ __forceinline__ void produce(const Producer& P, const Raw& x, const ChunkFlags& F, Slot* __restrict__ slot,
                                         SnapSlot* __restrict__ snap, unsigned* events) {
   const int lane = P.lane, t = lane & 15, g = lane >> 4;
@@ -197,7 +201,8 @@ __device__ __forceinline__ void produce(const Producer& P, const Raw& x, const C
     u32x4_t at_h, at_l, qt_h, qt_l, kh_h, kh_l, bh_h, bh_l;
     {
       float fr[8], fk[8], fb[8], Einv[8], Ee[8];
-      unpack8(x.r[hf], fr); unpack8(x.k[hf], fk); unpack8(x.b[hf], fb);
+      unpack8(x.r[hf], fr); unpack8(x.b[hf], fb);
+      if (MODE != SUMMARY) unpack8(x.k[hf], fk);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const float l2 = fmaxf(E[e], MIN_CUM_L2);
@@ -213,7 +218,7 @@ __device__ __forceinline__ void produce(const Producer& P, const Raw& x, const C
         uint32_t hi, lo;
         split2(fa[e] * Ee[e], fa[e + 1] * Ee[e + 1], hi, lo); at_h[j] = hi; at_l[j] = lo;
         split2(fr[e] * E[e], fr[e + 1] * E[e + 1], hi, lo); qt_h[j] = hi; qt_l[j] = lo;
-        split2(fk[e] * Einv[e], fk[e + 1] * Einv[e + 1], hi, lo); kh_h[j] = hi; kh_l[j] = lo;
+        if (MODE != SUMMARY) { split2(fk[e] * Einv[e], fk[e + 1] * Einv[e + 1], hi, lo); kh_h[j] = hi; kh_l[j] = lo; }
         split2(fb[e] * Einv[e], fb[e + 1] * Einv[e + 1], hi, lo); bh_h[j] = hi; bh_l[j] = lo;
       }
     }
@@ -241,17 +246,17 @@ __device__ __forceinline__ void produce(const Producer& P, const Raw& x, const C
       };
       if (!slow) {
         put(slot->AQ[0][0][t], r0h, true); put(slot->AQ[1][0][t], r0l, true);
-        put(slot->AQ[0][1][t], r1h, true); put(slot->AQ[1][1][t], r1l, true);
+        if (MODE != SUMMARY) { put(slot->AQ[0][1][t], r1h, true); put(slot->AQ[1][1][t], r1l, true); }
       } else {
         rare_path();
         put(slot->AQ[0][0][t], r0h, row0_keep); put(slot->AQ[1][0][t], r0l, row0_keep);
-        put(slot->AQ[0][1][t], r1h, row1_keep); put(slot->AQ[1][1][t], r1l, row1_keep);
+        if (MODE != SUMMARY) { put(slot->AQ[0][1][t], r1h, row1_keep); put(slot->AQ[1][1][t], r1l, row1_keep); }
       }
       if (F.snap >= 0) {
         rare_path();
         const bool sk = (keep_snap >> t) & 1u;
         put(snap->AQ[0][0][t], r0h, sk); put(snap->AQ[1][0][t], r0l, sk);
-        put(snap->AQ[0][1][t], r1h, sk); put(snap->AQ[1][1][t], r1l, sk);
+        if (MODE != SUMMARY) { put(snap->AQ[0][1][t], r1h, sk); put(snap->AQ[1][1][t], r1l, sk); }
       }
     }
     // ---- transposed update operands of key tiles 2hf, 2hf+1 by MFMA (at^T,
@@ -279,13 +284,14 @@ __device__ __forceinline__ void produce(const Producer& P, const Raw& x, const C
     // ---- partial Gram sums over this half's keys (accumulator layout: column n = lane%16, rows 4g..4g+3)
 #pragma unroll
     for (int part = 0; part < 3; ++part) {
-      const u32x4_t bA = part == 2 ? bh_l : bh_h, kA = part == 2 ? kh_l : kh_h;
+      const u32x4_t bA = part == 2 ? bh_l : bh_h;
       const u32x4_t aA = part == 2 ? at_l : at_h, qA = part == 2 ? qt_l : qt_h;
-      const u32x4_t aB = part == 1 ? at_l : at_h, qB = part == 1 ? qt_l : qt_h;
+      const u32x4_t aB = part == 1 ? at_l : at_h;
       const u32x4_t bB = part == 1 ? bh_l : bh_h, kB = part == 1 ? kh_l : kh_h;
       Gab = mfma(bA, aB, Gab);      // [m][n] = bh_m . at_n
       GabT = mfma(aA, bB, GabT);    // [m][n] = at_m . bh_n
       G1 = mfma(qA, bB, G1);      // Mbr^T[m][n] = qt_m . bh_n
+      if (MODE == SUMMARY) continue;
       G2 = mfma(aA, kB, G2);      // Mka^T[m][n] = at_m . kh_n
       G3 = mfma(qA, kB, G3);      // Mkr^T[m][n] = qt_m . kh_n
     }
@@ -338,7 +344,8 @@ __device__ __forceinline__ void produce(const Producer& P, const Raw& x, const C
     split2(d[2], d[3], hi1, lo1);
     slot->Mt[which][lane] = make_uint4(hi0, hi1, lo0, lo1);
   };
-  park(0, Pm); park(1, G1); park(2, G2); park(3, G3);
+  park(0, Pm); park(1, G1);
+  if (MODE != SUMMARY) { park(2, G2); park(3, G3); }
   if (lane == 0) {
     slot->snap = F.snap;
     slot->keep_end = (lastseg == 0) ? 1 : 0;
@@ -365,25 +372,27 @@ struct Ops {
   int keep_end;
 };
 
+template <int MODE>
 __device__ __forceinline__ void load_aq(Ops& o, const Slot* __restrict__ slot, int q, int lane) {
   const int n = lane & 15, g = lane >> 4;
 #pragma unroll
   for (int pl = 0; pl < 2; ++pl)
 #pragma unroll
-    for (int ar = 0; ar < 2; ++ar)
+    for (int ar = 0; ar < (MODE == SUMMARY ? 1 : 2); ++ar)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
         o.aq[pl][ar][j] = *reinterpret_cast<const u32x4_t*>(&slot->AQ[pl][ar][n][32 * j + 8 * g]);
   o.Ka = *reinterpret_cast<const u32x4_t*>(&slot->Mt[1][lane]);
-  o.Kr = *reinterpret_cast<const u32x4_t*>(&slot->Mt[3][lane]);
+  if (MODE != SUMMARY) o.Kr = *reinterpret_cast<const u32x4_t*>(&slot->Mt[3][lane]);
   const uint2 v0 = slot->VT[q][lane];
   o.vv = u32x4_t{v0.x, v0.y, v0.x, v0.y};
   o.keep_end = slot->keep_end;
 }
+template <int MODE>
 __device__ __forceinline__ void load_ops(Ops& o, const Slot* __restrict__ slot, int q, int lane) {
-  load_aq(o, slot, q, lane);
+  load_aq<MODE>(o, slot, q, lane);
   o.T = *reinterpret_cast<const u32x4_t*>(&slot->Mt[0][lane]);
-  o.Br = *reinterpret_cast<const u32x4_t*>(&slot->Mt[2][lane]);
+  if (MODE != SUMMARY) o.Br = *reinterpret_cast<const u32x4_t*>(&slot->Mt[2][lane]);
 }
 
 // Uniform output cursors of a consumer, moved by one chunk per call.
@@ -417,12 +426,13 @@ __device__ __forceinline__ void store_state_tile(void* p, int f32, size_t off, c
 }
 
 // The state-dependent part of one chunk.  `next` is the slot of the chunk handled after this one (null after the
-// last one); `next_ready` waits until its producer has published it.
-template <class WaitNext>
+// last one); `next_ready` waits until its producer has published it.  `emit` (PART only): whether the chunk's outputs are this
+// workgroup's to write.
+template <int MODE, class WaitNext>
 __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restrict__ slot,
                                         const Slot* __restrict__ next, const SnapSlot* __restrict__ snapslot,
                                         const Wkv7Args& A, int64_t b, int64_t h, int nvalid, bool is_snap, bool q2drop,
-                                        OutCursor& oc, WaitNext&& next_ready) {
+                                        bool emit, OutCursor& oc, WaitNext&& next_ready) {
   const int lane = C.lane, n = lane & 15, g = lane >> 4;
   const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
   // update operands of this chunk: needed last, so their latency hides behind the W / SA chain
@@ -454,12 +464,12 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
   f32x4_t W = zero4, Y = zero4;   // [token 4g+i][value n], two interleaved accumulation chains
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    W = mfma(o.aq[0][0][j], Sh[j], W); Y = mfma(o.aq[0][1][j], Sh[j], Y);
-    W = mfma(o.aq[0][0][j], Sl[j], W); Y = mfma(o.aq[0][1][j], Sl[j], Y);
-    W = mfma(o.aq[1][0][j], Sh[j], W); Y = mfma(o.aq[1][1][j], Sh[j], Y);
+    W = mfma(o.aq[0][0][j], Sh[j], W); if (MODE != SUMMARY) Y = mfma(o.aq[0][1][j], Sh[j], Y);
+    W = mfma(o.aq[0][0][j], Sl[j], W); if (MODE != SUMMARY) Y = mfma(o.aq[0][1][j], Sl[j], Y);
+    W = mfma(o.aq[1][0][j], Sh[j], W); if (MODE != SUMMARY) Y = mfma(o.aq[1][1][j], Sh[j], Y);
   }
   W = mfma(o.Ka, o.vv, W);                    // W += Mka^T V^T (hi and lo parts side by side)
-  Y = mfma(o.Kr, o.vv, Y);                    // Y += Mkr^T V^T
+  if (MODE != SUMMARY) Y = mfma(o.Kr, o.vv, Y);                    // Y += Mkr^T V^T
   const u32x4_t vv = o.vv;
   // a reset inside the chunk cuts the cotangent of later chunks off from the chunk start
   if (!keep_end) {
@@ -486,11 +496,15 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
       }
       const u32x4_t a0h = *reinterpret_cast<const u32x4_t*>(&snapslot->AQ[0][0][n][32 * j + 8 * g]);
       const u32x4_t a0l = *reinterpret_cast<const u32x4_t*>(&snapslot->AQ[1][0][n][32 * j + 8 * g]);
+      W = mfma(a0h, gh, W);
+      W = mfma(a0h, gl, W);
+      W = mfma(a0l, gh, W);
+      if (MODE == SUMMARY) continue;
       const u32x4_t a1h = *reinterpret_cast<const u32x4_t*>(&snapslot->AQ[0][1][n][32 * j + 8 * g]);
       const u32x4_t a1l = *reinterpret_cast<const u32x4_t*>(&snapslot->AQ[1][1][n][32 * j + 8 * g]);
-      W = mfma(a0h, gh, W); Y = mfma(a1h, gh, Y);
-      W = mfma(a0h, gl, W); Y = mfma(a1h, gl, Y);
-      W = mfma(a0l, gh, W); Y = mfma(a1l, gh, Y);
+      Y = mfma(a1h, gh, Y);
+      Y = mfma(a1h, gl, Y);
+      Y = mfma(a1l, gh, Y);
     }
   }
 
@@ -498,7 +512,7 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
   bool ok = true;
   if (next != nullptr) {
     ok = next_ready();
-    load_aq(o, next, C.q, lane);
+    load_aq<MODE>(o, next, C.q, lane);
   }
   uint32_t h0, l0, h1, l1;
   split2(W[0], W[1], h0, l0);
@@ -515,9 +529,11 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
   split2(SA[0], SA[1], h0, l0);
   split2(SA[2], SA[3], h1, l1);
   const u32x4_t sHH = {h0, h1, h0, h1}, sL0 = {l0, l1, 0u, 0u};
-  Y = mfma(o.Br, sHH, Y);
-  Y = mfma(o.Br, sL0, Y);                     // Y^T += Mbr^T SA^T
-  if (next != nullptr) o.Br = *reinterpret_cast<const u32x4_t*>(&next->Mt[2][lane]);
+  if (MODE != SUMMARY) {
+    Y = mfma(o.Br, sHH, Y);
+    Y = mfma(o.Br, sL0, Y);                   // Y^T += Mbr^T SA^T
+  }
+  if (MODE != SUMMARY && next != nullptr) o.Br = *reinterpret_cast<const u32x4_t*>(&next->Mt[2][lane]);
   // update, tile by tile: rows = keys.  G <- Gh + At^T DSA^T + Qt^T DY^T
 #pragma unroll
   for (int tile = 0; tile < 4; ++tile) {
@@ -527,6 +543,7 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
     acc = mfma(bt[0][tile], sL0, acc);
     C.S[tile] = acc;
   }
+  if (MODE == SUMMARY) return ok;
   // outputs: register i is token 4g+i, lanes n = 16 consecutive values
   const uint32_t y01 = pack_rn(Y[0], Y[1]), y23 = pack_rn(Y[2], Y[3]);
   char* const yl = oc.y + (size_t)oc.voff * 2;
@@ -534,9 +551,11 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
   // bytes of fp32; the exponent goes to a side array.
   const int kexp = dsa_scale_exponent(SA);
   const uint32_t d01 = pack_dsa2(SA[0], SA[1], kexp), d23 = pack_dsa2(SA[2], SA[3], kexp);
-  if (lane == 0) *oc.scale = kexp;
   char* const sl = oc.sa + (size_t)oc.voff * 2;
-  if (nvalid == CK) {
+  if (MODE == PART && !emit) {
+    rare_path();
+  } else if (nvalid == CK) {
+    if (lane == 0) *oc.scale = kexp;
     *reinterpret_cast<uint16_t*>(yl) = (uint16_t)(y01 & 0xffffu);
     *reinterpret_cast<uint16_t*>(yl + oc.tok_bytes) = (uint16_t)(y01 >> 16);
     *reinterpret_cast<uint16_t*>(yl + 2 * oc.tok_bytes) = (uint16_t)(y23 & 0xffffu);
@@ -546,6 +565,7 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
     *reinterpret_cast<uint16_t*>(sl + 2 * oc.tok_bytes) = (uint16_t)(d23 & 0xffffu);
     *reinterpret_cast<uint16_t*>(sl + 3 * oc.tok_bytes) = (uint16_t)(d23 >> 16);
   } else {
+    if (lane == 0) *oc.scale = kexp;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if (4 * g + i < nvalid) {
@@ -565,9 +585,14 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
 }  // namespace
 
 // Chunks are handled from the last one down; step j
-// handles chunk c(j) = nch - 1 - j in slot j % RING.  Producer p fills the slot once every consumer has released step j - RING,
+// handles chunk c(j) = c1 - 1 - j in slot j % RING.  Producer p fills the slot once every consumer has released step j - RING,
 // then publishes ready = j + 1; consumers take the steps in order.  Every wait is for a strictly earlier step, so
 // the hand-shake cannot cycle.
+//
+// MODE as in wkv7_fwd.hip, run backwards in time: where (sequence, head) workgroups leave most of the GPU idle, a first launch makes
+// the summaries of all parts but the first (G = 0 or the identity with dy = 0 behind the part), a second one folds those of the
+// parts after its own and runs.  Measured: see wkv7_bwd_parts.
+template <int MODE>
 __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_bwd_a_kernel(Wkv7Args A) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Slot* slots = reinterpret_cast<Slot*>(smem_raw);
@@ -575,17 +600,34 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_bwd_a_kernel(Wkv7Ar
   Sync* sy = reinterpret_cast<Sync*>(smem_raw + RING * sizeof(Slot) + sizeof(SnapSlot));
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int64_t b = blockIdx.x / A.H, h = blockIdx.x % A.H;
+  // head, part (0: the last of the sequence) and (SUMMARY) which half of the summary
+  const int per_head = MODE == SUMMARY ? 2 * A.n_part - 3 : MODE == PART ? A.n_part : 1;
+  const int64_t head = MODE == WHOLE ? (int64_t)blockIdx.x : (int64_t)(blockIdx.x / per_head);
+  const int unit = MODE == WHOLE ? 0 : (int)(blockIdx.x % per_head);
+  const bool map = MODE == SUMMARY && unit >= A.n_part - 1;           // this workgroup makes M
+  const int part = MODE == SUMMARY && map ? unit - (A.n_part - 2) : unit;
+  const int64_t b = head / A.H, h = head % A.H;
   int64_t L = seq_length(A.length, b, A.T, A.flags);
   L = L < A.T ? L : A.T;
   const int nch = (int)((A.T + CK - 1) / CK);
+  // chunks c1 - 1 down to c0; output from chunk c_out - 1 on
+  int c0 = 0, c1 = nch, c_out = nch, part0 = 0;
+  if (MODE != WHOLE) {
+    auto upto = [&](int p) { const int e = (A.n_part - p) * A.part_chunks; return e < nch ? e : nch; };
+    part0 = MODE == PART && part > 0 ? first_unusable(A, head, part, lane) : part;
+    c0 = (A.n_part - 1 - part) * A.part_chunks;
+    c1 = upto(part0);
+    c_out = upto(part);
+  }
+  const int n = c1 - c0;
   // the returned state is the reset state there (associative-scan rule), a constant
   const bool q2drop = (A.flags & 1u) && L < A.T && A.ns != nullptr && A.ns[b * A.T + L] != 0;
   // reverse sweep: does a cotangent of the returned state enter at token length-1?
-  const bool inject = A.gs_out != nullptr && !q2drop;
+  const bool inject = A.gs_out != nullptr && !q2drop && !map;
   if (threadIdx.x < sizeof(Sync) / sizeof(int)) reinterpret_cast<int*>(sy)[threadIdx.x] = 0;
   __syncthreads();
 
+  int unusable = 0;                       // SUMMARY: this wave's word
   if (wave < NCONS) {
     // the chunk-to-chunk dependency runs through the consumers: let them issue ahead of the producers
     __builtin_amdgcn_s_setprio(3);
@@ -593,43 +635,62 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_bwd_a_kernel(Wkv7Ar
     C.q = wave;
     C.lane = lane;
     const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
+    if (MODE == PART && part0 > 0) {
+      fold_parts(C.S, wave, lane, A, head, part0);
+    } else {
 #pragma unroll
-    for (int tile = 0; tile < 4; ++tile) C.S[tile] = zero4;
+      for (int tile = 0; tile < 4; ++tile)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          C.S[tile][i] = map && 16 * wave + (lane & 15) == 16 * tile + 4 * (lane >> 4) + i ? 1.f : 0.f;
+    }
 
-    const int64_t first_tok = (int64_t)(nch - 1) * CK;
+    const int64_t first_tok = (int64_t)(c1 - 1) * CK;
     OutCursor oc;
     oc.tok_bytes = (size_t)A.H * 64 * 2;
     const size_t el0 = (((size_t)b * A.T + first_tok) * A.H + h) * 64;
     oc.y = reinterpret_cast<char*>(A.gv) + el0 * 2;
     oc.sa = reinterpret_cast<char*>(A.dsa) + el0 * 2;
-    oc.scale = dsa_scales(A.e3, b, h, A.H, nch, nch - 1) + wave;
+    oc.scale = dsa_scales(A.e3, b, h, A.H, nch, c1 - 1) + wave;
 
     oc.voff = (uint32_t)((4 * (lane >> 4)) * (int)A.H * 64 + 16 * wave + (lane & 15));
     const int csnap = (L >= 1 && inject) ? (int)((L - 1) / CK) : -1;
+    // the next chunk whose entering cotangent sweep C starts a part from (below the workgroup's first chunk: none)
+    int end = -1;
+    if (MODE != SUMMARY && A.gends != nullptr) end = (c_out - 1) / A.end_chunks * A.end_chunks;
     Ops ops;
     bool ok = true;
-    if (nch > 0) {
+    if (n > 0) {
       ok = wait_ready(sy, 0, 1);
-      load_ops(ops, &slots[0], wave, lane);
+      load_ops<MODE>(ops, &slots[0], wave, lane);
     }
-    for (int j = 0; j < nch && ok; ++j) {
-      const int c = nch - 1 - j;
+    for (int j = 0; j < n && ok; ++j) {
+      const int c = c1 - 1 - j;
       const int nvalid = (c + 1 < nch || A.T % CK == 0) ? CK : (int)(A.T % CK);
       const int si = j % RING, sn = (j + 1) % RING;
-      const Slot* next = (j + 1 < nch) ? &slots[sn] : nullptr;
-      ok = consume(C, ops, &slots[si], next, snapslot, A, b, h, nvalid, c == csnap, q2drop, oc,
+      const Slot* next = (j + 1 < n) ? &slots[sn] : nullptr;
+      ok = consume<MODE>(C, ops, &slots[si], next, snapslot, A, b, h, nvalid, c == csnap, q2drop, c < c_out, oc,
                         [&]() { return wait_ready(sy, sn, j + 2); });
       // every LDS read of slot si has returned: its data went into the MFMAs above
       if (lane == 0) __hip_atomic_store(&sy->consumed[wave][si], j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (MODE != SUMMARY && c == end && end > 0) {
+        rare_path();
+        store_end(C.S, wave, lane, A.gends, A, head, end / A.end_chunks, end_kept(A, b, c));
+        end -= A.end_chunks;
+      }
     }
-    // cotangent of the input state; with length == 0 the returned state is the input state itself
-    const bool pass = L == 0 && inject;
+    if (MODE == SUMMARY) {
+      unusable = store_summary(C.S, wave, lane, *part_sum(A, head, part), map);
+    } else if (c0 == 0) {
+      // cotangent of the input state; with length == 0 the returned state is the input state itself
+      const bool pass = L == 0 && inject;
 #pragma unroll
-    for (int tile = 0; tile < 4; ++tile) {
-      const size_t off = state_off(A, b, h, wave, lane, tile);
-      f32x4_t gsv = C.S[tile];
-      if (pass) gsv += load_state_tile(A.gs_out, A.st_f32, off);
-      store_state_tile(A.gs, A.st_f32, off, gsv);
+      for (int tile = 0; tile < 4; ++tile) {
+        const size_t off = state_off(A, b, h, wave, lane, tile);
+        f32x4_t gsv = C.S[tile];
+        if (pass) gsv += load_state_tile(A.gs_out, A.st_f32, off);
+        store_state_tile(A.gs, A.st_f32, off, gsv);
+      }
     }
   } else {
     const int p = wave - NCONS;
@@ -638,47 +699,92 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_bwd_a_kernel(Wkv7Ar
     make_sel(P.sel, lane);
     Raw raw;
     uint32_t ns_mine = 0u;      // this lane's new_starts byte of the chunk loaded next: fetched a step ahead, like the operands
-    if (p < nch) {
-      ns_mine = chunk_flag_prefetch(A.ns, A.T, b, (int64_t)(nch - 1 - p) * CK, lane);
-      load_raw(raw, A, b, h, (int64_t)(nch - 1 - p) * CK, lane);
+    // every chunk counts once: in the launch after the summaries, where its output is written
+    unsigned* events = MODE == SUMMARY || (MODE == PART && part0 != part) ? nullptr : events_word(A.status);
+    if (p < n) {
+      ns_mine = chunk_flag_prefetch(A.ns, A.T, b, (int64_t)(c1 - 1 - p) * CK, lane);
+      load_raw<MODE>(raw, A, b, h, (int64_t)(c1 - 1 - p) * CK, lane);
     }
-    for (int j = p; j < nch; j += NPROD) {
-      const int c = nch - 1 - j;
-      const int64_t c0 = (int64_t)c * CK;
-      ChunkFlags F = chunk_flags_of(A.ns, ns_mine, A.flags, A.T, c0, L);
+    for (int j = p; j < n; j += NPROD) {
+      const int c = c1 - 1 - j;
+      const int64_t t0 = (int64_t)c * CK;
+      ChunkFlags F = chunk_flags_of(A.ns, ns_mine, A.flags, A.T, t0, L);
       if (!inject) F.snap = -1;
       const int si = j % RING;
       Slot* slot = &slots[si];
       if (j >= RING && !wait_consumed(sy, si, j - RING + 1, lane)) break;
       mask_raw(raw, F.nvalid, lane);
-      produce(P, raw, F, slot, snapslot, events_word(A.status));
-      if (j + NPROD < nch) {
+      if (MODE == SUMMARY && map) raw.v[0] = raw.v[1] = make_uint4(0, 0, 0, 0);
+      if (MODE == PART && part0 != part && c < c_out) events = events_word(A.status);
+      produce<MODE>(P, raw, F, slot, snapslot, events);
+      if (j + NPROD < n) {
         ns_mine = chunk_flag_prefetch(A.ns, A.T, b, (int64_t)(c - NPROD) * CK, lane);
-        load_raw(raw, A, b, h, (int64_t)(c - NPROD) * CK, lane);
+        load_raw<MODE>(raw, A, b, h, (int64_t)(c - NPROD) * CK, lane);
       }
-      if ((A.flags & FLAG_DROP_PUBLISH) && j + 1 == nch) break;
+      if ((A.flags & FLAG_DROP_PUBLISH) && j + 1 == n) break;
       // the release orders this wave's LDS writes before the sequence number
       if (lane == 0) __hip_atomic_store(&sy->ready[si], j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
+    if (MODE == SUMMARY) raw.k[0] = raw.k[1] = make_uint4(0, 0, 0, 0);
     retire_loads(raw, ns_mine);
   }
   __syncthreads();
-  if (head_broken(sy, A.status)) {
-    poison_token_rows(A.gv, 2, b, h, A.T, A.H);
+  const bool broken = head_broken(sy, A.status);
+  if (MODE == SUMMARY) {
+    if (wave < NCONS && lane == 0) part_flags(A, head, part)[(map ? 4 : 0) + wave] = unusable | (broken ? 1 : 0);
+    if (wave < NCONS && lane == 0 && !map && part == 0) part_flags(A, head, 0)[4 + wave] = 0;     // part 0 has no M
+  } else if (broken) {
+    const int64_t t0 = (int64_t)c0 * CK, rows = (int64_t)c_out * CK > A.T ? A.T - t0 : (int64_t)c_out * CK - t0;
+    poison_token_rows(A.gv, 2, b, h, A.T, A.H, t0, rows);
     // the workspace of this (sequence, head) reads as NaN for the next two sweeps: every tile gets the reserved exponent
-    for (int i = threadIdx.x; i < nch * NCONS; i += blockDim.x) dsa_scales(A.e3, b, h, A.H, nch, 0)[i] = DSA_BAD;
-    poison_state(A.gs, A.st_f32, b, h, A.H);
+    for (int i = threadIdx.x; i < (c_out - c0) * NCONS; i += blockDim.x) dsa_scales(A.e3, b, h, A.H, nch, c0)[i] = DSA_BAD;
+    if (A.gends != nullptr) poison_ends(A.gends, A, head, c0, c_out - 1);
+    if (c0 == 0) poison_state(A.gs, A.st_f32, b, h, A.H);
   }
 }
 
-// Reverse sweep of the backward pass: gv, the workspace dsa (cotangent of sa per token) and gs.
-hipError_t launch_wkv7_chunk_bwd_a(const Wkv7Args& A, hipStream_t stream) {
+// Parts of the backward's sweeps, by the time of a launch in units of a chunk's: its workgroups' rounds over 256 CUs times the chunks
+// of a part and START for filling the rings (4 us).  Sweeps B and C need nothing but the boundaries; sweep A needs a launch for
+// the summaries (as many workgroups again) and a fold of FOLD per part, and stays whole where that costs more.  Below a tenth
+// gained by this count the whole sequence was as fast or faster (192 heads of 700 tokens 217 and 222 us, 208 of 1000: 298 and 304).
+constexpr int CUS = 256, MAX_PARTS = 32, START = 4, FOLD = 1;
+Wkv7BwdSplit wkv7_bwd_parts(int64_t heads, int64_t T) {
+  const int64_t nch = (T + CK - 1) / CK;
+  auto rounds = [&](int64_t groups) { return (groups + CUS - 1) / CUS; };
+  Wkv7BwdSplit best = {1, (int)nch, false};
+  int64_t least = 3 * rounds(heads) * (nch + START) * 9 / 10;
+  for (int64_t p = 2; p <= MAX_PARTS && p <= nch; ++p) {
+    const int64_t c = (nch + p - 1) / p, np = (nch + c - 1) / c;
+    if (np < 2) continue;
+    const int64_t whole = rounds(heads) * (nch + START);
+    const int64_t parts = (rounds(heads * (2 * np - 3)) + rounds(heads * np)) * (c + START) + FOLD * np;
+    const int64_t cost = 2 * rounds(heads * np) * (c + START) + (parts < whole ? parts : whole);
+    if (cost < least) { least = cost; best = {(int)np, (int)c, parts < whole}; }
+  }
+  return best;
+}
+size_t wkv7_bwd_sums_bytes(int64_t heads, const Wkv7BwdSplit& S) {
+  return S.a_parts ? (size_t)heads * (S.n_end - 1) * (sizeof(PartSum) + 8 * sizeof(int)) : 0;
+}
+
+namespace {
+template <int MODE>
+hipError_t launch_mode(const Wkv7Args& A, int64_t groups, hipStream_t stream) {
   const size_t smem = RING * sizeof(Slot) + sizeof(SnapSlot) + sizeof(Sync);
   static LdsAttrOnce once;
-  const hipError_t attr = allow_dynamic_lds(once, reinterpret_cast<const void*>(wkv7_bwd_a_kernel), smem);
+  const hipError_t attr = allow_dynamic_lds(once, reinterpret_cast<const void*>(wkv7_bwd_a_kernel<MODE>), smem);
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL(wkv7_bwd_a_kernel, dim3((unsigned)(A.B * A.H)), dim3(64 * (NCONS + NPROD)), smem, stream, A);
+  hipLaunchKernelGGL(wkv7_bwd_a_kernel<MODE>, dim3((unsigned)groups), dim3(64 * (NCONS + NPROD)), smem, stream, A);
   return hipGetLastError();
+}
+}  // namespace
+
+// Reverse sweep of the backward pass: gv, the workspace dsa (cotangent of sa per token) and gs.
+hipError_t launch_wkv7_chunk_bwd_a(const Wkv7Args& A, hipStream_t stream) {
+  const int64_t heads = A.B * A.H;
+  if (A.n_part < 2) return launch_mode<WHOLE>(A, heads, stream);
+  const hipError_t e = launch_mode<SUMMARY>(A, heads * (2 * A.n_part - 3), stream);
+  return e != hipSuccess ? e : launch_mode<PART>(A, heads * A.n_part, stream);
 }
 
 }  // namespace hiprwkv

@@ -22,6 +22,7 @@
 // Range: as in the forward kernel, a chunk's total log decay per channel is capped at -80.
 #include "chunk_common.h"
 #include "wkv_args.h"
+#include "wkv7_parts.h"
 
 namespace hiprwkv {
 
@@ -472,6 +473,10 @@ __device__ __forceinline__ void consume(Consumer& C, const Slot* __restrict__ sl
 // Slot c % RING holds chunk c.  Producer p fills it once every consumer has released chunk c - RING, then
 // publishes ready = c + 1; consumers take chunks in order.  Every wait is for a strictly earlier chunk, so the
 // hand-shake cannot cycle.
+//
+// A workgroup runs one of the sequence's A.n_end parts (one: the whole sequence), from the state that the forward left at the
+// part's first chunk.  The open entry of a part's last token stays without e2 of the next one: the carry that sweep C enters the
+// part with has it (end_carry).
 __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_chunk_bwd_b_kernel(Wkv7Args A) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Slot* slots = reinterpret_cast<Slot*>(smem_raw);
@@ -479,10 +484,14 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_chunk_bwd_b_kernel(
   Sync* sy = reinterpret_cast<Sync*>(smem_raw + RING * sizeof(Slot) + sizeof(SnapSlot));
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int64_t b = blockIdx.x / A.H, h = blockIdx.x % A.H;
+  const int64_t head = blockIdx.x / A.n_end;
+  const int part = (int)(blockIdx.x % A.n_end);
+  const int64_t b = head / A.H, h = head % A.H;
   int64_t L = seq_length(A.length, b, A.T, A.flags);
   L = L < A.T ? L : A.T;
   const int nch = (int)((A.T + CK - 1) / CK);
+  // chunks c_in .. c_in + n - 1
+  const int c_in = part * A.end_chunks, n_own = part + 1 < A.n_end ? A.end_chunks : nch - c_in;
   const bool q2drop = (A.flags & 1u) && L < A.T && A.ns != nullptr && A.ns[b * A.T + L] != 0;
   const bool inject = A.gs_out != nullptr && !q2drop;   // a cotangent of the returned state exists
   if (threadIdx.x < sizeof(Sync) / sizeof(int)) reinterpret_cast<int*>(sy)[threadIdx.x] = 0;
@@ -495,26 +504,31 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_chunk_bwd_b_kernel(
     C.lane = lane;
     C.pend = 0.f;
     const int n = lane & 15, g = lane >> 4;
+    if (part > 0) {
+      load_end_cols(C.S, wave, lane, end_of(A.ends, A, head, part));
+    } else {
 #pragma unroll
-    for (int vt = 0; vt < 4; ++vt)
+      for (int vt = 0; vt < 4; ++vt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        C.S[vt][i] = ld_state_el(A.s, A.st_f32, state_el(A, b, h, 16 * vt + 4 * g + i, 16 * wave + n));
+        for (int i = 0; i < 4; ++i)
+          C.S[vt][i] = ld_state_el(A.s, A.st_f32, state_el(A, b, h, 16 * vt + 4 * g + i, 16 * wave + n));
+    }
     OutCursor oc;
     oc.tok_bytes = (size_t)A.H * 64 * 2;
-    const size_t el0 = (((size_t)b * A.T) * A.H + h) * 64;
+    const size_t el0 = (((size_t)b * A.T + (size_t)c_in * CK) * A.H + h) * 64;
     oc.gr = reinterpret_cast<char*>(A.gr) + el0 * 2;
     oc.ga = reinterpret_cast<char*>(A.ga) + el0 * 2;
-    oc.ef = A.e2 + f_record(b, h, A.H, nch, 0, wave);
+    oc.ef = A.e2 + f_record(b, h, A.H, nch, c_in, wave);
     oc.voff = (uint32_t)((4 * g) * (int)A.H * 64 + 16 * wave + n);
     const int csnap = (L >= 1 && inject) ? (int)((L - 1) / CK) : -1;
-    for (int c = 0; c < nch; ++c) {
+    for (int j = 0; j < n_own; ++j) {
+      const int c = c_in + j;
       const int nvalid = (c + 1 < nch || A.T % CK == 0) ? CK : (int)(A.T % CK);
-      const int si = c % RING;
-      if (!wait_ready(sy, si, c + 1)) break;
-      consume(C, &slots[si], snapslot, A, b, h, nvalid, c == csnap, c == 0, c + 1 == nch, oc);
+      const int si = j % RING;
+      if (!wait_ready(sy, si, j + 1)) break;
+      consume(C, &slots[si], snapslot, A, b, h, nvalid, c == csnap, j == 0, c + 1 == nch, oc);
       // every LDS read of slot si has returned: its data went into the MFMAs and stores above
-      if (lane == 0) __hip_atomic_store(&sy->consumed[wave][si], c + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (lane == 0) __hip_atomic_store(&sy->consumed[wave][si], j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
   } else {
     const int p = wave - NCONS;
@@ -523,35 +537,36 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_chunk_bwd_b_kernel(
     make_sel(P.sel, lane);
     Raw raw;
     uint32_t ns_mine = 0u;      // this lane's new_starts byte of the chunk loaded next: fetched a step ahead, like the operands
-    if (p < nch) {
-      ns_mine = chunk_flag_prefetch(A.ns, A.T, b, (int64_t)p * CK, lane);
-      load_raw(raw, A, b, h, (int64_t)p * CK, lane);
+    if (p < n_own) {
+      ns_mine = chunk_flag_prefetch(A.ns, A.T, b, (int64_t)(c_in + p) * CK, lane);
+      load_raw(raw, A, b, h, (int64_t)(c_in + p) * CK, lane);
     }
-    for (int c = p; c < nch; c += NPROD) {
-      const int64_t c0 = (int64_t)c * CK;
+    for (int j = p; j < n_own; j += NPROD) {
+      const int64_t c0 = (int64_t)(c_in + j) * CK;
       ChunkFlags F = chunk_flags_of(A.ns, ns_mine, A.flags, A.T, c0, L);
       if (!inject) F.snap = -1;
-      const int si = c % RING;
+      const int si = j % RING;
       Slot* slot = &slots[si];
-      if (c >= RING && !wait_consumed(sy, si, c - RING + 1, lane)) break;
+      if (j >= RING && !wait_consumed(sy, si, j - RING + 1, lane)) break;
       produce(P, raw, F, slot, snapslot, events_word(A.status));
-      if (c + NPROD < nch) {
+      if (j + NPROD < n_own) {
         ns_mine = chunk_flag_prefetch(A.ns, A.T, b, c0 + NPROD * CK, lane);
         load_raw(raw, A, b, h, c0 + NPROD * CK, lane);
       }
-      if ((A.flags & FLAG_DROP_PUBLISH) && c + 1 == nch) break;
+      if ((A.flags & FLAG_DROP_PUBLISH) && j + 1 == n_own) break;
       // the release orders this wave's LDS writes before the sequence number
-      if (lane == 0) __hip_atomic_store(&sy->ready[si], c + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (lane == 0) __hip_atomic_store(&sy->ready[si], j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     // (no retire_loads here: measured, this sweep is 5 % slower with it -- its producers are the bottleneck, and
     // keeping their operand registers alive to the end of the loop costs them more than the consumers gain)
   }
   __syncthreads();
   if (head_broken(sy, A.status)) {
-    poison_token_rows(A.gr, 2, b, h, A.T, A.H);
-    poison_token_rows(A.ga, 2, b, h, A.T, A.H);
-    for (size_t i = threadIdx.x; i < (size_t)nch * NCONS * F_REC; i += blockDim.x)
-      A.e2[f_record(b, h, A.H, nch, 0, 0) + i] = __uint_as_float(0x7fc00000u);
+    const int64_t t0 = (int64_t)c_in * CK, rows = part + 1 < A.n_end ? (int64_t)n_own * CK : A.T - t0;
+    poison_token_rows(A.gr, 2, b, h, A.T, A.H, t0, rows);
+    poison_token_rows(A.ga, 2, b, h, A.T, A.H, t0, rows);
+    for (size_t i = threadIdx.x; i < (size_t)n_own * NCONS * F_REC; i += blockDim.x)
+      A.e2[f_record(b, h, A.H, nch, c_in, 0) + i] = __uint_as_float(0x7fc00000u);
   }
 }
 
@@ -560,7 +575,7 @@ hipError_t launch_wkv7_chunk_bwd_b(const Wkv7Args& A, hipStream_t stream) {
   static LdsAttrOnce once;
   const hipError_t attr = allow_dynamic_lds(once, reinterpret_cast<const void*>(wkv7_chunk_bwd_b_kernel), smem);
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL(wkv7_chunk_bwd_b_kernel, dim3((unsigned)(A.B * A.H)), dim3(64 * (NCONS + NPROD)), smem, stream, A);
+  hipLaunchKernelGGL(wkv7_chunk_bwd_b_kernel, dim3((unsigned)(A.B * A.H * A.n_end)), dim3(64 * (NCONS + NPROD)), smem, stream, A);
   return hipGetLastError();
 }
 

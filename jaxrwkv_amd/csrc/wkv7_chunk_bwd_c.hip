@@ -24,6 +24,7 @@
 // Range: as in the forward kernel, a chunk's total log decay per channel is capped at -80.
 #include "chunk_common.h"
 #include "wkv_args.h"
+#include "wkv7_parts.h"
 
 namespace hiprwkv {
 
@@ -505,9 +506,13 @@ __device__ __forceinline__ void consume(Consumer& C, const Slot* __restrict__ sl
 
 }  // namespace
 
-// Step j handles chunk nch-1-j in slot j % RING.  Producer p fills the slot once every consumer has released step
+// Step j handles chunk c_end-1-j in slot j % RING.  Producer p fills the slot once every consumer has released step
 // j - RING, then publishes ready = j + 1; consumers take the steps in order.  Every wait is for a strictly earlier
 // step, so the hand-shake cannot cycle.
+//
+// A workgroup runs one of the sequence's A.n_end parts (one: the whole sequence), from the cotangent G that sweep A left behind the
+// part's last chunk.  c of the token t0 after the part, which the running sum continues with, is <G~_t0, S_{t0-1} diag(d_t0)> per
+// key, and G = G~_t0 diag(d_t0) + dsa_t0 a_t0^T: <G, S_{t0-1}> = c_t0 + e2_t0, with the e2 that sweep B left out of f there.
 __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_chunk_bwd_c_kernel(Wkv7Args A) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Slot* slots = reinterpret_cast<Slot*>(smem_raw);
@@ -515,10 +520,14 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_chunk_bwd_c_kernel(
   Sync* sy = reinterpret_cast<Sync*>(smem_raw + RING * sizeof(Slot) + sizeof(SnapSlot));
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int64_t b = blockIdx.x / A.H, h = blockIdx.x % A.H;
+  const int64_t head = blockIdx.x / A.n_end;
+  const int part = (int)(blockIdx.x % A.n_end);
+  const int64_t b = head / A.H, h = head % A.H;
   int64_t L = seq_length(A.length, b, A.T, A.flags);
   L = L < A.T ? L : A.T;
   const int nch = (int)((A.T + CK - 1) / CK);
+  // chunks c_end - 1 down to c_end - n_own
+  const int c_end = part + 1 < A.n_end ? (part + 1) * A.end_chunks : nch, n_own = c_end - part * A.end_chunks;
   const bool q2drop = (A.flags & 1u) && L < A.T && A.ns != nullptr && A.ns[b * A.T + L] != 0;
   const bool inject = A.gs_out != nullptr && !q2drop;   // a cotangent of the returned state exists
   if (threadIdx.x < sizeof(Sync) / sizeof(int)) reinterpret_cast<int*>(sy)[threadIdx.x] = 0;
@@ -532,20 +541,27 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_chunk_bwd_c_kernel(
     C.carry = 0.f;
     const int n = lane & 15, g = lane >> 4;
     const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
+    if (part + 1 < A.n_end) {
+      f32x4_t S[4];
+      load_end_cols(C.G, wave, lane, end_of(A.gends, A, head, part + 1));
+      load_end_cols(S, wave, lane, end_of(A.ends, A, head, part + 1));
+      C.carry = end_carry(C.G, S);
+    } else {
 #pragma unroll
-    for (int vt = 0; vt < 4; ++vt) C.G[vt] = zero4;
+      for (int vt = 0; vt < 4; ++vt) C.G[vt] = zero4;
+    }
     Cursor cu;
     cu.tok_bytes = (size_t)A.H * 64 * 2;
-    const size_t el0 = (((size_t)b * A.T + (size_t)(nch - 1) * CK) * A.H + h) * 64;
+    const size_t el0 = (((size_t)b * A.T + (size_t)(c_end - 1) * CK) * A.H + h) * 64;
     cu.gk = reinterpret_cast<char*>(A.gk) + el0 * 2;
     cu.gb = reinterpret_cast<char*>(A.gb) + el0 * 2;
     cu.gw = reinterpret_cast<char*>(A.gw) + el0 * 2;
     cu.voff = (uint32_t)((4 * g) * (int)A.H * 64 + 16 * wave + n);
     const int csnap = (L >= 1 && inject) ? (int)((L - 1) / CK) : -1;
     const int tail = (A.T % CK == 0) ? CK : (int)(A.T % CK);
-    for (int j = 0; j < nch; ++j) {
-      const int c = nch - 1 - j;
-      const int nvalid = (j == 0) ? tail : CK;
+    for (int j = 0; j < n_own; ++j) {
+      const int c = c_end - 1 - j;
+      const int nvalid = (c + 1 == nch) ? tail : CK;
       const int si = j % RING;
       if (!wait_ready(sy, si, j + 1)) break;
       consume(C, &slots[si], snapslot, A, b, h, nvalid, c == csnap, cu);
@@ -560,12 +576,12 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_chunk_bwd_c_kernel(
     make_sel(P.sel, lane);
     Raw raw;
     uint32_t ns_mine = 0u;      // this lane's new_starts byte of the chunk loaded next: fetched a step ahead, like the operands
-    if (p < nch) {
-      ns_mine = chunk_flag_prefetch(A.ns, A.T, b, (int64_t)(nch - 1 - p) * CK, lane);
-      load_raw(raw, A, b, h, (int64_t)(nch - 1 - p) * CK, lane);
+    if (p < n_own) {
+      ns_mine = chunk_flag_prefetch(A.ns, A.T, b, (int64_t)(c_end - 1 - p) * CK, lane);
+      load_raw(raw, A, b, h, (int64_t)(c_end - 1 - p) * CK, lane);
     }
-    for (int j = p; j < nch; j += NPROD) {
-      const int c = nch - 1 - j;
+    for (int j = p; j < n_own; j += NPROD) {
+      const int c = c_end - 1 - j;
       const int64_t c0 = (int64_t)c * CK;
       ChunkFlags F = chunk_flags_of(A.ns, ns_mine, A.flags, A.T, c0, L);
       if (!inject) F.snap = -1;
@@ -573,11 +589,11 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_chunk_bwd_c_kernel(
       Slot* slot = &slots[si];
       if (j >= RING && !wait_consumed(sy, si, j - RING + 1, lane)) break;
       produce(P, raw, F, slot, snapslot, events_word(A.status));
-      if (j + NPROD < nch) {
+      if (j + NPROD < n_own) {
         ns_mine = chunk_flag_prefetch(A.ns, A.T, b, (int64_t)(c - NPROD) * CK, lane);
         load_raw(raw, A, b, h, (int64_t)(c - NPROD) * CK, lane);
       }
-      if ((A.flags & FLAG_DROP_PUBLISH) && j + 1 == nch) break;
+      if ((A.flags & FLAG_DROP_PUBLISH) && j + 1 == n_own) break;
       // the release orders this wave's LDS writes before the sequence number
       if (lane == 0) __hip_atomic_store(&sy->ready[si], j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
@@ -585,9 +601,10 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_chunk_bwd_c_kernel(
   }
   __syncthreads();
   if (head_broken(sy, A.status)) {
-    poison_token_rows(A.gk, 2, b, h, A.T, A.H);
-    poison_token_rows(A.gb, 2, b, h, A.T, A.H);
-    poison_token_rows(A.gw, 2, b, h, A.T, A.H);
+    const int64_t t0 = (int64_t)(c_end - n_own) * CK, rows = c_end == nch ? A.T - t0 : (int64_t)n_own * CK;
+    poison_token_rows(A.gk, 2, b, h, A.T, A.H, t0, rows);
+    poison_token_rows(A.gb, 2, b, h, A.T, A.H, t0, rows);
+    poison_token_rows(A.gw, 2, b, h, A.T, A.H, t0, rows);
   }
 }
 
@@ -596,7 +613,7 @@ hipError_t launch_wkv7_chunk_bwd_c(const Wkv7Args& A, hipStream_t stream) {
   static LdsAttrOnce once;
   const hipError_t attr = allow_dynamic_lds(once, reinterpret_cast<const void*>(wkv7_chunk_bwd_c_kernel), smem);
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL(wkv7_chunk_bwd_c_kernel, dim3((unsigned)(A.B * A.H)), dim3(64 * (NCONS + NPROD)), smem, stream, A);
+  hipLaunchKernelGGL(wkv7_chunk_bwd_c_kernel, dim3((unsigned)(A.B * A.H * A.n_end)), dim3(64 * (NCONS + NPROD)), smem, stream, A);
   return hipGetLastError();
 }
 

@@ -31,6 +31,7 @@
 // of -80 (cap_chunk_decay), so that exp(-Lc) stays finite in fp32.
 #include "chunk_common.h"
 #include "wkv_args.h"
+#include "wkv7_parts.h"
 
 namespace hiprwkv {
 
@@ -40,9 +41,6 @@ using namespace chunk;
 
 constexpr int NPROD = 8;          // producer waves; producer p owns chunks p, p + NPROD, ...
 constexpr int RING = 10;          // slots in flight
-
-// What a workgroup does with its sequence (see wkv7_fwd_kernel): all of it, a part's summary, or a part.
-enum { WHOLE = 0, SUMMARY = 1, PART = 2 };
 
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x4_t __attribute__((ext_vector_type(4)));
@@ -619,77 +617,6 @@ __device__ __forceinline__ void flush_y(const Slot* __restrict__ slot, const Wkv
   if (r + 8 < nvalid) *reinterpret_cast<uint4*>(y0 + (size_t)8 * A.H * 128) = hi;
 }
 
-// A part's summary: S_end = S_start M + B for the state entering and leaving it, one record per (sequence, head, part) in fp32,
-// laid out as the operands that the fold takes (rows of 256 bytes instead: 64 cycles a KiB, 2.3 us a predecessor), and eight
-// words (one per consumer wave of the two workgroups that make it) that are not zero where the summary must not be used.
-struct PartSum {
-  f32x4_t M[4][4][64];     // [tile][jt], lane (x, g): M[key 16 tile + 4g + i][key 16 jt + x]
-  f32x4_t B[4][4][64];     // [q][tile]: consumer q's state tiles
-};
-constexpr float PART_MAX_GAIN = 4.f;
-__device__ __forceinline__ PartSum* part_sum(const Wkv7Args& A, int64_t head, int part) {
-  return reinterpret_cast<PartSum*>(A.parts) + head * (A.n_part - 1) + part;
-}
-__device__ __forceinline__ int* part_flags(const Wkv7Args& A, int64_t head, int part) {
-  return reinterpret_cast<int*>(reinterpret_cast<PartSum*>(A.parts) + A.B * A.H * (A.n_part - 1)) +
-         (head * (A.n_part - 1) + part) * 8;
-}
-
-// The state entering part `part` > 0, S <- S M + B over the summaries before it, in fp32.  The state tiles are the B operand
-// of the products M^T S^T as they are (k-slot g of step i of a tile is key 16 tile + 4g + i); a predecessor costs a consumer 64
-// instructions of 32 cycles and 20 KiB from the cache.
-__device__ __forceinline__ void fold_parts(Consumer& C, const Wkv7Args& A, int64_t head, int part) {
-#pragma unroll
-  for (int tile = 0; tile < 4; ++tile) C.S[tile] = part_sum(A, head, 0)->B[C.q][tile][C.lane];
-  if (part < 2) return;
-  // a predecessor's 20 KiB are requested while the one before it is multiplied
-  f32x4_t acc[4], m[4][4];
-  auto load_m = [&](int p, int tile) {
-#pragma unroll
-    for (int jt = 0; jt < 4; ++jt)
-      m[tile][jt] = part_sum(A, head, p)->M[tile][jt][C.lane];
-  };
-#pragma unroll
-  for (int jt = 0; jt < 4; ++jt) acc[jt] = part_sum(A, head, 1)->B[C.q][jt][C.lane];
-#pragma unroll
-  for (int tile = 0; tile < 4; ++tile) load_m(1, tile);
-  for (int p = 1; p < part; ++p) {
-    const int next = p + 1 < part ? p + 1 : p;
-    f32x4_t b[4];
-#pragma unroll
-    for (int jt = 0; jt < 4; ++jt) b[jt] = part_sum(A, head, next)->B[C.q][jt][C.lane];
-#pragma unroll
-    for (int tile = 0; tile < 4; ++tile) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int jt = 0; jt < 4; ++jt) acc[jt] = __builtin_amdgcn_mfma_f32_16x16x4f32(m[tile][jt][i], C.S[tile][i], acc[jt], 0, 0, 0);
-      load_m(next, tile);
-    }
-#pragma unroll
-    for (int jt = 0; jt < 4; ++jt) {
-      C.S[jt] = acc[jt];
-      acc[jt] = b[jt];
-    }
-  }
-}
-// writes a consumer's rows of one half of a summary; not zero if it must not be used
-__device__ __forceinline__ int store_summary(const Consumer& C, PartSum& ps, bool map) {
-  const int x = C.lane & 15, g = C.lane >> 4;
-  const float limit = map ? PART_MAX_GAIN : 3.0e38f;
-  bool bad = false;
-#pragma unroll
-  for (int tile = 0; tile < 4; ++tile) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      bad |= !(fabsf(C.S[tile][i]) <= limit);
-      if (map) reinterpret_cast<float*>(&ps.M[C.q][tile][16 * (x >> 2) + 4 * g + i])[x & 3] = C.S[tile][i];
-    }
-    if (!map) ps.B[C.q][tile][C.lane] = C.S[tile];
-  }
-  return __ballot(bad) != 0 ? 1 : 0;
-}
-
 }  // namespace
 
 // Step j handles chunk j in slot j % RING.  Producer p fills the slot once every consumer has released step j - RING,
@@ -733,10 +660,7 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_kernel(Wkv7Args
     const int end = j_out + A.part_chunks < nch ? j_out + A.part_chunks : nch;
     part0 = part;
     if (MODE == PART && part > 0) {
-      // the first part before this one whose summary is not usable; a lane looks at four of its eight words
-      const int4 f = lane < 2 * part ? *reinterpret_cast<const int4*>(part_flags(A, head, 0) + 4 * lane) : make_int4(0, 0, 0, 0);
-      const uint64_t bad = __ballot((f.x | f.y | f.z | f.w) != 0);
-      if (bad != 0) part0 = __builtin_ctzll(bad) >> 1;
+      part0 = first_unusable(A, head, part, lane);
     }
     j0 = part0 * A.part_chunks;
     n = end - j0;
@@ -775,7 +699,7 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_kernel(Wkv7Args
         for (int i = 0; i < 4; ++i)
           C.S[tile][i] = map && 16 * cq + (lane & 15) == 16 * tile + 4 * (lane >> 4) + i ? 1.f : 0.f;
     } else {
-      fold_parts(C, A, head, part0);
+      fold_parts(C.S, C.q, C.lane, A, head, part0);
     }
     // length == 0: the returned state is the input state (rwkv7.py:203), or the reset state under the associative rule
     if (L == 0 && (MODE == WHOLE || (MODE == PART && part == 0))) {
@@ -791,6 +715,8 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_kernel(Wkv7Args
     oc.voff = (uint32_t)((4 * (lane >> 4)) * (int)A.H * 64 + 16 * cq + (lane & 15));
     // the chunk of token length-1, if this workgroup writes the returned state
     const int csnap = MODE != SUMMARY && L >= 1 && (int)((L - 1) / CK) >= j_out ? (int)((L - 1) / CK) - j0 : -1;
+    // the next chunk boundary whose state the backward starts a part from
+    int end = PARK && A.ends != nullptr ? (j_out / A.end_chunks + 1) * A.end_chunks : nch;
     Ops ops;
     bool ok = true;
     if (n > 0) {
@@ -809,10 +735,15 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_kernel(Wkv7Args
                    });
       // every LDS read of slot si has returned: its data went into the MFMAs above
       if (lane == 0) __hip_atomic_store(&sy->consumed[cq][si], j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (PARK && j0 + j + 1 == end && end < nch) {
+        rare_path();
+        store_end(C.S, cq, lane, A.ends, A, head, end / A.end_chunks);
+        end += A.end_chunks;
+      }
       si = sn;
     }
     if (MODE == SUMMARY) {
-      unusable = store_summary(C, *part_sum(A, head, part), map);
+      unusable = store_summary(C.S, C.q, C.lane, *part_sum(A, head, part), map);
     } else if (j0 + n == nch) {
       // an operand beyond the fp16 range leaves inf or NaN in the carried state (until a reset discards it): count it
       count_nonfinite(C.S, lane, events_word(A.status));
@@ -868,6 +799,7 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_kernel(Wkv7Args
     const int64_t t0 = (int64_t)j_out * CK, rows = MODE == WHOLE || (int64_t)(j0 + n) * CK > A.T ? A.T - t0 : (int64_t)(j0 + n) * CK - t0;
     poison_token_rows(A.out, 2, b, h, A.T, A.H, t0, rows);
     poison_token_rows(A.sa, 2, b, h, A.T, A.H, t0, rows);
+    if (PARK && A.ends != nullptr) poison_ends(A.ends, A, head, j_out + 1, j0 + n);
     if (MODE == WHOLE || (L == 0 ? part == 0 : L - 1 >= t0 && L - 1 < t0 + rows)) poison_state(A.new_s, A.st_f32, b, h, A.H);
   }
 }

@@ -1,0 +1,146 @@
+// WKV7 sequences in parts, shared by the chunked kernels (wkv7_fwd.hip, wkv7_bwd_a.hip and their fp32 counterparts).
+//
+// Two things cross the boundary between two parts of a sequence:
+//   * summaries.  The state (in the reverse sweep the cotangent of the state) that leaves a part is an affine map of the one that
+//     enters it, S_end = S_start M + B.  Workgroups of a first launch make M and B of every part, those of a second one fold the
+//     summaries before theirs into their entering state.
+//   * ends.  What a launch carries past a boundary it also leaves in memory: the forward the states (when it keeps `sa`), the
+//     reverse sweep A their cotangents.  Sweeps B and C, which need nothing else from other parts, start from these.
+#pragma once
+#include "chunk_common.h"
+#include "wkv_args.h"
+
+namespace hiprwkv {
+namespace chunk {
+
+// What a workgroup does with its sequence: all of it, a part's summary, or a part.
+enum { WHOLE = 0, SUMMARY = 1, PART = 2 };
+
+// One record per (sequence, head, part) in fp32, laid out as the operands that the fold takes (rows of 256 bytes instead: 64
+// cycles a KiB, 2.3 us a predecessor), and eight words (one per consumer wave of the two workgroups that make it) that are not
+// zero where the summary must not be used.  Parts count in the direction of the sweep.
+struct PartSum {
+  f32x4_t M[4][4][64];     // [tile][jt], lane (x, g): M[key 16 tile + 4g + i][key 16 jt + x]
+  f32x4_t B[4][4][64];     // [q][tile]: consumer q's state tiles
+};
+constexpr float PART_MAX_GAIN = 4.f;
+__device__ __forceinline__ PartSum* part_sum(const Wkv7Args& A, int64_t head, int part) {
+  return reinterpret_cast<PartSum*>(A.parts) + head * (A.n_part - 1) + part;
+}
+__device__ __forceinline__ int* part_flags(const Wkv7Args& A, int64_t head, int part) {
+  return reinterpret_cast<int*>(reinterpret_cast<PartSum*>(A.parts) + A.B * A.H * (A.n_part - 1)) +
+         (head * (A.n_part - 1) + part) * 8;
+}
+// the first part before `part` whose summary is not usable, else `part`; a lane looks at four of its eight words
+__device__ __forceinline__ int first_unusable(const Wkv7Args& A, int64_t head, int part, int lane) {
+  const int4 f = lane < 2 * part ? *reinterpret_cast<const int4*>(part_flags(A, head, 0) + 4 * lane) : make_int4(0, 0, 0, 0);
+  const uint64_t bad = __ballot((f.x | f.y | f.z | f.w) != 0);
+  return bad != 0 ? __builtin_ctzll(bad) >> 1 : part;
+}
+
+// The state entering part `part` > 0, S <- S M + B over the summaries before it, in fp32.  The state tiles are the B operand
+// of the products M^T S^T as they are (k-slot g of step i of a tile is key 16 tile + 4g + i); a predecessor costs a consumer 64
+// instructions of 32 cycles and 20 KiB from the cache.
+__device__ __forceinline__ void fold_parts(f32x4_t (&S)[4], int q, int lane, const Wkv7Args& A, int64_t head, int part) {
+#pragma unroll
+  for (int tile = 0; tile < 4; ++tile) S[tile] = part_sum(A, head, 0)->B[q][tile][lane];
+  if (part < 2) return;
+  // a predecessor's 20 KiB are requested while the one before it is multiplied
+  f32x4_t acc[4], m[4][4];
+  auto load_m = [&](int p, int tile) {
+#pragma unroll
+    for (int jt = 0; jt < 4; ++jt)
+      m[tile][jt] = part_sum(A, head, p)->M[tile][jt][lane];
+  };
+#pragma unroll
+  for (int jt = 0; jt < 4; ++jt) acc[jt] = part_sum(A, head, 1)->B[q][jt][lane];
+#pragma unroll
+  for (int tile = 0; tile < 4; ++tile) load_m(1, tile);
+  for (int p = 1; p < part; ++p) {
+    const int next = p + 1 < part ? p + 1 : p;
+    f32x4_t b[4];
+#pragma unroll
+    for (int jt = 0; jt < 4; ++jt) b[jt] = part_sum(A, head, next)->B[q][jt][lane];
+#pragma unroll
+    for (int tile = 0; tile < 4; ++tile) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int jt = 0; jt < 4; ++jt) acc[jt] = __builtin_amdgcn_mfma_f32_16x16x4f32(m[tile][jt][i], S[tile][i], acc[jt], 0, 0, 0);
+      load_m(next, tile);
+    }
+#pragma unroll
+    for (int jt = 0; jt < 4; ++jt) {
+      S[jt] = acc[jt];
+      acc[jt] = b[jt];
+    }
+  }
+}
+// writes a consumer's rows of one half of a summary; not zero if it must not be used
+__device__ __forceinline__ int store_summary(const f32x4_t (&S)[4], int q, int lane, PartSum& ps, bool map) {
+  const int x = lane & 15, g = lane >> 4;
+  const float limit = map ? PART_MAX_GAIN : 3.0e38f;
+  bool bad = false;
+#pragma unroll
+  for (int tile = 0; tile < 4; ++tile) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      bad |= !(fabsf(S[tile][i]) <= limit);
+      if (map) reinterpret_cast<float*>(&ps.M[q][tile][16 * (x >> 2) + 4 * g + i])[x & 3] = S[tile][i];
+    }
+    if (!map) ps.B[q][tile][lane] = S[tile];
+  }
+  return __ballot(bad) != 0 ? 1 : 0;
+}
+
+// The matrix (64 values x 64 keys, fp32) at the boundary in front of part `part` >= 1 of the backward's parts
+__device__ __forceinline__ float* end_of(float* ends, const Wkv7Args& A, int64_t head, int part) {
+  return ends + (head * (A.n_end - 1) + part - 1) * 4096;
+}
+// consumer q's rows of it (tiles of a value-row split, as in the forward and in sweep A), bits cleared where `kept` is 0
+__device__ __forceinline__ void store_end(const f32x4_t (&S)[4], int q, int lane, float* ends, const Wkv7Args& A, int64_t head, int part,
+                                          uint32_t kept = 0xffffffffu) {
+  float* const p = end_of(ends, A, head, part) + (16 * q + (lane & 15)) * 64 + 4 * (lane >> 4);
+#pragma unroll
+  for (int tile = 0; tile < 4; ++tile)
+    *reinterpret_cast<u32x4_t*>(p + 16 * tile) = u32x4_t{__float_as_uint(S[tile][0]) & kept, __float_as_uint(S[tile][1]) & kept,
+                                                         __float_as_uint(S[tile][2]) & kept, __float_as_uint(S[tile][3]) & kept};
+}
+// For a cotangent in front of chunk c: exactly zero where the chunk starts a sequence (in sweep A what is not finite comes through
+// a reset as 0 times it, in sweep C it does not).  A mask and not a branch: with one, hipcc 7.2 left the first of the sixteen
+// registers unset on the path without a reset.
+__device__ __forceinline__ uint32_t end_kept(const Wkv7Args& A, int64_t b, int c) {
+  return A.ns != nullptr && A.ns[b * A.T + (int64_t)c * CK] != 0 ? 0u : 0xffffffffu;
+}
+// a workgroup whose hand-shake failed: NaN at the boundaries in front of chunks c0 .. c1
+__device__ __forceinline__ void poison_ends(float* ends, const Wkv7Args& A, int64_t head, int c0, int c1) {
+  for (int part = 1; part < A.n_end; ++part) {
+    if (part * A.end_chunks < c0 || part * A.end_chunks > c1) continue;
+    float* const p = end_of(ends, A, head, part);
+    for (int i = threadIdx.x; i < 4096; i += blockDim.x) p[i] = __uint_as_float(0x7fc00000u);
+  }
+}
+// key columns 16q .. of it (tiles of a key-column split, as in sweeps B and C): S[vt][i] = value 16 vt + 4g + i, key 16q + n
+__device__ __forceinline__ void load_end_cols(f32x4_t (&S)[4], int q, int lane, const float* p) {
+#pragma unroll
+  for (int vt = 0; vt < 4; ++vt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S[vt][i] = p[(16 * vt + 4 * (lane >> 4) + i) * 64 + 16 * q + (lane & 15)];
+}
+
+// The running sum of the decay gradient that enters a part of sweep C from the tokens after it (see wkv7_chunk_bwd_c.hip): with G
+// the cotangent of the state S between the parts, sum over the values of G S, one key per lane (all four lanes of a key).
+// Where the next token starts a sequence G is zero, whatever S holds.
+__device__ __forceinline__ float end_carry(const f32x4_t (&G)[4], const f32x4_t (&S)[4]) {
+  float p = 0.f;
+#pragma unroll
+  for (int vt = 0; vt < 4; ++vt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) p += G[vt][i] == 0.f ? 0.f : G[vt][i] * S[vt][i];
+  p += __shfl_xor(p, 16, 64);
+  p += __shfl_xor(p, 32, 64);
+  return p;
+}
+
+}  // namespace chunk
+}  // namespace hiprwkv

@@ -34,12 +34,24 @@ struct Wkv7Args {
   // Elements between the states of consecutive sequences in `s` / `new_s`; 0 = dense (H*64*64).  Honoured by the
   // small-T kernel only (states read and written inside a packed model state).
   int64_t s_bstride, new_s_bstride;
-  // forward, bf16 I/O: workspace for a sequence in parts (wkv7_fwd_parts), null: whole; the launcher sets the other two
+  // workspace for the summaries of a sequence in parts (forward: wkv7_fwd_parts, null: whole, the launcher sets the other two;
+  // sweep A: wkv7_bwd_parts, n_part < 2: whole)
   void* parts;
   int n_part, part_chunks;
+  // The parts of sweeps B and C: n_end of end_chunks chunks.  ends: the states at their boundaries, left by the forward that keeps
+  // sa (null there: none wanted); gends: the cotangents of these, left by sweep A.  (heads, n_end - 1, 64, 64) fp32.
+  float *ends, *gends;
+  int n_end, end_chunks;
 };
 int wkv7_fwd_parts(int64_t heads, int64_t T, int* chunks);
 size_t wkv7_fwd_parts_bytes(int64_t heads, int64_t T);
+// How the backward splits a sequence: n_end parts for sweeps B and C, and whether sweep A runs in these parts too
+struct Wkv7BwdSplit {
+  int n_end, end_chunks;
+  bool a_parts;
+};
+Wkv7BwdSplit wkv7_bwd_parts(int64_t heads, int64_t T);
+size_t wkv7_bwd_sums_bytes(int64_t heads, const Wkv7BwdSplit& S);      // summaries of sweep A
 
 // Wkv6Args::flags bit: w is (H,64), shared by every token and sequence (HIPRWKV_W_PER_HEAD)
 constexpr unsigned FLAG_W_PER_HEAD = 0x10u;

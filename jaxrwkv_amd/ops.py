@@ -153,6 +153,13 @@ def wkv7_fwd(r, w, k, v, a, b, s, length=None, new_starts=None, compat=True, wan
 
     T <= 8 runs on the small-T (decode) kernel unless ``small_t=False``; otherwise on a chunked matrix-core kernel
     (fp16 operands for bf16 I/O, fp32 operands for fp32 I/O); ``force_seq`` selects the sequential fp32 kernel."""
+    return _wkv7_fwd(r, w, k, v, a, b, s, length, new_starts, compat, want_sa, force_seq, small_t, debug_flags)[:3]
+
+
+def _wkv7_fwd(r, w, k, v, a, b, s, length=None, new_starts=None, compat=True, want_sa=False, force_seq=False,
+              small_t=True, debug_flags=0, want_ends=False):
+    """``wkv7_fwd`` with a fourth result: with ``want_ends`` the states that let the backward run the sequence in parts, where that
+    is of use."""
     lib = _lib.load()
     io = r.dtype
     r, w, k, v, a, b = (_dev(x, io) for x in (r, w, k, v, a, b))
@@ -166,11 +173,14 @@ def wkv7_fwd(r, w, k, v, a, b, s, length=None, new_starts=None, compat=True, wan
     sa = _empty_phased((B, T, H, N), _SA_DT[io], r.device, _phase(r) + 2) if want_sa else None
     nbytes = 0 if force_seq else lib.hiprwkv_wkv7_fwd_workspace_bytes(_DT[io], B, T, H, N)
     ws = _workspace(nbytes, r.device) if nbytes else None
-    rc = lib.hiprwkv_wkv7_fwd_parts(_stream(), _DT[io], _DT[s.dtype], B, T, H, N, _p(w), _p(r), _p(k), _p(v), _p(a), _p(b),
-                                    _p(s), _p(length), _p(new_starts), _p(y), _p(sa), _p(new_s), _p(ws), nbytes,
-                                    _flags(compat, force_seq, small_t, debug_flags))
+    ebytes = lib.hiprwkv_wkv7_ends_bytes(_DT[io], B, T, H, N) if want_sa and want_ends and not force_seq else 0
+    ends = _workspace(ebytes, r.device) if ebytes else None
+    fn, more = (lib.hiprwkv_wkv7_fwd_parts, ()) if ends is None else (lib.hiprwkv_wkv7_fwd_ends, (_p(ends),))
+    rc = fn(_stream(), _DT[io], _DT[s.dtype], B, T, H, N, _p(w), _p(r), _p(k), _p(v), _p(a), _p(b),
+            _p(s), _p(length), _p(new_starts), _p(y), _p(sa), _p(new_s), *more, _p(ws), nbytes,
+            _flags(compat, force_seq, small_t, debug_flags))
     _lib.check(rc, "hiprwkv_wkv7_fwd")
-    return new_s, y, sa
+    return new_s, y, sa, ends
 
 
 def _packed_state(t, B, H, N):
@@ -201,10 +211,11 @@ def wkv7_step(r, w, k, v, a, b, s, new_s, length=None, new_starts=None, compat=T
 
 
 def wkv7_bwd(r, w, k, v, a, b, s, length, new_starts, gy, sa, gs_out=None, compat=True, force_seq=False,
-             debug_flags=0):
+             debug_flags=0, ends=None):
     """Cotangents (gr, gw, gk, gv, ga, gb, gs) of ``wkv7_fwd`` for cotangents gy of y and gs_out of new_s.
 
-    bf16 inputs use the chunked MFMA kernels where they exist unless ``force_seq`` asks for the sequential ones."""
+    bf16 inputs use the chunked MFMA kernels where they exist unless ``force_seq`` asks for the sequential ones.  ``ends``: the
+    forward's (``_wkv7_fwd``), for the sequences in parts."""
     lib = _lib.load()
     io = r.dtype
     r, w, k, v, a, b, gy = (_dev(x, io) for x in (r, w, k, v, a, b, gy))
@@ -215,12 +226,16 @@ def wkv7_bwd(r, w, k, v, a, b, s, length, new_starts, gy, sa, gs_out=None, compa
     length, new_starts = _length_ns(length, new_starts, B, T, r.device)
     gw, gr, gk, gv, ga, gb = (_empty_like_phased(r, i) for i in range(1, 7))
     gs = torch.empty_like(s)
-    nbytes = lib.hiprwkv_wkv7_bwd_workspace_bytes(B, T, H, N)
+    if ends is None:
+        fn, more, nbytes = lib.hiprwkv_wkv7_bwd, (), lib.hiprwkv_wkv7_bwd_workspace_bytes(B, T, H, N)
+    else:
+        ends = _aligned(_dev(ends))
+        fn, more, nbytes = lib.hiprwkv_wkv7_bwd_ends, (_p(ends),), lib.hiprwkv_wkv7_bwd_ends_workspace_bytes(_DT[io], B, T, H, N)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=r.device)
-    rc = lib.hiprwkv_wkv7_bwd(_stream(), _DT[io], _DT[s.dtype], B, T, H, N, _p(w), _p(r), _p(k), _p(v), _p(a), _p(b),
-                              _p(s), _p(length), _p(new_starts), _p(gy), _p(sa), _p(gs_out),
-                              _p(gw), _p(gr), _p(gk), _p(gv), _p(ga), _p(gb), _p(gs), _p(ws), nbytes,
-                              _flags(compat, force_seq, debug=debug_flags))
+    rc = fn(_stream(), _DT[io], _DT[s.dtype], B, T, H, N, _p(w), _p(r), _p(k), _p(v), _p(a), _p(b),
+            _p(s), _p(length), _p(new_starts), _p(gy), _p(sa), _p(gs_out), *more,
+            _p(gw), _p(gr), _p(gk), _p(gv), _p(ga), _p(gb), _p(gs), _p(ws), nbytes,
+            _flags(compat, force_seq, debug=debug_flags))
     _lib.check(rc, "hiprwkv_wkv7_bwd")
     return gr, gw, gk, gv, ga, gb, gs
 
@@ -231,19 +246,20 @@ class _Wkv7(torch.autograd.Function):
     @staticmethod
     def forward(ctx, r, w, k, v, a, b, s, length, new_starts, compat, force_seq):
         need = any(x.requires_grad for x in (r, w, k, v, a, b, s))
-        new_s, y, sa = wkv7_fwd(r, w, k, v, a, b, s, length, new_starts, compat, want_sa=need, force_seq=force_seq)
+        new_s, y, sa, ends = _wkv7_fwd(r, w, k, v, a, b, s, length, new_starts, compat, want_sa=need, force_seq=force_seq,
+                                       want_ends=need)
         ctx.compat = compat
         ctx.force_seq = force_seq
-        ctx.save_for_backward(r, w, k, v, a, b, s, length, new_starts, sa)
+        ctx.save_for_backward(r, w, k, v, a, b, s, length, new_starts, sa, ends)
         return new_s, y
 
     @staticmethod
     def backward(ctx, gs_out, gy):
-        r, w, k, v, a, b, s, length, new_starts, sa = ctx.saved_tensors
+        r, w, k, v, a, b, s, length, new_starts, sa, ends = ctx.saved_tensors
         if gy is None:
             gy = torch.zeros_like(r)
         gr, gw, gk, gv, ga, gb, gs = wkv7_bwd(r, w, k, v, a, b, s, length, new_starts, gy, sa, gs_out, ctx.compat,
-                                              ctx.force_seq)
+                                              ctx.force_seq, ends=ends)
         return gr, gw, gk, gv, ga, gb, gs, None, None, None, None
 
 

@@ -1,0 +1,126 @@
+"""The WKV7 backward (bf16 I/O) with its sequences cut into parts (few sequences and heads) against the oracle and against the
+same sweeps over the whole sequence, which run where the forward left no states at the parts' boundaries.
+
+The bounds against the oracle are those of the whole sequence (test_gpu_wkv7_bwd_chunked; long sequences: test_wkv7_long of
+test_gpu_random_shapes).  The parts take two values of their own across a boundary: the state is the forward's, whose operands are
+fp16 (2^-11 each, as those of the residual sa that the whole sequence's state is built from), and the decay gradient's running
+sum is a product of two fp32 matrices instead of a sum over the tokens after.  So rms errors of the two are compared, a tenth
+more is allowed (measured: 0.93 to 1.02)."""
+import numpy as np
+import pytest
+import torch
+
+from tests.gpu_util import dev, host
+from tests.inputs import bf16_round, wkv7_inputs
+from tests.test_gpu_wkv7_bwd_chunked import NAMES, check, oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def run(x, compat, parts=True, gy=None):
+    from jaxrwkv_amd import ops
+    bf = torch.bfloat16
+    t = [dev(x[n], bf) for n in ("r", "w", "k", "v", "a", "b")] + [dev(x["s"]), dev(x["length"]), dev(x["new_starts"])]
+    _, _, sa, ends = ops._wkv7_fwd(*t, compat=compat, want_sa=True, want_ends=parts)
+    assert (ends is not None) == parts
+    g = ops.wkv7_bwd(*t, dev(x["dy"], bf), sa, dev(x["ds"]), compat=compat, ends=ends)
+    torch.cuda.synchronize()
+    return dict(zip(NAMES, (host(z) for z in g)))
+
+
+def boundary(B, T, H):
+    """tokens of a part"""
+    from jaxrwkv_amd import _lib
+    n = _lib.load().hiprwkv_wkv7_ends_bytes(1, B, T, H, 64) // (4096 * 4 * B * H) + 1
+    assert n >= 2
+    return 16 * -(-(-(-T // 16)) // n)
+
+
+@pytest.mark.parametrize("B,T,H,seed,p", [(1, 300, 1, 0, 0.0), (2, 289, 2, 1, 0.01), (3, 333, 12, 2, 0.004), (5, 260, 30, 3, 0.01)])
+@pytest.mark.parametrize("compat", [True, False])
+def test_against_the_oracle(B, T, H, seed, p, compat):
+    n = boundary(B, T, H)
+    x = wkv7_inputs(B, T, H, 64, seed=seed, bf16=True, p_reset=p, min_len_frac=0.0)
+    x["length"][0] = n                                 # the last token of the first part
+    x["new_starts"][-1, n] = True                      # a reset at the first token of the second
+    check(run(x, compat), oracle(x, compat))
+
+
+@pytest.mark.parametrize("L", ["0", "1", "n-1", "n", "n+1", "2n", "T-1", "T"])
+def test_lengths(L):
+    T = 297
+    n = boundary(1, T, 2)
+    x = wkv7_inputs(1, T, 2, 64, seed=7, bf16=True, p_reset=0.003)
+    x["length"][:] = {"0": 0, "1": 1, "n-1": n - 1, "n": n, "n+1": n + 1, "2n": min(2 * n, T), "T-1": T - 1, "T": T}[L]
+    for compat in (True, False):
+        check(run(x, compat), oracle(x, compat))
+
+
+def rms(a):
+    return float(np.sqrt(np.mean(np.square(a))))
+
+
+@pytest.mark.parametrize("decay", [-0.5, -2.5, -5.0, -8.0])
+@pytest.mark.parametrize("B,T,H", [(1, 1024, 2), (4, 777, 12), (3, 512, 40)])
+def test_errors_are_those_of_the_whole_sequence(B, T, H, decay):
+    x = wkv7_inputs(B, T, H, 64, seed=5, bf16=True, resets=False)
+    x["w"] = bf16_round(x["w"] + 0.5 + decay).astype(np.float64)
+    boundary(B, T, H)
+    ref, got, base = oracle(x, True), run(x, True), run(x, True, parts=False)
+    for n in NAMES:
+        new, old = rms(got[n] - ref[n]), rms(base[n] - ref[n])
+        print(f"B{B} T{T} H{H} decay {decay} g{n}: {old / rms(ref[n]):.2e} whole, in parts {new / old:.3f} of it")
+        assert new <= 1.1 * old + 1e-6 * rms(ref[n]), n
+
+
+@pytest.mark.parametrize("gain", [0.03, -0.03])
+def test_summaries_that_amplify_are_not_used(gain):
+    """As in test_gpu_wkv7_parts: a map that grows along one key; the parts before it then run its chunks themselves."""
+    T = 1200
+    n = boundary(1, T, 2)
+    x = wkv7_inputs(1, T, 2, 64, seed=6, bf16=True, resets=False, lengths=False)
+    x["w"][:] = -9.0
+    m = slice(T // 2, T // 2 + 160)
+    x["a"][:, m] = 0.0
+    x["a"][:, m, :, 5] = 1.0
+    x["b"][:, m] = bf16_round(gain * x["a"][:, m])
+    ref, got, base = oracle(x, True), run(x, True), run(x, True, parts=False)
+    for k in NAMES:
+        assert np.isfinite(got[k]).all()
+        assert rms(got[k] - ref[k]) <= 1.1 * rms(base[k] - ref[k]) + 1e-6 * rms(ref[k]), k
+
+
+def test_what_is_not_finite_stays_where_the_whole_sequence_has_it():
+    T = 640
+    n = boundary(1, T, 1)
+    x = wkv7_inputs(1, T, 1, 64, seed=8, bf16=True, resets=False, lengths=False)
+    x["new_starts"][:, n] = x["new_starts"][:, 2 * n + 5] = True
+    x["dy"][:, n + 20, 0, 3] = np.inf
+    got, base = run(x, True), run(x, True, parts=False)
+    for k in NAMES:
+        assert np.array_equal(np.isfinite(got[k]), np.isfinite(base[k])), k
+
+
+def test_numeric_events_count_once():
+    from jaxrwkv_amd import ops
+    x = wkv7_inputs(1, 1200, 1, 64, seed=7, bf16=True, resets=False, lengths=False)
+    x["w"][:, 700:716] = 3.0                            # e^-20 a token: a capped chunk
+
+    def events(parts):
+        before = ops.numeric_events()
+        run(x, True, parts)
+        return ops.numeric_events() - before
+
+    assert events(True) == events(False) > 0
+
+
+def test_autograd_takes_the_parts():
+    from jaxrwkv_amd import ops
+    x = wkv7_inputs(2, 300, 2, 64, seed=9, bf16=True, p_reset=0.01)
+    boundary(2, 300, 2)
+    t = [dev(x[n], torch.bfloat16).requires_grad_() for n in ("r", "w", "k", "v", "a", "b")] + [dev(x["s"]).requires_grad_()]
+    new_s, y = ops.wkv7(*t, dev(x["length"]), dev(x["new_starts"]))
+    g = torch.autograd.grad((y, new_s), t, (dev(x["dy"], torch.bfloat16), dev(x["ds"])))
+    want = run(x, True)
+    for n, z in zip(NAMES, g):
+        assert np.array_equal(host(z), want[n]), n
