@@ -123,7 +123,7 @@ int hiprwkv_wkv7_fwd(hiprwkv_stream stream, int io_dtype, int state_dtype,
                      void* out, void* sa, void* new_s, unsigned flags);
 
 /* The same with `workspace` (hiprwkv_wkv7_fwd_workspace_bytes, 0 where it is of no use; NULL: as hiprwkv_wkv7_fwd).  Where
- * B*H leaves most of the GPU idle, bf16 sequences are cut into parts whose summaries (state maps) are made first.  A
+ * B*H leaves most of the GPU idle, sequences are cut into parts whose summaries (state maps) are made first.  A
  * part whose hand-shake fails counts as one of its own in hiprwkv_handshake_failures and makes its own rows NaN. */
 size_t hiprwkv_wkv7_fwd_workspace_bytes(int io_dtype, int64_t B, int64_t T, int64_t H, int64_t N);
 int hiprwkv_wkv7_fwd_parts(hiprwkv_stream stream, int io_dtype, int state_dtype,

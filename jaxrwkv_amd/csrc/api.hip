@@ -157,9 +157,14 @@ int hiprwkv_wkv7_fwd(hiprwkv_stream stream, int io_dtype, int state_dtype, int64
                                 nullptr, 0, flags);
 }
 
+// whether sequences of this shape may run in parts
+static bool wkv7_in_parts(int io_dtype, int64_t B, int64_t T, int64_t H, int64_t N) {
+  return (io_dtype == HIPRWKV_BF16 || io_dtype == HIPRWKV_F32) && N == 64 && B > 0 && T > HIPRWKV_SMALL_T && H > 0 && B * H <= 0x7fffffffLL;
+}
+
 size_t hiprwkv_wkv7_fwd_workspace_bytes(int io_dtype, int64_t B, int64_t T, int64_t H, int64_t N) {
-  if (io_dtype != HIPRWKV_BF16 || N != 64 || B <= 0 || T <= HIPRWKV_SMALL_T || H <= 0 || B * H > 0x7fffffffLL) return 0;
-  return wkv7_fwd_parts_bytes(B * H, T);
+  if (!wkv7_in_parts(io_dtype, B, T, H, N)) return 0;
+  return wkv7_fwd_parts_bytes(B * H, T, io_dtype == HIPRWKV_F32);
 }
 
 int hiprwkv_wkv7_fwd_parts(hiprwkv_stream stream, int io_dtype, int state_dtype, int64_t B, int64_t T, int64_t H, int64_t N,
@@ -171,8 +176,8 @@ int hiprwkv_wkv7_fwd_parts(hiprwkv_stream stream, int io_dtype, int state_dtype,
 }
 
 size_t hiprwkv_wkv7_ends_bytes(int io_dtype, int64_t B, int64_t T, int64_t H, int64_t N) {
-  if (io_dtype != HIPRWKV_BF16 || N != 64 || B <= 0 || T <= HIPRWKV_SMALL_T || H <= 0 || B * H > 0x7fffffffLL) return 0;
-  return (size_t)(B * H) * (wkv7_bwd_parts(B * H, T).n_end - 1) * 4096 * sizeof(float);
+  if (!wkv7_in_parts(io_dtype, B, T, H, N)) return 0;
+  return (size_t)(B * H) * (wkv7_bwd_parts(B * H, T, io_dtype == HIPRWKV_F32).n_end - 1) * 4096 * sizeof(float);
 }
 
 int hiprwkv_wkv7_fwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype, int64_t B, int64_t T, int64_t H, int64_t N,
@@ -205,7 +210,7 @@ int hiprwkv_wkv7_fwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype, 
   A.status = status_word();
   A.parts = need != 0 ? workspace : nullptr;
   if (ends != nullptr && hiprwkv_wkv7_ends_bytes(io_dtype, B, T, H, N) != 0) {
-    const Wkv7BwdSplit S = wkv7_bwd_parts(B * H, T);
+    const Wkv7BwdSplit S = wkv7_bwd_parts(B * H, T, io_dtype == HIPRWKV_F32);
     A.ends = static_cast<float*>(ends); A.n_end = S.n_end; A.end_chunks = S.end_chunks;
   }
   // T <= 8 (decode) runs on the small-T kernel; otherwise the chunked matrix-core kernels (fp16 operands for bf16
@@ -270,7 +275,7 @@ int hiprwkv_wkv7_bwd(hiprwkv_stream stream, int io_dtype, int state_dtype, int64
 
 size_t hiprwkv_wkv7_bwd_ends_workspace_bytes(int io_dtype, int64_t B, int64_t T, int64_t H, int64_t N) {
   const size_t base = hiprwkv_wkv7_bwd_workspace_bytes(B, T, H, N), ends = hiprwkv_wkv7_ends_bytes(io_dtype, B, T, H, N);
-  return ends == 0 ? base : base + 16 + ends + wkv7_bwd_sums_bytes(B * H, wkv7_bwd_parts(B * H, T));
+  return ends == 0 ? base : base + 16 + ends + wkv7_bwd_sums_bytes(B * H, wkv7_bwd_parts(B * H, T, io_dtype == HIPRWKV_F32));
 }
 
 int hiprwkv_wkv7_bwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype, int64_t B, int64_t T, int64_t H, int64_t N,
@@ -306,7 +311,7 @@ int hiprwkv_wkv7_bwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype, 
   char* ws = static_cast<char*>(workspace);
   A.n_end = 1; A.end_chunks = (int)((T + 15) / 16);
   if (const size_t bytes = ends != nullptr ? hiprwkv_wkv7_ends_bytes(io_dtype, B, T, H, N) : 0) {
-    const Wkv7BwdSplit S = wkv7_bwd_parts(B * H, T);
+    const Wkv7BwdSplit S = wkv7_bwd_parts(B * H, T, io_dtype == HIPRWKV_F32);
     A.n_end = S.n_end; A.end_chunks = S.end_chunks;
     A.ends = const_cast<float*>(static_cast<const float*>(ends));
     char* const more = ws + (base + 15) / 16 * 16;

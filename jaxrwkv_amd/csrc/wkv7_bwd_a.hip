@@ -747,8 +747,12 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_bwd_a_kernel(Wkv7Ar
 // of a part and START for filling the rings (4 us).  Sweeps B and C need nothing but the boundaries; sweep A needs a launch for
 // the summaries (as many workgroups again) and a fold of FOLD per part, and stays whole where that costs more.  Below a tenth
 // gained by this count the whole sequence was as fast or faster (192 heads of 700 tokens 217 and 222 us, 208 of 1000: 298 and 304).
-constexpr int CUS = 256, MAX_PARTS = 32, START = 4, FOLD = 1;
-Wkv7BwdSplit wkv7_bwd_parts(int64_t heads, int64_t T) {
+// A chunk of the fp32 sweeps takes twice as long (2.7 us), so START and FOLD weigh half as much there.  Three sweeps, whole -> parts:
+// bf16 B=1 T=2048 H=32 545 -> 158 us, B=4 T=1024 H=16 287 -> 152, B=4 T=1024 H=32 293 -> 209, B=1 T=64 H=12 42 -> 33; fp32 1000 -> 269,
+// 519 -> 249, 549 -> 388, 57 -> 42.
+constexpr int CUS = 256, MAX_PARTS = 32;
+Wkv7BwdSplit wkv7_bwd_parts(int64_t heads, int64_t T, bool f32) {
+  const int64_t START = f32 ? 2 : 4, FOLD = 1;
   const int64_t nch = (T + CK - 1) / CK;
   auto rounds = [&](int64_t groups) { return (groups + CUS - 1) / CUS; };
   Wkv7BwdSplit best = {1, (int)nch, false};

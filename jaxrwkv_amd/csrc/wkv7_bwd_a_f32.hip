@@ -17,6 +17,7 @@
 // uses a second, masked set of row operands through which the cotangent of the returned state enters.
 #include "chunk_common.h"
 #include "wkv_args.h"
+#include "wkv7_parts.h"
 
 namespace hiprwkv {
 
@@ -70,6 +71,7 @@ struct Raw {
   float4 r[4], w[4], k[4], v[4], a[4], b[4];   // v holds dy
 };
 
+template <int MODE>
 __device__ __forceinline__ void load_raw(Raw& x, const Wkv7Args& A, int64_t b, int64_t h, int64_t c0, int lane) {
   const int t = lane & 15, g = lane >> 4;
   const int64_t tok = (c0 + t < A.T) ? c0 + t : A.T - 1;   // always a valid token; mask_raw zeroes the lanes beyond
@@ -78,7 +80,8 @@ __device__ __forceinline__ void load_raw(Raw& x, const Wkv7Args& A, int64_t b, i
 #pragma unroll
     for (int j = 0; j < 4; ++j) o[j] = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(p) + off + 16 * j);
   };
-  ld(A.r, x.r); ld(A.w, x.w); ld(A.k, x.k); ld(A.gy, x.v); ld(A.a, x.a); ld(A.b, x.b);
+  if (MODE != SUMMARY) ld(A.k, x.k);
+  ld(A.r, x.r); ld(A.w, x.w); ld(A.gy, x.v); ld(A.a, x.a); ld(A.b, x.b);
 }
 __device__ __forceinline__ void mask_raw(Raw& x, int nvalid, int lane) {
   if (nvalid != CK) {
@@ -102,6 +105,7 @@ __device__ __forceinline__ void put2(float* row, int hf, int g, const float (&f)
 
 // Everything of one chunk that does not depend on the carried state.  The two 32-key halves (j = 0,1 and j = 2,3) go
 // through the same pipeline one after the other, which keeps the live register set small.
+template <int MODE>
 __device__ __forceinline__ void produce(int lane, const Raw& x, const ChunkFlags& F, Slot* __restrict__ slot,
                                         SnapSlot* __restrict__ snap, TrTile* __restrict__ tr, unsigned* events) {
   const int t = lane & 15, g = lane >> 4;
@@ -193,7 +197,7 @@ __device__ __forceinline__ void produce(int lane, const Raw& x, const ChunkFlags
     {
       float fr[8], fk[8], fb[8];
       unpack2(x.r[2 * hf], x.r[2 * hf + 1], fr);
-      unpack2(x.k[2 * hf], x.k[2 * hf + 1], fk);
+      if (MODE != SUMMARY) unpack2(x.k[2 * hf], x.k[2 * hf + 1], fk);
       unpack2(x.b[2 * hf], x.b[2 * hf + 1], fb);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
@@ -206,7 +210,7 @@ __device__ __forceinline__ void produce(int lane, const Raw& x, const ChunkFlags
         const float fa0 = (t == 0) ? fa[e] : 0.f;
         fat[e] = fmaf(fa[e], row_prev0(E[e]), fa0);
         fqt[e] = fr[e] * E[e];
-        fkh[e] = fk[e] * einv;
+        fkh[e] = MODE == SUMMARY ? 0.f : fk[e] * einv;
         fbh[e] = fb[e] * einv;
       }
     }
@@ -224,18 +228,19 @@ __device__ __forceinline__ void produce(int lane, const Raw& x, const ChunkFlags
       put2(slot->BK[1][t], hf, g, fqt, ku);
     }
     put2(slot->AQ[0][t], hf, g, fbh, row_keep);
-    put2(slot->AQ[1][t], hf, g, fkh, row_keep);
+    if (MODE != SUMMARY) put2(slot->AQ[1][t], hf, g, fkh, row_keep);
     if (F.snap >= 0) {                            // the same rows masked for the cotangent entering at token length-1
       rare_path();
       const bool sk = (keep_snap >> t) & 1u;
       put2(snap->AQ[0][t], hf, g, fbh, sk);
-      put2(snap->AQ[1][t], hf, g, fkh, sk);
+      if (MODE != SUMMARY) put2(snap->AQ[1][t], hf, g, fkh, sk);
     }
     // ---- partial Gram sums over this half's keys
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       GabT = mfma_f(fat[e], fbh[e], GabT);  // Mba^T[m][n] = at_m . bh_n
       G1 = mfma_f(fqt[e], fbh[e], G1);      // Mbr^T[m][n] = qt_m . bh_n
+      if (MODE == SUMMARY) continue;
       G2 = mfma_f(fat[e], fkh[e], G2);      // Mka^T[m][n] = at_m . kh_n
       G3 = mfma_f(fqt[e], fkh[e], G3);      // Mkr^T[m][n] = qt_m . kh_n
     }
@@ -288,8 +293,10 @@ __device__ __forceinline__ void produce(int lane, const Raw& x, const ChunkFlags
   }
   slot->P[lane] = Pm;
   slot->Ka[lane] = G1;
-  slot->Br[lane] = G2;
-  slot->Kr[lane] = G3;
+  if (MODE != SUMMARY) {
+    slot->Br[lane] = G2;
+    slot->Kr[lane] = G3;
+  }
   if (lane == 0) {
     slot->snap = F.snap;
     slot->keep_end = (lastseg == 0) ? 1 : 0;
@@ -314,18 +321,21 @@ struct Ops {               // fetched a chunk ahead: everything the U / DSA / DV
   int keep_end;
 };
 
+template <int MODE>
 __device__ __forceinline__ void load_ops(Ops& o, const Slot* __restrict__ slot, int q, int lane) {
   const int n = lane & 15, g = lane >> 4;
 #pragma unroll
   for (int tile = 0; tile < 4; ++tile) {
     o.bh[tile] = *reinterpret_cast<const float4*>(&slot->AQ[0][n][16 * tile + 4 * g]);
-    o.kh[tile] = *reinterpret_cast<const float4*>(&slot->AQ[1][n][16 * tile + 4 * g]);
+    if (MODE != SUMMARY) o.kh[tile] = *reinterpret_cast<const float4*>(&slot->AQ[1][n][16 * tile + 4 * g]);
     o.gm[tile] = *reinterpret_cast<const float4*>(&slot->gamma[16 * tile + 4 * g]);
   }
   o.P = slot->P[lane];
   o.Ka = slot->Ka[lane];
-  o.Br = slot->Br[lane];
-  o.Kr = slot->Kr[lane];
+  if (MODE != SUMMARY) {
+    o.Br = slot->Br[lane];
+    o.Kr = slot->Kr[lane];
+  }
 #pragma unroll
   for (int i = 0; i < 4; ++i) o.vv[i] = slot->V[4 * g + i][16 * q + n];
   o.keep_end = slot->keep_end;
@@ -369,11 +379,12 @@ struct OutCursor {
 };
 
 // The cotangent-dependent part of one chunk.  SNAP: this chunk holds token length-1 and a cotangent of the returned
-// state exists (one chunk per sequence; a separate instantiation keeps the common path free of its branch).
-template <bool SNAP, class PeekNext, class WaitNext>
+// state exists (one chunk per sequence; a separate instantiation keeps the common path free of its branch).  SUMMARY: without gv.
+// `emit` (PART only): whether the chunk's outputs are this workgroup's to write.
+template <bool SNAP, int MODE, class PeekNext, class WaitNext>
 __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restrict__ slot,
                                         const Slot* __restrict__ next, const SnapSlot* __restrict__ snapslot,
-                                        const Wkv7Args& A, int64_t b, int64_t h, int nvalid,
+                                        const Wkv7Args& A, int64_t b, int64_t h, int nvalid, bool emit,
                                         OutCursor& oc, PeekNext&& peek_next, WaitNext&& next_ready) {
   const int lane = C.lane, n = lane & 15, g = lane >> 4;
   const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
@@ -392,17 +403,18 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
 #pragma unroll
   for (int tile = 0; tile < 4; ++tile) {
     const float bh[4] = {o.bh[tile].x, o.bh[tile].y, o.bh[tile].z, o.bh[tile].w};
-    const float kh[4] = {o.kh[tile].x, o.kh[tile].y, o.kh[tile].z, o.kh[tile].w};
+    float kh[4] = {0.f, 0.f, 0.f, 0.f};
+    if (MODE != SUMMARY) { kh[0] = o.kh[tile].x; kh[1] = o.kh[tile].y; kh[2] = o.kh[tile].z; kh[3] = o.kh[tile].w; }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       W = mfma_f(bh[i], C.S[tile][i], W);
-      Y = mfma_f(kh[i], C.S[tile][i], Y);
+      if (MODE != SUMMARY) Y = mfma_f(kh[i], C.S[tile][i], Y);
     }
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     W = mfma_f(o.Ka[i], o.vv[i], W);            // U += Mbr DY
-    Y = mfma_f(o.Kr[i], o.vv[i], Y);            // DV += Mkr DY
+    if (MODE != SUMMARY) Y = mfma_f(o.Kr[i], o.vv[i], Y);            // DV += Mkr DY
   }
   const f32x4_t vv = o.vv;
   // a reset inside the chunk cuts the cotangent of later chunks off from the chunk start
@@ -421,13 +433,14 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
       gs[0] *= sg.x; gs[1] *= sg.y; gs[2] *= sg.z; gs[3] *= sg.w;
       if (keep) C.S[tile] += gs;
       const float4 sb = *reinterpret_cast<const float4*>(&snapslot->AQ[0][n][16 * tile + 4 * g]);
-      const float4 sk = *reinterpret_cast<const float4*>(&snapslot->AQ[1][n][16 * tile + 4 * g]);
-      const float bh[4] = {sb.x, sb.y, sb.z, sb.w}, kh[4] = {sk.x, sk.y, sk.z, sk.w};
+      const float bh[4] = {sb.x, sb.y, sb.z, sb.w};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        W = mfma_f(bh[i], gs[i], W);
-        Y = mfma_f(kh[i], gs[i], Y);
-      }
+      for (int i = 0; i < 4; ++i) W = mfma_f(bh[i], gs[i], W);
+      if (MODE == SUMMARY) continue;
+      const float4 sk = *reinterpret_cast<const float4*>(&snapslot->AQ[1][n][16 * tile + 4 * g]);
+      const float kh[4] = {sk.x, sk.y, sk.z, sk.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) Y = mfma_f(kh[i], gs[i], Y);
     }
   }
   // G <- Gh + At^T DSA + Qt^T DY, rows = keys.  The Qt^T DY half, which depends on nothing computed here, runs between
@@ -447,7 +460,7 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    Y = mfma_f(o.Br[i], SA[i], Y);                                // DV += Mka DSA
+    if (MODE != SUMMARY) Y = mfma_f(o.Br[i], SA[i], Y);           // DV += Mka DSA
     C.S[0] = mfma_f(uat[0][i], SA[i], C.S[0]);
     C.S[1] = mfma_f(uat[1][i], SA[i], C.S[1]);
     C.S[2] = mfma_f(uat[2][i], SA[i], C.S[2]);
@@ -457,12 +470,15 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
   bool ok = true;
   if (next != nullptr) {
     ok = next_ready(peeked);
-    load_ops(o, next, C.q, lane);
+    load_ops<MODE>(o, next, C.q, lane);
   }
+  if (MODE == SUMMARY) return ok;
   // outputs: register i is token 4g+i, lanes n = 16 consecutive values
   float* const yl = oc.y + oc.voff;
   float* const sl = oc.sa + oc.voff;
-  if (nvalid == CK) {
+  if (MODE == PART && !emit) {
+    rare_path();
+  } else if (nvalid == CK) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) yl[i * oc.tok] = Y[i];
 #pragma unroll
@@ -484,9 +500,12 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
 
 }  // namespace
 
-// Chunks are handled from the last one down: step j handles chunk nch - 1 - j in slot j % RING.  Producer p fills the
+// Chunks are handled from the last one down: step j handles chunk c1 - 1 - j in slot j % RING.  Producer p fills the
 // slot once every consumer has released step j - RING, then publishes ready = j + 1; consumers take the steps in
 // order.  Every wait is for a strictly earlier step, so the hand-shake cannot cycle.
+//
+// MODE as in wkv7_bwd_a.hip: few sequences and heads run in parts behind a launch that makes their summaries.
+template <int MODE>
 __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_bwd_a_f32_kernel(Wkv7Args A) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Slot* slots = reinterpret_cast<Slot*>(smem_raw);
@@ -495,109 +514,170 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_bwd_a_f32_kernel(Wk
   Sync* sy = reinterpret_cast<Sync*>(smem_raw + RING * sizeof(Slot) + sizeof(SnapSlot) + NPROD * sizeof(TrTile));
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int64_t b = blockIdx.x / A.H, h = blockIdx.x % A.H;
+  // head, part (0: the last of the sequence) and (SUMMARY) which half of the summary
+  const int per_head = MODE == SUMMARY ? 2 * A.n_part - 3 : MODE == PART ? A.n_part : 1;
+  const int64_t head = MODE == WHOLE ? (int64_t)blockIdx.x : (int64_t)(blockIdx.x / per_head);
+  const int unit = MODE == WHOLE ? 0 : (int)(blockIdx.x % per_head);
+  const bool map = MODE == SUMMARY && unit >= A.n_part - 1;           // this workgroup makes M
+  const int part = MODE == SUMMARY && map ? unit - (A.n_part - 2) : unit;
+  const int64_t b = head / A.H, h = head % A.H;
   int64_t L = seq_length(A.length, b, A.T, A.flags);
   L = L < A.T ? L : A.T;
   const int nch = (int)((A.T + CK - 1) / CK);
+  // chunks c1 - 1 down to c0; output from chunk c_out - 1 on
+  int c0 = 0, c1 = nch, c_out = nch, part0 = 0;
+  if (MODE != WHOLE) {
+    auto upto = [&](int p) { const int e = (A.n_part - p) * A.part_chunks; return e < nch ? e : nch; };
+    part0 = MODE == PART && part > 0 ? first_unusable(A, head, part, lane) : part;
+    c0 = (A.n_part - 1 - part) * A.part_chunks;
+    c1 = upto(part0);
+    c_out = upto(part);
+  }
+  const int n = c1 - c0;
   // the returned state is the reset state there (associative-scan rule), a constant
   const bool q2drop = (A.flags & 1u) && L < A.T && A.ns != nullptr && A.ns[b * A.T + L] != 0;
   // does a cotangent of the returned state enter at token length-1?
-  const bool inject = A.gs_out != nullptr && !q2drop;
+  const bool inject = A.gs_out != nullptr && !q2drop && !map;
   if (threadIdx.x < sizeof(Sync) / sizeof(int)) reinterpret_cast<int*>(sy)[threadIdx.x] = 0;
   __syncthreads();
 
+  int unusable = 0;                   // SUMMARY: this wave's word
   if (wave < NCONS) {                 // waves 0..3: one consumer per SIMD; waves 4..7: one producer per SIMD
     __builtin_amdgcn_s_setprio(3);    // the chunk-to-chunk dependency runs through the consumers
     const int cq = wave;
     Consumer C;
     C.q = cq;
     C.lane = lane;
-    const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
+    if (MODE == PART && part0 > 0) {
+      fold_parts_f64(C.S, cq, lane, A, head, part0);
+    } else {
 #pragma unroll
-    for (int tile = 0; tile < 4; ++tile) C.S[tile] = zero4;
+      for (int tile = 0; tile < 4; ++tile)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          C.S[tile][i] = map && 16 * cq + (lane & 15) == 16 * tile + 4 * (lane >> 4) + i ? 1.f : 0.f;
+    }
     OutCursor oc;
     oc.tok = (size_t)A.H * 64;
-    const size_t el0 = (((size_t)b * A.T + (size_t)(nch - 1) * CK) * A.H + h) * 64;
+    const size_t el0 = (((size_t)b * A.T + (size_t)(c1 - 1) * CK) * A.H + h) * 64;
     oc.y = reinterpret_cast<float*>(A.gv) + el0;
     oc.sa = A.dsa + el0;
     oc.voff = (uint32_t)((4 * (lane >> 4)) * (int)A.H * 64 + 16 * cq + (lane & 15));
     const int csnap = (L >= 1 && inject) ? (int)((L - 1) / CK) : -1;
+    // the next chunk whose entering cotangent sweep C starts a part from (0: none)
+    int end = MODE != SUMMARY && A.gends != nullptr ? (c_out - 1) / A.end_chunks * A.end_chunks : 0;
     Ops ops;
     bool ok = true;
-    if (nch > 0) {
+    if (n > 0) {
       ok = wait_ready(sy, 0, 1);
-      load_ops(ops, &slots[0], cq, lane);
+      load_ops<MODE>(ops, &slots[0], cq, lane);
     }
-    for (int j = 0; j < nch && ok; ++j) {
-      const int c = nch - 1 - j;
-      const int nvalid = (j > 0 || A.T % CK == 0) ? CK : (int)(A.T % CK);
+    for (int j = 0; j < n && ok; ++j) {
+      const int c = c1 - 1 - j;
+      const int nvalid = (c + 1 < nch || A.T % CK == 0) ? CK : (int)(A.T % CK);
       const int si = j % RING, sn = (j + 1) % RING;
-      const Slot* next = (j + 1 < nch) ? &slots[sn] : nullptr;
+      const Slot* next = (j + 1 < n) ? &slots[sn] : nullptr;
       auto peek = [&]() { return peek_ready(sy, sn); };
       auto wait = [&](int peeked) { return wait_ready_peeked(sy, sn, j + 2, peeked); };
       if (c == csnap) {
         rare_path();
-        ok = consume<true>(C, ops, &slots[si], next, snapslot, A, b, h, nvalid, oc, peek, wait);
+        ok = consume<true, MODE>(C, ops, &slots[si], next, snapslot, A, b, h, nvalid, c < c_out, oc, peek, wait);
       } else {
-        ok = consume<false>(C, ops, &slots[si], next, snapslot, A, b, h, nvalid, oc, peek, wait);
+        ok = consume<false, MODE>(C, ops, &slots[si], next, snapslot, A, b, h, nvalid, c < c_out, oc, peek, wait);
       }
       // every LDS read of slot si has returned: its data went into the matrix instructions above
       if (lane == 0) __hip_atomic_store(&sy->consumed[cq][si], j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (MODE != SUMMARY && c == end && end > 0) {
+        rare_path();
+        store_end(C.S, cq, lane, A.gends, A, head, end / A.end_chunks, end_kept(A, b, c));
+        end -= A.end_chunks;
+      }
     }
-    // cotangent of the input state; with length == 0 the returned state is the input state itself
-    const bool pass = L == 0 && inject;
+    if (MODE == SUMMARY) {
+      unusable = store_summary(C.S, cq, lane, *part_sum(A, head, part), map);
+    } else if (c0 == 0) {
+      // cotangent of the input state; with length == 0 the returned state is the input state itself
+      const bool pass = L == 0 && inject;
 #pragma unroll
-    for (int tile = 0; tile < 4; ++tile) {
-      const size_t off = state_off(A, b, h, cq, lane, tile);
-      f32x4_t gsv = C.S[tile];
-      if (pass) gsv += load_state_tile(A.gs_out, A.st_f32, off);
-      store_state_tile(A.gs, A.st_f32, off, gsv);
+      for (int tile = 0; tile < 4; ++tile) {
+        const size_t off = state_off(A, b, h, cq, lane, tile);
+        f32x4_t gsv = C.S[tile];
+        if (pass) gsv += load_state_tile(A.gs_out, A.st_f32, off);
+        store_state_tile(A.gs, A.st_f32, off, gsv);
+      }
     }
   } else {
     const int p = wave - NCONS;
     Raw raw;
     uint32_t ns_mine = 0u;      // this lane's new_starts byte of the chunk loaded next: fetched a step ahead, like the operands
-    if (p < nch) {
-      ns_mine = chunk_flag_prefetch(A.ns, A.T, b, (int64_t)(nch - 1 - p) * CK, lane);
-      load_raw(raw, A, b, h, (int64_t)(nch - 1 - p) * CK, lane);
+    // every chunk counts once: in the launch after the summaries, where its output is written
+    unsigned* events = MODE == SUMMARY || (MODE == PART && part0 != part) ? nullptr : events_word(A.status);
+    if (p < n) {
+      ns_mine = chunk_flag_prefetch(A.ns, A.T, b, (int64_t)(c1 - 1 - p) * CK, lane);
+      load_raw<MODE>(raw, A, b, h, (int64_t)(c1 - 1 - p) * CK, lane);
     }
-    for (int j = p; j < nch; j += NPROD) {
-      const int c = nch - 1 - j;
-      const int64_t c0 = (int64_t)c * CK;
-      ChunkFlags F = chunk_flags_of(A.ns, ns_mine, A.flags, A.T, c0, L);
+    for (int j = p; j < n; j += NPROD) {
+      const int c = c1 - 1 - j;
+      const int64_t t0 = (int64_t)c * CK;
+      ChunkFlags F = chunk_flags_of(A.ns, ns_mine, A.flags, A.T, t0, L);
       if (!inject) F.snap = -1;
       const int si = j % RING;
       if (j >= RING && !wait_consumed_lazy(sy, si, j - RING + 1, lane)) break;
       mask_raw(raw, F.nvalid, lane);
-      produce(lane, raw, F, &slots[si], snapslot, &trs[p], events_word(A.status));
-      if (j + NPROD < nch) {
-        ns_mine = chunk_flag_prefetch(A.ns, A.T, b, (int64_t)(c - NPROD) * CK, lane);
-        load_raw(raw, A, b, h, (int64_t)(c - NPROD) * CK, lane);
+      if (MODE == SUMMARY && map) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) raw.v[q] = make_float4(0.f, 0.f, 0.f, 0.f);
       }
-      if ((A.flags & FLAG_DROP_PUBLISH) && j + 1 == nch) break;
+      if (MODE == PART && part0 != part && c < c_out) events = events_word(A.status);
+      produce<MODE>(lane, raw, F, &slots[si], snapslot, &trs[p], events);
+      if (j + NPROD < n) {
+        ns_mine = chunk_flag_prefetch(A.ns, A.T, b, (int64_t)(c - NPROD) * CK, lane);
+        load_raw<MODE>(raw, A, b, h, (int64_t)(c - NPROD) * CK, lane);
+      }
+      if ((A.flags & FLAG_DROP_PUBLISH) && j + 1 == n) break;
       // the release orders this wave's LDS writes before the sequence number
       if (lane == 0) __hip_atomic_store(&sy->ready[si], j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    if (MODE == SUMMARY) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) raw.k[q] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
     retire_loads(raw, ns_mine);
   }
   __syncthreads();
-  if (head_broken(sy, A.status)) {
-    poison_token_rows(A.gv, 4, b, h, A.T, A.H);
-    poison_token_rows(A.dsa, 4, b, h, A.T, A.H);
-    poison_state(A.gs, A.st_f32, b, h, A.H);
+  const bool broken = head_broken(sy, A.status);
+  if (MODE == SUMMARY) {
+    if (wave < NCONS && lane == 0) part_flags(A, head, part)[(map ? 4 : 0) + wave] = unusable | (broken ? 1 : 0);
+    if (wave < NCONS && lane == 0 && !map && part == 0) part_flags(A, head, 0)[4 + wave] = 0;     // part 0 has no M
+  } else if (broken) {
+    const int64_t t0 = (int64_t)c0 * CK, rows = (int64_t)c_out * CK > A.T ? A.T - t0 : (int64_t)c_out * CK - t0;
+    poison_token_rows(A.gv, 4, b, h, A.T, A.H, t0, rows);
+    poison_token_rows(A.dsa, 4, b, h, A.T, A.H, t0, rows);
+    if (A.gends != nullptr) poison_ends(A.gends, A, head, c0, c_out - 1);
+    if (c0 == 0) poison_state(A.gs, A.st_f32, b, h, A.H);
   }
 }
 
-// Reverse sweep of the backward pass with fp32 I/O: gv, the workspace dsa (cotangent of sa per token) and gs.
-hipError_t launch_wkv7_chunk_bwd_a_f32(const Wkv7Args& A, hipStream_t stream) {
+namespace {
+template <int MODE>
+hipError_t launch_mode(const Wkv7Args& A, int64_t groups, hipStream_t stream) {
   static_assert(RING <= MAX_RING, "the hand-shake words cover MAX_RING slots");
   const size_t smem = RING * sizeof(Slot) + sizeof(SnapSlot) + NPROD * sizeof(TrTile) + sizeof(Sync);
   static_assert(RING * sizeof(Slot) + sizeof(SnapSlot) + NPROD * sizeof(TrTile) + sizeof(Sync) <= 160 * 1024, "LDS of one CU");
   static LdsAttrOnce once;
-  const hipError_t attr = allow_dynamic_lds(once, reinterpret_cast<const void*>(wkv7_bwd_a_f32_kernel), smem);
+  const hipError_t attr = allow_dynamic_lds(once, reinterpret_cast<const void*>(wkv7_bwd_a_f32_kernel<MODE>), smem);
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL(wkv7_bwd_a_f32_kernel, dim3((unsigned)(A.B * A.H)), dim3(64 * (NCONS + NPROD)), smem, stream, A);
+  hipLaunchKernelGGL(wkv7_bwd_a_f32_kernel<MODE>, dim3((unsigned)groups), dim3(64 * (NCONS + NPROD)), smem, stream, A);
   return hipGetLastError();
+}
+}  // namespace
+
+// Reverse sweep of the backward pass with fp32 I/O: gv, the workspace dsa (cotangent of sa per token) and gs.
+hipError_t launch_wkv7_chunk_bwd_a_f32(const Wkv7Args& A, hipStream_t stream) {
+  const int64_t heads = A.B * A.H;
+  if (A.n_part < 2) return launch_mode<WHOLE>(A, heads, stream);
+  const hipError_t e = launch_mode<SUMMARY>(A, heads * (2 * A.n_part - 3), stream);
+  return e != hipSuccess ? e : launch_mode<PART>(A, heads * A.n_part, stream);
 }
 
 }  // namespace hiprwkv

@@ -23,6 +23,7 @@
 // and a remainder as in wkv7_fwd_f32.hip.
 #include "chunk_common.h"
 #include "wkv_args.h"
+#include "wkv7_parts.h"
 
 namespace hiprwkv {
 
@@ -465,9 +466,9 @@ __device__ __forceinline__ void consume(Consumer& C, const Slot* __restrict__ sl
 
 }  // namespace
 
-// Slot c % RING holds chunk c.  Producer p fills it once every consumer has released chunk c - RING, then
-// publishes ready = c + 1; consumers take chunks in order.  Every wait is for a strictly earlier chunk, so the
-// hand-shake cannot cycle.
+// Slot j % RING holds chunk c_in + j.  Producer p fills it once every consumer has released chunk j - RING, then
+// publishes ready = j + 1; consumers take chunks in order.  Every wait is for a strictly earlier chunk, so the
+// hand-shake cannot cycle.  A workgroup runs one of the sequence's A.n_end parts, as in wkv7_chunk_bwd_b.hip.
 __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_bwd_b_f32_kernel(Wkv7Args A) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Slot* slots = reinterpret_cast<Slot*>(smem_raw);
@@ -475,10 +476,14 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_bwd_b_f32_kernel(Wk
   Sync* sy = reinterpret_cast<Sync*>(smem_raw + RING * sizeof(Slot) + sizeof(SnapSlot));
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int64_t b = blockIdx.x / A.H, h = blockIdx.x % A.H;
+  const int64_t head = blockIdx.x / A.n_end;
+  const int part = (int)(blockIdx.x % A.n_end);
+  const int64_t b = head / A.H, h = head % A.H;
   int64_t L = seq_length(A.length, b, A.T, A.flags);
   L = L < A.T ? L : A.T;
   const int nch = (int)((A.T + CK - 1) / CK);
+  // chunks c_in .. c_in + n_own - 1
+  const int c_in = part * A.end_chunks, n_own = part + 1 < A.n_end ? A.end_chunks : nch - c_in;
   const bool q2drop = (A.flags & 1u) && L < A.T && A.ns != nullptr && A.ns[b * A.T + L] != 0;
   const bool inject = A.gs_out != nullptr && !q2drop;   // a cotangent of the returned state exists
   if (threadIdx.x < sizeof(Sync) / sizeof(int)) reinterpret_cast<int*>(sy)[threadIdx.x] = 0;
@@ -491,60 +496,66 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_bwd_b_f32_kernel(Wk
     C.lane = lane;
     C.pend = 0.f;
     const int n = lane & 15, g = lane >> 4;
+    if (part > 0) {
+      load_end_cols(C.S, wave, lane, end_of(A.ends, A, head, part));
+    } else {
 #pragma unroll
-    for (int vt = 0; vt < 4; ++vt)
+      for (int vt = 0; vt < 4; ++vt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        C.S[vt][i] = ld_state_el(A.s, A.st_f32, state_el(A, b, h, 16 * vt + 4 * g + i, 16 * wave + n));
+        for (int i = 0; i < 4; ++i)
+          C.S[vt][i] = ld_state_el(A.s, A.st_f32, state_el(A, b, h, 16 * vt + 4 * g + i, 16 * wave + n));
+    }
     OutCursor oc;
     oc.tok = (size_t)A.H * 64;
-    const size_t el0 = (((size_t)b * A.T) * A.H + h) * 64;
+    const size_t el0 = (((size_t)b * A.T + (size_t)c_in * CK) * A.H + h) * 64;
     oc.gr = reinterpret_cast<float*>(A.gr) + el0;
     oc.ga = reinterpret_cast<float*>(A.ga) + el0;
-    oc.ef = A.e2 + f_record(b, h, A.H, nch, 0, wave);
+    oc.ef = A.e2 + f_record(b, h, A.H, nch, c_in, wave);
     oc.voff = (uint32_t)((4 * g) * (int)A.H * 64 + 16 * wave + n);
     const int csnap = (L >= 1 && inject) ? (int)((L - 1) / CK) : -1;
-    if (nch > 0) fetch_ra(C, A, b, h, 0);
-    for (int c = 0; c < nch; ++c) {
+    if (n_own > 0) fetch_ra(C, A, b, h, (int64_t)c_in * CK);
+    for (int j = 0; j < n_own; ++j) {
+      const int c = c_in + j;
       const int nvalid = (c + 1 < nch || A.T % CK == 0) ? CK : (int)(A.T % CK);
-      const int si = c % RING;
-      if (!wait_ready(sy, si, c + 1)) break;
-      consume(C, &slots[si], snapslot, A, b, h, nvalid, c == csnap, c == 0, c + 1 < nch ? (int64_t)(c + 1) * CK : -1, oc);
+      const int si = j % RING;
+      if (!wait_ready(sy, si, j + 1)) break;
+      consume(C, &slots[si], snapslot, A, b, h, nvalid, c == csnap, j == 0, j + 1 < n_own ? (int64_t)(c + 1) * CK : -1, oc);
       // every LDS read of slot si has returned: its data went into the matrix instructions and stores above
-      if (lane == 0) __hip_atomic_store(&sy->consumed[wave][si], c + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (lane == 0) __hip_atomic_store(&sy->consumed[wave][si], j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
   } else {
     const int p = wave - NCONS;
     Raw raw;
     uint32_t ns_mine = 0u;      // this lane's new_starts byte of the chunk loaded next: fetched a step ahead, like the operands
-    if (p < nch) {
-      ns_mine = chunk_flag_prefetch(A.ns, A.T, b, (int64_t)p * CK, lane);
-      load_raw(raw, A, b, h, (int64_t)p * CK, lane);
+    if (p < n_own) {
+      ns_mine = chunk_flag_prefetch(A.ns, A.T, b, (int64_t)(c_in + p) * CK, lane);
+      load_raw(raw, A, b, h, (int64_t)(c_in + p) * CK, lane);
     }
-    for (int c = p; c < nch; c += NPROD) {
-      const int64_t c0 = (int64_t)c * CK;
+    for (int j = p; j < n_own; j += NPROD) {
+      const int64_t c0 = (int64_t)(c_in + j) * CK;
       ChunkFlags F = chunk_flags_of(A.ns, ns_mine, A.flags, A.T, c0, L);
       if (!inject) F.snap = -1;
-      const int si = c % RING;
-      if (c >= RING && !wait_consumed_lazy(sy, si, c - RING + 1, lane)) break;
+      const int si = j % RING;
+      if (j >= RING && !wait_consumed_lazy(sy, si, j - RING + 1, lane)) break;
       mask_raw(raw, F.nvalid, lane);
       produce(lane, raw, F, &slots[si], snapslot, events_word(A.status));
-      if (c + NPROD < nch) {
+      if (j + NPROD < n_own) {
         ns_mine = chunk_flag_prefetch(A.ns, A.T, b, c0 + (int64_t)NPROD * CK, lane);
         load_raw(raw, A, b, h, c0 + (int64_t)NPROD * CK, lane);
       }
-      if ((A.flags & FLAG_DROP_PUBLISH) && c + 1 == nch) break;
+      if ((A.flags & FLAG_DROP_PUBLISH) && j + 1 == n_own) break;
       // the release orders this wave's LDS writes before the sequence number
-      if (lane == 0) __hip_atomic_store(&sy->ready[si], c + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (lane == 0) __hip_atomic_store(&sy->ready[si], j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     retire_loads(raw, ns_mine);
   }
   __syncthreads();
   if (head_broken(sy, A.status)) {
-    poison_token_rows(A.gr, 4, b, h, A.T, A.H);
-    poison_token_rows(A.ga, 4, b, h, A.T, A.H);
-    for (size_t i = threadIdx.x; i < (size_t)nch * NCONS * F_REC; i += blockDim.x)
-      A.e2[f_record(b, h, A.H, nch, 0, 0) + i] = __uint_as_float(0x7fc00000u);
+    const int64_t t0 = (int64_t)c_in * CK, rows = part + 1 < A.n_end ? (int64_t)n_own * CK : A.T - t0;
+    poison_token_rows(A.gr, 4, b, h, A.T, A.H, t0, rows);
+    poison_token_rows(A.ga, 4, b, h, A.T, A.H, t0, rows);
+    for (size_t i = threadIdx.x; i < (size_t)n_own * NCONS * F_REC; i += blockDim.x)
+      A.e2[f_record(b, h, A.H, nch, c_in, 0) + i] = __uint_as_float(0x7fc00000u);
   }
 }
 
@@ -555,7 +566,7 @@ hipError_t launch_wkv7_chunk_bwd_b_f32(const Wkv7Args& A, hipStream_t stream) {
   static LdsAttrOnce once;
   const hipError_t attr = allow_dynamic_lds(once, reinterpret_cast<const void*>(wkv7_bwd_b_f32_kernel), smem);
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL(wkv7_bwd_b_f32_kernel, dim3((unsigned)(A.B * A.H)), dim3(64 * (NCONS + NPROD)), smem, stream, A);
+  hipLaunchKernelGGL(wkv7_bwd_b_f32_kernel, dim3((unsigned)(A.B * A.H * A.n_end)), dim3(64 * (NCONS + NPROD)), smem, stream, A);
   return hipGetLastError();
 }
 

@@ -16,6 +16,7 @@
 // and chunk, 64 per producer).  Chunks are handled from the last one down.
 #include "chunk_common.h"
 #include "wkv_args.h"
+#include "wkv7_parts.h"
 
 namespace hiprwkv {
 
@@ -469,9 +470,9 @@ __device__ __forceinline__ void consume(Consumer& C, const Slot* __restrict__ sl
 
 }  // namespace
 
-// Step j handles chunk nch-1-j in slot j % RING.  Producer p fills the slot once every consumer has released step
+// Step j handles chunk c_end-1-j in slot j % RING.  Producer p fills the slot once every consumer has released step
 // j - RING, then publishes ready = j + 1; consumers take the steps in order.  Every wait is for a strictly earlier
-// step, so the hand-shake cannot cycle.
+// step, so the hand-shake cannot cycle.  A workgroup runs one of the sequence's A.n_end parts, as in wkv7_chunk_bwd_c.hip.
 __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_bwd_c_f32_kernel(Wkv7Args A) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Slot* slots = reinterpret_cast<Slot*>(smem_raw);
@@ -479,10 +480,14 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_bwd_c_f32_kernel(Wk
   Sync* sy = reinterpret_cast<Sync*>(smem_raw + RING * sizeof(Slot) + sizeof(SnapSlot));
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int64_t b = blockIdx.x / A.H, h = blockIdx.x % A.H;
+  const int64_t head = blockIdx.x / A.n_end;
+  const int part = (int)(blockIdx.x % A.n_end);
+  const int64_t b = head / A.H, h = head % A.H;
   int64_t L = seq_length(A.length, b, A.T, A.flags);
   L = L < A.T ? L : A.T;
   const int nch = (int)((A.T + CK - 1) / CK);
+  // chunks c_end - 1 down to c_end - n_own
+  const int c_end = part + 1 < A.n_end ? (part + 1) * A.end_chunks : nch, n_own = c_end - part * A.end_chunks;
   const bool q2drop = (A.flags & 1u) && L < A.T && A.ns != nullptr && A.ns[b * A.T + L] != 0;
   const bool inject = A.gs_out != nullptr && !q2drop;   // a cotangent of the returned state exists
   if (threadIdx.x < sizeof(Sync) / sizeof(int)) reinterpret_cast<int*>(sy)[threadIdx.x] = 0;
@@ -496,29 +501,36 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_bwd_c_f32_kernel(Wk
     C.carry = 0.f;
     const int n = lane & 15, g = lane >> 4;
     const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
+    if (part + 1 < A.n_end) {
+      f32x4_t S[4];
+      load_end_cols(C.G, wave, lane, end_of(A.gends, A, head, part + 1));
+      load_end_cols(S, wave, lane, end_of(A.ends, A, head, part + 1));
+      C.carry = end_carry(C.G, S);
+    } else {
 #pragma unroll
-    for (int vt = 0; vt < 4; ++vt) C.G[vt] = zero4;
+      for (int vt = 0; vt < 4; ++vt) C.G[vt] = zero4;
+    }
     Cursor cu;
     cu.tok = (size_t)A.H * 64;
-    const size_t el0 = (((size_t)b * A.T + (size_t)(nch - 1) * CK) * A.H + h) * 64;
+    const size_t el0 = (((size_t)b * A.T + (size_t)(c_end - 1) * CK) * A.H + h) * 64;
     cu.gk = reinterpret_cast<float*>(A.gk) + el0;
     cu.gb = reinterpret_cast<float*>(A.gb) + el0;
     cu.gw = reinterpret_cast<float*>(A.gw) + el0;
-    cu.rec = reinterpret_cast<const float4*>(A.e2 + f_record(b, h, A.H, nch, nch - 1, wave)) + lane;
+    cu.rec = reinterpret_cast<const float4*>(A.e2 + f_record(b, h, A.H, nch, c_end - 1, wave)) + lane;
     cu.voff = (uint32_t)((4 * g) * (int)A.H * 64 + 16 * wave + n);
     C.f = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (nch > 0) {
+    if (n_own > 0) {
       C.f = *cu.rec;
-      fetch_kbw(C, A, b, h, (int64_t)(nch - 1) * CK);
+      fetch_kbw(C, A, b, h, (int64_t)(c_end - 1) * CK);
     }
     const int csnap = (L >= 1 && inject) ? (int)((L - 1) / CK) : -1;
     const int tail = (A.T % CK == 0) ? CK : (int)(A.T % CK);
-    for (int j = 0; j < nch; ++j) {
-      const int c = nch - 1 - j;
-      const int nvalid = (j == 0) ? tail : CK;
+    for (int j = 0; j < n_own; ++j) {
+      const int c = c_end - 1 - j;
+      const int nvalid = (c + 1 == nch) ? tail : CK;
       const int si = j % RING;
       if (!wait_ready(sy, si, j + 1)) break;
-      consume(C, &slots[si], snapslot, A, b, h, nvalid, c == csnap, j + 1 == nch, (int64_t)(c - 1) * CK, cu);
+      consume(C, &slots[si], snapslot, A, b, h, nvalid, c == csnap, j + 1 == n_own, (int64_t)(c - 1) * CK, cu);
       // every LDS read of slot si has returned: its data went into the matrix instructions and stores above
       if (lane == 0) __hip_atomic_store(&sy->consumed[wave][si], j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
@@ -526,12 +538,12 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_bwd_c_f32_kernel(Wk
     const int p = wave - NCONS;
     Raw raw;
     uint32_t ns_mine = 0u;      // this lane's new_starts byte of the chunk loaded next: fetched a step ahead, like the operands
-    if (p < nch) {
-      ns_mine = chunk_flag_prefetch(A.ns, A.T, b, (int64_t)(nch - 1 - p) * CK, lane);
-      load_raw(raw, A, b, h, (int64_t)(nch - 1 - p) * CK, lane);
+    if (p < n_own) {
+      ns_mine = chunk_flag_prefetch(A.ns, A.T, b, (int64_t)(c_end - 1 - p) * CK, lane);
+      load_raw(raw, A, b, h, (int64_t)(c_end - 1 - p) * CK, lane);
     }
-    for (int j = p; j < nch; j += NPROD) {
-      const int c = nch - 1 - j;
+    for (int j = p; j < n_own; j += NPROD) {
+      const int c = c_end - 1 - j;
       const int64_t c0 = (int64_t)c * CK;
       ChunkFlags F = chunk_flags_of(A.ns, ns_mine, A.flags, A.T, c0, L);
       if (!inject) F.snap = -1;
@@ -539,11 +551,11 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_bwd_c_f32_kernel(Wk
       if (j >= RING && !wait_consumed_lazy(sy, si, j - RING + 1, lane)) break;
       mask_raw(raw, F.nvalid, lane);
       produce(lane, raw, F, &slots[si], snapslot, events_word(A.status));
-      if (j + NPROD < nch) {
+      if (j + NPROD < n_own) {
         ns_mine = chunk_flag_prefetch(A.ns, A.T, b, (int64_t)(c - NPROD) * CK, lane);
         load_raw(raw, A, b, h, (int64_t)(c - NPROD) * CK, lane);
       }
-      if ((A.flags & FLAG_DROP_PUBLISH) && j + 1 == nch) break;
+      if ((A.flags & FLAG_DROP_PUBLISH) && j + 1 == n_own) break;
       // the release orders this wave's LDS writes before the sequence number
       if (lane == 0) __hip_atomic_store(&sy->ready[si], j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
@@ -551,9 +563,10 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_bwd_c_f32_kernel(Wk
   }
   __syncthreads();
   if (head_broken(sy, A.status)) {
-    poison_token_rows(A.gk, 4, b, h, A.T, A.H);
-    poison_token_rows(A.gb, 4, b, h, A.T, A.H);
-    poison_token_rows(A.gw, 4, b, h, A.T, A.H);
+    const int64_t t0 = (int64_t)(c_end - n_own) * CK, rows = c_end == nch ? A.T - t0 : (int64_t)n_own * CK;
+    poison_token_rows(A.gk, 4, b, h, A.T, A.H, t0, rows);
+    poison_token_rows(A.gb, 4, b, h, A.T, A.H, t0, rows);
+    poison_token_rows(A.gw, 4, b, h, A.T, A.H, t0, rows);
   }
 }
 
@@ -564,7 +577,7 @@ hipError_t launch_wkv7_chunk_bwd_c_f32(const Wkv7Args& A, hipStream_t stream) {
   static LdsAttrOnce once;
   const hipError_t attr = allow_dynamic_lds(once, reinterpret_cast<const void*>(wkv7_bwd_c_f32_kernel), smem);
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL(wkv7_bwd_c_f32_kernel, dim3((unsigned)(A.B * A.H)), dim3(64 * (NCONS + NPROD)), smem, stream, A);
+  hipLaunchKernelGGL(wkv7_bwd_c_f32_kernel, dim3((unsigned)(A.B * A.H * A.n_end)), dim3(64 * (NCONS + NPROD)), smem, stream, A);
   return hipGetLastError();
 }
 

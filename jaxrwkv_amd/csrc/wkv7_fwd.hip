@@ -808,23 +808,26 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_kernel(Wkv7Args
 // 256 CUs times the chunks of a part, the second launch and the fold cost PART_COST + 2 per part (8 us + 1.3 us).  No shape on
 // which it decides for parts was slower with them (B=5 T=1021 H=16: 49.9 -> 48.4 us, T=777 H=1 38.9 -> 30.7); below
 // about 600 tokens and above 85 heads the whole sequence is faster.
-constexpr int CUS = 256, MAX_PARTS = 32, PART_COST = 12;
-int wkv7_fwd_parts(int64_t heads, int64_t T, int* chunks) {
+// A chunk of the fp32 kernel takes four times as long (2.7 us): B=3 T=777 H=12 135 -> 83 us, T=512 H=12 91 -> 73, T=256 H=12 52.0
+// whole and 57.7 in parts.
+constexpr int CUS = 256, MAX_PARTS = 32;
+int wkv7_fwd_parts(int64_t heads, int64_t T, bool f32, int* chunks) {
+  const int64_t PART_COST = f32 ? 8 : 12, FOLD2 = f32 ? 2 : 4;      // FOLD2: of two parts
   const int64_t nch = (T + CK - 1) / CK;
   auto rounds = [&](int64_t groups) { return (groups + CUS - 1) / CUS; };
   int64_t best = nch * rounds(heads), best_chunks = nch;
   for (int64_t p = 2; p <= MAX_PARTS && p <= nch; ++p) {
     const int64_t c = (nch + p - 1) / p, np = (nch + c - 1) / c;
     if (np < 2) continue;
-    const int64_t cost = c * (rounds(heads * (2 * np - 3)) + rounds(heads * np)) + PART_COST + 2 * np;
+    const int64_t cost = c * (rounds(heads * (2 * np - 3)) + rounds(heads * np)) + PART_COST + FOLD2 * np / 2;
     if (cost < best) { best = cost; best_chunks = c; }
   }
   *chunks = (int)best_chunks;
   return (int)((nch + best_chunks - 1) / best_chunks);
 }
-size_t wkv7_fwd_parts_bytes(int64_t heads, int64_t T) {
+size_t wkv7_fwd_parts_bytes(int64_t heads, int64_t T, bool f32) {
   int c;
-  const int np = wkv7_fwd_parts(heads, T, &c);
+  const int np = wkv7_fwd_parts(heads, T, f32, &c);
   return np < 2 ? 0 : (size_t)heads * (np - 1) * (sizeof(PartSum) + 8 * sizeof(int));
 }
 
@@ -844,7 +847,7 @@ hipError_t launch_mode(const Wkv7Args& A, int64_t groups, hipStream_t stream) {
 hipError_t launch_wkv7_chunk_fwd(const Wkv7Args& A0, hipStream_t stream) {
   Wkv7Args A = A0;
   const int64_t heads = A.B * A.H;
-  A.n_part = A.parts != nullptr ? wkv7_fwd_parts(heads, A.T, &A.part_chunks) : 1;
+  A.n_part = A.parts != nullptr ? wkv7_fwd_parts(heads, A.T, false, &A.part_chunks) : 1;
   if (A.n_part < 2) return A.sa != nullptr ? launch_mode<true, WHOLE>(A, heads, stream) : launch_mode<false, WHOLE>(A, heads, stream);
   const hipError_t e = launch_mode<false, SUMMARY>(A, heads * (2 * A.n_part - 3), stream);
   if (e != hipSuccess) return e;

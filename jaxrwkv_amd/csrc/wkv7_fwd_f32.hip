@@ -22,6 +22,7 @@
 // Synchronisation, resets, `length` and the decay floor are those of the bf16 kernel (chunk_common.h).
 #include "chunk_common.h"
 #include "wkv_args.h"
+#include "wkv7_parts.h"
 
 namespace hiprwkv {
 
@@ -78,6 +79,7 @@ struct Raw {
   float4 r[4], w[4], k[4], v[4], a[4], b[4];
 };
 
+template <int MODE>
 __device__ __forceinline__ void load_raw(Raw& x, const Wkv7Args& A, int64_t b, int64_t h, int64_t c0, int lane) {
   const int t = lane & 15, g = lane >> 4;
   const int64_t tok = (c0 + t < A.T) ? c0 + t : A.T - 1;   // always a valid token; mask_raw zeroes the lanes beyond
@@ -86,7 +88,8 @@ __device__ __forceinline__ void load_raw(Raw& x, const Wkv7Args& A, int64_t b, i
 #pragma unroll
     for (int j = 0; j < 4; ++j) o[j] = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(p) + off + 16 * j);
   };
-  ld(A.r, x.r); ld(A.w, x.w); ld(A.k, x.k); ld(A.v, x.v); ld(A.a, x.a); ld(A.b, x.b);
+  if (MODE != SUMMARY) ld(A.r, x.r);
+  ld(A.w, x.w); ld(A.k, x.k); ld(A.v, x.v); ld(A.a, x.a); ld(A.b, x.b);
 }
 __device__ __forceinline__ void mask_raw(Raw& x, int nvalid, int lane) {
   if (nvalid != CK) {
@@ -109,7 +112,8 @@ __device__ __forceinline__ void put2(float* row, int hf, int g, const float (&f)
 }
 
 // Everything of one chunk that does not depend on the carried state.  The two 32-key halves (j = 0,1 and j = 2,3) go
-// through the same pipeline one after the other, which keeps the live register set small.
+// through the same pipeline one after the other, which keeps the live register set small.  SUMMARY: without what only y needs.
+template <int MODE>
 __device__ __forceinline__ void produce(int lane, const Raw& x, const ChunkFlags& F, Slot* __restrict__ slot,
                                         SnapSlot* __restrict__ snap, TrTile* __restrict__ tr, unsigned* events) {
   const int t = lane & 15, g = lane >> 4;
@@ -198,7 +202,7 @@ __device__ __forceinline__ void produce(int lane, const Raw& x, const ChunkFlags
     float fat[8], fqt[8], fkh[8], fbh[8], fke[8], fbe[8];
     {
       float fr[8], fk[8], fb[8];
-      unpack2(x.r[2 * hf], x.r[2 * hf + 1], fr);
+      if (MODE != SUMMARY) unpack2(x.r[2 * hf], x.r[2 * hf + 1], fr);
       unpack2(x.k[2 * hf], x.k[2 * hf + 1], fk);
       unpack2(x.b[2 * hf], x.b[2 * hf + 1], fb);
 #pragma unroll
@@ -209,7 +213,7 @@ __device__ __forceinline__ void produce(int lane, const Raw& x, const ChunkFlags
         const float einv = exp2_fast(-l2) * (2.f - fl);
         const float fa0 = (t == 0) ? fa[e] : 0.f; // the decay up to the previous token is 1 for the chunk's first token
         fat[e] = fmaf(fa[e], row_prev0(E[e]), fa0);
-        fqt[e] = fr[e] * E[e];
+        fqt[e] = MODE == SUMMARY ? 0.f : fr[e] * E[e];
         fkh[e] = fk[e] * einv;
         fbh[e] = fb[e] * einv;
         const float gam = row_last(E[e]);         // decay from the (last) segment start to the chunk end
@@ -244,12 +248,13 @@ __device__ __forceinline__ void produce(int lane, const Raw& x, const ChunkFlags
       }
     }
     put2(slot->AQ[0][t], hf, g, fat, row0_keep);
-    put2(slot->AQ[1][t], hf, g, fqt, row1_keep);
+    if (MODE != SUMMARY) put2(slot->AQ[1][t], hf, g, fqt, row1_keep);
     // ---- partial Gram sums over this half's keys
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       Gab = mfma_f(fbh[e], fat[e], Gab);    // [m][n] = bh_m . at_n
       G1 = mfma_f(fkh[e], fat[e], G1);      // Mka[m][n] = kh_m . at_n
+      if (MODE == SUMMARY) continue;
       G2 = mfma_f(fbh[e], fqt[e], G2);      // Mbr[m][n] = bh_m . qt_n
       G3 = mfma_f(fkh[e], fqt[e], G3);      // Mkr[m][n] = kh_m . qt_n
     }
@@ -303,8 +308,10 @@ __device__ __forceinline__ void produce(int lane, const Raw& x, const ChunkFlags
   }
   slot->P[lane] = Pm;
   slot->Ka[lane] = G1;
-  slot->Br[lane] = G2;
-  slot->Kr[lane] = G3;
+  if (MODE != SUMMARY) {
+    slot->Br[lane] = G2;
+    slot->Kr[lane] = G3;
+  }
   if (lane == 0) {
     slot->snap = F.snap;
     slot->keep_end = (lastseg == 0) ? 1 : 0;
@@ -328,17 +335,20 @@ struct Ops {               // fetched a chunk ahead: everything the W / SA / Y c
   int keep_end;
 };
 
+template <int MODE>
 __device__ __forceinline__ void load_ops(Ops& o, const Slot* __restrict__ slot, int q, int lane) {
   const int n = lane & 15, g = lane >> 4;
 #pragma unroll
   for (int tile = 0; tile < 4; ++tile) {
     o.at[tile] = *reinterpret_cast<const float4*>(&slot->AQ[0][n][16 * tile + 4 * g]);
-    o.qt[tile] = *reinterpret_cast<const float4*>(&slot->AQ[1][n][16 * tile + 4 * g]);
+    if (MODE != SUMMARY) o.qt[tile] = *reinterpret_cast<const float4*>(&slot->AQ[1][n][16 * tile + 4 * g]);
   }
   o.P = slot->P[lane];
   o.Ka = slot->Ka[lane];
-  o.Br = slot->Br[lane];
-  o.Kr = slot->Kr[lane];
+  if (MODE != SUMMARY) {
+    o.Br = slot->Br[lane];
+    o.Kr = slot->Kr[lane];
+  }
 #pragma unroll
   for (int i = 0; i < 4; ++i) o.vv[i] = slot->V[4 * g + i][16 * q + n];
   o.keep_end = slot->keep_end;
@@ -384,12 +394,13 @@ struct OutCursor {
 // The state-dependent part of one chunk.  SNAP: this chunk holds token length-1 (one chunk per sequence; a separate
 // instantiation keeps the common path free of its branch).  The instruction order is chosen so that a matrix
 // instruction never has to wait for a result it reads as A or B operand: the Ke^T V half of the state update, which
-// depends on nothing computed here, runs between W -> SA and SA -> its readers.
-template <bool SNAP, class PeekNext, class WaitNext>
+// depends on nothing computed here, runs between W -> SA and SA -> its readers.  `emit` (PART only): whether the chunk's outputs
+// are this workgroup's to write.
+template <bool SNAP, int MODE, class PeekNext, class WaitNext>
 __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restrict__ slot,
                                         const Slot* __restrict__ next, const SnapSlot* __restrict__ snapslot,
                                         const Wkv7Args& A, int64_t b, int64_t h, int nvalid, bool q2drop,
-                                        OutCursor& oc, PeekNext&& peek_next, WaitNext&& next_ready) {
+                                        bool emit, OutCursor& oc, PeekNext&& peek_next, WaitNext&& next_ready) {
   const int lane = C.lane, g = lane >> 4;
   const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
   const int peeked = next != nullptr ? peek_next() : 0;
@@ -406,17 +417,18 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
 #pragma unroll
   for (int tile = 0; tile < 4; ++tile) {
     const float at[4] = {o.at[tile].x, o.at[tile].y, o.at[tile].z, o.at[tile].w};
-    const float qt[4] = {o.qt[tile].x, o.qt[tile].y, o.qt[tile].z, o.qt[tile].w};
+    float qt[4] = {0.f, 0.f, 0.f, 0.f};
+    if (MODE != SUMMARY) { qt[0] = o.qt[tile].x; qt[1] = o.qt[tile].y; qt[2] = o.qt[tile].z; qt[3] = o.qt[tile].w; }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       W = mfma_f(at[i], C.S[tile][i], W);
-      Y = mfma_f(qt[i], C.S[tile][i], Y);
+      if (MODE != SUMMARY) Y = mfma_f(qt[i], C.S[tile][i], Y);
     }
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     W = mfma_f(o.Ka[i], o.vv[i], W);            // W += Mka^T V
-    Y = mfma_f(o.Kr[i], o.vv[i], Y);            // Y += Mkr^T V
+    if (MODE != SUMMARY) Y = mfma_f(o.Kr[i], o.vv[i], Y);            // Y += Mkr^T V
   }
   const f32x4_t vv = o.vv;
   // the state the snapshot starts from, before the update overwrites it
@@ -450,7 +462,7 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    Y = mfma_f(o.Br[i], SA[i], Y);                                // Y += Mbr^T SA
+    if (MODE != SUMMARY) Y = mfma_f(o.Br[i], SA[i], Y);           // Y += Mbr^T SA
     C.S[0] = mfma_f(ube[0][i], SA[i], C.S[0]);
     C.S[1] = mfma_f(ube[1][i], SA[i], C.S[1]);
     C.S[2] = mfma_f(ube[2][i], SA[i], C.S[2]);
@@ -460,7 +472,7 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
   bool ok = true;
   if (next != nullptr) {
     ok = next_ready(peeked);
-    load_ops(o, next, C.q, lane);
+    load_ops<MODE>(o, next, C.q, lane);
   }
   // state snapshot for `length`
   if (SNAP) {
@@ -480,10 +492,13 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
       store_state_tile(A.new_s, A.st_f32, state_off(A, b, h, C.q, lane, tile), q2drop ? zero4 : acc);
     }
   }
+  if (MODE == SUMMARY) return ok;
   // outputs: register i is token 4g+i, lanes n = 16 consecutive values
   float* const yl = oc.y + oc.voff;
   float* const sl = oc.sa != nullptr ? oc.sa + oc.voff : nullptr;
-  if (nvalid == CK) {
+  if (MODE == PART && !emit) {
+    rare_path();
+  } else if (nvalid == CK) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) yl[i * oc.tok] = Y[i];
     if (sl != nullptr) {
@@ -507,9 +522,13 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
 
 }  // namespace
 
-// Step j handles chunk j in slot j % RING.  Producer p fills the slot once every consumer has released step j - RING,
+// Step j handles chunk j0 + j in slot j % RING.  Producer p fills the slot once every consumer has released step j - RING,
 // then publishes ready = j + 1; consumers take the steps in order.  Every wait is for a strictly earlier step, so
 // the hand-shake cannot cycle.
+//
+// MODE as in wkv7_fwd.hip: where (sequence, head) workgroups leave most of the GPU idle, the sequence runs in parts behind a launch
+// that makes their summaries.
+template <int MODE>
 __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_f32_kernel(Wkv7Args A) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Slot* slots = reinterpret_cast<Slot*>(smem_raw);
@@ -518,15 +537,31 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_f32_kernel(Wkv7
   Sync* sy = reinterpret_cast<Sync*>(smem_raw + RING * sizeof(Slot) + sizeof(SnapSlot) + NPROD * sizeof(TrTile));
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int64_t b = blockIdx.x / A.H, h = blockIdx.x % A.H;
+  // head, part and (SUMMARY) which half of the summary
+  const int per_head = MODE == SUMMARY ? 2 * A.n_part - 3 : MODE == PART ? A.n_part : 1;
+  const int64_t head = MODE == WHOLE ? (int64_t)blockIdx.x : (int64_t)(blockIdx.x / per_head);
+  const int unit = MODE == WHOLE ? 0 : (int)(blockIdx.x % per_head);
+  const bool map = MODE == SUMMARY && unit >= A.n_part - 1;           // this workgroup makes M
+  const int part = MODE == SUMMARY && map ? unit - (A.n_part - 2) : unit;
+  const int64_t b = head / A.H, h = head % A.H;
   int64_t L = seq_length(A.length, b, A.T, A.flags);
   L = L < A.T ? L : A.T;
   const int nch = (int)((A.T + CK - 1) / CK);
+  // chunks j0 .. j0 + n - 1; output from chunk j_out on
+  int j0 = 0, n = nch, j_out = 0, part0 = 0;
+  if (MODE != WHOLE) {
+    j_out = part * A.part_chunks;
+    const int end = j_out + A.part_chunks < nch ? j_out + A.part_chunks : nch;
+    part0 = MODE == PART && part > 0 ? first_unusable(A, head, part, lane) : part;
+    j0 = part0 * A.part_chunks;
+    n = end - j0;
+  }
   // the returned state is the reset state there (associative-scan rule), a constant
   const bool q2drop = (A.flags & 1u) && L < A.T && A.ns != nullptr && A.ns[b * A.T + L] != 0;
   if (threadIdx.x < sizeof(Sync) / sizeof(int)) reinterpret_cast<int*>(sy)[threadIdx.x] = 0;
   __syncthreads();
 
+  int unusable = 0;                   // SUMMARY: this wave's word
   if (wave < NCONS) {                 // waves 0..3: one consumer per SIMD; waves 4..7: one producer per SIMD
     __builtin_amdgcn_s_setprio(3);    // the chunk-to-chunk dependency runs through the consumers
     const int cq = wave;
@@ -534,84 +569,133 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_f32_kernel(Wkv7
     C.q = cq;
     C.lane = lane;
     const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
+    if (MODE == WHOLE || (part0 == 0 && !map)) {
 #pragma unroll
-    for (int tile = 0; tile < 4; ++tile) C.S[tile] = load_state_tile(A.s, A.st_f32, state_off(A, b, h, cq, lane, tile));
+      for (int tile = 0; tile < 4; ++tile) C.S[tile] = load_state_tile(A.s, A.st_f32, state_off(A, b, h, cq, lane, tile));
+    } else if (MODE == SUMMARY) {
+#pragma unroll
+      for (int tile = 0; tile < 4; ++tile)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          C.S[tile][i] = map && 16 * cq + (lane & 15) == 16 * tile + 4 * (lane >> 4) + i ? 1.f : 0.f;
+    } else {
+      fold_parts_f64(C.S, cq, lane, A, head, part0);
+    }
     // length == 0: the returned state is the input state (rwkv7.py:203), or the reset state under the associative rule
-    if (L == 0) {
+    if (L == 0 && (MODE == WHOLE || (MODE == PART && part == 0))) {
 #pragma unroll
       for (int tile = 0; tile < 4; ++tile)
         store_state_tile(A.new_s, A.st_f32, state_off(A, b, h, cq, lane, tile), q2drop ? zero4 : C.S[tile]);
     }
     OutCursor oc;
     oc.tok = (size_t)A.H * 64;
-    const size_t el0 = (((size_t)b * A.T) * A.H + h) * 64;
+    const size_t el0 = (((size_t)b * A.T + (size_t)j0 * CK) * A.H + h) * 64;
     oc.y = reinterpret_cast<float*>(A.out) + el0;
     oc.sa = A.sa ? reinterpret_cast<float*>(A.sa) + el0 : nullptr;
     oc.voff = (uint32_t)((4 * (lane >> 4)) * (int)A.H * 64 + 16 * cq + (lane & 15));
-    const int csnap = L >= 1 ? (int)((L - 1) / CK) : -1;
+    // the chunk of token length-1, if this workgroup writes the returned state
+    const int csnap = MODE != SUMMARY && L >= 1 && (int)((L - 1) / CK) >= j_out ? (int)((L - 1) / CK) - j0 : -1;
+    // the next chunk boundary whose state the backward starts a part from
+    int end = MODE != SUMMARY && A.ends != nullptr ? (j_out / A.end_chunks + 1) * A.end_chunks : nch;
     Ops ops;
     bool ok = true;
-    if (nch > 0) {
+    if (n > 0) {
       ok = wait_ready(sy, 0, 1);
-      load_ops(ops, &slots[0], cq, lane);
+      load_ops<MODE>(ops, &slots[0], cq, lane);
     }
-    for (int j = 0; j < nch && ok; ++j) {
-      const int nvalid = (j + 1 < nch || A.T % CK == 0) ? CK : (int)(A.T % CK);
+    for (int j = 0; j < n && ok; ++j) {
+      const int nvalid = (j0 + j + 1 < nch || A.T % CK == 0) ? CK : (int)(A.T % CK);
       const int si = j % RING, sn = (j + 1) % RING;
-      const Slot* next = (j + 1 < nch) ? &slots[sn] : nullptr;
+      const Slot* next = (j + 1 < n) ? &slots[sn] : nullptr;
+      const bool emit = j0 + j >= j_out;
       auto peek = [&]() { return peek_ready(sy, sn); };
       auto wait = [&](int peeked) { return wait_ready_peeked(sy, sn, j + 2, peeked); };
-      if (j == csnap) {
+      if (MODE != SUMMARY && j == csnap) {
         rare_path();
-        ok = consume<true>(C, ops, &slots[si], next, snapslot, A, b, h, nvalid, q2drop, oc, peek, wait);
+        ok = consume<true, MODE>(C, ops, &slots[si], next, snapslot, A, b, h, nvalid, q2drop, emit, oc, peek, wait);
       } else {
-        ok = consume<false>(C, ops, &slots[si], next, snapslot, A, b, h, nvalid, q2drop, oc, peek, wait);
+        ok = consume<false, MODE>(C, ops, &slots[si], next, snapslot, A, b, h, nvalid, q2drop, emit, oc, peek, wait);
       }
       // every LDS read of slot si has returned: its data went into the matrix instructions above
       if (lane == 0) __hip_atomic_store(&sy->consumed[cq][si], j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (MODE != SUMMARY && j0 + j + 1 == end && end < nch) {
+        rare_path();
+        store_end(C.S, cq, lane, A.ends, A, head, end / A.end_chunks);
+        end += A.end_chunks;
+      }
     }
+    if (MODE == SUMMARY) unusable = store_summary(C.S, cq, lane, *part_sum(A, head, part), map);
   } else {
     const int p = wave - NCONS;
     Raw raw;
     uint32_t ns_mine = 0u;      // this lane's new_starts byte of the chunk loaded next: fetched a step ahead, like the operands
-    if (p < nch) {
-      ns_mine = chunk_flag_prefetch(A.ns, A.T, b, (int64_t)p * CK, lane);
-      load_raw(raw, A, b, h, (int64_t)p * CK, lane);
+    // every chunk counts once: in the launch after the summaries, where its output is written
+    unsigned* events = MODE == SUMMARY || (MODE == PART && part0 != part) ? nullptr : events_word(A.status);
+    if (p < n) {
+      ns_mine = chunk_flag_prefetch(A.ns, A.T, b, (int64_t)(j0 + p) * CK, lane);
+      load_raw<MODE>(raw, A, b, h, (int64_t)(j0 + p) * CK, lane);
     }
-    for (int j = p; j < nch; j += NPROD) {
-      const int64_t c0 = (int64_t)j * CK;
-      const ChunkFlags F = chunk_flags_of(A.ns, ns_mine, A.flags, A.T, c0, L);
+    for (int j = p; j < n; j += NPROD) {
+      const int64_t c0 = (int64_t)(j0 + j) * CK;
+      const ChunkFlags F = chunk_flags_of(A.ns, ns_mine, A.flags, A.T, c0, MODE == SUMMARY ? 0 : L);
       const int si = j % RING;
       if (j >= RING && !wait_consumed_lazy(sy, si, j - RING + 1, lane)) break;
       mask_raw(raw, F.nvalid, lane);
-      produce(lane, raw, F, &slots[si], snapslot, &trs[p], events_word(A.status));
-      if (j + NPROD < nch) {
-        ns_mine = chunk_flag_prefetch(A.ns, A.T, b, c0 + (int64_t)NPROD * CK, lane);
-        load_raw(raw, A, b, h, c0 + (int64_t)NPROD * CK, lane);
+      if (MODE == SUMMARY && map) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) raw.v[q] = make_float4(0.f, 0.f, 0.f, 0.f);
       }
-      if ((A.flags & FLAG_DROP_PUBLISH) && j + 1 == nch) break;
+      if (MODE == PART && part0 != part && j0 + j >= j_out) events = events_word(A.status);
+      produce<MODE>(lane, raw, F, &slots[si], snapslot, &trs[p], events);
+      if (j + NPROD < n) {
+        ns_mine = chunk_flag_prefetch(A.ns, A.T, b, c0 + (int64_t)NPROD * CK, lane);
+        load_raw<MODE>(raw, A, b, h, c0 + (int64_t)NPROD * CK, lane);
+      }
+      if ((A.flags & FLAG_DROP_PUBLISH) && j + 1 == n) break;
       // the release orders this wave's LDS writes before the sequence number
       if (lane == 0) __hip_atomic_store(&sy->ready[si], j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    if (MODE == SUMMARY) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) raw.r[q] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
     retire_loads(raw, ns_mine);
   }
   __syncthreads();
-  if (head_broken(sy, A.status)) {
-    poison_token_rows(A.out, 4, b, h, A.T, A.H);
-    poison_token_rows(A.sa, 4, b, h, A.T, A.H);
-    poison_state(A.new_s, A.st_f32, b, h, A.H);
+  const bool broken = head_broken(sy, A.status);
+  if (MODE == SUMMARY) {
+    if (wave < NCONS && lane == 0) part_flags(A, head, part)[(map ? 4 : 0) + wave] = unusable | (broken ? 1 : 0);
+    if (wave < NCONS && lane == 0 && !map && part == 0) part_flags(A, head, 0)[4 + wave] = 0;     // part 0 has no M
+  } else if (broken) {
+    const int64_t t0 = (int64_t)j_out * CK, rows = MODE == WHOLE || (int64_t)(j0 + n) * CK > A.T ? A.T - t0 : (int64_t)(j0 + n) * CK - t0;
+    poison_token_rows(A.out, 4, b, h, A.T, A.H, t0, rows);
+    poison_token_rows(A.sa, 4, b, h, A.T, A.H, t0, rows);
+    if (A.ends != nullptr) poison_ends(A.ends, A, head, j_out + 1, j0 + n);
+    if (MODE == WHOLE || (L == 0 ? part == 0 : L - 1 >= t0 && L - 1 < t0 + rows)) poison_state(A.new_s, A.st_f32, b, h, A.H);
   }
 }
 
-hipError_t launch_wkv7_chunk_fwd_f32(const Wkv7Args& A, hipStream_t stream) {
+namespace {
+template <int MODE>
+hipError_t launch_mode(const Wkv7Args& A, int64_t groups, hipStream_t stream) {
   static_assert(RING <= MAX_RING, "the hand-shake words cover MAX_RING slots");
   const size_t smem = RING * sizeof(Slot) + sizeof(SnapSlot) + NPROD * sizeof(TrTile) + sizeof(Sync);
   static_assert(RING * sizeof(Slot) + sizeof(SnapSlot) + NPROD * sizeof(TrTile) + sizeof(Sync) <= 160 * 1024, "LDS of one CU");
   static LdsAttrOnce once;
-  const hipError_t attr = allow_dynamic_lds(once, reinterpret_cast<const void*>(wkv7_fwd_f32_kernel), smem);
+  const hipError_t attr = allow_dynamic_lds(once, reinterpret_cast<const void*>(wkv7_fwd_f32_kernel<MODE>), smem);
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL(wkv7_fwd_f32_kernel, dim3((unsigned)(A.B * A.H)), dim3(64 * (NCONS + NPROD)), smem, stream, A);
+  hipLaunchKernelGGL(wkv7_fwd_f32_kernel<MODE>, dim3((unsigned)groups), dim3(64 * (NCONS + NPROD)), smem, stream, A);
   return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_wkv7_chunk_fwd_f32(const Wkv7Args& A0, hipStream_t stream) {
+  Wkv7Args A = A0;
+  const int64_t heads = A.B * A.H;
+  A.n_part = A.parts != nullptr ? wkv7_fwd_parts(heads, A.T, true, &A.part_chunks) : 1;
+  if (A.n_part < 2) return launch_mode<WHOLE>(A, heads, stream);
+  const hipError_t e = launch_mode<SUMMARY>(A, heads * (2 * A.n_part - 3), stream);
+  return e != hipSuccess ? e : launch_mode<PART>(A, heads * A.n_part, stream);
 }
 
 }  // namespace hiprwkv

@@ -76,6 +76,55 @@ __device__ __forceinline__ void fold_parts(f32x4_t (&S)[4], int q, int lane, con
     }
   }
 }
+// The same on the fp64 matrix instruction, for the fp32 kernels, at 64 cycles an instruction: with sums of 64 terms in fp32 the state
+// at a boundary was 1.4 times as far from 64 bits as the whole sequence's (B=1 T=1024 H=2, decay exp(-exp(-2.5))).  Its register i
+// holds row 4i + g of a tile where the fp32 one holds 4g + i; the last step turns the tiles back.
+__device__ __forceinline__ void fold_parts_f64(f32x4_t (&S)[4], int q, int lane, const Wkv7Args& A, int64_t head, int part) {
+  typedef double f64x4_t __attribute__((ext_vector_type(4)));
+  const int x = lane & 15, g = lane >> 4;
+  // element (row 4i + g, column x) of a 16x16 tile stored as [lane (x, row / 4)][row % 4]
+  auto el = [&](const f32x4_t* tile, int i) { return reinterpret_cast<const float*>(tile + 16 * i + x)[g]; };
+  f64x4_t s[4];
+#pragma unroll
+  for (int tile = 0; tile < 4; ++tile)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[tile][i] = (double)el(part_sum(A, head, 0)->B[q][tile], i);
+  for (int p = 1; p < part; ++p) {
+    const PartSum* const ps = part_sum(A, head, p);
+    f64x4_t acc[4];
+#pragma unroll
+    for (int jt = 0; jt < 4; ++jt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[jt][i] = (double)el(ps->B[q][jt], i);
+#pragma unroll
+    for (int tile = 0; tile < 4; ++tile) {
+      float m[4][4];
+#pragma unroll
+      for (int jt = 0; jt < 4; ++jt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) m[jt][i] = el(ps->M[tile][jt], i);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int jt = 0; jt < 4; ++jt) acc[jt] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)m[jt][i], s[tile][i], acc[jt], 0, 0, 0);
+    }
+#pragma unroll
+    for (int jt = 0; jt < 4; ++jt) s[jt] = acc[jt];
+  }
+#pragma unroll
+  for (int tile = 0; tile < 4; ++tile)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      // row 4g + i lies in register g of lane (x, i)
+      float r = 0.f;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float v = __shfl((float)s[tile][k], x + 16 * i, 64);
+        r = g == k ? v : r;
+      }
+      S[tile][i] = r;
+    }
+}
 // writes a consumer's rows of one half of a summary; not zero if it must not be used
 __device__ __forceinline__ int store_summary(const f32x4_t (&S)[4], int q, int lane, PartSum& ps, bool map) {
   const int x = lane & 15, g = lane >> 4;

@@ -43,14 +43,14 @@ struct Wkv7Args {
   float *ends, *gends;
   int n_end, end_chunks;
 };
-int wkv7_fwd_parts(int64_t heads, int64_t T, int* chunks);
-size_t wkv7_fwd_parts_bytes(int64_t heads, int64_t T);
+int wkv7_fwd_parts(int64_t heads, int64_t T, bool f32, int* chunks);
+size_t wkv7_fwd_parts_bytes(int64_t heads, int64_t T, bool f32);
 // How the backward splits a sequence: n_end parts for sweeps B and C, and whether sweep A runs in these parts too
 struct Wkv7BwdSplit {
   int n_end, end_chunks;
   bool a_parts;
 };
-Wkv7BwdSplit wkv7_bwd_parts(int64_t heads, int64_t T);
+Wkv7BwdSplit wkv7_bwd_parts(int64_t heads, int64_t T, bool f32);
 size_t wkv7_bwd_sums_bytes(int64_t heads, const Wkv7BwdSplit& S);      // summaries of sweep A
 
 // Wkv6Args::flags bit: w is (H,64), shared by every token and sequence (HIPRWKV_W_PER_HEAD)

@@ -36,7 +36,7 @@ def boundary(B, T, H):
     return 16 * -(-(-(-T // 16)) // n)
 
 
-@pytest.mark.parametrize("B,T,H,seed,p", [(1, 300, 1, 0, 0.0), (2, 289, 2, 1, 0.01), (3, 333, 12, 2, 0.004), (5, 260, 30, 3, 0.01)])
+@pytest.mark.parametrize("B,T,H,seed,p", [(1, 300, 1, 0, 0.0), (2, 289, 2, 1, 0.01), (3, 333, 12, 2, 0.004), (4, 260, 30, 3, 0.01)])
 @pytest.mark.parametrize("compat", [True, False])
 def test_against_the_oracle(B, T, H, seed, p, compat):
     n = boundary(B, T, H)
@@ -124,3 +124,77 @@ def test_autograd_takes_the_parts():
     want = run(x, True)
     for n, z in zip(NAMES, g):
         assert np.array_equal(host(z), want[n]), n
+
+
+# ------------------------------------------------------------------------------------------------ fp32 I/O, both directions
+def run32(x, compat, parts, monkeypatch):
+    from jaxrwkv_amd import _lib, ops
+    t = [dev(x[n]) for n in ("r", "w", "k", "v", "a", "b", "s", "length", "new_starts")]
+    with monkeypatch.context() as m:
+        if not parts:
+            m.setattr(_lib.load(), "hiprwkv_wkv7_fwd_workspace_bytes", lambda *_: 0)
+        new_s, y, sa, ends = ops._wkv7_fwd(*t, compat=compat, want_sa=True, want_ends=parts)
+    g = ops.wkv7_bwd(*t, dev(x["dy"]), sa, dev(x["ds"]), compat=compat, ends=ends)
+    torch.cuda.synchronize()
+    return dict(zip(("y", "new_s", "sa") + NAMES, (host(z) for z in (y, new_s, sa) + tuple(g))))
+
+
+def oracle32(x, compat):
+    from oracle import wkv7 as o7
+    new_s, y, sa = o7.wkv7_base(*(x[n] for n in ("r", "w", "k", "v", "a", "b", "s", "length", "new_starts")), compat=compat, return_sa=True)
+    return dict(oracle(x, compat), y=y, new_s=new_s, sa=sa)
+
+
+def boundary32(B, T, H):
+    from jaxrwkv_amd import _lib
+    lib = _lib.load()
+    assert lib.hiprwkv_wkv7_fwd_workspace_bytes(0, B, T, H, 64) > 0
+    n = lib.hiprwkv_wkv7_ends_bytes(0, B, T, H, 64) // (4096 * 4 * B * H) + 1
+    assert n >= 2
+    return 16 * -(-(-(-T // 16)) // n)
+
+
+@pytest.mark.parametrize("B,T,H,seed,p", [(1, 200, 1, 0, 0.0), (2, 241, 2, 1, 0.01), (3, 260, 12, 2, 0.004), (2, 250, 20, 3, 0.01)])
+@pytest.mark.parametrize("compat", [True, False])
+def test_fp32_against_the_oracle(B, T, H, seed, p, compat, monkeypatch):
+    """At the bounds of the whole sequence up to 260 tokens (test_gpu_wkv7, test_gpu_random_shapes)."""
+    from tests.gpu_util import assert_close
+    from tests.test_gpu_wkv7 import GRAD_ATOL
+    n = boundary32(B, T, H)
+    x = wkv7_inputs(B, T, H, 64, seed=seed, p_reset=p, min_len_frac=0.0)
+    for L in (0, 1, n - 1, n, n + 1, T):
+        x["length"][0] = L
+        x["new_starts"][-1, n] = L % 2 == 0
+        got, ref = run32(x, compat, True, monkeypatch), oracle32(x, compat)
+        for k in ("y", "new_s", "sa"):
+            assert_close(k, got[k], ref[k])
+        for k in NAMES:
+            assert_close("g" + k, got[k], ref[k], atol=GRAD_ATOL[k], scale_atol=True)
+
+
+@pytest.mark.parametrize("decay", [-0.5, -2.5, -5.0, -8.0])
+@pytest.mark.parametrize("B,T,H", [(1, 1024, 2), (3, 777, 12)])
+def test_fp32_errors_are_those_of_the_whole_sequence(B, T, H, decay, monkeypatch):
+    """Summaries and the products that fold them are fp32 as everything else, so the rms errors stay: a tenth more is allowed."""
+    x = wkv7_inputs(B, T, H, 64, seed=5, resets=False)
+    x["w"] = (x["w"] + 0.5 + decay).astype(np.float32).astype(np.float64)
+    boundary32(B, T, H)
+    ref, got, base = oracle32(x, True), run32(x, True, True, monkeypatch), run32(x, True, False, monkeypatch)
+    worst = []
+    for k in ref:
+        new, old = rms(got[k] - ref[k]), rms(base[k] - ref[k])
+        print(f"B{B} T{T} H{H} decay {decay} {k}: {old / rms(ref[k]):.2e} whole, in parts {new / old:.3f} of it")
+        worst.append((new / old, k))
+    assert max(worst)[0] <= 1.1, worst
+
+
+def test_fp32_summaries_that_amplify_are_not_used(monkeypatch):
+    x = wkv7_inputs(1, 900, 2, 64, seed=6, resets=False, lengths=False)
+    boundary32(1, 900, 2)
+    x["w"][:] = -9.0
+    x["a"][:, 400:560] = 0.0
+    x["a"][:, 400:560, :, 5] = 1.0
+    x["b"][:, 400:560] = (0.03 * x["a"][:, 400:560]).astype(np.float32)
+    ref, got, base = oracle32(x, True), run32(x, True, True, monkeypatch), run32(x, True, False, monkeypatch)
+    for k in ref:
+        assert rms(got[k] - ref[k]) <= 1.1 * rms(base[k] - ref[k]), k
