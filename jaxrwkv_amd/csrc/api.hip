@@ -1033,8 +1033,8 @@ int hiprwkv_wkv4_mix_bwd(hiprwkv_stream stream, int io_dtype, int64_t B, int64_t
 }
 
 int hiprwkv_gemm(hiprwkv_stream stream, int n_jobs, const hiprwkv_gemm_job* jobs) {
-  if (n_jobs <= 0 || n_jobs > GEMM_MAX_JOBS || jobs == nullptr)
-    return fail(HIPRWKV_EINVAL, "gemm: 1 to %d jobs", GEMM_MAX_JOBS);
+  if (n_jobs <= 0 || n_jobs > HIPRWKV_GEMM_MAX_JOBS || jobs == nullptr)
+    return fail(HIPRWKV_EINVAL, "gemm: 1 to %d jobs", HIPRWKV_GEMM_MAX_JOBS);
   GemmArgs A;
   memset(&A, 0, sizeof(A));
   A.n_jobs = n_jobs;
@@ -1050,7 +1050,7 @@ int hiprwkv_gemm(hiprwkv_stream stream, int n_jobs, const hiprwkv_gemm_job* jobs
       if (p == nullptr || !aligned16(p)) return fail(HIPRWKV_EINVAL, "gemm: job %d: null or misaligned tensor pointer (16 bytes)", i);
     if (J.aux != nullptr && !aligned16(J.aux)) return fail(HIPRWKV_EINVAL, "gemm: job %d: misaligned tensor pointer (16 bytes)", i);
     tiles += (int64_t)((J.N + 511) / 512 * 8) * ((J.M + 511) / 512 * 8);
-    A.job[i] = J;
+    static_cast<hiprwkv_gemm_job&>(A.job[i]) = J;
   }
   if (tiles > 0x7fffffffLL) return fail(HIPRWKV_EINVAL, "gemm: too many tiles for one launch");
   return gate_done("gemm", launch_gemm(A, 1, static_cast<hipStream_t>(stream)));

@@ -207,8 +207,11 @@ __device__ __forceinline__ void finish(const GemmArgs& A, const GemmJob& J, int 
     for (int i = 0; i < 4; ++i) v[i] = rnd(v[i]);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      v[i] = J.act == GEMM_ADD ? v[i] + h[i] : J.act == GEMM_DTANH ? v[i] * (1.f - h[i] * h[i]) : v[i] * (h[i] * (1.f - h[i]));
+      v[i] = J.act == GEMM_ADD ? v[i] + h[i] : J.act == GEMM_DTANH ? v[i] * (1.f - h[i] * h[i])
+           : J.act == GEMM_DRELUSQ ? 2.f * v[i] * fmaxf(h[i], 0.f) : v[i] * (h[i] * (1.f - h[i]));
   } else {
+    if (J.raw != nullptr)
+      *reinterpret_cast<uint2*>(static_cast<bf16_t*>(J.raw) + el) = make_uint2(chunk::pack_rn(v[0], v[1]), chunk::pack_rn(v[2], v[3]));
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = activate(v[i], J.act);
   }
@@ -272,19 +275,19 @@ __device__ __forceinline__ void tile_gemm_body(const GemmArgs& A, const GemmJob&
 
 // job and tile of a workgroup: along the longer side of the tile grid eight tiles at a time, one per XCD; all tiles across from
 // each on the same XCD
-__device__ __forceinline__ bool tile_of(const GemmArgs& A, int tm, int& ji, int& n0, int& m0) {
+__device__ __forceinline__ bool tile_of(const GemmArgs& A, int tm, int tn, int& ji, int& n0, int& m0) {
   ji = 0;
   for (int i = 1; i < A.n_jobs; ++i) ji = (int)blockIdx.x >= A.job[i].tile0 ? i : ji;
   const int M = A.job[ji].M, N = A.job[ji].N;
-  const int mt = (M + tm - 1) / tm, nt = (N + TG - 1) / TG, local = (int)blockIdx.x - A.job[ji].tile0;
+  const int mt = (M + tm - 1) / tm, nt = (N + tn - 1) / tn, local = (int)blockIdx.x - A.job[ji].tile0;
   const int across = mt < nt ? mt : nt;
   const int p = local / (8 * across) * 8 + local % 8, q = local % (8 * across) / 8;
-  n0 = (mt < nt ? p : q) * TG;
+  n0 = (mt < nt ? p : q) * tn;
   m0 = (mt < nt ? q : p) * tm;
   return n0 < N && m0 < M;
 }
-int tiles_of(const GemmJob& J, int tm) {
-  const int mt = (J.M + tm - 1) / tm, nt = (J.N + TG - 1) / TG;
+int tiles_of(const GemmJob& J, int tm, int tn) {
+  const int mt = (J.M + tm - 1) / tm, nt = (J.N + tn - 1) / tn;
   return ((mt < nt ? nt : mt) + 7) / 8 * 8 * (mt < nt ? mt : nt);
 }
 
@@ -296,7 +299,7 @@ int tiles_of(const GemmJob& J, int tm) {
 // 64-row tiles, 19.9 with 128.  Bound by the wait for the weights (47 to 55 % of the waves' time in a step of 256 users,
 // profiles/rwkv7_model_bf16.md); five and seven steps in flight took as long, and so did a first step that differs from tile to
 // tile.
-constexpr int stream_step(int tm) { return (tm + TG) * TG; }       // bf16 values of a step in LDS: TM rows of x, TG of w
+constexpr int stream_step(int tm, int tn) { return (tm + tn) * TG; }     // bf16 values of a step in LDS: TM rows of x, TN of w
 typedef __attribute__((address_space(3))) uint16_t* lds_u16_ptr;
 
 // 16 bytes per lane to 1 KiB of LDS at `lds` (a wave-uniform address).  In assembly because the compiler waits for every request
@@ -305,32 +308,44 @@ __device__ __forceinline__ void request_lds(u32x4_t rs, int voff, int soff, uint
   asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(rs), "s"(soff), "{m0}"(lds) : "memory");
 }
 
-// ROWS (64 or 128) rows of m or n by 64 of k; with TR the operand lies k-major and so does its piece of LDS
+// ROWS (64 or 128) rows of m or n by 64 of k; with TR the operand lies k-major and so does its piece of LDS.  The last step of a K
+// that is no multiple of 64 asks for the last k again where there are no more; what it gives is masked (`keep`).
 template <bool TR, int ROWS>
 struct StreamOperand {
   static constexpr int PIECES = ROWS / 32;                           // requests of a wave per step
   static constexpr int PER_ROW = TR ? ROWS / 8 : TG / 8;             // 16-byte pieces of an LDS row
   static constexpr int LINES = 64 / PER_ROW;                         // LDS rows that a request fills
   u32x4_t rs;
-  int voff[PIECES], stride, last, at;
+  int voff[PIECES], stride, last, at, lane, R, over;
   static __device__ __forceinline__ int swizzle(int q) {
     return TR ? 2 * ((q ^ (q >> 3)) & 3) : (q & 3) | ((q >> 1) & 4);
   }
-  __device__ __forceinline__ StreamOperand(const void* base, int R, int K, int r0, int wave, int lane) {
-    last = K / TG - 1;
+  __device__ __forceinline__ StreamOperand(const void* base, int R_, int K, int r0, int wave, int lane_) : lane(lane_), R(R_) {
+    last = (K - 1) / TG;
+    over = (last + 1) * TG - K;                                      // of the last step
     stride = TR ? TG * R * 2 : TG * 2;
     const uint64_t first = reinterpret_cast<uint64_t>(static_cast<const bf16_t*>(base) + (TR ? (int64_t)r0 : (int64_t)r0 * K));
     rs = u32x4_t{(uint32_t)first, (uint32_t)(first >> 32) & 0xffffu, 0x7fffffffu, 0x00020000u};      // as make_rsrc
     at = wave * PIECES * 1024;
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
-      const int q = LINES * (PIECES * wave + i) + lane / PER_ROW, c = 8 * ((lane % PER_ROW) ^ swizzle(q));
+      const int q = line(i), c = column(i);
       voff[i] = TR ? (q * R + (r0 + c < R ? c : R - 8 - r0)) * 2 : ((r0 + q < R ? q : R - 1 - r0) * K + c) * 2;
     }
   }
+  __device__ __forceinline__ int line(int i) const { return LINES * (at / 1024 + i) + lane / PER_ROW; }
+  __device__ __forceinline__ int column(int i) const { return 8 * ((lane % PER_ROW) ^ swizzle(line(i))); }
   __device__ __forceinline__ void request(int s, uint16_t* lds) const {
     const int soff = (s < last ? s : last) * stride;
     const uint32_t to = (uint32_t)(uintptr_t)(lds_u16_ptr)(lds) + at;
+    if (s >= last && over != 0) {
+#pragma unroll
+      for (int i = 0; i < PIECES; ++i) {
+        const int k = TR ? line(i) : column(i), past = k - (TG - over - (TR ? 1 : 8));      // beyond the last that there is
+        request_lds(rs, voff[i] - (past > 0 ? past * (TR ? 2 * R : 2) : 0), soff, to + 1024 * i);
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) request_lds(rs, voff[i], soff, to + 1024 * i);
   }
@@ -345,80 +360,108 @@ struct StreamOperand {
     return *reinterpret_cast<const u32x4_t*>(lds + n * TG + 8 * ((4 * kh + g) ^ swizzle(n)));
   }
 };
+// v with its eight k (from k0 on) cleared from `end` on
+__device__ __forceinline__ u32x4_t keep_k(u32x4_t v, int k0, int end) {
+#pragma unroll
+  for (int c = 0; c < 4; ++c) v[c] = k0 + 2 * c + 1 < end ? v[c] : k0 + 2 * c < end ? v[c] & 0xffffu : 0u;
+  return v;
+}
 
-// TM x 64 tiles, four waves of TM/2 x 32
-template <int TM, int BUFS, bool KM, bool KN>
+// TM x TN tiles, four waves of TM/2 x TN/2
+template <int TM, int TN, int BUFS, bool KM, bool KN>
 __device__ __forceinline__ void stream_gemm_body(const GemmArgs& A, const GemmJob& J, int n0, int m0, uint16_t* lds) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-  constexpr int MT = TM / 32, STEP = stream_step(TM), IN_STEP = TM / 32 + TG / 32;
-  const int all = J.K / TG;
+  constexpr int MT = TM / 32, NT = TN / 32, STEP = stream_step(TM, TN), IN_STEP = TM / 32 + TN / 32;
+  const int all = (J.K + TG - 1) / TG;
   const int s0 = all * (int)blockIdx.y / (int)gridDim.y, s1 = all * ((int)blockIdx.y + 1) / (int)gridDim.y;
   typedef StreamOperand<KM, TM> OpX;
-  typedef StreamOperand<KN, TG> OpW;
+  typedef StreamOperand<KN, TN> OpW;
   const OpX X(J.x, J.M, J.K, m0, wave, lane);
   const OpW W(J.w, J.N, J.K, n0, wave, lane);
-  f32x4_t acc[2][MT];
+  f32x4_t acc[NT][MT];
 #pragma unroll
-  for (int i = 0; i < 2 * MT; ++i) acc[i / MT][i % MT] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const int wn = 32 * (wave & 1), wm = TM / 2 * (wave >> 1);
+  for (int i = 0; i < NT * MT; ++i) acc[i / MT][i % MT] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int wn = TN / 2 * (wave & 1), wm = TM / 2 * (wave >> 1);
   auto request = [&](int s, int buf) {
     X.request(s, lds + buf * STEP);
     W.request(s, lds + buf * STEP + TM * TG);
   };
 #pragma unroll
   for (int j = 0; j < BUFS - 1; ++j) request(s0 + j, j);
-  auto step = [&](int s, int buf) {
-    // this wave's part of step s has arrived; after the barrier all parts, and nobody reads the buffer of step s - 1 any more
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(IN_STEP * (BUFS - 2)) : "memory");
-    request(s + BUFS - 1, (buf + BUFS - 1) % BUFS);
+  // `end`: k of this step that there are (64 but for the last step of a K that is no multiple of it)
+  auto compute = [&](int buf, bool whole, int end) {
     const uint16_t* const xs = lds + buf * STEP;
     const uint16_t* const ws = xs + TM * TG;
 #pragma unroll
     for (int kh = 0; kh < 2; ++kh) {
-      u32x4_t wf[2], xf[MT];
+      u32x4_t wf[NT], xf[MT];
 #pragma unroll
-      for (int t = 0; t < 2; ++t) wf[t] = OpW::frag(ws, wn + 16 * t + (KN ? 4 * (r & 3) : r), kh, r, g);
+      for (int t = 0; t < NT; ++t) wf[t] = OpW::frag(ws, wn + 16 * t + (KN ? 4 * (r & 3) : r), kh, r, g);
 #pragma unroll
       for (int u = 0; u < MT; ++u) xf[u] = OpX::frag(xs, wm + 16 * u + (KM ? 4 * (r & 3) : r), kh, r, g);
+      if (!whole) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) wf[t] = keep_k(wf[t], 32 * kh + 8 * g, end);
+#pragma unroll
+        for (int u = 0; u < MT; ++u) xf[u] = keep_k(xf[u], 32 * kh + 8 * g, end);
+      }
 #pragma unroll
       for (int u = 0; u < MT; ++u)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) acc[t][u] = mfma(wf[t], xf[u], acc[t][u]);
+        for (int t = 0; t < NT; ++t) acc[t][u] = mfma(wf[t], xf[u], acc[t][u]);
     }
   };
+  auto arrive = [&](int s, int buf) {
+    // this wave's part of step s has arrived; after the barrier all parts, and nobody reads the buffer of step s - 1 any more
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(IN_STEP * (BUFS - 2)) : "memory");
+    request(s + BUFS - 1, (buf + BUFS - 1) % BUFS);
+  };
+  const int tail = s1 == all && J.K % TG != 0 ? 1 : 0, sw = s1 - tail;          // whole steps
   int s = s0;
-  for (; s + BUFS <= s1; s += BUFS)
+  for (; s + BUFS <= sw; s += BUFS)
 #pragma unroll
-    for (int j = 0; j < BUFS; ++j) step(s + j, j);
+    for (int j = 0; j < BUFS; ++j) {
+      arrive(s + j, j);
+      compute(j, true, TG);
+    }
+  int buf = 0;
 #pragma unroll
   for (int j = 0; j < BUFS - 1; ++j)
-    if (s + j < s1) step(s + j, j);
+    if (s + j < sw) {
+      arrive(s + j, j);
+      compute(j, true, TG);
+      buf = j + 1;
+    }
+  if (tail) {
+    arrive(s1 - 1, buf);
+    compute(buf, false, J.K % TG);
+  }
   // the requests beyond the last step write to LDS as well: none may be under way when the workgroup gives its LDS back
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int u = 0; u < MT; ++u) finish(A, J, n0 + wn + 16 * t + 4 * g, m0 + wm + 16 * u + r, acc[t][u]);
 }
 
-template <int TM, int BUFS>
+template <int TM, int TN, int BUFS>
 __global__ __launch_bounds__(256) void stream_gemm_kernel(GemmArgs A) {
   extern __shared__ __align__(1024) uint16_t stream_lds[];
   int ji, n0, m0;
-  if (!tile_of(A, TM, ji, n0, m0)) return;
+  if (!tile_of(A, TM, TN, ji, n0, m0)) return;
   const GemmJob J = A.job[ji];
   switch ((J.km ? 2 : 0) + (J.kn ? 1 : 0)) {
-    case 0: stream_gemm_body<TM, BUFS, false, false>(A, J, n0, m0, stream_lds); break;
-    case 1: stream_gemm_body<TM, BUFS, false, true>(A, J, n0, m0, stream_lds); break;
-    case 2: stream_gemm_body<TM, BUFS, true, false>(A, J, n0, m0, stream_lds); break;
-    default: stream_gemm_body<TM, BUFS, true, true>(A, J, n0, m0, stream_lds); break;
+    case 0: stream_gemm_body<TM, TN, BUFS, false, false>(A, J, n0, m0, stream_lds); break;
+    case 1: stream_gemm_body<TM, TN, BUFS, false, true>(A, J, n0, m0, stream_lds); break;
+    case 2: stream_gemm_body<TM, TN, BUFS, true, false>(A, J, n0, m0, stream_lds); break;
+    default: stream_gemm_body<TM, TN, BUFS, true, true>(A, J, n0, m0, stream_lds); break;
   }
 }
-template <int TM, int BUFS>
+template <int TM, int TN, int BUFS>
 hipError_t launch_stream(const GemmArgs& A, int tiles, int split, hipStream_t stream) {
   static LdsAttrOnce attr;
-  constexpr size_t bytes = (size_t)BUFS * stream_step(TM) * 2;
-  const auto kernel = stream_gemm_kernel<TM, BUFS>;
+  constexpr size_t bytes = (size_t)BUFS * stream_step(TM, TN) * 2;
+  const auto kernel = stream_gemm_kernel<TM, TN, BUFS>;
   hipError_t e = allow_dynamic_lds(attr, reinterpret_cast<const void*>(kernel), bytes);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(kernel, dim3(tiles, split), dim3(256), bytes, stream, A);
@@ -428,7 +471,7 @@ hipError_t launch_stream(const GemmArgs& A, int tiles, int split, hipStream_t st
 __global__ __launch_bounds__(256) void tile_gemm_kernel(GemmArgs A) {
   __shared__ __align__(16) TileLds lds;
   int ji, n0, m0;
-  if (!tile_of(A, TG, ji, n0, m0)) return;
+  if (!tile_of(A, TG, TG, ji, n0, m0)) return;
   const GemmJob J = A.job[ji];
   switch ((J.km ? 4 : 0) + (J.kn ? 2 : 0) + (J.K % TG == 0 ? 1 : 0)) {
     case 0: tile_gemm_body<false, false, false>(A, J, n0, m0, lds); break;
@@ -456,36 +499,72 @@ int gemm_split(int M, int64_t K, int64_t N) {
 // Up to 32 rows the streaming kernel (K a multiple of 32, N of 16, no aux): its operand loads touch a cache line per lane,
 // 64 cycles a KiB, which a stream of weights can afford but repeated reads of x cannot (8192 columns of 2048: 14 us at 32
 // rows, 16 at 33, 21 at 64; tiled 15 us up to 128 rows, 22 at 256).
-// From 33 rows the tiles: through registers only where some K of the launch is no multiple of a step (the second low-rank factors),
-// else straight to LDS, which was never slower (48 to 4084 rows, 768 to 2048 channels).  128-row tiles, which read the weights
-// half as often, where they are one round that fills the GPU: below that 64-row tiles use more CUs (256 rows of 1024 channels), above
-// it the last round is nearly empty (4084 rows into the low-rank sizes: 288 tiles 37 us, 576 small ones 34, through registers 36).
+// From 33 rows tiles, straight to LDS (through registers where an operand of a narrow K is no multiple of a step: the second low-rank
+// factors, which the other kernel would mostly mask).  Which: a CU's LDS is the bound (the operands of a step are written at 64 bytes a
+// cycle and read twice at 128: 4 (TM + TN) cycles a step, measured 0.29 us for 64 x 64, 0.40 for 128 x 64, 0.59 for 128 x 128), so the
+// tile that takes the fewest steps a CU times TM + TN.  Products of one K run in rounds over the CUs; of several, the longest or the
+// mean counts and 128 x 128 tiles leave too few to balance.  Weights that no cache holds, us with 64x64, 128x64, 128x128 tiles:
+// 2048 rows: three 768x768 22.2 / 20.2 / 17.9, 768 into 3072 23.1 / 19.2 / 17.4, 3072 into 768 24.0 / 25.5 / 33; with the weights'
+// cotangents: of 768x768 14.0 / 17.0 / 29, of three 41 / 36.6 / 44, of 3072 into 768 43 / 35 / 40.  512 rows: 2048 into 8192 36 / 29 / 25,
+// 8192 into 2048 37 / 52 / 75.  4084 rows: three 2048x2048 225 / 161 / 116.  256 rows of 2048 into 8192: 21 / 18.8 / 24.  The
+// wait of a step is not it: four steps in flight took as long as three (one workgroup per CU), and so did reading half a step ahead
+// of its products.
 constexpr int CUS = 256, WIDE_TILES = 192;
 hipError_t launch_gemm(GemmArgs A, int split, hipStream_t stream) {
-  bool skinny = A.part == nullptr, stream_k = true;
-  int M = 0, tiles = 0;
+  bool skinny = A.part == nullptr, stream_k = true, same_k = true;
+  int M = 0, longest = 0, tiles = 0;
+  // the longest first: what is left at the end is short
+  for (int i = 1; i < A.n_jobs; ++i)
+    for (int j = i; j > 0 && A.job[j].K > A.job[j - 1].K; --j) { const GemmJob t = A.job[j]; A.job[j] = A.job[j - 1]; A.job[j - 1] = t; }
   for (int i = 0; i < A.n_jobs; ++i) {
     const GemmJob& J = A.job[i];
     M = J.M > M ? J.M : M;
-    stream_k = stream_k && J.K % TG == 0;
-    skinny = skinny && J.M < GEMM_TILE_ROWS && !J.km && J.aux == nullptr && J.K % 32 == 0 && J.N % 16 == 0;
+    longest = J.K > longest ? J.K : longest;
+    same_k = same_k && J.K == A.job[0].K;
+    stream_k = stream_k && (J.K % TG == 0 || J.K >= 4 * TG);
+    skinny = skinny && J.M < GEMM_TILE_ROWS && !J.km && J.aux == nullptr && J.raw == nullptr && J.K % 32 == 0 && J.N % 16 == 0;
   }
-  auto place = [&](int tm) {
+  auto place = [&](int tm, int tn) {
     tiles = 0;
     for (int i = 0; i < A.n_jobs; ++i) {
       GemmJob& J = A.job[i];
       J.tile0 = tiles;
-      tiles += skinny ? J.N / 16 : tiles_of(J, tm);
+      tiles += skinny ? J.N / 16 : tiles_of(J, tm, tn);
     }
   };
   const dim3 block(64 * GEMM_WAVES);
-  if (!skinny && stream_k) {
-    place(2 * TG);
-    if (M > TG && tiles * split >= WIDE_TILES && tiles * split <= CUS) return launch_stream<2 * TG, 4>(A, tiles, split, stream);
-    place(TG);
-    return launch_stream<TG, 4>(A, tiles, split, stream);
+  if (!skinny && stream_k && (split > 1 || A.part != nullptr)) {
+    place(2 * TG, TG);
+    if (M > TG && tiles * split >= WIDE_TILES && tiles * split <= CUS) return launch_stream<2 * TG, TG, 4>(A, tiles, split, stream);
+    place(TG, TG);
+    return launch_stream<TG, TG, 4>(A, tiles, split, stream);
   }
-  place(TG);
+  if (!skinny && stream_k) {
+    auto cost = [&](int tm, int tn) {
+      int64_t n = 0, steps = 0, area = 0;
+      for (int i = 0; i < A.n_jobs; ++i) {
+        const int64_t t = tiles_of(A.job[i], tm, tn);
+        n += t;
+        area += (int64_t)A.job[i].M * A.job[i].N;
+        steps += t * ((A.job[i].K + TG - 1) / TG);
+      }
+      const int64_t one = (longest + TG - 1) / TG, mean = (steps + CUS - 1) / CUS;
+      if (tn > TG && 100 * area < 85 * n * tm * tn) return INT64_MAX;         // mostly edges (the low-rank inputs alone: 38 us and 34)
+      return (same_k ? (n + CUS - 1) / CUS * one : mean > one ? mean : one) * (tm + tn);
+    };
+    const int64_t small = cost(TG, TG), wide = M > TG ? cost(2 * TG, TG) : small, large = M > TG && same_k ? cost(2 * TG, 2 * TG) : wide;
+    if (large < wide && large < small) {
+      place(2 * TG, 2 * TG);
+      return tiles > CUS ? launch_stream<2 * TG, 2 * TG, 2>(A, tiles, split, stream) : launch_stream<2 * TG, 2 * TG, 3>(A, tiles, split, stream);
+    }
+    if (wide < small) {
+      place(2 * TG, TG);
+      return tiles > CUS ? launch_stream<2 * TG, TG, 3>(A, tiles, split, stream) : launch_stream<2 * TG, TG, 4>(A, tiles, split, stream);
+    }
+    place(TG, TG);
+    return launch_stream<TG, TG, 4>(A, tiles, split, stream);
+  }
+  place(TG, TG);
   if (!skinny) hipLaunchKernelGGL(tile_gemm_kernel, dim3(tiles, split), dim3(256), 0, stream, A);
   else if (M <= 16) hipLaunchKernelGGL(skinny_gemm_kernel<1>, dim3(tiles), block, 0, stream, A);
   else hipLaunchKernelGGL(skinny_gemm_kernel<2>, dim3(tiles), block, 0, stream, A);

@@ -168,11 +168,13 @@ hipError_t launch_rwkv7_pre(int io_f32, const PreArgs& A, hipStream_t stream);
 hipError_t launch_rwkv7_pre_bwd(int io_f32, const PreArgs& A, void* const* dparam, hipStream_t stream);
 
 // Several products per launch (rwkv7_gemm.hip), bf16: out[m][n] = f(sum_k x(m, k) w(n, k)).  The job is the C ABI's
-// (hiprwkv_gemm_job); tile0 is the launcher's.
-using GemmJob = ::hiprwkv_gemm_job;
+// (hiprwkv_gemm_job) and more; tile0 is the launcher's.
+struct GemmJob : ::hiprwkv_gemm_job {
+  void* raw;           // without aux: the product itself, beside f of it in out; may be null
+};
 constexpr int GEMM_ACT_NONE = 0, GEMM_ACT_TANH = 1, GEMM_ACT_SIGMOID = 2, GEMM_ACT_RELUSQ = 3;      // f without aux
-constexpr int GEMM_ADD = 0, GEMM_DTANH = 1, GEMM_DSIGMOID = 2;                                      // f with aux
-constexpr int GEMM_MAX_JOBS = HIPRWKV_GEMM_MAX_JOBS;
+constexpr int GEMM_ADD = 0, GEMM_DTANH = 1, GEMM_DSIGMOID = 2, GEMM_DRELUSQ = 3;                    // f with aux
+constexpr int GEMM_MAX_JOBS = 12;
 constexpr int GEMM_TILE_ROWS = 33;     // rows from which the kernel with LDS tiles takes over
 constexpr int GEMM_MAX_SPLIT = 8;
 struct GemmArgs {

@@ -54,3 +54,26 @@ def test_tanh_of_small_values(M, K):
     blocks7._gemm([(out, x, w, 0, 1, 1, None)])
     want = torch.tanh((x.double() @ w.double()).bfloat16().double())
     assert ((out.double() - want).abs() <= 2.0 ** -8 * want.abs()).all()
+
+
+# a last step that is not full, in each tile: 64 x 64, 128 x 64, 128 x 128 with three buffers and with two
+@pytest.mark.parametrize("km,kn", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N", [(72, 136), (264, 2056), (2048, 776), (2056, 2312)])
+@pytest.mark.parametrize("K", [256, 264, 376, 520])
+def test_product_of_any_k(M, N, K, km, kn):
+    from jaxrwkv_amd import blocks7
+    K += 1 if km and kn and K > 256 else 0                # without rows of k, K may be odd
+    g = torch.Generator("cuda").manual_seed(M + N + K)
+
+    def operand(rows, k_major):                           # what lies behind the last k of an operand must not be seen
+        shape, used = ((K + 64, rows), slice(0, K)) if k_major else ((rows + 1, K), slice(0, rows))
+        full = torch.randn(shape, device="cuda", generator=g).bfloat16()
+        full[used.stop:] = float("nan")
+        return full[used]
+    x, w = operand(M, km), operand(N, kn)
+    guard = torch.full((M + 2, N), 7.0, device="cuda", dtype=torch.bfloat16)
+    blocks7._gemm([(guard[1:-1], x, w, km, kn, 0, None)])
+    want = (x.double().T if km else x.double()) @ (w.double() if kn else w.double().T)
+    d = (guard[1:-1].double() - want).abs()
+    assert (d <= want.abs() * 2.0 ** -8 + 2.0 ** -18 * K ** 0.5).all()
+    assert (guard[0] == 7).all() and (guard[-1] == 7).all()
