@@ -426,6 +426,40 @@ typedef struct hiprwkv_rwkv7_decode_args {
 size_t hiprwkv_rwkv7_decode_workspace_bytes(const hiprwkv_rwkv7_decode_args* args);
 int hiprwkv_rwkv7_decode(hiprwkv_stream stream, const hiprwkv_rwkv7_decode_args* args);
 
+/* ---- The stack of RWKV-7 blocks over whole sequences -------------------------------------
+ * rwkv7.py:190-198, :223-291 without the norms around the stack, bf16, all tokens of B sequences through L layers.  C = 64 H, at most
+ * 4096; F and the four inner sizes multiples of 8; no array of 2 GiB or more; parameters stacked over the layers, one contiguous array
+ * each, in the orders of hiprwkv_rwkv7_decode_args.
+ *   forward : from x (B,T,C) and the states the residual stream as a sum xs + dx.  state (B,L,2+64,C): rows 0 and 1 are the token-shift
+ *             states, read there and written in new_state; s, new_s (L,B,64,C): the recurrence's, as arrays of their own.
+ *             saved: L allocations of hiprwkv_rwkv7_stack_saved_bytes for the backward, or null without one to come.
+ *   backward: from g_xs, g_dx and, where not null, the cotangents of the new shift states g_shift (2,L,B,C) and recurrence states g_s
+ *             (L,B,64,C) to g_x and every parameter's (grad, same order as param; rows of layer 0 of v0, v1, v2 are left alone).  The
+ *             forward's x, xs, state, s and saved go in again; there is no cotangent of the states. */
+typedef struct hiprwkv_rwkv7_block_params {
+  const void *x_r, *x_w, *x_k, *x_v, *x_a, *x_g;
+  const void *w0, *w1, *w2, *a0, *a1, *a2, *v0, *v1, *v2, *g1, *g2, *k_k, *k_a, *r_k;
+  const void *receptance, *key, *value, *output, *lnx_w, *lnx_b, *ffn_x_k, *ffn_key, *ffn_value, *ln1_w, *ln1_b, *ln2_w, *ln2_b;
+} hiprwkv_rwkv7_block_params;
+typedef struct hiprwkv_rwkv7_stack_args {
+  int64_t B, T, L, C, H, F, d_decay, d_aaa, d_mv, d_gate;
+  const void *x, *state, *s;
+  void *new_state, *new_s;
+  const int32_t* length;
+  const uint8_t* new_starts;
+  void *xs, *dx;
+  void* const* saved;
+  void* workspace;
+  uint64_t workspace_bytes, flags;
+  const void *g_xs, *g_dx, *g_shift, *g_s;
+  void* g_x;
+  hiprwkv_rwkv7_block_params param, grad;
+} hiprwkv_rwkv7_stack_args;
+size_t hiprwkv_rwkv7_stack_saved_bytes(const hiprwkv_rwkv7_stack_args* args);
+size_t hiprwkv_rwkv7_stack_workspace_bytes(const hiprwkv_rwkv7_stack_args* args, int backward);
+int hiprwkv_rwkv7_stack_fwd(hiprwkv_stream stream, const hiprwkv_rwkv7_stack_args* args);
+int hiprwkv_rwkv7_stack_bwd(hiprwkv_stream stream, const hiprwkv_rwkv7_stack_args* args);
+
 /* ---- RWKV-7 time-mixing stages around the op ------------------------------------------
  * The element-wise work the reference does in jnp on either side of inner_loop (rwkv7.py:248-252, 257 and :263-265),
  * fused into one pass each; it has no counterpart among the reference's ffi targets.  `rows` = number of tokens

@@ -39,6 +39,14 @@ class GemmJob(ctypes.Structure):
                 + [(n, ctypes.c_int32) for n in ("M", "N", "K", "km", "kn", "act", "tile0", "pad")])
 
 
+class Rwkv7StackArgs(ctypes.Structure):
+    """``hiprwkv_rwkv7_stack_args``; ``param`` and ``grad`` in the order of blocks7.NAMES"""
+    _fields_ = ([(n, _i64) for n in "B T L C H F d_decay d_aaa d_mv d_gate".split()]
+                + [(n, _vp) for n in "x state s new_state new_s length new_starts xs dx saved workspace".split()]
+                + [("workspace_bytes", ctypes.c_uint64), ("flags", ctypes.c_uint64)]
+                + [(n, _vp) for n in "g_xs g_dx g_shift g_s g_x".split()] + [("param", _vp * 33), ("grad", _vp * 33)])
+
+
 # name -> (restype, argtypes); mirrors include/hiprwkv.h declaration by declaration
 SIGNATURES = {
     "hiprwkv_last_error": (ctypes.c_char_p, []),
@@ -100,6 +108,10 @@ SIGNATURES = {
     "hiprwkv_gemm": (_int, [_vp, _int, ctypes.POINTER(GemmJob)]),
     "hiprwkv_rwkv7_decode_workspace_bytes": (_sz, [ctypes.POINTER(Rwkv7DecodeArgs)]),
     "hiprwkv_rwkv7_decode": (_int, [_vp, ctypes.POINTER(Rwkv7DecodeArgs)]),
+    "hiprwkv_rwkv7_stack_saved_bytes": (_sz, [ctypes.POINTER(Rwkv7StackArgs)]),
+    "hiprwkv_rwkv7_stack_workspace_bytes": (_sz, [ctypes.POINTER(Rwkv7StackArgs), _int]),
+    "hiprwkv_rwkv7_stack_fwd": (_int, [_vp, ctypes.POINTER(Rwkv7StackArgs)]),
+    "hiprwkv_rwkv7_stack_bwd": (_int, [_vp, ctypes.POINTER(Rwkv7StackArgs)]),
     "hiprwkv_rwkv7_premix": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 7),
     "hiprwkv_rwkv7_postmix": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 8 + [ctypes.c_float, _vp]),
     "hiprwkv_rwkv7_premix_bwd": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 11),

@@ -6,6 +6,8 @@ written out over the library's kernels and ``torch.mm``, writes every layer's pa
 stacked arrays, and adds up nothing that a kernel can add on its way (the second cotangents of r, k and v, the value
 residual's).  The low-rank factors of decay, gates and value residual run several to a launch (``hiprwkv_gemm``) in bf16.
 """
+import ctypes
+
 import torch
 from torch.autograd.function import once_differentiable
 
@@ -372,9 +374,111 @@ def covers(params, x, state):
                and p[f + "1"].numel() == p[f + "2"].numel() == n * p[f + "1"].shape[-1] for f in "wavg")
 
 
+#: rows x channels^2 up to which the stack is launched from native code.  A layer costs the host 0.3 ms forward (and 0.8 backward)
+#: from Python; its products, which are this package's own there, take that time at 1600 rows of 2048 channels, and the library's,
+#: which the separate steps use, are a fifth faster beyond.
+NATIVE_ROWS_C2, NATIVE_ROWS = 6 * 10 ** 9, 8192
+
+
+def _native(params, x, state, grad):
+    """Whether native code launches the stack (``hiprwkv_rwkv7_stack_args``): bf16, all parameters or none trained and not the state,
+    the shapes that the model has (the separate steps take any that multiply), channels in whole 128-column tiles."""
+    B, T, C = x.shape
+    M = B * T
+    p = dict(zip(NAMES, params))
+    L, H, N = p["r_k"].shape
+    F = p["ffn_key"].shape[1]
+    sizes = (F, *(p[f + "1"].shape[-1] for f in "wavg"))
+    shapes = {"ffn_key": (L, F, C), "ffn_value": (L, C, F)}
+    return (x.dtype == torch.bfloat16 and M * C * C <= NATIVE_ROWS_C2 and M <= NATIVE_ROWS and T > 8 and N == 64 and C == H * N
+            and C % 128 == 0 and F <= 8 * C and all(d % 8 == 0 for d in sizes) and state.shape == (B, L, 2 + N, C)
+            and state.is_contiguous() and state.data_ptr() % 16 == 0 and not ops.autocast_elsewhere(x)
+            and all(p[n].shape == shapes.get(n, (L, C, C)) for n in _PRODUCTS)
+            and not (grad and (state.requires_grad or not all(t.requires_grad for t in params))))
+
+
+def _stack_args(x, state, s, ns, length, params, xs):
+    """The arguments that both directions share."""
+    p = dict(zip(NAMES, params))
+    (L, H, _), (B, T, C) = p["r_k"].shape, x.shape
+    A = _lib.Rwkv7StackArgs(B=B, T=T, L=L, C=C, H=H, F=p["ffn_key"].shape[1], d_decay=p["w1"].shape[-1], d_aaa=p["a1"].shape[-1],
+                            d_mv=p["v1"].shape[-1], d_gate=p["g1"].shape[-1])
+    A.x, A.state, A.s, A.length, A.new_starts, A.xs = map(ops._p, (x, state, s, length, ns, xs))
+    A.param[:] = [t.data_ptr() for t in params]
+    return A
+
+
+def _stack_fwd(x, state, ns, length, params, compat, keep):
+    """Returns (xs, dx, new_state) and, with ``keep``, what the backward reads besides them and the arguments."""
+    lib = _lib.load()
+    x = ops._aligned(x.contiguous())
+    s = state[:, :, 2:].transpose(0, 1).contiguous()
+    xs, dx, new_s, new_state = torch.empty_like(x), torch.empty_like(x), torch.empty_like(s), torch.empty_like(state)
+    A = _stack_args(x, state, s, ns, length, params, xs)
+    A.dx, A.new_s, A.new_state, A.flags = dx.data_ptr(), new_s.data_ptr(), new_state.data_ptr(), _lib.COMPAT_ASSOC if compat else 0
+    nbytes = lib.hiprwkv_rwkv7_stack_saved_bytes(ctypes.byref(A)) if keep else 0
+    saved = [ops._workspace(nbytes, x.device) for _ in range(A.L if keep else 0)]
+    arr = ops._ptr_array(saved)
+    A.saved = ctypes.addressof(arr) if keep else None
+    A.workspace_bytes = lib.hiprwkv_rwkv7_stack_workspace_bytes(ctypes.byref(A), 0)
+    ws = ops._workspace(A.workspace_bytes, x.device)
+    A.workspace = ws.data_ptr()
+    _lib.check(lib.hiprwkv_rwkv7_stack_fwd(ops._stream(), ctypes.byref(A)), "hiprwkv_rwkv7_stack_fwd")
+    new_state[:, :, 2:].copy_(new_s.transpose(0, 1))
+    return xs, dx, new_state, (x, xs, s, *saved)
+
+
+class _Stack(torch.autograd.Function):
+    """``_Blocks`` launched from native code."""
+
+    @staticmethod
+    def forward(ctx, x, state, ns, length, compat, *params):
+        ctx.set_materialize_grads(False)
+        xs, dx, new_state, saved = _stack_fwd(x, state, ns, length, params, compat, True)
+        ctx.compat, ctx.n = compat, len(saved)
+        ctx.save_for_backward(*saved, state, ns, length, *params)
+        return xs, dx, new_state
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, g_x, g_dx, g_state):
+        lib = _lib.load()
+        tensors = ctx.saved_tensors
+        x, xs, s, *saved = map(ops._aligned, tensors[:ctx.n])
+        state, ns, length, *params = tensors[ctx.n:]
+        state = ops._aligned(state.contiguous())                      # a saved-tensor hook may have moved it
+        params = [ops._aligned(t.contiguous()) for t in params]
+        A = _stack_args(x, state, s, ns, length, params, xs)
+        g_x, g_dx = (torch.zeros_like(x) if g is None else ops._aligned(ops._dev(g, x.dtype)) for g in (g_x, g_dx))
+        if g_state is not None:
+            g_state = g_state.to(x.dtype).transpose(0, 1)
+            g_shift, g_s = g_state[:, :, :2].permute(2, 0, 1, 3).contiguous(), g_state[:, :, 2:].contiguous()
+            A.g_shift, A.g_s = g_shift.data_ptr(), g_s.data_ptr()
+        residual = ("v0", "v1", "v2")                                 # the first layer has no value residual
+        grads = [None if A.L == 1 and n in residual else torch.empty_like(t) for n, t in zip(NAMES, params)]
+        for n, g in zip(NAMES, grads):
+            if g is not None and n in residual:
+                g[0].zero_()
+        A.grad[:] = [ops._p(g) for g in grads]
+        out = torch.empty_like(x)
+        A.g_xs, A.g_dx, A.g_x, A.flags = g_x.data_ptr(), g_dx.data_ptr(), out.data_ptr(), _lib.COMPAT_ASSOC if ctx.compat else 0
+        arr = ops._ptr_array(saved)
+        A.saved = ctypes.addressof(arr)
+        A.workspace_bytes = lib.hiprwkv_rwkv7_stack_workspace_bytes(ctypes.byref(A), 1)
+        ws = ops._workspace(A.workspace_bytes, x.device)
+        A.workspace = ws.data_ptr()
+        _lib.check(lib.hiprwkv_rwkv7_stack_bwd(ops._stream(), ctypes.byref(A)), "hiprwkv_rwkv7_stack_bwd")
+        return (out if ctx.needs_input_grad[0] else None, None, None, None, None, *grads)
+
+
 def run(params, x, state, ns, length, grad):
     """The stack on x (B,T,C) and state (B,L,2+N,C): returns (x, dx, new_state) whose sum x + dx is the residual stream."""
     if grad:
         length = None if length is None else length.clone()          # the caller may change its own before the backward
+    if _native(params, x, state, grad):
+        if grad:
+            return _Stack.apply(x, state, ns, length, HipRWKV.assoc_compat, *params)
+        return _stack_fwd(x, state, ns, length, params, HipRWKV.assoc_compat, False)[:3]
+    if grad:
         return _Blocks.apply(x, state, ns, length, *params)
     return _run(x, state, ns, length, params, None)[:3]

@@ -935,6 +935,69 @@ int hiprwkv_rwkv7_decode(hiprwkv_stream stream, const hiprwkv_rwkv7_decode_args*
   return gate_done("rwkv7_decode", launch_rwkv7_decode(D, static_cast<hipStream_t>(stream)));
 }
 
+namespace {
+bool stack_sizes_ok(const hiprwkv_rwkv7_stack_args& D) {
+  for (int64_t n : {D.B, D.T, D.L, D.C, D.H, D.F, D.d_decay, D.d_aaa, D.d_mv, D.d_gate})
+    if (n <= 0 || n > 0x7fffffffLL) return false;
+  if (D.B * D.T > 0x7fffffffLL || D.H > 64 || D.C != D.H * 64) return false;
+  for (int64_t n : {D.F, D.d_decay, D.d_aaa, D.d_mv, D.d_gate})
+    if (n % 8 != 0 || std::max(n, D.C) * std::max(D.B * D.T, D.C) * 2 >= 0x7fffffffLL || n * 256 >= 0x7fffffffLL) return false;
+  return D.B * D.T * 256 < 0x7fffffffLL;
+}
+int check_stack(const char* op, const hiprwkv_rwkv7_stack_args* args, bool backward) {
+  if (args == nullptr) return fail(HIPRWKV_EINVAL, "%s: null arguments", op);
+  const hiprwkv_rwkv7_stack_args& D = *args;
+  if (!stack_sizes_ok(D)) return fail(HIPRWKV_EINVAL, "%s: sizes must be positive, C = 64 H at most 4096, inner sizes multiples of 8, arrays below 2 GiB", op);
+  if (D.flags & ~(uint64_t)HIPRWKV_COMPAT_ASSOC) return fail(HIPRWKV_EINVAL, "%s: unknown flag bits", op);
+  const void* req[] = {D.x, D.state, D.s, D.xs, D.workspace};
+  const void* fwd[] = {D.new_state, D.new_s, D.dx};
+  const void* bwd[] = {D.g_xs, D.g_dx, D.g_x};
+  bool ok = true;
+  for (const void* p : req) ok = ok && p != nullptr && aligned16(p);
+  for (const void* p : backward ? bwd : fwd) ok = ok && p != nullptr && aligned16(p);
+  for (const void* p : {D.g_shift, D.g_s}) ok = ok && (p == nullptr || aligned16(p));
+  constexpr int n = sizeof(D.param) / sizeof(void*);
+  const void* const* par = reinterpret_cast<const void* const*>(&D.param);
+  const void* const* gra = reinterpret_cast<const void* const*>(&D.grad);
+  for (int i = 0; i < n; ++i) {
+    const void* const* const of_v = par + i;
+    const bool residual = of_v == &D.param.v0 || of_v == &D.param.v1 || of_v == &D.param.v2;
+    ok = ok && par[i] != nullptr && aligned16(par[i]);
+    if (backward) ok = ok && (gra[i] != nullptr ? aligned16(gra[i]) : residual && D.L == 1);
+  }
+  if (backward && D.saved == nullptr) ok = false;
+  for (int64_t l = 0; ok && D.saved != nullptr && l < D.L; ++l) ok = D.saved[l] != nullptr && aligned16(D.saved[l]);
+  if (!ok) return fail(HIPRWKV_EINVAL, "%s: null or misaligned tensor pointer (16 bytes)", op);
+  if (!backward && (D.state == D.new_state || D.s == D.new_s)) return fail(HIPRWKV_EINVAL, "%s: states and new states must be different arrays", op);
+  const size_t need = rwkv7_stack_workspace(D, backward);
+  if (D.workspace_bytes < need)
+    return fail(HIPRWKV_ENOSPACE, "%s: workspace has %llu bytes, %zu needed", op, (unsigned long long)D.workspace_bytes, need);
+  return HIPRWKV_OK;
+}
+}  // namespace
+
+size_t hiprwkv_rwkv7_stack_saved_bytes(const hiprwkv_rwkv7_stack_args* args) {
+  return args == nullptr || !stack_sizes_ok(*args) ? 0 : rwkv7_stack_saved(*args);
+}
+
+size_t hiprwkv_rwkv7_stack_workspace_bytes(const hiprwkv_rwkv7_stack_args* args, int backward) {
+  return args == nullptr || !stack_sizes_ok(*args) ? 0 : rwkv7_stack_workspace(*args, backward != 0);
+}
+
+int hiprwkv_rwkv7_stack_fwd(hiprwkv_stream stream, const hiprwkv_rwkv7_stack_args* args) {
+  if (int rc = check_stack("rwkv7_stack_fwd", args, false)) return rc;
+  hipError_t e = hipSuccess;
+  if (int rc = launch_rwkv7_stack_fwd(*args, static_cast<hipStream_t>(stream), e)) return rc;
+  return gate_done("rwkv7_stack_fwd", e);
+}
+
+int hiprwkv_rwkv7_stack_bwd(hiprwkv_stream stream, const hiprwkv_rwkv7_stack_args* args) {
+  if (int rc = check_stack("rwkv7_stack_bwd", args, true)) return rc;
+  hipError_t e = hipSuccess;
+  if (int rc = launch_rwkv7_stack_bwd(*args, static_cast<hipStream_t>(stream), e)) return rc;
+  return gate_done("rwkv7_stack_bwd", e);
+}
+
 // ---- WKV4 with the receptance applied, sequences cut into parts where the batch leaves the GPU idle
 namespace {
 size_t wkv4_part_bytes(int64_t B, int64_t T, int64_t C, int floats) {

@@ -128,7 +128,24 @@ __global__ __launch_bounds__(PRE_THREADS) void rwkv7_pre_bwd_kernel(PreArgs A) {
         o[c] = gv[c] * (vf[c] - v[c]) * s * (1.f - s);
         part[NP - 1][c] = fmaf(lv, o[c], part[NP - 1][c]);
       }
+      if (A.gvf != nullptr) {
+        float y[8];
+        in(A.gvf, el, y);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) o2[c] += y[c];
+      }
       put(A.dv, o1); put(A.dvf, o2); put(A.dxv, o);
+    } else if (A.dv_sum != nullptr) {
+      float y[8];
+      in(A.gv, el, o); in(A.gv2, el, y);
+#pragma unroll
+      for (int c = 0; c < 8; ++c) o[c] += y[c];
+      if (A.gvf != nullptr) {
+        in(A.gvf, el, y);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) o[c] += y[c];
+      }
+      put(A.dv_sum, o);
     }
 #pragma unroll
     for (int c = 0; c < 8; ++c) {

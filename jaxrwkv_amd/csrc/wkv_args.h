@@ -161,6 +161,8 @@ struct PreArgs {
   const void *gr, *gr2;                        // two cotangents of r to be added up in dr; may be null
   void* dr;
   void *dxw, *dk, *dv, *dvf, *dxv, *dxa;
+  const void* gvf;                             // added to dvf (or to dv_sum); may be null, may be dvf
+  void* dv_sum;                                // without the value residual: gv + gv2 + gvf; may be null
   float* part;                                 // workspace (rwkv7_pre_bwd_rows, 4 or 5, H*64)
 };
 int64_t rwkv7_pre_bwd_rows(int64_t rows, int64_t H);
@@ -174,7 +176,7 @@ struct GemmJob : ::hiprwkv_gemm_job {
 };
 constexpr int GEMM_ACT_NONE = 0, GEMM_ACT_TANH = 1, GEMM_ACT_SIGMOID = 2, GEMM_ACT_RELUSQ = 3;      // f without aux
 constexpr int GEMM_ADD = 0, GEMM_DTANH = 1, GEMM_DSIGMOID = 2, GEMM_DRELUSQ = 3;                    // f with aux
-constexpr int GEMM_MAX_JOBS = 12;
+constexpr int GEMM_MAX_JOBS = 14;
 constexpr int GEMM_TILE_ROWS = 33;     // rows from which the kernel with LDS tiles takes over
 constexpr int GEMM_MAX_SPLIT = 8;
 struct GemmArgs {
@@ -188,6 +190,12 @@ hipError_t launch_gemm(GemmArgs A, int split, hipStream_t stream);
 using Rwkv7Decode = ::hiprwkv_rwkv7_decode_args;
 size_t rwkv7_decode_workspace(const Rwkv7Decode& D);
 hipError_t launch_rwkv7_decode(const Rwkv7Decode& D, hipStream_t stream);
+
+using Rwkv7Stack = ::hiprwkv_rwkv7_stack_args;
+size_t rwkv7_stack_saved(const Rwkv7Stack& D);
+size_t rwkv7_stack_workspace(const Rwkv7Stack& D, bool backward);
+int launch_rwkv7_stack_fwd(const Rwkv7Stack& D, hipStream_t stream, hipError_t& e);      // an entry point's error, or e
+int launch_rwkv7_stack_bwd(const Rwkv7Stack& D, hipStream_t stream, hipError_t& e);
 
 // Raises a kernel's dynamic-LDS limit once per kernel and device instead of at every enqueue (the attribute call
 // goes to the driver; hipGetDevice does not).
