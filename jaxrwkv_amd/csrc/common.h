@@ -25,6 +25,13 @@ __device__ __forceinline__ int64_t seq_length(const uint32_t* length, int64_t b,
   return (flags & FLAG_LENGTH_I32) && (int32_t)L < 0 ? 0 : (int64_t)L;
 }
 
+// in-sequence index of the token whose xn a token-shift state keeps: x[length - 1] with the wrap-around of negative indices
+__device__ __forceinline__ int64_t last_token(const int32_t* length, int64_t b, int64_t T) {
+  if (length == nullptr) return T - 1;
+  const int64_t t = ((int64_t)length[b] - 1) % T;
+  return t < 0 ? t + T : t;
+}
+
 // 8 consecutive elements <-> 8 floats (pointer must be 16-byte aligned for bf16, 32 for fp32)
 __device__ __forceinline__ void ld8(const float* p, float (&o)[8]) {
   float4 a = *reinterpret_cast<const float4*>(p);

@@ -105,13 +105,6 @@ struct Held<bf16_t> {
   }
 };
 
-// in-sequence index of the token whose xn the state keeps: x[length - 1] with the wrap-around of negative indices
-__device__ __forceinline__ int64_t last_token(const int32_t* length, int64_t b, int64_t T) {
-  if (length == nullptr) return T - 1;
-  const int64_t t = ((int64_t)length[b] - 1) % T;
-  return t < 0 ? t + T : t;
-}
-
 // GROUP: tokens whose loads are in flight together, chosen by the launcher so that runs are whole groups (a decode step's token has
 // none before it; with groups of four its loads were asked for four times, partial sums of a product among them: 256 rows of 2048
 // channels, six outputs 10.7 -> 8.1 us, one 10.4 -> 7.2)

@@ -31,6 +31,25 @@ __device__ __forceinline__ float activate(float x, int act) {
   return !th ? q : fabsf(x) < 0.25f ? series : 1.f - 2.f * q;
 }
 
+// The job of a tile.  The first tiles are read at once and the job after them: as a loop over the jobs' own first tiles a grid of seven
+// began with seven reads that waited for each other.
+__device__ __forceinline__ int job_of(const GemmArgs& A, int tile) {
+  int ji = 0;
+#pragma unroll
+  for (int i = 1; i < GEMM_MAX_JOBS; ++i) ji = tile >= A.tile0[i] ? i : ji;      // beyond the last: INT_MAX
+  return ji;
+}
+// columns (or tiles) of a job -> the first tiles; returns their number
+template <typename F>
+int place_jobs(GemmArgs& A, F&& tiles_of_job) {
+  int tiles = 0;
+  for (int i = 0; i < GEMM_MAX_JOBS; ++i) {
+    A.tile0[i] = i < A.n_jobs ? tiles : INT_MAX;
+    if (i < A.n_jobs) tiles += tiles_of_job(A.job[i]);
+  }
+  return tiles;
+}
+
 // Weight-streaming product for few rows: bound by reading w once.  A workgroup owns 16 columns of one product and 16 MT
 // rows; its eight waves split K (every wave of the grid then streams a run of k of sixteen weight rows, so that many
 // short streams are in flight however small N is) and add their 16x16 tiles through LDS.  The weights' rows are the
@@ -39,14 +58,13 @@ __device__ __forceinline__ float activate(float x, int act) {
 template <int MT>
 __global__ __launch_bounds__(64 * GEMM_WAVES) void skinny_gemm_kernel(GemmArgs A) {
   __shared__ f32x4_t red[GEMM_WAVES][MT][64];
-  int ji = 0;
-  for (int i = 1; i < A.n_jobs; ++i) ji = (int)blockIdx.x >= A.job[i].tile0 ? i : ji;
+  const int ji = job_of(A, blockIdx.x);
   const GemmJob J = A.job[ji];
   const bf16_t* const jx = static_cast<const bf16_t*>(J.x);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-  const int n0 = ((int)blockIdx.x - J.tile0) * 16;
-  const int steps = J.K / 32;
-  const int s0 = steps * wave / GEMM_WAVES, s1 = steps * (wave + 1) / GEMM_WAVES;
+  const int n0 = ((int)blockIdx.x - A.tile0[ji]) * 16;
+  const int steps = J.K / 32, part = wave + GEMM_WAVES * (int)blockIdx.y, parts = GEMM_WAVES * (int)gridDim.y;
+  const int s0 = steps * part / parts, s1 = steps * (part + 1) / parts;
   f32x4_t acc[MT];
   const bf16_t* xp[MT];
 #pragma unroll
@@ -99,11 +117,181 @@ __global__ __launch_bounds__(64 * GEMM_WAVES) void skinny_gemm_kernel(GemmArgs A
     for (int q = 1; q < GEMM_WAVES; ++q) s += red[q][wave][lane];
     // lane (column m = lane % 16, g) holds n = 4g .. 4g+3
     const int m = 16 * wave + r;
-    if (m < J.M) {
+    if (m < J.M && A.part != nullptr) {
+      *reinterpret_cast<f32x4_t*>(A.part + ((size_t)blockIdx.y * J.M + m) * J.N + n0 + 4 * g) = s;
+    } else if (m < J.M) {
       const uint2 o = make_uint2(chunk::pack_rn(activate(s[0], J.act), activate(s[1], J.act)),
                                  chunk::pack_rn(activate(s[2], J.act), activate(s[3], J.act)));
       *reinterpret_cast<uint2*>(static_cast<bf16_t*>(J.out) + (size_t)m * J.N + n0 + 4 * g) = o;
     }
+  }
+}
+
+// sum over the 16 lanes of a DPP row, delivered to all of them
+__device__ __forceinline__ float row_sum(float x) {
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x128, 0xf, 0xf, false));   // row_ror:8
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x124, 0xf, 0xf, false));   // row_ror:4
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x122, 0xf, 0xf, false));   // row_ror:2
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x121, 0xf, 0xf, false));   // row_ror:1
+  return x;
+}
+
+__device__ __forceinline__ float half_of(const u32x4_t v, int e) {        // value e of eight
+  return __uint_as_float(e & 1 ? v[e >> 1] & 0xffff0000u : v[e >> 1] << 16);
+}
+
+// What ln_shiftmix_kernel and the product above do, in one launch for one or two rows (a decode step of few users).  There a launch of
+// its own costs more than doing the norm again in every workgroup: its rows come from the cache while the weights, requested first, are
+// on their way.  Everything else that comes from memory is requested before the norm as well: each wait that follows one costs 1 us of
+// the 5 to 8.  xn lies in LDS; token shift and interpolation are applied to the eight values that a lane hands to a matrix instruction.
+// Workgroup 0 writes the residual stream and the state's shift row.
+// G: rows; AHEAD_W: steps of K whose weights are requested first; NT: times 16 columns of a workgroup.
+template <int G, int AHEAD_W, int NT>
+__global__ __launch_bounds__(64 * GEMM_WAVES) void head_gemm_kernel(LnMixArgs N, GemmArgs A) {
+  extern __shared__ __align__(16) uint16_t head_xn[];            // (rows, C + 8)
+  __shared__ f32x4_t red[GEMM_WAVES][NT][64];
+  __shared__ float sums[2][4 * GEMM_WAVES * G];                  // one per 16 lanes and row
+  const int ji = job_of(A, blockIdx.x);
+  const GemmJob J = A.job[ji];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r = lane & 15, g = lane >> 4;
+  const int C = (int)N.C, M = G, T = (int)N.T, stride = C + 8;
+  const int n0 = ((int)blockIdx.x - A.tile0[ji]) * 16 * NT;
+  const int steps = C / 32;
+  const int s0 = steps * wave / GEMM_WAVES, s1 = steps * (wave + 1) / GEMM_WAVES;
+  const bf16_t* const wp = static_cast<const bf16_t*>(J.w) + (size_t)(n0 + r) * C + 8 * g;
+  const uint16_t* const wk = static_cast<const uint16_t*>(J.w) + (size_t)(8 * g) * J.N + n0 + r;
+  auto weights = [&](int s, int q) {
+    if (!J.kn) return *reinterpret_cast<const u32x4_t*>(wp + (size_t)16 * q * C + 32 * s);
+    u32x4_t w;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint16_t* p = wk + (size_t)(32 * s + 2 * i) * J.N + 16 * q;
+      w[i] = (uint32_t)p[0] | ((uint32_t)p[J.N] << 16);
+    }
+    return w;
+  };
+  const int m = r < M ? r : M - 1, b = m / T, t = m - b * T;
+  const bool reset = N.ns != nullptr && N.ns[m] != 0;
+  const bf16_t* const cur = reinterpret_cast<const bf16_t*>(head_xn) + m * stride + 8 * g;
+  const bf16_t* const row = static_cast<const bf16_t*>(N.prev) + (size_t)b * N.prev_bstride + 8 * g;
+  const bf16_t* const mix = static_cast<const bf16_t*>(J.aux) + 8 * g;
+  auto at = [&](const bf16_t* p, int s) { return *reinterpret_cast<const u32x4_t*>(p + 32 * s); };
+  constexpr int AHEAD_X = 4;
+  u32x4_t w[AHEAD_W][NT], before[AHEAD_X], share[AHEAD_X];
+  const int c = 8 * tid, cc = c < C ? c : 0;                     // the norm: eight channels per thread
+  const u32x4_t lnw = *reinterpret_cast<const u32x4_t*>(static_cast<const bf16_t*>(N.ln_w) + cc);
+  const u32x4_t lnb = *reinterpret_cast<const u32x4_t*>(static_cast<const bf16_t*>(N.ln_b) + cc);
+#pragma unroll
+  for (int u = 0; u < AHEAD_W; ++u) {
+    const int s = s0 + u < steps ? s0 + u : steps - 1;
+#pragma unroll
+    for (int q = 0; q < NT; ++q) w[u][q] = weights(s, q);
+    if (u < AHEAD_X) { before[u] = at(row, s); share[u] = at(mix, s); }
+  }
+  const float invC = 1.f / (float)C;
+  auto block_sums = [&](float (&v)[G], float* buf) {
+#pragma unroll
+    for (int j = 0; j < G; ++j) {
+      v[j] = row_sum(v[j]);
+      if ((tid & 15) == 0) buf[(tid >> 4) * G + j] = v[j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < G; ++j) {                                // 32 sums, two by each of 16 lanes
+      v[j] = buf[(2 * (tid & 15)) * G + j] + buf[(2 * (tid & 15) + 1) * G + j];
+      v[j] = row_sum(v[j]);
+    }
+  };
+  {
+    float x[G][8], sum[G], sq[G];
+#pragma unroll
+    for (int j = 0; j < G; ++j) {
+      const size_t el = (size_t)j * C + cc;
+      ld8(static_cast<const bf16_t*>(N.x) + el, x[j]);
+      if (N.dx != nullptr || N.n_part > 1) {
+        float d[8];
+        if (N.n_part > 1) {                    // a product's partial sums
+          ld8(N.part + el, d);
+#pragma unroll 4
+          for (int p = 1; p < N.n_part; ++p) {
+            float q[8];
+            ld8(N.part + (size_t)p * M * C + el, q);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) d[e] += q[e];
+          }
+#pragma unroll
+          for (int e = 0; e < 8; ++e) d[e] = rnd(d[e]);
+        } else {
+          ld8(static_cast<const bf16_t*>(N.dx) + el, d);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[j][e] = rnd(x[j][e] + d[e]);
+        if (blockIdx.x == 0 && c < C) st8(static_cast<bf16_t*>(N.xs) + el, x[j]);
+      }
+      sum[j] = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sum[j] += c < C ? x[j][e] : 0.f;
+    }
+    block_sums(sum, sums[0]);
+#pragma unroll
+    for (int j = 0; j < G; ++j) {
+      sum[j] *= invC;
+      sq[j] = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) { const float d = x[j][e] - sum[j]; sq[j] = c < C ? fmaf(d, d, sq[j]) : 0.f; }
+    }
+    block_sums(sq, sums[1]);
+#pragma unroll
+    for (int j = 0; j < G; ++j) {
+      if (c >= C) break;
+      const float rstd = rsqrtf(sq[j] * invC + N.eps);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[j][e] = fmaf((x[j][e] - sum[j]) * rstd, half_of(lnw, e), half_of(lnb, e));
+      st8(reinterpret_cast<bf16_t*>(head_xn) + j * stride + c, x[j]);
+      const int nb = j / T;
+      if (blockIdx.x == 0 && j - nb * T == (int)last_token(N.length, nb, T))
+        st8(static_cast<bf16_t*>(N.shift) + (size_t)nb * N.shift_bstride + c, x[j]);
+    }
+  }
+  __syncthreads();
+  f32x4_t acc[NT];
+#pragma unroll
+  for (int q = 0; q < NT; ++q) acc[q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  auto step = [&](const u32x4_t (&ws)[NT], const u32x4_t prev, const u32x4_t part, int s) {
+    float x[8], f[8];
+    u32x4_t p = prev;
+    ld8(cur + 32 * s, x);
+    if (t > 0) p = *reinterpret_cast<const u32x4_t*>(cur + 32 * s - stride);
+    u32x4_t o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = fmaf((reset ? 0.f : half_of(p, e)) - x[e], half_of(part, e), x[e]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = chunk::pack_rn(f[2 * e], f[2 * e + 1]);
+#pragma unroll
+    for (int q = 0; q < NT; ++q) acc[q] = mfma(ws[q], o, acc[q]);
+  };
+#pragma unroll
+  for (int u = 0; u < AHEAD_W; ++u)
+    if (s0 + u < s1) {
+      if (u < AHEAD_X) step(w[u], before[u], share[u], s0 + u);
+      else step(w[u], at(row, s0 + u), at(mix, s0 + u), s0 + u);
+    }
+  for (int s = s0 + AHEAD_W; s < s1; ++s) {
+    u32x4_t ws[NT];
+#pragma unroll
+    for (int q = 0; q < NT; ++q) ws[q] = weights(s, q);
+    step(ws, at(row, s), at(mix, s), s);
+  }
+#pragma unroll
+  for (int q = 0; q < NT; ++q) red[wave][q][lane] = acc[q];
+  __syncthreads();
+  if (wave < NT && r < M) {
+    f32x4_t v = red[0][wave][lane];
+#pragma unroll
+    for (int q = 1; q < GEMM_WAVES; ++q) v += red[q][wave][lane];
+    const uint2 o = make_uint2(chunk::pack_rn(activate(v[0], J.act), activate(v[1], J.act)),
+                               chunk::pack_rn(activate(v[2], J.act), activate(v[3], J.act)));
+    *reinterpret_cast<uint2*>(static_cast<bf16_t*>(J.out) + (size_t)r * J.N + n0 + 16 * wave + 4 * g) = o;
   }
 }
 
@@ -276,10 +464,9 @@ __device__ __forceinline__ void tile_gemm_body(const GemmArgs& A, const GemmJob&
 // job and tile of a workgroup: along the longer side of the tile grid eight tiles at a time, one per XCD; all tiles across from
 // each on the same XCD
 __device__ __forceinline__ bool tile_of(const GemmArgs& A, int tm, int tn, int& ji, int& n0, int& m0) {
-  ji = 0;
-  for (int i = 1; i < A.n_jobs; ++i) ji = (int)blockIdx.x >= A.job[i].tile0 ? i : ji;
+  ji = job_of(A, blockIdx.x);
   const int M = A.job[ji].M, N = A.job[ji].N;
-  const int mt = (M + tm - 1) / tm, nt = (N + tn - 1) / tn, local = (int)blockIdx.x - A.job[ji].tile0;
+  const int mt = (M + tm - 1) / tm, nt = (N + tn - 1) / tn, local = (int)blockIdx.x - A.tile0[ji];
   const int across = mt < nt ? mt : nt;
   const int p = local / (8 * across) * 8 + local % 8, q = local % (8 * across) / 8;
   n0 = (mt < nt ? p : q) * tn;
@@ -487,11 +674,12 @@ __global__ __launch_bounds__(256) void tile_gemm_kernel(GemmArgs A) {
 
 }  // namespace
 
-// Parts that a product's K is split into: enough tiles for about two workgroups per CU, at least 256 of k each
+// Parts that a product's K is split into: enough tiles for about two workgroups per CU, at least 256 of k each (few rows: three
+// steps of a wave.  One user's value projection of 3072 into 768 had 48 workgroups)
 int gemm_split(int M, int64_t K, int64_t N) {
-  if (M < GEMM_TILE_ROWS) return 1;
-  const int64_t tiles = (M + TG - 1) / TG * ((N + TG - 1) / TG);
-  const int64_t want = 512 / tiles, most = K / 256;
+  const bool skinny = M < GEMM_TILE_ROWS;
+  const int64_t tiles = skinny ? (N + 15) / 16 : (M + TG - 1) / TG * ((N + TG - 1) / TG);
+  const int64_t want = 512 / tiles, most = skinny ? K / (32 * GEMM_WAVES * 3) : K / 256;
   const int64_t n = want < most ? want : most;
   return (int)(n < 1 ? 1 : n > GEMM_MAX_SPLIT ? GEMM_MAX_SPLIT : n);
 }
@@ -511,7 +699,7 @@ int gemm_split(int M, int64_t K, int64_t N) {
 // of its products.
 constexpr int CUS = 256, WIDE_TILES = 192;
 hipError_t launch_gemm(GemmArgs A, int split, hipStream_t stream) {
-  bool skinny = A.part == nullptr, stream_k = true, same_k = true;
+  bool skinny = true, stream_k = true, same_k = true;
   int M = 0, longest = 0, tiles = 0;
   // the longest first: what is left at the end is short
   for (int i = 1; i < A.n_jobs; ++i)
@@ -524,14 +712,7 @@ hipError_t launch_gemm(GemmArgs A, int split, hipStream_t stream) {
     stream_k = stream_k && (J.K % TG == 0 || J.K >= 4 * TG);
     skinny = skinny && J.M < GEMM_TILE_ROWS && !J.km && J.aux == nullptr && J.raw == nullptr && J.K % 32 == 0 && J.N % 16 == 0;
   }
-  auto place = [&](int tm, int tn) {
-    tiles = 0;
-    for (int i = 0; i < A.n_jobs; ++i) {
-      GemmJob& J = A.job[i];
-      J.tile0 = tiles;
-      tiles += skinny ? J.N / 16 : tiles_of(J, tm, tn);
-    }
-  };
+  auto place = [&](int tm, int tn) { tiles = place_jobs(A, [&](const GemmJob& J) { return skinny ? J.N / 16 : tiles_of(J, tm, tn); }); };
   const dim3 block(64 * GEMM_WAVES);
   if (!skinny && stream_k && (split > 1 || A.part != nullptr)) {
     place(2 * TG, TG);
@@ -566,9 +747,23 @@ hipError_t launch_gemm(GemmArgs A, int split, hipStream_t stream) {
   }
   place(TG, TG);
   if (!skinny) hipLaunchKernelGGL(tile_gemm_kernel, dim3(tiles, split), dim3(256), 0, stream, A);
-  else if (M <= 16) hipLaunchKernelGGL(skinny_gemm_kernel<1>, dim3(tiles), block, 0, stream, A);
-  else hipLaunchKernelGGL(skinny_gemm_kernel<2>, dim3(tiles), block, 0, stream, A);
+  else if (M <= 16) hipLaunchKernelGGL(skinny_gemm_kernel<1>, dim3(tiles, split), block, 0, stream, A);
+  else hipLaunchKernelGGL(skinny_gemm_kernel<2>, dim3(tiles, split), block, 0, stream, A);
   return hipGetLastError();
+}
+
+template <int G, int AHEAD_W, int NT>
+static hipError_t launch_head(const LnMixArgs& N, GemmArgs& A, hipStream_t stream) {
+  const int tiles = place_jobs(A, [](const GemmJob& J) { return J.N / (16 * NT); });
+  hipLaunchKernelGGL((head_gemm_kernel<G, AHEAD_W, NT>), dim3(tiles), dim3(64 * GEMM_WAVES), (size_t)G * (N.C + 8) * 2, stream, N, A);
+  return hipGetLastError();
+}
+// 32 columns a workgroup from 1025 channels on: with 16 there are two turns of workgroups, each with its norm (24 layers of 2048
+// channels, one user: 1536 us with 16, 1360 with 32, 1439 with norms of their own)
+hipError_t launch_head_gemm(const LnMixArgs& N, GemmArgs A, hipStream_t stream) {
+  const bool one = A.job[0].M == 1;
+  if (N.C <= 1024) return one ? launch_head<1, 4, 1>(N, A, stream) : launch_head<2, 4, 1>(N, A, stream);
+  return one ? launch_head<1, 8, 2>(N, A, stream) : launch_head<2, 8, 2>(N, A, stream);
 }
 
 }  // namespace hiprwkv

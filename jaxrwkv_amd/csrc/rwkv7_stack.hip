@@ -100,7 +100,7 @@ struct Forward {
     one = K.D.saved == nullptr ? K.layer(A, false) : Layer();
     v_first = K.D.saved == nullptr ? A.take(n) : nullptr;
     dx = A.take(n);
-    parts = A.take<float>(K.rows < GEMM_TILE_ROWS ? 0 : n * GEMM_MAX_SPLIT);
+    parts = A.take<float>(n * GEMM_MAX_SPLIT);
     wkv_bytes = hiprwkv_wkv7_fwd_workspace_bytes(HIPRWKV_BF16, K.D.B, K.D.T, K.D.H, 64);
     wkv = wkv_bytes ? A.take<char>(wkv_bytes) : nullptr;
   }

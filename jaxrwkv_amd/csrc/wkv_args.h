@@ -180,12 +180,17 @@ constexpr int GEMM_MAX_JOBS = 14;
 constexpr int GEMM_TILE_ROWS = 33;     // rows from which the kernel with LDS tiles takes over
 constexpr int GEMM_MAX_SPLIT = 8;
 struct GemmArgs {
-  GemmJob job[GEMM_MAX_JOBS];
   int n_jobs;
+  int tile0[GEMM_MAX_JOBS];  // the launcher's: a job's first tile; side by side, so that a workgroup finds its job with one load
+  GemmJob job[GEMM_MAX_JOBS];
   float* part;         // not null: (split, M, N) fp32 partial sums instead of out; one job, no f
 };
 int gemm_split(int M, int64_t K, int64_t N);
 hipError_t launch_gemm(GemmArgs A, int split, hipStream_t stream);
+// The same products of one or two rows of norm and interpolation (LnMixArgs: bf16, C a multiple of 64, at most 4096; mix and
+// out unused): a job's x is that of its aux, the mix vector (C,); K = C, N a multiple of 32, not km.
+constexpr int HEAD_GEMM_ROWS = 2;
+hipError_t launch_head_gemm(const LnMixArgs& N, GemmArgs A, hipStream_t stream);
 
 using Rwkv7Decode = ::hiprwkv_rwkv7_decode_args;
 size_t rwkv7_decode_workspace(const Rwkv7Decode& D);

@@ -77,3 +77,10 @@ def test_calls_that_the_native_step_does_not_cover():
     assert ops.rwkv7_decode(params, x[:2], st[:4:2], None, None) is None                # a state that is not contiguous
     params["blocks"]["att"]["w0"] = params["blocks"]["att"]["w0"].float()
     assert ops.rwkv7_decode(params, x[:1], st[:1], None, None) is None
+
+
+@pytest.mark.parametrize("B,T,C", [(1, 1, 768), (2, 1, 1088), (1, 2, 2048), (1, 1, 4096), (1, 2, 64), (3, 1, 1024)])
+def test_native_decode_step_of_few_rows(B, T, C, monkeypatch):
+    """Norms inside the products and second low-rank products inside the recurrence: two tokens of a sequence and
+    of two, widths from one step of a wave to several, inner sizes beyond one round of requests, one row too many."""
+    test_native_decode_step(B, T, C, True, monkeypatch)
