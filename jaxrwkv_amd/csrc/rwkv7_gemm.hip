@@ -31,6 +31,10 @@ __device__ __forceinline__ float activate(float x, int act) {
   return !th ? q : fabsf(x) < 0.25f ? series : 1.f - 2.f * q;
 }
 
+__device__ __forceinline__ float half_of(const u32x4_t v, int e) {        // value e of eight
+  return __uint_as_float(e & 1 ? v[e >> 1] & 0xffff0000u : v[e >> 1] << 16);
+}
+
 // The job of a tile.  The first tiles are read at once and the job after them: as a loop over the jobs' own first tiles a grid of seven
 // began with seven reads that waited for each other.
 __device__ __forceinline__ int job_of(const GemmArgs& A, int tile) {
@@ -134,10 +138,6 @@ __device__ __forceinline__ float row_sum(float x) {
   x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x122, 0xf, 0xf, false));   // row_ror:2
   x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x121, 0xf, 0xf, false));   // row_ror:1
   return x;
-}
-
-__device__ __forceinline__ float half_of(const u32x4_t v, int e) {        // value e of eight
-  return __uint_as_float(e & 1 ? v[e >> 1] & 0xffff0000u : v[e >> 1] << 16);
 }
 
 // What ln_shiftmix_kernel and the product above do, in one launch for one or two rows (a decode step of few users).  There a launch of
@@ -379,32 +379,59 @@ struct TileOperand {
   }
 };
 
-// f and the store of one lane's four consecutive columns
-__device__ __forceinline__ void finish(const GemmArgs& A, const GemmJob& J, int n, int m, f32x4_t v) {
-  if (n >= J.N || m >= J.M) return;
-  if (A.part != nullptr) {
-    *reinterpret_cast<f32x4_t*>(A.part + ((size_t)blockIdx.y * J.M + m) * J.N + n) = v;
-    return;
+// A tile's results.  Partial sums go to memory as they lie; everything else is rounded first, whatever follows (a separate product would
+// be stored there), so the tile goes through LDS as bf16 and out as rows of whole cache lines, eight values a lane, f in a loop whose
+// code is short: with f inlined at each of a lane's sixteen stores of 8 bytes, key projections of 2048 rows (768 into 3072, relu^2 beside
+// the product) took 31.8 us, 22.4 now, their backward with the weights' cotangents 53.5, 47.8 now; 256 rows of r, k, v and the low-rank inputs
+// (2048 channels) 25.4, 22.2 now.
+template <int TM, int TN>
+struct TileOut {
+  static constexpr int STRIDE = TN + 8;
+  static constexpr size_t BYTES = (size_t)TM * STRIDE * 2;
+  // columns n .. n + 3 of row m of the tile
+  static __device__ __forceinline__ void put(const GemmArgs& A, const GemmJob& J, uint16_t* lds, int n0, int m0, int n, int m, f32x4_t v) {
+    if (A.part != nullptr) {
+      if (n0 + n < J.N && m0 + m < J.M)
+        *reinterpret_cast<f32x4_t*>(A.part + ((size_t)blockIdx.y * J.M + m0 + m) * J.N + n0 + n) = v;
+      return;
+    }
+    *reinterpret_cast<uint2*>(lds + m * STRIDE + n) = make_uint2(chunk::pack_rn(v[0], v[1]), chunk::pack_rn(v[2], v[3]));
   }
-  const size_t el = (size_t)m * J.N + n;
-  if (J.aux != nullptr) {
-    const uint2 q = *reinterpret_cast<const uint2*>(static_cast<const bf16_t*>(J.aux) + el);
-    const float h[4] = {__uint_as_float(q.x << 16), __uint_as_float(q.x & 0xffff0000u), __uint_as_float(q.y << 16),
-                        __uint_as_float(q.y & 0xffff0000u)};
+  // by all 256 threads, after a barrier
+  static __device__ __forceinline__ void write(const GemmArgs& A, const GemmJob& J, const uint16_t* lds, int n0, int m0) {
+    if (A.part != nullptr) return;
+    constexpr int PIECES = TN / 8;
+#pragma unroll 1
+    for (int i = threadIdx.x; i < TM * PIECES; i += 256) {
+      const int m = i / PIECES, n = 8 * (i % PIECES);
+      if (m0 + m >= J.M || n0 + n >= J.N) continue;
+      const size_t el = (size_t)(m0 + m) * J.N + n0 + n;
+      u32x4_t q = *reinterpret_cast<const u32x4_t*>(lds + m * STRIDE + n);
+      if (J.aux != nullptr || J.act != GEMM_ACT_NONE) {
+        if (J.raw != nullptr) *reinterpret_cast<u32x4_t*>(static_cast<bf16_t*>(J.raw) + el) = q;
+        float v[8], h[8];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = rnd(v[i]);
+        for (int e = 0; e < 8; ++e) v[e] = half_of(q, e);
+        if (J.aux != nullptr) {
+          ld8(static_cast<const bf16_t*>(J.aux) + el, h);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      v[i] = J.act == GEMM_ADD ? v[i] + h[i] : J.act == GEMM_DTANH ? v[i] * (1.f - h[i] * h[i])
-           : J.act == GEMM_DRELUSQ ? 2.f * v[i] * fmaxf(h[i], 0.f) : v[i] * (h[i] * (1.f - h[i]));
-  } else {
-    if (J.raw != nullptr)
-      *reinterpret_cast<uint2*>(static_cast<bf16_t*>(J.raw) + el) = make_uint2(chunk::pack_rn(v[0], v[1]), chunk::pack_rn(v[2], v[3]));
+          for (int e = 0; e < 8; ++e)
+            v[e] = J.act == GEMM_ADD ? v[e] + h[e] : J.act == GEMM_DTANH ? v[e] * (1.f - h[e] * h[e])
+                 : J.act == GEMM_DRELUSQ ? 2.f * v[e] * fmaxf(h[e], 0.f) : v[e] * (h[e] * (1.f - h[e]));
+        } else if (J.act == GEMM_ACT_RELUSQ) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = activate(v[i], J.act);
+          for (int e = 0; e < 8; ++e) { const float p = fmaxf(v[e], 0.f); v[e] = p * p; }
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = activate(v[e], J.act);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q[e] = chunk::pack_rn(v[2 * e], v[2 * e + 1]);
+      }
+      *reinterpret_cast<u32x4_t*>(static_cast<bf16_t*>(J.out) + el) = q;
+    }
   }
-  *reinterpret_cast<uint2*>(static_cast<bf16_t*>(J.out) + el) = make_uint2(chunk::pack_rn(v[0], v[1]), chunk::pack_rn(v[2], v[3]));
-}
+};
 
 template <bool KM, bool KN, bool EXACT>
 __device__ __forceinline__ void tile_gemm_body(const GemmArgs& A, const GemmJob& J, int n0, int m0, TileLds& lds) {
@@ -455,10 +482,15 @@ __device__ __forceinline__ void tile_gemm_body(const GemmArgs& A, const GemmJob&
       compute(j & 1);
     }
   }
+  typedef TileOut<TG, TG> Out;
+  uint16_t* const out = &lds[0][0][0][0];
+  __syncthreads();                               // every wave has read the last step
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int u = 0; u < 2; ++u) finish(A, J, n0 + wn + 16 * t + 4 * g, m0 + wm + 16 * u + r, acc[t][u]);
+    for (int u = 0; u < 2; ++u) Out::put(A, J, out, n0, m0, wn + 16 * t + 4 * g, wm + 16 * u + r, acc[t][u]);
+  __syncthreads();
+  Out::write(A, J, out, n0, m0);
 }
 
 // job and tile of a workgroup: along the longer side of the tile grid eight tiles at a time, one per XCD; all tiles across from
@@ -623,12 +655,17 @@ __device__ __forceinline__ void stream_gemm_body(const GemmArgs& A, const GemmJo
     arrive(s1 - 1, buf);
     compute(buf, false, J.K % TG);
   }
-  // the requests beyond the last step write to LDS as well: none may be under way when the workgroup gives its LDS back
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // the requests beyond the last step write to LDS as well: none may be under way when the tile goes there, nor may a wave read the last
+  // step
+  typedef TileOut<TM, TN> Out;
+  static_assert(Out::BYTES <= (size_t)BUFS * STEP * 2, "the tile fits in the buffers");
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int u = 0; u < MT; ++u) finish(A, J, n0 + wn + 16 * t + 4 * g, m0 + wm + 16 * u + r, acc[t][u]);
+    for (int u = 0; u < MT; ++u) Out::put(A, J, lds, n0, m0, wn + 16 * t + 4 * g, wm + 16 * u + r, acc[t][u]);
+  __syncthreads();
+  Out::write(A, J, lds, n0, m0);
 }
 
 template <int TM, int TN, int BUFS>
