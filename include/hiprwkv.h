@@ -373,6 +373,12 @@ int hiprwkv_rwkv7_pre(hiprwkv_stream stream, int io_dtype, int64_t rows, int64_t
                       const void* k, const void* xa, const void* v, const void* v_first, const void* xv, const void* w0,
                       const void* a0, const void* v0, const void* k_k, const void* k_a, void* w, void* k_out,
                       void* v_out, void* a_out, void* b_out);
+/* The same with the low-rank terms made on the way, HIPRWKV_BF16 only: term i = hid[i] (rows, d[i]) times w2[i] (d[i], H*64), rounded, in
+ * the order xw, xa, g, xv; all go to out[i], or, with out NULL, g alone to g.  d multiples of 8; without v_first three terms. */
+int hiprwkv_rwkv7_lora_pre(hiprwkv_stream stream, int io_dtype, int64_t rows, int64_t H, int64_t N, const void* const* hid,
+                           const void* const* w2, const int64_t* d, const void* k, const void* v, const void* v_first, const void* w0,
+                           const void* a0, const void* v0, const void* k_k, const void* k_a, void* const* out, void* g, void* w,
+                           void* k_out, void* v_out, void* a_out, void* b_out);
 size_t hiprwkv_rwkv7_pre_bwd_workspace_bytes(int64_t rows, int64_t H, int64_t N);
 /* From the cotangents of w, k_out, v_out, a_out, b_out to those of the inputs; dparam: (H, 64) io_dtype arrays of w0, a0,
  * k_k, k_a and, with v_first, v0.  gk_out2, gv_out2 (may be NULL) are added to gk_out and gv_out; dr (may be NULL) = gr + gr2:

@@ -100,6 +100,7 @@ SIGNATURES = {
                                   + [_vp] * 6 + [_i64, _vp]),
     "hiprwkv_rwkv7_ln_shiftmix_bwd_workspace_bytes": (_sz, [_i64] * 3 + [_int]),
     "hiprwkv_rwkv7_ln_shiftmix_bwd": (_int, [_vp, _int, _i64, _i64, _i64, _int] + [_vp] * 5 + [_i64] + [_vp] * 10 + [_sz]),
+    "hiprwkv_rwkv7_lora_pre": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 18),
     "hiprwkv_rwkv7_pre": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 16),
     "hiprwkv_rwkv7_pre_bwd_workspace_bytes": (_sz, [_i64] * 3),
     "hiprwkv_rwkv7_pre_bwd": (_int, [_vp, _int, _i64, _i64, _i64] + [_vp] * 29 + [_sz]),

@@ -57,17 +57,29 @@ def _grouped(p, like):
             and all(p[n].shape[-1] % 8 == 0 for n in ("w1", "a1", "v1", "g1")))
 
 
-def _lora_fwd(p, mix, names, like):
+def _lora_pre_fwd(p, mix, names, k, v, v_first, keep):
+    """``_lora_fwd`` and ``ops._pre_fwd`` for the products that ``_grouped`` takes: the second factors are made where the gates are.
+    k, v, v_first (None: the first layer) (M, C); without ``keep`` the gate's result alone is there of the low-rank terms."""
+    lib = _lib.load()
+    M, C = k.shape
+    H, N = p["r_k"].shape
+    e = lambda: torch.empty_like(k)
+    hid = {n: torch.empty((M, p[n + "1"].shape[-1]), dtype=k.dtype, device=k.device) for n, _ in names}
+    _gemm([(hid[n], mix[n], p[n + "1"], 0, 1, act, None) for n, act in names])
+    lora = {n: e() if keep or n == "g" else None for n, _ in names}
+    w, k2, v2, a, b = e(), e(), None if v_first is None else e(), e(), e()
+    sizes = (ctypes.c_int64 * len(names))(*(h.shape[1] for h in hid.values()))
+    P = ops._p
+    _lib.check(lib.hiprwkv_rwkv7_lora_pre(
+        ops._stream(), ops._DT[k.dtype], M, H, N, ops._ptr_array(list(hid.values())), ops._ptr_array([p[n + "2"] for n, _ in names]),
+        sizes, P(k), P(v), P(v_first), P(p["w0"]), P(p["a0"]), None if v_first is None else P(p["v0"]), P(p["k_k"]), P(p["k_a"]),
+        ops._ptr_array(list(lora.values())) if keep else None, P(lora["g"]), P(w), P(k2), P(v2), P(a), P(b)), "hiprwkv_rwkv7_lora_pre")
+    return hid, lora, (w, k2, v2, a, b)
+
+
+def _lora_fwd(p, mix, names):
     """Hidden values (activation applied) and results of the low-rank terms ``names``; mix: name -> (M, C) input."""
     hid, out = {}, {}
-    if _grouped(p, like):
-        M, C = like.shape
-        for n, _ in names:
-            hid[n] = torch.empty((M, p[n + "1"].shape[-1]), dtype=like.dtype, device=like.device)
-            out[n] = torch.empty_like(like)
-        _gemm([(hid[n], mix[n], p[n + "1"], 0, 1, act, None) for n, act in names])
-        _gemm([(out[n], hid[n], p[n + "2"], 0, 1, _NONE, None) for n, _ in names])
-        return hid, out
     for n, act in names:
         h = mix[n] @ p[n + "1"]
         hid[n] = torch.tanh_(h) if act == _TANH else torch.sigmoid_(h) if act == _SIGMOID else h
@@ -131,13 +143,17 @@ def _layer_fwd(i, p, x, dx, st, nst, v_first, ns, length, need):
     # `covers` has seen the call's own tensors; under an autocast that the caller overlooked products come out in another type
     ops._one_dtype(x.dtype, r)
     mix = {"w": xw, "a": xa, "g": xg, "v": xv}
-    hid, lora = _lora_fwd(p, mix, _LORA if i else _LORA[:3], r)
+    names = _LORA if i else _LORA[:3]
+    par = lambda n: p[n].reshape(C)
+    if _grouped(p, r):
+        hid, lora, pre = _lora_pre_fwd(p, mix, names, k, v, v_first if i else None, keep)
+    else:
+        hid, lora = _lora_fwd(p, mix, names)
+        pre = ops._pre_fwd(heads(lora["w"]), heads(k), heads(lora["a"]), heads(v), heads(v_first) if i else None,
+                           heads(lora["v"]) if i else None, par("w0"), par("a0"), par("v0") if i else None, par("k_k"), par("k_a"))
     if i == 0:
         v_first = v
-    par = lambda n: p[n].reshape(C)
-    pre = ops._pre_fwd(heads(lora["w"]), heads(k), heads(lora["a"]), heads(v), heads(v_first) if i else None,
-                       heads(lora["v"]) if i else None, par("w0"), par("a0"), par("v0") if i else None, par("k_k"), par("k_a"))
-    w, k2, v2, a, b = pre
+    w, k2, v2, a, b = (None if t is None else heads(t) for t in pre)
     if i == 0:
         v2 = heads(v)
     s = st[:, 2:].reshape(B, H, N, N)

@@ -870,6 +870,33 @@ int hiprwkv_rwkv7_pre(hiprwkv_stream stream, int io_dtype, int64_t rows, int64_t
   return gate_done("rwkv7_pre", launch_rwkv7_pre(io_dtype == HIPRWKV_F32, A, static_cast<hipStream_t>(stream)));
 }
 
+int hiprwkv_rwkv7_lora_pre(hiprwkv_stream stream, int io_dtype, int64_t rows, int64_t H, int64_t N, const void* const* hid,
+                           const void* const* w2, const int64_t* d, const void* k, const void* v, const void* v_first, const void* w0,
+                           const void* a0, const void* v0, const void* k_k, const void* k_a, void* const* out, void* g, void* w,
+                           void* k_out, void* v_out, void* a_out, void* b_out) {
+  LoraPreArgs X;
+  memset(&X, 0, sizeof(X));
+  PreArgs& A = X.P;
+  A.rows = rows; A.H = H;
+  A.k = k; A.v = v; A.vf = v_first;
+  A.w0 = w0; A.a0 = a0; A.v0 = v0; A.k_k = k_k; A.k_a = k_a;
+  A.w = w; A.k_out = k_out; A.v_out = v_out; A.a_out = a_out; A.b_out = b_out;
+  if (hid == nullptr || w2 == nullptr || d == nullptr) return fail(HIPRWKV_EINVAL, "rwkv7_lora_pre: null pointer array");
+  if (io_dtype != HIPRWKV_BF16) return fail(HIPRWKV_EINVAL, "rwkv7_lora_pre: dtype must be HIPRWKV_BF16");
+  if (int rc = check_pre("rwkv7_lora_pre", io_dtype, N, A, {k, w0, a0, k_k, k_a, out != nullptr ? out[2] : g, w, k_out, a_out, b_out}, {v, v_first, v0, v_out})) return rc;
+  if ((rows + 63) / 64 * H > 0x7fffffffLL || rows > 0x7fffffffLL - 64) return fail(HIPRWKV_EINVAL, "rwkv7_lora_pre: too many rows");
+  for (int i = 0; i < (v_first != nullptr ? 4 : 3); ++i) {
+    if (d[i] <= 0 || d[i] % 8 != 0 || std::max(rows, H * N) * d[i] >= 0x7fffffffLL)
+      return fail(HIPRWKV_EINVAL, "rwkv7_lora_pre: inner sizes must be positive multiples of 8, arrays below 4 GiB");
+    for (const void* p : {hid[i], w2[i]})
+      if (p == nullptr || !aligned16(p)) return fail(HIPRWKV_EINVAL, "rwkv7_lora_pre: null or misaligned tensor pointer (16 bytes)");
+    if (out != nullptr && (out[i] == nullptr || !aligned16(out[i])))
+      return fail(HIPRWKV_EINVAL, "rwkv7_lora_pre: null or misaligned tensor pointer (16 bytes)");
+    X.hid[i] = hid[i]; X.w2[i] = w2[i]; X.d[i] = (int)d[i]; X.out[i] = out != nullptr ? out[i] : i == 2 ? g : nullptr;
+  }
+  return gate_done("rwkv7_lora_pre", launch_rwkv7_lora_pre(X, static_cast<hipStream_t>(stream)));
+}
+
 size_t hiprwkv_rwkv7_pre_bwd_workspace_bytes(int64_t rows, int64_t H, int64_t N) {
   return rows <= 0 || H <= 0 || N <= 0 ? 0 : (size_t)rwkv7_pre_bwd_rows(rows, H) * 5 * H * N * sizeof(float);
 }

@@ -4,6 +4,7 @@
 //   * the low-rank factors of decay, gate, value residual and output gate in whole-sequence passes, forward and backward
 //     (rwkv7.py:237-245): narrow on one side, so that a library call of 10-18 us each is mostly launch and latency.
 #include "chunk_common.h"
+#include "rwkv7_pre.h"
 #include "wkv_args.h"
 
 namespace hiprwkv {
@@ -709,6 +710,113 @@ __global__ __launch_bounds__(256) void tile_gemm_kernel(GemmArgs A) {
   }
 }
 
+// The second low-rank products of 64 tokens and one head, and everything element-wise behind them.  In separate launches the products'
+// results made a trip through memory each way: 4084 tokens, 32 heads (inner sizes 96, 96, 64, 288) 44 + 36 us, here 68; 2048 tokens, 12
+// heads 11.3 + 9.6, here 16.3.  The vector units take 27 of the 68 (the element-wise part), the barrier of each of ten steps most of the
+// rest; four waves of twice the tile took as long.  The factors' steps of 64 of k follow each other without a stop, two in flight; their
+// products wait in LDS, rounded, for the last one.  Heads run fastest through the grid: an XCD reads the rows of hidden values that its
+// eight neighbours read as well, and of the weights only its own heads'.
+constexpr int LORA_THREADS = 512;
+template <bool VMIX>
+__global__ __launch_bounds__(LORA_THREADS) void lora_pre_kernel(LoraPreArgs A) {
+  constexpr int NF = VMIX ? 4 : 3;
+  __shared__ __align__(16) TileLds lds;
+  __shared__ __align__(16) uint16_t low[NF][TG][TG_RS];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r = lane & 15, g = lane >> 4;
+  const int H = (int)A.P.H, C = 64 * H, h = (int)blockIdx.x % H, m0 = (int)blockIdx.x / H * TG, M = (int)A.P.rows;
+  const int row = tid >> 3, col = 8 * (tid & 7);                 // of the tiles: a token or a k, and eight k or channels
+  const bool live = m0 + row < M;
+  const int mc = live ? m0 + row : M - 1;
+  const size_t el = (size_t)mc * C + 64 * h + col;
+  int first[NF + 1];                              // a factor's first step
+  first[0] = 0;
+#pragma unroll
+  for (int f = 0; f < NF; ++f) first[f + 1] = first[f] + (A.d[f] + TG - 1) / TG;
+  const int all = first[NF];
+  auto factor = [&](int s) {
+    int f = 0;
+#pragma unroll
+    for (int i = 1; i < NF; ++i) f = s >= first[i] ? i : f;
+    return f;
+  };
+  auto load = [&](u32x4_t& x, u32x4_t& w, int s_) {
+    const int s = s_ < all ? s_ : all - 1, f = factor(s);
+    int at = first[0], d = A.d[0];
+    const bf16_t *hid = static_cast<const bf16_t*>(A.hid[0]), *w2 = static_cast<const bf16_t*>(A.w2[0]);
+#pragma unroll
+    for (int i = 1; i < NF; ++i) {
+      at = f == i ? first[i] : at;
+      d = f == i ? A.d[i] : d;
+      hid = f == i ? static_cast<const bf16_t*>(A.hid[i]) : hid;
+      w2 = f == i ? static_cast<const bf16_t*>(A.w2[i]) : w2;
+    }
+    const int k0 = (s - at) * TG;
+    const int kx = k0 + col, kw = k0 + row;
+    auto at16 = [](const bf16_t* p, uint32_t el) { return *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const char*>(p) + 2u * el); };
+    if (k0 + TG <= d) {
+      x = at16(hid, (uint32_t)mc * (uint32_t)d + (uint32_t)kx);
+      w = at16(w2, (uint32_t)kw * (uint32_t)C + (uint32_t)(64 * h + col));
+    } else {
+      x = at16(hid, (uint32_t)mc * (uint32_t)d + (uint32_t)(kx < d ? kx : d - 8));
+      w = at16(w2, (uint32_t)(kw < d ? kw : d - 1) * (uint32_t)C + (uint32_t)(64 * h + col));
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        x[c] = kx < d ? x[c] : 0u;
+        w[c] = kw < d ? w[c] : 0u;
+      }
+    }
+  };
+  u32x4_t x[2], w[2], kq, vq, vfq;
+  load(x[0], w[0], 0);
+  load(x[1], w[1], 1);
+  kq = *reinterpret_cast<const u32x4_t*>(static_cast<const bf16_t*>(A.P.k) + el);
+  if (VMIX) {
+    vq = *reinterpret_cast<const u32x4_t*>(static_cast<const bf16_t*>(A.P.v) + el);
+    vfq = *reinterpret_cast<const u32x4_t*>(static_cast<const bf16_t*>(A.P.vf) + el);
+  }
+  f32x4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  const int wn = 16 * (wave & 3), wm = 32 * (wave >> 2);
+  auto step = [&](int s, int buf) {
+    *reinterpret_cast<u32x4_t*>(&lds[buf][0][row][col]) = x[buf];
+    *reinterpret_cast<u32x4_t*>(&lds[buf][1][row][col]) = w[buf];
+    load(x[buf], w[buf], s + 2);
+    __syncthreads();
+#pragma unroll
+    for (int kh = 0; kh < 2; ++kh) {
+      const u32x4_t wf = TileOperand<true, true>::frag(lds[buf][1], wn, kh, r, g);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) acc[u] = mfma(wf, TileOperand<false, true>::frag(lds[buf][0], wm + 16 * u, kh, r, g), acc[u]);
+    }
+    const int f = factor(s);
+    if (s + 1 == all || factor(s + 1) != f) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        *reinterpret_cast<uint2*>(&low[f][wm + 16 * u + r][wn + 4 * g]) = make_uint2(chunk::pack_rn(acc[u][0], acc[u][1]), chunk::pack_rn(acc[u][2], acc[u][3]));
+        acc[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+  };
+  int s = 0;
+  for (; s + 2 <= all; s += 2) { step(s, 0); step(s + 1, 1); }
+  if (s < all) step(s, 0);
+  __syncthreads();
+  u32x4_t q[4];
+#pragma unroll
+  for (int f = 0; f < 4; ++f) {
+    q[f] = f < NF ? *reinterpret_cast<const u32x4_t*>(&low[f < NF ? f : 0][row][col]) : u32x4_t{0u, 0u, 0u, 0u};
+    if (f < NF && live && A.out[f] != nullptr) *reinterpret_cast<u32x4_t*>(static_cast<bf16_t*>(A.out[f]) + el) = q[f];
+  }
+  float xw[8], k[8], xa[8], v[8], vf[8], xv[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    xw[e] = half_of(q[0], e); xa[e] = half_of(q[1], e); xv[e] = half_of(q[3], e);
+    k[e] = half_of(kq, e);
+    v[e] = VMIX ? half_of(vq, e) : 0.f;
+    vf[e] = VMIX ? half_of(vfq, e) : 0.f;
+  }
+  pre_unit<bf16_t, VMIX>(A.P, el, (size_t)64 * h + col, live, xw, k, xa, v, vf, xv);
+}
+
 }  // namespace
 
 // Parts that a product's K is split into: enough tiles for about two workgroups per CU, at least 256 of k each (few rows: three
@@ -801,6 +909,13 @@ hipError_t launch_head_gemm(const LnMixArgs& N, GemmArgs A, hipStream_t stream) 
   const bool one = A.job[0].M == 1;
   if (N.C <= 1024) return one ? launch_head<1, 4, 1>(N, A, stream) : launch_head<2, 4, 1>(N, A, stream);
   return one ? launch_head<1, 8, 2>(N, A, stream) : launch_head<2, 8, 2>(N, A, stream);
+}
+
+hipError_t launch_rwkv7_lora_pre(const LoraPreArgs& A, hipStream_t stream) {
+  const dim3 grid((unsigned)((A.P.rows + TG - 1) / TG * A.P.H)), block(LORA_THREADS);
+  if (A.P.vf != nullptr) hipLaunchKernelGGL(lora_pre_kernel<true>, grid, block, 0, stream, A);
+  else hipLaunchKernelGGL(lora_pre_kernel<false>, grid, block, 0, stream, A);
+  return hipGetLastError();
 }
 
 }  // namespace hiprwkv

@@ -13,6 +13,7 @@
 // A workgroup works on one head and steps over the tokens with the parameter sums in registers; they meet in LDS and leave
 // as one row per workgroup, which launch_reduce_parts adds up.
 #include "common.h"
+#include "rwkv7_pre.h"
 #include "wkv_args.h"
 
 namespace hiprwkv {
@@ -22,23 +23,6 @@ namespace {
 constexpr int PRE_THREADS = 256;            // 32 units
 constexpr int PRE_UNITS = PRE_THREADS / 8;
 
-__device__ __forceinline__ float sigmoidf(float z) { return 1.f / (1.f + __expf(-z)); }
-__device__ __forceinline__ float softplusf(float z) { return fmaxf(z, 0.f) + __logf(1.f + __expf(-fabsf(z))); }
-
-template <typename T>
-__device__ __forceinline__ float round_io(float x);
-template <>
-__device__ __forceinline__ float round_io<float>(float x) { return x; }
-template <>
-__device__ __forceinline__ float round_io<bf16_t>(float x) { return bf16_to_f32(f32_to_bf16(x)); }
-
-// sum over the 8 lanes of half a DPP row, delivered to all of them
-__device__ __forceinline__ float oct_sum(float x) {
-  x = quad_sum(x);
-  x += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x141, 0xf, 0xf, true));   // row_half_mirror
-  return x;
-}
-
 template <typename T, bool VMIX>
 __global__ __launch_bounds__(PRE_THREADS) void rwkv7_pre_kernel(PreArgs A) {
   // units beyond the end redo the last one: whole rows stay active for the reductions
@@ -46,37 +30,11 @@ __global__ __launch_bounds__(PRE_THREADS) void rwkv7_pre_kernel(PreArgs A) {
   unit = unit < A.rows * A.H ? unit : A.rows * A.H - 1;
   const int c8 = 8 * (threadIdx.x & 7);
   const size_t el = (size_t)unit * 64 + c8, ch = (size_t)(unit % A.H) * 64 + c8;
-  auto in = [&](const void* p, size_t i, float (&o)[8]) { ld8(reinterpret_cast<const T*>(p) + i, o); };
-  auto put = [&](void* p, const float (&o)[8]) { st8(reinterpret_cast<T*>(p) + el, o); };
-  float xw[8], k[8], xa[8], v[8], vf[8], xv[8], p0[8], p1[8], p2[8], o[8];
-  in(A.xw, el, xw); in(A.k, el, k); in(A.xa, el, xa);
-  if (VMIX) { in(A.v, el, v); in(A.vf, el, vf); in(A.xv, el, xv); }
-  in(A.w0, ch, p0); in(A.k_k, ch, p1); in(A.k_a, ch, p2);
-#pragma unroll
-  for (int c = 0; c < 8; ++c) o[c] = -softplusf(-(p0[c] + xw[c])) - 0.5f;
-  put(A.w, o);
-  if (VMIX) {
-    float pv[8];
-    in(A.v0, ch, pv);
-#pragma unroll
-    for (int c = 0; c < 8; ++c) o[c] = fmaf(vf[c] - v[c], sigmoidf(pv[c] + xv[c]), v[c]);
-    put(A.v_out, o);
-  }
-  in(A.a0, ch, p0);
-  float kk[8], ss = 0.f;
-#pragma unroll
-  for (int c = 0; c < 8; ++c) { kk[c] = k[c] * p1[c]; ss = fmaf(kk[c], kk[c], ss); }
-  const float inv = 1.f / fmaxf(sqrtf(oct_sum(ss)), 1e-12f);
-  float ko[8], bo[8];
-#pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    const float a = round_io<T>(sigmoidf(p0[c] + xa[c]));
-    kk[c] *= inv;
-    ko[c] = k[c] * (1.f + (a - 1.f) * p2[c]);
-    o[c] = -kk[c];
-    bo[c] = kk[c] * a;
-  }
-  put(A.k_out, ko); put(A.a_out, o); put(A.b_out, bo);
+  auto in = [&](const void* p, float (&o)[8]) { ld8(reinterpret_cast<const T*>(p) + el, o); };
+  float xw[8], k[8], xa[8], v[8], vf[8], xv[8];
+  in(A.xw, xw); in(A.k, k); in(A.xa, xa);
+  if (VMIX) { in(A.v, v); in(A.vf, vf); in(A.xv, xv); }
+  pre_unit<T, VMIX>(A, el, ch, true, xw, k, xa, v, vf, xv);
 }
 
 // Workgroup b: head b % H, tokens (b / H) * PRE_UNITS + unit, stepping by PRE_UNITS * (gridDim.x / H)

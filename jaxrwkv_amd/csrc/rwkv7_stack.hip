@@ -6,7 +6,7 @@
 // derivative are applied where a product is stored, and the cotangents that several layers or kernels give are added where one is made.
 // Forward and backward now: 4 x 512 tokens 12.7 -> 7.6 ms (the GPU's time), 1 x 23 tokens 11.0 -> 3.0; 8 layers of 1024 channels,
 // 4 x 19 tokens 8.2 -> 2.5; forward alone of 24 layers of 2048 channels, 3 x 346 tokens 8.1 -> 7.7.
-//   forward:  norm, shift, six interpolations | r, k, v, first low-rank factors | second ones | gates | recurrence | group norm, bonus,
+//   forward:  norm, shift, six interpolations | r, k, v, first low-rank factors | second ones, gates | recurrence | group norm, bonus,
 //             gate | output | norm, shift, interpolation | key | value
 //   backward: value | key | norm | output | group norm | recurrence | gates | r, k, v, low-rank factors (three launches) | norm, each
 //             product's two cotangents in one launch
@@ -197,19 +197,19 @@ int launch_rwkv7_stack_fwd(const Rwkv7Stack& D, hipStream_t stream, hipError_t& 
       for (int i = 0; i < n_lora; ++i) G.add(S.hid[i], S.mix[LORA_MIX[i]], f1[i], M, K.d[i], C, 0, 1, act[i]);
       HIPRWKV_TRY(G.launch(stream));
     }
-    {
-      Products G;
-      for (int i = 0; i < n_lora; ++i) G.add(S.lora[i], S.hid[i], f2[i], M, C, K.d[i], 0, 1);
-      HIPRWKV_TRY(G.launch(stream));
+    LoraPreArgs X;
+    memset(&X, 0, sizeof(X));
+    for (int i = 0; i < n_lora; ++i) {
+      X.hid[i] = S.hid[i]; X.w2[i] = f2[i]; X.d[i] = (int)K.d[i];
+      X.out[i] = keep || i == 2 ? S.lora[i] : nullptr;
     }
-    PreArgs R;
-    memset(&R, 0, sizeof(R));
+    PreArgs& R = X.P;
     R.rows = M; R.H = D.H;
-    R.xw = S.lora[0]; R.k = S.k; R.xa = S.lora[1];
-    if (l) { R.v = S.v; R.vf = v_first; R.xv = S.lora[3]; R.v0 = of(P.v0, l, C); R.v_out = S.v2; }
+    R.k = S.k;
+    if (l) { R.v = S.v; R.vf = v_first; R.v0 = of(P.v0, l, C); R.v_out = S.v2; }
     R.w0 = of(P.w0, l, C); R.a0 = of(P.a0, l, C); R.k_k = of(P.k_k, l, C); R.k_a = of(P.k_a, l, C);
     R.w = S.w; R.k_out = S.k2; R.a_out = S.a; R.b_out = S.b;
-    HIPRWKV_TRY(launch_rwkv7_pre(0, R, stream));
+    HIPRWKV_TRY(launch_rwkv7_lora_pre(X, stream));
     const size_t states = (size_t)D.B * 64 * C;
     HIPRWKV_TRY_RC(hiprwkv_wkv7_fwd_ends(stream, HIPRWKV_BF16, HIPRWKV_BF16, D.B, D.T, D.H, 64, S.w, S.r, S.k2, S.v2, S.a, S.b,
                                          of(D.s, l, states), reinterpret_cast<const uint32_t*>(D.length), D.new_starts, S.yw, S.sa,

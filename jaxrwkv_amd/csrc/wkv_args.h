@@ -187,6 +187,16 @@ struct GemmArgs {
 };
 int gemm_split(int M, int64_t K, int64_t N);
 hipError_t launch_gemm(GemmArgs A, int split, hipStream_t stream);
+// The second low-rank products and launch_rwkv7_pre in one pass, bf16: xw, xa, g, xv = hid[i] (rows, d[i]) times w2[i] (d[i], H*64), g to
+// out[2], the others, which P's fields of their name do not give, to out[i] where that is not null.  d multiples of 8; without the value
+// residual (P.vf null) hid[3], w2[3] and d[3] are not looked at.
+struct LoraPreArgs {
+  PreArgs P;
+  const void *hid[4], *w2[4];
+  int d[4];
+  void* out[4];
+};
+hipError_t launch_rwkv7_lora_pre(const LoraPreArgs& A, hipStream_t stream);
 // The same products of one or two rows of norm and interpolation (LnMixArgs: bf16, C a multiple of 64, at most 4096; mix and
 // out unused): a job's x is that of its aux, the mix vector (C,); K = C, N a multiple of 32, not km.
 constexpr int HEAD_GEMM_ROWS = 2;
