@@ -54,7 +54,7 @@ def _grouped(p, like):
     """Whether the grouped products take the low-rank factors beside a (M, C) array: bf16, inner sizes multiples of 8, no
     operand of 2 GiB."""
     return (like.dtype == torch.bfloat16 and like.numel() < 2 ** 30
-            and all(p[n].shape[-1] % 8 == 0 for n in ("w1", "a1", "v1", "g1")))
+            and all(p[n].shape[-1] % 8 == 0 and p[n].shape[-1] * max(like.shape) < 2 ** 30 for n in ("w1", "a1", "v1", "g1")))
 
 
 def _lora_pre_fwd(p, mix, names, k, v, v_first, keep):

@@ -857,6 +857,7 @@ hipError_t launch_gemm(GemmArgs A, int split, hipStream_t stream) {
     stream_k = stream_k && (J.K % TG == 0 || J.K >= 4 * TG);
     skinny = skinny && J.M < GEMM_TILE_ROWS && !J.km && J.aux == nullptr && J.raw == nullptr && J.K % 32 == 0 && J.N % 16 == 0;
   }
+  stream_k = stream_k || longest >= 16 * TG;       // beside a long one the short ones' masked steps do not count
   auto place = [&](int tm, int tn) { tiles = place_jobs(A, [&](const GemmJob& J) { return skinny ? J.N / 16 : tiles_of(J, tm, tn); }); };
   const dim3 block(64 * GEMM_WAVES);
   if (!skinny && stream_k && (split > 1 || A.part != nullptr)) {

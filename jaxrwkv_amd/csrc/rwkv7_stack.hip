@@ -8,7 +8,7 @@
 // 4 x 19 tokens 8.2 -> 2.5; forward alone of 24 layers of 2048 channels, 3 x 346 tokens 8.1 -> 7.7.
 //   forward:  norm, shift, six interpolations | r, k, v, first low-rank factors | second ones, gates | recurrence | group norm, bonus,
 //             gate | output | norm, shift, interpolation | key | value
-//   backward: value | key | norm | output | group norm | recurrence | gates | r, k, v, low-rank factors (three launches) | norm, each
+//   backward: value | key | norm | output | group norm | recurrence | gates | r, k, v, low-rank factors (two launches) | norm, each
 //             product's two cotangents in one launch
 // Values are rounded where the separate operations store them, and a cotangent that is a sum of several once instead of after each.
 #include "common.h"
@@ -332,14 +332,13 @@ int launch_rwkv7_stack_bwd(const Rwkv7Stack& D, hipStream_t stream, hipError_t& 
       }
       HIPRWKV_TRY(Q.launch(stream));
     }
-    Products Q, V;
+    Products Q;
     for (int i = 0; i < n_lora; ++i) {
       bf16_t* const out = W.dmix[LORA_MIX[i]];
       Q.add(out, W.dh[i], f1[i], M, C, K.d[i], 0, 0, GEMM_ADD, i == 3 ? out : nullptr);      // the value residual's on top of v's
-      V.add(to(d1[i], l, C * K.d[i]), S.mix[LORA_MIX[i]], W.dh[i], C, K.d[i], M, 1, 1);
+      Q.add(to(d1[i], l, C * K.d[i]), S.mix[LORA_MIX[i]], W.dh[i], C, K.d[i], M, 1, 1);
     }
     HIPRWKV_TRY(Q.launch(stream));
-    HIPRWKV_TRY(V.launch(stream));
     const void* const mixv[6] = {of(P.x_r, l, C), of(P.x_w, l, C), of(P.x_k, l, C), of(P.x_v, l, C), of(P.x_a, l, C), of(P.x_g, l, C)};
     void* const dhead1[8] = {to(G.x_r, l, C), to(G.x_w, l, C), to(G.x_k, l, C), to(G.x_v, l, C), to(G.x_a, l, C), to(G.x_g, l, C),
                              to(G.ln1_w, l, C), to(G.ln1_b, l, C)};

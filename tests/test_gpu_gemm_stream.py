@@ -37,6 +37,21 @@ def test_several_products_in_one_launch():
         assert ((o.double() - want).abs() <= want.abs() * 2.0 ** -8 + 2.0 ** -14).all()
 
 
+def test_long_and_short_products_in_one_launch():
+    """Beside a long product the short ones go straight to LDS as well, whatever their K."""
+    from jaxrwkv_amd import blocks7
+    g = torch.Generator("cuda").manual_seed(6)
+    jobs, want = [], []
+    for M, N, K, km, kn in ((200, 32, 1030, 1, 1), (136, 264, 8, 0, 0), (72, 128, 40, 0, 1), (72, 72, 72, 1, 0), (64, 64, 5, 1, 1)):
+        x = torch.randn((K, M) if km else (M, K), device="cuda", generator=g).bfloat16()
+        w = torch.randn((K, N) if kn else (N, K), device="cuda", generator=g).bfloat16()
+        jobs.append((torch.empty((M, N), device="cuda", dtype=torch.bfloat16), x, w, km, kn, 0, None))
+        want.append((x.double().T if km else x.double()) @ (w.double() if kn else w.double().T))
+    blocks7._gemm(jobs)
+    for j, v in zip(jobs, want):
+        assert ((j[0].double() - v).abs() <= v.abs() * 2.0 ** -8 + 2.0 ** -18 * 1030 ** 0.5).all()
+
+
 @pytest.mark.parametrize("M,K", [(8, 64), (40, 64), (40, 72)])
 def test_tanh_of_small_values(M, K):
     """The first low-rank factor of the decay starts at zero, so its hidden values start small: tanh keeps their relative precision.
