@@ -100,7 +100,8 @@ struct Forward {
     one = K.D.saved == nullptr ? K.layer(A, false) : Layer();
     v_first = K.D.saved == nullptr ? A.take(n) : nullptr;
     dx = A.take(n);
-    parts = A.take<float>(n * GEMM_MAX_SPLIT);
+    const int out = gemm_split((int)K.rows, K.C, K.C), val = gemm_split((int)K.rows, K.F, K.C), most = out > val ? out : val;
+    parts = A.take<float>(most > 1 ? n * most : 0);
     wkv_bytes = hiprwkv_wkv7_fwd_workspace_bytes(HIPRWKV_BF16, K.D.B, K.D.T, K.D.H, 64);
     wkv = wkv_bytes ? A.take<char>(wkv_bytes) : nullptr;
   }
