@@ -391,9 +391,11 @@ def covers(params, x, state):
 
 
 #: rows x channels^2 up to which the stack is launched from native code.  A layer costs the host 0.3 ms forward (and 0.8 backward)
-#: from Python; its products, which are this package's own there, take that time at 1600 rows of 2048 channels, and the library's,
-#: which the separate steps use, are a fifth faster beyond.
-NATIVE_ROWS_C2, NATIVE_ROWS = 6 * 10 ** 9, 8192
+#: from Python; beyond, the library's large products, which the separate steps use, are worth it.  Native / steps in ms: forward of
+#: 24 layers of 2048 channels 1000 rows 5.7 / 7.7, 1400 8.4 / 8.0 (a third of a round of tiles is empty), 2000 9.5 / 9.9, 2800 12.7 / 13.0,
+#: 3063 13.3 / 13.3, 4084 16.8 / 15.7, 8168 31.7 / 26.0; 24 of 1024, 8000 rows 12.0 / 12.5; 12 of 1024, 16000 rows 12.0 / 11.4; training steps of
+#: 6 of 2048, 2000 rows 9.6 / 9.7; 8 of 1024, 8000 rows 16.2 / 17.2; 6 of 768, 8192 rows 9.9 / 11.6.  NATIVE_ROWS bounds the workspace.
+NATIVE_ROWS_C2, NATIVE_ROWS = 12 * 10 ** 9, 8192
 
 
 def _native(params, x, state, grad):

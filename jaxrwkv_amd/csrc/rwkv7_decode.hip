@@ -10,7 +10,7 @@
 //     7  key projection with relu(.)^2                                        rwkv7_gemm.hip
 //     8  value projection                                                     rwkv7_gemm.hip
 // Measured (eager, host included), general path -> separate launches -> now: 12 layers of 768 channels, one user 5.4 ms -> 0.57 -> 0.41
-// a step, two 0.43, 16 0.61 -> 0.54; 24 layers of 2048 channels, one user 1.61 -> 1.36, 16 1.89 -> 1.69, 256 10.9 -> 3.6 -> 3.4 (7.5
+// a step, two 0.43, 16 0.61 -> 0.54; 24 layers of 2048 channels, one user 1.61 -> 1.36, 16 1.89 -> 1.69, 256 10.9 -> 3.6 -> 3.2 (7.5
 // with the weight-streaming product alone: 51 us a launch at 256 rows, 18 tiled).  Norms inside the products: one user 0.50 -> 0.42 (12 x
 // 768), three as long as before; second low-rank products inside the recurrence 0.42 -> 0.41.
 // References: /root/reference/src/jaxrwkv/rwkv7.py:190-198, :223-267, :269-291.  Products accumulate in fp32 and are rounded

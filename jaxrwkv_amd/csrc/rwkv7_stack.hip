@@ -4,8 +4,8 @@
 // channels, 4 x 512 tokens, forward and backward: 12.9 ms, of which the GPU worked 9.9; 4 x 64 tokens as long).  From here a launch
 // costs 2 to 3 us and there are fewer of them: products that do not wait for each other share one (rwkv7_gemm.hip), relu^2 and its
 // derivative are applied where a product is stored, and the cotangents that several layers or kernels give are added where one is made.
-// Forward and backward now: 4 x 512 tokens 12.7 -> 7.6 ms (the GPU's time), 1 x 23 tokens 11.0 -> 3.0; 8 layers of 1024 channels,
-// 4 x 19 tokens 8.2 -> 2.5; forward alone of 24 layers of 2048 channels, 3 x 346 tokens 8.1 -> 7.7.
+// Forward and backward now: 4 x 512 tokens 12.7 -> 6.8 ms (the GPU's time), 1 x 23 tokens 11.0 -> 3.0; 8 layers of 1024 channels,
+// 4 x 19 tokens 8.2 -> 2.5; forward alone of 24 layers of 2048 channels, 4 x 250 tokens 7.7 -> 5.7, 3 x 39 7.8 -> 2.4.
 //   forward:  norm, shift, six interpolations | r, k, v, first low-rank factors | second ones, gates | recurrence | group norm, bonus,
 //             gate | output | norm, shift, interpolation | key | value
 //   backward: value | key | norm | output | group norm | recurrence | gates | r, k, v, low-rank factors (two launches) | norm, each
