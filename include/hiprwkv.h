@@ -134,8 +134,8 @@ int hiprwkv_wkv7_fwd_parts(hiprwkv_stream stream, int io_dtype, int state_dtype,
                            void* out, void* sa, void* new_s, void* workspace, size_t workspace_bytes, unsigned flags);
 
 /* The same for a call with a backward to come: `ends` (hiprwkv_wkv7_ends_bytes, 0 where it is of no use, 16-byte aligned; NULL: none
- * wanted; not with HIPRWKV_FORCE_SEQ) receives the states at which hiprwkv_wkv7_bwd_ends, given the same array, cuts the
- * sequence into parts that run at the same time. */
+ * wanted; not with HIPRWKV_FORCE_SEQ) receives what hiprwkv_wkv7_bwd_ends, given the same array, needs of the states at which it
+ * cuts the sequence into parts that run at the same time (the layout is the library's own). */
 size_t hiprwkv_wkv7_ends_bytes(int io_dtype, int64_t B, int64_t T, int64_t H, int64_t N);
 int hiprwkv_wkv7_fwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype,
                           int64_t B, int64_t T, int64_t H, int64_t N,

@@ -177,7 +177,8 @@ int hiprwkv_wkv7_fwd_parts(hiprwkv_stream stream, int io_dtype, int state_dtype,
 
 size_t hiprwkv_wkv7_ends_bytes(int io_dtype, int64_t B, int64_t T, int64_t H, int64_t N) {
   if (!wkv7_in_parts(io_dtype, B, T, H, N)) return 0;
-  return (size_t)(B * H) * (wkv7_bwd_parts(B * H, T, io_dtype == HIPRWKV_F32).n_end - 1) * 4096 * sizeof(float);
+  const bool f32 = io_dtype == HIPRWKV_F32;
+  return wkv7_ends_bytes(B * H, wkv7_bwd_parts(B * H, T, f32), f32);
 }
 
 int hiprwkv_wkv7_fwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype, int64_t B, int64_t T, int64_t H, int64_t N,
@@ -212,6 +213,7 @@ int hiprwkv_wkv7_fwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype, 
   if (ends != nullptr && hiprwkv_wkv7_ends_bytes(io_dtype, B, T, H, N) != 0) {
     const Wkv7BwdSplit S = wkv7_bwd_parts(B * H, T, io_dtype == HIPRWKV_F32);
     A.ends = static_cast<float*>(ends); A.n_end = S.n_end; A.end_chunks = S.end_chunks;
+    A.sa_in = sa;
   }
   // T <= 8 (decode) runs on the small-T kernel; otherwise the chunked matrix-core kernels (fp16 operands for bf16
   // I/O, fp32 operands for fp32 I/O); HIPRWKV_FORCE_SEQ selects the sequential kernel
@@ -221,6 +223,7 @@ int hiprwkv_wkv7_fwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype, 
   hipError_t e = small_t ? launch_wkv7_small_t_fwd(A, st)
                : !chunked ? launch_wkv7_seq_fwd(A, st)
                : A.io_f32 ? launch_wkv7_chunk_fwd_f32(A, st) : launch_wkv7_chunk_fwd(A, st);
+  if (e == hipSuccess && A.ends != nullptr && !A.io_f32) e = launch_wkv7_ends(A, st);
   if (e != hipSuccess) return fail(HIPRWKV_ELAUNCH, "wkv7_fwd: %s", hipGetErrorString(e));
   return HIPRWKV_OK;
 }
@@ -274,8 +277,10 @@ int hiprwkv_wkv7_bwd(hiprwkv_stream stream, int io_dtype, int state_dtype, int64
 }
 
 size_t hiprwkv_wkv7_bwd_ends_workspace_bytes(int io_dtype, int64_t B, int64_t T, int64_t H, int64_t N) {
-  const size_t base = hiprwkv_wkv7_bwd_workspace_bytes(B, T, H, N), ends = hiprwkv_wkv7_ends_bytes(io_dtype, B, T, H, N);
-  return ends == 0 ? base : base + 16 + ends + wkv7_bwd_sums_bytes(B * H, wkv7_bwd_parts(B * H, T, io_dtype == HIPRWKV_F32));
+  const size_t base = hiprwkv_wkv7_bwd_workspace_bytes(B, T, H, N);
+  if (hiprwkv_wkv7_ends_bytes(io_dtype, B, T, H, N) == 0) return base;
+  const Wkv7BwdSplit S = wkv7_bwd_parts(B * H, T, io_dtype == HIPRWKV_F32);
+  return base + 16 + wkv7_ends_bytes(B * H, S, true) + wkv7_bwd_sums_bytes(B * H, S);      // the cotangents are matrices in both types
 }
 
 int hiprwkv_wkv7_bwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype, int64_t B, int64_t T, int64_t H, int64_t N,
@@ -310,13 +315,13 @@ int hiprwkv_wkv7_bwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype, 
   const size_t one = base / 3 - PHASE_SPAN;
   char* ws = static_cast<char*>(workspace);
   A.n_end = 1; A.end_chunks = (int)((T + 15) / 16);
-  if (const size_t bytes = ends != nullptr ? hiprwkv_wkv7_ends_bytes(io_dtype, B, T, H, N) : 0) {
+  if (ends != nullptr && hiprwkv_wkv7_ends_bytes(io_dtype, B, T, H, N) != 0) {
     const Wkv7BwdSplit S = wkv7_bwd_parts(B * H, T, io_dtype == HIPRWKV_F32);
     A.n_end = S.n_end; A.end_chunks = S.end_chunks;
     A.ends = const_cast<float*>(static_cast<const float*>(ends));
     char* const more = ws + (base + 15) / 16 * 16;
     A.gends = reinterpret_cast<float*>(more);
-    if (S.a_parts) { A.parts = more + bytes; A.n_part = S.n_end; A.part_chunks = S.end_chunks; }
+    if (S.a_parts) { A.parts = more + wkv7_ends_bytes(B * H, S, true); A.n_part = S.n_end; A.part_chunks = S.end_chunks; }
   }
   A.dsa = reinterpret_cast<float*>(at_phase(ws, r, 3));
   A.e2 = reinterpret_cast<float*>(at_phase(reinterpret_cast<char*>(A.dsa) + one, r, 5));

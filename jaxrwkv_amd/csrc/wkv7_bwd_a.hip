@@ -747,9 +747,10 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_bwd_a_kernel(Wkv7Ar
 // of a part and START for filling the rings (4 us).  Sweeps B and C need nothing but the boundaries; sweep A needs a launch for
 // the summaries (as many workgroups again) and a fold of FOLD per part, and stays whole where that costs more.  Below a tenth
 // gained by this count the whole sequence was as fast or faster (192 heads of 700 tokens 217 and 222 us, 208 of 1000: 298 and 304).
-// A chunk of the fp32 sweeps takes twice as long (2.7 us), so START and FOLD weigh half as much there.  Three sweeps, whole -> parts:
-// bf16 B=1 T=2048 H=32 545 -> 158 us, B=4 T=1024 H=16 287 -> 152, B=4 T=1024 H=32 293 -> 209, B=1 T=64 H=12 42 -> 33; fp32 1000 -> 269,
-// 519 -> 249, 549 -> 388, 57 -> 42.
+// A chunk of the fp32 sweeps takes twice as long (2.7 us): START weighs half as much there, FOLD the same, since the fp32 fold runs on
+// the fp64 instruction.  In bf16 the records of the states (wkv7_ends.hip) cost the forward about two thirds of a chunk's time each.
+// Forward and the three sweeps, whole -> parts: bf16 B=1 T=2048 H=32 592 -> 226 us, B=4 T=1024 H=16 330 -> 203, B=4 T=1024 H=32
+// 344 -> 271, B=4 T=260 H=30 119 -> 106, B=1 T=128 H=12 67 -> 51; fp32 1135 -> 410, 625 -> 356, 706 -> 548, 216 -> 176, 115 -> 78.
 constexpr int CUS = 256, MAX_PARTS = 32;
 Wkv7BwdSplit wkv7_bwd_parts(int64_t heads, int64_t T, bool f32) {
   const int64_t START = f32 ? 2 : 4, FOLD = 1;
@@ -762,13 +763,17 @@ Wkv7BwdSplit wkv7_bwd_parts(int64_t heads, int64_t T, bool f32) {
     if (np < 2) continue;
     const int64_t whole = rounds(heads) * (nch + START);
     const int64_t parts = (rounds(heads * (2 * np - 3)) + rounds(heads * np)) * (c + START) + FOLD * np;
-    const int64_t cost = 2 * rounds(heads * np) * (c + START) + (parts < whole ? parts : whole);
+    const int64_t ends = f32 ? 0 : rounds(heads * (np - 1)) * (c + START) * 2 / 3;
+    const int64_t cost = 2 * rounds(heads * np) * (c + START) + (parts < whole ? parts : whole) + ends;
     if (cost < least) { least = cost; best = {(int)np, (int)c, parts < whole}; }
   }
   return best;
 }
 size_t wkv7_bwd_sums_bytes(int64_t heads, const Wkv7BwdSplit& S) {
   return S.a_parts ? (size_t)heads * (S.n_end - 1) * (sizeof(PartSum) + 8 * sizeof(int)) : 0;
+}
+size_t wkv7_ends_bytes(int64_t heads, const Wkv7BwdSplit& S, bool f32) {
+  return (size_t)heads * (S.n_end - 1) * (f32 ? 4096 * sizeof(float) : sizeof(EndSum));
 }
 
 namespace {

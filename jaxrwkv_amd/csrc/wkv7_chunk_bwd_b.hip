@@ -103,17 +103,6 @@ __device__ __forceinline__ void split8(const float4 lo4, const float4 hi4, u32x4
   split2(hi4.z, hi4.w, a, b); h[3] = a; l[3] = b;
 }
 
-// the same for eight fp16 values (11 significant bits: the pair is exact)
-__device__ __forceinline__ void split8h(const uint4 raw, u32x4_t& h, u32x4_t& l) {
-  typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
-  const h8_t x = __builtin_bit_cast(h8_t, raw);
-  uint32_t a, b;
-  split2((float)x[0], (float)x[1], a, b); h[0] = a; l[0] = b;
-  split2((float)x[2], (float)x[3], a, b); h[1] = a; l[1] = b;
-  split2((float)x[4], (float)x[5], a, b); h[2] = a; l[2] = b;
-  split2((float)x[6], (float)x[7], a, b); h[3] = a; l[3] = b;
-}
-
 __device__ __forceinline__ void produce(const Producer& P, const Raw& x, const ChunkFlags& F, Slot* __restrict__ slot,
                                         SnapSlot* __restrict__ snap, unsigned* events) {
   const int lane = P.lane, t = lane & 15, g = lane >> 4;
@@ -474,8 +463,8 @@ __device__ __forceinline__ void consume(Consumer& C, const Slot* __restrict__ sl
 // publishes ready = c + 1; consumers take chunks in order.  Every wait is for a strictly earlier chunk, so the
 // hand-shake cannot cycle.
 //
-// A workgroup runs one of the sequence's A.n_end parts (one: the whole sequence), from the state that the forward left at the
-// part's first chunk.  The open entry of a part's last token stays without e2 of the next one: the carry that sweep C enters the
+// A workgroup runs one of the sequence's A.n_end parts (one: the whole sequence), from the state at the part's first chunk
+// (fold_ends).  The open entry of a part's last token stays without e2 of the next one: the carry that sweep C enters the
 // part with has it (end_carry).
 __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_chunk_bwd_b_kernel(Wkv7Args A) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -504,15 +493,7 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_chunk_bwd_b_kernel(
     C.lane = lane;
     C.pend = 0.f;
     const int n = lane & 15, g = lane >> 4;
-    if (part > 0) {
-      load_end_cols(C.S, wave, lane, end_of(A.ends, A, head, part));
-    } else {
-#pragma unroll
-      for (int vt = 0; vt < 4; ++vt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          C.S[vt][i] = ld_state_el(A.s, A.st_f32, state_el(A, b, h, 16 * vt + 4 * g + i, 16 * wave + n));
-    }
+    fold_ends(C.S, wave, lane, A, head, part);
     OutCursor oc;
     oc.tok_bytes = (size_t)A.H * 64 * 2;
     const size_t el0 = (((size_t)b * A.T + (size_t)c_in * CK) * A.H + h) * 64;

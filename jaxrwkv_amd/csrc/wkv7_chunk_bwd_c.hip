@@ -121,17 +121,6 @@ __device__ __forceinline__ void split8(const float4 lo4, const float4 hi4, u32x4
   split2(hi4.z, hi4.w, a, b); h[3] = a; l[3] = b;
 }
 
-// the same for eight fp16 values (11 significant bits: the pair is exact)
-__device__ __forceinline__ void split8h(const uint4 raw, u32x4_t& h, u32x4_t& l) {
-  typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
-  const h8_t x = __builtin_bit_cast(h8_t, raw);
-  uint32_t a, b;
-  split2((float)x[0], (float)x[1], a, b); h[0] = a; l[0] = b;
-  split2((float)x[2], (float)x[3], a, b); h[1] = a; l[1] = b;
-  split2((float)x[4], (float)x[5], a, b); h[2] = a; l[2] = b;
-  split2((float)x[6], (float)x[7], a, b); h[3] = a; l[3] = b;
-}
-
 __device__ __forceinline__ void produce(const Producer& P, const Raw& x, const ChunkFlags& F, Slot* __restrict__ slot,
                                         SnapSlot* __restrict__ snap, unsigned* events) {
   const int lane = P.lane, t = lane & 15, g = lane >> 4;
@@ -544,7 +533,7 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_chunk_bwd_c_kernel(
     if (part + 1 < A.n_end) {
       f32x4_t S[4];
       load_end_cols(C.G, wave, lane, end_of(A.gends, A, head, part + 1));
-      load_end_cols(S, wave, lane, end_of(A.ends, A, head, part + 1));
+      fold_ends(S, wave, lane, A, head, part + 1);
       C.carry = end_carry(C.G, S);
     } else {
 #pragma unroll

@@ -715,8 +715,6 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_kernel(Wkv7Args
     oc.voff = (uint32_t)((4 * (lane >> 4)) * (int)A.H * 64 + 16 * cq + (lane & 15));
     // the chunk of token length-1, if this workgroup writes the returned state
     const int csnap = MODE != SUMMARY && L >= 1 && (int)((L - 1) / CK) >= j_out ? (int)((L - 1) / CK) - j0 : -1;
-    // the next chunk boundary whose state the backward starts a part from
-    int end = PARK && A.ends != nullptr ? (j_out / A.end_chunks + 1) * A.end_chunks : nch;
     Ops ops;
     bool ok = true;
     if (n > 0) {
@@ -735,11 +733,6 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_kernel(Wkv7Args
                    });
       // every LDS read of slot si has returned: its data went into the MFMAs above
       if (lane == 0) __hip_atomic_store(&sy->consumed[cq][si], j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-      if (PARK && j0 + j + 1 == end && end < nch) {
-        rare_path();
-        store_end(C.S, cq, lane, A.ends, A, head, end / A.end_chunks);
-        end += A.end_chunks;
-      }
       si = sn;
     }
     if (MODE == SUMMARY) {
@@ -799,7 +792,6 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_kernel(Wkv7Args
     const int64_t t0 = (int64_t)j_out * CK, rows = MODE == WHOLE || (int64_t)(j0 + n) * CK > A.T ? A.T - t0 : (int64_t)(j0 + n) * CK - t0;
     poison_token_rows(A.out, 2, b, h, A.T, A.H, t0, rows);
     poison_token_rows(A.sa, 2, b, h, A.T, A.H, t0, rows);
-    if (PARK && A.ends != nullptr) poison_ends(A.ends, A, head, j_out + 1, j0 + n);
     if (MODE == WHOLE || (L == 0 ? part == 0 : L - 1 >= t0 && L - 1 < t0 + rows)) poison_state(A.new_s, A.st_f32, b, h, A.H);
   }
 }

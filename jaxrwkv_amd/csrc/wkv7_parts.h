@@ -4,14 +4,28 @@
 //   * summaries.  The state (in the reverse sweep the cotangent of the state) that leaves a part is an affine map of the one that
 //     enters it, S_end = S_start M + B.  Workgroups of a first launch make M and B of every part, those of a second one fold the
 //     summaries before theirs into their entering state.
-//   * ends.  What a launch carries past a boundary it also leaves in memory: the forward the states (when it keeps `sa`), the
-//     reverse sweep A their cotangents.  Sweeps B and C, which need nothing else from other parts, start from these.
+//   * ends.  Sweeps B and C need nothing from other parts but the state at a boundary and its cotangent.  The cotangents are left in
+//     memory by sweep A, which carries them past the boundaries, the states in fp32 by the forward (when it keeps `sa`).  The
+//     bf16 forward carries its state with fp16 operands, five bits fewer than sweep B's pairs (gw came out up to 1.1 % further from
+//     64 bits from there), so in bf16 a launch of its own (wkv7_ends.hip) leaves a record per part, EndSum, and the sweeps fold those
+//     before their part.
 #pragma once
 #include "chunk_common.h"
 #include "wkv_args.h"
 
 namespace hiprwkv {
 namespace chunk {
+
+// eight fp16 values (11 significant bits) as bf16 hi and lo parts; the pair is exact
+__device__ __forceinline__ void split8h(const uint4 raw, u32x4_t& h, u32x4_t& l) {
+  typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
+  const h8_t x = __builtin_bit_cast(h8_t, raw);
+  uint32_t a, b;
+  split2((float)x[0], (float)x[1], a, b); h[0] = a; l[0] = b;
+  split2((float)x[2], (float)x[3], a, b); h[1] = a; l[1] = b;
+  split2((float)x[4], (float)x[5], a, b); h[2] = a; l[2] = b;
+  split2((float)x[6], (float)x[7], a, b); h[3] = a; l[3] = b;
+}
 
 // What a workgroup does with its sequence: all of it, a part's summary, or a part.
 enum { WHOLE = 0, SUMMARY = 1, PART = 2 };
@@ -167,6 +181,36 @@ __device__ __forceinline__ void poison_ends(float* ends, const Wkv7Args& A, int6
     if (part * A.end_chunks < c0 || part * A.end_chunks > c1) continue;
     float* const p = end_of(ends, A, head, part);
     for (int i = threadIdx.x; i < 4096; i += blockDim.x) p[i] = __uint_as_float(0x7fc00000u);
+  }
+}
+// bf16: what a part does to the state.  With sa_t known (the residual) the state is linear key by key, so the map is a decay per key.
+struct EndSum {
+  f32x4_t S[4][4][64];     // [consumer q][value tile]: the part's own contribution, tiles of a key-column split
+  float decay[64];         // per key; negative where the part holds a reset: nothing that entered is left
+};
+__device__ __forceinline__ EndSum* end_sum(const Wkv7Args& A, int64_t head, int part) {
+  return reinterpret_cast<EndSum*>(A.ends) + head * (A.n_end - 1) + part;
+}
+// The state in front of part `part` >= 0, key columns 16q ..: S[vt][i] = value 16 vt + 4g + i, key 16q + n
+__device__ __forceinline__ void fold_ends(f32x4_t (&S)[4], int q, int lane, const Wkv7Args& A, int64_t head, int part) {
+  const size_t el = ((size_t)head * 64 + 4 * (lane >> 4)) * 64 + 16 * q + (lane & 15);
+#pragma unroll
+  for (int vt = 0; vt < 4; ++vt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const size_t e = el + (size_t)(16 * vt + i) * 64;
+      S[vt][i] = A.st_f32 ? static_cast<const float*>(A.s)[e] : bf16_to_f32(static_cast<const uint16_t*>(A.s)[e]);
+    }
+#pragma unroll 4
+  for (int p = 0; p < part; ++p) {
+    const EndSum* const e = end_sum(A, head, p);
+    const float d = e->decay[16 * q + (lane & 15)];
+#pragma unroll
+    for (int vt = 0; vt < 4; ++vt) {
+      const f32x4_t add = e->S[q][vt][lane];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) S[vt][i] = d < 0.f ? add[i] : fmaf(S[vt][i], d, add[i]);
+    }
   }
 }
 // key columns 16q .. of it (tiles of a key-column split, as in sweeps B and C): S[vt][i] = value 16 vt + 4g + i, key 16q + n

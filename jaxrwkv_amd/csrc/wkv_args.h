@@ -38,8 +38,9 @@ struct Wkv7Args {
   // sweep A: wkv7_bwd_parts, n_part < 2: whole)
   void* parts;
   int n_part, part_chunks;
-  // The parts of sweeps B and C: n_end of end_chunks chunks.  ends: the states at their boundaries, left by the forward that keeps
-  // sa (null there: none wanted); gends: the cotangents of these, left by sweep A.  (heads, n_end - 1, 64, 64) fp32.
+  // The parts of sweeps B and C: n_end of end_chunks chunks.  ends, made with the forward that keeps sa (null there: none wanted):
+  // fp32 I/O the states at their boundaries, (heads, n_end - 1, 64, 64) fp32, bf16 I/O records that give them (wkv7_parts.h);
+  // gends: the cotangents of these states, left by sweep A.
   float *ends, *gends;
   int n_end, end_chunks;
 };
@@ -52,6 +53,7 @@ struct Wkv7BwdSplit {
 };
 Wkv7BwdSplit wkv7_bwd_parts(int64_t heads, int64_t T, bool f32);
 size_t wkv7_bwd_sums_bytes(int64_t heads, const Wkv7BwdSplit& S);      // summaries of sweep A
+size_t wkv7_ends_bytes(int64_t heads, const Wkv7BwdSplit& S, bool f32);
 
 // Wkv6Args::flags bit: w is (H,64), shared by every token and sequence (HIPRWKV_W_PER_HEAD)
 constexpr unsigned FLAG_W_PER_HEAD = 0x10u;
@@ -238,6 +240,7 @@ hipError_t launch_wkv7_small_t_fwd(const Wkv7Args& A, hipStream_t stream);
 hipError_t launch_wkv6_small_t_fwd(const Wkv6Args& A, hipStream_t stream);
 hipError_t launch_wkv7_chunk_bwd_a(const Wkv7Args& A, hipStream_t stream);
 hipError_t launch_wkv7_chunk_bwd_b(const Wkv7Args& A, hipStream_t stream);
+hipError_t launch_wkv7_ends(const Wkv7Args& A, hipStream_t stream);
 hipError_t launch_wkv7_chunk_bwd_c(const Wkv7Args& A, hipStream_t stream);
 hipError_t launch_wkv7_seq_bwd_a(const Wkv7Args& A, hipStream_t stream);
 hipError_t launch_wkv7_seq_bwd_b(const Wkv7Args& A, hipStream_t stream);
