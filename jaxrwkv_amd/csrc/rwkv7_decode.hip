@@ -121,8 +121,10 @@ __global__ __launch_bounds__(256, LORA ? 1 : 6) void decode_core_kernel(CoreArgs
         for (int f = 0; f < 4; ++f)
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
-            const float xs = j0 + 32 * u + first < A.d[f] ? x[f][u] : 0.f;
-            const uint32_t q[4] = {w[f][u].x, w[f][u].y, w[f][u].z, w[f][u].w};
+            // beyond the factor the last row is read again: both are cleared, either may not be finite
+            const uint32_t have = j0 + 32 * u < A.d[f] ? 0xffffffffu : 0u;
+            const float xs = __uint_as_float(__float_as_uint(x[f][u]) & have);
+            const uint32_t q[4] = {w[f][u].x & have, w[f][u].y & have, w[f][u].z & have, w[f][u].w & have};
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
               acc[f][2 * c] = fmaf(xs, __uint_as_float(q[c] << 16), acc[f][2 * c]);

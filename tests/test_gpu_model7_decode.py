@@ -84,3 +84,22 @@ def test_native_decode_step_of_few_rows(B, T, C, monkeypatch):
     """Norms inside the products and second low-rank products inside the recurrence: two tokens of a sequence and
     of two, widths from one step of a wave to several, inner sizes beyond one round of requests, one row too many."""
     test_native_decode_step(B, T, C, True, monkeypatch)
+
+
+@pytest.mark.parametrize("name", ["w2", "a2", "g2", "v2"])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf")])
+def test_few_rows_with_a_factor_that_is_not_finite(name, value, monkeypatch):
+    """The last row of a second low-rank factor is what requests beyond it re-read: it is not part of other rows' sums."""
+    from jaxrwkv_amd import ops
+    from jaxrwkv_amd.model7 import RWKV7, randomize_weights
+    params = randomize_weights(3, 2, 128, 208, dtype=torch.bfloat16, device="cuda", zero_init=False)
+    params["blocks"]["att"][name][1, -1, 5] = value
+    g = torch.Generator("cuda").manual_seed(3)
+    state = (0.1 * torch.randn((1, 2, 66, 128), device="cuda", generator=g)).bfloat16()
+    tok = torch.tensor([[7]], device="cuda")
+    with torch.no_grad():
+        got = RWKV7.forward(params, tok, state)
+        monkeypatch.setattr(ops, "rwkv7_decode", lambda *a: None)
+        want = RWKV7.forward(params, tok, state)
+    for a, b in zip(got, want):
+        assert torch.equal(torch.isfinite(a), torch.isfinite(b))
