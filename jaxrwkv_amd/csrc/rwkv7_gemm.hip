@@ -506,10 +506,13 @@ __device__ __forceinline__ bool tile_of(const GemmArgs& A, int tm, int tn, int& 
   m0 = (mt < nt ? q : p) * tm;
   return n0 < N && m0 < M;
 }
+// workgroups of a job: the longer side comes in eights, what is beyond it returns at once
 int tiles_of(const GemmJob& J, int tm, int tn) {
   const int mt = (J.M + tm - 1) / tm, nt = (J.N + tn - 1) / tn;
   return ((mt < nt ? nt : mt) + 7) / 8 * 8 * (mt < nt ? mt : nt);
 }
+// those of them that work
+int64_t real_tiles(const GemmJob& J, int tm, int tn) { return (int64_t)((J.M + tm - 1) / tm) * ((J.N + tn - 1) / tn); }
 
 // The same tiles with the operands requested straight into LDS, BUFS - 1 steps ahead: no registers are held by what is in
 // flight.  K is a multiple of the step.  A wave's request fills eight rows of 128 bytes as they lie, so rows cannot be padded:
@@ -839,9 +842,11 @@ int gemm_split(int M, int64_t K, int64_t N) {
 // mean counts and 128 x 128 tiles leave too few to balance.  Weights that no cache holds, us with 64x64, 128x64, 128x128 tiles:
 // 2048 rows: three 768x768 22.2 / 20.2 / 17.9, 768 into 3072 23.1 / 19.2 / 17.4, 3072 into 768 24.0 / 25.5 / 33; with the weights'
 // cotangents: of 768x768 14.0 / 17.0 / 29, of three 41 / 36.6 / 44, of 3072 into 768 43 / 35 / 40.  512 rows: 2048 into 8192 36 / 29 / 25,
-// 8192 into 2048 37 / 52 / 75.  4084 rows: three 2048x2048 225 / 161 / 116.  256 rows of 2048 into 8192: 21 / 18.8 / 24.  The
-// wait of a step is not it: four steps in flight took as long as three (one workgroup per CU), and so did reading half a step ahead
-// of its products.
+// 8192 into 2048 37 / 52 / 75.  4084 rows: three 2048x2048 225 / 161 / 116.  256 rows of 2048 into 8192: 21 / 18.8 / 24.
+// Empty workgroups of the 128 x 128 tiles do not count: with them, and as edges, 24 layers of 2048 channels fell back to 128 x 64 at
+// 2200 rows, 12.9 ms forward, now 12.0, at 2600 14.6, now 12.8, at 3200 18.7, now 14.8.  Those of the smaller tiles do: 12 layers of 768
+// channels were 1 % slower without them (700 and 1500 rows).  The wait of a step is not it: four steps in flight took as long as three
+// (one workgroup per CU), and so did reading half a step ahead of its products.
 constexpr int CUS = 256, WIDE_TILES = 192;
 hipError_t launch_gemm(GemmArgs A, int split, hipStream_t stream) {
   bool skinny = true, stream_k = true, same_k = true;
@@ -870,7 +875,7 @@ hipError_t launch_gemm(GemmArgs A, int split, hipStream_t stream) {
     auto cost = [&](int tm, int tn) {
       int64_t n = 0, steps = 0, area = 0;
       for (int i = 0; i < A.n_jobs; ++i) {
-        const int64_t t = tiles_of(A.job[i], tm, tn);
+        const int64_t t = tn > TG ? real_tiles(A.job[i], tm, tn) : tiles_of(A.job[i], tm, tn);
         n += t;
         area += (int64_t)A.job[i].M * A.job[i].N;
         steps += t * ((A.job[i].K + TG - 1) / TG);

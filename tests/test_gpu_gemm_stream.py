@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 # K from one step to more than two turns of the buffers, M and N around the tile's edge and at one row past it
 @pytest.mark.parametrize("km,kn", [(0, 0), (0, 1), (1, 0), (1, 1)])
 @pytest.mark.parametrize("M,N,K", [(40, 8, 64), (64, 64, 128), (72, 72, 192), (256, 200, 256), (136, 64, 320), (64, 1032, 576), (520, 136, 2048), (136, 6144, 320),
-                                   (264, 8200, 192)])
+                                   (264, 8200, 192), (2200, 2048, 192)])
 def test_product(M, N, K, km, kn):
     from jaxrwkv_amd import blocks7
     g = torch.Generator("cuda").manual_seed(M + N + K)
