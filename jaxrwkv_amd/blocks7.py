@@ -390,12 +390,14 @@ def covers(params, x, state):
                and p[f + "1"].numel() == p[f + "2"].numel() == n * p[f + "1"].shape[-1] for f in "wavg")
 
 
-#: rows x channels^2 up to which the stack is launched from native code.  A layer costs the host 0.3 ms forward (and 0.8 backward)
-#: from Python; beyond, the library's large products, which the separate steps use, are worth it.  Native / steps in ms: forward of
-#: 24 layers of 2048 channels 1000 rows 5.7 / 7.7, 1400 8.4 / 8.0 (a third of a round of tiles is empty), 2000 9.5 / 9.9, 2800 12.7 / 13.0,
-#: 3063 13.3 / 13.3, 4084 16.8 / 15.7, 8168 31.7 / 26.0; 24 of 1024, 8000 rows 12.0 / 12.5; 12 of 1024, 16000 rows 12.0 / 11.4; training steps of
-#: 6 of 2048, 2000 rows 9.6 / 9.7; 8 of 1024, 8000 rows 16.2 / 17.2; 6 of 768, 8192 rows 9.9 / 11.6.  NATIVE_ROWS bounds the workspace.
-NATIVE_ROWS_C2, NATIVE_ROWS = 12 * 10 ** 9, 8192
+#: rows x channels^2 up to which the stack is launched from native code: up to 1536 channels, and beyond.  A layer costs the host 0.3 ms
+#: forward (and 0.8 backward) from Python; from some size on the library's large products, which the separate steps use, are worth it.
+#: Of wide models they are better by more than the host's time, but for sizes that fill the native products' rounds.  Native / steps in ms:
+#: forward of 24 layers of 2048 channels 1000 rows 5.8 / 7.7, 1100 7.3 / 8.0, 1200 8.2 / 8.2, 1400 8.6 / 8.2, 1600 9.1 / 9.3, 2000 9.7 / 10.1,
+#: 2200 12.0 / 11.6, 2500 12.6 / 11.8, 4000 17.0 / 15.9; 6 of 4096, 300 rows 2.24 / 2.41, 600 3.5 / 3.2; 8 of 1536, 2500 rows 3.36 / 3.38, 4000
+#: 4.5 / 4.6; 24 of 1024, 5000 rows 9.4 / 9.5, 8000 12.5 / 13.1; training steps of 4 of 2048, 1200 rows 5.2 / 5.7, 1600 6.18 / 6.19, 2400
+#: 8.7 / 8.4; 4 of 1536, 3000 rows 7.5 / 8.0, 4000 9.56 / 9.56; 8 of 1024, 8000 rows 16.9 / 17.4.  NATIVE_ROWS bounds the workspace.
+NATIVE_ROWS_C2, NATIVE_ROWS_C2_WIDE, NATIVE_ROWS = 9 * 10 ** 9, 5 * 10 ** 9, 8192
 
 
 def _native(params, x, state, grad):
@@ -408,7 +410,8 @@ def _native(params, x, state, grad):
     F = p["ffn_key"].shape[1]
     sizes = (F, *(p[f + "1"].shape[-1] for f in "wavg"))
     shapes = {"ffn_key": (L, F, C), "ffn_value": (L, C, F)}
-    return (x.dtype == torch.bfloat16 and M * C * C <= NATIVE_ROWS_C2 and M <= NATIVE_ROWS and T > 8 and N == 64 and C == H * N
+    most = NATIVE_ROWS_C2 if C <= 1536 else NATIVE_ROWS_C2_WIDE
+    return (x.dtype == torch.bfloat16 and M * C * C <= most and M <= NATIVE_ROWS and T > 8 and N == 64 and C == H * N
             and C % 128 == 0 and F <= 8 * C and all(d % 8 == 0 for d in sizes) and state.shape == (B, L, 2 + N, C)
             and state.is_contiguous() and state.data_ptr() % 16 == 0 and not ops.autocast_elsewhere(x)
             and all(p[n].shape == shapes.get(n, (L, C, C)) for n in _PRODUCTS)
