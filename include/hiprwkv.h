@@ -134,8 +134,8 @@ int hiprwkv_wkv7_fwd_parts(hiprwkv_stream stream, int io_dtype, int state_dtype,
                            void* out, void* sa, void* new_s, void* workspace, size_t workspace_bytes, unsigned flags);
 
 /* The same for a call with a backward to come: `ends` (hiprwkv_wkv7_ends_bytes, 0 where it is of no use, 16-byte aligned; NULL: none
- * wanted; not with HIPRWKV_FORCE_SEQ) receives what hiprwkv_wkv7_bwd_ends, given the same array, needs of the states at which it
- * cuts the sequence into parts that run at the same time (the layout is the library's own). */
+ * wanted; not with HIPRWKV_FORCE_SEQ) goes on to hiprwkv_wkv7_bwd_ends, which then cuts the sequence into parts that run at the
+ * same time.  It holds what is needed of the states there, put in by this call (HIPRWKV_F32) or by the backward itself. */
 size_t hiprwkv_wkv7_ends_bytes(int io_dtype, int64_t B, int64_t T, int64_t H, int64_t N);
 int hiprwkv_wkv7_fwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype,
                           int64_t B, int64_t T, int64_t H, int64_t N,
@@ -187,7 +187,7 @@ int hiprwkv_wkv7_bwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype,
                           const void* w, const void* r, const void* k, const void* v,
                           const void* a, const void* b, const void* s,
                           const uint32_t* length, const uint8_t* new_starts,
-                          const void* gy, const void* sa, const void* gs_out, const void* ends,
+                          const void* gy, const void* sa, const void* gs_out, void* ends,
                           void* gw, void* gr, void* gk, void* gv, void* ga, void* gb, void* gs,
                           void* workspace, size_t workspace_bytes, unsigned flags);
 

@@ -210,10 +210,9 @@ int hiprwkv_wkv7_fwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype, 
   A.flags = flags;
   A.status = status_word();
   A.parts = need != 0 ? workspace : nullptr;
-  if (ends != nullptr && hiprwkv_wkv7_ends_bytes(io_dtype, B, T, H, N) != 0) {
-    const Wkv7BwdSplit S = wkv7_bwd_parts(B * H, T, io_dtype == HIPRWKV_F32);
+  if (A.io_f32 && ends != nullptr && hiprwkv_wkv7_ends_bytes(io_dtype, B, T, H, N) != 0) {      // in bf16 the backward fills it
+    const Wkv7BwdSplit S = wkv7_bwd_parts(B * H, T, true);
     A.ends = static_cast<float*>(ends); A.n_end = S.n_end; A.end_chunks = S.end_chunks;
-    A.sa_in = sa;
   }
   // T <= 8 (decode) runs on the small-T kernel; otherwise the chunked matrix-core kernels (fp16 operands for bf16
   // I/O, fp32 operands for fp32 I/O); HIPRWKV_FORCE_SEQ selects the sequential kernel
@@ -223,7 +222,6 @@ int hiprwkv_wkv7_fwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype, 
   hipError_t e = small_t ? launch_wkv7_small_t_fwd(A, st)
                : !chunked ? launch_wkv7_seq_fwd(A, st)
                : A.io_f32 ? launch_wkv7_chunk_fwd_f32(A, st) : launch_wkv7_chunk_fwd(A, st);
-  if (e == hipSuccess && A.ends != nullptr && !A.io_f32) e = launch_wkv7_ends(A, st);
   if (e != hipSuccess) return fail(HIPRWKV_ELAUNCH, "wkv7_fwd: %s", hipGetErrorString(e));
   return HIPRWKV_OK;
 }
@@ -286,7 +284,7 @@ size_t hiprwkv_wkv7_bwd_ends_workspace_bytes(int io_dtype, int64_t B, int64_t T,
 int hiprwkv_wkv7_bwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype, int64_t B, int64_t T, int64_t H, int64_t N,
                           const void* w, const void* r, const void* k, const void* v, const void* a, const void* b,
                           const void* s, const uint32_t* length, const uint8_t* new_starts, const void* gy, const void* sa,
-                          const void* gs_out, const void* ends, void* gw, void* gr, void* gk, void* gv, void* ga, void* gb,
+                          const void* gs_out, void* ends, void* gw, void* gr, void* gk, void* gv, void* ga, void* gb,
                           void* gs, void* workspace, size_t workspace_bytes, unsigned flags) {
   int rc = check_matrix_shape("wkv7_bwd", io_dtype, state_dtype, B, T, H, N);
   if (rc) return rc;
@@ -318,7 +316,7 @@ int hiprwkv_wkv7_bwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype, 
   if (ends != nullptr && hiprwkv_wkv7_ends_bytes(io_dtype, B, T, H, N) != 0) {
     const Wkv7BwdSplit S = wkv7_bwd_parts(B * H, T, io_dtype == HIPRWKV_F32);
     A.n_end = S.n_end; A.end_chunks = S.end_chunks;
-    A.ends = const_cast<float*>(static_cast<const float*>(ends));
+    A.ends = static_cast<float*>(ends);
     char* const more = ws + (base + 15) / 16 * 16;
     A.gends = reinterpret_cast<float*>(more);
     if (S.a_parts) { A.parts = more + wkv7_ends_bytes(B * H, S, true); A.n_part = S.n_end; A.part_chunks = S.end_chunks; }

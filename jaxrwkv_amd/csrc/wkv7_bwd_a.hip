@@ -35,6 +35,7 @@
 // to a total of -80, so that 1/E_s stays finite in fp32 (cap_chunk_decay), as in the forward kernel.
 #include "chunk_common.h"
 #include "wkv_args.h"
+#include "wkv7_ends.h"
 #include "wkv7_parts.h"
 
 namespace hiprwkv {
@@ -592,7 +593,8 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
 // MODE as in wkv7_fwd.hip, run backwards in time: where (sequence, head) workgroups leave most of the GPU idle, a first launch makes
 // the summaries of all parts but the first (G = 0 or the identity with dy = 0 behind the part), a second one folds those of the
 // parts after its own and runs.  Measured: see wkv7_bwd_parts.
-template <int MODE>
+// ENDS (the first launch of a backward in parts): behind its own workgroups come those that make the records for sweeps B and C.
+template <int MODE, bool ENDS>
 __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_bwd_a_kernel(Wkv7Args A) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Slot* slots = reinterpret_cast<Slot*>(smem_raw);
@@ -602,6 +604,11 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_bwd_a_kernel(Wkv7Ar
   const int lane = threadIdx.x & 63;
   // head, part (0: the last of the sequence) and (SUMMARY) which half of the summary
   const int per_head = MODE == SUMMARY ? 2 * A.n_part - 3 : MODE == PART ? A.n_part : 1;
+  if (ENDS && blockIdx.x >= A.B * A.H * per_head) {
+    static_assert(NCONS + NPROD == 2 * END_GROUPS, "all waves of a workgroup take part");
+    make_ends(A, blockIdx.x - A.B * A.H * per_head, smem_raw);
+    return;
+  }
   const int64_t head = MODE == WHOLE ? (int64_t)blockIdx.x : (int64_t)(blockIdx.x / per_head);
   const int unit = MODE == WHOLE ? 0 : (int)(blockIdx.x % per_head);
   const bool map = MODE == SUMMARY && unit >= A.n_part - 1;           // this workgroup makes M
@@ -748,9 +755,11 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_bwd_a_kernel(Wkv7Ar
 // the summaries (as many workgroups again) and a fold of FOLD per part, and stays whole where that costs more.  Below a tenth
 // gained by this count the whole sequence was as fast or faster (192 heads of 700 tokens 217 and 222 us, 208 of 1000: 298 and 304).
 // A chunk of the fp32 sweeps takes twice as long (2.7 us): START weighs half as much there, FOLD the same, since the fp32 fold runs on
-// the fp64 instruction.  In bf16 the records of the states (wkv7_ends.hip) cost the forward about two thirds of a chunk's time each.
-// Forward and the three sweeps, whole -> parts: bf16 B=1 T=2048 H=32 592 -> 226 us, B=4 T=1024 H=16 330 -> 203, B=4 T=1024 H=32
-// 344 -> 271, B=4 T=260 H=30 119 -> 106, B=1 T=128 H=12 67 -> 51; fp32 1135 -> 410, 625 -> 356, 706 -> 548, 216 -> 176, 115 -> 78.
+// the fp64 instruction.  In bf16 the records of the states (wkv7_ends.h) are made in sweep A's first launch.  Of all counts of parts, sweep A
+// whole or not, the rule's was the fastest or within 2 % of it at 16 shapes from B=1 T=48 H=12 to B=4 T=777 H=12 and B=1 T=4096 H=12.
+// Forward and the three sweeps, whole -> parts: bf16 B=1 T=2048 H=32 592 -> 224 us, B=4 T=1024 H=16 331 -> 195, B=4 T=1024 H=32
+// 345 -> 255, B=4 T=260 H=30 120 -> 97, B=1 T=128 H=12 67 -> 48; fp32 B=1 T=2048 H=32 1135 -> 410, B=4 T=1024 H=16 625 -> 356, B=4 T=1024
+// H=32 706 -> 548, B=4 T=260 H=30 216 -> 176, B=1 T=128 H=12 115 -> 78.
 constexpr int CUS = 256, MAX_PARTS = 32;
 Wkv7BwdSplit wkv7_bwd_parts(int64_t heads, int64_t T, bool f32) {
   const int64_t START = f32 ? 2 : 4, FOLD = 1;
@@ -761,10 +770,12 @@ Wkv7BwdSplit wkv7_bwd_parts(int64_t heads, int64_t T, bool f32) {
   for (int64_t p = 2; p <= MAX_PARTS && p <= nch; ++p) {
     const int64_t c = (nch + p - 1) / p, np = (nch + c - 1) / c;
     if (np < 2) continue;
-    const int64_t whole = rounds(heads) * (nch + START);
-    const int64_t parts = (rounds(heads * (2 * np - 3)) + rounds(heads * np)) * (c + START) + FOLD * np;
-    const int64_t ends = f32 ? 0 : rounds(heads * (np - 1)) * (c + START) * 2 / 3;
-    const int64_t cost = 2 * rounds(heads * np) * (c + START) + (parts < whole ? parts : whole) + ends;
+    // bf16: rounds that the records' workgroups (two thirds of a part's time) add to sweep A's first launch
+    auto more = [&](int64_t first) { return f32 ? 0 : (rounds(first + heads * (np - 1)) - rounds(first)) * (c + START) * 2 / 3; };
+    const int64_t maps = heads * (2 * np - 3);
+    const int64_t whole = rounds(heads) * (nch + START) + more(heads);
+    const int64_t parts = (rounds(maps) + rounds(heads * np)) * (c + START) + FOLD * np + more(maps);
+    const int64_t cost = 2 * rounds(heads * np) * (c + START) + (parts < whole ? parts : whole) + (f32 ? 0 : np / 4);      // B and C fold records
     if (cost < least) { least = cost; best = {(int)np, (int)c, parts < whole}; }
   }
   return best;
@@ -777,23 +788,27 @@ size_t wkv7_ends_bytes(int64_t heads, const Wkv7BwdSplit& S, bool f32) {
 }
 
 namespace {
-template <int MODE>
+template <int MODE, bool ENDS>
 hipError_t launch_mode(const Wkv7Args& A, int64_t groups, hipStream_t stream) {
-  const size_t smem = RING * sizeof(Slot) + sizeof(SnapSlot) + sizeof(Sync);
+  constexpr size_t smem = RING * sizeof(Slot) + sizeof(SnapSlot) + sizeof(Sync);
+  static_assert(!ENDS || END_LDS <= smem, "the records' sums fit beside nothing else");
   static LdsAttrOnce once;
-  const hipError_t attr = allow_dynamic_lds(once, reinterpret_cast<const void*>(wkv7_bwd_a_kernel<MODE>), smem);
+  const hipError_t attr = allow_dynamic_lds(once, reinterpret_cast<const void*>(wkv7_bwd_a_kernel<MODE, ENDS>), smem);
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL(wkv7_bwd_a_kernel<MODE>, dim3((unsigned)groups), dim3(64 * (NCONS + NPROD)), smem, stream, A);
+  if (ENDS) groups += A.B * A.H * (A.n_end - 1);
+  hipLaunchKernelGGL((wkv7_bwd_a_kernel<MODE, ENDS>), dim3((unsigned)groups), dim3(64 * (NCONS + NPROD)), smem, stream, A);
   return hipGetLastError();
 }
 }  // namespace
 
-// Reverse sweep of the backward pass: gv, the workspace dsa (cotangent of sa per token) and gs.
+// Reverse sweep of the backward pass: gv, the workspace dsa (cotangent of sa per token) and gs; with parts to come (A.n_end >= 2) the
+// records in A.ends and the cotangents in A.gends.
 hipError_t launch_wkv7_chunk_bwd_a(const Wkv7Args& A, hipStream_t stream) {
   const int64_t heads = A.B * A.H;
-  if (A.n_part < 2) return launch_mode<WHOLE>(A, heads, stream);
-  const hipError_t e = launch_mode<SUMMARY>(A, heads * (2 * A.n_part - 3), stream);
-  return e != hipSuccess ? e : launch_mode<PART>(A, heads * A.n_part, stream);
+  if (A.n_end < 2) return launch_mode<WHOLE, false>(A, heads, stream);
+  if (A.n_part < 2) return launch_mode<WHOLE, true>(A, heads, stream);
+  const hipError_t e = launch_mode<SUMMARY, true>(A, heads * (2 * A.n_part - 3), stream);
+  return e != hipSuccess ? e : launch_mode<PART, false>(A, heads * A.n_part, stream);
 }
 
 }  // namespace hiprwkv

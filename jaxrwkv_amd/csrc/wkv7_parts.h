@@ -7,8 +7,8 @@
 //   * ends.  Sweeps B and C need nothing from other parts but the state at a boundary and its cotangent.  The cotangents are left in
 //     memory by sweep A, which carries them past the boundaries, the states in fp32 by the forward (when it keeps `sa`).  The
 //     bf16 forward carries its state with fp16 operands, five bits fewer than sweep B's pairs (gw came out up to 1.1 % further from
-//     64 bits from there), so in bf16 a launch of its own (wkv7_ends.hip) leaves a record per part, EndSum, and the sweeps fold those
-//     before their part.
+//     64 bits from there), so in bf16 workgroups beside sweep A (wkv7_ends.h) leave a record per part, EndSum, and the sweeps
+//     fold those before their part.
 #pragma once
 #include "chunk_common.h"
 #include "wkv_args.h"
@@ -212,6 +212,9 @@ __device__ __forceinline__ void fold_ends(f32x4_t (&S)[4], int q, int lane, cons
       for (int i = 0; i < 4; ++i) S[vt][i] = d < 0.f ? add[i] : fmaf(S[vt][i], d, add[i]);
     }
   }
+  // the loads are waited for here and not, as far as the compiler can tell, in the chunk loop that follows
+#pragma unroll
+  for (int vt = 0; vt < 4; ++vt) asm volatile("" : "+v"(S[vt]));
 }
 // key columns 16q .. of it (tiles of a key-column split, as in sweeps B and C): S[vt][i] = value 16 vt + 4g + i, key 16q + n
 __device__ __forceinline__ void load_end_cols(f32x4_t (&S)[4], int q, int lane, const float* p) {

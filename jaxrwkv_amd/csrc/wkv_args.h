@@ -38,9 +38,9 @@ struct Wkv7Args {
   // sweep A: wkv7_bwd_parts, n_part < 2: whole)
   void* parts;
   int n_part, part_chunks;
-  // The parts of sweeps B and C: n_end of end_chunks chunks.  ends, made with the forward that keeps sa (null there: none wanted):
-  // fp32 I/O the states at their boundaries, (heads, n_end - 1, 64, 64) fp32, bf16 I/O records that give them (wkv7_parts.h);
-  // gends: the cotangents of these states, left by sweep A.
+  // The parts of sweeps B and C: n_end of end_chunks chunks.  ends: fp32 I/O the states at their boundaries, (heads, n_end - 1, 64,
+  // 64) fp32, left by the forward that keeps sa (null there: none wanted); bf16 I/O records that give them (wkv7_ends.h), made beside
+  // sweep A; gends: the cotangents of these states, left by sweep A.
   float *ends, *gends;
   int n_end, end_chunks;
 };
@@ -240,7 +240,6 @@ hipError_t launch_wkv7_small_t_fwd(const Wkv7Args& A, hipStream_t stream);
 hipError_t launch_wkv6_small_t_fwd(const Wkv6Args& A, hipStream_t stream);
 hipError_t launch_wkv7_chunk_bwd_a(const Wkv7Args& A, hipStream_t stream);
 hipError_t launch_wkv7_chunk_bwd_b(const Wkv7Args& A, hipStream_t stream);
-hipError_t launch_wkv7_ends(const Wkv7Args& A, hipStream_t stream);
 hipError_t launch_wkv7_chunk_bwd_c(const Wkv7Args& A, hipStream_t stream);
 hipError_t launch_wkv7_seq_bwd_a(const Wkv7Args& A, hipStream_t stream);
 hipError_t launch_wkv7_seq_bwd_b(const Wkv7Args& A, hipStream_t stream);
