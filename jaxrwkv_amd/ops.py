@@ -67,6 +67,8 @@ def _empty_phased(shape, dtype, device, phase):
 
 def _empty_like_phased(ref, steps):
     """Like ``torch.empty_like(ref)``, ``steps`` 128-byte phases past ``ref``'s own."""
+    if ref.nbytes < _PHASED_MIN_BYTES:
+        return torch.empty_like(ref)
     return _empty_phased(tuple(ref.shape), ref.dtype, ref.device, _phase(ref) + steps)
 
 
