@@ -438,7 +438,8 @@ int hiprwkv_rwkv7_decode(hiprwkv_stream stream, const hiprwkv_rwkv7_decode_args*
  * each, in the orders of hiprwkv_rwkv7_decode_args.
  *   forward : from x (B,T,C) and the states the residual stream as a sum xs + dx.  state (B,L,2+64,C): rows 0 and 1 are the token-shift
  *             states, read there and written in new_state; s, new_s (L,B,64,C): the recurrence's, as arrays of their own.
- *             saved: L allocations of hiprwkv_rwkv7_stack_saved_bytes for the backward, or null without one to come.
+ *             saved: L allocations for the backward, or null without one to come; of layer l hiprwkv_rwkv7_stack_saved_layer_bytes,
+ *             of any hiprwkv_rwkv7_stack_saved_bytes.
  *   backward: from g_xs, g_dx and, where not null, the cotangents of the new shift states g_shift (2,L,B,C) and recurrence states g_s
  *             (L,B,64,C) to g_x and every parameter's (grad, same order as param; rows of layer 0 of v0, v1, v2 are left alone).  The
  *             forward's x, xs, state, s and saved go in again; there is no cotangent of the states. */
@@ -462,6 +463,7 @@ typedef struct hiprwkv_rwkv7_stack_args {
   hiprwkv_rwkv7_block_params param, grad;
 } hiprwkv_rwkv7_stack_args;
 size_t hiprwkv_rwkv7_stack_saved_bytes(const hiprwkv_rwkv7_stack_args* args);
+size_t hiprwkv_rwkv7_stack_saved_layer_bytes(const hiprwkv_rwkv7_stack_args* args, int64_t layer);
 size_t hiprwkv_rwkv7_stack_workspace_bytes(const hiprwkv_rwkv7_stack_args* args, int backward);
 int hiprwkv_rwkv7_stack_fwd(hiprwkv_stream stream, const hiprwkv_rwkv7_stack_args* args);
 int hiprwkv_rwkv7_stack_bwd(hiprwkv_stream stream, const hiprwkv_rwkv7_stack_args* args);

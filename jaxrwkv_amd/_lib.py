@@ -110,6 +110,7 @@ SIGNATURES = {
     "hiprwkv_rwkv7_decode_workspace_bytes": (_sz, [ctypes.POINTER(Rwkv7DecodeArgs)]),
     "hiprwkv_rwkv7_decode": (_int, [_vp, ctypes.POINTER(Rwkv7DecodeArgs)]),
     "hiprwkv_rwkv7_stack_saved_bytes": (_sz, [ctypes.POINTER(Rwkv7StackArgs)]),
+    "hiprwkv_rwkv7_stack_saved_layer_bytes": (_sz, [ctypes.POINTER(Rwkv7StackArgs), _i64]),
     "hiprwkv_rwkv7_stack_workspace_bytes": (_sz, [ctypes.POINTER(Rwkv7StackArgs), _int]),
     "hiprwkv_rwkv7_stack_fwd": (_int, [_vp, ctypes.POINTER(Rwkv7StackArgs)]),
     "hiprwkv_rwkv7_stack_bwd": (_int, [_vp, ctypes.POINTER(Rwkv7StackArgs)]),

@@ -157,7 +157,8 @@ def _layer_fwd(i, p, x, dx, st, nst, v_first, ns, length, need):
     if i == 0:
         v2 = heads(v)
     s = st[:, 2:].reshape(B, H, N, N)
-    new_s, yw, sa, ends = ops._wkv7_fwd(heads(r), w, k2, v2, a, b, s, length, ns, HipRWKV.assoc_compat, want_sa=keep, want_ends=keep)
+    new_s, yw, sa, ends = ops._wkv7_fwd(heads(r), w, k2, v2, a, b, s, length, ns, HipRWKV.assoc_compat, want_sa=keep,
+                                        want_ends=keep and x.dtype == torch.float32)
     nst[:, 2:] = new_s.view(B, N, C)
     y = flat(ops._postmix_fwd(yw, heads(r), k2, v2, heads(lora["g"]), par("lnx_w"), par("lnx_b"), par("r_k"), EPS_X))
     dx1 = torch.mm(y, p["output"].T).view(B, T, C)
@@ -244,7 +245,7 @@ def _layer_bwd(i, p, grad, scratch, S, ns, length, g_x, g_dx, g_state, g_in, g_v
     # the recurrence
     gs_out = None if g_state is None else g_state[:, 2:].reshape(B, H, N, N)
     gr2, gw, gk2, gv2, ga, gb, gs = ops.wkv7_bwd(heads(S["r"]), S["w"], S["k2"], S["v2"], S["a"], S["b"], S["s"], length, ns,
-                                                 gyw, S["sa"], gs_out, HipRWKV.assoc_compat, ends=S["ends"])
+                                                 gyw, S["sa"], gs_out, HipRWKV.assoc_compat, ends=S["ends"], parts=True)
     if g_in is not None:
         g_in[:, 2:] = gs.reshape(B, N, C)
     # gates
@@ -437,8 +438,8 @@ def _stack_fwd(x, state, ns, length, params, compat, keep):
     xs, dx, new_s, new_state = torch.empty_like(x), torch.empty_like(x), torch.empty_like(s), torch.empty_like(state)
     A = _stack_args(x, state, s, ns, length, params, xs)
     A.dx, A.new_s, A.new_state, A.flags = dx.data_ptr(), new_s.data_ptr(), new_state.data_ptr(), _lib.COMPAT_ASSOC if compat else 0
-    nbytes = lib.hiprwkv_rwkv7_stack_saved_bytes(ctypes.byref(A)) if keep else 0
-    saved = [ops._workspace(nbytes, x.device) for _ in range(A.L if keep else 0)]
+    sizes = [lib.hiprwkv_rwkv7_stack_saved_layer_bytes(ctypes.byref(A), i) for i in (0, A.L // 2, A.L - 1)] if keep else ()
+    saved = [ops._workspace(sizes[0 if i == 0 else 2 if i == A.L - 1 else 1], x.device) for i in range(A.L if keep else 0)]
     arr = ops._ptr_array(saved)
     A.saved = ctypes.addressof(arr) if keep else None
     A.workspace_bytes = lib.hiprwkv_rwkv7_stack_workspace_bytes(ctypes.byref(A), 0)

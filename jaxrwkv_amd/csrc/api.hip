@@ -1006,8 +1006,15 @@ int check_stack(const char* op, const hiprwkv_rwkv7_stack_args* args, bool backw
 }
 }  // namespace
 
+size_t hiprwkv_rwkv7_stack_saved_layer_bytes(const hiprwkv_rwkv7_stack_args* args, int64_t layer) {
+  return args == nullptr || !stack_sizes_ok(*args) || layer < 0 || layer >= args->L ? 0 : rwkv7_stack_saved(*args, layer);
+}
+
 size_t hiprwkv_rwkv7_stack_saved_bytes(const hiprwkv_rwkv7_stack_args* args) {
-  return args == nullptr || !stack_sizes_ok(*args) ? 0 : rwkv7_stack_saved(*args);
+  size_t most = 0;
+  if (args != nullptr)
+    for (int64_t layer : {(int64_t)0, args->L / 2, args->L - 1}) most = std::max(most, hiprwkv_rwkv7_stack_saved_layer_bytes(args, layer));
+  return most;
 }
 
 size_t hiprwkv_rwkv7_stack_workspace_bytes(const hiprwkv_rwkv7_stack_args* args, int backward) {

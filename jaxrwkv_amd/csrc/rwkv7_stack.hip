@@ -35,11 +35,12 @@ struct Arena {
   }
 };
 
-// What the backward reads of a layer's forward.  Without a backward to come all layers use the same memory.
+// What the backward reads of a layer's forward, without what at_layer puts in its place.  Without a backward to come all layers use the
+// same memory (`l` then is any layer between the first and the last).
 struct Layer {
   bf16_t *x, *mix[6], *r, *k, *v, *hid[4], *lora[4], *w, *k2, *v2, *a, *b, *yw, *y, *x2, *xk2, *ff, *fr;      // hid, lora: w, a, g, v
   float *stats1, *stats2;
-  void *sa, *ends;
+  void* sa;
 };
 constexpr int MIX_R = 0, MIX_W = 1, MIX_K = 2, MIX_V = 3, MIX_A = 4, MIX_G = 5;
 constexpr int LORA_MIX[4] = {MIX_W, MIX_A, MIX_G, MIX_V};
@@ -51,21 +52,26 @@ struct Stack {
     d[0] = D.d_decay; d[1] = D.d_aaa; d[2] = D.d_gate; d[3] = D.d_mv;
   }
   size_t ends_bytes() const { return hiprwkv_wkv7_ends_bytes(HIPRWKV_BF16, D.B, D.T, D.H, 64); }
-  Layer layer(Arena& A, bool keep) const {
+  Layer layer(Arena& A, bool keep, int64_t l) const {
     Layer S;
+    memset(&S, 0, sizeof(S));
     const size_t n = rows * C;
-    S.x = A.take(n);
+    const bool first = keep && l == 0, last = keep && l == D.L - 1;
+    if (!first) S.x = A.take(n);
     for (auto& m : S.mix) m = A.take(n);
     S.r = A.take(n); S.k = A.take(n); S.v = A.take(n);
-    for (int i = 0; i < 4; ++i) { S.hid[i] = A.take(rows * d[i]); S.lora[i] = A.take(n); }
-    S.w = A.take(n); S.k2 = A.take(n); S.v2 = A.take(n); S.a = A.take(n); S.b = A.take(n);
-    S.yw = A.take(n); S.y = A.take(n); S.x2 = A.take(n); S.xk2 = A.take(n); S.fr = A.take(rows * F);
-    S.ff = nullptr; S.stats1 = S.stats2 = nullptr; S.sa = S.ends = nullptr;
+    for (int i = 0; i < (first ? 3 : 4); ++i) {
+      S.hid[i] = A.take(rows * d[i]);
+      if (keep || i == 2) S.lora[i] = A.take(n);           // the gate's alone is read again in the forward
+    }
+    S.w = A.take(n); S.k2 = A.take(n); S.a = A.take(n); S.b = A.take(n);
+    if (!first) S.v2 = A.take(n);
+    S.yw = A.take(n); S.y = A.take(n); S.xk2 = A.take(n); S.fr = A.take(rows * F);
+    if (!last) S.x2 = A.take(n);
     if (keep) {
       S.ff = A.take(rows * F);
       S.stats1 = A.take<float>(2 * rows); S.stats2 = A.take<float>(2 * rows);
       S.sa = A.take(n);
-      if (const size_t e = ends_bytes()) S.ends = A.take<char>(e);
     }
     return S;
   }
@@ -97,7 +103,7 @@ struct Forward {
   size_t wkv_bytes;
   Forward(const Stack& K, Arena& A) {
     const size_t n = K.rows * K.C;
-    one = K.D.saved == nullptr ? K.layer(A, false) : Layer();
+    one = K.D.saved == nullptr ? K.layer(A, false, 0) : Layer();
     v_first = K.D.saved == nullptr ? A.take(n) : nullptr;
     dx = A.take(n);
     const int out = gemm_split((int)K.rows, K.C, K.C), val = gemm_split((int)K.rows, K.F, K.C), most = out > val ? out : val;
@@ -111,16 +117,19 @@ struct Backward {
   bf16_t *gff, *gxk2, *dx2, *dx, *gy, *gyw, *gr1, *gk1, *gv1, *gg, *gr2, *gw, *gk2, *gv2, *ga, *gb, *gs, *gr, *dl[4], *dk, *dv, *dvf,
       *dmix[6], *dh[4];
   float* part;
-  void* wkv;
+  void *wkv, *ends;
   size_t wkv_bytes;
   Backward(const Stack& K, Arena& A) {
     const auto& D = K.D;
     const size_t n = K.rows * K.C;
-    gff = A.take(K.rows * K.F);
-    for (bf16_t** p : {&gxk2, &dx2, &dx, &gy, &gyw, &gr1, &gk1, &gv1, &gg, &gr2, &gw, &gk2, &gv2, &ga, &gb, &gr, &dk, &dv, &dvf}) *p = A.take(n);
+    // gy and gyw come when gff has been read for the last time, the six of dmix when the recurrence's cotangents have
+    gff = A.take(K.rows * K.F > 2 * n + 1024 ? K.rows * K.F : 2 * n + 1024);
+    gy = gff; gyw = gff + (n + 511) / 512 * 512 + 64;
+    for (bf16_t** p : {&gxk2, &dx2, &dx, &gr1, &gk1, &gv1, &gg, &gr2, &gw, &gk2, &gv2, &ga, &gb, &gr, &dk, &dv, &dvf}) *p = A.take(n);
+    bf16_t* const over[6] = {gr2, gw, gk2, gv2, ga, gb};
+    for (int i = 0; i < 6; ++i) dmix[i] = over[i];
     gs = A.take((size_t)D.B * D.H * 4096);
     for (int i = 0; i < 4; ++i) { dl[i] = i == 2 ? gg : A.take(n); dh[i] = A.take(K.rows * K.d[i]); }
-    for (auto& m : dmix) m = A.take(n);
     size_t bytes = hiprwkv_rwkv7_ln_shiftmix_bwd_workspace_bytes(D.B, D.T, D.C, 6);
     for (size_t b : {hiprwkv_rwkv7_ln_shiftmix_bwd_workspace_bytes(D.B, D.T, D.C, 1),
                      hiprwkv_rwkv7_postmix_bwd2_workspace_bytes(D.B * D.T, D.H, 64),
@@ -130,6 +139,7 @@ struct Backward {
     wkv_bytes = K.ends_bytes() ? hiprwkv_wkv7_bwd_ends_workspace_bytes(HIPRWKV_BF16, D.B, D.T, D.H, 64)
                                : hiprwkv_wkv7_bwd_workspace_bytes(D.B, D.T, D.H, 64);
     wkv = A.take<char>(wkv_bytes);
+    ends = K.ends_bytes() ? A.take<char>(K.ends_bytes()) : nullptr;      // in bf16 the recurrence's backward fills it itself
   }
 };
 
@@ -138,9 +148,9 @@ void* to(const void* p, int64_t l, size_t n) { return const_cast<bf16_t*>(of(p, 
 
 }  // namespace
 
-size_t rwkv7_stack_saved(const Rwkv7Stack& D) {
+size_t rwkv7_stack_saved(const Rwkv7Stack& D, int64_t l) {
   Arena A{nullptr};
-  Stack(D).layer(A, true);
+  Stack(D).layer(A, true, l);
   return A.used;
 }
 size_t rwkv7_stack_workspace(const Rwkv7Stack& D, bool backward) {
@@ -181,7 +191,7 @@ int launch_rwkv7_stack_fwd(const Rwkv7Stack& D, hipStream_t stream, hipError_t& 
   };
   for (int64_t l = 0; l < D.L; ++l) {
     Arena own{keep ? static_cast<char*>(D.saved[l]) : nullptr};
-    Layer S = keep ? K.layer(own, true) : W.one;
+    Layer S = keep ? K.layer(own, true, l) : W.one;
     if (l == 0 && keep) v_first = S.v;
     S = at_layer(K, S, l, v_first);
     const void* const mixv[6] = {of(P.x_r, l, C), of(P.x_w, l, C), of(P.x_k, l, C), of(P.x_v, l, C), of(P.x_a, l, C), of(P.x_g, l, C)};
@@ -212,9 +222,9 @@ int launch_rwkv7_stack_fwd(const Rwkv7Stack& D, hipStream_t stream, hipError_t& 
     R.w = S.w; R.k_out = S.k2; R.a_out = S.a; R.b_out = S.b;
     HIPRWKV_TRY(launch_rwkv7_lora_pre(X, stream));
     const size_t states = (size_t)D.B * 64 * C;
-    HIPRWKV_TRY_RC(hiprwkv_wkv7_fwd_ends(stream, HIPRWKV_BF16, HIPRWKV_BF16, D.B, D.T, D.H, 64, S.w, S.r, S.k2, S.v2, S.a, S.b,
+    HIPRWKV_TRY_RC(hiprwkv_wkv7_fwd_parts(stream, HIPRWKV_BF16, HIPRWKV_BF16, D.B, D.T, D.H, 64, S.w, S.r, S.k2, S.v2, S.a, S.b,
                                          of(D.s, l, states), reinterpret_cast<const uint32_t*>(D.length), D.new_starts, S.yw, S.sa,
-                                         to(D.new_s, l, states), S.ends, W.wkv, W.wkv_bytes, (unsigned)D.flags | HIPRWKV_LENGTH_I32));
+                                         to(D.new_s, l, states), W.wkv, W.wkv_bytes, (unsigned)D.flags | HIPRWKV_LENGTH_I32));
     HIPRWKV_TRY(launch_rwkv7_postmix(0, M, D.H, S.yw, S.r, S.k2, S.v2, S.lora[2], of(P.lnx_w, l, C), of(P.lnx_b, l, C), of(P.r_k, l, C),
                                      EPS_X, S.y, stream));
     Products O;
@@ -248,7 +258,7 @@ int launch_rwkv7_stack_bwd(const Rwkv7Stack& D, hipStream_t stream, hipError_t& 
   const bf16_t* v_first;
   {
     Arena first{static_cast<char*>(D.saved[0])};
-    v_first = K.layer(first, true).v;
+    v_first = K.layer(first, true, 0).v;
   }
   auto head = [&](int n_out, const bf16_t* x, float* stats, const void* w, const void* b, int64_t l, int srow, const void* const* mix,
                   bf16_t* const* g, const void* gx, void* out, void* const* dparam) {
@@ -265,7 +275,7 @@ int launch_rwkv7_stack_bwd(const Rwkv7Stack& D, hipStream_t stream, hipError_t& 
   const void *g_x = D.g_xs, *g_dx = D.g_dx;
   for (int64_t l = D.L - 1; l >= 0; --l) {
     Arena own{static_cast<char*>(D.saved[l])};
-    const Layer S = at_layer(K, K.layer(own, true), l, v_first);
+    const Layer S = at_layer(K, K.layer(own, true, l), l, v_first);
     // channel mixing
     {
       Products Q;
@@ -296,7 +306,7 @@ int launch_rwkv7_stack_bwd(const Rwkv7Stack& D, hipStream_t stream, hipError_t& 
     // the recurrence
     HIPRWKV_TRY_RC(hiprwkv_wkv7_bwd_ends(stream, HIPRWKV_BF16, HIPRWKV_BF16, D.B, D.T, D.H, 64, S.w, S.r, S.k2, S.v2, S.a, S.b,
                                          of(D.s, l, states), reinterpret_cast<const uint32_t*>(D.length), D.new_starts, W.gyw, S.sa,
-                                         D.g_s == nullptr ? nullptr : of(D.g_s, l, states), S.ends, W.gw, W.gr2, W.gk2, W.gv2, W.ga,
+                                         D.g_s == nullptr ? nullptr : of(D.g_s, l, states), W.ends, W.gw, W.gr2, W.gk2, W.gv2, W.ga,
                                          W.gb, W.gs, W.wkv, W.wkv_bytes, (unsigned)D.flags | HIPRWKV_LENGTH_I32));
     // gates; the value residual's cotangents of all layers meet in W.dvf and in the first layer's values
     PreArgs R;

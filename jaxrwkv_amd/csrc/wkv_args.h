@@ -209,7 +209,7 @@ size_t rwkv7_decode_workspace(const Rwkv7Decode& D);
 hipError_t launch_rwkv7_decode(const Rwkv7Decode& D, hipStream_t stream);
 
 using Rwkv7Stack = ::hiprwkv_rwkv7_stack_args;
-size_t rwkv7_stack_saved(const Rwkv7Stack& D);
+size_t rwkv7_stack_saved(const Rwkv7Stack& D, int64_t l);
 size_t rwkv7_stack_workspace(const Rwkv7Stack& D, bool backward);
 int launch_rwkv7_stack_fwd(const Rwkv7Stack& D, hipStream_t stream, hipError_t& e);      // an entry point's error, or e
 int launch_rwkv7_stack_bwd(const Rwkv7Stack& D, hipStream_t stream, hipError_t& e);

@@ -158,10 +158,16 @@ def wkv7_fwd(r, w, k, v, a, b, s, length=None, new_starts=None, compat=True, wan
     return _wkv7_fwd(r, w, k, v, a, b, s, length, new_starts, compat, want_sa, force_seq, small_t, debug_flags)[:3]
 
 
+def _wkv7_ends(io, B, T, H, N, device):
+    """Memory that goes along to a backward in parts, None where the sequence runs whole."""
+    nbytes = _lib.load().hiprwkv_wkv7_ends_bytes(_DT[io], B, T, H, N)
+    return _workspace(nbytes, device) if nbytes else None
+
+
 def _wkv7_fwd(r, w, k, v, a, b, s, length=None, new_starts=None, compat=True, want_sa=False, force_seq=False,
               small_t=True, debug_flags=0, want_ends=False):
-    """``wkv7_fwd`` with a fourth result: with ``want_ends`` the states that let the backward run the sequence in parts, where that
-    is of use."""
+    """``wkv7_fwd`` with a fourth result: with ``want_ends`` what lets the backward run the sequence in parts, where that is of use
+    (fp32: filled here; bf16: memory that the backward fills)."""
     lib = _lib.load()
     io = r.dtype
     r, w, k, v, a, b = (_dev(x, io) for x in (r, w, k, v, a, b))
@@ -175,8 +181,7 @@ def _wkv7_fwd(r, w, k, v, a, b, s, length=None, new_starts=None, compat=True, wa
     sa = _empty_phased((B, T, H, N), _SA_DT[io], r.device, _phase(r) + 2) if want_sa else None
     nbytes = 0 if force_seq else lib.hiprwkv_wkv7_fwd_workspace_bytes(_DT[io], B, T, H, N)
     ws = _workspace(nbytes, r.device) if nbytes else None
-    ebytes = lib.hiprwkv_wkv7_ends_bytes(_DT[io], B, T, H, N) if want_sa and want_ends and not force_seq else 0
-    ends = _workspace(ebytes, r.device) if ebytes else None
+    ends = _wkv7_ends(io, B, T, H, N, r.device) if want_sa and want_ends and not force_seq else None
     fn, more = (lib.hiprwkv_wkv7_fwd_parts, ()) if ends is None else (lib.hiprwkv_wkv7_fwd_ends, (_p(ends),))
     rc = fn(_stream(), _DT[io], _DT[s.dtype], B, T, H, N, _p(w), _p(r), _p(k), _p(v), _p(a), _p(b),
             _p(s), _p(length), _p(new_starts), _p(y), _p(sa), _p(new_s), *more, _p(ws), nbytes,
@@ -213,11 +218,11 @@ def wkv7_step(r, w, k, v, a, b, s, new_s, length=None, new_starts=None, compat=T
 
 
 def wkv7_bwd(r, w, k, v, a, b, s, length, new_starts, gy, sa, gs_out=None, compat=True, force_seq=False,
-             debug_flags=0, ends=None):
+             debug_flags=0, ends=None, parts=False):
     """Cotangents (gr, gw, gk, gv, ga, gb, gs) of ``wkv7_fwd`` for cotangents gy of y and gs_out of new_s.
 
     bf16 inputs use the chunked MFMA kernels where they exist unless ``force_seq`` asks for the sequential ones.  ``ends``: the
-    forward's (``_wkv7_fwd``), for the sequences in parts."""
+    forward's (``_wkv7_fwd``), for the sequences in parts; with ``parts`` bf16 inputs need none."""
     lib = _lib.load()
     io = r.dtype
     r, w, k, v, a, b, gy = (_dev(x, io) for x in (r, w, k, v, a, b, gy))
@@ -228,6 +233,8 @@ def wkv7_bwd(r, w, k, v, a, b, s, length, new_starts, gy, sa, gs_out=None, compa
     length, new_starts = _length_ns(length, new_starts, B, T, r.device)
     gw, gr, gk, gv, ga, gb = (_empty_like_phased(r, i) for i in range(1, 7))
     gs = torch.empty_like(s)
+    if parts and ends is None and io == torch.bfloat16 and not force_seq:
+        ends = _wkv7_ends(io, B, T, H, N, r.device)
     if ends is None:
         fn, more, nbytes = lib.hiprwkv_wkv7_bwd, (), lib.hiprwkv_wkv7_bwd_workspace_bytes(B, T, H, N)
     else:
@@ -249,7 +256,7 @@ class _Wkv7(torch.autograd.Function):
     def forward(ctx, r, w, k, v, a, b, s, length, new_starts, compat, force_seq):
         need = any(x.requires_grad for x in (r, w, k, v, a, b, s))
         new_s, y, sa, ends = _wkv7_fwd(r, w, k, v, a, b, s, length, new_starts, compat, want_sa=need, force_seq=force_seq,
-                                       want_ends=need)
+                                       want_ends=need and r.dtype == torch.float32)
         ctx.compat = compat
         ctx.force_seq = force_seq
         ctx.save_for_backward(r, w, k, v, a, b, s, length, new_starts, sa, ends)
@@ -261,7 +268,7 @@ class _Wkv7(torch.autograd.Function):
         if gy is None:
             gy = torch.zeros_like(r)
         gr, gw, gk, gv, ga, gb, gs = wkv7_bwd(r, w, k, v, a, b, s, length, new_starts, gy, sa, gs_out, ctx.compat,
-                                              ctx.force_seq, ends=ends)
+                                              ctx.force_seq, ends=ends, parts=True)
         return gr, gw, gk, gv, ga, gb, gs, None, None, None, None
 
 
