@@ -413,8 +413,8 @@ def _native(params, x, state, grad):
     shapes = {"ffn_key": (L, F, C), "ffn_value": (L, C, F)}
     most = NATIVE_ROWS_C2 if C <= 1536 else NATIVE_ROWS_C2_WIDE
     return (x.dtype == torch.bfloat16 and M * C * C <= most and M <= NATIVE_ROWS and T > 8 and N == 64 and C == H * N
-            and C % 128 == 0 and F <= 8 * C and all(d % 8 == 0 for d in sizes) and state.shape == (B, L, 2 + N, C)
-            and state.is_contiguous() and state.data_ptr() % 16 == 0 and not ops.autocast_elsewhere(x)
+            and C % 128 == 0 and F <= 8 * C and all(d % 8 == 0 and max(d, C) * max(M, C, 256) < 2 ** 30 for d in sizes)
+            and state.shape == (B, L, 2 + N, C) and state.is_contiguous() and state.data_ptr() % 16 == 0 and not ops.autocast_elsewhere(x)
             and all(p[n].shape == shapes.get(n, (L, C, C)) for n in _PRODUCTS)
             and not (grad and (state.requires_grad or not all(t.requires_grad for t in params))))
 

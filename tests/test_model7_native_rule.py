@@ -23,3 +23,9 @@ def test_sizes(B, T, C, native):
     """Where the separate steps' library products were measured faster (2048 channels: 2200 rows forward 11.6 ms against 12.9), or the
     workspace would be large, the call takes them."""
     assert case(B, T, C) == native
+
+
+@pytest.mark.parametrize("B,T,C,d,native", [(1, 9, 128, 2 ** 20, True), (1, 9, 128, 2 ** 22, False), (4, 512, 768, 2 ** 19, False), (1, 9, 128, 12, False)])
+def test_inner_sizes(B, T, C, d, native):
+    """What the native code refuses (operands of 2 GiB, sizes that are no multiple of 8) takes the separate steps."""
+    assert case(B, T, C, d) == native
