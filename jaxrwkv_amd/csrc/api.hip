@@ -889,7 +889,7 @@ int hiprwkv_rwkv7_lora_pre(hiprwkv_stream stream, int io_dtype, int64_t rows, in
   if (int rc = check_pre("rwkv7_lora_pre", io_dtype, N, A, {k, w0, a0, k_k, k_a, out != nullptr ? out[2] : g, w, k_out, a_out, b_out}, {v, v_first, v0, v_out})) return rc;
   if ((rows + 63) / 64 * H > 0x7fffffffLL || rows > 0x7fffffffLL - 64) return fail(HIPRWKV_EINVAL, "rwkv7_lora_pre: too many rows");
   for (int i = 0; i < (v_first != nullptr ? 4 : 3); ++i) {
-    if (d[i] <= 0 || d[i] % 8 != 0 || std::max(rows, H * N) * d[i] >= 0x7fffffffLL)
+    if (d[i] <= 0 || d[i] % 8 != 0 || d[i] > 0x7fffffffLL || std::max(rows, H * N) * d[i] >= 0x7fffffffLL)
       return fail(HIPRWKV_EINVAL, "rwkv7_lora_pre: inner sizes must be positive multiples of 8, arrays below 4 GiB");
     for (const void* p : {hid[i], w2[i]})
       if (p == nullptr || !aligned16(p)) return fail(HIPRWKV_EINVAL, "rwkv7_lora_pre: null or misaligned tensor pointer (16 bytes)");
