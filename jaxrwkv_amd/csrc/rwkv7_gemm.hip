@@ -20,8 +20,8 @@ constexpr int GEMM_WAVES = 8;
 // f of a product, which is rounded to bf16 first, where the separate product would be stored
 __device__ __forceinline__ float rnd(float x) { return bf16_to_f32(f32_to_bf16(x)); }
 // tanh is 1 - 2 / (1 + e^2x) where that keeps its value to 1e-6 (its error is 1e-7 of one whatever x is) and the series below (the
-// next term is 62/2835 x^8).  This code is inlined at every store of every kernel here and its length costs all of them, so tanh
-// and sigmoid share the quotient.
+// next term is 62/2835 x^8).  This code is inlined at every store of the kernels of few rows and its length costs them, so tanh
+// and sigmoid share the quotient; the tiles apply it in one loop (TileOut::write).
 __device__ __forceinline__ float activate(float x, int act) {
   if (act == GEMM_ACT_NONE) return x;
   x = rnd(x);
@@ -296,16 +296,14 @@ __global__ __launch_bounds__(64 * GEMM_WAVES) void head_gemm_kernel(LnMixArgs N,
   }
 }
 
-// 64 x 64 tiles through registers, any K, 64 of it per step through two LDS buffers: a thread carries two 16-byte pieces of either operand, requested two
-// steps ahead, and four workgroups share a CU, so loads, LDS writes and matrix instructions of different workgroups
-// overlap.  An operand that lies k-major (km, kn) goes to LDS as it lies and is read with the transposing load.  Workgroups go
+// 64 x 64 tiles through registers, 64 of K per step through two LDS buffers, for products of a short K alone in their launch (the second
+// low-rank factors of a decode step): a thread carries two 16-byte pieces of either operand, requested two steps ahead, and four
+// workgroups share a CU, so loads, LDS writes and matrix instructions of different workgroups overlap.  An operand that lies k-major (km, kn) goes to LDS as it lies and is read with the transposing load.  Workgroups go
 // to the eight XCDs round-robin; the tiles that share a piece of the longer operand run on one XCD, whose L2 reads it once.
-// Its waves wait half of their time at 4084 rows and three quarters in a decode step (profiles/rwkv7_model_bf16.md): a step moves
-// 16 KiB in, 16 KiB to LDS and 32 KiB from it for 32 matrix instructions.  Weights straight from memory into the matrix operands
-// were slower (a cache line per lane), and so were four steps in flight.  Where one product leaves CUs idle
-// (a decode step's output and value projections: 128 tiles) K is split over gridDim.y and the parts are added by the norm
-// that reads the result.  Low-rank products at 4084 tokens of 2048 channels, through registers: 36 us for the four into the inner
-// sizes (74 with the row tiles of a narrow product on one XCD), 47 us out of them (67 MB written).
+// Its waves wait for 63 % of their time in a decode step of 256 users (profiles/rwkv7_model_bf16.md): a step moves 16 KiB in, 16 KiB to
+// LDS and 32 KiB from it for 32 matrix instructions.  Weights straight from memory into the matrix operands were slower (a cache line
+// per lane), and so were four steps in flight.  Where one product leaves CUs idle K is split over gridDim.y, in these tiles and those
+// below (a decode step's output and value projections: 128 tiles), and the parts are added by the norm that reads the result.
 constexpr int TG = 64, TG_RS = TG + 8;         // tile edge; LDS row stride: 16-byte rows 144 bytes apart
 constexpr int AHEAD = 2;                       // steps whose operands are in flight (four: 212 registers, 1.6 times slower for short K)
 typedef uint16_t TileLds[2][2][TG][TG_RS];     // [buffer][x | w]
@@ -514,14 +512,16 @@ int tiles_of(const GemmJob& J, int tm, int tn) {
 // those of them that work
 int64_t real_tiles(const GemmJob& J, int tm, int tn) { return (int64_t)((J.M + tm - 1) / tm) * ((J.N + tn - 1) / tn); }
 
-// The same tiles with the operands requested straight into LDS, BUFS - 1 steps ahead: no registers are held by what is in
-// flight.  K is a multiple of the step.  A wave's request fills eight rows of 128 bytes as they lie, so rows cannot be padded:
-// 16-byte piece p of row q lies at p ^ swizzle(q) instead (no bank conflicts counted).  Weights that no cache holds, against the
-// tiles through registers: 64 rows of 2048 channels into 8192 columns 19.0 -> 15.3 us, K = 8192 into 2048 unsplit 57.9 -> 37.8;
+// Tiles of 64 or 128 rows and columns with the operands requested straight into LDS, BUFS - 1 steps ahead: no registers are held by what
+// is in flight.  Any K (launch_gemm: from 256 on, multiples of the step, or beside a product of 1024): the last step of one that is no
+// multiple is masked where it is read.  A wave's request fills 1 KiB as it lies, eight rows of 128 bytes or, of a 128-wide k-major
+// operand, four of 256, so rows cannot be padded: 16-byte piece p of row q lies at p ^ swizzle(q) instead (no bank conflicts counted in
+// the loop).  Weights that no cache holds, 64 x 64 tiles against those through registers: 64 rows of 2048 channels into 8192 columns 19.0 -> 15.3 us, K = 8192 into 2048 unsplit 57.9 -> 37.8;
 // 128 rows 19.3 -> 15.4; r, k, v and the low-rank inputs at 128 rows 20.5 -> 16.6; 256 rows into 8192 columns 23.5 -> 22.8 with
-// 64-row tiles, 19.9 with 128.  Bound by the wait for the weights (47 to 55 % of the waves' time in a step of 256 users,
-// profiles/rwkv7_model_bf16.md); five and seven steps in flight took as long, and so did a first step that differs from tile to
-// tile.
+// 64-row tiles, 19.9 with 128.  Bound by a step's way through LDS (see launch_gemm): in a step of 256 users (128 x 64, 17.8 us for 43.7 MB
+// read) the waves wait for half of their time, for arriving operands and each other, an LDS read is why in 1 %, and the matrix units work
+// a fifth of it (profiles/rwkv7_model_bf16.md); five and seven steps in flight took as long, and so did a first step that differs from tile
+// to tile.
 constexpr int stream_step(int tm, int tn) { return (tm + tn) * TG; }     // bf16 values of a step in LDS: TM rows of x, TN of w
 typedef __attribute__((address_space(3))) uint16_t* lds_u16_ptr;
 
@@ -836,17 +836,18 @@ int gemm_split(int M, int64_t K, int64_t N) {
 // 64 cycles a KiB, which a stream of weights can afford but repeated reads of x cannot (8192 columns of 2048: 14 us at 32
 // rows, 16 at 33, 21 at 64; tiled 15 us up to 128 rows, 22 at 256).
 // From 33 rows tiles, straight to LDS (through registers where an operand of a narrow K is no multiple of a step: the second low-rank
-// factors, which the other kernel would mostly mask).  Which: a CU's LDS is the bound (the operands of a step are written at 64 bytes a
-// cycle and read twice at 128: 4 (TM + TN) cycles a step, measured 0.29 us for 64 x 64, 0.40 for 128 x 64, 0.59 for 128 x 128), so the
-// tile that takes the fewest steps a CU times TM + TN.  Products of one K run in rounds over the CUs; of several, the longest or the
-// mean counts and 128 x 128 tiles leave too few to balance.  Weights that no cache holds, us with 64x64, 128x64, 128x128 tiles:
-// 2048 rows: three 768x768 22.2 / 20.2 / 17.9, 768 into 3072 23.1 / 19.2 / 17.4, 3072 into 768 24.0 / 25.5 / 33; with the weights'
-// cotangents: of 768x768 14.0 / 17.0 / 29, of three 41 / 36.6 / 44, of 3072 into 768 43 / 35 / 40.  512 rows: 2048 into 8192 36 / 29 / 25,
-// 8192 into 2048 37 / 52 / 75.  4084 rows: three 2048x2048 225 / 161 / 116.  256 rows of 2048 into 8192: 21 / 18.8 / 24.
-// Empty workgroups of the 128 x 128 tiles do not count: with them, and as edges, 24 layers of 2048 channels fell back to 128 x 64 at
-// 2200 rows, 12.9 ms forward, now 12.0, at 2600 14.6, now 12.8, at 3200 18.7, now 14.8.  Those of the smaller tiles do: 12 layers of 768
-// channels were 1 % slower without them (700 and 1500 rows).  The wait of a step is not it: four steps in flight took as long as three
-// (one workgroup per CU), and so did reading half a step ahead of its products.
+// factors, which the other kernel would mostly mask).  Which: a step takes in proportion to what passes through a CU's LDS (its operands
+// are written at 64 bytes a cycle and read twice at 128: 4 (TM + TN) cycles; measured 0.29 us for 64 x 64, 0.40 for 128 x 64, 0.59 for 128
+// x 128; by the counters the waves wait for what arrives, not for what they read, so the writing half rather), so the tile that takes the
+// fewest steps a CU times TM + TN.  Products of one K run in rounds over the CUs; of several, the longest or the mean counts and 128 x 128
+// tiles leave too few to balance.  Weights that no cache holds, us with 64x64, 128x64, 128x128 tiles: 2048 rows: three 768x768 22.2 / 20.2
+// / 17.9, 768 into 3072 23.1 / 19.2 / 17.4, 3072 into 768 24.0 / 25.5 / 33; with the weights' cotangents: of 768x768 14.0 / 17.0 / 29, of
+// three 41 / 36.6 / 44, of 3072 into 768 43 / 35 / 40.  512 rows: 2048 into 8192 36 / 29 / 25, 8192 into 2048 37 / 52 / 75.  4084 rows:
+// three 2048x2048 225 / 161 / 116.  256 rows of 2048 into 8192: 21 / 18.8 / 24. Empty workgroups of the 128 x 128 tiles do not count: with
+// them, and as edges, 24 layers of 2048 channels fell back to 128 x 64 at 2200 rows, 12.9 ms forward, now 12.0, at 2600 14.6, now 12.8, at
+// 3200 18.7, now 14.8.  Those of the smaller tiles do: 12 layers of 768 channels were 1 % slower without them (700 and 1500 rows).  More
+// requests in flight change nothing: four steps took as long as three (one workgroup per CU), and so did reading half a step ahead of its
+// products.
 constexpr int CUS = 256, WIDE_TILES = 192;
 hipError_t launch_gemm(GemmArgs A, int split, hipStream_t stream) {
   bool skinny = true, stream_k = true, same_k = true;
