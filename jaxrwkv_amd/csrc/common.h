@@ -17,6 +17,29 @@ __device__ __forceinline__ float ld_f(const bf16_t* p) { return bf16_to_f32(p->b
 __device__ __forceinline__ void st_f(float* p, float x) { *p = x; }
 __device__ __forceinline__ void st_f(bf16_t* p, float x) { p->bits = f32_to_bf16(x); }
 
+// x as it is stored in bf16, or in the type T
+__device__ __forceinline__ float rnd(float x) { return bf16_to_f32(f32_to_bf16(x)); }
+template <typename T>
+__device__ __forceinline__ float round_io(float x);
+template <>
+__device__ __forceinline__ float round_io<float>(float x) { return x; }
+template <>
+__device__ __forceinline__ float round_io<bf16_t>(float x) { return rnd(x); }
+
+__device__ __forceinline__ float sigmoidf(float z) { return 1.f / (1.f + __expf(-z)); }
+// softplus(z) = log(1 + e^z) = max(z, 0) + log(1 + e^-|z|): the argument of the logarithm lies in (1, 2], where the
+// hardware logarithm is accurate to a few 1e-7 absolute (log1pf, a software routine, made the kernel of the decay three times slower)
+__device__ __forceinline__ float softplusf(float z) { return fmaxf(z, 0.f) + __logf(1.f + __expf(-fabsf(z))); }
+
+// sum over the 16 lanes of a DPP row, delivered to all of them
+__device__ __forceinline__ float row_sum(float x) {
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x128, 0xf, 0xf, false));   // row_ror:8
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x124, 0xf, 0xf, false));   // row_ror:4
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x122, 0xf, 0xf, false));   // row_ror:2
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x121, 0xf, 0xf, false));   // row_ror:1
+  return x;
+}
+
 // Tokens of sequence b that count: at most T.  FLAG_LENGTH_I32 (HIPRWKV_LENGTH_I32): the array is int32, negative = 0.
 constexpr unsigned FLAG_LENGTH_I32 = 0x40u;
 __device__ __forceinline__ int64_t seq_length(const uint32_t* length, int64_t b, int64_t T, unsigned flags) {

@@ -35,15 +35,6 @@ constexpr int MAX_WAVES = 8;           // 512 threads: C <= 4096, and 256 regist
 template <int NOUT>
 constexpr int BWD_GROUP_OF = NOUT == 6 ? 1 : 2;
 
-// sum over the 16 lanes of a DPP row, delivered to all of them
-__device__ __forceinline__ float row_sum(float x) {
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x128, 0xf, 0xf, false));   // row_ror:8
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x124, 0xf, 0xf, false));   // row_ror:4
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x122, 0xf, 0xf, false));   // row_ror:2
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x121, 0xf, 0xf, false));   // row_ror:1
-  return x;
-}
-
 // G sums over the workgroup at once.  `buf` is not read by anyone when a thread gets here (callers alternate two).
 template <int G>
 __device__ __forceinline__ void block_sum(float (&x)[G], float* buf) {
@@ -63,13 +54,6 @@ __device__ __forceinline__ void block_sum(float (&x)[G], float* buf) {
 #pragma unroll
       for (int j = 0; j < G; ++j) x[j] += buf[(r + q) * G + j];
 }
-
-template <typename T>
-__device__ __forceinline__ float round_io(float x);
-template <>
-__device__ __forceinline__ float round_io<float>(float x) { return x; }
-template <>
-__device__ __forceinline__ float round_io<bf16_t>(float x) { return bf16_to_f32(f32_to_bf16(x)); }
 
 template <typename T>
 __device__ __forceinline__ void zero_or_ld8(const T* p, bool take, float (&o)[8]) {

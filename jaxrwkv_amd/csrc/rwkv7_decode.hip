@@ -23,10 +23,6 @@ namespace hiprwkv {
 namespace {
 
 // ---------------------------------------------------------------------------------------------------------------
-__device__ __forceinline__ float sigmoidf(float z) { return 1.f / (1.f + __expf(-z)); }
-__device__ __forceinline__ float softplusf(float z) { return fmaxf(z, 0.f) + __logf(1.f + __expf(-fabsf(z))); }
-__device__ __forceinline__ float rnd(float x) { return bf16_to_f32(f32_to_bf16(x)); }
-
 // sum over the wave, delivered to every lane
 __device__ __forceinline__ float wave_sum(float x) {
 #pragma unroll

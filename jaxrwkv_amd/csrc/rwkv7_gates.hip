@@ -23,11 +23,6 @@ namespace {
 
 constexpr int GATE_THREADS = 256;
 
-__device__ __forceinline__ float sigmoidf(float z) { return 1.f / (1.f + __expf(-z)); }
-// softplus(z) = log(1 + e^z) = max(z, 0) + log(1 + e^-|z|): the argument of the logarithm lies in (1, 2], where the
-// hardware logarithm is accurate to a few 1e-7 absolute (log1pf, a software routine, made this kernel three times slower)
-__device__ __forceinline__ float softplusf(float z) { return fmaxf(z, 0.f) + __logf(1.f + __expf(-fabsf(z))); }
-
 template <typename T, bool SIGMOID>   // SIGMOID: the gate a = sigmoid(a0 + x) instead of the decay
 __global__ __launch_bounds__(GATE_THREADS) void rwkv7_decay_kernel(int64_t rows, int64_t C, const T* __restrict__ x,
                                                                     const T* __restrict__ w0, T* __restrict__ w) {

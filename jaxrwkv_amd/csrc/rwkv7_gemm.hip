@@ -18,7 +18,6 @@ using chunk::mfma;
 constexpr int GEMM_WAVES = 8;
 
 // f of a product, which is rounded to bf16 first, where the separate product would be stored
-__device__ __forceinline__ float rnd(float x) { return bf16_to_f32(f32_to_bf16(x)); }
 // tanh is 1 - 2 / (1 + e^2x) where that keeps its value to 1e-6 (its error is 1e-7 of one whatever x is) and the series below (the
 // next term is 62/2835 x^8).  This code is inlined at every store of the kernels of few rows and its length costs them, so tanh
 // and sigmoid share the quotient; the tiles apply it in one loop (TileOut::write).
@@ -130,15 +129,6 @@ __global__ __launch_bounds__(64 * GEMM_WAVES) void skinny_gemm_kernel(GemmArgs A
       *reinterpret_cast<uint2*>(static_cast<bf16_t*>(J.out) + (size_t)m * J.N + n0 + 4 * g) = o;
     }
   }
-}
-
-// sum over the 16 lanes of a DPP row, delivered to all of them
-__device__ __forceinline__ float row_sum(float x) {
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x128, 0xf, 0xf, false));   // row_ror:8
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x124, 0xf, 0xf, false));   // row_ror:4
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x122, 0xf, 0xf, false));   // row_ror:2
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x121, 0xf, 0xf, false));   // row_ror:1
-  return x;
 }
 
 // What ln_shiftmix_kernel and the product above do, in one launch for one or two rows (a decode step of few users).  There a launch of

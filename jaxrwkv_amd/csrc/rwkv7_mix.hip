@@ -19,15 +19,6 @@ namespace hiprwkv {
 
 namespace {
 
-// sum over the 16 lanes of a DPP row, delivered to all of them
-__device__ __forceinline__ float row_sum(float x) {
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x128, 0xf, 0xf, false));   // row_ror:8
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x124, 0xf, 0xf, false));   // row_ror:4
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x122, 0xf, 0xf, false));   // row_ror:2
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x121, 0xf, 0xf, false));   // row_ror:1
-  return x;
-}
-
 // four consecutive elements <-> four floats (pointer 8-byte aligned for bf16, 16 for fp32)
 __device__ __forceinline__ void ld4(const float* p, float (&o)[4]) {
   const float4 x = *reinterpret_cast<const float4*>(p);

@@ -8,16 +8,6 @@ namespace hiprwkv {
 
 namespace {
 
-__device__ __forceinline__ float sigmoidf(float z) { return 1.f / (1.f + __expf(-z)); }
-__device__ __forceinline__ float softplusf(float z) { return fmaxf(z, 0.f) + __logf(1.f + __expf(-fabsf(z))); }
-
-template <typename T>
-__device__ __forceinline__ float round_io(float x);
-template <>
-__device__ __forceinline__ float round_io<float>(float x) { return x; }
-template <>
-__device__ __forceinline__ float round_io<bf16_t>(float x) { return bf16_to_f32(f32_to_bf16(x)); }
-
 // sum over the 8 lanes of half a DPP row, delivered to all of them
 __device__ __forceinline__ float oct_sum(float x) {
   x = quad_sum(x);
