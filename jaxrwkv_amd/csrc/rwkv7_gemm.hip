@@ -17,7 +17,7 @@ using chunk::mfma;
 
 constexpr int GEMM_WAVES = 8;
 
-// f of a product, which is rounded to bf16 first, where the separate product would be stored
+// f of a product, which is rounded to bf16 first, where the separate product would be stored.
 // tanh is 1 - 2 / (1 + e^2x) where that keeps its value to 1e-6 (its error is 1e-7 of one whatever x is) and the series below (the
 // next term is 62/2835 x^8).  This code is inlined at every store of the kernels of few rows and its length costs them, so tanh
 // and sigmoid share the quotient; the tiles apply it in one loop (TileOut::write).
