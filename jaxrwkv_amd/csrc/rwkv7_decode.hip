@@ -9,10 +9,9 @@
 //     6  residual addition, norm, shift and interpolation                     (rwkv7_block.hip)
 //     7  key projection with relu(.)^2                                        rwkv7_gemm.hip
 //     8  value projection                                                     rwkv7_gemm.hip
-// Measured (eager, host included), general path -> separate launches -> now: 12 layers of 768 channels, one user 5.4 ms -> 0.57 -> 0.41
-// a step, two 0.43, 16 0.61 -> 0.54; 24 layers of 2048 channels, one user 1.61 -> 1.36, 16 1.89 -> 1.69, 256 10.9 -> 3.6 -> 3.2 (7.5
-// with the weight-streaming product alone: 51 us a launch at 256 rows, 18 tiled).  Norms inside the products: one user 0.50 -> 0.42 (12 x
-// 768), three as long as before; second low-rank products inside the recurrence 0.42 -> 0.41.
+// Measured (eager, host included), with the general path's operations, with a launch for each line above, and now: 12 layers of 768 channels, one
+// user 5.4 ms, 0.57, 0.32 a step, 16 users -, 0.61, 0.50; 24 layers of 2048 channels, one user -, 1.61, 1.21, 16 -, 1.89, 1.66, 256 10.9, 3.6, 3.1.
+// Norms inside the products: three users as long as with norms of their own, two 0.50 -> 0.42 ms (12 x 768; 0.32 now).
 // References: /root/reference/src/jaxrwkv/rwkv7.py:190-198, :223-267, :269-291.  Products accumulate in fp32 and are rounded
 // once; the values between the gates, the recurrence and the group norm are rounded where the general path stores them.
 #include "chunk_common.h"
@@ -23,18 +22,18 @@ namespace hiprwkv {
 namespace {
 
 // ---------------------------------------------------------------------------------------------------------------
-// sum over the wave, delivered to every lane
+// Sum over the wave, delivered to every lane: rows of 16 lanes by DPP, the four rows through scalar registers.  Every lane of the wave takes
+// part.  (Six __shfl_xor are six trips through LDS in series, about 100 cycles each; a step's four sums were a sixth of the kernel below.)
 __device__ __forceinline__ float wave_sum(float x) {
-#pragma unroll
-  for (int o = 32; o; o >>= 1) x += __shfl_xor(x, o, 64);
-  return x;
+  const int v = __float_as_int(row_sum(x));
+  const float a = __int_as_float(__builtin_amdgcn_readlane(v, 0)) + __int_as_float(__builtin_amdgcn_readlane(v, 16));
+  const float b = __int_as_float(__builtin_amdgcn_readlane(v, 32)) + __int_as_float(__builtin_amdgcn_readlane(v, 48));
+  return a + b;
 }
 
 struct CoreArgs {
   int64_t T, H;
   const bf16_t *r, *k, *v, *vf, *xw, *xa, *xv, *g;          // (B,T,H,64); vf null: the first layer
-  const bf16_t *hid[4], *w2[4];   // or the factors of xw, xa, g, xv: (B,T,d) and (d,H,64), d a multiple of 32
-  int d[4];
   const bf16_t *w0, *a0, *v0, *k_k, *k_a, *ln_w, *ln_b, *r_k;   // (H,64)
   float eps;
   const bf16_t* s;             // states: H*64*64 elements per sequence, bstride apart
@@ -46,20 +45,18 @@ struct CoreArgs {
   bf16_t* y;
 };
 
-// One workgroup per (sequence, head); thread (row i = tid/4, quarter q = tid%4) holds 16 elements of state row i, as in
-// the small-T kernel of the op, whose state traffic (2 x 8 KB per head) is the bound.  The state is requested first; wave 0
-// (one lane per channel) meanwhile turns the projections into the op's inputs and hands them over through LDS, and takes
-// y back through LDS for the group norm, the bonus and the gate.  B=256 H=32: the state alone is 134 MB each way.
-// LORA: the second low-rank products are made here, each workgroup its head's 64 columns (one launch less, but their weights are read
-// once per sequence).  Eight lanes read a row of a factor, a wave eight rows, the requests of 128 rows of all four together.
-template <bool LORA>
-__global__ __launch_bounds__(256, LORA ? 1 : 6) void decode_core_kernel(CoreArgs A) {
-  __shared__ __align__(16) float lora[LORA ? 16 : 1][4][64];      // [wave, 16 of its lanes][factor][channel]; then lora[0] the results
-  __shared__ float ch[5][64];            // d, k', a_i, b_i, r
+// One workgroup per (head, sequence); thread (row i = tid/4, quarter q = tid%4) holds 16 elements of state row i, as in
+// the small-T kernel of the op, whose state traffic (2 x 8 KB per head) is the bound.  The state is requested first; waves 0 and 1
+// (one lane per channel) meanwhile turn the projections into the op's inputs and hand them over through LDS, wave 0 takes
+// y back through LDS for the group norm, the bonus and the gate.  B=256 H=32: the state alone is 67 MB each way; 38.5 us a launch with one
+// wave for all of that and its sums through LDS, 34.6 now (3.9 TB/s): a workgroup's chain of dependent steps, six workgroups a CU.
+__global__ __launch_bounds__(256, 6) void decode_core_kernel(CoreArgs A) {
+  __shared__ __align__(16) float ch[5][64];            // d, k', a_i, b_i, r
   __shared__ float vs[64], ys[64];
-  const int64_t b = blockIdx.x / A.H, h = blockIdx.x % A.H;
+  const int64_t b = blockIdx.y, h = blockIdx.x;
   const int tid = threadIdx.x, i = tid >> 2, q = tid & 3, c0 = 16 * q;
-  const bool lead = tid < 64;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const bool keys = wave == 0, values = wave == 1;     // which part of the op's inputs a wave makes
   int64_t L = A.T;
   if (A.length != nullptr) { L = A.length[b]; L = L < 0 ? 0 : L < A.T ? L : A.T; }
   const bool compat = (A.flags & 1u) != 0;
@@ -76,88 +73,40 @@ __global__ __launch_bounds__(256, LORA ? 1 : 6) void decode_core_kernel(CoreArgs
     st8(A.new_s + sel + 8, hi);
   };
   if (L == 0) put_state();
-  const size_t cel = (size_t)h * 64 + tid;
+  const size_t cel = (size_t)h * 64 + lane;
   float w0 = 0.f, a0 = 0.f, v0 = 0.f, k_k = 0.f, k_a = 0.f, ln_w = 0.f, ln_b = 0.f, r_k = 0.f;
-  if (lead) {
-    w0 = ld_f(A.w0 + cel); a0 = ld_f(A.a0 + cel); k_k = ld_f(A.k_k + cel); k_a = ld_f(A.k_a + cel);
+  if (keys) {
+    a0 = ld_f(A.a0 + cel); k_k = ld_f(A.k_k + cel); k_a = ld_f(A.k_a + cel);
     ln_w = ld_f(A.ln_w + cel); ln_b = ld_f(A.ln_b + cel); r_k = ld_f(A.r_k + cel);
+  } else if (values) {
+    w0 = ld_f(A.w0 + cel);
     if (A.vf != nullptr) v0 = ld_f(A.v0 + cel);
   }
   for (int64_t t = 0; t < A.T; ++t) {
     float v = 0.f, gate = 0.f, bonus = 0.f, k = 0.f, r = 0.f, vf = 0.f, xw = 0.f, xa = 0.f, xv = 0.f;
-    const size_t el = (((size_t)b * A.T + t) * A.H + h) * 64 + tid;
-    if (lead) {
-      k = ld_f(A.k + el); r = ld_f(A.r + el); v = ld_f(A.v + el);
-      if (A.vf != nullptr) vf = ld_f(A.vf + el);
-      if (!LORA) {
-        xw = ld_f(A.xw + el); xa = ld_f(A.xa + el); gate = ld_f(A.g + el);
-        if (A.vf != nullptr) xv = ld_f(A.xv + el);
-      }
+    const size_t el = (((size_t)b * A.T + t) * A.H + h) * 64 + lane;
+    if (keys) {
+      k = ld_f(A.k + el); r = ld_f(A.r + el);
+      xa = ld_f(A.xa + el); gate = ld_f(A.g + el);
+    } else if (values) {
+      v = ld_f(A.v + el); xw = ld_f(A.xw + el);
+      if (A.vf != nullptr) { vf = ld_f(A.vf + el); xv = ld_f(A.xv + el); }
     }
-    if (LORA) {
-      const int wave = tid >> 6, lane = tid & 63, first = 8 * wave + (lane >> 3), c8 = 8 * (lane & 7);
-      const size_t row = (size_t)b * A.T + t;
-      float acc[4][8];
-#pragma unroll
-      for (int f = 0; f < 4; ++f)
-#pragma unroll
-        for (int c = 0; c < 8; ++c) acc[f][c] = 0.f;
-      for (int j0 = 0; j0 < A.d[0] || j0 < A.d[1] || j0 < A.d[2] || j0 < A.d[3]; j0 += 128) {
-        uint4 w[4][4];
-        float x[4][4];
-#pragma unroll
-        for (int f = 0; f < 4; ++f)
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int j = j0 + 32 * u + first, jj = j < A.d[f] ? j : A.d[f] - 1;      // no factor (d = 0): that of the decay, unused
-            w[f][u] = *reinterpret_cast<const uint4*>(A.w2[f] + ((size_t)(jj < 0 ? 0 : jj) * A.H + h) * 64 + c8);
-            x[f][u] = ld_f(A.hid[f] + row * A.d[f] + (jj < 0 ? 0 : jj));
-          }
-#pragma unroll
-        for (int f = 0; f < 4; ++f)
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            // beyond the factor the last row is read again: both are cleared, either may not be finite
-            const uint32_t have = j0 + 32 * u < A.d[f] ? 0xffffffffu : 0u;
-            const float xs = __uint_as_float(__float_as_uint(x[f][u]) & have);
-            const uint32_t q[4] = {w[f][u].x & have, w[f][u].y & have, w[f][u].z & have, w[f][u].w & have};
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-              acc[f][2 * c] = fmaf(xs, __uint_as_float(q[c] << 16), acc[f][2 * c]);
-              acc[f][2 * c + 1] = fmaf(xs, __uint_as_float(q[c] & 0xffff0000u), acc[f][2 * c + 1]);
-            }
-          }
-      }
-#pragma unroll
-      for (int f = 0; f < 4; ++f) {
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-          acc[f][c] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc[f][c]), 0x128, 0xf, 0xf, false));   // row_ror:8
-        if ((lane & 8) == 0) st8(&lora[tid >> 4][f][c8], acc[f]);
-      }
-      __syncthreads();
-      float s = 0.f;
-#pragma unroll
-      for (int u = 0; u < 16; ++u) s += lora[u][wave][lane];
-      __syncthreads();
-      lora[0][wave][lane] = rnd(s);
-      __syncthreads();
-      if (lead) { xw = lora[0][0][tid]; xa = lora[0][1][tid]; gate = lora[0][2][tid]; xv = lora[0][3][tid]; }
-    }
-    if (lead) {
-      if (A.vf != nullptr) v = rnd(fmaf(vf - v, sigmoidf(v0 + xv), v));
+    if (keys) {
       const float a = rnd(sigmoidf(a0 + xa));
-      const float w = rnd(-softplusf(-(w0 + xw)) - 0.5f);
       float kk = k * k_k;
       kk *= 1.f / fmaxf(sqrtf(wave_sum(kk * kk)), 1e-12f);
       const float kp = rnd(k * (1.f + (a - 1.f) * k_a));
       bonus = wave_sum(r * kp * r_k);
-      ch[0][tid] = __expf(-__expf(w));
-      ch[1][tid] = kp;
-      ch[2][tid] = rnd(-kk);
-      ch[3][tid] = rnd(kk * a);
-      ch[4][tid] = r;
-      vs[tid] = v;
+      ch[1][lane] = kp;
+      ch[2][lane] = rnd(-kk);
+      ch[3][lane] = rnd(kk * a);
+      ch[4][lane] = r;
+    } else if (values) {
+      if (A.vf != nullptr) v = rnd(fmaf(vf - v, sigmoidf(v0 + xv), v));
+      const float w = rnd(-softplusf(-(w0 + xw)) - 0.5f);
+      ch[0][lane] = __expf(-__expf(w));
+      vs[lane] = v;
     }
     __syncthreads();
     if (ns != nullptr && ns[t]) {
@@ -168,6 +117,7 @@ __global__ __launch_bounds__(256, LORA ? 1 : 6) void decode_core_kernel(CoreArgs
 #pragma unroll
     for (int c = 0; c < 16; ++c) p = fmaf(S[c], ch[2][c0 + c], p);
     const float sa = quad_sum(p), vi = vs[i];
+    if (keys) v = vs[lane];                            // before wave 1 writes the next token's
     float y = 0.f;
 #pragma unroll
     for (int c = 0; c < 16; ++c) {
@@ -179,13 +129,154 @@ __global__ __launch_bounds__(256, LORA ? 1 : 6) void decode_core_kernel(CoreArgs
     if (q == 0) ys[i] = rnd(y);
     if (t == L - 1) put_state();
     __syncthreads();
-    if (lead) {
-      const float yv = ys[tid];
+    if (keys) {
+      const float yv = ys[lane];
       const float d = yv - wave_sum(yv) * (1.f / 64.f);
       const float rstd = rsqrtf(wave_sum(d * d) * (1.f / 64.f) + A.eps);
       st_f(A.y + el, (d * rstd * ln_w + ln_b + bonus * v) * gate);
     }
   }
+}
+
+// The same for one or two tokens in all (a decode step of few users), where a workgroup's time is a chain of instructions and latencies
+// and CUs stand idle: sixteen waves, four elements of the state a lane, the op's inputs made by four waves, and the second low-rank
+// products here as well (one launch less; their weights are read once per sequence).  Eight lanes read a row of a factor; four waves take a
+// factor, and the wave that needs a product adds their parts.  What a wave reads is named by a table in the arguments: as conditions in the
+// code every choice became a branch that waited for its own loads.  768 channels, one user: 8.1 us a launch with four waves, 5.8 now.
+struct FewArgs {
+  int64_t T, H;
+  const bf16_t* par[4][4];     // (H,64) parameters of waves 0 to 3: a0 k_k ln_w ln_b | a0 k_a r_k | w0 | v0
+  const bf16_t* tok[4][2];     // (B,T,H,64): k | k r | | v v_first
+  const bf16_t *hid[4], *w2[4];   // the factors of xw, xa, g, xv: (B,T,d) and (d,H,64), d a multiple of 32 or 0 (none)
+  int d[4];
+  const bf16_t* s;
+  bf16_t* new_s;
+  int64_t bstride;
+  const int32_t* length;
+  const uint8_t* ns;
+  bf16_t* y;
+  float eps;
+  unsigned flags;
+  int vmix;                    // there is a value residual
+};
+__global__ __launch_bounds__(1024) void decode_few_kernel(FewArgs A) {
+  __shared__ __align__(16) float lora[16][4][64];                 // [wave][16 of its lanes][channel]
+  __shared__ __align__(16) float ch[5][64];                       // d, k', a_i, b_i, r
+  __shared__ float vs[64], ys[64], gs[64], bonus_s;
+  const int64_t b = blockIdx.y, h = blockIdx.x;
+  const int tid = threadIdx.x, i = tid >> 4, c0 = 4 * (tid & 15);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, q = wave & 3, f = wave >> 2;
+  const int d = A.d[f];
+  const size_t sel = (size_t)b * A.bstride + ((size_t)h * 64 + i) * 64 + c0, cel = (size_t)h * 64 + lane;
+  uint2 s4 = *reinterpret_cast<const uint2*>(A.s + sel);
+  uint32_t pv[4];                                                 // as they lie: a conversion would wait for them
+#pragma unroll
+  for (int z = 0; z < 4; ++z) pv[z] = A.par[q][z][cel].bits;
+  int64_t L = A.T;
+  if (A.length != nullptr) { L = A.length[b]; L = L < 0 ? 0 : L < A.T ? L : A.T; }
+  const bool compat = (A.flags & 1u) != 0;
+  const uint8_t* ns = A.ns ? A.ns + b * A.T : nullptr;
+  const bool q2drop = compat && L < A.T && ns != nullptr && ns[L] != 0;
+  float S[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int64_t t = 0; t < A.T; ++t) {
+    const size_t row = (size_t)b * A.T + t, el = (row * A.H + h) * 64 + lane;
+    uint32_t u0v = A.tok[q][0][el].bits, u1v = A.tok[q][1][el].bits;
+    {
+      const int first = 8 * q + (lane >> 3), c8 = 8 * (lane & 7);
+      const bf16_t *hid = A.hid[f] + row * d + first, *w2 = A.w2[f] + ((size_t)first * A.H + h) * 64 + c8;
+      const size_t stride = (size_t)32 * 64 * A.H;
+      float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      for (int j0 = 0; j0 < d; j0 += 128) {
+        uint4 w[4];
+        uint32_t x[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int uu = j0 + 32 * u < d ? u : 0;                // beyond the factor: read again, not used
+          w[u] = *reinterpret_cast<const uint4*>(w2 + uu * stride);
+          x[u] = hid[32 * uu].bits;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (j0 + 32 * u < d) {
+            const uint32_t q4[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
+            const float xu = __uint_as_float(x[u] << 16);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+              acc[2 * c] = fmaf(xu, __uint_as_float(q4[c] << 16), acc[2 * c]);
+              acc[2 * c + 1] = fmaf(xu, __uint_as_float(q4[c] & 0xffff0000u), acc[2 * c + 1]);
+            }
+          }
+        hid += 128;
+        w2 += 4 * stride;
+      }
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+        acc[c] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc[c]), 0x128, 0xf, 0xf, false));   // row_ror:8
+      if ((lane & 8) == 0) st8(&lora[wave][lane >> 4][c8], acc);
+    }
+    __syncthreads();
+    asm volatile("" : "+v"(u0v), "+v"(u1v), "+v"(pv[0]), "+v"(pv[1]), "+v"(pv[2]), "+v"(pv[3]));      // conversions stay behind the barrier
+    const float p0 = __uint_as_float(pv[0] << 16), p1 = __uint_as_float(pv[1] << 16), p2 = __uint_as_float(pv[2] << 16), p3 = __uint_as_float(pv[3] << 16);
+    const float u0 = __uint_as_float(u0v << 16), u1 = __uint_as_float(u1v << 16);
+    auto low = [&](int of) {
+      float s = 0.f;
+#pragma unroll
+      for (int u = 0; u < 16; ++u) s += lora[4 * of + (u >> 2)][u & 3][lane];
+      return rnd(s);
+    };
+    if (wave == 0) {
+      float kk = u0 * p1;
+      kk *= 1.f / fmaxf(sqrtf(wave_sum(kk * kk)), 1e-12f);
+      const float a = rnd(sigmoidf(p0 + low(1)));
+      ch[2][lane] = rnd(-kk);
+      ch[3][lane] = rnd(kk * a);
+    } else if (wave == 1) {
+      const float a = rnd(sigmoidf(p0 + low(1)));
+      const float kp = rnd(u0 * (1.f + (a - 1.f) * p1));
+      ch[1][lane] = kp;
+      ch[4][lane] = u1;
+      bonus_s = wave_sum(u1 * kp * p2);                           // every lane the same
+    } else if (wave == 2) {
+      const float w = rnd(-softplusf(-(p0 + low(0))) - 0.5f);
+      ch[0][lane] = __expf(-__expf(w));
+    } else if (wave == 3) {
+      vs[lane] = A.vmix ? rnd(fmaf(u1 - u0, sigmoidf(p0 + low(3)), u0)) : u0;
+    } else if (wave == 4) {
+      gs[lane] = low(2);
+    }
+    __syncthreads();
+    if (t == 0) {
+      asm volatile("" : "+v"(s4.x), "+v"(s4.y));
+      S[0] = __uint_as_float(s4.x << 16); S[1] = __uint_as_float(s4.x & 0xffff0000u);
+      S[2] = __uint_as_float(s4.y << 16); S[3] = __uint_as_float(s4.y & 0xffff0000u);
+    }
+    if (ns != nullptr && ns[t]) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) S[c] = 0.f;
+    }
+    float p = 0.f;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) p = fmaf(S[c], ch[2][c0 + c], p);
+    const float sa = row_sum(p), vi = vs[i];
+    float y = 0.f;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      S[c] = fmaf(S[c], ch[0][c0 + c], fmaf(vi, ch[1][c0 + c], sa * ch[3][c0 + c]));
+      y = fmaf(S[c], ch[4][c0 + c], y);
+    }
+    y = row_sum(y);
+    if (compat && t + 1 < A.T && ns != nullptr && ns[t + 1]) y = 0.f;
+    if ((tid & 15) == 0) ys[i] = rnd(y);
+    if (t == L - 1) s4 = make_uint2(chunk::pack_rn(S[0], S[1]), chunk::pack_rn(S[2], S[3]));
+    __syncthreads();
+    if (wave == 0) {                                              // the others wait at the next token's first barrier
+      const float yv = ys[lane];
+      const float dv = yv - wave_sum(yv) * (1.f / 64.f);
+      const float rstd = rsqrtf(wave_sum(dv * dv) * (1.f / 64.f) + A.eps);
+      st_f(A.y + el, (dv * rstd * p2 + p3 + bonus_s * vs[lane]) * gs[lane]);
+    }
+  }
+  *reinterpret_cast<uint2*>(A.new_s + sel) = q2drop ? make_uint2(0u, 0u) : s4;      // L = 0: the state itself
 }
 
 }  // namespace
@@ -272,17 +363,32 @@ hipError_t launch_rwkv7_decode(const Rwkv7Decode& D, hipStream_t stream) {
     add(mix[4], layer(D.a1, l, C * D.d_aaa), ha, C, D.d_aaa, 1, GEMM_ACT_NONE);
     add(mix[5], layer(D.g1, l, C * D.d_gate), hg, C, D.d_gate, 1, GEMM_ACT_SIGMOID);
     if (l) add(mix[3], layer(D.v1, l, C * D.d_mv), hv, C, D.d_mv, 1, GEMM_ACT_NONE);
-    CoreArgs A;
-    memset(&A, 0, sizeof(A));
+    const dim3 heads((unsigned)D.H, (unsigned)D.B);
+    const bf16_t *const w0 = layer(D.w0, l, C), *const a0 = layer(D.a0, l, C), *const v0 = layer(D.v0, l, C), *const k_k = layer(D.k_k, l, C),
+                 *const k_a = layer(D.k_a, l, C), *const r_k = layer(D.r_k, l, C), *const ln_w = layer(D.lnx_w, l, C), *const ln_b = layer(D.lnx_b, l, C);
+    const bf16_t* const s = st + (size_t)l * row_state + 2 * C;
+    bf16_t* const new_s = nst + (size_t)l * row_state + 2 * C;
     if (few) {
       const int of_mix[7] = {0, 2, 3, 1, 4, 5, 3};
       for (int i = 0; i < G.n_jobs; ++i) G.job[i].aux = mv[of_mix[i]];
       HIPRWKV_TRY(launch_head_gemm(ln1, G, stream));
+      FewArgs A = {};
       const bf16_t* const second[4] = {layer(D.w2, l, C * D.d_decay), layer(D.a2, l, C * D.d_aaa), layer(D.g2, l, C * D.d_gate),
                                        layer(l ? D.v2 : D.w2, l, C * D.d_mv)};
       const bf16_t* const first[4] = {hw, ha, hg, l ? hv : hw};
       const int64_t d[4] = {D.d_decay, D.d_aaa, D.d_gate, l ? D.d_mv : 0};
-      for (int i = 0; i < 4; ++i) { A.hid[i] = first[i]; A.w2[i] = second[i]; A.d[i] = (int)d[i]; }
+      const bf16_t* const par[4][4] = {{a0, k_k, ln_w, ln_b}, {a0, k_a, r_k, r_k}, {w0, w0, w0, w0}, {l ? v0 : w0, w0, w0, w0}};
+      const bf16_t* const tok[4][2] = {{k, k}, {k, r}, {k, k}, {vl, l ? vf : vl}};
+      for (int i = 0; i < 4; ++i) {
+        A.hid[i] = first[i]; A.w2[i] = second[i]; A.d[i] = (int)d[i];
+        for (int z = 0; z < 4; ++z) A.par[i][z] = par[i][z];
+        for (int z = 0; z < 2; ++z) A.tok[i][z] = tok[i][z];
+      }
+      A.T = D.T; A.H = D.H; A.eps = 64e-5f; A.vmix = l > 0;
+      A.s = s; A.new_s = new_s; A.bstride = seq_state;
+      A.length = D.length; A.ns = D.new_starts; A.flags = (unsigned)D.flags; A.y = y;
+      hipLaunchKernelGGL(decode_few_kernel, heads, dim3(1024), 0, stream, A);
+      HIPRWKV_TRY(hipGetLastError());
     } else {
       HIPRWKV_TRY(launch_gemm(G, 1, stream));
       G.n_jobs = 0;
@@ -291,17 +397,15 @@ hipError_t launch_rwkv7_decode(const Rwkv7Decode& D, hipStream_t stream) {
       add(hg, layer(D.g2, l, C * D.d_gate), g, D.d_gate, C, 1, GEMM_ACT_NONE);
       if (l) add(hv, layer(D.v2, l, C * D.d_mv), xv, D.d_mv, C, 1, GEMM_ACT_NONE);
       HIPRWKV_TRY(launch_gemm(G, 1, stream));
+      CoreArgs A = {};
+      A.T = D.T; A.H = D.H;
+      A.r = r; A.k = k; A.v = vl; A.vf = l ? vf : nullptr; A.xw = xw; A.xa = xa; A.xv = xv; A.g = g;
+      A.w0 = w0; A.a0 = a0; A.v0 = v0; A.k_k = k_k; A.k_a = k_a; A.r_k = r_k; A.ln_w = ln_w; A.ln_b = ln_b; A.eps = 64e-5f;
+      A.s = s; A.new_s = new_s; A.bstride = seq_state;
+      A.length = D.length; A.ns = D.new_starts; A.flags = (unsigned)D.flags; A.y = y;
+      hipLaunchKernelGGL(decode_core_kernel, heads, dim3(256), 0, stream, A);
+      HIPRWKV_TRY(hipGetLastError());
     }
-    A.T = D.T; A.H = D.H;
-    A.r = r; A.k = k; A.v = vl; A.vf = l ? vf : nullptr; A.xw = xw; A.xa = xa; A.xv = xv; A.g = g;
-    A.w0 = layer(D.w0, l, C); A.a0 = layer(D.a0, l, C); A.v0 = layer(D.v0, l, C);
-    A.k_k = layer(D.k_k, l, C); A.k_a = layer(D.k_a, l, C); A.r_k = layer(D.r_k, l, C);
-    A.ln_w = layer(D.lnx_w, l, C); A.ln_b = layer(D.lnx_b, l, C); A.eps = 64e-5f;
-    A.s = st + (size_t)l * row_state + 2 * C; A.new_s = nst + (size_t)l * row_state + 2 * C; A.bstride = seq_state;
-    A.length = D.length; A.ns = D.new_starts; A.flags = (unsigned)D.flags; A.y = y;
-    if (few) hipLaunchKernelGGL(decode_core_kernel<true>, dim3((unsigned)(D.B * D.H)), dim3(256), 0, stream, A);
-    else hipLaunchKernelGGL(decode_core_kernel<false>, dim3((unsigned)(D.B * D.H)), dim3(256), 0, stream, A);
-    HIPRWKV_TRY(hipGetLastError());
     G.n_jobs = 0;
     add(y, layer(D.output, l, C * C), dx, C, C, 0, GEMM_ACT_NONE);
     n_part = split_out;
