@@ -7,6 +7,8 @@
 #include "rwkv7_pre.h"
 #include "wkv_args.h"
 
+#include <type_traits>
+
 namespace hiprwkv {
 
 namespace {
@@ -54,21 +56,48 @@ int place_jobs(GemmArgs& A, F&& tiles_of_job) {
   return tiles;
 }
 
+__device__ __forceinline__ uint2 lds_tr4(const uint16_t* p) {      // see wkv7_fwd.hip
+  typedef short s16x4_t __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4_t* lds_ptr;
+  return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p)));
+}
+
+// Sixteen columns of a KN weight (the low-rank factors) by 32 of k for one wave: two lanes read a row, and the matrix operand (column r, k =
+// 8g ..) comes out of a KiB of LDS that only this wave uses, by the transposing read.  As eight reads of two bytes a lane these factors held
+// up the launch that they share with r, k and v: 6.9 us a launch (768 channels, one user), 6.0 now.
+constexpr int KN_LDS = 512;                    // values a wave
+struct KnWeights {
+  const uint16_t* at;
+  int N, lane;
+  __device__ __forceinline__ KnWeights(const void* w, int N_, int n0, int lane_)
+      : at(static_cast<const uint16_t*>(w) + (size_t)(lane_ >> 1) * N_ + n0 + 8 * (lane_ & 1)), N(N_), lane(lane_) {}
+  __device__ __forceinline__ u32x4_t load(int s, int n = 0) const { return *reinterpret_cast<const u32x4_t*>(at + (size_t)32 * s * N + n); }
+  // in the order of the wave's LDS instructions: the next piece may follow at once
+  __device__ __forceinline__ u32x4_t operand(u32x4_t v, uint16_t* lds) const {
+    *reinterpret_cast<u32x4_t*>(lds + 8 * lane) = v;
+    const int r = lane & 15, g = lane >> 4;
+    const uint16_t* q = lds + (8 * g + (r >> 2)) * 16 + 4 * (r & 3);
+    const uint2 lo = lds_tr4(q), hi = lds_tr4(q + 4 * 16);
+    return u32x4_t{lo.x, lo.y, hi.x, hi.y};
+  }
+};
+
 // Weight-streaming product for few rows: bound by reading w once.  A workgroup owns 16 columns of one product and 16 MT
 // rows; its eight waves split K (every wave of the grid then streams a run of k of sixteen weight rows, so that many
 // short streams are in flight however small N is) and add their 16x16 tiles through LDS.  The weights' rows are the
-// matrix instruction's A operand straight from memory, 16 bytes per lane, no LDS; x comes from the cache.  KN weights (the
-// low-rank factors, a tenth of the bytes) are gathered two bytes at a time.
-template <int MT>
+// matrix instruction's A operand straight from memory, 16 bytes per lane, no LDS; x comes from the cache.  KN weights: KnWeights.
+// ONE: a single product, whose arguments are then one load away.
+template <int MT, bool ONE>
 __global__ __launch_bounds__(64 * GEMM_WAVES) void skinny_gemm_kernel(GemmArgs A) {
   __shared__ f32x4_t red[GEMM_WAVES][MT][64];
-  const int ji = job_of(A, blockIdx.x);
+  __shared__ __align__(16) uint16_t kn_lds[GEMM_WAVES][KN_LDS];
+  const int ji = ONE ? 0 : job_of(A, blockIdx.x);
   const GemmJob J = A.job[ji];
   const bf16_t* const jx = static_cast<const bf16_t*>(J.x);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-  const int n0 = ((int)blockIdx.x - A.tile0[ji]) * 16;
-  const int steps = J.K / 32, part = wave + GEMM_WAVES * (int)blockIdx.y, parts = GEMM_WAVES * (int)gridDim.y;
-  const int s0 = steps * part / parts, s1 = steps * (part + 1) / parts;
+  const int n0 = ONE ? (int)blockIdx.x * 16 : ((int)blockIdx.x - A.tile0[ji]) * 16;
+  const int steps = J.K / 32, part = wave + GEMM_WAVES * (int)blockIdx.y, log_parts = 3 + A.log_split;
+  const int s0 = steps * part >> log_parts, s1 = steps * (part + 1) >> log_parts;
   f32x4_t acc[MT];
   const bf16_t* xp[MT];
 #pragma unroll
@@ -77,40 +106,34 @@ __global__ __launch_bounds__(64 * GEMM_WAVES) void skinny_gemm_kernel(GemmArgs A
     const int m = 16 * t + r;
     xp[t] = jx + (size_t)(m < J.M ? m : J.M - 1) * J.K + 8 * g;
   }
-  auto step = [&](const u32x4_t w, int s) {
+  const bf16_t* const wp = static_cast<const bf16_t*>(J.w) + (size_t)(n0 + r) * J.K + 8 * g;
+  const KnWeights wk(J.w, J.N, n0, lane);
+  // COUNT steps whose loads are all requested before the first product; four at most, with eight fewer workgroups share a CU (24 layers of 2048
+  // channels, 16 users: 1752 us a step with eight, 1664 with four; one step after the other for what is left over: 1684)
+  auto steps_of = [&](auto count, int s) {
+    constexpr int COUNT = decltype(count)::value;
+    u32x4_t w[COUNT], x[COUNT][MT];
 #pragma unroll
-    for (int t = 0; t < MT; ++t) acc[t] = mfma(w, *reinterpret_cast<const u32x4_t*>(xp[t] + 32 * s), acc[t]);
+    for (int u = 0; u < COUNT; ++u) w[u] = J.kn ? wk.load(s + u) : *reinterpret_cast<const u32x4_t*>(wp + 32 * (s + u));
+#pragma unroll
+    for (int u = 0; u < COUNT; ++u) {
+#pragma unroll
+      for (int t = 0; t < MT; ++t) x[u][t] = *reinterpret_cast<const u32x4_t*>(xp[t] + 32 * (s + u));
+    }
+#pragma unroll
+    for (int u = 0; u < COUNT; ++u) {
+      const u32x4_t wf = J.kn ? wk.operand(w[u], kn_lds[wave]) : w[u];
+#pragma unroll
+      for (int t = 0; t < MT; ++t) acc[t] = mfma(wf, x[u][t], acc[t]);
+    }
   };
-  if (!J.kn) {
-    const bf16_t* wp = static_cast<const bf16_t*>(J.w) + (size_t)(n0 + r) * J.K + 8 * g;
-    constexpr int UN = MT == 1 ? 8 : 4;
-    int s = s0;
-    for (; s + UN <= s1; s += UN) {
-      u32x4_t w[UN];
-#pragma unroll
-      for (int u = 0; u < UN; ++u) w[u] = *reinterpret_cast<const u32x4_t*>(wp + 32 * (s + u));
-#pragma unroll
-      for (int u = 0; u < UN; ++u) step(w[u], s + u);
-    }
-    for (; s < s1; ++s) step(*reinterpret_cast<const u32x4_t*>(wp + 32 * s), s);
-  } else {
-    const uint16_t* wp = static_cast<const uint16_t*>(J.w) + (size_t)(8 * g) * J.N + n0 + r;
-    auto gather = [&](int s) {
-      u32x4_t w;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint16_t* p = wp + (size_t)(32 * s + 2 * i) * J.N;
-        w[i] = (uint32_t)p[0] | ((uint32_t)p[J.N] << 16);
-      }
-      return w;
-    };
-    int s = s0;
-    for (; s + 2 <= s1; s += 2) {
-      const u32x4_t w0 = gather(s), w1 = gather(s + 1);
-      step(w0, s);
-      step(w1, s + 1);
-    }
-    if (s < s1) step(gather(s), s);
+  constexpr int UN = 4;
+  int s = s0;
+  for (; s + UN <= s1; s += UN) steps_of(std::integral_constant<int, UN>(), s);
+  switch (s1 - s) {
+    case 3: steps_of(std::integral_constant<int, 3>(), s); break;
+    case 2: steps_of(std::integral_constant<int, 2>(), s); break;
+    case 1: steps_of(std::integral_constant<int, 1>(), s); break;
   }
 #pragma unroll
   for (int t = 0; t < MT; ++t) red[wave][t][lane] = acc[t];
@@ -132,157 +155,183 @@ __global__ __launch_bounds__(64 * GEMM_WAVES) void skinny_gemm_kernel(GemmArgs A
 }
 
 // What ln_shiftmix_kernel and the product above do, in one launch for one or two rows (a decode step of few users).  There a launch of
-// its own costs more than doing the norm again in every workgroup: its rows come from the cache while the weights, requested first, are
-// on their way.  Everything else that comes from memory is requested before the norm as well: each wait that follows one costs 1 us of
-// the 5 to 8.  xn lies in LDS; token shift and interpolation are applied to the eight values that a lane hands to a matrix instruction.
+// its own costs more than doing the norm again in every workgroup while the weights are on their way.  Such a kernel is a chain of
+// latencies: 0.4 us until the arguments are there, 0.4 to 0.6 for its rows, 1.4 for weights that no cache holds, 0.2 for a barrier, 2.2 ns an
+// instruction of a wave that has its SIMD to itself.  So the rows are requested before the weights (memory answers a wave in order), and a
+// wave normalises the channels of its own part of K alone: sixteen lanes a row, eight channels a lane and turn.  One barrier, for the sums:
+// mean and squares about it are combined from those of the eight parts, which is as precise as a second pass.  The interpolated values go to
+// the matrix instruction's layout through LDS that only this wave uses.  768 channels, one user: 7.4 and 6.2 us a launch (r, k, v; key), now 6.0 and 4.9, of which 1.7 are the launch.
 // Workgroup 0 writes the residual stream and the state's shift row.
-// G: rows; AHEAD_W: steps of K whose weights are requested first; NT: times 16 columns of a workgroup.
-template <int G, int AHEAD_W, int NT>
+// G: rows; TURNS: times 128 channels of a wave; NT: times 16 columns of a workgroup.
+template <int G, int TURNS, int NT>
 __global__ __launch_bounds__(64 * GEMM_WAVES) void head_gemm_kernel(LnMixArgs N, GemmArgs A) {
-  extern __shared__ __align__(16) uint16_t head_xn[];            // (rows, C + 8)
-  __shared__ f32x4_t red[GEMM_WAVES][NT][64];
-  __shared__ float sums[2][4 * GEMM_WAVES * G];                  // one per 16 lanes and row
+  __shared__ __align__(16) u32x4_t ops[GEMM_WAVES][G][16 * TURNS];       // 8 channels each
+  __shared__ f32x4_t red[GEMM_WAVES][NT][4][G];
+  __shared__ __align__(16) uint16_t kn_lds[GEMM_WAVES][KN_LDS];
+  __shared__ float2 sums[G][16];                                 // mean and squares about it of a wave's channels
+  constexpr int AHEAD_W = TURNS < 2 ? 4 : 8;                     // steps of K whose weights are requested first
   const int ji = job_of(A, blockIdx.x);
   const GemmJob J = A.job[ji];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r = lane & 15, g = lane >> 4;
-  const int C = (int)N.C, M = G, T = (int)N.T, stride = C + 8;
+  const int C = (int)N.C, T = (int)N.T;
   const int n0 = ((int)blockIdx.x - A.tile0[ji]) * 16 * NT;
-  const int steps = C / 32;
-  const int s0 = steps * wave / GEMM_WAVES, s1 = steps * (wave + 1) / GEMM_WAVES;
-  const bf16_t* const wp = static_cast<const bf16_t*>(J.w) + (size_t)(n0 + r) * C + 8 * g;
-  const uint16_t* const wk = static_cast<const uint16_t*>(J.w) + (size_t)(8 * g) * J.N + n0 + r;
-  auto weights = [&](int s, int q) {
-    if (!J.kn) return *reinterpret_cast<const u32x4_t*>(wp + (size_t)16 * q * C + 32 * s);
-    u32x4_t w;
+  const int steps = C / 32, s0 = steps * wave / GEMM_WAVES, s1 = steps * (wave + 1) / GEMM_WAVES, count = 32 * (s1 - s0);
+  // the norm: row j, channels 32 s0 + 8 (r + 16 i) ..
+  const int j = G == 1 ? 0 : g & 1, b = T == 1 ? j : 0, t = T == 1 ? 0 : j;
+  const bool reset = N.ns != nullptr && N.ns[j] != 0;
+  const int first = 32 * s0 + 8 * r;
+  u32x4_t x[TURNS], lnw[TURNS], lnb[TURNS], share[TURNS], before[TURNS];
+  f32x4_t d[4][TURNS][2];                        // what the residual stream gains: a product, or its first four partial sums
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint16_t* p = wk + (size_t)(32 * s + 2 * i) * J.N + 16 * q;
-      w[i] = (uint32_t)p[0] | ((uint32_t)p[J.N] << 16);
-    }
-    return w;
-  };
-  const int m = r < M ? r : M - 1, b = m / T, t = m - b * T;
-  const bool reset = N.ns != nullptr && N.ns[m] != 0;
-  const bf16_t* const cur = reinterpret_cast<const bf16_t*>(head_xn) + m * stride + 8 * g;
-  const bf16_t* const row = static_cast<const bf16_t*>(N.prev) + (size_t)b * N.prev_bstride + 8 * g;
-  const bf16_t* const mix = static_cast<const bf16_t*>(J.aux) + 8 * g;
-  auto at = [&](const bf16_t* p, int s) { return *reinterpret_cast<const u32x4_t*>(p + 32 * s); };
-  constexpr int AHEAD_X = 4;
-  u32x4_t w[AHEAD_W][NT], before[AHEAD_X], share[AHEAD_X];
-  const int c = 8 * tid, cc = c < C ? c : 0;                     // the norm: eight channels per thread
-  const u32x4_t lnw = *reinterpret_cast<const u32x4_t*>(static_cast<const bf16_t*>(N.ln_w) + cc);
-  const u32x4_t lnb = *reinterpret_cast<const u32x4_t*>(static_cast<const bf16_t*>(N.ln_b) + cc);
+  for (int i = 0; i < TURNS; ++i) {
+    x[i] = lnw[i] = lnb[i] = share[i] = before[i] = u32x4_t{0u, 0u, 0u, 0u};
 #pragma unroll
-  for (int u = 0; u < AHEAD_W; ++u) {
-    const int s = s0 + u < steps ? s0 + u : steps - 1;
-#pragma unroll
-    for (int q = 0; q < NT; ++q) w[u][q] = weights(s, q);
-    if (u < AHEAD_X) { before[u] = at(row, s); share[u] = at(mix, s); }
+    for (int p = 0; p < 4; ++p) d[p][i][0] = d[p][i][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
-  const float invC = 1.f / (float)C;
-  auto block_sums = [&](float (&v)[G], float* buf) {
+  if (g < G) {                                   // only the lanes that a row has: a request costs the CU by its lanes
 #pragma unroll
-    for (int j = 0; j < G; ++j) {
-      v[j] = row_sum(v[j]);
-      if ((tid & 15) == 0) buf[(tid >> 4) * G + j] = v[j];
-    }
-    __syncthreads();
+    for (int i = 0; i < TURNS; ++i) {
+      const int c = 8 * r + 128 * i < count ? first + 128 * i : 0;       // beyond the part: read, not used
+      auto at = [&](const void* p, size_t el) { return *reinterpret_cast<const u32x4_t*>(static_cast<const bf16_t*>(p) + el); };
+      x[i] = at(N.x, (size_t)j * C + c);
+      if (N.n_part > 1) {
 #pragma unroll
-    for (int j = 0; j < G; ++j) {                                // 32 sums, two by each of 16 lanes
-      v[j] = buf[(2 * (tid & 15)) * G + j] + buf[(2 * (tid & 15) + 1) * G + j];
-      v[j] = row_sum(v[j]);
-    }
-  };
-  {
-    float x[G][8], sum[G], sq[G];
-#pragma unroll
-    for (int j = 0; j < G; ++j) {
-      const size_t el = (size_t)j * C + cc;
-      ld8(static_cast<const bf16_t*>(N.x) + el, x[j]);
-      if (N.dx != nullptr || N.n_part > 1) {
-        float d[8];
-        if (N.n_part > 1) {                    // a product's partial sums
-          ld8(N.part + el, d);
-#pragma unroll 4
-          for (int p = 1; p < N.n_part; ++p) {
-            float q[8];
-            ld8(N.part + (size_t)p * M * C + el, q);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) d[e] += q[e];
+        for (int p = 0; p < 4; ++p)
+          if (p < 2 || p < N.n_part) {
+            const f32x4_t* q = reinterpret_cast<const f32x4_t*>(N.part + (size_t)(p * G + j) * C + c);
+            d[p][i][0] = q[0];
+            d[p][i][1] = q[1];
           }
-#pragma unroll
-          for (int e = 0; e < 8; ++e) d[e] = rnd(d[e]);
-        } else {
-          ld8(static_cast<const bf16_t*>(N.dx) + el, d);
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[j][e] = rnd(x[j][e] + d[e]);
-        if (blockIdx.x == 0 && c < C) st8(static_cast<bf16_t*>(N.xs) + el, x[j]);
+      } else if (N.dx != nullptr) {
+        d[0][i][0] = __builtin_bit_cast(f32x4_t, at(N.dx, (size_t)j * C + c));
       }
-      sum[j] = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) sum[j] += c < C ? x[j][e] : 0.f;
-    }
-    block_sums(sum, sums[0]);
-#pragma unroll
-    for (int j = 0; j < G; ++j) {
-      sum[j] *= invC;
-      sq[j] = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) { const float d = x[j][e] - sum[j]; sq[j] = c < C ? fmaf(d, d, sq[j]) : 0.f; }
-    }
-    block_sums(sq, sums[1]);
-#pragma unroll
-    for (int j = 0; j < G; ++j) {
-      if (c >= C) break;
-      const float rstd = rsqrtf(sq[j] * invC + N.eps);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x[j][e] = fmaf((x[j][e] - sum[j]) * rstd, half_of(lnw, e), half_of(lnb, e));
-      st8(reinterpret_cast<bf16_t*>(head_xn) + j * stride + c, x[j]);
-      const int nb = j / T;
-      if (blockIdx.x == 0 && j - nb * T == (int)last_token(N.length, nb, T))
-        st8(static_cast<bf16_t*>(N.shift) + (size_t)nb * N.shift_bstride + c, x[j]);
+      lnw[i] = at(N.ln_w, c);
+      lnb[i] = at(N.ln_b, c);
+      share[i] = at(J.aux, c);
+      before[i] = at(N.prev, (size_t)b * N.prev_bstride + c);
     }
   }
+  const bf16_t* const wp = static_cast<const bf16_t*>(J.w) + (size_t)(n0 + r) * C + 8 * g;
+  const KnWeights wk(J.w, J.N, n0, lane);
+  auto weights = [&](int s, int q) {
+    return J.kn ? wk.load(s, 16 * q) : *reinterpret_cast<const u32x4_t*>(wp + (size_t)16 * q * C + 32 * s);
+  };
+  auto operand = [&](u32x4_t v) { return J.kn ? wk.operand(v, kn_lds[wave]) : v; };
+  u32x4_t w[AHEAD_W][NT];
+#pragma unroll
+  for (int u = 0; u < AHEAD_W; ++u)
+#pragma unroll
+    for (int q = 0; q < NT; ++q) w[u][q] = weights(s0 + u < s1 ? s0 + u : steps - 1, q);
+  // the residual stream, rounded as it is stored
+  float sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < TURNS; ++i) {
+    const bool have = 8 * r + 128 * i < count;
+    if (N.n_part > 1) {
+      f32x4_t lo = d[0][i][0] + d[1][i][0], hi = d[0][i][1] + d[1][i][1];
+      lo = lo + d[2][i][0]; hi = hi + d[2][i][1];
+      lo = lo + d[3][i][0]; hi = hi + d[3][i][1];
+      for (int p = 4; p < N.n_part; ++p) {
+        const f32x4_t* q = reinterpret_cast<const f32x4_t*>(N.part + (size_t)(p * G + j) * C + (have ? first + 128 * i : 0));
+        lo += q[0];
+        hi += q[1];
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float s0_ = e < 2 ? lo[2 * e] : hi[2 * e - 4], s1_ = e < 2 ? lo[2 * e + 1] : hi[2 * e - 3];
+        x[i][e] = chunk::pack_rn(half_of(x[i], 2 * e) + rnd(s0_), half_of(x[i], 2 * e + 1) + rnd(s1_));
+      }
+    } else if (N.dx != nullptr) {
+      const u32x4_t dx = __builtin_bit_cast(u32x4_t, d[0][i][0]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        x[i][e] = chunk::pack_rn(half_of(x[i], 2 * e) + half_of(dx, 2 * e), half_of(x[i], 2 * e + 1) + half_of(dx, 2 * e + 1));
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sum += have ? half_of(x[i], e) : 0.f;
+  }
+  const float mine = row_sum(sum) / (float)(count > 0 ? count : 1);
+  float sq = 0.f;
+#pragma unroll
+  for (int i = 0; i < TURNS; ++i) {
+    const bool have = 8 * r + 128 * i < count;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) { const float v = half_of(x[i], e) - mine; sq = have ? fmaf(v, v, sq) : sq; }
+  }
+  sq = row_sum(sq);
+  if (r == 0 && g < G) sums[g][wave] = make_float2(mine, sq);
   __syncthreads();
+  const float invC = 1.f / (float)C;
+  const float2 of = sums[j][r & 7];
+  const float n = r < 8 ? 32.f * (float)(steps * (r + 1) / GEMM_WAVES - steps * r / GEMM_WAVES) : 0.f;
+  const float mean = row_sum(n * of.x) * invC, off = of.x - mean;
+  const float rstd = rsqrtf(row_sum(r < 8 ? fmaf(n * off, off, of.y) : 0.f) * invC + N.eps);
+  u32x4_t xn[TURNS];
+#pragma unroll
+  for (int i = 0; i < TURNS; ++i) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      xn[i][e] = chunk::pack_rn(fmaf((half_of(x[i], 2 * e) - mean) * rstd, half_of(lnw[i], 2 * e), half_of(lnb[i], 2 * e)),
+                                fmaf((half_of(x[i], 2 * e + 1) - mean) * rstd, half_of(lnw[i], 2 * e + 1), half_of(lnb[i], 2 * e + 1)));
+    u32x4_t p = before[i];
+    if (G > 1 && T > 1) {                        // the second token follows the first, sixteen lanes below
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t q = (uint32_t)__shfl((int)xn[i][e], lane - 16, 64);
+        p[e] = t > 0 ? q : p[e];
+      }
+    }
+    u32x4_t o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float lo = half_of(xn[i], 2 * e), hi = half_of(xn[i], 2 * e + 1);
+      o[e] = chunk::pack_rn(fmaf((reset ? 0.f : half_of(p, 2 * e)) - lo, half_of(share[i], 2 * e), lo),
+                            fmaf((reset ? 0.f : half_of(p, 2 * e + 1)) - hi, half_of(share[i], 2 * e + 1), hi));
+    }
+    if (g < G) ops[wave][j][r + 16 * i] = o;
+  }
+  // a wave's own writes and reads of LDS are in order
   f32x4_t acc[NT];
 #pragma unroll
   for (int q = 0; q < NT; ++q) acc[q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  auto step = [&](const u32x4_t (&ws)[NT], const u32x4_t prev, const u32x4_t part, int s) {
-    float x[8], f[8];
-    u32x4_t p = prev;
-    ld8(cur + 32 * s, x);
-    if (t > 0) p = *reinterpret_cast<const u32x4_t*>(cur + 32 * s - stride);
-    u32x4_t o;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) f[e] = fmaf((reset ? 0.f : half_of(p, e)) - x[e], half_of(part, e), x[e]);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = chunk::pack_rn(f[2 * e], f[2 * e + 1]);
-#pragma unroll
-    for (int q = 0; q < NT; ++q) acc[q] = mfma(ws[q], o, acc[q]);
-  };
+  const u32x4_t* const op = ops[wave][r < G ? r : G - 1] + g;
 #pragma unroll
   for (int u = 0; u < AHEAD_W; ++u)
     if (s0 + u < s1) {
-      if (u < AHEAD_X) step(w[u], before[u], share[u], s0 + u);
-      else step(w[u], at(row, s0 + u), at(mix, s0 + u), s0 + u);
+      const u32x4_t o = op[4 * u];
+#pragma unroll
+      for (int q = 0; q < NT; ++q) acc[q] = mfma(operand(w[u][q]), o, acc[q]);
     }
   for (int s = s0 + AHEAD_W; s < s1; ++s) {
     u32x4_t ws[NT];
 #pragma unroll
     for (int q = 0; q < NT; ++q) ws[q] = weights(s, q);
-    step(ws, at(row, s), at(mix, s), s);
+    const u32x4_t o = op[4 * (s - s0)];
+#pragma unroll
+    for (int q = 0; q < NT; ++q) acc[q] = mfma(operand(ws[q]), o, acc[q]);
   }
+  if (r < G) {
 #pragma unroll
-  for (int q = 0; q < NT; ++q) red[wave][q][lane] = acc[q];
+    for (int q = 0; q < NT; ++q) red[wave][q][g][r] = acc[q];
+  }
   __syncthreads();
-  if (wave < NT && r < M) {
-    f32x4_t v = red[0][wave][lane];
+  if (wave < NT && r < G) {
+    f32x4_t v = red[0][wave][g][r];
 #pragma unroll
-    for (int q = 1; q < GEMM_WAVES; ++q) v += red[q][wave][lane];
+    for (int q = 1; q < GEMM_WAVES; ++q) v += red[q][wave][g][r];
     const uint2 o = make_uint2(chunk::pack_rn(activate(v[0], J.act), activate(v[1], J.act)),
                                chunk::pack_rn(activate(v[2], J.act), activate(v[3], J.act)));
     *reinterpret_cast<uint2*>(static_cast<bf16_t*>(J.out) + (size_t)r * J.N + n0 + 16 * wave + 4 * g) = o;
+  }
+  if (blockIdx.x == 0 && g < G) {
+#pragma unroll
+    for (int i = 0; i < TURNS; ++i) {
+      if (8 * r + 128 * i >= count) break;
+      const int c = first + 128 * i;
+      if (N.dx != nullptr || N.n_part > 1) *reinterpret_cast<u32x4_t*>(static_cast<bf16_t*>(N.xs) + (size_t)j * C + c) = x[i];
+      if (t == (int)last_token(N.length, b, T))
+        *reinterpret_cast<u32x4_t*>(static_cast<bf16_t*>(N.shift) + (size_t)b * N.shift_bstride + c) = xn[i];
+    }
   }
 }
 
@@ -297,12 +346,6 @@ __global__ __launch_bounds__(64 * GEMM_WAVES) void head_gemm_kernel(LnMixArgs N,
 constexpr int TG = 64, TG_RS = TG + 8;         // tile edge; LDS row stride: 16-byte rows 144 bytes apart
 constexpr int AHEAD = 2;                       // steps whose operands are in flight (four: 212 registers, 1.6 times slower for short K)
 typedef uint16_t TileLds[2][2][TG][TG_RS];     // [buffer][x | w]
-
-__device__ __forceinline__ uint2 lds_tr4(const uint16_t* p) {      // see wkv7_fwd.hip
-  typedef short s16x4_t __attribute__((ext_vector_type(4)));
-  typedef __attribute__((address_space(3))) s16x4_t* lds_ptr;
-  return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p)));
-}
 
 using chunk::rsrc_t;
 using chunk::make_rsrc;
@@ -818,8 +861,10 @@ int gemm_split(int M, int64_t K, int64_t N) {
   const bool skinny = M < GEMM_TILE_ROWS;
   const int64_t tiles = skinny ? (N + 15) / 16 : (M + TG - 1) / TG * ((N + TG - 1) / TG);
   const int64_t want = 512 / tiles, most = skinny ? K / (32 * GEMM_WAVES * 3) : K / 256;
-  const int64_t n = want < most ? want : most;
-  return (int)(n < 1 ? 1 : n > GEMM_MAX_SPLIT ? GEMM_MAX_SPLIT : n);
+  int64_t n = want < most ? want : most;
+  n = n < 1 ? 1 : n > GEMM_MAX_SPLIT ? GEMM_MAX_SPLIT : n;
+  while (skinny && (n & (n - 1)) != 0) n &= n - 1;               // a power of two: a wave finds its part by a shift
+  return (int)n;
 }
 
 // Up to 32 rows the streaming kernel (K a multiple of 32, N of 16, no aux): its operand loads touch a cache line per lane,
@@ -889,23 +934,28 @@ hipError_t launch_gemm(GemmArgs A, int split, hipStream_t stream) {
   }
   place(TG, TG);
   if (!skinny) hipLaunchKernelGGL(tile_gemm_kernel, dim3(tiles, split), dim3(256), 0, stream, A);
-  else if (M <= 16) hipLaunchKernelGGL(skinny_gemm_kernel<1>, dim3(tiles, split), block, 0, stream, A);
-  else hipLaunchKernelGGL(skinny_gemm_kernel<2>, dim3(tiles, split), block, 0, stream, A);
+  else {
+    while (2 << A.log_split <= split) ++A.log_split;             // gemm_split: a power of two
+    auto kernel = A.n_jobs == 1 ? (M <= 16 ? skinny_gemm_kernel<1, true> : skinny_gemm_kernel<2, true>)
+                                : (M <= 16 ? skinny_gemm_kernel<1, false> : skinny_gemm_kernel<2, false>);
+    hipLaunchKernelGGL(kernel, dim3(tiles, split), block, 0, stream, A);
+  }
   return hipGetLastError();
 }
 
-template <int G, int AHEAD_W, int NT>
+template <int G, int TURNS, int NT>
 static hipError_t launch_head(const LnMixArgs& N, GemmArgs& A, hipStream_t stream) {
   const int tiles = place_jobs(A, [](const GemmJob& J) { return J.N / (16 * NT); });
-  hipLaunchKernelGGL((head_gemm_kernel<G, AHEAD_W, NT>), dim3(tiles), dim3(64 * GEMM_WAVES), (size_t)G * (N.C + 8) * 2, stream, N, A);
+  hipLaunchKernelGGL((head_gemm_kernel<G, TURNS, NT>), dim3(tiles), dim3(64 * GEMM_WAVES), 0, stream, N, A);
   return hipGetLastError();
 }
 // 32 columns a workgroup from 1025 channels on: with 16 there are two turns of workgroups, each with its norm (24 layers of 2048
-// channels, one user: 1536 us with 16, 1360 with 32, 1439 with norms of their own)
+// channels, one user, before requests were bundled: 1536 us with 16, 1360 with 32, 1439 with norms of their own; 1213 now)
 hipError_t launch_head_gemm(const LnMixArgs& N, GemmArgs A, hipStream_t stream) {
   const bool one = A.job[0].M == 1;
-  if (N.C <= 1024) return one ? launch_head<1, 4, 1>(N, A, stream) : launch_head<2, 4, 1>(N, A, stream);
-  return one ? launch_head<1, 8, 2>(N, A, stream) : launch_head<2, 8, 2>(N, A, stream);
+  if (N.C <= 1024) return one ? launch_head<1, 1, 1>(N, A, stream) : launch_head<2, 1, 1>(N, A, stream);
+  if (N.C <= 2048) return one ? launch_head<1, 2, 2>(N, A, stream) : launch_head<2, 2, 2>(N, A, stream);
+  return one ? launch_head<1, 4, 2>(N, A, stream) : launch_head<2, 4, 2>(N, A, stream);
 }
 
 hipError_t launch_rwkv7_lora_pre(const LoraPreArgs& A, hipStream_t stream) {

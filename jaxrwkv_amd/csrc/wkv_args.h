@@ -186,6 +186,7 @@ struct GemmArgs {
   int tile0[GEMM_MAX_JOBS];  // the launcher's: a job's first tile; side by side, so that a workgroup finds its job with one load
   GemmJob job[GEMM_MAX_JOBS];
   float* part;         // not null: (split, M, N) fp32 partial sums instead of out; one job, no f
+  int log_split;       // the launcher's, few rows
 };
 int gemm_split(int M, int64_t K, int64_t N);
 hipError_t launch_gemm(GemmArgs A, int split, hipStream_t stream);

@@ -92,3 +92,25 @@ def test_product_of_any_k(M, N, K, km, kn):
     d = (guard[1:-1].double() - want).abs()
     assert (d <= want.abs() * 2.0 ** -8 + 2.0 ** -18 * K ** 0.5).all()
     assert (guard[0] == 7).all() and (guard[-1] == 7).all()
+
+
+# few rows: a wave's steps of K from none to one more than a round of requests, one and two tiles of rows, either layout of the weights
+@pytest.mark.parametrize("kn", [0, 1])
+@pytest.mark.parametrize("M", [1, 16, 17, 32])
+@pytest.mark.parametrize("K", [32, 256, 544, 768, 1280, 1792, 2048, 2336])
+def test_product_of_few_rows(M, K, kn):
+    test_product(M, 48, K, 0, kn)
+
+
+def test_products_of_few_rows_in_one_launch():
+    from jaxrwkv_amd import blocks7
+    g = torch.Generator("cuda").manual_seed(7)
+    jobs, want = [], []
+    for N, K, kn in ((64, 768, 0), (32, 768, 1), (16, 96, 1), (80, 32, 0)):
+        x = torch.randn((5, K), device="cuda", generator=g).bfloat16()
+        w = torch.randn((K, N) if kn else (N, K), device="cuda", generator=g).bfloat16()
+        jobs.append((torch.empty((5, N), device="cuda", dtype=torch.bfloat16), x, w, 0, kn, 0, None))
+        want.append(x.double() @ (w.double() if kn else w.double().T))
+    blocks7._gemm(jobs)
+    for j, v in zip(jobs, want):
+        assert ((j[0].double() - v).abs() <= v.abs() * 2.0 ** -8 + 2.0 ** -18 * 768 ** 0.5).all()
