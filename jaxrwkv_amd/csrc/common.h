@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 namespace hiprwkv {
 
@@ -80,6 +81,69 @@ __device__ __forceinline__ void st8(bf16_t* p, const float (&o)[8]) {
   for (int i = 0; i < 4; ++i)
     w[i] = (uint32_t)f32_to_bf16(o[2 * i]) | ((uint32_t)f32_to_bf16(o[2 * i + 1]) << 16);
   *reinterpret_cast<uint4*>(p) = make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// Eight values kept as they lie in memory: in bf16 half the registers of eight floats
+template <typename T>
+struct Held;
+template <>
+struct Held<float> {
+  float v[8];
+  __device__ __forceinline__ void load(const float* p) { ld8(p, v); }
+  __device__ __forceinline__ void pin() {}
+  __device__ __forceinline__ float operator[](int c) const { return v[c]; }
+};
+template <>
+struct Held<bf16_t> {
+  uint32_t v[4];
+  __device__ __forceinline__ void load(const bf16_t* p) {
+    const uint4 a = *reinterpret_cast<const uint4*>(p);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+  }
+  // in a loop: keeps the compiler from unpacking once in front of it
+  __device__ __forceinline__ void pin() { asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3])); }
+  __device__ __forceinline__ float operator[](int c) const {
+    return __uint_as_float((c & 1) ? (v[c >> 1] & 0xffff0000u) : (v[c >> 1] << 16));
+  }
+};
+
+// Four consecutive values kept as they lie in memory
+template <typename T>
+struct Held4;
+template <>
+struct Held4<float> {
+  float4 v;
+  __device__ __forceinline__ void load(const float* p) { v = *reinterpret_cast<const float4*>(p); }
+  __device__ __forceinline__ void pin() {}
+  __device__ __forceinline__ float operator[](int c) const { return c == 0 ? v.x : c == 1 ? v.y : c == 2 ? v.z : v.w; }
+};
+template <>
+struct Held4<bf16_t> {
+  uint32_t v[2];
+  __device__ __forceinline__ void load(const bf16_t* p) {
+    const uint2 a = *reinterpret_cast<const uint2*>(p);
+    v[0] = a.x; v[1] = a.y;
+  }
+  __device__ __forceinline__ void pin() { asm volatile("" : "+v"(v[0]), "+v"(v[1])); }
+  __device__ __forceinline__ float operator[](int c) const {
+    return __uint_as_float((c & 1) ? (v[c >> 1] & 0xffff0000u) : (v[c >> 1] << 16));
+  }
+};
+template <typename T, int E>
+using HeldOf = std::conditional_t<E == 8, Held<T>, Held4<T>>;
+template <typename T, int E>
+__device__ __forceinline__ void ld_n(const T* p, float (&o)[E]) {
+  HeldOf<T, E> h;
+  h.load(p);
+#pragma unroll
+  for (int c = 0; c < E; ++c) o[c] = h[c];
+}
+template <typename T>
+__device__ __forceinline__ void st_n(T* p, const float (&o)[8]) { st8(p, o); }
+__device__ __forceinline__ void st_n(float* p, const float (&o)[4]) { *reinterpret_cast<float4*>(p) = make_float4(o[0], o[1], o[2], o[3]); }
+__device__ __forceinline__ void st_n(bf16_t* p, const float (&o)[4]) {
+  *reinterpret_cast<uint2*>(p) = make_uint2((uint32_t)f32_to_bf16(o[0]) | ((uint32_t)f32_to_bf16(o[1]) << 16),
+                                            (uint32_t)f32_to_bf16(o[2]) | ((uint32_t)f32_to_bf16(o[3]) << 16));
 }
 
 // IEEE half: the forward residual sa of the bf16 paths (11 significant bits where bf16 has 8)

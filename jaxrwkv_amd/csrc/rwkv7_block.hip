@@ -9,7 +9,7 @@
 // Memory bound.  As separate operations (addition, cast to fp32, norm, cast back, gather of the state row, shift and
 // interpolation) the six-output head of a layer moved 21 token tensors in bf16 units, this moves 9.  Measured in bf16 at
 // B=4 T=1021 C=2048: 37 us (4.1 TB/s) and 24 us with one output, against 72 and 55 us for the separate kernels; backward
-// with six cotangents at B=4 T=512 C=768: 27 + 9 us with its reduction, against 66 us for the shift kernel alone.
+// with six cotangents at B=4 T=512 C=768: 13 + 5 us with its reduction, against 66 us for the shift kernel alone.
 // A workgroup spans all channels (eight per thread, one 16-byte access in bf16) and walks a run of consecutive tokens,
 // GROUP at a time so that the loads of a group are in flight together and a pair of barriers serves all of them; the
 // xn of the token before stays in registers.  The first token of a run needs the xn of the one before it, which is
@@ -31,9 +31,6 @@ namespace hiprwkv {
 namespace {
 
 constexpr int MAX_WAVES = 8;           // 512 threads: C <= 4096, and 256 registers per thread (with 16 waves the kernels spill)
-// The same, backward: with six cotangents one token is eight 16-byte loads per thread, and two spill.
-template <int NOUT>
-constexpr int BWD_GROUP_OF = NOUT == 6 ? 1 : 2;
 
 // G sums over the workgroup at once.  `buf` is not read by anyone when a thread gets here (callers alternate two).
 template <int G>
@@ -64,30 +61,6 @@ __device__ __forceinline__ void zero_or_ld8(const T* p, bool take, float (&o)[8]
     for (int c = 0; c < 8; ++c) o[c] = 0.f;
   }
 }
-
-// Eight values kept as they lie in memory: in bf16 half the registers of eight floats
-template <typename T>
-struct Held;
-template <>
-struct Held<float> {
-  float v[8];
-  __device__ __forceinline__ void load(const float* p) { ld8(p, v); }
-  __device__ __forceinline__ void pin() {}
-  __device__ __forceinline__ float operator[](int c) const { return v[c]; }
-};
-template <>
-struct Held<bf16_t> {
-  uint32_t v[4];
-  __device__ __forceinline__ void load(const bf16_t* p) {
-    const uint4 a = *reinterpret_cast<const uint4*>(p);
-    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-  }
-  // in a loop: keeps the compiler from unpacking once in front of it
-  __device__ __forceinline__ void pin() { asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3])); }
-  __device__ __forceinline__ float operator[](int c) const {
-    return __uint_as_float((c & 1) ? (v[c >> 1] & 0xffff0000u) : (v[c >> 1] << 16));
-  }
-};
 
 // GROUP: tokens whose loads are in flight together, chosen by the launcher so that runs are whole groups (a decode step's token has
 // none before it; with groups of four its loads were asked for four times, partial sums of a product among them: 256 rows of 2048
@@ -200,19 +173,24 @@ __global__ __launch_bounds__(64 * MAX_WAVES) void ln_shiftmix_kernel(LnMixArgs A
   }
 }
 
-template <typename T, int NOUT>
+// The loads of a token are requested a token ahead: with the few waves that a SIMD has (512 workgroups at 2048 tokens of 768 channels) a token
+// took 6.5 us when its loads were waited for, most of it latency.  E channels a thread: four up to 2048 channels (eight make a token's chain
+// of instructions twice as long, spill with six cotangents and leave a quarter of the lanes idle at 768), eight beyond, where four need more
+// threads than registers allow.  B=4 T=512 C=768, six cotangents: 26.2 us waiting, two tokens' loads at a time with one (14.7 us); requested ahead
+// 22.1 and 10.6 with eight channels, 13.0 and 9.0 with four.
+template <typename T, int NOUT, int E>
 __global__ __launch_bounds__(64 * MAX_WAVES) void ln_shiftmix_bwd_kernel(LnMixArgs A) {
   constexpr int NG = NOUT ? NOUT : 1;          // cotangent tensors
-  constexpr int BWD_GROUP = BWD_GROUP_OF<NOUT>;
   constexpr int NP = NOUT + 2;                 // parameter cotangents: mix_0.., ln_w, ln_b
-  __shared__ float buf[2][2 * BWD_GROUP * MAX_WAVES * 4];
+  constexpr bool AHEAD = NOUT != 6 || E != 8;  // there the registers do not hold them
+  __shared__ float buf[2][2 * MAX_WAVES * 4];
   const int64_t C = A.C, Tn = A.T, total = A.B * A.T;
-  const int c8 = threadIdx.x * 8;
-  const bool on = c8 < C;
-  const int cc = on ? c8 : 0;
+  const int ce = threadIdx.x * E;
+  const bool on = ce < C;
+  const int cc = on ? ce : 0;
   const float invC = 1.f / (float)C;
-  float acc[NP][8];
-  Held<T> w, bias, m[NG];
+  float acc[NP][E];
+  HeldOf<T, E> w, bias, m[NG];
   w.load(reinterpret_cast<const T*>(A.ln_w) + cc);
   bias.load(reinterpret_cast<const T*>(A.ln_b) + cc);
 #pragma unroll
@@ -220,117 +198,116 @@ __global__ __launch_bounds__(64 * MAX_WAVES) void ln_shiftmix_bwd_kernel(LnMixAr
 #pragma unroll
   for (int i = 0; i < NP; ++i)
 #pragma unroll
-    for (int c = 0; c < 8; ++c) acc[i][c] = 0.f;
+    for (int c = 0; c < E; ++c) acc[i][c] = 0.f;
   const int64_t n0 = (int64_t)blockIdx.x * A.run;
   const int64_t n1 = (n0 + A.run < total ? n0 + A.run : total) - 1;      // last token of the run
+  // a token's cotangents and the one of xs, xs and its statistics of the token before; threads beyond C read channels that others have
+  HeldOf<T, E> g[NG], gx, x0, x1;
+  float2 st0, st1;
+  auto request = [&](int64_t n) {
+#pragma unroll
+    for (int i = 0; i < NG; ++i) g[i].load(reinterpret_cast<const T*>(A.g[i]) + n * C + cc);
+    if (A.gx != nullptr) gx.load(reinterpret_cast<const T*>(A.gx) + n * C + cc);
+  };
+  auto request_x = [&](int64_t n) {
+    n = n < 0 ? 0 : n;
+    x1.load(reinterpret_cast<const T*>(A.xs) + n * C + cc);
+    st1 = *reinterpret_cast<const float2*>(A.stats + 2 * n);
+  };
+  request_x(n1);
+  x0 = x1; st0 = st1;
   // sum_i g_i mix_i of the token after, if that token takes its shifted value from the one before it
-  float gm_next[8];
+  float gm_next[E];
 #pragma unroll
-  for (int c = 0; c < 8; ++c) gm_next[c] = 0.f;
+  for (int c = 0; c < E; ++c) gm_next[c] = 0.f;
   if (NOUT != 0 && n1 + 1 < total && (n1 + 1) % Tn != 0 && !(A.ns != nullptr && A.ns[n1 + 1] != 0)) {
+    request(n1 + 1);
 #pragma unroll
-    for (int i = 0; i < NOUT; ++i) {
-      float g[8];
-      zero_or_ld8(reinterpret_cast<const T*>(A.g[i]) + (n1 + 1) * C + cc, on, g);
+    for (int i = 0; i < NOUT; ++i)
 #pragma unroll
-      for (int c = 0; c < 8; ++c) gm_next[c] = fmaf(g[c], m[i][c], gm_next[c]);
-    }
+      for (int c = 0; c < E; ++c) gm_next[c] = fmaf(g[i][c], m[i][c], gm_next[c]);
   }
+  if (AHEAD) request(n1);
+  request_x(n1 - 1);
   int ph = 0;
-  for (int64_t top = n1; top >= n0; top -= BWD_GROUP, ph ^= 1) {
+  int64_t b = n1 / Tn, t = n1 - b * Tn;
+  for (int64_t n = n1; n >= n0; --n, ph ^= 1) {
+    if (!AHEAD) request(n);
     w.pin(); bias.pin();
 #pragma unroll
     for (int i = 0; i < NOUT; ++i) m[i].pin();
-    float gx[BWD_GROUP][8], xh[BWD_GROUP][8], rstd[BWD_GROUP], red[2 * BWD_GROUP];
-    // xs of the group's tokens and of the one before the group
-    float xs[BWD_GROUP + 1][8];
-    float2 st[BWD_GROUP + 1];
+    const float rstd = st0.y;
+    const bool reset = NOUT != 0 && A.ns != nullptr && A.ns[n] != 0;
+    float xh[E], dxn[E], red[2];
+    x0.pin();
 #pragma unroll
-    for (int j = 0; j <= BWD_GROUP; ++j) {
-      int64_t n = top - j;
-      n = n < 0 ? 0 : n;
-      if (NOUT != 0 || j < BWD_GROUP) {
-        zero_or_ld8(reinterpret_cast<const T*>(A.xs) + n * C + cc, on, xs[j]);
-        st[j] = *reinterpret_cast<const float2*>(A.stats + 2 * n);
+    for (int c = 0; c < E; ++c) xh[c] = (x0[c] - st0.x) * rstd;
+    if (NOUT == 0) {
+#pragma unroll
+      for (int c = 0; c < E; ++c) dxn[c] = g[0][c];
+    } else {
+      float pv[E], d[E], gm[E];
+      if (t == 0) ld_n(reinterpret_cast<const T*>(A.prev) + b * A.prev_bstride + cc, pv);
+#pragma unroll
+      for (int c = 0; c < E; ++c) {
+        const float xn = round_io<T>(fmaf(xh[c], w[c], bias[c]));
+        const float xb = round_io<T>(fmaf((x1[c] - st1.x) * st1.y, w[c], bias[c]));
+        d[c] = (reset ? 0.f : (t == 0 ? pv[c] : xb)) - xn;
+        gm[c] = 0.f;
+        dxn[c] = 0.f;
       }
+#pragma unroll
+      for (int i = 0; i < NOUT; ++i) {
+        g[i].pin();
+#pragma unroll
+        for (int c = 0; c < E; ++c) {
+          const float gi = g[i][c];
+          dxn[c] += gi;
+          gm[c] = fmaf(gi, m[i][c], gm[c]);
+          acc[i][c] = fmaf(gi, d[c], acc[i][c]);
+        }
+      }
+      const bool last_of_seq = t == Tn - 1;
+#pragma unroll
+      for (int c = 0; c < E; ++c) dxn[c] += (last_of_seq ? 0.f : gm_next[c]) - gm[c];
+      if (A.gshift != nullptr && t == last_token(A.length, b, Tn)) {
+        float gs[E];
+        ld_n(reinterpret_cast<const T*>(A.gshift) + b * C + cc, gs);
+#pragma unroll
+        for (int c = 0; c < E; ++c) dxn[c] += gs[c];
+      }
+#pragma unroll
+      for (int c = 0; c < E; ++c) gm_next[c] = reset ? 0.f : gm[c];
+      if (t == 0 && on && A.dprev != nullptr) st_n(reinterpret_cast<T*>(A.dprev) + b * C + ce, gm_next);
     }
+    // what the token before needs, while the sums below wait for each other
+    const HeldOf<T, E> gx_now = gx;
+    if (AHEAD && n > n0) request(n - 1);
+    x0 = x1; st0 = st1;
+    if (NOUT != 0 || n > n0) request_x(n - 2);
+    red[0] = red[1] = 0.f;
 #pragma unroll
-    for (int j = 0; j < BWD_GROUP; ++j) {
-      const int64_t n = top - j;
-      const bool live = n >= n0;
-      const int64_t nn = live ? n : n0;
-      const int64_t b = nn / Tn, t = nn - b * Tn;
-      rstd[j] = st[j].y;
-      float dxn[8];
-#pragma unroll
-      for (int c = 0; c < 8; ++c) xh[j][c] = (xs[j][c] - st[j].x) * st[j].y;
-      if (NOUT == 0) {
-        zero_or_ld8(reinterpret_cast<const T*>(A.g[0]) + nn * C + cc, on && live, dxn);
-      } else {
-        const bool reset = A.ns != nullptr && A.ns[nn] != 0;
-        float pv[8], d[8];
-        if (t == 0) ld8(reinterpret_cast<const T*>(A.prev) + b * A.prev_bstride + cc, pv);
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          const float xn = round_io<T>(fmaf(xh[j][c], w[c], bias[c]));
-          const float xb = round_io<T>(fmaf((xs[j + 1][c] - st[j + 1].x) * st[j + 1].y, w[c], bias[c]));
-          d[c] = (reset ? 0.f : (t == 0 ? pv[c] : xb)) - xn;
-        }
-        float gm[8];
-#pragma unroll
-        for (int c = 0; c < 8; ++c) { gm[c] = 0.f; dxn[c] = 0.f; }
-#pragma unroll
-        for (int i = 0; i < NOUT; ++i) {
-          float g[8];
-          zero_or_ld8(reinterpret_cast<const T*>(A.g[i]) + nn * C + cc, on && live, g);
-#pragma unroll
-          for (int c = 0; c < 8; ++c) {
-            dxn[c] += g[c];
-            gm[c] = fmaf(g[c], m[i][c], gm[c]);
-            acc[i][c] = fmaf(g[c], d[c], acc[i][c]);
-          }
-        }
-        if (live) {
-          const bool last_of_seq = t == Tn - 1;
-#pragma unroll
-          for (int c = 0; c < 8; ++c) dxn[c] += (last_of_seq ? 0.f : gm_next[c]) - gm[c];
-          if (A.gshift != nullptr && t == last_token(A.length, b, Tn)) {
-            float gs[8];
-            zero_or_ld8(reinterpret_cast<const T*>(A.gshift) + b * C + cc, on, gs);
-#pragma unroll
-            for (int c = 0; c < 8; ++c) dxn[c] += gs[c];
-          }
-#pragma unroll
-          for (int c = 0; c < 8; ++c) gm_next[c] = reset ? 0.f : gm[c];
-          if (t == 0 && on && A.dprev != nullptr) st8(reinterpret_cast<T*>(A.dprev) + b * C + c8, gm_next);
-        }
-      }
-      red[2 * j] = red[2 * j + 1] = 0.f;
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        acc[NOUT][c] = fmaf(dxn[c], xh[j][c], acc[NOUT][c]);
-        acc[NOUT + 1][c] += dxn[c];
-        gx[j][c] = dxn[c] * w[c];
-        red[2 * j] += gx[j][c];
-        red[2 * j + 1] = fmaf(gx[j][c], xh[j][c], red[2 * j + 1]);
-      }
+    for (int c = 0; c < E; ++c) {
+      acc[NOUT][c] = fmaf(dxn[c], xh[c], acc[NOUT][c]);
+      acc[NOUT + 1][c] += dxn[c];
+      const float gw = dxn[c] * w[c];
+      red[0] += gw;
+      red[1] = fmaf(gw, xh[c], red[1]);
     }
+    if (!on) red[0] = red[1] = 0.f;
     block_sum(red, buf[ph]);
+    if (on) {
+      const float s1 = red[0] * invC, s2 = red[1] * invC;
+      float o[E];
 #pragma unroll
-    for (int j = 0; j < BWD_GROUP; ++j) {
-      const int64_t n = top - j;
-      if (n < n0 || !on) break;
-      const float s1 = red[2 * j] * invC, s2 = red[2 * j + 1] * invC;
-      float o[8];
-      zero_or_ld8(reinterpret_cast<const T*>(A.gx) + n * C + c8, A.gx != nullptr, o);
-#pragma unroll
-      for (int c = 0; c < 8; ++c) o[c] += rstd[j] * (gx[j][c] - s1 - xh[j][c] * s2);
-      st8(reinterpret_cast<T*>(A.dxs) + n * C + c8, o);
+      for (int c = 0; c < E; ++c) o[c] = (A.gx != nullptr ? gx_now[c] : 0.f) + rstd * (dxn[c] * w[c] - s1 - xh[c] * s2);
+      st_n(reinterpret_cast<T*>(A.dxs) + n * C + ce, o);
     }
+    if (--t < 0) { t = Tn - 1; --b; }
   }
   if (on) {
 #pragma unroll
-    for (int i = 0; i < NP; ++i) st8(A.part + ((size_t)blockIdx.x * NP + i) * C + c8, acc[i]);
+    for (int i = 0; i < NP; ++i) st_n(A.part + ((size_t)blockIdx.x * NP + i) * C + ce, acc[i]);
   }
 }
 
@@ -413,8 +390,10 @@ hipError_t launch_ln_shiftmix(int io_f32, int n_out, LnMixArgs A, hipStream_t st
 
 hipError_t launch_ln_shiftmix_bwd(int io_f32, int n_out, LnMixArgs A, void* const* dparam, hipStream_t stream) {
   A.run = ln_shiftmix_bwd_run(A.B * A.T);
-  const dim3 grid((unsigned)((A.B * A.T + A.run - 1) / A.run)), block((unsigned)((A.C / 8 + 63) / 64 * 64));
-  HIPRWKV_BLOCK_DISPATCH(ln_shiftmix_bwd_kernel)
+  const bool four = A.C <= 4 * 64 * MAX_WAVES;
+  const dim3 grid((unsigned)((A.B * A.T + A.run - 1) / A.run)), block((unsigned)((A.C / (four ? 4 : 8) + 63) / 64 * 64));
+  if (four) { HIPRWKV_BLOCK_DISPATCH(ln_shiftmix_bwd_kernel, HIPRWKV_COMMA 4) }
+  else { HIPRWKV_BLOCK_DISPATCH(ln_shiftmix_bwd_kernel, HIPRWKV_COMMA 8) }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   ReduceArgs R;

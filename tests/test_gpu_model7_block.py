@@ -41,7 +41,7 @@ def both(fn, ref, tensors, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n_mix", [0, 1, 6])
-@pytest.mark.parametrize("B,T,C,with_dx", [(1, 1, 8, False), (3, 1, 128, True), (3, 45, 72, True), (2, 9, 2056, True),
+@pytest.mark.parametrize("B,T,C,with_dx", [(1, 1, 8, False), (3, 1, 128, True), (3, 45, 72, True), (2, 9, 2048, True), (2, 9, 2056, True),
                                            (1, 4100, 64, False)])
 def test_ln_shiftmix(B, T, C, with_dx, n_mix, dtype):
     from jaxrwkv_amd import ops
