@@ -429,12 +429,13 @@ struct TileOut {
     }
     *reinterpret_cast<uint2*>(lds + m * STRIDE + n) = make_uint2(chunk::pack_rn(v[0], v[1]), chunk::pack_rn(v[2], v[3]));
   }
-  // by all 256 threads, after a barrier
+  // by all threads of a workgroup, after a barrier
+  template <int THREADS>
   static __device__ __forceinline__ void write(const GemmArgs& A, const GemmJob& J, const uint16_t* lds, int n0, int m0) {
     if (A.part != nullptr) return;
     constexpr int PIECES = TN / 8;
 #pragma unroll 1
-    for (int i = threadIdx.x; i < TM * PIECES; i += 256) {
+    for (int i = threadIdx.x; i < TM * PIECES; i += THREADS) {
       const int m = i / PIECES, n = 8 * (i % PIECES);
       if (m0 + m >= J.M || n0 + n >= J.N) continue;
       const size_t el = (size_t)(m0 + m) * J.N + n0 + n;
@@ -522,7 +523,7 @@ __device__ __forceinline__ void tile_gemm_body(const GemmArgs& A, const GemmJob&
 #pragma unroll
     for (int u = 0; u < 2; ++u) Out::put(A, J, out, n0, m0, wn + 16 * t + 4 * g, wm + 16 * u + r, acc[t][u]);
   __syncthreads();
-  Out::write(A, J, out, n0, m0);
+  Out::write<256>(A, J, out, n0, m0);
 }
 
 // job and tile of a workgroup: along the longer side of the tile grid eight tiles at a time, one per XCD; all tiles across from
@@ -545,13 +546,13 @@ int tiles_of(const GemmJob& J, int tm, int tn) {
 // those of them that work
 int64_t real_tiles(const GemmJob& J, int tm, int tn) { return (int64_t)((J.M + tm - 1) / tm) * ((J.N + tn - 1) / tn); }
 
-// Tiles of 64 or 128 rows and columns with the operands requested straight into LDS, BUFS - 1 steps ahead: no registers are held by what
+// Tiles of 64 to 256 rows and 64 or 128 columns with the operands requested straight into LDS, BUFS - 1 steps ahead: no registers are held by what
 // is in flight.  Any K (launch_gemm: from 256 on, multiples of the step, or beside a product of 1024): the last step of one that is no
 // multiple is masked where it is read.  A wave's request fills 1 KiB as it lies, eight rows of 128 bytes or, of a 128-wide k-major
 // operand, four of 256, so rows cannot be padded: 16-byte piece p of row q lies at p ^ swizzle(q) instead (no bank conflicts counted in
 // the loop).  Weights that no cache holds, 64 x 64 tiles against those through registers: 64 rows of 2048 channels into 8192 columns 19.0 -> 15.3 us, K = 8192 into 2048 unsplit 57.9 -> 37.8;
 // 128 rows 19.3 -> 15.4; r, k, v and the low-rank inputs at 128 rows 20.5 -> 16.6; 256 rows into 8192 columns 23.5 -> 22.8 with
-// 64-row tiles, 19.9 with 128.  Bound by a step's way through LDS (see launch_gemm): in a step of 256 users (128 x 64, 17.8 us for 43.7 MB
+// 64-row tiles, 19.9 with 128, 19.2 with eight waves.  Bound by a step's way through LDS (see launch_gemm): in a step of 256 users (128 x 64, 17.8 us for 43.7 MB
 // read) the waves wait for half of their time, for arriving operands and each other, an LDS read is why in 1 %, and the matrix units work
 // a fifth of it (profiles/rwkv7_model_bf16.md); five and seven steps in flight took as long, and so did a first step that differs from tile
 // to tile.
@@ -564,11 +565,11 @@ __device__ __forceinline__ void request_lds(u32x4_t rs, int voff, int soff, uint
   asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(rs), "s"(soff), "{m0}"(lds) : "memory");
 }
 
-// ROWS (64 or 128) rows of m or n by 64 of k; with TR the operand lies k-major and so does its piece of LDS.  The last step of a K
+// ROWS (64, 128 or 256) rows of m or n by 64 of k; with TR the operand lies k-major and so does its piece of LDS.  The last step of a K
 // that is no multiple of 64 asks for the last k again where there are no more; what it gives is masked (`keep`).
-template <bool TR, int ROWS>
+template <bool TR, int ROWS, int WAVES>
 struct StreamOperand {
-  static constexpr int PIECES = ROWS / 32;                           // requests of a wave per step
+  static constexpr int PIECES = ROWS / 8 / WAVES;                           // requests of a wave per step
   static constexpr int PER_ROW = TR ? ROWS / 8 : TG / 8;             // 16-byte pieces of an LDS row
   static constexpr int LINES = 64 / PER_ROW;                         // LDS rows that a request fills
   u32x4_t rs;
@@ -623,21 +624,21 @@ __device__ __forceinline__ u32x4_t keep_k(u32x4_t v, int k0, int end) {
   return v;
 }
 
-// TM x TN tiles, four waves of TM/2 x TN/2
-template <int TM, int TN, int BUFS, bool KM, bool KN>
+// TM x TN tiles, WM x WN waves
+template <int TM, int TN, int BUFS, int WM, int WN, bool KM, bool KN>
 __device__ __forceinline__ void stream_gemm_body(const GemmArgs& A, const GemmJob& J, int n0, int m0, uint16_t* lds) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-  constexpr int MT = TM / 32, NT = TN / 32, STEP = stream_step(TM, TN), IN_STEP = TM / 32 + TN / 32;
+  constexpr int WAVES = WM * WN, MT = TM / WM / 16, NT = TN / WN / 16, STEP = stream_step(TM, TN), IN_STEP = (TM + TN) / 8 / WAVES;
   const int all = (J.K + TG - 1) / TG;
   const int s0 = all * (int)blockIdx.y / (int)gridDim.y, s1 = all * ((int)blockIdx.y + 1) / (int)gridDim.y;
-  typedef StreamOperand<KM, TM> OpX;
-  typedef StreamOperand<KN, TN> OpW;
+  typedef StreamOperand<KM, TM, WAVES> OpX;
+  typedef StreamOperand<KN, TN, WAVES> OpW;
   const OpX X(J.x, J.M, J.K, m0, wave, lane);
   const OpW W(J.w, J.N, J.K, n0, wave, lane);
   f32x4_t acc[NT][MT];
 #pragma unroll
   for (int i = 0; i < NT * MT; ++i) acc[i / MT][i % MT] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const int wn = TN / 2 * (wave & 1), wm = TM / 2 * (wave >> 1);
+  const int wn = TN / WN * (wave % WN), wm = TM / WM * (wave / WN);
   auto request = [&](int s, int buf) {
     X.request(s, lds + buf * STEP);
     W.request(s, lds + buf * STEP + TM * TG);
@@ -702,30 +703,30 @@ __device__ __forceinline__ void stream_gemm_body(const GemmArgs& A, const GemmJo
 #pragma unroll
     for (int u = 0; u < MT; ++u) Out::put(A, J, lds, n0, m0, wn + 16 * t + 4 * g, wm + 16 * u + r, acc[t][u]);
   __syncthreads();
-  Out::write(A, J, lds, n0, m0);
+  Out::template write<64 * WM * WN>(A, J, lds, n0, m0);
 }
 
-template <int TM, int TN, int BUFS>
-__global__ __launch_bounds__(256) void stream_gemm_kernel(GemmArgs A) {
+template <int TM, int TN, int BUFS, int WM, int WN>
+__global__ __launch_bounds__(64 * WM * WN) void stream_gemm_kernel(GemmArgs A) {
   extern __shared__ __align__(1024) uint16_t stream_lds[];
   int ji, n0, m0;
   if (!tile_of(A, TM, TN, ji, n0, m0)) return;
   const GemmJob J = A.job[ji];
   switch ((J.km ? 2 : 0) + (J.kn ? 1 : 0)) {
-    case 0: stream_gemm_body<TM, TN, BUFS, false, false>(A, J, n0, m0, stream_lds); break;
-    case 1: stream_gemm_body<TM, TN, BUFS, false, true>(A, J, n0, m0, stream_lds); break;
-    case 2: stream_gemm_body<TM, TN, BUFS, true, false>(A, J, n0, m0, stream_lds); break;
-    default: stream_gemm_body<TM, TN, BUFS, true, true>(A, J, n0, m0, stream_lds); break;
+    case 0: stream_gemm_body<TM, TN, BUFS, WM, WN, false, false>(A, J, n0, m0, stream_lds); break;
+    case 1: stream_gemm_body<TM, TN, BUFS, WM, WN, false, true>(A, J, n0, m0, stream_lds); break;
+    case 2: stream_gemm_body<TM, TN, BUFS, WM, WN, true, false>(A, J, n0, m0, stream_lds); break;
+    default: stream_gemm_body<TM, TN, BUFS, WM, WN, true, true>(A, J, n0, m0, stream_lds); break;
   }
 }
-template <int TM, int TN, int BUFS>
+template <int TM, int TN, int BUFS, int WM, int WN>
 hipError_t launch_stream(const GemmArgs& A, int tiles, int split, hipStream_t stream) {
   static LdsAttrOnce attr;
   constexpr size_t bytes = (size_t)BUFS * stream_step(TM, TN) * 2;
-  const auto kernel = stream_gemm_kernel<TM, TN, BUFS>;
+  const auto kernel = stream_gemm_kernel<TM, TN, BUFS, WM, WN>;
   hipError_t e = allow_dynamic_lds(attr, reinterpret_cast<const void*>(kernel), bytes);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kernel, dim3(tiles, split), dim3(256), bytes, stream, A);
+  hipLaunchKernelGGL(kernel, dim3(tiles, split), dim3(64 * WM * WN), bytes, stream, A);
   return hipGetLastError();
 }
 
@@ -872,20 +873,25 @@ int gemm_split(int M, int64_t K, int64_t N) {
 // rows, 16 at 33, 21 at 64; tiled 15 us up to 128 rows, 22 at 256).
 // From 33 rows tiles, straight to LDS (through registers where an operand of a narrow K is no multiple of a step: the second low-rank
 // factors, which the other kernel would mostly mask).  Which: a step takes in proportion to what passes through a CU's LDS (its operands
-// are written at 64 bytes a cycle and read twice at 128: 4 (TM + TN) cycles; measured 0.29 us for 64 x 64, 0.40 for 128 x 64, 0.59 for 128
-// x 128; by the counters the waves wait for what arrives, not for what they read, so the writing half rather), so the tile that takes the
-// fewest steps a CU times TM + TN.  Products of one K run in rounds over the CUs; of several, the longest or the mean counts and 128 x 128
-// tiles leave too few to balance.  Weights that no cache holds, us with 64x64, 128x64, 128x128 tiles: 2048 rows: three 768x768 22.2 / 20.2
-// / 17.9, 768 into 3072 23.1 / 19.2 / 17.4, 3072 into 768 24.0 / 25.5 / 33; with the weights' cotangents: of 768x768 14.0 / 17.0 / 29, of
-// three 41 / 36.6 / 44, of 3072 into 768 43 / 35 / 40.  512 rows: 2048 into 8192 36 / 29 / 25, 8192 into 2048 37 / 52 / 75.  4084 rows:
-// three 2048x2048 225 / 161 / 116.  256 rows of 2048 into 8192: 21 / 18.8 / 24. Empty workgroups of the 128 x 128 tiles do not count: with
+// are written at 64 bytes a cycle and read twice at 128: 4 (TM + TN) cycles; measured 0.29 us for 64 x 64, 0.40 for 128 x 64, 0.54 for 128
+// x 128, 0.79 for 256 x 128 with one workgroup a CU; by the counters the waves wait for what arrives, not for what they read), so the tile
+// that takes the fewest steps a CU times TM + TN.  Products of one K run in rounds over the CUs; of several, the longest or the mean counts.
+// Eight waves from 128 rows on: one reads LDS while the other of its SIMD multiplies.  us with four waves and with eight, weights that no
+// cache holds: three 768x768 of 2048 rows in 128 x 128 tiles 14.4 / 13.3, one in 128 x 64 7.7 / 6.8, its K = 3072 22.2 / 21.0; the same in
+// a training step, 768 into 3072 forward 128 x 128 24.9 / 22.2 and, without transposed operands, 256 x 128 20.6; its two backward products
+// in one launch 128 x 64 47.4 / 41.3, 128 x 128 43.6 / 37.8, 64 x 64 52.8; K = 3072 backward 128 x 64 33.4 / 34.5, 128 x 128 with three
+// buffers 31.3; six of 768 x 768 and the low-rank ones 41.2 / 38.2 and 37.8; r, k, v and the low-rank inputs 26.6 / 25.0, 24.9 / 22.8,
+// 256 x 128 26.1 (transposed ones among them).  4084 rows, three 2048 x 2048: 128 x 128 102 / 99, 256 x 128 95.  Large tiles of several K
+// leave less to balance: they have to be a tenth better by that count.  Products split over K keep four waves (256 rows of 8192 columns
+// 14.7 / 15.0).  512 rows: 2048 into 8192 64 x 64 36, 128 x 64 29, 128 x 128 25, 8192 into 2048 37 / 52 / 75.
+// Empty workgroups of the tiles of 128 columns do not count: with
 // them, and as edges, 24 layers of 2048 channels fell back to 128 x 64 at 2200 rows, 12.9 ms forward, now 12.0, at 2600 14.6, now 12.8, at
 // 3200 18.7, now 14.8.  Those of the smaller tiles do: 12 layers of 768 channels were 1 % slower without them (700 and 1500 rows).  More
-// requests in flight change nothing: four steps took as long as three (one workgroup per CU), and so did reading half a step ahead of its
-// products.
+// requests in flight change nothing: four steps took as long as three (one workgroup per CU), and so did two groups of waves half a step apart
+// and tiles handed out in blocks of several rows and columns an XCD.
 constexpr int CUS = 256, WIDE_TILES = 192;
 hipError_t launch_gemm(GemmArgs A, int split, hipStream_t stream) {
-  bool skinny = true, stream_k = true, same_k = true;
+  bool skinny = true, stream_k = true, same_k = true, plain = true;
   int M = 0, longest = 0, tiles = 0;
   // the longest first: what is left at the end is short
   for (int i = 1; i < A.n_jobs; ++i)
@@ -895,6 +901,7 @@ hipError_t launch_gemm(GemmArgs A, int split, hipStream_t stream) {
     M = J.M > M ? J.M : M;
     longest = J.K > longest ? J.K : longest;
     same_k = same_k && J.K == A.job[0].K;
+    plain = plain && !J.km && !J.kn;
     stream_k = stream_k && (J.K % TG == 0 || J.K >= 4 * TG);
     skinny = skinny && J.M < GEMM_TILE_ROWS && !J.km && J.aux == nullptr && J.raw == nullptr && J.K % 32 == 0 && J.N % 16 == 0;
   }
@@ -903,9 +910,9 @@ hipError_t launch_gemm(GemmArgs A, int split, hipStream_t stream) {
   const dim3 block(64 * GEMM_WAVES);
   if (!skinny && stream_k && (split > 1 || A.part != nullptr)) {
     place(2 * TG, TG);
-    if (M > TG && tiles * split >= WIDE_TILES && tiles * split <= CUS) return launch_stream<2 * TG, TG, 4>(A, tiles, split, stream);
+    if (M > TG && tiles * split >= WIDE_TILES && tiles * split <= CUS) return launch_stream<2 * TG, TG, 4, 2, 2>(A, tiles, split, stream);
     place(TG, TG);
-    return launch_stream<TG, TG, 4>(A, tiles, split, stream);
+    return launch_stream<TG, TG, 4, 2, 2>(A, tiles, split, stream);
   }
   if (!skinny && stream_k) {
     auto cost = [&](int tm, int tn) {
@@ -920,17 +927,22 @@ hipError_t launch_gemm(GemmArgs A, int split, hipStream_t stream) {
       if (tn > TG && 100 * area < 85 * n * tm * tn) return INT64_MAX;         // mostly edges (the low-rank inputs alone: 38 us and 34)
       return (same_k ? (n + CUS - 1) / CUS * one : mean > one ? mean : one) * (tm + tn);
     };
-    const int64_t small = cost(TG, TG), wide = M > TG ? cost(2 * TG, TG) : small, large = M > TG && same_k ? cost(2 * TG, 2 * TG) : wide;
-    if (large < wide && large < small) {
+    const int64_t small = cost(TG, TG), wide = M > TG ? cost(2 * TG, TG) : small, large = M > TG ? cost(2 * TG, 2 * TG) : wide;
+    const int64_t huge = M > 2 * TG && same_k && plain ? cost(4 * TG, 2 * TG) : large;
+    if (huge < large && huge < wide && huge < small) {
+      place(4 * TG, 2 * TG);
+      return launch_stream<4 * TG, 2 * TG, 3, 4, 2>(A, tiles, split, stream);
+    }
+    if (large < (same_k ? wide : wide - wide / 11) && large < small) {
       place(2 * TG, 2 * TG);
-      return tiles > CUS ? launch_stream<2 * TG, 2 * TG, 2>(A, tiles, split, stream) : launch_stream<2 * TG, 2 * TG, 3>(A, tiles, split, stream);
+      return tiles > CUS ? launch_stream<2 * TG, 2 * TG, 2, 2, 4>(A, tiles, split, stream) : launch_stream<2 * TG, 2 * TG, 3, 2, 4>(A, tiles, split, stream);
     }
     if (wide < small) {
       place(2 * TG, TG);
-      return tiles > CUS ? launch_stream<2 * TG, TG, 3>(A, tiles, split, stream) : launch_stream<2 * TG, TG, 4>(A, tiles, split, stream);
+      return tiles > CUS ? launch_stream<2 * TG, TG, 3, 4, 2>(A, tiles, split, stream) : launch_stream<2 * TG, TG, 4, 4, 2>(A, tiles, split, stream);
     }
     place(TG, TG);
-    return launch_stream<TG, TG, 4>(A, tiles, split, stream);
+    return launch_stream<TG, TG, 4, 2, 2>(A, tiles, split, stream);
   }
   place(TG, TG);
   if (!skinny) hipLaunchKernelGGL(tile_gemm_kernel, dim3(tiles, split), dim3(256), 0, stream, A);

@@ -114,3 +114,25 @@ def test_products_of_few_rows_in_one_launch():
     blocks7._gemm(jobs)
     for j, v in zip(jobs, want):
         assert ((j[0].double() - v).abs() <= v.abs() * 2.0 ** -8 + 2.0 ** -18 * 768 ** 0.5).all()
+
+
+# 256 x 128 tiles: the edge of a tile each way, one turn of the buffers and more, a last step that is not full
+@pytest.mark.parametrize("M,N", [(2056, 3080), (2040, 3072)])
+@pytest.mark.parametrize("K", [256, 264, 320, 520])
+def test_product_in_the_largest_tiles(M, N, K):
+    test_product_of_any_k(M, N, K, 0, 0)
+
+
+def test_products_of_several_k_in_large_tiles():
+    """A product of few steps and one of many, 128 x 128 tiles, transposed operands."""
+    from jaxrwkv_amd import blocks7
+    g = torch.Generator("cuda").manual_seed(8)
+    jobs, want = [], []
+    for M, N, K, km, kn in ((2056, 3080, 264, 0, 1), (776, 3080, 2056, 1, 1)):
+        x = torch.randn((K, M) if km else (M, K), device="cuda", generator=g).bfloat16()
+        w = torch.randn((K, N) if kn else (N, K), device="cuda", generator=g).bfloat16()
+        jobs.append((torch.empty((M, N), device="cuda", dtype=torch.bfloat16), x, w, km, kn, 0, None))
+        want.append((x.double().T if km else x.double()) @ (w.double() if kn else w.double().T))
+    blocks7._gemm(jobs)
+    for j, v in zip(jobs, want):
+        assert ((j[0].double() - v).abs() <= v.abs() * 2.0 ** -8 + 2.0 ** -18 * 2056 ** 0.5).all()
