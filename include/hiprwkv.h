@@ -75,7 +75,10 @@ extern "C" {
  * consumer waves' wait runs out (a few milliseconds), every wave still ends normally, the outputs of every
  * (sequence, head) are NaN and hiprwkv_handshake_failures() has advanced by B*H per kernel. */
 #define HIPRWKV_DEBUG_DROP_PUBLISH 0x100u
-/* Every flag a production caller may pass.  Entry points refuse other bits, and refuse HIPRWKV_DEBUG_DROP_PUBLISH
+/* hiprwkv_wkv7_fwd*, hiprwkv_wkv6_fwd*: new_s is written in io_dtype (rounded once from the fp32 state of the kernel) instead of
+ * state_dtype, which then is s's type alone; s and new_s have to be different arrays where the two types differ. */
+#define HIPRWKV_NEW_STATE_IO 0x200u
+/* Every flag a production caller may pass, but for HIPRWKV_NEW_STATE_IO, which only the entry points above take.  Entry points refuse other bits, and refuse HIPRWKV_DEBUG_DROP_PUBLISH
  * unless the process runs with HIPRWKV_ENABLE_DEBUG_FLAGS=1 in its environment. */
 #define HIPRWKV_PUBLIC_FLAGS (HIPRWKV_COMPAT_ASSOC | HIPRWKV_FORCE_SEQ | HIPRWKV_NO_SMALL_T | HIPRWKV_W_PER_HEAD | HIPRWKV_CKPT_READY | HIPRWKV_LENGTH_I32 | HIPRWKV_W_RAW)
 

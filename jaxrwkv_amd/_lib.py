@@ -16,6 +16,7 @@ W_PER_HEAD = 0x10
 CKPT_READY = 0x20
 LENGTH_I32 = 0x40
 W_RAW = 0x80
+NEW_STATE_IO = 0x200             # the forwards of WKV7 and WKV6 alone
 DEBUG_DROP_PUBLISH = 0x100      # refused unless the process runs with HIPRWKV_ENABLE_DEBUG_FLAGS=1
 PUBLIC_FLAGS = COMPAT_ASSOC | FORCE_SEQ | NO_SMALL_T | W_PER_HEAD | CKPT_READY | LENGTH_I32 | W_RAW
 

@@ -95,9 +95,9 @@ void* scratch_base() {
 // Public flag bits are accepted everywhere; the test hook HIPRWKV_DEBUG_DROP_PUBLISH only in a process that sets the
 // environment variable HIPRWKV_ENABLE_DEBUG_FLAGS=1, so that a stray bit cannot turn a production call's outputs
 // into NaN.  Unknown bits are refused.
-int check_flags(const char* op, unsigned flags) {
-  if (flags & ~(HIPRWKV_PUBLIC_FLAGS | HIPRWKV_DEBUG_DROP_PUBLISH))
-    return fail(HIPRWKV_EINVAL, "%s: unknown flag bits 0x%x", op, flags & ~(HIPRWKV_PUBLIC_FLAGS | HIPRWKV_DEBUG_DROP_PUBLISH));
+int check_flags(const char* op, unsigned flags, bool new_state_io = false) {
+  const unsigned known = HIPRWKV_PUBLIC_FLAGS | HIPRWKV_DEBUG_DROP_PUBLISH | (new_state_io ? HIPRWKV_NEW_STATE_IO : 0u);
+  if (flags & ~known) return fail(HIPRWKV_EINVAL, "%s: unknown flag bits 0x%x", op, flags & ~known);
   if (flags & HIPRWKV_DEBUG_DROP_PUBLISH) {
     static const bool enabled = [] { const char* e = getenv("HIPRWKV_ENABLE_DEBUG_FLAGS"); return e != nullptr && e[0] == '1'; }();
     if (!enabled)
@@ -187,7 +187,9 @@ int hiprwkv_wkv7_fwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype, 
                           void* new_s, void* ends, void* workspace, size_t workspace_bytes, unsigned flags) {
   int rc = check_matrix_shape("wkv7_fwd", io_dtype, state_dtype, B, T, H, N);
   if (rc) return rc;
-  if ((rc = check_flags("wkv7_fwd", flags)) != HIPRWKV_OK) return rc;
+  if ((rc = check_flags("wkv7_fwd", flags, true)) != HIPRWKV_OK) return rc;
+  if ((flags & HIPRWKV_NEW_STATE_IO) && io_dtype != state_dtype && s == new_s)
+    return fail(HIPRWKV_EINVAL, "wkv7_fwd: s and new_s must be different arrays where their types differ");
   const void* req[] = {w, r, k, v, a, b, s, out, new_s};
   for (const void* p : req) {
     if (p == nullptr) return fail(HIPRWKV_EINVAL, "wkv7_fwd: null tensor pointer");
@@ -206,7 +208,7 @@ int hiprwkv_wkv7_fwd_ends(hiprwkv_stream stream, int io_dtype, int state_dtype, 
   A.w = w; A.r = r; A.k = k; A.v = v; A.a = a; A.b = b; A.s = s;
   A.length = length; A.ns = new_starts;
   A.out = out; A.sa = sa; A.new_s = new_s;
-  A.io_f32 = io_dtype == HIPRWKV_F32; A.st_f32 = state_dtype == HIPRWKV_F32;
+  A.io_f32 = io_dtype == HIPRWKV_F32; A.st_f32 = state_dtype == HIPRWKV_F32; A.new_st_f32 = (flags & HIPRWKV_NEW_STATE_IO) ? A.io_f32 : A.st_f32;
   A.flags = flags;
   A.status = status_word();
   A.parts = need != 0 ? workspace : nullptr;
@@ -251,7 +253,7 @@ int hiprwkv_wkv7_step(hiprwkv_stream stream, int io_dtype, int state_dtype, int6
   A.w = w; A.r = r; A.k = k; A.v = v; A.a = a; A.b = b; A.s = s;
   A.length = length; A.ns = new_starts;
   A.out = out; A.new_s = new_s;
-  A.io_f32 = io_dtype == HIPRWKV_F32; A.st_f32 = state_dtype == HIPRWKV_F32;
+  A.io_f32 = io_dtype == HIPRWKV_F32; A.st_f32 = A.new_st_f32 = state_dtype == HIPRWKV_F32;
   A.flags = flags;
   A.s_bstride = s_batch_stride; A.new_s_bstride = new_s_batch_stride;
   const hipError_t e = launch_wkv7_small_t_fwd(A, static_cast<hipStream_t>(stream));
@@ -358,7 +360,9 @@ int hiprwkv_wkv6_fwd_parts(hiprwkv_stream stream, int io_dtype, int state_dtype,
                            size_t workspace_bytes, unsigned flags) {
   int rc = check_matrix_shape("wkv6_fwd", io_dtype, state_dtype, B, T, H, N);
   if (rc) return rc;
-  if ((rc = check_flags("wkv6_fwd", flags)) != HIPRWKV_OK) return rc;
+  if ((rc = check_flags("wkv6_fwd", flags, true)) != HIPRWKV_OK) return rc;
+  if ((flags & HIPRWKV_NEW_STATE_IO) && io_dtype != state_dtype && s == new_s)
+    return fail(HIPRWKV_EINVAL, "wkv6_fwd: s and new_s must be different arrays where their types differ");
   const void* req[] = {r, k, v, w, u, s, out, new_s};
   for (const void* p : req) {
     if (p == nullptr) return fail(HIPRWKV_EINVAL, "wkv6_fwd: null tensor pointer");
@@ -374,7 +378,7 @@ int hiprwkv_wkv6_fwd_parts(hiprwkv_stream stream, int io_dtype, int state_dtype,
   A.r = r; A.k = k; A.v = v; A.w = w; A.u = u; A.s = s;
   A.length = length; A.ns = new_starts;
   A.out = out; A.new_s = new_s;
-  A.io_f32 = io_dtype == HIPRWKV_F32; A.st_f32 = state_dtype == HIPRWKV_F32;
+  A.io_f32 = io_dtype == HIPRWKV_F32; A.st_f32 = state_dtype == HIPRWKV_F32; A.new_st_f32 = (flags & HIPRWKV_NEW_STATE_IO) ? A.io_f32 : A.st_f32;
   A.flags = flags;
   A.parts = need != 0 ? workspace : nullptr;
   A.status = status_word();
@@ -414,7 +418,7 @@ int hiprwkv_wkv6_step(hiprwkv_stream stream, int io_dtype, int state_dtype, int6
   A.r = r; A.k = k; A.v = v; A.w = w; A.u = u; A.s = s;
   A.length = length; A.ns = new_starts;
   A.out = out; A.new_s = new_s;
-  A.io_f32 = io_dtype == HIPRWKV_F32; A.st_f32 = state_dtype == HIPRWKV_F32;
+  A.io_f32 = io_dtype == HIPRWKV_F32; A.st_f32 = A.new_st_f32 = state_dtype == HIPRWKV_F32;
   A.flags = flags;
   A.s_bstride = s_batch_stride; A.new_s_bstride = new_s_batch_stride;
   const hipError_t e = launch_wkv6_small_t_fwd(A, static_cast<hipStream_t>(stream));

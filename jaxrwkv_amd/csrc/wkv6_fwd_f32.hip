@@ -299,7 +299,7 @@ __device__ __forceinline__ void store_state_tile(const Wkv6Args& A, int64_t b, i
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const size_t off = state_off(A, b, h, 16 * tile + 4 * g + i, 16 * q + n);
-    if (A.st_f32) reinterpret_cast<float*>(A.new_s)[off] = v[i];
+    if (A.new_st_f32) reinterpret_cast<float*>(A.new_s)[off] = v[i];
     else reinterpret_cast<uint16_t*>(A.new_s)[off] = f32_to_bf16(v[i]);
   }
 }
@@ -483,7 +483,7 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv6_fwd_f32_kernel(Wkv6
   __syncthreads();
   if (head_broken(sy, A.status)) {
     poison_token_rows(A.out, 4, b, h, A.T, A.H);
-    poison_state(A.new_s, A.st_f32, b, h, A.H);
+    poison_state(A.new_s, A.new_st_f32, b, h, A.H);
   }
 }
 

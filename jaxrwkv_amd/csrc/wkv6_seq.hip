@@ -67,7 +67,7 @@ struct Fwd6Step {
     const size_t base = ((size_t)id.b * A->H + id.h) * N64 * N64;
 #pragma unroll
     for (int c = 0; c < 16; ++c)
-      st_state6(A->new_s, A->st_f32, base + (size_t)(id.q * 16 + c) * N64 + id.line, id.q2drop ? 0.f : S[c]);
+      st_state6(A->new_s, A->new_st_f32, base + (size_t)(id.q * 16 + c) * N64 + id.line, id.q2drop ? 0.f : S[c]);
   }
   __device__ __forceinline__ void step(int tl, int64_t t, float (*sin)[F6_CH][N64], float (*sout)[F6_CH][N64],
                                        const uint8_t* sns) {

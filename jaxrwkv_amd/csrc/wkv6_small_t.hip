@@ -48,7 +48,11 @@ __global__ __launch_bounds__(256) void wkv6_small_t_kernel(Wkv6Args A) {
     for (int c = 0; c < 16; ++c) S[c] = ld_f(p + (size_t)c * 64);
   }
   ld16<IO>(A.u, (size_t)h * 64 + c0, u);
-  if (L == 0) st_col<ST>(A.new_s, sel_out, S, q2drop);
+  auto put_state = [&]() {
+    if (A.new_st_f32) st_col<float>(A.new_s, sel_out, S, q2drop);
+    else st_col<bf16_t>(A.new_s, sel_out, S, q2drop);
+  };
+  if (L == 0) put_state();
   for (int64_t t = 0; t < A.T; ++t) {
     const size_t tel = (((size_t)b * A.T + t) * A.H + h) * 64;
     float w[16], r[16], k[16];
@@ -74,7 +78,7 @@ __global__ __launch_bounds__(256) void wkv6_small_t_kernel(Wkv6Args A) {
     }
     const float y = quad_sum(y0 + y1);
     if (q == 0) st_f(reinterpret_cast<IO*>(A.out) + tel + j, y);
-    if (t == L - 1) st_col<ST>(A.new_s, sel_out, S, q2drop);
+    if (t == L - 1) put_state();
   }
 }
 

@@ -536,7 +536,7 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
         acc[2] = C.S[tile][2] * sg.z; acc[3] = C.S[tile][3] * sg.w;
       }
       acc = mfma_h(su, sv, acc);
-      store_state_tile(A.new_s, A.st_f32, state_off(A, b, h, C.q, lane, tile), q2drop ? zero4 : acc);
+      store_state_tile(A.new_s, A.new_st_f32, state_off(A, b, h, C.q, lane, tile), q2drop ? zero4 : acc);
     }
   }
   // state update, tile by tile: rows = keys.  S <- S diag(gamma) + Be^T SA^T + Ke^T V^T; a reset inside the chunk
@@ -705,7 +705,7 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_kernel(Wkv7Args
     if (L == 0 && (MODE == WHOLE || (MODE == PART && part == 0))) {
 #pragma unroll
       for (int tile = 0; tile < 4; ++tile)
-        store_state_tile(A.new_s, A.st_f32, state_off(A, b, h, cq, lane, tile), q2drop ? zero4 : C.S[tile]);
+        store_state_tile(A.new_s, A.new_st_f32, state_off(A, b, h, cq, lane, tile), q2drop ? zero4 : C.S[tile]);
     }
     OutCursor oc;
     oc.tok_bytes = (size_t)A.H * 64 * 2;
@@ -792,7 +792,7 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_kernel(Wkv7Args
     const int64_t t0 = (int64_t)j_out * CK, rows = MODE == WHOLE || (int64_t)(j0 + n) * CK > A.T ? A.T - t0 : (int64_t)(j0 + n) * CK - t0;
     poison_token_rows(A.out, 2, b, h, A.T, A.H, t0, rows);
     poison_token_rows(A.sa, 2, b, h, A.T, A.H, t0, rows);
-    if (MODE == WHOLE || (L == 0 ? part == 0 : L - 1 >= t0 && L - 1 < t0 + rows)) poison_state(A.new_s, A.st_f32, b, h, A.H);
+    if (MODE == WHOLE || (L == 0 ? part == 0 : L - 1 >= t0 && L - 1 < t0 + rows)) poison_state(A.new_s, A.new_st_f32, b, h, A.H);
   }
 }
 

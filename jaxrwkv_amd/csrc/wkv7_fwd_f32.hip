@@ -489,7 +489,7 @@ __device__ __forceinline__ bool consume(Consumer& C, Ops& o, const Slot* __restr
       }
       acc = mfma_tt(sk, vv, acc);     // the order of the update below: a snapshot at the chunk end has its bits
       acc = mfma_tt(sb, SA, acc);
-      store_state_tile(A.new_s, A.st_f32, state_off(A, b, h, C.q, lane, tile), q2drop ? zero4 : acc);
+      store_state_tile(A.new_s, A.new_st_f32, state_off(A, b, h, C.q, lane, tile), q2drop ? zero4 : acc);
     }
   }
   if (MODE == SUMMARY) return ok;
@@ -585,7 +585,7 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_f32_kernel(Wkv7
     if (L == 0 && (MODE == WHOLE || (MODE == PART && part == 0))) {
 #pragma unroll
       for (int tile = 0; tile < 4; ++tile)
-        store_state_tile(A.new_s, A.st_f32, state_off(A, b, h, cq, lane, tile), q2drop ? zero4 : C.S[tile]);
+        store_state_tile(A.new_s, A.new_st_f32, state_off(A, b, h, cq, lane, tile), q2drop ? zero4 : C.S[tile]);
     }
     OutCursor oc;
     oc.tok = (size_t)A.H * 64;
@@ -671,7 +671,7 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_f32_kernel(Wkv7
     poison_token_rows(A.out, 4, b, h, A.T, A.H, t0, rows);
     poison_token_rows(A.sa, 4, b, h, A.T, A.H, t0, rows);
     if (A.ends != nullptr) poison_ends(A.ends, A, head, j_out + 1, j0 + n);
-    if (MODE == WHOLE || (L == 0 ? part == 0 : L - 1 >= t0 && L - 1 < t0 + rows)) poison_state(A.new_s, A.st_f32, b, h, A.H);
+    if (MODE == WHOLE || (L == 0 ? part == 0 : L - 1 >= t0 && L - 1 < t0 + rows)) poison_state(A.new_s, A.new_st_f32, b, h, A.H);
   }
 }
 

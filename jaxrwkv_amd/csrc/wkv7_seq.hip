@@ -60,7 +60,7 @@ struct FwdStep {
   __device__ __forceinline__ void snapshot() {
     const size_t base = (((size_t)id.b * A->H + id.h) * N64 + id.line) * N64 + id.q * 16;
 #pragma unroll
-    for (int c = 0; c < 16; ++c) st_state(A->new_s, A->st_f32, base + c, id.q2drop ? 0.f : S[c]);
+    for (int c = 0; c < 16; ++c) st_state(A->new_s, A->new_st_f32, base + c, id.q2drop ? 0.f : S[c]);
   }
   __device__ __forceinline__ void step(int tl, int64_t t, float (*sin)[FWD_CH][N64], float (*sout)[FWD_CH][N64],
                                        const uint8_t* sns) {

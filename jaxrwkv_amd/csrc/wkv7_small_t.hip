@@ -45,7 +45,11 @@ __global__ __launch_bounds__(256) void wkv7_small_t_kernel(Wkv7Args A) {
   const size_t sel_out = (size_t)b * (A.new_s_bstride ? (size_t)A.new_s_bstride : dense) + in_head;
   float S[16];
   ld16<ST>(A.s, sel, S);
-  if (L == 0) st16<ST>(A.new_s, sel_out, S, q2drop);   // rwkv7.py:203
+  auto put_state = [&]() {
+    if (A.new_st_f32) st16<float>(A.new_s, sel_out, S, q2drop);
+    else st16<bf16_t>(A.new_s, sel_out, S, q2drop);
+  };
+  if (L == 0) put_state();   // rwkv7.py:203
   for (int64_t t = 0; t < A.T; ++t) {
     const size_t tel = (((size_t)b * A.T + t) * A.H + h) * 64;
     float w[16], r[16], k[16], a[16], bb[16];
@@ -80,7 +84,7 @@ __global__ __launch_bounds__(256) void wkv7_small_t_kernel(Wkv7Args A) {
         else reinterpret_cast<_Float16*>(A.sa)[tel + i] = (_Float16)sa;
       }
     }
-    if (t == L - 1) st16<ST>(A.new_s, sel_out, S, q2drop);
+    if (t == L - 1) put_state();
   }
 }
 

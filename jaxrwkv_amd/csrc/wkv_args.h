@@ -18,7 +18,7 @@ struct Wkv7Args {
   void* out;
   void* sa;       // forward residual (may be null): fp32 beside fp32 I/O, IEEE half beside bf16 I/O
   void* new_s;
-  int io_f32, st_f32;
+  int io_f32, st_f32, new_st_f32;      // I/O, s, new_s
   unsigned flags;
   // backward only
   const void* gy;
@@ -65,7 +65,7 @@ struct Wkv6Args {
   const uint8_t* ns;
   void* out;
   void* new_s;
-  int io_f32, st_f32;
+  int io_f32, st_f32, new_st_f32;      // I/O, s, new_s
   unsigned flags;
   // backward only
   const void* gy;

@@ -158,6 +158,14 @@ def wkv7_fwd(r, w, k, v, a, b, s, length=None, new_starts=None, compat=True, wan
     return _wkv7_fwd(r, w, k, v, a, b, s, length, new_starts, compat, want_sa, force_seq, small_t, debug_flags)[:3]
 
 
+def _new_state(s, io, state_io):
+    """Memory for a forward's new state beside the state ``s``, and the flag that goes with it.  ``state_io``: a caller rounds the state to
+    the I/O type; from fp32 to bf16 the kernel does that (a launch of 3 us and 7 us of the host less)."""
+    if state_io and s.dtype == torch.float32 and io == torch.bfloat16:
+        return torch.empty(s.shape, dtype=io, device=s.device), _lib.NEW_STATE_IO
+    return torch.empty_like(s), 0
+
+
 def _wkv7_ends(io, B, T, H, N, device):
     """Memory that goes along to a backward in parts, None where the sequence runs whole."""
     nbytes = _lib.load().hiprwkv_wkv7_ends_bytes(_DT[io], B, T, H, N)
@@ -165,9 +173,9 @@ def _wkv7_ends(io, B, T, H, N, device):
 
 
 def _wkv7_fwd(r, w, k, v, a, b, s, length=None, new_starts=None, compat=True, want_sa=False, force_seq=False,
-              small_t=True, debug_flags=0, want_ends=False):
+              small_t=True, debug_flags=0, want_ends=False, state_io=False):
     """``wkv7_fwd`` with a fourth result: with ``want_ends`` what lets the backward run the sequence in parts, where that is of use
-    (fp32: filled here; bf16: memory that the backward fills)."""
+    (fp32: filled here; bf16: memory that the backward fills).  ``state_io``: see ``_new_state``."""
     lib = _lib.load()
     io = r.dtype
     r, w, k, v, a, b = (_dev(x, io) for x in (r, w, k, v, a, b))
@@ -176,7 +184,7 @@ def _wkv7_fwd(r, w, k, v, a, b, s, length=None, new_starts=None, compat=True, wa
     assert s.shape == (B, H, N, N), (s.shape, r.shape)
     length, new_starts = _length_ns(length, new_starts, B, T, r.device)
     y = _empty_like_phased(r, 1)
-    new_s = torch.empty_like(s)
+    new_s, state_flag = _new_state(s, io, state_io)
     # the residual for the backward pass: fp32 beside fp32 I/O, fp16 beside bf16 I/O
     sa = _empty_phased((B, T, H, N), _SA_DT[io], r.device, _phase(r) + 2) if want_sa else None
     nbytes = 0 if force_seq else lib.hiprwkv_wkv7_fwd_workspace_bytes(_DT[io], B, T, H, N)
@@ -185,7 +193,7 @@ def _wkv7_fwd(r, w, k, v, a, b, s, length=None, new_starts=None, compat=True, wa
     fn, more = (lib.hiprwkv_wkv7_fwd_parts, ()) if ends is None else (lib.hiprwkv_wkv7_fwd_ends, (_p(ends),))
     rc = fn(_stream(), _DT[io], _DT[s.dtype], B, T, H, N, _p(w), _p(r), _p(k), _p(v), _p(a), _p(b),
             _p(s), _p(length), _p(new_starts), _p(y), _p(sa), _p(new_s), *more, _p(ws), nbytes,
-            _flags(compat, force_seq, small_t, debug_flags))
+            _flags(compat, force_seq, small_t, debug_flags) | state_flag)
     _lib.check(rc, "hiprwkv_wkv7_fwd")
     return new_s, y, sa, ends
 
@@ -272,23 +280,24 @@ class _Wkv7(torch.autograd.Function):
         return gr, gw, gk, gv, ga, gb, gs, None, None, None, None
 
 
-def wkv7(r, w, k, v, a, b, s, length=None, new_starts=None, compat=True, force_seq=False):
-    """Differentiable WKV7: returns (new_s, y).  ``force_seq`` runs the sequential fp32 kernels whatever the dtype."""
+def wkv7(r, w, k, v, a, b, s, length=None, new_starts=None, compat=True, force_seq=False, state_io=False):
+    """Differentiable WKV7: returns (new_s, y).  ``force_seq`` runs the sequential fp32 kernels whatever the dtype.  ``state_io``: the
+    caller will round new_s to r's type, so it may come in that already."""
     B, T = r.shape[:2]
     if not _needs_grad(r, w, k, v, a, b, s):
-        return wkv7_fwd(r, w, k, v, a, b, s, length, new_starts, compat, force_seq=force_seq)[:2]
+        return _wkv7_fwd(r, w, k, v, a, b, s, length, new_starts, compat, force_seq=force_seq, state_io=state_io)[:2]
     length, new_starts = _length_ns(length, new_starts, B, T, r.device, keep=True)
     return _Wkv7.apply(r, w, k, v, a, b, s, length, new_starts, compat, force_seq)
 
 
 # ----------------------------------------------------------------------------- WKV6
 def wkv6_fwd(r, k, v, w, u, s, length=None, new_starts=None, compat=True, force_seq=False, small_t=True,
-             debug_flags=0):
+             debug_flags=0, state_io=False):
     """r,k,v (B,T,H,N); w (B,T,H,N), or (H,N) for a log decay shared by all tokens (RWKV-5); u (H,N);
     s (B,H,N,N) [key, value].  Returns (new_s, y).
 
     T <= 8 runs on the small-T (decode) kernel unless ``small_t=False``; otherwise bf16 inputs run on the chunked
-    MFMA kernel unless ``force_seq`` asks for the sequential fp32 one."""
+    MFMA kernel unless ``force_seq`` asks for the sequential fp32 one.  ``state_io``: see ``_new_state``."""
     lib = _lib.load()
     io = r.dtype
     B, T, H, N = r.shape
@@ -299,12 +308,12 @@ def wkv6_fwd(r, k, v, w, u, s, length=None, new_starts=None, compat=True, force_
     s = _dev(s)
     length, new_starts = _length_ns(length, new_starts, B, T, r.device)
     y = _empty_like_phased(r, 1)
-    new_s = torch.empty_like(s)
+    new_s, state_flag = _new_state(s, io, state_io)
     nbytes = 0 if force_seq else lib.hiprwkv_wkv6_fwd_workspace_bytes(_DT[io], B, T, H, N)
     ws = _workspace(nbytes, r.device) if nbytes else None
     rc = lib.hiprwkv_wkv6_fwd_parts(_stream(), _DT[io], _DT[s.dtype], B, T, H, N, _p(r), _p(k), _p(v), _p(w), _p(u), _p(s),
                                     _p(length), _p(new_starts), _p(y), _p(new_s), _p(ws), nbytes,
-                                    _flags(compat, force_seq, small_t, debug_flags) | (_lib.W_PER_HEAD if per_head else 0))
+                                    _flags(compat, force_seq, small_t, debug_flags) | state_flag | (_lib.W_PER_HEAD if per_head else 0))
     _lib.check(rc, "hiprwkv_wkv6_fwd")
     return new_s, y
 
@@ -381,11 +390,11 @@ class _Wkv6(torch.autograd.Function):
         return gr, gk, gv, gw.reshape(ctx.shapes[0]), gu.reshape(ctx.shapes[1]), gs, None, None, None, None
 
 
-def wkv6(r, k, v, w, u, s, length=None, new_starts=None, compat=True, force_seq=False):
-    """Differentiable WKV6: returns (new_s, y).  ``force_seq`` runs the sequential fp32 kernels whatever the dtype."""
+def wkv6(r, k, v, w, u, s, length=None, new_starts=None, compat=True, force_seq=False, state_io=False):
+    """Differentiable WKV6: returns (new_s, y).  ``force_seq`` and ``state_io`` as in ``wkv7``."""
     B, T = r.shape[:2]
     if not _needs_grad(r, k, v, w, u, s):
-        return wkv6_fwd(r, k, v, w, u, s, length, new_starts, compat, force_seq=force_seq)
+        return wkv6_fwd(r, k, v, w, u, s, length, new_starts, compat, force_seq=force_seq, state_io=state_io)
     length, new_starts = _length_ns(length, new_starts, B, T, r.device, keep=True)
     return _Wkv6.apply(r, k, v, w, u, s, length, new_starts, compat, force_seq)
 

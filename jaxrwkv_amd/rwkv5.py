@@ -27,7 +27,7 @@ class HipRWKV:
         B, T, H, N = r.shape
         logw = torch.log(w.float().reshape(H, -1)).expand(H, N).to(r.dtype).contiguous()   # HIPRWKV_W_PER_HEAD
         u = time_first.reshape(H, -1).expand(H, N).contiguous()
-        new_s, y = ops.wkv6(r, k, v, logw, u, s, length, new_starts, cls.assoc_compat)
+        new_s, y = ops.wkv6(r, k, v, logw, u, s, length, new_starts, cls.assoc_compat, state_io=True)
         new_s = new_s.to(r.dtype)
         if not batched:
             new_s, y = new_s[0], y[0]

@@ -22,7 +22,7 @@ class HipRWKV:
         else:
             w = w.reshape(r.shape)
         new_s, y = ops.wkv6(r, k, v, w, time_first.reshape(r.shape[2], r.shape[3]), s, length, new_starts,
-                            cls.assoc_compat)
+                            cls.assoc_compat, state_io=True)
         new_s = new_s.to(r.dtype)
         if not batched:
             new_s, y = new_s[0], y[0]

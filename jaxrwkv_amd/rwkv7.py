@@ -29,7 +29,7 @@ class HipRWKV:
             r, w, k, v, a, b, s = (x[None] for x in (r, w, k, v, a, b, s))
             if torch.is_tensor(new_starts) and new_starts.dim() == 1:
                 new_starts = new_starts[None]
-        new_s, y = ops.wkv7(r, w, k, v, a, b, s, length, new_starts, cls.assoc_compat, cls.force_seq)
+        new_s, y = ops.wkv7(r, w, k, v, a, b, s, length, new_starts, cls.assoc_compat, cls.force_seq, state_io=True)
         new_s = new_s.to(r.dtype)
         if not batched:
             new_s, y = new_s[0], y[0]
