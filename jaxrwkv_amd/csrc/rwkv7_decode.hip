@@ -32,9 +32,11 @@ __device__ __forceinline__ float wave_sum(float x) {
 }
 
 struct CoreArgs {
-  int64_t T, H;
-  const bf16_t *r, *k, *v, *vf, *xw, *xa, *xv, *g;          // (B,T,H,64); vf null: the first layer
-  const bf16_t *w0, *a0, *v0, *k_k, *k_a, *ln_w, *ln_b, *r_k;   // (H,64)
+  int64_t B, T, H;
+  int per;                     // sequences of a workgroup
+  const bf16_t* par[2][6];     // (H,64) parameters of waves 0 and 1: a0 k_k k_a r_k ln_w ln_b | w0 v0
+  const bf16_t* tok[2][4];     // (B,T,H,64): k r xa g | v xw v_first xv
+  int vmix;                    // there is a value residual
   float eps;
   const bf16_t* s;             // states: H*64*64 elements per sequence, bstride apart
   bf16_t* new_s;
@@ -45,95 +47,120 @@ struct CoreArgs {
   bf16_t* y;
 };
 
-// One workgroup per (head, sequence); thread (row i = tid/4, quarter q = tid%4) holds 16 elements of state row i, as in
-// the small-T kernel of the op, whose state traffic (2 x 8 KB per head) is the bound.  The state is requested first; waves 0 and 1
-// (one lane per channel) meanwhile turn the projections into the op's inputs and hand them over through LDS, wave 0 takes
-// y back through LDS for the group norm, the bonus and the gate.  B=256 H=32: the state alone is 67 MB each way; 38.5 us a launch with one
-// wave for all of that and its sums through LDS, 34.6 now (3.9 TB/s): a workgroup's chain of dependent steps, six workgroups a CU.
-__global__ __launch_bounds__(256, 6) void decode_core_kernel(CoreArgs A) {
+// A workgroup has one head of `per` consecutive sequences, one after the other; thread (row i = tid/4, quarter q = tid%4) holds 16 elements
+// of state row i, as in the small-T kernel of the op, whose state traffic (2 x 8 KB per head) is the bound.  Waves 0 and 1 (one lane per
+// channel) turn the projections into the op's inputs and hand them over through LDS, wave 0 takes y back through LDS for the group norm,
+// the bonus and the gate.  A sequence is a chain of waits; the state and the operands of the next one are requested before this one's are
+// used, so that memory works through it.  B=256 H=32: the state alone is 67 MB each way; 38.5 us a launch with one wave for the op's inputs
+// and sums by way of LDS, 34.6 with a workgroup a sequence (six of them a CU), 31.3 now with four a CU (4.6 TB/s; five 32.1, and for six the
+// registers spill: 51).
+constexpr int CORE_PER_CU = 4;
+__global__ __launch_bounds__(256, CORE_PER_CU) void decode_core_kernel(CoreArgs A) {
   __shared__ __align__(16) float ch[5][64];            // d, k', a_i, b_i, r
   __shared__ float vs[64], ys[64];
-  const int64_t b = blockIdx.y, h = blockIdx.x;
+  const int h = blockIdx.x;
+  const int64_t b0 = (int64_t)blockIdx.y * A.per, b1 = b0 + A.per < A.B ? b0 + A.per : A.B;
   const int tid = threadIdx.x, i = tid >> 2, q = tid & 3, c0 = 16 * q;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const bool keys = wave == 0, values = wave == 1;     // which part of the op's inputs a wave makes
-  int64_t L = A.T;
-  if (A.length != nullptr) { L = A.length[b]; L = L < 0 ? 0 : L < A.T ? L : A.T; }
-  const bool compat = (A.flags & 1u) != 0;
-  const uint8_t* ns = A.ns ? A.ns + b * A.T : nullptr;
-  const bool q2drop = compat && L < A.T && ns != nullptr && ns[L] != 0;
-  const size_t sel = (size_t)b * A.bstride + ((size_t)h * 64 + i) * 64 + c0;
-  float S[16];
-  ld16<bf16_t>(A.s, sel, S);
-  auto put_state = [&]() {
-    float lo[8], hi[8];
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, role = wave & 1;
+  const bool maker = wave < 2;                         // wave 0: what comes of k, r, a and the end; wave 1: decay and values
+  const size_t in_state = ((size_t)h * 64 + i) * 64 + c0;
+  uint4 s0, s1;                                        // the next sequence's state and first token, as they lie
+  uint32_t tk[4];
+  auto request_token = [&](int64_t row) {
 #pragma unroll
-    for (int c = 0; c < 8; ++c) { lo[c] = q2drop ? 0.f : S[c]; hi[c] = q2drop ? 0.f : S[8 + c]; }
-    st8(A.new_s + sel, lo);
-    st8(A.new_s + sel + 8, hi);
+    for (int z = 0; z < 4; ++z) tk[z] = A.tok[role][z][(row * A.H + h) * 64 + lane].bits;
   };
-  if (L == 0) put_state();
-  const size_t cel = (size_t)h * 64 + lane;
-  float w0 = 0.f, a0 = 0.f, v0 = 0.f, k_k = 0.f, k_a = 0.f, ln_w = 0.f, ln_b = 0.f, r_k = 0.f;
-  if (keys) {
-    a0 = ld_f(A.a0 + cel); k_k = ld_f(A.k_k + cel); k_a = ld_f(A.k_a + cel);
-    ln_w = ld_f(A.ln_w + cel); ln_b = ld_f(A.ln_b + cel); r_k = ld_f(A.r_k + cel);
-  } else if (values) {
-    w0 = ld_f(A.w0 + cel);
-    if (A.vf != nullptr) v0 = ld_f(A.v0 + cel);
+  auto request = [&](int64_t b) {
+    const uint4* p = reinterpret_cast<const uint4*>(A.s + (size_t)b * A.bstride + in_state);
+    s0 = p[0];
+    s1 = p[1];
+    if (maker) request_token(b * A.T);
+  };
+  uint32_t pv[6] = {0u, 0u, 0u, 0u, 0u, 0u};
+  if (maker) {
+#pragma unroll
+    for (int z = 0; z < 6; ++z) pv[z] = A.par[role][z][h * 64 + lane].bits;
   }
-  for (int64_t t = 0; t < A.T; ++t) {
-    float v = 0.f, gate = 0.f, bonus = 0.f, k = 0.f, r = 0.f, vf = 0.f, xw = 0.f, xa = 0.f, xv = 0.f;
-    const size_t el = (((size_t)b * A.T + t) * A.H + h) * 64 + lane;
-    if (keys) {
-      k = ld_f(A.k + el); r = ld_f(A.r + el);
-      xa = ld_f(A.xa + el); gate = ld_f(A.g + el);
-    } else if (values) {
-      v = ld_f(A.v + el); xw = ld_f(A.xw + el);
-      if (A.vf != nullptr) { vf = ld_f(A.vf + el); xv = ld_f(A.xv + el); }
-    }
-    if (keys) {
-      const float a = rnd(sigmoidf(a0 + xa));
-      float kk = k * k_k;
-      kk *= 1.f / fmaxf(sqrtf(wave_sum(kk * kk)), 1e-12f);
-      const float kp = rnd(k * (1.f + (a - 1.f) * k_a));
-      bonus = wave_sum(r * kp * r_k);
-      ch[1][lane] = kp;
-      ch[2][lane] = rnd(-kk);
-      ch[3][lane] = rnd(kk * a);
-      ch[4][lane] = r;
-    } else if (values) {
-      if (A.vf != nullptr) v = rnd(fmaf(vf - v, sigmoidf(v0 + xv), v));
-      const float w = rnd(-softplusf(-(w0 + xw)) - 0.5f);
-      ch[0][lane] = __expf(-__expf(w));
-      vs[lane] = v;
-    }
-    __syncthreads();
-    if (ns != nullptr && ns[t]) {
+  request(b0);
+  const bool compat = (A.flags & 1u) != 0;
+  for (int64_t b = b0; b < b1; ++b) {
+    int64_t L = A.T;
+    if (A.length != nullptr) { L = A.length[b]; L = L < 0 ? 0 : L < A.T ? L : A.T; }
+    const uint8_t* ns = A.ns ? A.ns + b * A.T : nullptr;
+    const bool q2drop = compat && L < A.T && ns != nullptr && ns[L] != 0;
+    bf16_t* const out = A.new_s + (size_t)b * A.bstride + in_state;
+    asm volatile("" : "+v"(s0.x), "+v"(s0.y), "+v"(s0.z), "+v"(s0.w), "+v"(s1.x), "+v"(s1.y), "+v"(s1.z), "+v"(s1.w));
+    float S[16];
+    {
+      const uint32_t w[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
 #pragma unroll
-      for (int c = 0; c < 16; ++c) S[c] = 0.f;
+      for (int c = 0; c < 8; ++c) {
+        S[2 * c] = __uint_as_float(w[c] << 16);
+        S[2 * c + 1] = __uint_as_float(w[c] & 0xffff0000u);
+      }
     }
-    float p = 0.f;
+    auto put_state = [&]() {
+      float lo[8], hi[8];
 #pragma unroll
-    for (int c = 0; c < 16; ++c) p = fmaf(S[c], ch[2][c0 + c], p);
-    const float sa = quad_sum(p), vi = vs[i];
-    if (keys) v = vs[lane];                            // before wave 1 writes the next token's
-    float y = 0.f;
+      for (int c = 0; c < 8; ++c) { lo[c] = q2drop ? 0.f : S[c]; hi[c] = q2drop ? 0.f : S[8 + c]; }
+      st8(out, lo);
+      st8(out + 8, hi);
+    };
+    if (L == 0) put_state();
+    for (int64_t t = 0; t < A.T; ++t) {
+      asm volatile("" : "+v"(tk[0]), "+v"(tk[1]), "+v"(tk[2]), "+v"(tk[3]));
+      const float t0 = __uint_as_float(tk[0] << 16), t1 = __uint_as_float(tk[1] << 16), t2 = __uint_as_float(tk[2] << 16),
+                  t3 = __uint_as_float(tk[3] << 16);
+      if (t + 1 < A.T) {
+        if (maker) request_token(b * A.T + t + 1);
+      } else if (b + 1 < b1) {
+        request(b + 1);
+      }
+      asm volatile("" : "+v"(pv[0]), "+v"(pv[1]), "+v"(pv[2]), "+v"(pv[3]), "+v"(pv[4]), "+v"(pv[5]));
+      auto param = [&](int z) { return __uint_as_float(pv[z] << 16); };
+      float bonus = 0.f, v = 0.f;
+      if (wave == 0) {
+        const float a = rnd(sigmoidf(param(0) + t2));
+        float kk = t0 * param(1);
+        kk *= 1.f / fmaxf(sqrtf(wave_sum(kk * kk)), 1e-12f);
+        const float kp = rnd(t0 * (1.f + (a - 1.f) * param(2)));
+        bonus = wave_sum(t1 * kp * param(3));
+        ch[1][lane] = kp;
+        ch[2][lane] = rnd(-kk);
+        ch[3][lane] = rnd(kk * a);
+        ch[4][lane] = t1;
+      } else if (wave == 1) {
+        const float w = rnd(-softplusf(-(param(0) + t1)) - 0.5f);
+        ch[0][lane] = __expf(-__expf(w));
+        vs[lane] = A.vmix ? rnd(fmaf(t2 - t0, sigmoidf(param(1) + t3), t0)) : t0;
+      }
+      __syncthreads();
+      if (ns != nullptr && ns[t]) {
 #pragma unroll
-    for (int c = 0; c < 16; ++c) {
-      S[c] = fmaf(S[c], ch[0][c0 + c], fmaf(vi, ch[1][c0 + c], sa * ch[3][c0 + c]));
-      y = fmaf(S[c], ch[4][c0 + c], y);
-    }
-    y = quad_sum(y);
-    if (compat && t + 1 < A.T && ns != nullptr && ns[t + 1]) y = 0.f;
-    if (q == 0) ys[i] = rnd(y);
-    if (t == L - 1) put_state();
-    __syncthreads();
-    if (keys) {
-      const float yv = ys[lane];
-      const float d = yv - wave_sum(yv) * (1.f / 64.f);
-      const float rstd = rsqrtf(wave_sum(d * d) * (1.f / 64.f) + A.eps);
-      st_f(A.y + el, (d * rstd * ln_w + ln_b + bonus * v) * gate);
+        for (int c = 0; c < 16; ++c) S[c] = 0.f;
+      }
+      float p = 0.f;
+#pragma unroll
+      for (int c = 0; c < 16; ++c) p = fmaf(S[c], ch[2][c0 + c], p);
+      const float sa = quad_sum(p), vi = vs[i];
+      if (wave == 0) v = vs[lane];                       // before wave 1 writes the next token's
+      float y = 0.f;
+#pragma unroll
+      for (int c = 0; c < 16; ++c) {
+        S[c] = fmaf(S[c], ch[0][c0 + c], fmaf(vi, ch[1][c0 + c], sa * ch[3][c0 + c]));
+        y = fmaf(S[c], ch[4][c0 + c], y);
+      }
+      y = quad_sum(y);
+      if (compat && t + 1 < A.T && ns != nullptr && ns[t + 1]) y = 0.f;
+      if (q == 0) ys[i] = rnd(y);
+      if (t == L - 1) put_state();
+      __syncthreads();
+      if (wave == 0) {
+        const float yv = ys[lane];
+        const float d = yv - wave_sum(yv) * (1.f / 64.f);
+        const float rstd = rsqrtf(wave_sum(d * d) * (1.f / 64.f) + A.eps);
+        st_f(A.y + ((b * A.T + t) * A.H + h) * 64 + lane, (d * rstd * param(4) + param(5) + bonus * v) * t3);
+      }
     }
   }
 }
@@ -398,12 +425,16 @@ hipError_t launch_rwkv7_decode(const Rwkv7Decode& D, hipStream_t stream) {
       if (l) add(hv, layer(D.v2, l, C * D.d_mv), xv, D.d_mv, C, 1, GEMM_ACT_NONE);
       HIPRWKV_TRY(launch_gemm(G, 1, stream));
       CoreArgs A = {};
-      A.T = D.T; A.H = D.H;
-      A.r = r; A.k = k; A.v = vl; A.vf = l ? vf : nullptr; A.xw = xw; A.xa = xa; A.xv = xv; A.g = g;
-      A.w0 = w0; A.a0 = a0; A.v0 = v0; A.k_k = k_k; A.k_a = k_a; A.r_k = r_k; A.ln_w = ln_w; A.ln_b = ln_b; A.eps = 64e-5f;
+      const bf16_t* const par[2][6] = {{a0, k_k, k_a, r_k, ln_w, ln_b}, {w0, l ? v0 : w0, w0, w0, w0, w0}};
+      const bf16_t* const tok[2][4] = {{k, r, xa, g}, {vl, xw, l ? vf : vl, l ? xv : vl}};
+      memcpy(A.par, par, sizeof(par));
+      memcpy(A.tok, tok, sizeof(tok));
+      A.B = D.B; A.T = D.T; A.H = D.H; A.eps = 64e-5f; A.vmix = l > 0;
+      // as many workgroups as the GPU holds at once
+      A.per = (int)((D.B * D.H + 256 * CORE_PER_CU - 1) / (256 * CORE_PER_CU));
       A.s = s; A.new_s = new_s; A.bstride = seq_state;
       A.length = D.length; A.ns = D.new_starts; A.flags = (unsigned)D.flags; A.y = y;
-      hipLaunchKernelGGL(decode_core_kernel, heads, dim3(256), 0, stream, A);
+      hipLaunchKernelGGL(decode_core_kernel, dim3((unsigned)D.H, (unsigned)((D.B + A.per - 1) / A.per)), dim3(256), 0, stream, A);
       HIPRWKV_TRY(hipGetLastError());
     }
     G.n_jobs = 0;

@@ -103,3 +103,9 @@ def test_few_rows_with_a_factor_that_is_not_finite(name, value, monkeypatch):
         want = RWKV7.forward(params, tok, state)
     for a, b in zip(got, want):
         assert torch.equal(torch.isfinite(a), torch.isfinite(b))
+
+
+@pytest.mark.parametrize("B,T,C", [(250, 1, 320), (31, 8, 2112), (129, 1, 4096)])
+def test_recurrence_of_several_sequences_a_workgroup(B, T, C, monkeypatch):
+    """More heads than the GPU holds workgroups of: two to nine sequences one after the other, the last workgroup with fewer."""
+    test_native_decode_step(B, T, C, True, monkeypatch)
