@@ -594,7 +594,7 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_bwd_a_f32_kernel(Wk
       }
     }
     if (MODE == SUMMARY) {
-      unusable = store_summary(C.S, cq, lane, *part_sum(A, head, part), map);
+      unusable = store_summary<true>(C.S, cq, lane, *part_sum(A, head, part), map);
     } else if (c0 == 0) {
       // cotangent of the input state; with length == 0 the returned state is the input state itself
       const bool pass = L == 0 && inject;

@@ -736,7 +736,7 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_kernel(Wkv7Args
       si = sn;
     }
     if (MODE == SUMMARY) {
-      unusable = store_summary(C.S, C.q, C.lane, *part_sum(A, head, part), map);
+      unusable = store_summary<false>(C.S, C.q, C.lane, *part_sum(A, head, part), map);
     } else if (j0 + n == nch) {
       // an operand beyond the fp16 range leaves inf or NaN in the carried state (until a reset discards it): count it
       count_nonfinite(C.S, lane, events_word(A.status));

@@ -624,7 +624,7 @@ __global__ __launch_bounds__(64 * (NCONS + NPROD)) void wkv7_fwd_f32_kernel(Wkv7
         end += A.end_chunks;
       }
     }
-    if (MODE == SUMMARY) unusable = store_summary(C.S, cq, lane, *part_sum(A, head, part), map);
+    if (MODE == SUMMARY) unusable = store_summary<true>(C.S, cq, lane, *part_sum(A, head, part), map);
   } else {
     const int p = wave - NCONS;
     Raw raw;

@@ -34,8 +34,8 @@ enum { WHOLE = 0, SUMMARY = 1, PART = 2 };
 // cycles a KiB, 2.3 us a predecessor), and eight words (one per consumer wave of the two workgroups that make it) that are not
 // zero where the summary must not be used.  Parts count in the direction of the sweep.
 struct PartSum {
-  f32x4_t M[4][4][64];     // [tile][jt], lane (x, g): M[key 16 tile + 4g + i][key 16 jt + x]
-  f32x4_t B[4][4][64];     // [q][tile]: consumer q's state tiles
+  f32x4_t M[4][4][64];     // [tile][jt], lane (x, g): M[key 16 tile + 4g + i][key 16 jt + x]; for the fp64 fold key 16 tile + 4i + g
+  f32x4_t B[4][4][64];     // [q][tile]: consumer q's state tiles, their keys in the same order
 };
 constexpr float PART_MAX_GAIN = 4.f;
 __device__ __forceinline__ PartSum* part_sum(const Wkv7Args& A, int64_t head, int part) {
@@ -92,35 +92,47 @@ __device__ __forceinline__ void fold_parts(f32x4_t (&S)[4], int q, int lane, con
 }
 // The same on the fp64 matrix instruction, for the fp32 kernels, at 64 cycles an instruction: with sums of 64 terms in fp32 the state
 // at a boundary was 1.4 times as far from 64 bits as the whole sequence's (B=1 T=1024 H=2, decay exp(-exp(-2.5))).  Its register i
-// holds row 4i + g of a tile where the fp32 one holds 4g + i; the last step turns the tiles back.
+// holds row 4i + g of a tile where the fp32 one holds 4g + i; the summaries lie in that order, so that a lane's operands are 16 bytes
+// (gathered from the fp32 order they were 80 requests of four bytes a predecessor, waited for tile by tile), and the last step turns the
+// tiles back.  B=3 T=777 H=12: forward in five parts 46.5 -> 41.2 us, sweep A in seven 51.6 -> 39.8.
 __device__ __forceinline__ void fold_parts_f64(f32x4_t (&S)[4], int q, int lane, const Wkv7Args& A, int64_t head, int part) {
   typedef double f64x4_t __attribute__((ext_vector_type(4)));
   const int x = lane & 15, g = lane >> 4;
-  // element (row 4i + g, column x) of a 16x16 tile stored as [lane (x, row / 4)][row % 4]
-  auto el = [&](const f32x4_t* tile, int i) { return reinterpret_cast<const float*>(tile + 16 * i + x)[g]; };
-  f64x4_t s[4];
+  f64x4_t s[4], acc[4];
+  f32x4_t m[4][4], b[4];
+  auto load_b = [&](int p) {
 #pragma unroll
-  for (int tile = 0; tile < 4; ++tile)
+    for (int jt = 0; jt < 4; ++jt) b[jt] = part_sum(A, head, p)->B[q][jt][lane];
+  };
+  auto load_m = [&](int p, int tile) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) s[tile][i] = (double)el(part_sum(A, head, 0)->B[q][tile], i);
-  for (int p = 1; p < part; ++p) {
-    const PartSum* const ps = part_sum(A, head, p);
-    f64x4_t acc[4];
+    for (int jt = 0; jt < 4; ++jt) m[tile][jt] = part_sum(A, head, p)->M[tile][jt][lane];
+  };
+  auto widen = [&](f64x4_t (&o)[4]) {
 #pragma unroll
     for (int jt = 0; jt < 4; ++jt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[jt][i] = (double)el(ps->B[q][jt], i);
+      for (int i = 0; i < 4; ++i) o[jt][i] = (double)b[jt][i];
+  };
+  load_b(0);
+  widen(s);
+  if (part > 1) {
+    load_b(1);
+#pragma unroll
+    for (int tile = 0; tile < 4; ++tile) load_m(1, tile);
+  }
+  // a predecessor's 20 KiB are requested while the one before it is multiplied
+  for (int p = 1; p < part; ++p) {
+    const int next = p + 1 < part ? p + 1 : p;
+    widen(acc);
+    load_b(next);
 #pragma unroll
     for (int tile = 0; tile < 4; ++tile) {
-      float m[4][4];
-#pragma unroll
-      for (int jt = 0; jt < 4; ++jt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) m[jt][i] = el(ps->M[tile][jt], i);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int jt = 0; jt < 4; ++jt) acc[jt] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)m[jt][i], s[tile][i], acc[jt], 0, 0, 0);
+        for (int jt = 0; jt < 4; ++jt) acc[jt] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)m[tile][jt][i], s[tile][i], acc[jt], 0, 0, 0);
+      load_m(next, tile);
     }
 #pragma unroll
     for (int jt = 0; jt < 4; ++jt) s[jt] = acc[jt];
@@ -139,7 +151,8 @@ __device__ __forceinline__ void fold_parts_f64(f32x4_t (&S)[4], int q, int lane,
       S[tile][i] = r;
     }
 }
-// writes a consumer's rows of one half of a summary; not zero if it must not be used
+// writes a consumer's rows of one half of a summary, in the order of the fold that reads it; not zero if it must not be used
+template <bool F64>
 __device__ __forceinline__ int store_summary(const f32x4_t (&S)[4], int q, int lane, PartSum& ps, bool map) {
   const int x = lane & 15, g = lane >> 4;
   const float limit = map ? PART_MAX_GAIN : 3.0e38f;
@@ -149,9 +162,11 @@ __device__ __forceinline__ int store_summary(const f32x4_t (&S)[4], int q, int l
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       bad |= !(fabsf(S[tile][i]) <= limit);
-      if (map) reinterpret_cast<float*>(&ps.M[q][tile][16 * (x >> 2) + 4 * g + i])[x & 3] = S[tile][i];
+      // key x of the tile is (x >> 2, x & 3) as (lane, register) of the fp32 instruction's operand and the other way round of the fp64 one's
+      if (map) reinterpret_cast<float*>(&ps.M[q][tile][16 * (F64 ? x & 3 : x >> 2) + 4 * g + i])[F64 ? x >> 2 : x & 3] = S[tile][i];
+      else if (F64) reinterpret_cast<float*>(&ps.B[q][tile][16 * i + x])[g] = S[tile][i];
     }
-    if (!map) ps.B[q][tile][lane] = S[tile];
+    if (!map && !F64) ps.B[q][tile][lane] = S[tile];
   }
   return __ballot(bad) != 0 ? 1 : 0;
 }
