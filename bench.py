@@ -29,9 +29,9 @@ B, T, H, N = 8, 4096, 32, 64
 # figures in profiles/), each with the sha1 prefix of the kernel source it was measured on: when the source has
 # changed since, `roofline.traffic` is null instead of a stale figure.
 MEASURED_TRAFFIC = {
-    "wkv7_fwd": (948.7e6, "wkv7_fwd.hip", "3826360bc53f", "profiles/wkv7_fwd_B8_T4096_H32_bf16.md"),
+    "wkv7_fwd": (948.7e6, "wkv7_fwd.hip", "26833ac91fd2", "profiles/wkv7_fwd_B8_T4096_H32_bf16.md"),
     "wkv4_fwd": (4028.7e6, "wkv4.hip", "224549c5651e", "profiles/wkv4_fwd_B32_T4096_C2560_f32.md"),
-    "wkv6_fwd": (688.4e6, "wkv6_fwd.hip", "ffdebea1aab9", "profiles/wkv6_fwd_bwd_B16_T2048_H32_bf16.md"),
+    "wkv6_fwd": (688.4e6, "wkv6_fwd.hip", "970ca6495ddd", "profiles/wkv6_fwd_bwd_B16_T2048_H32_bf16.md"),
 }
 
 
