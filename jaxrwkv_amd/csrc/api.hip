@@ -1131,7 +1131,7 @@ int hiprwkv_wkv4_mix_bwd(hiprwkv_stream stream, int io_dtype, int64_t B, int64_t
     ReduceArgs R;
     R.part = A.gw; R.rows = B * A.nz; R.nk = 2; R.C = C;
     R.out[0] = gw; R.out[1] = gu;
-    e = launch_reduce_parts(A.io_f32, R, st);
+    e = reduce_parts(A.io_f32, R, nullptr, st);
   }
   return gate_done("wkv4_mix_bwd", e);
 }

@@ -313,13 +313,22 @@ __global__ __launch_bounds__(64 * MAX_WAVES) void ln_shiftmix_bwd_kernel(LnMixAr
 
 // out_k[c] = sum over p of part[p][k][c]; a workgroup owns 64 consecutive of the nk*C columns, its sixteen waves every sixteenth row.
 // Bound by the wait for the rows, eight of a wave's in flight; with four waves and four rows a training step of
-// 12 layers of 768 channels and 2048 tokens (its 50 sums, up to 512 rows of 6144 columns) took 8.6 us each on average, now 4.8.
+// 12 layers of 768 channels and 2048 tokens (its 50 sums, up to 512 rows of 6144 columns) took 8.6 us each on average, then 4.8, about 2 of
+// them the launch.  Three of a layer's four go into one now (26 launches: the step 6341 -> 6237 us).
 constexpr int REDUCE_WAVES = 16;
 template <typename T>
-__global__ __launch_bounds__(64 * REDUCE_WAVES) void reduce_parts_kernel(ReduceArgs A) {
+__global__ __launch_bounds__(64 * REDUCE_WAVES) void reduce_parts_kernel(ReduceJobs J) {
   __shared__ float red[REDUCE_WAVES][64];
+  int64_t block = blockIdx.x;
+  int ji = 0;
+  for (; ji + 1 < J.n; ++ji) {
+    const int64_t blocks = ((int64_t)J.job[ji].nk * J.job[ji].C + 63) / 64;
+    if (block < blocks) break;
+    block -= blocks;
+  }
+  const ReduceArgs& A = J.job[ji];
   const int64_t cols = (int64_t)A.nk * A.C;
-  const int64_t col = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
+  const int64_t col = block * 64 + (threadIdx.x & 63);
   const int wv = threadIdx.x >> 6;
   float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (col < cols) {
@@ -345,11 +354,24 @@ __global__ __launch_bounds__(64 * REDUCE_WAVES) void reduce_parts_kernel(ReduceA
 
 }  // namespace
 
-hipError_t launch_reduce_parts(int io_f32, const ReduceArgs& A, hipStream_t stream) {
-  const dim3 grid((unsigned)(((int64_t)A.nk * A.C + 63) / 64)), block(64 * REDUCE_WAVES);
-  if (io_f32) hipLaunchKernelGGL(reduce_parts_kernel<float>, grid, block, 0, stream, A);
-  else hipLaunchKernelGGL(reduce_parts_kernel<bf16_t>, grid, block, 0, stream, A);
+hipError_t launch_reduce_parts(int io_f32, const ReduceJobs& J, hipStream_t stream) {
+  int64_t blocks = 0;
+  for (int i = 0; i < J.n; ++i) blocks += ((int64_t)J.job[i].nk * J.job[i].C + 63) / 64;
+  const dim3 grid((unsigned)blocks), block(64 * REDUCE_WAVES);
+  if (io_f32) hipLaunchKernelGGL(reduce_parts_kernel<float>, grid, block, 0, stream, J);
+  else hipLaunchKernelGGL(reduce_parts_kernel<bf16_t>, grid, block, 0, stream, J);
   return hipGetLastError();
+}
+hipError_t reduce_parts(int io_f32, const ReduceArgs& A, ReduceJobs* later, hipStream_t stream) {
+  if (later != nullptr) {
+    later->job[later->n++] = A;
+    return hipSuccess;
+  }
+  ReduceJobs J;
+  memset(&J, 0, sizeof(J));
+  J.n = 1;
+  J.job[0] = A;
+  return launch_reduce_parts(io_f32, J, stream);
 }
 
 // Tokens per workgroup.  Forward: 8 keep the re-reading of the token before a run at an eighth; shorter runs while that
@@ -388,7 +410,7 @@ hipError_t launch_ln_shiftmix(int io_f32, int n_out, LnMixArgs A, hipStream_t st
   return hipGetLastError();
 }
 
-hipError_t launch_ln_shiftmix_bwd(int io_f32, int n_out, LnMixArgs A, void* const* dparam, hipStream_t stream) {
+hipError_t launch_ln_shiftmix_bwd(int io_f32, int n_out, LnMixArgs A, void* const* dparam, hipStream_t stream, ReduceJobs* later) {
   A.run = ln_shiftmix_bwd_run(A.B * A.T);
   const bool four = A.C <= 4 * 64 * MAX_WAVES;
   const dim3 grid((unsigned)((A.B * A.T + A.run - 1) / A.run)), block((unsigned)((A.C / (four ? 4 : 8) + 63) / 64 * 64));
@@ -399,7 +421,7 @@ hipError_t launch_ln_shiftmix_bwd(int io_f32, int n_out, LnMixArgs A, void* cons
   ReduceArgs R;
   R.part = A.part; R.rows = grid.x; R.nk = n_out + 2; R.C = A.C;
   for (int i = 0; i < n_out + 2; ++i) R.out[i] = dparam[i];
-  return launch_reduce_parts(io_f32, R, stream);
+  return reduce_parts(io_f32, R, later, stream);
 }
 
 }  // namespace hiprwkv

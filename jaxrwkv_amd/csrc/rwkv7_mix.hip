@@ -302,7 +302,7 @@ hipError_t launch_rwkv7_postmix_bwd(int io_f32, int64_t rows, int64_t H, const v
                                     const void* v, const void* g, const void* ln_w, const void* ln_b, const void* r_k,
                                     float eps, const void* go, void* gy, void* gr, void* gk, void* gv, void* gg,
                                     float* gln_w, float* gln_b, float* gr_k, float* part, void* const* dparam,
-                                    hipStream_t stream) {
+                                    hipStream_t stream, ReduceJobs* later) {
   const int np = (int)(H * 64);
   if (part == nullptr) {
     hipLaunchKernelGGL(zero_f32_kernel, dim3((np + 255) / 256), dim3(256), 0, stream, gln_w, np);
@@ -326,7 +326,7 @@ hipError_t launch_rwkv7_postmix_bwd(int io_f32, int64_t rows, int64_t H, const v
   ReduceArgs R;
   R.part = part; R.rows = row_blocks; R.nk = 3; R.C = np;
   for (int i = 0; i < 3; ++i) R.out[i] = dparam[i];
-  return launch_reduce_parts(io_f32, R, stream);
+  return reduce_parts(io_f32, R, later, stream);
 }
 
 }  // namespace hiprwkv

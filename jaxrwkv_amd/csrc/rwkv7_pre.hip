@@ -192,7 +192,7 @@ hipError_t launch_rwkv7_pre(int io_f32, const PreArgs& A, hipStream_t stream) {
 }
 
 // dparam: w0, a0, k_k, k_a and, with the value residual, v0
-hipError_t launch_rwkv7_pre_bwd(int io_f32, const PreArgs& A, void* const* dparam, hipStream_t stream) {
+hipError_t launch_rwkv7_pre_bwd(int io_f32, const PreArgs& A, void* const* dparam, hipStream_t stream, ReduceJobs* later) {
   const int64_t nrb = rwkv7_pre_bwd_rows(A.rows, A.H);
   const dim3 grid((unsigned)(nrb * A.H)), block(BWD_THREADS);
   const bool vmix = A.vf != nullptr;
@@ -208,7 +208,7 @@ hipError_t launch_rwkv7_pre_bwd(int io_f32, const PreArgs& A, void* const* dpara
   ReduceArgs R;
   R.part = A.part; R.rows = nrb; R.nk = vmix ? 5 : 4; R.C = A.H * 64;
   for (int i = 0; i < R.nk; ++i) R.out[i] = dparam[i];
-  return launch_reduce_parts(io_f32, R, stream);
+  return reduce_parts(io_f32, R, later, stream);
 }
 
 }  // namespace hiprwkv

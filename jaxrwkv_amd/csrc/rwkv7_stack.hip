@@ -116,7 +116,7 @@ struct Forward {
 struct Backward {
   bf16_t *gff, *gxk2, *dx2, *dx, *gy, *gyw, *gr1, *gk1, *gv1, *gg, *gr2, *gw, *gk2, *gv2, *ga, *gb, *gs, *gr, *dl[4], *dk, *dv, *dvf,
       *dmix[6], *dh[4];
-  float* part;
+  float *part, *parts[3];      // the first head's; channel mixing's head, group norm, gates
   void *wkv, *ends;
   size_t wkv_bytes;
   Backward(const Stack& K, Arena& A) {
@@ -130,12 +130,17 @@ struct Backward {
     for (int i = 0; i < 6; ++i) dmix[i] = over[i];
     gs = A.take((size_t)D.B * D.H * 4096);
     for (int i = 0; i < 4; ++i) { dl[i] = i == 2 ? gg : A.take(n); dh[i] = A.take(K.rows * K.d[i]); }
-    size_t bytes = hiprwkv_rwkv7_ln_shiftmix_bwd_workspace_bytes(D.B, D.T, D.C, 6);
-    for (size_t b : {hiprwkv_rwkv7_ln_shiftmix_bwd_workspace_bytes(D.B, D.T, D.C, 1),
-                     hiprwkv_rwkv7_postmix_bwd2_workspace_bytes(D.B * D.T, D.H, 64),
-                     hiprwkv_rwkv7_pre_bwd_workspace_bytes(D.B * D.T, D.H, 64)})
-      bytes = b > bytes ? b : bytes;
-    part = reinterpret_cast<float*>(A.take<char>(bytes));
+    // workgroups' rows of sums: three kernels' side by side, which one launch adds up, then the first head's in the same memory (more of them
+    // than of the three together, but for models of a head or two)
+    const size_t bytes = hiprwkv_rwkv7_ln_shiftmix_bwd_workspace_bytes(D.B, D.T, D.C, 6);
+    const size_t each[3] = {hiprwkv_rwkv7_ln_shiftmix_bwd_workspace_bytes(D.B, D.T, D.C, 1),
+                            hiprwkv_rwkv7_postmix_bwd2_workspace_bytes(D.B * D.T, D.H, 64),
+                            hiprwkv_rwkv7_pre_bwd_workspace_bytes(D.B * D.T, D.H, 64)};
+    size_t at[4] = {0, 0, 0, 0};
+    for (int i = 0; i < 3; ++i) at[i + 1] = at[i] + (each[i] + 255) / 256 * 256;
+    char* const rows = A.take<char>(bytes > at[3] ? bytes : at[3]);
+    part = reinterpret_cast<float*>(rows);
+    for (int i = 0; i < 3; ++i) parts[i] = reinterpret_cast<float*>(rows + at[i]);
     wkv_bytes = K.ends_bytes() ? hiprwkv_wkv7_bwd_ends_workspace_bytes(HIPRWKV_BF16, D.B, D.T, D.H, 64)
                                : hiprwkv_wkv7_bwd_workspace_bytes(D.B, D.T, D.H, 64);
     wkv = A.take<char>(wkv_bytes);
@@ -261,16 +266,16 @@ int launch_rwkv7_stack_bwd(const Rwkv7Stack& D, hipStream_t stream, hipError_t& 
     v_first = K.layer(first, true, 0).v;
   }
   auto head = [&](int n_out, const bf16_t* x, float* stats, const void* w, const void* b, int64_t l, int srow, const void* const* mix,
-                  bf16_t* const* g, const void* gx, void* out, void* const* dparam) {
+                  bf16_t* const* g, const void* gx, void* out, void* const* dparam, float* part, ReduceJobs* later) {
     LnMixArgs N;
     memset(&N, 0, sizeof(N));
     N.B = D.B; N.T = D.T; N.C = D.C; N.eps = EPS; N.ns = D.new_starts; N.length = D.length;
     N.xs = const_cast<bf16_t*>(x); N.stats = stats; N.ln_w = w; N.ln_b = b;
     N.prev = st + l * row_state + srow * C; N.prev_bstride = D.L * row_state;
-    N.gx = gx; N.dxs = out; N.part = W.part;
+    N.gx = gx; N.dxs = out; N.part = part;
     if (D.g_shift != nullptr) N.gshift = static_cast<const bf16_t*>(D.g_shift) + ((size_t)srow * D.L + l) * D.B * C;
     for (int i = 0; i < n_out; ++i) { N.mix[i] = mix[i]; N.g[i] = g[i]; }
-    return launch_ln_shiftmix_bwd(0, n_out, N, dparam, stream);
+    return launch_ln_shiftmix_bwd(0, n_out, N, dparam, stream, later);
   };
   const void *g_x = D.g_xs, *g_dx = D.g_dx;
   for (int64_t l = D.L - 1; l >= 0; --l) {
@@ -290,8 +295,11 @@ int launch_rwkv7_stack_bwd(const Rwkv7Stack& D, hipStream_t stream, hipError_t& 
       HIPRWKV_TRY(Q.launch(stream));
     }
     const void* const fmix[1] = {of(P.ffn_x_k, l, C)};
+    ReduceJobs sums;
+    memset(&sums, 0, sizeof(sums));
     void* const dhead2[3] = {to(G.ffn_x_k, l, C), to(G.ln2_w, l, C), to(G.ln2_b, l, C)};
-    HIPRWKV_TRY(head(1, S.x2, S.stats2, of(P.ln2_w, l, C), of(P.ln2_b, l, C), l, 0, fmix, &W.gxk2, g_x, W.dx2, dhead2));
+    HIPRWKV_TRY(head(1, S.x2, S.stats2, of(P.ln2_w, l, C), of(P.ln2_b, l, C), l, 0, fmix, &W.gxk2, g_x, W.dx2, dhead2, W.parts[0],
+                     &sums));
     // time mixing: output projection, group norm and gate
     {
       Products Q;
@@ -302,7 +310,7 @@ int launch_rwkv7_stack_bwd(const Rwkv7Stack& D, hipStream_t stream, hipError_t& 
     void* const dpost[3] = {to(G.lnx_w, l, C), to(G.lnx_b, l, C), to(G.r_k, l, C)};
     HIPRWKV_TRY(launch_rwkv7_postmix_bwd(0, M, D.H, S.yw, S.r, S.k2, S.v2, S.lora[2], of(P.lnx_w, l, C), of(P.lnx_b, l, C),
                                          of(P.r_k, l, C), EPS_X, W.gy, W.gyw, W.gr1, W.gk1, W.gv1, W.gg, nullptr, nullptr, nullptr,
-                                         W.part, dpost, stream));
+                                         W.parts[1], dpost, stream, &sums));
     // the recurrence
     HIPRWKV_TRY_RC(hiprwkv_wkv7_bwd_ends(stream, HIPRWKV_BF16, HIPRWKV_BF16, D.B, D.T, D.H, 64, S.w, S.r, S.k2, S.v2, S.a, S.b,
                                          of(D.s, l, states), reinterpret_cast<const uint32_t*>(D.length), D.new_starts, W.gyw, S.sa,
@@ -319,9 +327,10 @@ int launch_rwkv7_stack_bwd(const Rwkv7Stack& D, hipStream_t stream, hipError_t& 
     R.dxw = W.dl[0]; R.dk = W.dk; (l ? R.dv : R.dv_sum) = W.dv; R.dxa = W.dl[1];
     R.gvf = l == D.L - 1 ? nullptr : W.dvf;
     if (l) { R.v = S.v; R.vf = v_first; R.xv = S.lora[3]; R.v0 = of(P.v0, l, C); R.dvf = W.dvf; R.dxv = W.dl[3]; }
-    R.part = W.part;
+    R.part = W.parts[2];
     void* const dpre[5] = {to(G.w0, l, C), to(G.a0, l, C), to(G.k_k, l, C), to(G.k_a, l, C), l ? to(G.v0, l, C) : nullptr};
-    HIPRWKV_TRY(launch_rwkv7_pre_bwd(0, R, dpre, stream));
+    HIPRWKV_TRY(launch_rwkv7_pre_bwd(0, R, dpre, stream, &sums));
+    HIPRWKV_TRY(launch_reduce_parts(0, sums, stream));
     // projections
     const int n_lora = l ? 4 : 3;
     const void* const f1[4] = {of(P.w1, l, C * K.d[0]), of(P.a1, l, C * K.d[1]), of(P.g1, l, C * K.d[2]), of(P.v1, l, C * K.d[3])};
@@ -354,7 +363,7 @@ int launch_rwkv7_stack_bwd(const Rwkv7Stack& D, hipStream_t stream, hipError_t& 
     void* const dhead1[8] = {to(G.x_r, l, C), to(G.x_w, l, C), to(G.x_k, l, C), to(G.x_v, l, C), to(G.x_a, l, C), to(G.x_g, l, C),
                              to(G.ln1_w, l, C), to(G.ln1_b, l, C)};
     void* const out = l ? W.dx : D.g_x;
-    HIPRWKV_TRY(head(6, S.x, S.stats1, of(P.ln1_w, l, C), of(P.ln1_b, l, C), l, 1, mixv, W.dmix, W.dx2, out, dhead1));
+    HIPRWKV_TRY(head(6, S.x, S.stats1, of(P.ln1_w, l, C), of(P.ln1_b, l, C), l, 1, mixv, W.dmix, W.dx2, out, dhead1, W.part, nullptr));
     g_x = g_dx = out;
   }
   return HIPRWKV_OK;

@@ -146,10 +146,16 @@ struct ReduceArgs {
   int nk;
   void* out[8];                  // nk arrays (C,)
 };
-hipError_t launch_reduce_parts(int io_f32, const ReduceArgs& A, hipStream_t stream);
+// Several of them in one launch: where a launcher below is given one, its sum is added to it instead of launched
+struct ReduceJobs {
+  int n;
+  ReduceArgs job[3];
+};
+hipError_t launch_reduce_parts(int io_f32, const ReduceJobs& J, hipStream_t stream);
+hipError_t reduce_parts(int io_f32, const ReduceArgs& A, ReduceJobs* later, hipStream_t stream);
 int64_t ln_shiftmix_bwd_run(int64_t rows);
 hipError_t launch_ln_shiftmix(int io_f32, int n_out, LnMixArgs A, hipStream_t stream);
-hipError_t launch_ln_shiftmix_bwd(int io_f32, int n_out, LnMixArgs A, void* const* dparam, hipStream_t stream);
+hipError_t launch_ln_shiftmix_bwd(int io_f32, int n_out, LnMixArgs A, void* const* dparam, hipStream_t stream, ReduceJobs* later = nullptr);
 
 // Element-wise work between the projections and the WKV op (rwkv7_pre.hip); token tensors (rows, H, 64), parameters (H, 64)
 struct PreArgs {
@@ -169,7 +175,7 @@ struct PreArgs {
 };
 int64_t rwkv7_pre_bwd_rows(int64_t rows, int64_t H);
 hipError_t launch_rwkv7_pre(int io_f32, const PreArgs& A, hipStream_t stream);
-hipError_t launch_rwkv7_pre_bwd(int io_f32, const PreArgs& A, void* const* dparam, hipStream_t stream);
+hipError_t launch_rwkv7_pre_bwd(int io_f32, const PreArgs& A, void* const* dparam, hipStream_t stream, ReduceJobs* later = nullptr);
 
 // Several products per launch (rwkv7_gemm.hip), bf16: out[m][n] = f(sum_k x(m, k) w(n, k)).  The job is the C ABI's
 // (hiprwkv_gemm_job) and more; tile0 is the launcher's.
@@ -284,7 +290,7 @@ hipError_t launch_rwkv7_postmix_bwd(int io_f32, int64_t rows, int64_t H, const v
                                     const void* v, const void* g, const void* ln_w, const void* ln_b, const void* r_k,
                                     float eps, const void* go, void* gy, void* gr, void* gk, void* gv, void* gg,
                                     float* gln_w, float* gln_b, float* gr_k, float* part, void* const* dparam,
-                                    hipStream_t stream);
+                                    hipStream_t stream, ReduceJobs* later = nullptr);
 int64_t rwkv7_postmix_bwd_rows(int64_t rows, int64_t H);
 
 }  // namespace hiprwkv
