@@ -712,11 +712,15 @@ __global__ __launch_bounds__(64 * WM * WN) void stream_gemm_kernel(GemmArgs A) {
   int ji, n0, m0;
   if (!tile_of(A, TM, TN, ji, n0, m0)) return;
   const GemmJob J = A.job[ji];
-  switch ((J.km ? 2 : 0) + (J.kn ? 1 : 0)) {
-    case 0: stream_gemm_body<TM, TN, BUFS, WM, WN, false, false>(A, J, n0, m0, stream_lds); break;
-    case 1: stream_gemm_body<TM, TN, BUFS, WM, WN, false, true>(A, J, n0, m0, stream_lds); break;
-    case 2: stream_gemm_body<TM, TN, BUFS, WM, WN, true, false>(A, J, n0, m0, stream_lds); break;
-    default: stream_gemm_body<TM, TN, BUFS, WM, WN, true, true>(A, J, n0, m0, stream_lds); break;
+  if constexpr (TM > 2 * TG) {                   // launch_gemm gives these tiles no transposed operands
+    stream_gemm_body<TM, TN, BUFS, WM, WN, false, false>(A, J, n0, m0, stream_lds);
+  } else {
+    switch ((J.km ? 2 : 0) + (J.kn ? 1 : 0)) {
+      case 0: stream_gemm_body<TM, TN, BUFS, WM, WN, false, false>(A, J, n0, m0, stream_lds); break;
+      case 1: stream_gemm_body<TM, TN, BUFS, WM, WN, false, true>(A, J, n0, m0, stream_lds); break;
+      case 2: stream_gemm_body<TM, TN, BUFS, WM, WN, true, false>(A, J, n0, m0, stream_lds); break;
+      default: stream_gemm_body<TM, TN, BUFS, WM, WN, true, true>(A, J, n0, m0, stream_lds); break;
+    }
   }
 }
 template <int TM, int TN, int BUFS, int WM, int WN>
